@@ -178,7 +178,7 @@ def _head(r, embedding, gain):
 
 # How far the successor stands out: it has a share of 0.95 and more on average.
 T5_GAIN = {'small': 0.75, 'base': 0.65, 'large': 0.7, 'xl': 0.42}
-HYBRID_GAIN = {768: 6.0, 1024: 4.0, 2048: 1.8}
+HYBRID_GAIN = {768: 0.75, 1024: 0.65, 2048: 0.47}
 LATENT_GAIN = {768: 0.6, 1024: 0.52, 2048: 0.4}
 
 
@@ -270,7 +270,8 @@ def _lm_params(case, config):
     for b in (1, 2):
       out[f'{p}norm{b}'] = norm(W)
       if case['family'] == 'hybrid':
-        out[f'{p}norm{b}b'] = norm(W)
+        # (where tokens are chosen the embedding is to be seen behind the branches)
+        out[f'{p}norm{b}b'] = norm(W) * (0.25 if case['kind'] == 'generate' else 1)
       else:
         out[f'{p}hc{b}.in'] = 1.0 / STREAMS + 0.1 * r.normal(STREAMS)
         out[f'{p}hc{b}.out'] = 1.0 + 0.1 * r.normal(STREAMS)
@@ -580,8 +581,8 @@ def tolerance(case):
     if case['dtype'] == 'float32':  # 3e-7
       return {'rel': 2e-6, 'max': 1e-5, 'differ': 0.0}
     return {'rel': 0.025, 'max': 0.06, 'differ': 0.002}  # 0.006, 0.015
-  if kind == 'generate':  # 0.026, 0.05: logarithms of probabilities near 1
-    return {'rel': 0.1, 'max': 0.2, 'differ': 0.002}
+  if kind == 'generate':  # 0.0024, 0.0033
+    return {'rel': 0.01, 'max': 0.015, 'differ': 0.002}
   if kind == 'encode':  # 0.013, 0.07
     return {'rel': 0.05, 'max': 0.25}
   if kind == 'step':  # 0.006, 0.04
