@@ -38,6 +38,7 @@ struct WinArgs {
   t5d_window_attention a;
   t5d_ragged b;
   int HP, gs, splits;
+  int tiles;  // window_rows_kernel: tiles of rows of the longest portion
   float* parts;  // [S, G, splits, gs, HP + 2]
   const int32_t* gate;
   // window_rows_kernel over a span instead of rings: position first[s] + i of
@@ -218,20 +219,55 @@ __device__ __forceinline__ f32x4_v mfma(const Frag& x, const Frag& y, f32x4_v c)
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, y.v, c, 0, 0, 0);
 }
 
-template <int DT, bool SPAN = false>
+typedef __attribute__((address_space(3))) void* lds_void_t;
+typedef __attribute__((address_space(1))) const void* glb_void_t;
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4_v;
+typedef __attribute__((address_space(3))) s16x4_v* lds_s16x4_t;
+
+// A running maximum is raised, and what has been summed rescaled, only when a
+// score passes it by this much (in powers of two): weights then reach 2^8, which
+// their two terms and the float32 sums hold as well as weights up to 1.
+constexpr float kMaxSlack = 8.0f;
+
+// Keys and values of 64 positions at a time go from memory straight into LDS (no
+// staging registers), one tile ahead in a second pair of buffers, one barrier per
+// tile.  Rows lie in LDS as they are; the 16-byte pieces of a row are exchanged by
+// an XOR with its number, which each lane applies to the address it fetches, so
+// that 16 rows of one piece (key operands) and 8 rows of one 32-byte pair (value
+// operands) cover all banks.  The operands of V^T are read with the transposing
+// LDS read: 16 lanes give it 4 keys x 16 dims and get 4 keys of a dim each.
+// BIAS: with slopes, or a scale that is not positive.
+// Per tile and wavefront 96 matrix instructions (1536 cycles) stand against ~390
+// vector instructions (1950 cycles with the 32 exponentials): what bounds the kernel
+// is that the two hardly overlap at two wavefronts per SIMD (36 % and 40 % busy;
+// without any loads it would be 7 % faster).  Measured, heads of 128 over 1024
+// positions, 4 x 4096 tokens: 8 heads over 2 key/value heads 206 -> 115 us, 8 heads
+// over expanded latents in pieces of 2048 118 -> 60 us each.  The kernel before
+// staged tiles through registers, with a second barrier and V transposed on the way
+// by 4-byte stores, masked every tile and rescaled in every tile.
+template <int DT, bool SPAN, bool BIAS>
 __global__ void __launch_bounds__(256, DT <= 4 ? 2 : 1)
 window_rows_kernel(WinArgs g) {
   constexpr int HP = DT * 32, VT = DT * 2, KB = 64, MT = 2;
-  constexpr int KS = HP + 8, VS = KB + 8;        // LDS row strides (elements)
-  constexpr int NVP = (VT + 3) / 4;              // V pair pieces per thread
-  __shared__ __align__(16) bf16_t s_k[KB * KS];  // [key][dim]
-  __shared__ __align__(16) bf16_t s_v[HP * VS];  // [dim][key]
+  constexpr int PP = HP / 8;  // 16-byte pieces per row
+  // buffers of their own, so that the compiler can tell a read of one tile from a
+  // load of the next
+  __shared__ uint4 s_k0[KB * PP], s_v0[KB * PP], s_k1[KB * PP], s_v1[KB * PP];
   T5D_GATED(g.gate);
   const t5d_window_attention& a = g.a;
-  const int seq = blockIdx.y, kv = blockIdx.z, gs = g.gs;
+  // The tiles of one (portion, key/value head) read the same keys and values:
+  // consecutive block ids go round-robin over the 8 XCDs, so theirs are 8 apart.
+  const int gs = g.gs;
+  const int pair = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / g.tiles);
+  if (pair >= a.G * g.b.S) return;
+  const int seq = pair / a.G, kv = pair - seq * a.G;
   const int off = g.b.seq_off[seq];
   const int rows = (g.b.seq_off[seq + 1] - off) * gs;
-  const int r0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * (64 * MT);
+  // Long tiles first, where the next 256 blocks begin the other way round: the two
+  // tiles of a CU are then a long one and a short one.
+  const int nth = (int)(blockIdx.x >> 3) % g.tiles;
+  const bool turn = (pair >> 3) * g.tiles / 32 % 2 != 0;
+  const int r0 = (turn ? nth : g.tiles - 1 - nth) * (64 * MT);
   if (r0 >= rows) return;
   const int start = g.b.seq_start[seq];
   const int lane = threadIdx.x & 63;
@@ -257,7 +293,7 @@ window_rows_kernel(WinArgs g) {
     head[mt] = kv * gs + (r - t * gs);
     tok[mt] = off + t;
     pos[mt] = start + t;
-    slope2[mt] = a.slopes != nullptr ? a.slopes[head[mt]] * kLog2e : 0.f;
+    slope2[mt] = BIAS && a.slopes != nullptr ? a.slopes[head[mt]] * kLog2e : 0.f;
     mx[mt] = a.sink != nullptr ? a.sink[head[mt]] * kLog2e : kNoMax;
     l[mt] = a.sink != nullptr && gq == 0 ? 1.f : 0.f;
     const bf16_t* q = reinterpret_cast<const bf16_t*>(a.q_rows) +
@@ -279,101 +315,143 @@ window_rows_kernel(WinArgs g) {
   const int wi_hi = start + min(rw + 16 * MT - 1, rows - 1) / gs;
   const int j_begin = max(0, i_lo - W + 1) & ~(KB - 1);
 
-  uint4 kr[DT], va[NVP], vb[NVP];
-  const int kpiece = threadIdx.x % (HP / 8), krow = threadIdx.x / (HP / 8);
-  constexpr int KRS = 256 / (HP / 8);            // key rows per pass
-  const int vpair = threadIdx.x & 31, vcol = threadIdx.x >> 5;
-  auto fetch = [&](int jt) {
-    const size_t r = (size_t)(SPAN ? jt - first : jt % a.ring);
-#pragma unroll
-    for (int i = 0; i < DT; ++i)
-      kr[i] = *reinterpret_cast<const uint4*>(K + (r + krow + KRS * i) * ld_kv +
-                                              8 * kpiece);
-#pragma unroll
-    for (int i = 0; i < NVP; ++i)
-      if (vcol + 8 * i < HP / 8) {
-        const bf16_t* v = V + (r + 2 * vpair) * ld_kv + 8 * (vcol + 8 * i);
-        va[i] = *reinterpret_cast<const uint4*>(v);
-        vb[i] = *reinterpret_cast<const uint4*>(v + ld_kv);
-      }
+  // what to exchange the pieces of a row by: keys, then pairs of values
+  const auto k_swap = [](int row) {
+    return PP >= 16 ? row & 15 : (row / (16 / PP)) & (PP - 1);
   };
-  fetch(j_begin);
-  for (int jt = j_begin; jt <= i_hi; jt += KB) {
-    __syncthreads();  // the previous tile has been read
+  const auto v_swap = [](int row) {
+    return PP >= 16 ? row & 7 : (row / (16 / PP)) & (PP / 2 - 1);
+  };
+  int k_off[DT], v_off[DT];  // of the pieces this lane fetches
+#pragma unroll
+  for (int i = 0; i < DT; ++i) {
+    const int f = (wave * DT + i) * 64 + lane, row = f / PP, piece = f % PP;
+    k_off[i] = row * ld_kv + 8 * (piece ^ k_swap(row));
+    v_off[i] = row * ld_kv + 8 * (piece ^ (2 * v_swap(row)));
+  }
+  const auto fetch = [&](int jt, uint4* sk, uint4* sv) {
+    const size_t r = (size_t)(SPAN ? jt - first : jt % a.ring) * ld_kv;
 #pragma unroll
     for (int i = 0; i < DT; ++i)
-      *reinterpret_cast<uint4*>(s_k + (krow + KRS * i) * KS + 8 * kpiece) = kr[i];
+      __builtin_amdgcn_global_load_lds((glb_void_t)(K + r + k_off[i]),
+                                       (lds_void_t)(sk + (wave * DT + i) * 64), 16, 0,
+                                       0);
 #pragma unroll
-    for (int i = 0; i < NVP; ++i)
-      if (vcol + 8 * i < HP / 8) {
-        // keys 2p and 2p + 1 of 8 dims: one word per dim
-        uint32_t* dst = reinterpret_cast<uint32_t*>(
-            s_v + (size_t)(8 * (vcol + 8 * i)) * VS + 2 * vpair);
-        auto put = [&](int e, uint32_t x, uint32_t y) {
-          dst[(2 * e) * (VS / 2)] = (x & 0xFFFFu) | (y << 16);
-          dst[(2 * e + 1) * (VS / 2)] = (x >> 16) | (y & 0xFFFF0000u);
-        };
-        put(0, va[i].x, vb[i].x);
-        put(1, va[i].y, vb[i].y);
-        put(2, va[i].z, vb[i].z);
-        put(3, va[i].w, vb[i].w);
-      }
-    __syncthreads();
-    if (jt + KB <= i_hi) fetch(jt + KB);
-    if (!wave_on || jt > wi_hi || jt + KB - 1 <= wi_lo - W) continue;
-
+    for (int i = 0; i < DT; ++i)
+      __builtin_amdgcn_global_load_lds((glb_void_t)(V + r + v_off[i]),
+                                       (lds_void_t)(sv + (wave * DT + i) * 64), 16, 0,
+                                       0);
+  };
+  const int k_row = n16 * PP, k_x = k_swap(n16);
+  const int v_key = 4 * gq + (n16 >> 2);
+  const int v_at = v_key * PP * 16 + 8 * (n16 & 3), v_x = 32 * v_swap(v_key);
+  const auto attend = [&](int jt, const uint4* sk, const uint4* sv) {
+    if (!wave_on || jt > wi_hi || jt + KB - 1 <= wi_lo - W) return;
     f32x4_v s[4][MT];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) s[t][mt] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+    // Operands are read one group ahead of the products that take them; the fences
+    // keep the compiler from reading each group when it is due.
+    Frag kf[2][4];
+    const auto keys = [&](int kk) {
 #pragma unroll
-    for (int kk = 0; kk < DT; ++kk)
+      for (int t = 0; t < 4; ++t)
+        kf[kk & 1][t].u = sk[16 * t * PP + k_row + ((4 * kk + gq) ^ k_x)];
+    };
+    keys(0);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        Frag kf;
-        kf.u = *reinterpret_cast<const uint4*>(s_k + (16 * t + n16) * KS + 32 * kk +
-                                               8 * gq);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) s[t][mt] = mfma(kf, qf[mt][kk], s[t][mt]);
-      }
-    const bool edge = !(jt + KB - 1 <= wi_lo && jt > wi_hi - W);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int d0 = pos[mt] - jt - 4 * gq;  // distance to this lane's first key
-      float top = mx[mt];
+    for (int kk = 0; kk < DT; ++kk) {
+      if (kk + 1 < DT) keys(kk + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int dist = d0 - 16 * t - i;
-          float v = fmaf(s[t][mt][i], scale2, -slope2[mt] * (float)dist);
-          if (edge) v = dist >= 0 && dist < W ? v : -INFINITY;
-          s[t][mt][i] = v;
-          top = fmaxf(top, v);
-        }
-      top = rows_max(top);
-      const float alpha = __builtin_amdgcn_exp2f(mx[mt] - top);
-      mx[mt] = top;
+        for (int mt = 0; mt < MT; ++mt)
+          s[t][mt] = mfma(kf[kk & 1][t], qf[mt][kk], s[t][mt]);
+    }
+    // V^T of dims 32 (n % (VT / 2)) .. + 31 and keys 32 (n / (VT / 2)) .. + 31
+    constexpr int NV = VT / 2;
+    Frag vf[2][2];
+    const auto values = [&](int n) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const char* v = reinterpret_cast<const char*>(sv) + 32 * (n / NV) * PP * 16 +
+                        v_at + ((32 * (2 * (n % NV) + j)) ^ v_x);
+        union { s16x4_v h[2]; Frag f; } x;
+        x.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)v);
+        x.h[1] =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(v + 16 * PP * 16));
+        vf[n & 1][j] = x.f;
+      }
+    };
+    const bool edge = !(jt + KB - 1 <= wi_lo && jt > wi_hi - W);
+    float top[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int d0 = pos[mt] - jt - 4 * gq;  // distance to this lane's first key
+      if constexpr (BIAS) {
+        const float far = -slope2[mt] * (float)d0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            s[t][mt][i] = fmaf(s[t][mt][i], scale2,
+                               fmaf(slope2[mt], (float)(16 * t + i), far));
+      }
+      if (edge) {
+        asm volatile("");  // (a branch: the compiler would select in every tile)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            s[t][mt][i] = (uint32_t)(d0 - 16 * t - i) < (uint32_t)W ? s[t][mt][i]
+                                                                    : -INFINITY;
+      }
+      top[mt] = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) top[mt] = fmaxf(top[mt], s[t][mt][i]);
+      top[mt] = rows_max(top[mt]) * (BIAS ? 1.f : scale2);
+    }
+    bool raise = false;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) raise |= top[mt] > mx[mt] + kMaxSlack;
+    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+      asm volatile("");
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const float to = fmaxf(mx[mt], top[mt]);
+        const float alpha = __builtin_amdgcn_exp2f(mx[mt] - to);
+        mx[mt] = to;
+        l[mt] *= alpha;
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[vt][mt][i] *= alpha;
+      }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
       float sum = 0.f;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float p = __builtin_amdgcn_exp2f(s[t][mt][i] - top);
+          const float p = __builtin_amdgcn_exp2f(
+              BIAS ? s[t][mt][i] - mx[mt] : fmaf(s[t][mt][i], scale2, -mx[mt]));
           s[t][mt][i] = p;
           sum += p;
         }
-      l[mt] = l[mt] * alpha + sum;
-#pragma unroll
-      for (int vt = 0; vt < VT; ++vt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[vt][mt][i] *= alpha;
+      l[mt] += sum;
     }
+    values(0);
+    // weights of keys {16 (2 kb) + 4 gq + 0..3, 16 (2 kb + 1) + 4 gq + 0..3}
+    Frag hi[2][MT], lo[2][MT];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      // weights of keys {16 (2 kb) + 4 gq + 0..3, 16 (2 kb + 1) + 4 gq + 0..3}
-      Frag hi[MT], lo[MT];
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         uint32_t h[4], r[4];
@@ -384,23 +462,45 @@ window_rows_kernel(WinArgs g) {
           h[e] = pack_bf16x2(p0, p1);
           r[e] = pack_bf16x2(p0 - bf16lo_to_f32(h[e]), p1 - bf16hi_to_f32(h[e]));
         }
-        hi[mt].u = make_uint4(h[0], h[1], h[2], h[3]);
-        lo[mt].u = make_uint4(r[0], r[1], r[2], r[3]);
+        hi[kb][mt].u = make_uint4(h[0], h[1], h[2], h[3]);
+        lo[kb][mt].u = make_uint4(r[0], r[1], r[2], r[3]);
       }
 #pragma unroll
-      for (int vt = 0; vt < VT; ++vt) {
-        const bf16_t* v = s_v + (16 * vt + n16) * VS + 32 * kb + 4 * gq;
-        const uint2 x = *reinterpret_cast<const uint2*>(v);
-        const uint2 y = *reinterpret_cast<const uint2*>(v + 16);
-        Frag vf;
-        vf.u = make_uint4(x.x, x.y, y.x, y.y);
+    for (int n = 0; n < 2 * NV; ++n) {
+      if (n + 1 < 2 * NV) values(n + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      // (four products between two that add to the same tile)
+      const int kb = n / NV, vt = 2 * (n % NV);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          o[vt][mt] = mfma(vf, hi[mt], o[vt][mt]);
-          o[vt][mt] = mfma(vf, lo[mt], o[vt][mt]);
-        }
-      }
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          o[vt + j][mt] = mfma(vf[n & 1][j], hi[kb][mt], o[vt + j][mt]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          o[vt + j][mt] = mfma(vf[n & 1][j], lo[kb][mt], o[vt + j][mt]);
     }
+  };
+  // All my loads have landed and my reads of the other tile have returned; behind
+  // the barrier everyone's have.
+  const auto meet = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  fetch(j_begin, s_k0, s_v0);
+  for (int jt = j_begin; jt <= i_hi; jt += 2 * KB) {
+    meet();
+    if (jt + KB <= i_hi) fetch(jt + KB, s_k1, s_v1);
+    attend(jt, s_k0, s_v0);
+    if (jt + KB > i_hi) break;
+    meet();
+    if (jt + 2 * KB <= i_hi) fetch(jt + 2 * KB, s_k0, s_v0);
+    attend(jt + KB, s_k1, s_v1);
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
@@ -709,19 +809,30 @@ static WinArgs win_args(const t5d_window_attention& a, const t5d_ragged& b, int 
   return g;
 }
 
+template <bool SPAN>
+static void launch_rows_tiles(hipStream_t s, WinArgs g) {
+  g.tiles = ((int64_t)g.b.max_len * g.gs + 127) / 128;
+  const int64_t pairs = (int64_t)g.b.S * g.a.G;
+  const dim3 grid((unsigned)((pairs + 7) / 8 * 8 * g.tiles)), block(256);
+#define T5D_ROWS(DT_)                                                              \
+  do {                                                                             \
+    if (g.a.slopes != nullptr || !(g.a.scale > 0.f))                               \
+      hipLaunchKernelGGL((window_rows_kernel<DT_, SPAN, true>), grid, block, 0, s, g); \
+    else                                                                           \
+      hipLaunchKernelGGL((window_rows_kernel<DT_, SPAN, false>), grid, block, 0, s, g); \
+  } while (0)
+  if (g.HP == 32) T5D_ROWS(1);
+  else if (g.HP == 64) T5D_ROWS(2);
+  else if (g.HP == 128) T5D_ROWS(4);
+  else T5D_ROWS(8);
+#undef T5D_ROWS
+}
+
 int launch_window_span(hipStream_t s, const t5d_window_attention& a,
                        const t5d_ragged& b, const t5d_span& span, int ld_kv) {
   WinArgs g = win_args(a, b, t5d_window_head_pad(a.D, a.Dv));
   g.span_off = span.off; g.span_first = span.first; g.ld_kv = ld_kv;
-  const int64_t tiles = ((int64_t)b.max_len * g.gs + 127) / 128;
-  const dim3 grid((unsigned)tiles, b.S, a.G), block(256);
-#define T5D_SPAN(DT_) \
-  hipLaunchKernelGGL((window_rows_kernel<DT_, true>), grid, block, 0, s, g)
-  if (g.HP == 32) T5D_SPAN(1);
-  else if (g.HP == 64) T5D_SPAN(2);
-  else if (g.HP == 128) T5D_SPAN(4);
-  else T5D_SPAN(8);
-#undef T5D_SPAN
+  launch_rows_tiles<true>(s, g);
   T5D_CHECK_LAUNCH("window attention (span)");
   return T5D_OK;
 }
@@ -825,12 +936,7 @@ extern "C" int t5d_window_attention_run(void* stream, const t5d_window_attention
     hipLaunchKernelGGL(window_append_kernel<float>, agrid, ablock, 0, s, g);
   T5D_CHECK_LAUNCH("window attention (append)");
   if (variant == 2 || (variant == 0 && can_rows)) {
-    const int64_t tiles = ((int64_t)b->max_len * g.gs + 127) / 128;
-    const dim3 grid((unsigned)tiles, b->S, a->G), block(256);
-    if (g.HP == 32) hipLaunchKernelGGL(window_rows_kernel<1>, grid, block, 0, s, g);
-    else if (g.HP == 64) hipLaunchKernelGGL(window_rows_kernel<2>, grid, block, 0, s, g);
-    else if (g.HP == 128) hipLaunchKernelGGL(window_rows_kernel<4>, grid, block, 0, s, g);
-    else hipLaunchKernelGGL(window_rows_kernel<8>, grid, block, 0, s, g);
+    launch_rows_tiles<false>(s, g);
     T5D_CHECK_LAUNCH("window attention (rows)");
     return T5D_OK;
   }

@@ -273,6 +273,39 @@ def test_window_attention_step_kernel(H, G, D, Dv, window):
       assert rel(row, wants[s][starts[s] + step]) < 1e-2, (step, s)
 
 
+@pytest.mark.parametrize('H,G,D,scale,bias', [
+    (4, 2, 128, 0.3, False), (4, 2, 64, 0.3, True), (2, 2, 32, -0.4, False),
+    (2, 1, 200, 0.0, False)])
+def test_window_attention_rows_with_scores_that_climb(H, G, D, scale, bias):
+  """The rows kernel raises its running maximum only when a score passes it by a
+  margin: keys whose scores grow by steps below and above it, then fall again,
+  without slopes (both signs of the scale, and none) and with them."""
+  T, portion = 200, 137
+  a = Attention(torch.bfloat16, H, G, D, D, 0, 1, portion, T, seed=D, scale=scale,
+                bias=bias, norms=False)
+  x = a.sequence(T)
+  size = np.concatenate([np.linspace(0.1, 1, 60), np.linspace(1, 12, 80),
+                         np.linspace(12, 0.2, T - 140)])
+  keys = slice(a.off[1], a.off[1] + G * D)
+  x[:, keys] = (x[:, keys].float() * dev(size)[:, None]).to(torch.bfloat16)
+  got = np.concatenate([a.run([(0, 0)], [x[:portion]], 2),
+                        a.run([(0, portion)], [x[portion:]], 2)])
+  assert rel(got, a.oracle(x)) < a.tol
+
+
+def test_window_attention_rows_of_many_tiles():
+  """More tiles than one round of the compute units takes: the portions whose
+  tiles run in the other order, beside short ones."""
+  lens = [3, 64, 1, 70, 1100]
+  a = Attention(torch.bfloat16, 8, 2, 32, 32, 300, 5, 1100, 1100)
+  seqs = [a.sequence(n) for n in lens]
+  got = a.run([(s, 0) for s in range(5)], seqs, 2)
+  at = 0
+  for x in seqs:
+    assert rel(got[at:at + len(x)], a.oracle(x)) < a.tol, len(x)
+    at += len(x)
+
+
 @pytest.mark.parametrize('bias,sink,norms', [(False, True, True),
                                              (True, False, True),
                                              (True, True, False)])
