@@ -3,18 +3,15 @@
 // (batch item, head), t5x/examples/t5/layers.py:52-129 with the encoder's
 // bidirectional bias (layers.py:560-677) and mask (network.py:325-328).
 //
-// A workgroup takes 64 queries of one (item, head), a wavefront 16 of them.
-// Two passes over the keys, 16 at a time, both on the matrix cores:
-//   pass 1: S^T = K Q^T (keys as MFMA rows, so a lane ends up with 4
-//           consecutive keys of ONE query), scores rounded where the reference
-//           rounds them, running max / sum per lane, combined at the end;
-//   pass 2: S^T again, P = bf16(exp(s - max) / sum) written 4 keys at a time
-//           into a small LDS tile, read back as the B operand of
-//           out^T = V^T P^T, 32 keys per step.  V is given transposed in
-//           32-key blocks ([B, H, Ep / 32, 64, 32], what t5d_gemm_rows' value
-//           layout writes), so a fragment is one contiguous 1 KB.
-// Masked keys get the reference's -1e10 (so a padded query attends uniformly,
-// as it does there); keys beyond E do not exist and get -inf.
+// Two kernels on the matrix cores, chosen by length: enc_attn_ring_kernel up to 128
+// positions (64 queries per workgroup, scores kept in registers between a pass over
+// the keys and one over the values), enc_attn_tile_kernel beyond (128 queries, one
+// pass).  Both form S^T = K Q^T, keys as matrix rows, so that a lane ends up with 4
+// consecutive keys of ONE query, which is the operand order of out^T = V^T P^T; V is
+// given transposed in 32-key blocks ([B, H, Ep / 32, 64, 32], what t5d_gemm_rows'
+// value layout writes).  Scores are rounded where the reference rounds them.
+// Masked keys weigh nothing beside a valid one, and a padded query attends uniformly
+// over all keys, as with the reference's -1e10; keys beyond E do not exist.
 #include <math.h>
 
 #include "common.h"
@@ -37,207 +34,15 @@ struct EncAttnArgs {
   const int32_t* len; // [B] valid prefix length (with `valid`: last valid + 1)
   const uint32_t* valid;  // optional [B, (E + 31) / 32]: bit e = position e valid
   bf16_t* out;        // [B*E, H*64]
-  int H, E, Ep, q_stride, k_stride;
+  int B, H, E, Ep, q_stride, k_stride;
 };
 
 constexpr int kMaxEncLen = 2048;
 
-__global__ void __launch_bounds__(256)
-enc_attn_kernel(EncAttnArgs a) {
-  __shared__ __attribute__((aligned(16))) bf16_t s_p[4][16][32];
-  __shared__ float s_bias[2 * kMaxEncLen];  // this head's bias by distance
-  __shared__ uint32_t s_valid[kMaxEncLen / 32];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int l16 = lane & 15, gq = lane >> 4;
-  const int h = blockIdx.y, b = blockIdx.z;
-  const int q0 = blockIdx.x * 64 + wave * 16;
-  const int E = a.E;
-  for (int i = threadIdx.x; i < 2 * E - 1; i += 256)
-    s_bias[i] = bf16_to_f32(a.bias[(size_t)h * (2 * E - 1) + i]);
-  int n = a.len[b];
-  n = n < 0 ? 0 : (n > E ? E : n);
-  // Which positions are valid: the prefix [0, n), or the caller's bits (a
-  // padding token inside the text: encoder_input_tokens > 0 element-wise).
-  const int words = (E + 31) >> 5;
-  for (int i = threadIdx.x; i < words; i += 256) {
-    const int left = n - 32 * i;
-    const uint32_t prefix =
-        left >= 32 ? 0xffffffffu : (left <= 0 ? 0u : ((1u << left) - 1u));
-    s_valid[i] = a.valid ? (a.valid[(size_t)b * words + i] & prefix) : prefix;
-  }
-  __syncthreads();
-  if (q0 >= E) return;
-  auto is_valid = [&](int pos) {
-    return pos < E && ((s_valid[pos >> 5] >> (pos & 31)) & 1u) != 0;
-  };
-  const float kMasked = -9999220736.0f;  // bf16(-1e10) exactly, layers.py:309-311
-  const size_t row0 = (size_t)b * E;
-
-  // B operand of S^T: lane (col = query l16, g) holds Q[q][32c + 8g .. +8]
-  const int qi = min(q0 + l16, E - 1);
-  FragE qb[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-    qb[c].u = *reinterpret_cast<const uint4*>(
-        a.q + (row0 + qi) * a.q_stride + h * 64 + 32 * c + 8 * gq);
-  const bool q_valid = is_valid(q0 + l16);
-  const float* bias_row = s_bias + (E - 1) - qi;
-
-  // Keys past the valid length get -1e10, whose exp underflows to exactly 0
-  // next to any valid key: when all 16 queries of this wavefront are valid,
-  // the key tiles that hold only padding are skipped.  (A padded query attends
-  // uniformly over ALL keys, so a wavefront with one walks them all.)
-  const bool all_valid =
-      q0 + 15 < E &&
-      ((s_valid[q0 >> 5] >> (q0 & 31)) & 0xffffu) == 0xffffu;  // q0 % 16 == 0
-  const int n_tiles = all_valid ? (n + 15) >> 4 : (E + 15) >> 4;
-
-  // K tile kt as the A operand: lane (row = key l16, g) holds K[key][32c + 8g .. +8].
-  // It is fetched with four neighbouring lanes on 64 contiguous bytes of one key
-  // (16 requests per instruction instead of 64: this kernel walks every key
-  // tile twice, and fetched in operand order the L1's tag lookups bound it) and
-  // moved to operand order by `operand_k` when it is consumed.
-  const OperandLanes ol(lane);
-  auto load_k = [&](int kt, FragE (&ka)[2]) {
-    const int key_row = min(16 * kt + ol.ld_row, E - 1);
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-      ka[c].u = *reinterpret_cast<const uint4*>(
-          a.k + (row0 + key_row) * a.k_stride + h * 64 + 32 * c + 8 * ol.ld_piece);
-  };
-  // scores of key tile kt for this lane: keys 16 kt + 4 g + i of query l16
-  auto score_tile = [&](int kt, const FragE (&ka)[2], float (&s)[4]) {
-    f32x4_e acc = (f32x4_e){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      FragE kop;
-      kop.u = ol.to_operand(ka[c].u);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop.v, qb[c].v, acc, 0, 0, 0);
-    }
-    // validity of the tile's 16 keys: one (broadcast) LDS word, which holds
-    // the prefix when the caller gave no bits.  Deliberately without a branch
-    // on a.valid here: with one between the matrix instructions above and the
-    // first read of their result, the compiler's wait-state count followed
-    // the fall-through side only and the taken side read the accumulator 6
-    // issue slots after the v_mfma (9 are needed; at 4 a stale value comes
-    // back).
-    const uint32_t tile_bits = (s_valid[kt >> 1] >> ((kt & 1) * 16)) & 0xffffu;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int key = 16 * kt + 4 * gq + i;
-      float x = round_bf16(acc[i]);
-      if (key < E) {
-        const bool ok = q_valid && ((tile_bits >> (4 * gq + i)) & 1u) != 0;
-        x = ok ? round_bf16(x + bias_row[key]) : kMasked;
-      } else {
-        x = -INFINITY;
-      }
-      s[i] = x;
-    }
-  };
-
-  // The running maximum starts at a finite floor: a lane whose 4 keys of the
-  // first tile all lie beyond E (E < 16) has only -inf scores, and
-  // exp(-inf - (-inf)) would poison its sum.
-  float m = -3.0e38f, l = 0.f;
-  {
-    FragE kcur[2], knext[2];
-    load_k(0, kcur);
-    for (int kt = 0; kt < n_tiles; ++kt) {
-      if (kt + 1 < n_tiles) load_k(kt + 1, knext);  // in flight during this tile
-      float s[4];
-      score_tile(kt, kcur, s);
-      const float tm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-      const float nm = fmaxf(m, tm);
-      float add = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) add += __expf(s[i] - nm);
-      l = l * __expf(m - nm) + add;  // exp(-inf - finite) == 0 on the first tile
-      m = nm;
-      kcur[0] = knext[0];
-      kcur[1] = knext[1];
-    }
-  }
-  // combine the 4 lanes (g) that share a query
-#pragma unroll
-  for (int o = 16; o <= 32; o <<= 1) {
-    const float om = __shfl_xor(m, o, 64), ol = __shfl_xor(l, o, 64);
-    const float nm = fmaxf(m, om);
-    l = l * __expf(m - nm) + ol * __expf(om - nm);
-    m = nm;
-  }
-  const float inv = 1.0f / l;
-
-  f32x4_e oc[4];
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt) oc[dt] = (f32x4_e){0.f, 0.f, 0.f, 0.f};
-  const bf16_t* vbase = a.vt + ((size_t)b * a.H + h) * 64 * (size_t)a.Ep;
-  // V^T fragments of a 32-key step: lane (row = d l16, g) holds
-  // V^T[16 dt + l16][32 (kb / 2) + 8 g .. +8], 1 KB contiguous per fragment
-  auto load_v = [&](int kb, FragE (&va)[4]) {  // kb even: block kb / 2
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-      va[dt].u = *reinterpret_cast<const uint4*>(
-          vbase + ((size_t)(kb >> 1) * 64 + 16 * dt + l16) * 32 + 8 * gq);
-  };
-  FragE kcur[2][2], knext[2][2], vcur[4], vnext[4];
-  load_k(0, kcur[0]);
-  if (1 < n_tiles) load_k(1, kcur[1]);
-  load_v(0, vcur);
-  for (int kb = 0; kb < n_tiles; kb += 2) {  // 32 keys per step
-    if (kb + 2 < n_tiles) {
-      load_k(kb + 2, knext[0]);
-      if (kb + 3 < n_tiles) load_k(kb + 3, knext[1]);
-      load_v(kb + 2, vnext);
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      float s[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-      if (kb + t < n_tiles) score_tile(kb + t, kcur[t], s);
-      uint2 pk;
-      pk.x = pack_bf16x2(__expf(s[0] - m) * inv, __expf(s[1] - m) * inv);
-      pk.y = pack_bf16x2(__expf(s[2] - m) * inv, __expf(s[3] - m) * inv);
-      *reinterpret_cast<uint2*>(&s_p[wave][l16][16 * t + 4 * gq]) = pk;
-    }
-    // LDS traffic stays inside the wavefront: its own writes are visible to it
-    // once they have completed.
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-    FragE pb;  // B: lane (col = query l16, g) holds P[q][8g .. +8] of the 32
-    pb.u = *reinterpret_cast<const uint4*>(&s_p[wave][l16][8 * gq]);
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-      oc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vcur[dt].v, pb.v, oc[dt],
-                                                       0, 0, 0);
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      kcur[t][0] = knext[t][0];
-      kcur[t][1] = knext[t][1];
-    }
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) vcur[dt] = vnext[dt];
-  }
-  // oc[dt][i]: out[q = l16][d = 16 dt + 4 g + i]
-  if (q0 + l16 < E) {
-    bf16_t* o = a.out + (row0 + q0 + l16) * (size_t)(a.H * 64) + h * 64 + 4 * gq;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      uint2 pk;
-      pk.x = pack_bf16x2(oc[dt][0], oc[dt][1]);
-      pk.y = pack_bf16x2(oc[dt][2], oc[dt][3]);
-      *reinterpret_cast<uint2*>(o + 16 * dt) = pk;
-    }
-  }
-}
-
-// ---- the same attention for E <= 512, scores kept in registers ---------------
-// enc_attn_kernel walks the keys twice and forms every score twice, each
-// wavefront fetching K and V for itself.  For encoder lengths up to 512 the 16
-// x E scores of a wavefront fit its registers as bfloat16 pairs (they ARE
-// bfloat16 values at that point), so here
-//   pass 1 forms the scores once, keeps them, and tracks max / sum as before;
+// ---- up to 128 positions: scores kept in registers ------------------------------
+// The 16 x E scores of a wavefront fit its registers as bfloat16 pairs (they ARE
+// bfloat16 values at that point), so
+//   pass 1 forms the scores once, keeps them, and tracks max / sum;
 //   pass 2 turns the kept scores into P in registers, already in the layout
 //          of the matrix cores' B operand: a lane holds keys 4g .. 4g+3 of two
 //          neighbouring 16-key tiles, and the V^T operand is read from LDS in
@@ -250,10 +55,6 @@ enc_attn_kernel(EncAttnArgs a) {
 // fragments from there.  One barrier per 64 keys, placed by hand with the wait
 // for "all but my newest two loads"; the stages are separate arrays and the
 // loops are unrolled so that every stage is named at compile time.
-// Scores, maxima, sums and probabilities have the bits of enc_attn_kernel's;
-// the products of a 32-key step enter the matrix instruction in another key
-// order, so an output can differ from enc_attn_kernel's in its last bit (1
-// in 4000 measured).
 typedef __attribute__((address_space(3))) void* enc_lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* enc_glb_ptr_t;
 
@@ -293,7 +94,7 @@ enc_attn_ring_kernel(EncAttnArgs a) {
     s_lim[1][i] = i < E ? kMasked : -INFINITY;
   }
   __syncthreads();
-  // Key tiles each wavefront walks (as in enc_attn_kernel: the valid prefix
+  // Key tiles each wavefront walks (the valid prefix
   // when all of its 16 queries are valid — the keys beyond add exact zeros —
   // else every key; none when its queries lie beyond E) and what the
   // workgroup as a whole must fetch, in 64-key blocks.
@@ -515,6 +316,318 @@ enc_attn_ring_kernel(EncAttnArgs a) {
   }
 }
 
+// ---- beyond 128 positions: one pass ----------------------------------------------
+// A workgroup takes 128 queries of one (item, head), a wavefront 32, and walks 64
+// keys at a time once: scores as above (rounded where the reference rounds them),
+// weights relative to a running maximum that is raised only when a score passes it
+// by kMaxSlack powers of two, rounded to bfloat16 as they enter the second product
+// and divided by their float32 sum at the end.  K and V^T tiles go from memory
+// straight into LDS, one tile ahead in a second pair of buffers, one barrier per
+// tile; 16-byte pieces are exchanged within a row (XOR) so that operand reads cover
+// all banks.  A masked key is left out (-inf: next to a valid one its weight is an
+// exact zero) and a padded query scores 0 with every key that exists (it attends
+// uniformly), both in tiles that hold one of the two only; a wavefront of padded
+// queries alone forms no scores.
+// What bounds it: ~260 vector instructions per tile and wavefront (the two roundings
+// of a score, its exponential) against 32 matrix instructions; 49 KB of LDS and 164
+// registers let three workgroups share a CU.  Measured beside the kernels that were
+// here before (two passes over the keys; up to 512 positions the one above with 8
+// blocks of 64): 7 x 16 heads x 1032 (400 and more valid) 203 -> 82 us, 2 x 16 x 2048
+// 243 -> 82, 64 x 16 x 512 (all valid) 261 -> 159, 32 x 12 x 512 (128 and more) 98 ->
+// 66, 64 x 16 x 300 95 -> 73, 64 x 12 x 132 32 -> 31; at 64 positions the one above is
+// the better one (256 x 12: 24 against 28 us), at 16 by far (512 x 12: 26 / 40), as
+// half or more of a 128-query tile is then empty.
+constexpr float kMaxSlack = 8.0f;
+constexpr float kLog2eE = 1.4426950408889634f;
+
+__global__ void __launch_bounds__(256, 3)
+enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
+  constexpr int MT = 2, KB = 64;
+  __shared__ uint4 s_k0[512], s_v0[512], s_k1[512], s_v1[512];
+  // from 16 entries before the table (queries past the end) to 64 behind it (keys
+  // past the end): neither's scores are used
+  __shared__ float s_bias[16 + 2 * kMaxEncLen + 64];
+  __shared__ uint32_t s_valid[kMaxEncLen / 32 + 2];
+  // consecutive block ids go round-robin over the 8 XCDs: the tiles of one (item,
+  // head) are 8 apart
+  const int pair = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / tiles);
+  const int b = pair / a.H, h = pair - b * a.H;
+  if (b >= a.B) return;
+  const int tile = (blockIdx.x >> 3) % tiles;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, gq = lane >> 4;
+  const int E = a.E;
+  const size_t row0 = (size_t)b * E;
+
+  // the pieces this lane fetches: keys (rows of 128 bytes, clamped at the last),
+  // V^T (blocks of 32 keys: rows of 64 bytes)
+  const char* k_at = reinterpret_cast<const char*>(a.k) + (size_t)h * 128;
+  const char* v_at = reinterpret_cast<const char*>(a.vt) +
+                     ((size_t)b * a.H + h) * 128 * (size_t)a.Ep;
+  int k_row[2], k_piece[2], v_blk[2], v_off[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int f = (wave * 2 + i) * 64 + lane;
+    k_row[i] = f >> 3;
+    k_piece[i] = 16 * ((f & 7) ^ ((k_row[i] >> 1) & 7));
+    v_blk[i] = f >> 8;
+    const int d = (f >> 2) & 63;
+    v_off[i] = d * 64 + 16 * ((f & 3) ^ ((d >> 2) & 3));
+  }
+  const auto fetch = [&](int jt, uint4* sk, uint4* sv) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const size_t row = row0 + min(jt + k_row[i], E - 1);
+      __builtin_amdgcn_global_load_lds(
+          (enc_glb_ptr_t)(k_at + row * a.k_stride * 2 + k_piece[i]),
+          (enc_lds_ptr_t)(sk + (wave * 2 + i) * 64), 16, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int blk = min((jt >> 5) + v_blk[i], (a.Ep >> 5) - 1);
+      __builtin_amdgcn_global_load_lds(
+          (enc_glb_ptr_t)(v_at + (size_t)blk * 4096 + v_off[i]),
+          (enc_lds_ptr_t)(sv + (wave * 2 + i) * 64), 16, 0, 0);
+    }
+  };
+  fetch(0, s_k0, s_v0);
+
+  for (int i = threadIdx.x; i < 2 * E - 1; i += 256)
+    s_bias[16 + i] = bf16_to_f32(a.bias[(size_t)h * (2 * E - 1) + i]);
+  int n = a.len[b];
+  n = n < 0 ? 0 : (n > E ? E : n);
+  const int words = (E + 31) >> 5;
+  for (int i = threadIdx.x; i < kMaxEncLen / 32 + 2; i += 256) {
+    const int left = n - 32 * i;
+    uint32_t prefix =
+        left >= 32 ? 0xffffffffu : (left <= 0 ? 0u : ((1u << left) - 1u));
+    if (a.valid && i < words) prefix &= a.valid[(size_t)b * words + i];
+    s_valid[i] = prefix;
+  }
+  const int q0 = tile * 128 + wave * 32;
+  FragE qb[MT][2];
+  int qi[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    qi[mt] = min(q0 + 16 * mt + l16, E - 1);  // past the end: not stored
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      qb[mt][c].u = *reinterpret_cast<const uint4*>(
+          a.q + (row0 + qi[mt]) * a.q_stride + h * 64 + 32 * c + 8 * gq);
+  }
+  __syncthreads();
+  // Keys each wavefront of the workgroup walks: the valid prefix if all of its
+  // queries are valid, else all there are (none past the end).
+  int my_keys = 0, wg_keys = 0;
+  bool my_valid = false, my_padding = false;  // all queries are
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const int qw = tile * 128 + w * 32;
+    const uint32_t want = qw + 32 <= E ? 0xffffffffu : qw < E ? (1u << (E - qw)) - 1 : 0;
+    const bool valid = qw < E && (s_valid[qw >> 5] & want) == want;
+    const int keys = qw >= E ? 0 : valid ? n : E;
+    if (w == wave) {
+      my_keys = keys;
+      my_valid = valid;
+      my_padding = qw >= E || (s_valid[qw >> 5] & want) == 0;
+    }
+    wg_keys = max(wg_keys, keys);
+  }
+  my_keys = __builtin_amdgcn_readfirstlane(my_keys);
+  wg_keys = __builtin_amdgcn_readfirstlane(wg_keys);
+
+  float mx[MT], l[MT];
+  f32x4_e oc[4][MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    mx[mt] = -1e30f;
+    l[mt] = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) oc[dt][mt] = (f32x4_e){0.f, 0.f, 0.f, 0.f};
+  }
+  const int k_read = l16 * 8, k_x = (l16 >> 1) & 7;
+  const int v_read = l16 * 64 + 16 * ((gq >> 1) ^ ((l16 >> 2) & 3)) + 8 * (gq & 1);
+  const auto attend = [&](int jt, const uint4* sk, const uint4* sv) {
+    if (jt >= my_keys) return;
+    FragE pb[2][MT];
+    if (my_padding) {
+      // every key that exists weighs the same: no scores
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        uint32_t w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = jt + 32 * kb + 16 * (e >> 1) + 4 * gq + 2 * (e & 1);
+          w[e] = (key < E ? 0x3F80u : 0u) | (key + 1 < E ? 0x3F800000u : 0u);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+            l[mt] += (float)((key < E) + (key + 1 < E));
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          pb[kb][mt].u = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+    } else {
+    f32x4_e s[4][MT];
+    FragE kf[4][2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        kf[t][c].u = sk[16 * t * 8 + k_read + ((4 * c + gq) ^ k_x)];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) s[t][mt] = (f32x4_e){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          s[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][c].v, qb[mt][c].v,
+                                                             s[t][mt], 0, 0, 0);
+    // bias by key - query: 16 keys further on is 16 queries further back
+    const float* near = s_bias + 16 + (E - 1) - qi[0] + jt + 4 * gq;
+    float bias[5][4];
+#pragma unroll
+    for (int t = 0; t < 5; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        bias[t][i] = near[16 * (t - 1) + i];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const float* add = bias[t - mt + 1];
+        const uint32_t r01 = pack_bf16x2(s[t][mt][0], s[t][mt][1]);
+        const uint32_t r23 = pack_bf16x2(s[t][mt][2], s[t][mt][3]);
+        const uint32_t x01 =
+            pack_bf16x2(bf16lo_to_f32(r01) + add[0], bf16hi_to_f32(r01) + add[1]);
+        const uint32_t x23 =
+            pack_bf16x2(bf16lo_to_f32(r23) + add[2], bf16hi_to_f32(r23) + add[3]);
+        s[t][mt][0] = bf16lo_to_f32(x01);
+        s[t][mt][1] = bf16hi_to_f32(x01);
+        s[t][mt][2] = bf16lo_to_f32(x23);
+        s[t][mt][3] = bf16hi_to_f32(x23);
+      }
+    const uint32_t v0 = s_valid[jt >> 5], v1 = s_valid[(jt >> 5) + 1];
+    if (!my_valid || (v0 & v1) != 0xffffffffu) {
+      asm volatile("");  // (a branch: the compiler would select in every tile)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const bool q_valid = (s_valid[qi[mt] >> 5] >> (qi[mt] & 31)) & 1u;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int key = 16 * t + 4 * gq + i;
+            const bool exists = jt + key < E;
+            const bool ok = ((t < 2 ? v0 : v1) >> (key & 31)) & 1u;
+            const float x = q_valid ? s[t][mt][i] : 0.f;
+            s[t][mt][i] = (q_valid ? ok : exists) ? x : -INFINITY;
+          }
+      }
+    }
+    bool raise = false;
+    float top[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      top[mt] = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) top[mt] = fmaxf(top[mt], s[t][mt][i]);
+      top[mt] = rows_max(top[mt]) * kLog2eE;
+      raise |= top[mt] > mx[mt] + kMaxSlack;
+    }
+    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+      asm volatile("");
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const float to = fmaxf(mx[mt], top[mt]);
+        const float alpha = __builtin_amdgcn_exp2f(mx[mt] - to);
+        mx[mt] = to;
+        l[mt] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) oc[dt][mt][i] *= alpha;
+      }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(s[t][mt][i], kLog2eE, -mx[mt]));
+          s[t][mt][i] = p;
+          sum += p;
+        }
+      l[mt] += sum;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        pb[kb][mt].u = make_uint4(pack_bf16x2(s[2 * kb][mt][0], s[2 * kb][mt][1]),
+                                  pack_bf16x2(s[2 * kb][mt][2], s[2 * kb][mt][3]),
+                                  pack_bf16x2(s[2 * kb + 1][mt][0], s[2 * kb + 1][mt][1]),
+                                  pack_bf16x2(s[2 * kb + 1][mt][2], s[2 * kb + 1][mt][3]));
+    }
+    }
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      FragE va[4];
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const char* v = reinterpret_cast<const char*>(sv) + kb * 4096 + dt * 1024;
+        const uint2 x = *reinterpret_cast<const uint2*>(v + v_read);
+        const uint2 y = *reinterpret_cast<const uint2*>(v + (v_read ^ 32));
+        va[dt].u = make_uint4(x.x, x.y, y.x, y.y);
+      }
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          oc[dt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              va[dt].v, pb[kb][mt].v, oc[dt][mt], 0, 0, 0);
+    }
+  };
+  // All my loads have landed and my reads of the other tile have returned; behind
+  // the barrier everyone's have.
+  const auto meet = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int jt = 0; jt < wg_keys; jt += 2 * KB) {
+    meet();
+    if (jt + KB < wg_keys) fetch(jt + KB, s_k1, s_v1);
+    attend(jt, s_k0, s_v0);
+    if (jt + KB >= wg_keys) break;
+    meet();
+    if (jt + 2 * KB < wg_keys) fetch(jt + 2 * KB, s_k0, s_v0);
+    attend(jt + KB, s_k1, s_v1);
+  }
+  // (a workgroup without keys has loads of the first tile under way)
+  __builtin_amdgcn_s_waitcnt(0x0070);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const float inv = 1.0f / rows_sum(l[mt]);
+    const int q = q0 + 16 * mt + l16;
+    if (q >= E) continue;
+    bf16_t* o = a.out + (row0 + q) * (size_t)(a.H * 64) + h * 64 + 4 * gq;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+      *reinterpret_cast<uint2*>(o + 16 * dt) =
+          make_uint2(pack_bf16x2(oc[dt][mt][0] * inv, oc[dt][mt][1] * inv),
+                     pack_bf16x2(oc[dt][mt][2] * inv, oc[dt][mt][3] * inv));
+  }
+}
+
 // ---- float32 -------------------------------------------------------------------
 // The exactness-test dtype: plain vector arithmetic, one wavefront per query
 // row.  Scores (lane = key, ascending head dim), bias and mask summed first and
@@ -613,8 +726,8 @@ extern "C" int t5d_encoder_attention_variant(
     int variant) {
   T5D_REQUIRE(variant >= 0 && variant <= 2 && (variant != 2 || E <= 512),
               T5D_EINVAL,
-              "t5d_encoder_attention_variant: variant %d (0 chosen here, 1 "
-              "scores formed twice, 2 scores kept in registers: E <= 512)",
+              "t5d_encoder_attention_variant: variant %d (0, 1, and 2 where "
+              "E <= 512)",
               variant);
   T5D_REQUIRE(q && k && v_t && rel_bias && enc_len && out, T5D_EINVAL,
               "t5d_encoder_attention: null pointer");
@@ -630,27 +743,25 @@ extern "C" int t5d_encoder_attention_variant(
               T5D_EINVAL, "t5d_encoder_attention: operand alignment");
   T5D_REQUIRE(E <= kMaxEncLen, T5D_ELIMIT,
               "t5d_encoder_attention: E=%d beyond %d", E, kMaxEncLen);
-  T5D_REQUIRE(H <= 65535 && B <= 65535, T5D_ELIMIT,
-              "t5d_encoder_attention: H=%d B=%d beyond the launch grid", H, B);
+  T5D_REQUIRE(H <= 65535 && B <= 65535 &&
+                  (E <= 128 ||
+                   ((int64_t)B * H + 7) * ((E + 127) / 128) < (1LL << 31)),
+              T5D_ELIMIT, "t5d_encoder_attention: H=%d B=%d beyond the launch grid",
+              H, B);
   EncAttnArgs a;
   a.q = (const bf16_t*)q; a.k = (const bf16_t*)k; a.vt = (const bf16_t*)v_t;
   a.bias = (const bf16_t*)rel_bias; a.len = enc_len; a.out = (bf16_t*)out;
   a.valid = valid_bits;
-  a.H = H; a.E = E; a.Ep = Ep; a.q_stride = q_stride; a.k_stride = k_stride;
-  dim3 grid((E + 63) / 64, H, B), block(256);
-  if (variant == 1)
-    hipLaunchKernelGGL(enc_attn_kernel, grid, block, 0, as_stream(stream), a);
-  else if (E <= 128)
-    hipLaunchKernelGGL(enc_attn_ring_kernel<2>, grid, block, 0,
-                       as_stream(stream), a);
-  else if (E <= 256)
-    hipLaunchKernelGGL(enc_attn_ring_kernel<4>, grid, block, 0,
-                       as_stream(stream), a);
-  else if (E <= 512)
-    hipLaunchKernelGGL(enc_attn_ring_kernel<8>, grid, block, 0,
-                       as_stream(stream), a);
-  else
-    hipLaunchKernelGGL(enc_attn_kernel, grid, block, 0, as_stream(stream), a);
+  a.B = B; a.H = H; a.E = E; a.Ep = Ep; a.q_stride = q_stride; a.k_stride = k_stride;
+  if (E <= 128) {
+    hipLaunchKernelGGL(enc_attn_ring_kernel<2>, dim3((E + 63) / 64, H, B), dim3(256),
+                       0, as_stream(stream), a);
+  } else {
+    const int tiles = (E + 127) / 128;
+    const unsigned groups = ((unsigned)B * H + 7) / 8 * 8 * tiles;
+    hipLaunchKernelGGL(enc_attn_tile_kernel, dim3(groups), dim3(256), 0,
+                       as_stream(stream), a, tiles);
+  }
   T5D_CHECK_LAUNCH("t5d_encoder_attention");
   return T5D_OK;
 }

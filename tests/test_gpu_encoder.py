@@ -224,6 +224,39 @@ def test_encoder_attention(ops, B, E, H):
   np.testing.assert_allclose(got, want, atol=2e-2, rtol=2**-6)
 
 
+@pytest.mark.parametrize('E', [128, 129, 159, 160, 192, 193, 257, 513])
+def test_encoder_attention_at_the_edges_of_its_tiles(ops, E):
+  """Lengths around 32 (a wavefront's queries, a block of values), 64 (a tile of
+  keys) and 128 (a workgroup's queries), and items whose valid part ends at and
+  around those edges, with every query of a wavefront valid, none, and some; in
+  one item a padding token inside the text.  Scores climb along the keys, so the
+  running maximum is raised again and again."""
+  from t5x_amd import network
+  H, lens = 2, np.array([E, 1, 32, 33, 64, 65, 96, 127], np.int32)
+  B = len(lens)
+  rs = np.random.RandomState(E)
+  bf = lambda x: ot5.bf16_round(x.astype(np.float32))
+  q = bf(0.2 + rs.randn(B, E, H, 64) * 0.125)
+  k = bf(rs.randn(B, E, H, 64) + np.linspace(-1, 2, E)[None, :, None, None])
+  v = bf(rs.randn(B, E, H, 64))
+  rel_emb = rs.randn(H, 32).astype(np.float32)
+  valid = np.arange(E)[None, :] < lens[:, None]
+  valid[0, E // 2] = False
+  want = _enc_attn_oracle(q, k, v, rel_emb, None, valid)
+  bucket = network.relative_position_bucket(np.arange(-(E - 1), E),
+                                            bidirectional=True)
+  rel_bias = dev(ot5.bf16_round(rel_emb)[:, bucket], torch.bfloat16).contiguous()
+  v_t = torch.zeros((B, H, 64, (E + 31) // 32 * 32), dtype=torch.bfloat16,
+                    device='cuda')
+  v_t[..., :E] = dev(v, torch.bfloat16).permute(0, 2, 3, 1)
+  out = ops.encoder_attention(
+      *(dev(x, torch.bfloat16).reshape(B * E, H * 64) for x in (q, k)),
+      ops.tile_cross_value(v_t), rel_bias, dev(lens),
+      valid_bits=ops.pack_valid_bits(dev(valid)))
+  np.testing.assert_allclose(host(out).reshape(B, E, H, 64), want, atol=2e-2,
+                             rtol=2**-6)
+
+
 def test_encoder_attention_repeated_launches(ops):
   """30 launches of the attention kernel for lengths up to 512 (K and V go
   through a ring of LDS stages behind hand-placed barriers) at 8 x 12 heads x
