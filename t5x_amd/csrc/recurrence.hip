@@ -58,6 +58,25 @@ __device__ __forceinline__ float log_decay(const t5d_recurrence& a, float z, int
   return -expf(a.A_log[h]) * softplus_f(z);
 }
 
+// The same for the chunk kernel, which spent most of its instructions on them:
+// quotients as a reciprocal and one step of Newton (within an ulp, as the division),
+// log2(1 + e^z) with what rounding took from 1 + e added back to first order.
+__device__ __forceinline__ float reciprocal_f(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return x > 1e30f ? r : fmaf(fmaf(-x, r, 1.0f), r, r);  // (infinity: 0)
+}
+__device__ __forceinline__ float sigmoid_quick(float z) {
+  return reciprocal_f(1.0f + exp_f(-z));
+}
+__device__ __forceinline__ float softplus_log2(float z) {
+  constexpr float kLog2e = 1.4426950408889634f;
+  const float e = __builtin_amdgcn_exp2f(-kLog2e * fabsf(z));
+  const float u = 1.0f + e;
+  const float lost = (e - (u - 1.0f)) * kLog2e;
+  const float l = fmaf(lost, __builtin_amdgcn_rcpf(u), __builtin_amdgcn_logf(u));
+  return fmaf(fmaxf(z, 0.0f), kLog2e, l);
+}
+
 // One channel of q, k or v of the token at row m: the projection itself, or its
 // causal convolution and silu.  `first`: row of the portion's first token; cc:
 // channel of the convolution; x: value at row m.
@@ -273,50 +292,108 @@ struct ChunkLayout {
   __host__ __device__ size_t size() const { return pc() + dp; }
 };
 
-// 16 tokens of one projection column, through the convolution and silu if there
-// is one (TM: at least its taps).  i0: the chunk's first token within the portion.
-template <int TM, typename T>
-__device__ __forceinline__ void chunk_column(const RecArgs& g, int m0, int n, int i0,
-                                             int pos0, int slot, int col, int cc,
-                                             float (&y)[kChunk]) {
+// The chunk's columns of q, k, the decay and v, one per thread and 512 per round, into
+// LDS: q, k and v through the convolution and silu if there is one (TM: at least its
+// taps).  Two columns of a thread are requested before either is used, and rows past
+// the end are the last one again (no branches between the loads); such tokens have no
+// key, no query, no value and no decay.  chunk, n: which chunk, its tokens.
+template <int TM, int DP, typename T>
+__device__ __forceinline__ void chunk_columns(const RecArgs& g, int chunk, int n, int m0,
+                                              int h, int seq, float* s_q, float* s_k,
+                                              float* s_g, float* s_v, int vp, int vs) {
+  constexpr int C = kChunk, LS = DP + 4, N = TM > 0 ? TM : 1;
   const t5d_recurrence& a = g.a;
-  const T* p = reinterpret_cast<const T*>(a.proj) + (size_t)m0 * a.ld_proj + col;
-  float x[kChunk];
+  const int tid = threadIdx.x, hg = h / (a.H / a.G);
+  const int slot = g.b.seq_slot[seq], pos0 = g.b.seq_start[seq] + chunk * C;
+  const bool power = a.decay == T5D_DECAY_SIGMOID_POWER;
+  const float rate = power ? a.decay_power : expf(a.A_log[h]);
+  struct Column {
+    int kind, c;        // 0 q, 1 k, 2 decay, 3 v; column within it
+    float x[C];
+    float w[N], before[N];  // before[j]: the value j tokens before the chunk
+  };
+  const auto load = [&](Column& y, int u) {
+    y.kind = min(__builtin_amdgcn_readfirstlane(u) / DP, 3);  // (DP % 64 == 0)
+    y.c = u - y.kind * DP;
+    const int c = y.c < (y.kind == 3 ? a.Dv : a.D) ? y.c : 0;
+    if (y.kind == 2) {
+      const float* z = a.low + (size_t)m0 * a.ld_low + a.off_z + (size_t)h * a.D + c;
 #pragma unroll
-  for (int t = 0; t < kChunk; ++t)
-    x[t] = t < n ? to_f32<T>(p[(size_t)t * a.ld_proj]) : 0.f;
-  if constexpr (TM == 0) {
-#pragma unroll
-    for (int t = 0; t < kChunk; ++t) y[t] = x[t];
-    return;
-  }
-  constexpr int N = TM > 0 ? TM : 1;
-  float w[N], before[N];  // before[j]: the value j tokens before the chunk
-  const T* ring = reinterpret_cast<const T*>(a.conv_ring) +
-                  (size_t)slot * a.taps * g.C + cc;
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    w[j] = j < a.taps ? a.conv[(size_t)cc * a.taps + a.taps - 1 - j] : 0.f;
-    before[j] = 0.f;
-    if (j > 0 && j < a.taps) {
-      if (i0 >= j)
-        before[j] = to_f32<T>(p[-(ptrdiff_t)j * a.ld_proj]);
-      else if (pos0 >= j)
-        before[j] = to_f32<T>(ring[(size_t)((pos0 - j) % a.taps) * g.C]);
+      for (int t = 0; t < C; ++t) y.x[t] = z[(size_t)min(t, n - 1) * a.ld_low];
+      y.w[0] = a.decay_bias[(size_t)h * a.D + c];
+      return;
     }
-  }
+    const int col = (y.kind == 0 ? a.off_q + hg * a.D
+                     : y.kind == 1 ? a.off_k + hg * a.D : a.off_v + h * a.Dv) + c;
+    const int cc = (y.kind == 0 ? hg * a.D
+                    : y.kind == 1 ? (a.G + hg) * a.D : 2 * a.G * a.D + h * a.Dv) + c;
+    const T* p = reinterpret_cast<const T*>(a.proj) + (size_t)m0 * a.ld_proj + col;
 #pragma unroll
-  for (int t = 0; t < kChunk; ++t) {
-    float s = 0.f;
+    for (int t = 0; t < C; ++t) y.x[t] = to_f32<T>(p[(size_t)min(t, n - 1) * a.ld_proj]);
+    if constexpr (TM > 0) {
+      const T* ring = reinterpret_cast<const T*>(a.conv_ring) +
+                      (size_t)slot * a.taps * g.C + cc;
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-      s = fmaf(w[j], t >= j ? x[t >= j ? t - j : 0] : before[t >= j ? 0 : j - t], s);
-    y[t] = s * sigmoid_f(s);
+      for (int j = 0; j < N; ++j) {
+        y.w[j] = j < a.taps ? a.conv[(size_t)cc * a.taps + a.taps - 1 - j] : 0.f;
+        y.before[j] = 0.f;
+        if (j > 0 && j < a.taps) {
+          if (chunk * C >= j)
+            y.before[j] = to_f32<T>(p[-(ptrdiff_t)j * a.ld_proj]);
+          else if (pos0 >= j)
+            y.before[j] = to_f32<T>(ring[(size_t)((pos0 - j) % a.taps) * g.C]);
+        }
+      }
+    }
+  };
+  const auto finish = [&](const Column& y) {
+    float v[C];
+    if (y.kind == 2) {
+      const float sign = power ? -1.f : 1.f;
+#pragma unroll
+      for (int t = 0; t < C; ++t) {  // the exponential of log_decay
+        const float z = sign * (y.x[t] + y.w[0]);
+        v[t] = __builtin_amdgcn_exp2f(-rate * softplus_log2(z));
+      }
+    } else if constexpr (TM > 0) {
+#pragma unroll
+      for (int t = 0; t < C; ++t) {
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          sum = fmaf(y.w[j], t >= j ? y.x[t >= j ? t - j : 0] : y.before[t >= j ? 0 : j - t],
+                     sum);
+        v[t] = sum * sigmoid_quick(sum);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < C; ++t) v[t] = y.x[t];
+    }
+    if (y.c >= (y.kind == 3 ? vp : DP)) return;
+    const bool there = y.c < (y.kind == 3 ? a.Dv : a.D);
+    float* dst = (y.kind == 0 ? s_q : y.kind == 1 ? s_k : y.kind == 2 ? s_g : s_v) + y.c;
+    const int stride = y.kind == 3 ? vs : LS;
+    const float none = y.kind == 2 ? 1.f : 0.f;
+#pragma unroll
+    for (int t = 0; t < C; ++t) dst[t * stride] = there && t < n ? v[t] : none;
+  };
+  for (int u = tid; u < 3 * DP + vp; u += 512) {
+    Column y0, y1;
+    const bool more = __builtin_amdgcn_readfirstlane(u) + 256 < 3 * DP + vp;
+    load(y0, u);
+    if (more) load(y1, u + 256);
+    finish(y0);
+    if (more) finish(y1);
   }
 }
 
 constexpr int kChunkTaps = 8;  // longest convolution of the chunk kernel
 
+// Columns of q, k, v and the decay through convolution, silu and norms; A and B on
+// the vector ALUs, k_s decayed on its way down the chunk; then, with the delta rule,
+// T = (I + diag(beta) A)^-1 diag(beta), 16 x 16, and everything that is applied to
+// whole columns on the matrix cores: Wk = T (k P), Us = T v, and with M = B T
+// Qs = q P - M (k P), Os = M v.
 template <int DP, bool DELTA, typename T>
 __global__ void __launch_bounds__(256, DP <= 128 ? 4 : DP <= 256 ? 2 : 1)
 recurrence_chunk_kernel(RecArgs g) {
@@ -326,62 +403,28 @@ recurrence_chunk_kernel(RecArgs g) {
   __shared__ __align__(16) float s_g[C * LS];
   __shared__ __align__(16) float s_a[C][C];
   __shared__ __align__(16) float s_b[C][C];
+  __shared__ __align__(16) float s_t[C][C];
   __shared__ float s_beta[C];
-  extern __shared__ float s_v[];  // [C][vp]
+  extern __shared__ float s_v[];  // [C][vp + 4]
   T5D_GATED(g.gate);
   const t5d_recurrence& a = g.a;
   const int chunk = blockIdx.x, h = blockIdx.y, seq = blockIdx.z;
-  const int hg = h / (a.H / a.G);
   const int off = g.b.seq_off[seq];
   const int n = min(C, g.b.seq_off[seq + 1] - off - chunk * C);
   if (n <= 0) return;
   const int m0 = off + chunk * C;
   const int tid = threadIdx.x;
-  const int vp = (a.Dv + 15) / 16 * 16;
-  const int slot = g.b.seq_slot[seq], pos0 = g.b.seq_start[seq] + chunk * C;
-  // Columns of q, k, v and the decay; tokens past the end have no key, no query,
-  // no value and no decay.
-  for (int u = tid; u < 3 * DP + vp; u += 256) {
-    const int kind = u < DP ? 0 : u < 2 * DP ? 1 : u < 2 * DP + vp ? 2 : 3;
-    const int c = kind == 3 ? u - 2 * DP - vp : u - kind * DP;
-    float y[C];
-    if (c >= (kind == 2 ? a.Dv : a.D)) {
-#pragma unroll
-      for (int t = 0; t < C; ++t) y[t] = kind == 3 ? 1.f : 0.f;
-    } else if (kind == 3) {
-      const float* z = a.low + (size_t)m0 * a.ld_low + a.off_z + (size_t)h * a.D + c;
-#pragma unroll
-      for (int t = 0; t < C; ++t) y[t] = t < n ? z[(size_t)t * a.ld_low] : 0.f;
-#pragma unroll
-      for (int t = 0; t < C; ++t)
-        y[t] = t < n ? exp_f(log_decay(a, y[t], h, c)) : 1.f;
-    } else {
-      const int col = kind == 0 ? a.off_q + hg * a.D + c
-                      : kind == 1 ? a.off_k + hg * a.D + c : a.off_v + h * a.Dv + c;
-      const int cc = kind == 0 ? hg * a.D + c
-                     : kind == 1 ? (a.G + hg) * a.D + c
-                                 : 2 * a.G * a.D + h * a.Dv + c;
-      if (a.taps == 0)
-        chunk_column<0, T>(g, m0, n, chunk * C, pos0, slot, col, cc, y);
-      else if (a.taps <= 4)
-        chunk_column<4, T>(g, m0, n, chunk * C, pos0, slot, col, cc, y);
-      else
-        chunk_column<kChunkTaps, T>(g, m0, n, chunk * C, pos0, slot, col, cc, y);
-#pragma unroll
-      for (int t = 0; t < C; ++t)  // the convolution reaches past the end
-        if (t >= n) y[t] = 0.f;
-    }
-    float* dst = kind == 0 ? s_q : kind == 1 ? s_k : kind == 2 ? s_v : s_g;
-    const int stride = kind == 2 ? vp : LS;
-#pragma unroll
-    for (int t = 0; t < C; ++t) dst[t * stride + c] = y[t];
-  }
-  if (tid < C)
-    s_beta[tid] =
-        DELTA && tid < n
-            ? sigmoid_f(to_f32<T>(reinterpret_cast<const T*>(
-                  a.proj)[(size_t)(m0 + tid) * a.ld_proj + a.off_beta + h]))
-            : 0.f;
+  const int vp = (a.Dv + 15) / 16 * 16, vs = vp + 4;
+  if (a.taps == 0)
+    chunk_columns<0, DP, T>(g, chunk, n, m0, h, seq, s_q, s_k, s_g, s_v, vp, vs);
+  else if (a.taps <= 4)
+    chunk_columns<4, DP, T>(g, chunk, n, m0, h, seq, s_q, s_k, s_g, s_v, vp, vs);
+  else
+    chunk_columns<kChunkTaps, DP, T>(g, chunk, n, m0, h, seq, s_q, s_k, s_g, s_v, vp, vs);
+  if (DELTA && tid < C)
+    s_beta[tid] = tid < n ? sigmoid_f(to_f32<T>(reinterpret_cast<const T*>(
+                                a.proj)[(size_t)(m0 + tid) * a.ld_proj + a.off_beta + h]))
+                          : 0.f;
   s_a[tid >> 4][tid & 15] = 0.f;
   s_b[tid >> 4][tid & 15] = 0.f;
   __syncthreads();
@@ -414,135 +457,144 @@ recurrence_chunk_kernel(RecArgs g) {
   }
   __syncthreads();
   {
-    // 32 lanes per source token s, which walk t = s .. 15 with k_s decayed on
-    // the way; source j then source 15 - j, 17 steps for everyone.
-    constexpr int E = (DP + 127) / 128;
-    const int j = tid >> 5, c0 = 4 * (tid & 31);
+    // B and, with the delta rule, A: half of the wavefronts each, 16 lanes (without
+    // it 32) per source token, which walk t = s .. 15 with k_s decayed on the way;
+    // source j, then source 15 - j: 17 steps for everyone.
+    constexpr int LPS = DELTA ? 16 : 32, E = (DP + 4 * LPS - 1) / (4 * LPS);
+    const bool keys = DELTA && tid >= 128;
+    const int j = (tid / LPS) & 7, c0 = 4 * (tid % LPS);
+    const float* other = keys ? s_k : s_q;
+    float(*dst)[C] = keys ? s_a : s_b;
+    float4 x[E];
 #pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-      const int s = pass == 0 ? j : C - 1 - j;
-      float4 x[E];
+    for (int i = 0; i <= C; ++i) {
+      const bool second = i >= C - j;
+      const int s = second ? C - 1 - j : j, t = second ? i - 1 : j + i;
+      float sum = 0.f;
 #pragma unroll
-      for (int e = 0; e < E; ++e)
-        x[e] = c0 + 128 * e < DP
-                   ? *reinterpret_cast<const float4*>(s_k + s * LS + c0 + 128 * e)
-                   : make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int t = s; t < C; ++t) {
-        float ka = 0.f, qa = 0.f;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          if (c0 + 128 * e >= DP) continue;
-          const int o = t * LS + c0 + 128 * e;
-          if (t > s) {
-            const float4 w = *reinterpret_cast<const float4*>(s_g + o);
-            x[e].x *= w.x; x[e].y *= w.y; x[e].z *= w.z; x[e].w *= w.w;
-          }
-          const float4 y = *reinterpret_cast<const float4*>(s_q + o);
-          qa = fmaf(x[e].x, y.x, qa); qa = fmaf(x[e].y, y.y, qa);
-          qa = fmaf(x[e].z, y.z, qa); qa = fmaf(x[e].w, y.w, qa);
-          if (DELTA) {
-            const float4 z = *reinterpret_cast<const float4*>(s_k + o);
-            ka = fmaf(x[e].x, z.x, ka); ka = fmaf(x[e].y, z.y, ka);
-            ka = fmaf(x[e].z, z.z, ka); ka = fmaf(x[e].w, z.w, ka);
-          }
+      for (int e = 0; e < E; ++e) {
+        const int c = c0 + 4 * LPS * e;
+        if (DP % (4 * LPS) != 0 && c >= DP) continue;
+        const int o = t * LS + c;
+        if (t == s) {
+          x[e] = *reinterpret_cast<const float4*>(s_k + o);
+        } else {
+          const float4 w = *reinterpret_cast<const float4*>(s_g + o);
+          x[e].x *= w.x; x[e].y *= w.y; x[e].z *= w.z; x[e].w *= w.w;
         }
-        auto over32 = [](float f) {
-          f = lanes16_sum(f);
-          const auto w = __builtin_amdgcn_permlane16_swap(
-              __float_as_uint(f), __float_as_uint(f), false, false);
-          return __uint_as_float(w[0]) + __uint_as_float(w[1]);
-        };
-        qa = over32(qa);
-        if (DELTA) ka = over32(ka);
-        if ((tid & 31) == 0) {
-          s_b[t][s] = qa;
-          if (DELTA && t > s) s_a[t][s] = ka;
-        }
+        const float4 y = *reinterpret_cast<const float4*>(other + o);
+        sum = fmaf(x[e].x, y.x, sum); sum = fmaf(x[e].y, y.y, sum);
+        sum = fmaf(x[e].z, y.z, sum); sum = fmaf(x[e].w, y.w, sum);
       }
+      sum = lanes16_sum(sum);
+      if constexpr (LPS == 32) {
+        const auto w = __builtin_amdgcn_permlane16_swap(
+            __float_as_uint(sum), __float_as_uint(sum), false, false);
+        sum = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+      }
+      if (tid % LPS == 0 && (!keys || t > s)) dst[t][s] = sum;
     }
   }
   __syncthreads();
 
   const ChunkLayout lay(DP, vp);
   float* w = g.wchunk + ((chunk_base(off, seq) + chunk) * a.H + h) * lay.size();
-  // A thread per channel, then per value column: the triangular solve and the
-  // products with B down the column.
-  for (int c = tid; c < DP + vp; c += 256) {
-    const bool channel = c < DP;
-    const int vc = c - DP;
-    // (a zero the compiler cannot see through: it would otherwise read all of A
-    // and B into registers ahead of this loop)
-    int z = 0;
-    asm volatile("" : "+s"(z));
-    float x[C], run = 1.f;
-    float* sq = s_q + c;
-    float* sk = s_k + c;
-    float* sg = s_g + c;  // of a channel: read and written by this thread alone
-#pragma unroll
-    for (int t = 0; t < C; ++t) {
-      __builtin_amdgcn_sched_barrier(0);
-      float rhs;
-      if (channel) {
-        run *= sg[t * LS];
-        rhs = sk[t * LS] * run;
-      } else {
-        rhs = s_v[t * vp + vc];
-      }
-      if (DELTA) {
-#pragma unroll
-        for (int s = 0; s < t; ++s) rhs = fmaf(-s_a[t + z][s], x[s], rhs);
-        rhs *= s_beta[t];
-      }
-      x[t] = rhs;
-      if (channel) {
-        float y = sq[t * LS] * run;
-        if (DELTA) {
-#pragma unroll
-          for (int s = 0; s <= t; ++s) y = fmaf(-s_b[t + z][s], x[s], y);
-        }
-        sq[t * LS] = y;
-      }
-    }
-    if (channel) {
-      w[lay.pc() + c] = run;
-      float back = 1.f;
-#pragma unroll
-      for (int t = C - 1; t >= 0; --t) {
-        const float gt = sg[t * LS];
-        sg[t * LS] = sk[t * LS] * back;
-        back *= gt;
-        if (DELTA) sk[t * LS] = x[t];
-      }
-    } else {
-      float4* us = reinterpret_cast<float4*>(w + lay.us()) + (vc >> 4) * 64 + (vc & 15);
-      float4* os = reinterpret_cast<float4*>(w + lay.os()) + (vc >> 4) * 64 + (vc & 15);
-      float y[C];
+  if (tid >= 128) {
+    // a column of T per thread
+    if (DELTA && tid < 128 + C) {
+      const int c = tid - 128;
+      float x[C];
 #pragma unroll
       for (int t = 0; t < C; ++t) {
-        __builtin_amdgcn_sched_barrier(0);
-        y[t] = 0.f;
+        float r = t == c ? 1.f : 0.f;
 #pragma unroll
-        for (int s = 0; s <= t; ++s) y[t] = fmaf(s_b[t + z][s], x[s], y[t]);
+        for (int s = 0; s < t; ++s) r = fmaf(-s_a[t][s], x[s], r);
+        x[t] = r * s_beta[t];
+        s_t[t][c] = x[t];
       }
+    }
+  } else {
+    // a channel per thread: k P, q P, Kh and the whole decay
+    for (int c = tid; c < DP; c += 128) {
+      float k[C], run = 1.f, back = 1.f;
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        us[16 * q4] = make_float4(x[4 * q4], x[4 * q4 + 1], x[4 * q4 + 2], x[4 * q4 + 3]);
-        os[16 * q4] = make_float4(y[4 * q4], y[4 * q4 + 1], y[4 * q4 + 2], y[4 * q4 + 3]);
+      for (int t = 0; t < C; ++t) {
+        const int o = t * LS + c;
+        run *= s_g[o];
+        k[t] = s_k[o];
+        s_k[o] = k[t] * run;
+        s_q[o] *= run;
+      }
+      w[lay.pc() + c] = run;
+#pragma unroll
+      for (int t = C - 1; t >= 0; --t) {
+        const float gt = s_g[t * LS + c];
+        s_g[t * LS + c] = k[t] * back;
+        back *= gt;
       }
     }
   }
   __syncthreads();
-  for (int f = tid; f < DP * 4; f += 256) {
-    const int tile = f >> 6, l = f & 63, x = l & 15, g4 = l >> 4;
-    const int o = x * LS + 16 * tile + 4 * g4;
-    if (DELTA)
-      reinterpret_cast<float4*>(w + lay.wk())[f] =
-          *reinterpret_cast<const float4*>(s_k + o);
-    reinterpret_cast<float4*>(w + lay.qs())[f] =
-        *reinterpret_cast<const float4*>(s_q + o);
-    const float* kh = s_g + 4 * g4 * LS + 16 * tile + x;
-    reinterpret_cast<float4*>(w + lay.kh())[f] =
-        make_float4(kh[0], kh[LS], kh[2 * LS], kh[3 * LS]);
+  // Tiles of 16 channels, then of 16 value columns, dealt to the wavefronts.
+  const int lane = tid & 63, x = lane & 15, g4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const auto four = [](const float* p, float (&v)[4]) {
+    const float4 f = *reinterpret_cast<const float4*>(p);
+    v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+  };
+  const auto times = [](const float (&l)[4], const float (&r)[4], f32x4_v acc) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(l[i], r[i], acc, 0, 0, 0);
+    return acc;
+  };
+  const auto put = [](float* p, int at, f32x4_v v) {
+    reinterpret_cast<float4*>(p)[at] = make_float4(v[0], v[1], v[2], v[3]);
+  };
+  const f32x4_v zero = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+  float tm[4], bm[4], mm[4];  // rows x of T, B and M, columns 4 g + i
+  four(&s_b[x][4 * g4], bm);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) mm[i] = bm[i];
+  if (DELTA) {
+    four(&s_t[x][4 * g4], tm);
+    float tc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) tc[i] = s_t[4 * g4 + i][x];
+    const f32x4_v m = times(tc, bm, zero);  // M^T: rows 4 g + i, column x
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mm[i] = m[i];
+  }
+  for (int tile = wave; tile < DP / 16; tile += 4) {
+    const int at = tile * 64 + lane;
+    f32x4_v q;
+    {
+      const float4 f = *reinterpret_cast<const float4*>(s_q + x * LS + 16 * tile + 4 * g4);
+      q = (f32x4_v){f.x, f.y, f.z, f.w};
+    }
+    const int o = 4 * g4 * LS + 16 * tile + x;
+    if (DELTA) {
+      float r[4], minus[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        r[i] = s_k[o + i * LS];
+        minus[i] = -r[i];
+      }
+      put(w + lay.wk(), at, times(r, tm, zero));
+      q = times(minus, mm, q);
+    }
+    put(w + lay.qs(), at, q);
+    put(w + lay.kh(), at,
+        (f32x4_v){s_g[o], s_g[o + LS], s_g[o + 2 * LS], s_g[o + 3 * LS]});
+  }
+  for (int tile = wave; tile < vp / 16; tile += 4) {
+    const int at = tile * 64 + lane;
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = s_v[(4 * g4 + i) * vs + 16 * tile + x];
+    put(w + lay.us(), at,
+        DELTA ? times(tm, v, zero) : (f32x4_v){v[0], v[1], v[2], v[3]});
+    put(w + lay.os(), at, times(mm, v, zero));
   }
 }
 
@@ -916,7 +968,7 @@ static void launch_chunks(hipStream_t s, const RecArgs& g) {
   const int vts = (g.a.Dv + 15) / 16, pairs = g.a.H * g.b.S;
   const dim3 grid(g.chunks, g.a.H, g.b.S), block(256);
   const dim3 chain((pairs + 7) / 8 * 8 * vts);
-  const size_t lds = (size_t)kChunk * vts * 16 * sizeof(float);
+  const size_t lds = (size_t)kChunk * (vts * 16 + 4) * sizeof(float);
 #define T5D_CH(E_)                                                               \
   do {                                                                           \
     hipLaunchKernelGGL((recurrence_chunk_kernel<64 * E_, DELTA, T>), grid, block, \
