@@ -394,6 +394,12 @@ constexpr int kChunkTaps = 8;  // longest convolution of the chunk kernel
 // T = (I + diag(beta) A)^-1 diag(beta), 16 x 16, and everything that is applied to
 // whole columns on the matrix cores: Wk = T (k P), Us = T v, and with M = B T
 // Qs = q P - M (k P), Os = M v.
+// What bounds it: vector instructions (57 % of their slots; 1640 per wavefront, half of
+// them silu and decays) with four workgroups per CU, then 42 KB written per chunk and
+// head.  4 x 4096 tokens, 8 heads of 128: delta rule 160 us, gated linear attention
+// 103 us; 301 and 240 us with the triangular solve and the products with B down each
+// column on the vector ALUs, divisions instead of sigmoid_quick, the library's
+// logarithm, and loads that branches kept from being in flight together.
 template <int DP, bool DELTA, typename T>
 __global__ void __launch_bounds__(256, DP <= 128 ? 4 : DP <= 256 ? 2 : 1)
 recurrence_chunk_kernel(RecArgs g) {
@@ -600,8 +606,14 @@ recurrence_chunk_kernel(RecArgs g) {
 
 // Walks the chunks of one (sequence, head) for 16 value columns.  Each of 4
 // wavefronts holds NTW tiles of 16 channels x 16 columns of the state.
+// What bounds it: the chain of a step at one wavefront per SIMD where sequences are
+// few (24 dependent matrix products = 770 of its 1930 cycles, the exchange of partial
+// sums behind one barrier, the next step's first operands).  256 steps of 32
+// (sequence, head) pairs: 206 us with the delta rule, 153 without; 225 and 187 us
+// with the requests, their address arithmetic and the read-out in the chain's way and
+// a wait for every request each fourth step (at the head of the loop).
 template <int NTW, bool DELTA>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, NTW <= 2 ? 2 : 1)
 recurrence_chain_kernel(RecArgs g) {
   constexpr int DP = 64 * NTW;
   __shared__ float4 s_u[2][4][64];
@@ -624,8 +636,6 @@ recurrence_chain_kernel(RecArgs g) {
   const bool col_ok = col < a.Dv;
   const ChunkLayout lay(DP, vp);
   const int nc = (len + kChunk - 1) / kChunk;
-  const size_t stride = (size_t)a.H * lay.size();
-  const float* base = g.wchunk + (chunk_base(off, seq) * a.H + h) * lay.size();
 
   float* state = a.state + ((size_t)slot * a.H + h) * a.D * a.Dv + col;
   f32x4_v st[NTW];
@@ -636,27 +646,43 @@ recurrence_chain_kernel(RecArgs g) {
       const int d = 16 * (wave * NTW + t) + 4 * g4 + i;
       st[t][i] = start > 0 && col_ok && d < a.D ? state[(size_t)d * a.Dv] : 0.f;
     }
-  float* out = g.wo + ((size_t)off * a.H + h) * a.Dv + col;
+  const size_t row = (size_t)a.H * a.Dv;  // of the read-outs
+  float* out = g.wo + (size_t)off * row + (size_t)h * a.Dv + col +
+               (size_t)(4 * g4 + wave) * row;
 
   struct Operands {
-    float4 wk[NTW], qs[NTW], kh[NTW], pc[NTW], us, os;
+    float4 wk[NTW], qs[NTW], kh[NTW], pc[NTW], us;
+    float os;
   };
-  auto load = [&](Operands& o, int c) {
-    const float* w = base + (size_t)c * stride;
+  // Operands: a uniform base per chunk, which stops at the last one, and offsets
+  // within a chunk that never change.
+  const size_t stride = (size_t)a.H * lay.size() * sizeof(float);
+  const char* next = reinterpret_cast<const char*>(
+      g.wchunk + (chunk_base(off, seq) * a.H + h) * lay.size());
+  int to_load = nc;  // chunks not yet requested
+  const uint32_t at = (wave * NTW * 64 + lane) * 16;
+  const uint32_t at_pc = (wave * NTW * 4 + g4) * 16;
+  const uint32_t at_us = (vt * 64 + lane) * 16, at_os = at_us + 4 * wave;
+  const auto piece = [&](size_t of, uint32_t o) {
+    return *reinterpret_cast<const float4*>(next + 4 * of + o);
+  };
+  auto load = [&](Operands& o) {
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
-      const int tile = wave * NTW + t;
-      if (DELTA)
-        o.wk[t] = reinterpret_cast<const float4*>(w + lay.wk())[tile * 64 + lane];
-      o.qs[t] = reinterpret_cast<const float4*>(w + lay.qs())[tile * 64 + lane];
-      o.kh[t] = reinterpret_cast<const float4*>(w + lay.kh())[tile * 64 + lane];
-      o.pc[t] = reinterpret_cast<const float4*>(w + lay.pc())[tile * 4 + g4];
+      if (DELTA) o.wk[t] = piece(lay.wk(), at + 1024 * t);
+      o.qs[t] = piece(lay.qs(), at + 1024 * t);
+      o.kh[t] = piece(lay.kh(), at + 1024 * t);
+      o.pc[t] = piece(lay.pc(), at_pc + 64 * t);
     }
-    o.us = reinterpret_cast<const float4*>(w + lay.us())[vt * 64 + lane];
+    o.us = piece(lay.us(), at_us);
     // (only the row this wavefront stores is used)
-    o.os.x = (w + lay.os())[(vt * 64 + lane) * 4 + wave];
+    o.os = *reinterpret_cast<const float*>(next + 4 * lay.os() + at_os);
+    next += --to_load > 0 ? stride : 0;
   };
-  auto step = [&](const Operands& o, int c) {
+  // A step: u (behind it the exchange of the wavefronts' parts), the read-out's
+  // product and the requests for a later chunk while the parts are on their way,
+  // the state's update, and the read-out behind its products.
+  auto step = [&](const Operands& o, Operands& later, int c) {
     const int buf = c & 1;
     f32x4_v u = (f32x4_v){0.f, 0.f, 0.f, 0.f}, r = u;
     if (DELTA) {
@@ -667,7 +693,10 @@ recurrence_chain_kernel(RecArgs g) {
         for (int i = 0; i < 4; ++i)
           u = __builtin_amdgcn_mfma_f32_16x16x4f32(wk[i], st[t][i], u, 0, 0, 0);
       }
+      s_u[buf][wave][lane] = make_float4(u[0], u[1], u[2], u[3]);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    load(later);
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
       const float qs[4] = {o.qs[t].x, o.qs[t].y, o.qs[t].z, o.qs[t].w};
@@ -675,46 +704,54 @@ recurrence_chain_kernel(RecArgs g) {
       for (int i = 0; i < 4; ++i)
         r = __builtin_amdgcn_mfma_f32_16x16x4f32(qs[i], st[t][i], r, 0, 0, 0);
     }
-    if (DELTA) s_u[buf][wave][lane] = make_float4(u[0], u[1], u[2], u[3]);
     s_o[buf][wave][lane] = make_float4(r[0], r[1], r[2], r[3]);
+#pragma unroll
+    for (int t = 0; t < NTW; ++t) {
+      st[t][0] *= o.pc[t].x; st[t][1] *= o.pc[t].y;
+      st[t][2] *= o.pc[t].z; st[t][3] *= o.pc[t].w;
+    }
     __syncthreads();
     float uu[4] = {o.us.x, o.us.y, o.us.z, o.us.w};
+    float y[4];
     if (DELTA) {
       const float4 p0 = s_u[buf][0][lane], p1 = s_u[buf][1][lane];
       const float4 p2 = s_u[buf][2][lane], p3 = s_u[buf][3][lane];
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        y[p] = reinterpret_cast<const float*>(&s_o[buf][p][lane])[wave];
       uu[0] -= (p0.x + p1.x) + (p2.x + p3.x);
       uu[1] -= (p0.y + p1.y) + (p2.y + p3.y);
       uu[2] -= (p0.z + p1.z) + (p2.z + p3.z);
       uu[3] -= (p0.w + p1.w) + (p2.w + p3.w);
+    } else {
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        y[p] = reinterpret_cast<const float*>(&s_o[buf][p][lane])[wave];
     }
 #pragma unroll
-    for (int t = 0; t < NTW; ++t) {
-      const float kh[4] = {o.kh[t].x, o.kh[t].y, o.kh[t].z, o.kh[t].w};
-      st[t][0] *= o.pc[t].x; st[t][1] *= o.pc[t].y;
-      st[t][2] *= o.pc[t].z; st[t][3] *= o.pc[t].w;
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int t = 0; t < NTW; ++t) {
+        const float kh[4] = {o.kh[t].x, o.kh[t].y, o.kh[t].z, o.kh[t].w};
         st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[i], uu[i], st[t], 0, 0, 0);
-    }
+      }
+    __builtin_amdgcn_sched_barrier(0);
     // the read-out of tokens 4 g + wave
-    float y = o.os.x;
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-      y += reinterpret_cast<const float*>(&s_o[buf][p][lane])[wave];
-    const int tok = kChunk * c + 4 * g4 + wave;
-    if (tok < len && col_ok) out[(size_t)tok * a.H * a.Dv] = y;
+    const float sum = (((o.os + y[0]) + y[1]) + y[2]) + y[3];
+    if (kChunk * c + 4 * g4 + wave < len && col_ok) *out = sum;
+    out += kChunk * row;
   };
-  // The operands of the next chunks are on their way while one is multiplied.
-  constexpr int DEPTH = NTW <= 4 ? 4 : 2;
+  // The operands of the next chunks are on their way while one is multiplied.  The
+  // compiler waits for all of them at the head of a loop, hence 16 steps per round.
+  constexpr int DEPTH = NTW <= 4 ? 4 : 2, ROUND = NTW <= 2 ? 4 * DEPTH : DEPTH;
   Operands o[DEPTH];
 #pragma unroll
-  for (int i = 0; i + 1 < DEPTH; ++i) load(o[i], min(i, nc - 1));
-  for (int c0 = 0; c0 < nc; c0 += DEPTH) {
+  for (int i = 0; i + 1 < DEPTH; ++i) load(o[i]);
+  for (int c0 = 0; c0 < nc; c0 += ROUND) {
 #pragma unroll
-    for (int i = 0; i < DEPTH; ++i) {
+    for (int i = 0; i < ROUND; ++i) {
       if (c0 + i >= nc) break;
-      load(o[(i + DEPTH - 1) % DEPTH], min(c0 + i + DEPTH - 1, nc - 1));
-      step(o[i], c0 + i);
+      step(o[i % DEPTH], o[(i + DEPTH - 1) % DEPTH], c0 + i);
     }
   }
 #pragma unroll

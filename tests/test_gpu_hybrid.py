@@ -486,6 +486,34 @@ class Recurrence:
     return 1e-5 if self.dt == torch.float32 else 4e-3
 
 
+@pytest.mark.parametrize('dt', DTYPES)
+@pytest.mark.parametrize('delta,D,Dv,taps', [(True, 128, 40, 4), (True, 40, 128, 6),
+                                             (False, 128, 48, 0), (True, 200, 20, 0)])
+@pytest.mark.parametrize('kind', ['same keys', 'large', 'no memory'])
+def test_recurrence_chunks_of_hard_inputs(dt, delta, D, Dv, taps, kind):
+  """Chunks against the oracle where their algebra is at its worst: one key
+  throughout, written with step sizes near 1 and kept without decay (the triangular
+  systems are full of ones), projections that saturate every gate and decay, decays
+  that leave nothing; lengths off the chunk."""
+  r = Recurrence(dt, delta, 2, 1, D, Dv, taps, 1, seed=D + taps)
+  T = 77
+  x, z = r.sequence(T)
+  zs = slice(r.low_off[0], r.low_off[0] + 2 * D)
+  if kind == 'same keys':
+    x[:, r.off[1]:r.off[1] + D] = x[:1, r.off[1]:r.off[1] + D]
+    x[:, r.off[3]:r.off[3] + 2] = 9.0
+    z[:, zs] = -30.0 if delta else 30.0
+  elif kind == 'large':
+    x *= 25.0
+    # (the oracle's sigmoid, (1 + tanh) / 2, is exact to 1e-16, a root of it only
+    # where it is not far below 1e-9)
+    z[:, zs] = 25.0 * z[:, zs] if delta else (25.0 * z[:, zs]).clamp(-12, 60)
+  else:
+    z[:, zs] = 90.0 if delta else -90.0
+  want = r.oracle((x, z))
+  assert rel(r.run([(0, 0, T)], [(x, z)], 3), want) < r.tol
+
+
 def seq_cols(x, at, n):
   return x[:, at:at + n]
 
