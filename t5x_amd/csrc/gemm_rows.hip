@@ -93,11 +93,10 @@ constexpr int kRowsMT = 8, kRowsNT = 4;        // MFMA tiles per wavefront
 // What a wavefront does with its finished accumulator tiles (m0: its first
 // row, nt0: its first 16-column tile) when the product was formed as C, for
 // the value layout:
-template <int NT>
+template <int MT, int NT>
 __device__ __forceinline__ void rows_epilogue_values(
-    const RowsGemmArgs& g, const f32x4_r (&acc)[kRowsMT][NT], int m0,
+    const RowsGemmArgs& g, const f32x4_r (&acc)[MT][NT], int m0,
     int nt0, int n_tiles, int l16, int gq) {
-  constexpr int MT = kRowsMT;
   // acc[mt][nt][i]: row m = m0 + 16 mt + 4 gq + i, column n = 16 (nt0 + nt) + l16
   // (values layout [B, H, Ep / 32, 64, 32]: 4 consecutive positions per store)
 #pragma unroll
@@ -135,21 +134,28 @@ __device__ __forceinline__ void rows_epilogue_values(
 // DENSE: one of the epilogues of t5d_dense instead: 1 = T5D_EPI_CLAMPED_GLU (first
 // column of a pair: gate, second: up), 2 = float32 rows.
 constexpr int kRowsStageBytes = 16 * 144;
-template <int NT, int DENSE>
+template <int DENSE, bool SCALED, int MT, int NT>
 __device__ __forceinline__ void rows_epilogue_staged(
-    const RowsGemmArgs& g, const f32x4_r (&acc)[kRowsMT][NT], int m0, int nt0,
+    const RowsGemmArgs& g, const f32x4_r (&acc)[MT][NT], int m0, int nt0,
     int n_tiles, int lane, char* stage) {
   static_assert(NT == 3 || NT == 4, "a wavefront's slice: 48 or 64 columns");
-  constexpr int MT = kRowsMT;
   const int l16 = lane & 15, gq = lane >> 4;
-  // int8 weights: the scale of each of this lane's 4 columns (1 otherwise)
+  // int8 weights: the scale of each of this lane's 4 columns
   float4 sc[NT];
+  if constexpr (SCALED) {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-    sc[nt] = (g.scales && nt0 + nt < n_tiles)
-                 ? *reinterpret_cast<const float4*>(g.scales +
-                                                    16 * (nt0 + nt) + 4 * gq)
-                 : make_float4(1.f, 1.f, 1.f, 1.f);
+    for (int nt = 0; nt < NT; ++nt)
+      sc[nt] = (g.scales && nt0 + nt < n_tiles)
+                   ? *reinterpret_cast<const float4*>(g.scales +
+                                                      16 * (nt0 + nt) + 4 * gq)
+                   : make_float4(1.f, 1.f, 1.f, 1.f);
+  }
+  const auto value = [&](int mt, int nt, int i) {
+    if constexpr (SCALED)
+      return acc[mt][nt][i] * reinterpret_cast<const float*>(&sc[nt])[i];
+    else
+      return acc[mt][nt][i];
+  };
   if constexpr (DENSE == 2) {
     // a lane holds 4 consecutive columns of one row: 64 bytes per row and store
 #pragma unroll
@@ -161,8 +167,8 @@ __device__ __forceinline__ void rows_epilogue_staged(
         if (nt0 + nt >= n_tiles) continue;
         const int n = 16 * (nt0 + nt) + 4 * gq;
         float* o = g.C32 + (size_t)m * g.ldc + n;
-        const float4 v = make_float4(acc[mt][nt][0] * sc[nt].x, acc[mt][nt][1] * sc[nt].y,
-                                     acc[mt][nt][2] * sc[nt].z, acc[mt][nt][3] * sc[nt].w);
+        const float4 v = make_float4(value(mt, nt, 0), value(mt, nt, 1),
+                                     value(mt, nt, 2), value(mt, nt, 3));
         if ((g.ldc & 3) == 0 && n + 4 <= g.n_store) {
           *reinterpret_cast<float4*>(o) = v;
         } else {
@@ -191,17 +197,17 @@ __device__ __forceinline__ void rows_epilogue_staged(
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const auto a = __builtin_amdgcn_permlane32_swap(
-            __float_as_uint(acc[mt][nt][2] * sc[nt].z),
-            __float_as_uint(acc[mt][nt][0] * sc[nt].x), false, false);
+            __float_as_uint(value(mt, nt, 2)),
+            __float_as_uint(value(mt, nt, 0)), false, false);
         const auto b = __builtin_amdgcn_permlane32_swap(
-            __float_as_uint(acc[mt][nt][3] * sc[nt].w),
-            __float_as_uint(acc[mt][nt][1] * sc[nt].y), false, false);
+            __float_as_uint(value(mt, nt, 3)),
+            __float_as_uint(value(mt, nt, 1)), false, false);
         // [0]: the value (own in the lower half), [1]: its gate
         float h0, h1;
         if constexpr (DENSE == 1) {
-          h0 = clamped_glu(__uint_as_float(a[0]), __uint_as_float(a[1]),
+          h0 = clamped_glu_bf16(__uint_as_float(a[0]), __uint_as_float(a[1]),
                            g.glu_limit, g.glu_alpha, g.glu_add);
-          h1 = clamped_glu(__uint_as_float(b[0]), __uint_as_float(b[1]),
+          h1 = clamped_glu_bf16(__uint_as_float(b[0]), __uint_as_float(b[1]),
                            g.glu_limit, g.glu_alpha, g.glu_add);
         } else {
           h0 = round_bf16(gelu_sigmoid_form(round_bf16(__uint_as_float(a[0])))) *
@@ -227,13 +233,32 @@ __device__ __forceinline__ void rows_epilogue_staged(
   const int piece = lane % PP, prow = lane / PP;
   const int n = 16 * nt0 + 8 * piece;
   const bool n_ok = nt0 + (piece >> 1) < n_tiles;
+  // The residual of AHEAD slices is under way while one is added (16384 x 768 x 768,
+  // which waited for each slice: 31.9 -> 28.2 us with the bank conflicts gone too).
+  constexpr int AHEAD = 4;
+  const bool residual = g.epilogue == T5D_EPI_RESIDUAL;
+  uint4 res[AHEAD][2];
+  const auto fetch = [&](int mt) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int m = m0 + 16 * mt + RPI * j + prow;
+      res[mt % AHEAD][j] = make_uint4(0, 0, 0, 0);
+      if (prow < RPI && RPI * j + prow < 16 && m < g.M && n_ok)
+        res[mt % AHEAD][j] =
+            *reinterpret_cast<const uint4*>(g.residual + (size_t)m * g.N + n);
+    }
+  };
+  if (residual) {
+#pragma unroll
+    for (int mt = 0; mt < (AHEAD < MT ? AHEAD : MT); ++mt) fetch(mt);
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
       *reinterpret_cast<uint2*>(stage + l16 * 144 + (16 * nt + 4 * gq) * 2) =
-          pack4(acc[mt][nt][0] * sc[nt].x, acc[mt][nt][1] * sc[nt].y,
-                acc[mt][nt][2] * sc[nt].z, acc[mt][nt][3] * sc[nt].w);
+          pack4(value(mt, nt, 0), value(mt, nt, 1),
+                value(mt, nt, 2), value(mt, nt, 3));
     asm volatile("" ::: "memory");
     uint4 back[2];
 #pragma unroll
@@ -241,11 +266,27 @@ __device__ __forceinline__ void rows_epilogue_staged(
       back[j] = *reinterpret_cast<const uint4*>(
           stage + min(RPI * j + prow, 15) * 144 + piece * 16);
     asm volatile("" ::: "memory");
+    if (residual) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        uint4& q = back[j];
+        const uint4 r = res[mt % AHEAD][j];
+        q.x = pack_bf16x2(bf16lo_to_f32(q.x) + bf16lo_to_f32(r.x),
+                          bf16hi_to_f32(q.x) + bf16hi_to_f32(r.x));
+        q.y = pack_bf16x2(bf16lo_to_f32(q.y) + bf16lo_to_f32(r.y),
+                          bf16hi_to_f32(q.y) + bf16hi_to_f32(r.y));
+        q.z = pack_bf16x2(bf16lo_to_f32(q.z) + bf16lo_to_f32(r.z),
+                          bf16hi_to_f32(q.z) + bf16hi_to_f32(r.z));
+        q.w = pack_bf16x2(bf16lo_to_f32(q.w) + bf16lo_to_f32(r.w),
+                          bf16hi_to_f32(q.w) + bf16hi_to_f32(r.w));
+      }
+      if (mt + AHEAD < MT) fetch(mt + AHEAD);
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int row = RPI * j + prow;
       if (prow >= RPI || row >= 16) continue;
-      uint4 q = back[j];
+      const uint4 q = back[j];
       const int m = m0 + 16 * mt + row;
       if (m >= g.M || !n_ok) continue;
       size_t o;
@@ -256,18 +297,6 @@ __device__ __forceinline__ void rows_epilogue_staged(
         o = ((((size_t)b * g.H + hh) * 2 + c) * g.Ep + e) * 32 + jj;
       } else {
         o = (size_t)m * g.N + n;
-      }
-      if (g.epilogue == T5D_EPI_RESIDUAL) {
-        const uint4 r = *reinterpret_cast<const uint4*>(
-            g.residual + (size_t)m * g.N + n);
-        q.x = pack_bf16x2(bf16lo_to_f32(q.x) + bf16lo_to_f32(r.x),
-                          bf16hi_to_f32(q.x) + bf16hi_to_f32(r.x));
-        q.y = pack_bf16x2(bf16lo_to_f32(q.y) + bf16lo_to_f32(r.y),
-                          bf16hi_to_f32(q.y) + bf16hi_to_f32(r.y));
-        q.z = pack_bf16x2(bf16lo_to_f32(q.z) + bf16lo_to_f32(r.z),
-                          bf16hi_to_f32(q.z) + bf16hi_to_f32(r.z));
-        q.w = pack_bf16x2(bf16lo_to_f32(q.w) + bf16lo_to_f32(r.w),
-                          bf16hi_to_f32(q.w) + bf16hi_to_f32(r.w));
       }
       *reinterpret_cast<uint4*>(g.C + o) = q;
     }
@@ -378,11 +407,11 @@ rows_gemm_kernel(RowsGemmArgs g) {
   if (SWAP) {
     // (the loop ends with a barrier: every wavefront is done with the tiles)
     static_assert(sizeof(s_t[0]) >= 4 * kRowsStageBytes, "stage too small");
-    rows_epilogue_staged<NT, DENSE>(
+    rows_epilogue_staged<DENSE, sizeof(WT) == 1>(
         g, acc, m0, nt0, n_tiles, lane,
         reinterpret_cast<char*>(&s_t[0][0][0]) + wave * kRowsStageBytes);
   } else {
-    rows_epilogue_values<NT>(g, acc, m0, nt0, n_tiles, l16, gq);
+    rows_epilogue_values(g, acc, m0, nt0, n_tiles, l16, gq);
   }
 }
 
@@ -398,13 +427,14 @@ rows_gemm_kernel(RowsGemmArgs g) {
 // the K loop handles three k-tiles per round, so that the compiler can tell a
 // read of one stage from a load into another and adds no wait of its own.
 // An activation tile is fetched with lane 4 q + j reading row q, piece
-// (j + q / 4) % 4 — four neighbouring lanes still read 64 contiguous bytes —
-// which puts piece p of row r at slot 4 r + (p - r / 4) % 4, so that the 16
-// lanes of a quarter wavefront read 16 slots that differ mod 16.  The LDS
-// still counts bank conflicts for these reads (its rule for 16-byte reads is
-// not the plain one; other rotations measured the same or worse), but the
-// alternative without any — every lane fetching its own operand piece, 16
-// rows per quarter wavefront — loses more in the fetch (185 us against 174).
+// j ^ swap(q / 4) — four neighbouring lanes still read 64 contiguous bytes —
+// which puts piece p of row r at slot 4 r + (p ^ swap(r / 4)).  A 16-byte read
+// serves 16 lanes at a time: 0..3 and 12..15 of one quarter wavefront with 4..11
+// of its neighbour, which want the neighbouring piece.  With swap = 0, 0, 3, 3
+// their 16 slots differ mod 16.  (Slots that differ within a quarter, by a
+// rotation or an XOR by r / 4, made 40 % of the LDS cycles bank conflicts:
+// 8192 x 1024 x 5632 gated 97 us, 16384 x 768 x 4096 gated 123 us, now
+// 90 and 115 us.)
 // bfloat16 weights (int8 tiles must be widened on the way).
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* glb_ptr_t;
@@ -422,15 +452,15 @@ typedef __attribute__((address_space(1))) const void* glb_ptr_t;
 template <bool SWAP, int NT, int WN, int DENSE = 0, bool GROUPED = false>
 __global__ void __launch_bounds__(128 * WN, WN == 2 ? 2 : 1)
 rows_gemm_direct_kernel(RowsGemmArgs g) {
-  constexpr int MT = kRowsMT;
+  constexpr int MT = kRowsMT, BM = 32 * MT, ATILES = 2 * MT;
   constexpr int WAVES = 2 * WN;         // 2 rows of WN wavefronts
   constexpr int BN = WN * NT * 16;      // columns of the workgroup tile
-  constexpr int AL = 16 / WAVES;        // activation tiles a wavefront loads per stage
+  constexpr int AL = ATILES / WAVES;    // activation tiles a wavefront loads per stage
   constexpr int WTILES = WN * NT;       // weight tiles of a stage
   // weight tiles a wavefront loads per stage; when they do not divide evenly
   // some wavefronts load a tile a second time (same bytes to the same place)
   constexpr int WL = (WTILES + WAVES - 1) / WAVES;
-  constexpr int TILES = 16 + WN * NT;
+  constexpr int TILES = ATILES + WN * NT;
   // Before every barrier: all but my newest AL + WL loads have landed AND all
   // my reads of LDS have returned, s_waitcnt vmcnt(AL + WL) lgkmcnt(0).  The
   // second half matters: the barrier orders instructions that have been
@@ -441,7 +471,7 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   // one wrong 16-row slice in about one launch in ten at 16384 x 768).
   constexpr int kWaitStage = 0x070 | (AL + WL);
   constexpr int kWaitAll = 0x070;
-  // [tile][lane]: tiles 0..15 activations (rows 16 t ..), then the weights
+  // [tile][lane]: activations (rows 16 t ..), then the weights
   __shared__ uint4 s_t0[TILES][64];
   __shared__ uint4 s_t1[TILES][64];
   __shared__ uint4 s_t2[TILES][64];
@@ -463,17 +493,18 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, gq = lane >> 4;
-  const int m_blocks = (g.M + kRowsBM - 1) / kRowsBM;
+  const int m_blocks = (g.M + BM - 1) / BM;
   const int m_blk = GROUPED ? 0 : blockIdx.x % m_blocks;
   const int n_blk = GROUPED ? group_n_blk : blockIdx.x / m_blocks;
   const int wm = wave / WN, wn = wave % WN;
-  const int m0 = m_blk * kRowsBM + wm * (16 * MT);
+  const int m0 = m_blk * BM + wm * (16 * MT);
   const int nt0 = n_blk * (BN / 16) + wn * NT;
   const int KT = g.K >> 5, n_tiles = g.N >> 4;
 
+  const auto swap = [](int q) { return q & 2 ? 3 : 0; };
   const int ld_row = lane >> 2;
-  const int ld_piece = ((lane & 3) + (ld_row >> 2)) & 3;
-  const int read_slot = 4 * l16 + ((gq - (l16 >> 2)) & 3);
+  const int ld_piece = (lane & 3) ^ swap(ld_row >> 2);
+  const int read_slot = 4 * l16 + (gq ^ swap(l16 >> 2));
   // this wavefront's tiles of every stage: activation tiles wave + WAVES i,
   // weight tiles wave + WAVES i (rows / tiles past the edge clamped: their
   // products are discarded in the epilogue)
@@ -481,7 +512,7 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   const char* wtile[WL];
 #pragma unroll
   for (int i = 0; i < AL; ++i) {
-    int row = min(m_blk * kRowsBM + 16 * (wave + WAVES * i) + ld_row, g.M - 1);
+    int row = min(m_blk * BM + 16 * (wave + WAVES * i) + ld_row, g.M - 1);
     if constexpr (GROUPED) row = group_row(g.grp, row);
     arow[i] = reinterpret_cast<const char*>(g.A + (size_t)row * g.lda +
                                             8 * ld_piece);
@@ -507,13 +538,13 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
     _Pragma("unroll") for (int i = 0; i < WL; ++i)                             \
       __builtin_amdgcn_global_load_lds(                                        \
           (glb_ptr_t)(wtile[i] + (size_t)(kt_) * 1024),                        \
-          (lds_ptr_t)&S_[16 + (wave + WAVES * i) % WTILES][0], 16, 0, 0);      \
+          (lds_ptr_t)&S_[ATILES + (wave + WAVES * i) % WTILES][0], 16, 0, 0);      \
   } while (0)
 #define T5D_ROWS_MULTIPLY(S_)                                                  \
   do {                                                                         \
     FragR wb[NT];                                                              \
     _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                          \
-      wb[nt].u = S_[16 + wn * NT + nt][lane];                                  \
+      wb[nt].u = S_[ATILES + wn * NT + nt][lane];                                  \
     _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) {                        \
       FragR xa;                                                                \
       xa.u = S_[wm * MT + mt][read_slot];                                      \
@@ -570,11 +601,11 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   if (SWAP) {
     static_assert(sizeof(s_t0) >= WAVES * kRowsStageBytes, "stage too small");
     __syncthreads();  // every wavefront is done with the ring
-    rows_epilogue_staged<NT, DENSE>(
+    rows_epilogue_staged<DENSE, false>(
         g, acc, m0, nt0, n_tiles, lane,
         reinterpret_cast<char*>(&s_t0[0][0]) + wave * kRowsStageBytes);
   } else {
-    rows_epilogue_values<NT>(g, acc, m0, nt0, n_tiles, l16, gq);
+    rows_epilogue_values(g, acc, m0, nt0, n_tiles, l16, gq);
   }
 }
 

@@ -163,7 +163,7 @@ __device__ __forceinline__ void store_result(const DenseArgs& g, int m, int n,
   if (gated(g)) {
     const int f = (n >> 4) * 8 + (n & 7);
     reinterpret_cast<bf16_t*>(g.C)[(size_t)m * (g.N >> 1) + f] =
-        f32_to_bf16(clamped_glu(v, v_gate, g.glu_limit, g.glu_alpha, g.glu_add));
+        f32_to_bf16(clamped_glu_bf16(v, v_gate, g.glu_limit, g.glu_alpha, g.glu_add));
     return;
   }
   const size_t o = (size_t)m * g.ldc + n;

@@ -73,6 +73,38 @@ def test_clamped_glu(dt, M, K, F):
   assert rel(host(got), want) < (1e-6 if dt == torch.float32 else 4e-3)
 
 
+@pytest.mark.parametrize('M', [3, 200, 300, 2000])
+def test_clamped_glu_far_from_zero(M):
+  """Gates at which the exponential vanishes or overflows, passed through the product
+  unchanged.  Bound: half a bfloat16 step (7 stored bits: 2^-8) and the float32 steps of the
+  unit (an argument of 88 carries its own rounding of 2^-24 into the exponent: 1e-5);
+  results under 1e-30 (gates below -60) may vanish."""
+  from t5x_amd import ops
+  rs = np.random.RandomState(M)
+  K = 64
+  gates = np.concatenate([s * np.geomspace(1e-6, 3e38, 40) for s in (1, -1)] +
+                         [np.zeros(1), np.linspace(-90, 90, 61)])
+  a = np.zeros((M, K))
+  a[:, :32] = rs.choice(gates, (M, 32))
+  a[:, 32:] = rs.choice([-3e38, -7.5, -1.0, 0.0, 1e-3, 2.0, 1e30], (M, 32))
+  a = dev(a, torch.bfloat16)
+  gate, up = np.zeros((K, 32)), np.zeros((K, 32))
+  gate[np.arange(32), np.arange(32)] = up[np.arange(32, 64), np.arange(32)] = 1
+  for limit, alpha, add in ((7.0, 1.702, 1.0), (np.inf, 1.0, 0.0)):
+    got = host(ops.dense(a, ops.pack_weight(dev(gate), torch.bfloat16,
+                                            gate_kernel=dev(up)),
+                         glu=(limit, alpha, add)))
+    x = host(a).astype(np.float64)
+    g, u = np.minimum(x[:, :32], limit), np.clip(x[:, 32:], -limit, limit)
+    s = np.where(g > 0, 1 / (1 + np.exp(-np.abs(alpha * g))),
+                 np.exp(-np.abs(alpha * g)) / (1 + np.exp(-np.abs(alpha * g))))
+    want = g * s * (u + add)
+    keep = np.abs(want) < 3e38  # beyond it: infinity, or a factor that vanished
+    ok = np.abs(got - want) <= (2**-8 + 2e-5) * np.abs(want) + 1e-30 * np.abs(u + add)
+    assert np.all(ok | ~keep)
+    assert not np.any(np.isnan(got[keep]))
+
+
 @pytest.mark.parametrize('dt', DTYPES)
 @pytest.mark.parametrize('width,ld', [(40, 64), (64, 64), (90, 128), (37, 64)])
 def test_embed_sinusoid(dt, width, ld):
