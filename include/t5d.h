@@ -165,7 +165,8 @@ int t5d_gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
                   int Ep);
 
 /* t5d_gemm_rows with the workgroup tile of the caller's choice: tile 1 =
- * 256 rows x 128 columns (4 wavefronts, two workgroups per CU), tile 2 =
+ * 256 rows x 128 columns (4 wavefronts, two workgroups per CU; 128 or 64 rows
+ * where bfloat16 weights leave CUs without a workgroup otherwise), tile 2 =
  * 256 x 256 and tile 3 = 256 x 192 (8 wavefronts, one workgroup per CU;
  * bfloat16 weights and K >= 64, otherwise tile 1 is used), tile 0 = what
  * t5d_gemm_rows picks from the shape.  Results have the same bits for every

@@ -440,7 +440,7 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* glb_ptr_t;
 
 // WN: wavefront columns of the workgroup, 2 (256 x 128 tile, 4 wavefronts, two
-// workgroups per CU) or 4 (256 x 256, 8 wavefronts, one per CU).
+// workgroups per CU; 128 and 64 rows with MT 4 and 2) or 4 (256 x 256, 8 wavefronts, one per CU).
 // Measured on the gated MLP input projection of the T5.1.1-base encoder
 // (16384 x 768 x 4096): 182 -> 176 us per launch with the ring alone, 123 us
 // with the epilogue below (the library tanh and the 8-byte stores were a
@@ -449,10 +449,11 @@ typedef __attribute__((address_space(1))) const void* glb_ptr_t;
 // 257 us: with one wavefront per SIMD nothing covers the operand reads from
 // LDS.
 // GROUPED: see GroupTiles (gemm_tiles.h).
-template <bool SWAP, int NT, int WN, int DENSE = 0, bool GROUPED = false>
-__global__ void __launch_bounds__(128 * WN, WN == 2 ? 2 : 1)
+template <bool SWAP, int NT, int WN, int DENSE = 0, bool GROUPED = false,
+          int MT = kRowsMT>
+__global__ void __launch_bounds__(128 * WN, MT < 8 ? 3 : WN == 2 ? 2 : 1)
 rows_gemm_direct_kernel(RowsGemmArgs g) {
-  constexpr int MT = kRowsMT, BM = 32 * MT, ATILES = 2 * MT;
+  constexpr int BM = 32 * MT, ATILES = 2 * MT;
   constexpr int WAVES = 2 * WN;         // 2 rows of WN wavefronts
   constexpr int BN = WN * NT * 16;      // columns of the workgroup tile
   constexpr int AL = ATILES / WAVES;    // activation tiles a wavefront loads per stage
@@ -538,13 +539,13 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
     _Pragma("unroll") for (int i = 0; i < WL; ++i)                             \
       __builtin_amdgcn_global_load_lds(                                        \
           (glb_ptr_t)(wtile[i] + (size_t)(kt_) * 1024),                        \
-          (lds_ptr_t)&S_[ATILES + (wave + WAVES * i) % WTILES][0], 16, 0, 0);      \
+          (lds_ptr_t)&S_[ATILES + (wave + WAVES * i) % WTILES][0], 16, 0, 0);  \
   } while (0)
 #define T5D_ROWS_MULTIPLY(S_)                                                  \
   do {                                                                         \
     FragR wb[NT];                                                              \
     _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                          \
-      wb[nt].u = S_[ATILES + wn * NT + nt][lane];                                  \
+      wb[nt].u = S_[ATILES + wn * NT + nt][lane];                              \
     _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) {                        \
       FragR xa;                                                                \
       xa.u = S_[wm * MT + mt][read_slot];                                      \
@@ -613,7 +614,7 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
 
 using namespace t5d;
 
-// Three workgroup tiles.  256 x 256 (8 wavefronts, one workgroup per CU)
+// Three widths of workgroup tile.  256 x 256 (8 wavefronts, one workgroup per CU)
 // halves the operand bytes per flop of 256 x 128 (4 wavefronts, two per CU)
 // and measures 3-11 % faster whenever its workgroups fill the 256 CUs
 // evenly; 256 x 192 (8 wavefronts of 128 x 48) is for the shapes where
@@ -641,6 +642,41 @@ extern "C" int t5d_gemm_rows_tile(int w_dtype, int64_t M, int K, int N) {
   return pick;
 }
 
+// Rows of the 128-column tile of bfloat16 weights.  A workgroup of 256 rows lasts as
+// long on an empty chip as on a full one (its k-steps follow one another), so while
+// there are fewer workgroups than CUs they are made lower: 128 rows, or 64.  Results
+// have the same bits.  Measured, us with 256 / 128 / 64 rows:
+//   600 x 2048 x 768 residual  34.6 / 20.8 / 16.7   (15 rows of workgroups of 64)
+//   2000 x 2048 x 768          35.3 / 22.5 / 17.6
+//   1000 x 5120 x 2048         70.9 / 45.5 / 39.6
+//   600 x 768 x 4096 gated     16.9 / 11.3 / 13.4
+//   4000 x 768 x 768           17.7 / 13.1 / 14.2
+// and no gain from where 128 rows give more than one workgroup per CU (8192 x 1024 x
+// 1024, 512 of them: 22.7 / 22.6 / 26.0; 1000 x 2048 x 5120, 320: 33.3 / 37.1 / 36.5).
+static int rows_of_tile(int M, int N) {
+  const int n_blocks = (N + kRowsBN - 1) / kRowsBN;
+  if ((int64_t)((M + 63) / 64) * n_blocks <= 256) return 64;
+  if ((int64_t)((M + 127) / 128) * n_blocks <= 256) return 128;
+  return 256;
+}
+
+// rows_gemm_direct_kernel with 128 columns and the rows that suit the shape.
+template <bool SWAP, int DENSE>
+static void launch_rows_128(hipStream_t s, const RowsGemmArgs& g) {
+  const int rows = rows_of_tile(g.M, g.N);
+  const dim3 grid((unsigned)((g.M + rows - 1) / rows) *
+                  ((g.N + kRowsBN - 1) / kRowsBN));
+  if (rows == 64)
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<SWAP, kRowsNT, 2, DENSE, false, 2>),
+                       grid, dim3(256), 0, s, g);
+  else if (rows == 128)
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<SWAP, kRowsNT, 2, DENSE, false, 4>),
+                       grid, dim3(256), 0, s, g);
+  else
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<SWAP, kRowsNT, 2, DENSE>), grid,
+                       dim3(256), 0, s, g);
+}
+
 // Picks the workgroup tile (tile 0) and launches checked arguments.
 static int launch_rows(hipStream_t s, int w_dtype, const RowsGemmArgs& g,
                        int tile) {
@@ -661,8 +697,7 @@ static int launch_rows(hipStream_t s, int w_dtype, const RowsGemmArgs& g,
       hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 4, D_>),     \
                          dim3((unsigned)wgs256), dim3(512), 0, s, g);         \
     else if (g.K >= 64)                                                       \
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 2, D_>),     \
-                         grid, block, 0, s, g);                               \
+      launch_rows_128<true, D_>(s, g);                                        \
     else                                                                      \
       hipLaunchKernelGGL((rows_gemm_kernel<bf16_t, true, D_>), grid, block, 0, \
                          s, g);                                               \
@@ -689,11 +724,9 @@ static int launch_rows(hipStream_t s, int w_dtype, const RowsGemmArgs& g,
                          wblock, 0, s, g);
   } else if (w_dtype == T5D_BF16 && g.K >= 64) {
     if (swap)
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 2>), grid,
-                         block, 0, s, g);
+      launch_rows_128<true, 0>(s, g);
     else
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<false, kRowsNT, 2>), grid,
-                         block, 0, s, g);
+      launch_rows_128<false, 0>(s, g);
   } else if (w_dtype == T5D_BF16) {
     if (swap)
       hipLaunchKernelGGL((rows_gemm_kernel<bf16_t, true>), grid, block, 0, s, g);

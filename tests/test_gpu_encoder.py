@@ -137,6 +137,46 @@ def test_gemm_rows_plain_entry_point(ops):
     ops.gemm_rows(a, pw, tile=4)
 
 
+@pytest.mark.parametrize('M', [129, 191, 192, 193, 640, 1000, 4104])
+@pytest.mark.parametrize('K,N', [(64, 16), (96, 208), (160, 832)])
+def test_gemm_rows_of_low_tiles(ops, M, K, N):
+  """Tiles of 64, 128 and 256 rows (by the number of workgroups) at their edges: the bits
+  of the 256 x 256 tile, which adds up K in the same order, and of the whole in parts."""
+  rs = np.random.RandomState(M + N)
+  a = dev(rs.randn(M, K).astype(np.float32), torch.bfloat16)
+  w0, w1 = (dev((rs.randn(K, N) / np.sqrt(K)).astype(np.float32)) for _ in range(2))
+  plain = ops.pack_weight(w0, torch.bfloat16)
+  gated = ops.pack_weight(w0, torch.bfloat16, gate_kernel=w1)
+  res = dev(rs.randn(M, N).astype(np.float32), torch.bfloat16)
+  for w, kw in ((plain, {}), (plain, {'residual': res}), (gated, {})):
+    assert torch.equal(ops.gemm_rows(a, w, tile=1, **kw),
+                       ops.gemm_rows(a, w, tile=2, **kw))
+  want = a.float() @ w0.to(torch.bfloat16).float()
+  wide = ops.dense(a, plain, out_dtype=torch.float32)
+  assert bool(((wide - want).abs() <= 1e-5 * (1 + want.abs())).all())
+  assert torch.equal(ops.dense(a, plain), wide.to(torch.bfloat16))
+  unit = ops.dense(a, gated, glu=(7.0, 1.702, 1.0))
+  parts = [ops.dense(a[m:m + 128].contiguous(), gated, glu=(7.0, 1.702, 1.0))
+           for m in range(0, M, 128)]
+  # few rows are added up in another split of K: one bfloat16 step, or the sums' own noise
+  parts = torch.cat(parts).float()
+  assert bool(((unit.float() - parts).abs() <= 2.0**-7 * parts.abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize('B,E,H', [(1, 132, 1), (5, 60, 4), (3, 344, 13)])
+def test_gemm_rows_head_layouts_of_low_tiles(ops, B, E, H):
+  from t5x_amd import _lib
+  rs = np.random.RandomState(E)
+  a = dev(rs.randn(B * E, 96).astype(np.float32), torch.bfloat16)
+  pw = ops.pack_weight(dev((rs.randn(96, 64 * H) / 10).astype(np.float32)),
+                       torch.bfloat16)
+  Ep = (E + 31) // 32 * 32
+  rows = ops.gemm_rows(a, pw, tile=1).view(B, E, H, 64)
+  keys, vals = (ops.gemm_rows(a, pw, layout=l, E=E, Ep=Ep, tile=1)
+                for l in (_lib.OUT_HEADS_KEY, _lib.OUT_HEADS_VALUE))
+  _check_head_layouts(ops, rows, keys, vals, B, E, Ep, H)
+
+
 def _check_head_layouts(ops, rows, keys, vals, B, E, Ep, H):
   plain_k = torch.zeros((B, H, Ep, 64), dtype=rows.dtype, device='cuda')
   plain_k[:, :, :E] = rows.permute(0, 2, 1, 3)
