@@ -897,6 +897,50 @@ def test_cross_attention_step(ops, dt, B, beams, H, E):
                              rtol=TOL[dt])
 
 
+@pytest.mark.parametrize('beams', [1, 2, 3, 8])
+@pytest.mark.parametrize('E', [4, 60, 64, 132, 256, 260, 1020])
+def test_float32_cross_attention_reads_no_position_past_the_length(ops, E, beams):
+  """Lengths that no read divides, NaN in keys and values past them.  Bound: float32
+  sums of 64 products and of up to 1020 values of size 1, 2^-24 each step: 1e-5."""
+  rs = np.random.RandomState(E + beams)
+  B, H, D = 3, 2, 64
+  lens = np.array([E, max(2, E - 5), 1], np.int32)
+  k, v = rs.randn(B, H, E, D), rs.randn(B, H, D, E)
+  q = 0.125 * rs.randn(B * beams, H * D)
+  for b, n in enumerate(lens):
+    k[b, :, n:], v[b, :, :, n:] = np.nan, np.nan
+  out = host(ops.cross_attention_step(
+      dev(q, torch.float32), dev(k, torch.float32), dev(v, torch.float32), dev(lens),
+      beams)).reshape(B, beams, H, D)
+  for b, n in enumerate(lens):
+    s = np.einsum('qhd,hkd->qhk', q.reshape(B, beams, H, D)[b], k[b, :, :n])
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = np.einsum('qhk,hdk->qhd', p / p.sum(-1, keepdims=True), v[b, :, :, :n])
+    np.testing.assert_allclose(out[b], want, atol=1e-5)
+
+
+@pytest.mark.parametrize('L,t', [(32, 0), (64, 63), (260, 258), (512, 511), (1024, 3),
+                                 (1024, 1023)])
+def test_float32_self_attention_step_of_one_to_sixteen_wavefronts(ops, L, t):
+  rs = np.random.RandomState(L + t)
+  R, H, D = 2, 3, 64
+  qkv = rs.randn(R, 3, H, D)
+  qkv[:, 0] *= 0.125
+  ck, cv = rs.randn(R, H, D, L), rs.randn(R, H, D, L)
+  bias = rs.randn(H, L)
+  dk, dv = dev(ck, torch.float32), dev(cv, torch.float32)
+  out = host(ops.self_attention_step(
+      dev(qkv.reshape(R, -1), torch.float32), dk, dv, dev(bias, torch.float32),
+      torch.tensor(t, dtype=torch.int32, device='cuda'))).reshape(R, H, D)
+  ck[..., t], cv[..., t] = qkv[:, 1], qkv[:, 2]
+  np.testing.assert_array_equal(host(dk), ck.astype(np.float32))
+  np.testing.assert_array_equal(host(dv), cv.astype(np.float32))
+  s = np.einsum('rhd,rhdj->rhj', qkv[:, 0], ck[..., :t + 1]) + bias[:, t::-1][:, :t + 1]
+  p = np.exp(s - s.max(-1, keepdims=True))
+  want = np.einsum('rhj,rhdj->rhd', p / p.sum(-1, keepdims=True), cv[..., :t + 1])
+  np.testing.assert_allclose(out, want, atol=1e-5)  # as above
+
+
 @pytest.mark.parametrize('B,beams,H,E', [(3, 4, 2, 512), (32, 4, 12, 512),
                                          (40, 1, 12, 256), (64, 1, 16, 512),
                                          (20, 2, 12, 96)])
