@@ -562,6 +562,22 @@ recurrence_chunk_kernel(RecArgs g) {
     reinterpret_cast<float4*>(p)[at] = make_float4(v[0], v[1], v[2], v[3]);
   };
   const f32x4_v zero = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+  // The products multiply the zeros above the diagonals of T and M by what later
+  // tokens hold, which is no zero where that is infinite or NaN: an operand with such
+  // a value goes down its column over s <= t alone, so that a token never reaches an
+  // earlier one, as on the token by token path.
+  const auto not_finite = [](const float (&v)[4]) {
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bad |= !(fabsf(v[i]) < INFINITY);
+    return __builtin_amdgcn_ballot_w64(bad) != 0;
+  };
+  const auto down = [](const float (&row)[C], int t, const float* p, int stride) {
+    float sum = 0.f;
+#pragma unroll 1
+    for (int s = 0; s <= t; ++s) sum = fmaf(row[s], p[s * stride], sum);
+    return sum;
+  };
   float tm[4], bm[4], mm[4];  // rows x of T, B and M, columns 4 g + i
   four(&s_b[x][4 * g4], bm);
 #pragma unroll
@@ -571,10 +587,25 @@ recurrence_chunk_kernel(RecArgs g) {
     float tc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) tc[i] = s_t[4 * g4 + i][x];
-    const f32x4_v m = times(tc, bm, zero);  // M^T: rows 4 g + i, column x
+    if (not_finite(tc)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) mm[i] = m[i];
+      for (int i = 0; i < 4; ++i) {
+        mm[i] = 0.f;
+#pragma unroll 1
+        for (int k = 4 * g4 + i; k <= x; ++k)
+          mm[i] = fmaf(s_b[x][k], s_t[k][4 * g4 + i], mm[i]);
+      }
+    } else {
+      const f32x4_v m = times(tc, bm, zero);  // M^T: rows 4 g + i, column x
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mm[i] = m[i];
+    }
+    // M for `down` (A is no longer needed; every wavefront writes the same)
+    *reinterpret_cast<float4*>(&s_a[x][4 * g4]) =
+        make_float4(mm[0], mm[1], mm[2], mm[3]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
+  const float(*s_m)[C] = DELTA ? s_a : s_b;
   for (int tile = wave; tile < DP / 16; tile += 4) {
     const int at = tile * 64 + lane;
     f32x4_v q;
@@ -590,8 +621,19 @@ recurrence_chunk_kernel(RecArgs g) {
         r[i] = s_k[o + i * LS];
         minus[i] = -r[i];
       }
-      put(w + lay.wk(), at, times(r, tm, zero));
-      q = times(minus, mm, q);
+      if (not_finite(r)) {
+        f32x4_v k;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float* column = s_k + 16 * tile + 4 * g4 + i;
+          k[i] = down(s_t[x], x, column, LS);
+          q[i] -= down(s_m[x], x, column, LS);
+        }
+        put(w + lay.wk(), at, k);
+      } else {
+        put(w + lay.wk(), at, times(r, tm, zero));
+        q = times(minus, mm, q);
+      }
     }
     put(w + lay.qs(), at, q);
     put(w + lay.kh(), at,
@@ -602,9 +644,20 @@ recurrence_chunk_kernel(RecArgs g) {
     float v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = s_v[(4 * g4 + i) * vs + 16 * tile + x];
-    put(w + lay.us(), at,
-        DELTA ? times(tm, v, zero) : (f32x4_v){v[0], v[1], v[2], v[3]});
-    put(w + lay.os(), at, times(mm, v, zero));
+    f32x4_v u = (f32x4_v){v[0], v[1], v[2], v[3]}, y;
+    if (not_finite(v)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float* column = s_v + 16 * tile + x;
+        if (DELTA) u[i] = down(s_t[4 * g4 + i], 4 * g4 + i, column, vs);
+        y[i] = down(s_m[4 * g4 + i], 4 * g4 + i, column, vs);
+      }
+    } else {
+      if (DELTA) u = times(tm, v, zero);
+      y = times(mm, v, zero);
+    }
+    put(w + lay.us(), at, u);
+    put(w + lay.os(), at, y);
   }
 }
 

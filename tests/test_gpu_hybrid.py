@@ -546,6 +546,33 @@ def test_recurrence_chunks_of_hard_inputs(dt, delta, D, Dv, taps, kind):
   assert rel(r.run([(0, 0, T)], [(x, z)], 3), want) < r.tol
 
 
+@pytest.mark.parametrize('dt', DTYPES)
+@pytest.mark.parametrize('delta,D,Dv,taps', [(True, 128, 40, 4), (False, 64, 48, 0),
+                                             (True, 200, 20, 0), (False, 40, 72, 4)])
+@pytest.mark.parametrize('what', ['q', 'k', 'v', 'beta', 'decay'])
+@pytest.mark.parametrize('value', [float('nan'), float('inf')])
+def test_a_token_that_is_not_finite_leaves_earlier_ones_alone(dt, delta, D, Dv, taps,
+                                                              what, value):
+  """In the middle of a chunk: the tokens before it as without it, and what is finite
+  where the tokens are taken one by one is finite."""
+  r = Recurrence(dt, delta, 2, 1, D, Dv, taps, 1, seed=D)
+  T, at = 77, 41
+  x, z = r.sequence(T)
+  want = r.oracle((x, z))
+  if what == 'decay':
+    z[at, r.low_off[0] + 3] = value
+  else:
+    x[at, r.off[['q', 'k', 'v', 'beta'].index(what)] + (what != 'beta')] = value
+  got, alone = (r.run([(0, 0, T)], [(x, z)], variant) for variant in (3, 2))
+  assert rel(got[:at], want[:at]) < r.tol
+  # (not the other way round for an infinite value: one by one it reaches the output
+  # through all channels of the state, whose infinities of both signs make a NaN, in a
+  # chunk through one product with its key, which stays infinite)
+  assert np.isfinite(got[np.isfinite(alone)]).all()
+  if np.isnan(value):
+    assert np.array_equal(np.isfinite(got), np.isfinite(alone))
+
+
 def seq_cols(x, at, n):
   return x[:, at:at + n]
 
