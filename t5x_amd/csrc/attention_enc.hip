@@ -344,8 +344,9 @@ __global__ void __launch_bounds__(256, 3)
 enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   constexpr int MT = 2, KB = 64;
   __shared__ uint4 s_k0[512], s_v0[512], s_k1[512], s_v1[512];
-  // from 16 entries before the table (queries past the end) to 64 behind it (keys
-  // past the end): neither's scores are used
+  // 16 entries before the table (zeros: queries past the end, which are not stored but
+  // do decide with the others of their wavefront when maxima are raised) and 64 behind
+  // it (keys past the end, whose scores are replaced before they are looked at)
   __shared__ float s_bias[16 + 2 * kMaxEncLen + 64];
   __shared__ uint32_t s_valid[kMaxEncLen / 32 + 2];
   // consecutive block ids go round-robin over the 8 XCDs: the tiles of one (item,
@@ -393,6 +394,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   };
   fetch(0, s_k0, s_v0);
 
+  if (threadIdx.x < 16) s_bias[threadIdx.x] = 0.f;
   for (int i = threadIdx.x; i < 2 * E - 1; i += 256)
     s_bias[16 + i] = bf16_to_f32(a.bias[(size_t)h * (2 * E - 1) + i]);
   int n = a.len[b];
