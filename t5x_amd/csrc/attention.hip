@@ -324,8 +324,12 @@ attn_step_kernel(AttnArgs a) {
 // dim for the value product (a lane reads its own row, 64 positions of it).  What
 // bounds it at the few rows it is used for is the wait for memory: keys, and values
 // where registers allow (WM <= 4 wavefronts), are requested before the queries are
-// looked at (one value at a time behind the probabilities: 8 rows of 6 heads over 64
-// positions 9.7 us, now 6.8).
+// looked at, and nothing past the length.  us per launch, with one value at a time
+// behind the probabilities / with requests for all positions / now:
+//   8 items, 6 heads, 64 positions, all valid    8.6 / 5.9 / 5.5
+//   64 items, 12 heads, 256, all valid            69 / 22.3 / 20.8
+//   64 items, 12 heads, 256, 40 valid            7.7 / 20.2 / 6.2
+//   64 items, 12 heads, 512, 60 valid           11.1 / 35.2 / 7.6
 template <int NQ, int WM>
 __global__ void __launch_bounds__(64 * WM)
 cross_attn_f32_kernel(AttnArgs a) {
@@ -333,16 +337,19 @@ cross_attn_f32_kernel(AttnArgs a) {
   __shared__ float s_red[WM][NQ];
   __shared__ float s_p[NQ][WM * 64];
   __shared__ float s_out[WM][NQ][kD];
-  T5D_GATED(a.gate);
+  T5D_GATE_READ(a.gate);
   const int h = blockIdx.x, b = blockIdx.y;
+  int n = a.index[b];  // (one wait for both)
+  T5D_GATE_TEST();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nwaves = blockDim.x >> 6;
   const int HD = a.H * kD;
-  int n = a.index[b];
   n = n < 0 ? 0 : (n > a.S ? a.S : n);
   bool uniform = false;
   if (n == 0) { uniform = true; n = a.S; }
+  // wavefronts without a position leave (barriers wait for those that are there)
+  if (wave * 64 >= n) return;
+  const int nwaves = (n + 63) >> 6, threads = 64 * nwaves;
   const float* kbase = reinterpret_cast<const float*>(a.k) +
                        ((size_t)b * a.H + h) * (size_t)a.S * kD;
   const float* vbase = reinterpret_cast<const float*>(a.v) +
@@ -350,27 +357,35 @@ cross_attn_f32_kernel(AttnArgs a) {
   const float* qbase = reinterpret_cast<const float*>(a.q);
   const int j = wave * 64 + lane;
   const int jb = wave * 64, je = min(n, jb + 64);
-  // keys of this lane's position, values of this lane's row
+  // keys of this lane's position, values of this lane's row: nothing past the length
+  // but the last position's keys again and the rest of its four values
   float4 key[kD / 4], value[16];
   const auto request_keys = [&] {
-    const float4* row = reinterpret_cast<const float4*>(
-        kbase + (size_t)min(j, a.S - 1) * kD);
+    const float4* row =
+        reinterpret_cast<const float4*>(kbase + (size_t)min(j, n - 1) * kD);
 #pragma unroll
     for (int c = 0; c < kD / 4; ++c) key[c] = row[c];
   };
   // (rows of a multiple of 4 floats, aligned: checked by the caller)
   const auto request_values = [&] {
-    const float* row = vbase + (size_t)lane * a.S;
+    const float* row = vbase + (size_t)lane * a.S + jb;
+    if (jb + 64 <= n) {
 #pragma unroll
-    for (int c = 0; c < 16; ++c)
-      value[c] = *reinterpret_cast<const float4*>(row + min(jb + 4 * c, a.S - 4));
+      for (int c = 0; c < 16; ++c) value[c] = *reinterpret_cast<const float4*>(row + 4 * c);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 16; ++c) {
+        value[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (jb + 4 * c < n) value[c] = *reinterpret_cast<const float4*>(row + 4 * c);
+      }
+    }
   };
   constexpr bool kAhead = WM <= 4;
   if constexpr (kAhead) {
     request_keys();
     request_values();
   }
-  for (int e = threadIdx.x; e < NQ * kD; e += blockDim.x) {
+  for (int e = threadIdx.x; e < NQ * kD; e += threads) {
     const int qi = e / kD, d = e % kD;
     s_q[qi][d] = qi < a.nq
                      ? qbase[(size_t)(b * a.nq + qi) * a.q_stride + h * kD + d]
@@ -446,7 +461,7 @@ cross_attn_f32_kernel(AttnArgs a) {
 #pragma unroll
   for (int qi = 0; qi < NQ; ++qi) s_out[wave][qi][lane] = o[qi];
   __syncthreads();
-  for (int e = threadIdx.x; e < NQ * kD; e += blockDim.x) {
+  for (int e = threadIdx.x; e < NQ * kD; e += threads) {
     const int qi = e / kD, d = e % kD;
     if (qi >= a.nq) continue;
     float acc = s_out[0][qi][d];
