@@ -5,8 +5,8 @@
 //
 // Two kernels on the matrix cores, chosen by length: enc_attn_ring_kernel up to 128
 // positions (64 queries per workgroup, scores kept in registers between a pass over
-// the keys and one over the values), enc_attn_tile_kernel beyond (128 queries, one
-// pass).  Both form S^T = K Q^T, keys as matrix rows, so that a lane ends up with 4
+// the keys and one over the values), enc_attn_tile_kernel beyond (128 queries or 64,
+// one pass).  Both form S^T = K Q^T, keys as matrix rows, so that a lane ends up with 4
 // consecutive keys of ONE query, which is the operand order of out^T = V^T P^T; V is
 // given transposed in 32-key blocks ([B, H, Ep / 32, 64, 32], what t5d_gemm_rows'
 // value layout writes).  Scores are rounded where the reference rounds them.
@@ -317,7 +317,7 @@ enc_attn_ring_kernel(EncAttnArgs a) {
 }
 
 // ---- beyond 128 positions: one pass ----------------------------------------------
-// A workgroup takes 128 queries of one (item, head), a wavefront 32, and walks 64
+// A workgroup takes 64 MT queries of one (item, head), a wavefront 16 MT, and walks 64
 // keys at a time once: scores as above (rounded where the reference rounds them),
 // weights relative to a running maximum that is raised only when a score passes it
 // by kMaxSlack powers of two, rounded to bfloat16 as they enter the second product
@@ -340,9 +340,10 @@ enc_attn_ring_kernel(EncAttnArgs a) {
 constexpr float kMaxSlack = 8.0f;
 constexpr float kLog2eE = 1.4426950408889634f;
 
+template <int MT>  // 16 queries each per wavefront: 2 or 1
 __global__ void __launch_bounds__(256, 3)
 enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
-  constexpr int MT = 2, KB = 64;
+  constexpr int KB = 64, QW = 16 * MT;  // keys per tile, queries per wavefront
   __shared__ uint4 s_k0[512], s_v0[512], s_k1[512], s_v1[512];
   // 16 entries before the table (zeros: queries past the end, which are not stored but
   // do decide with the others of their wavefront when maxima are raised) and 64 behind
@@ -407,7 +408,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
     if (a.valid && i < words) prefix &= a.valid[(size_t)b * words + i];
     s_valid[i] = prefix;
   }
-  const int q0 = tile * 128 + wave * 32;
+  const int q0 = (tile * 4 + wave) * QW;
   FragE qb[MT][2];
   int qi[MT];
 #pragma unroll
@@ -425,14 +426,16 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   bool my_valid = false, my_padding = false;  // all queries are
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
-    const int qw = tile * 128 + w * 32;
-    const uint32_t want = qw + 32 <= E ? 0xffffffffu : qw < E ? (1u << (E - qw)) - 1 : 0;
-    const bool valid = qw < E && (s_valid[qw >> 5] & want) == want;
+    const int qw = (tile * 4 + w) * QW;
+    const uint32_t all = MT == 2 ? 0xffffffffu : 0xffffu;
+    const uint32_t want = qw + QW <= E ? all : qw < E ? (1u << (E - qw)) - 1 : 0;
+    const uint32_t there = qw < E ? (s_valid[qw >> 5] >> (qw & 31)) & want : 0;
+    const bool valid = qw < E && there == want;
     const int keys = qw >= E ? 0 : valid ? n : E;
     if (w == wave) {
       my_keys = keys;
       my_valid = valid;
-      my_padding = qw >= E || (s_valid[qw >> 5] & want) == 0;
+      my_padding = there == 0;
     }
     wg_keys = max(wg_keys, keys);
   }
@@ -706,6 +709,23 @@ enc_attn_f32_kernel(EncAttnF32Args a) {
   a.out[((size_t)b * a.E + e) * HD + h * kHeadDim + lane] = acc;
 }
 
+// Whether enc_attn_tile_kernel takes 64 queries per workgroup: while those are at most
+// 4 per CU (3 run at a time).  A workgroup of 128 lasts longer than one of 64, whatever
+// else the chip does, and longer still if some of its queries are padding (they then
+// walk all keys beside the others'): one text of 500 tokens had been faster two passes
+// and 64 queries at a time.  Measured, us with 128 / 64 (workgroups of 64):
+//   1 x 12 heads x 512, 300 and more valid (96)   17.9 / 13.4
+//   2 x 12 x 512, 128 and more (192)              18.7 / 13.6
+//   8 x 12 x 200, 80 and more (384)               10.6 / 10.7
+//   8 x 12 x 512, 200 and more (768)              26.9 / 21.6
+//   4 x 16 x 1032, 400 and more (1088)            53.4 / 49.7
+//   16 x 12 x 512, 200 and more (1536)            37.8 / 36.9
+//   32 x 12 x 200, 80 and more (1536)             20.0 / 22.6
+//   7 x 16 x 1032, 400 and more (1904)            71.5 / 73.8
+static bool one_pass_64(int B, int H, int E) {
+  return (int64_t)B * H * ((E + 63) / 64) <= 1024;
+}
+
 }  // namespace t5d
 
 using namespace t5d;
@@ -759,10 +779,15 @@ extern "C" int t5d_encoder_attention_variant(
     hipLaunchKernelGGL(enc_attn_ring_kernel<2>, dim3((E + 63) / 64, H, B), dim3(256),
                        0, as_stream(stream), a);
   } else {
-    const int tiles = (E + 127) / 128;
-    const unsigned groups = ((unsigned)B * H + 7) / 8 * 8 * tiles;
-    hipLaunchKernelGGL(enc_attn_tile_kernel, dim3(groups), dim3(256), 0,
-                       as_stream(stream), a, tiles);
+    const bool low = one_pass_64(B, H, E);
+    const int tiles = low ? (E + 63) / 64 : (E + 127) / 128;
+    const dim3 groups(((unsigned)B * H + 7) / 8 * 8 * tiles);
+    if (low)
+      hipLaunchKernelGGL(enc_attn_tile_kernel<1>, groups, dim3(256), 0,
+                         as_stream(stream), a, tiles);
+    else
+      hipLaunchKernelGGL(enc_attn_tile_kernel<2>, groups, dim3(256), 0,
+                         as_stream(stream), a, tiles);
   }
   T5D_CHECK_LAUNCH("t5d_encoder_attention");
   return T5D_OK;

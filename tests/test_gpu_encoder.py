@@ -264,13 +264,15 @@ def test_encoder_attention(ops, B, E, H):
   np.testing.assert_allclose(got, want, atol=2e-2, rtol=2**-6)
 
 
+@pytest.mark.parametrize('copies', [1, 24])
 @pytest.mark.parametrize('E', [128, 129, 159, 160, 192, 193, 257, 513])
-def test_encoder_attention_at_the_edges_of_its_tiles(ops, E):
+def test_encoder_attention_at_the_edges_of_its_tiles(ops, E, copies):
   """Lengths around 32 (a wavefront's queries, a block of values), 64 (a tile of
   keys) and 128 (a workgroup's queries), and items whose valid part ends at and
   around those edges, with every query of a wavefront valid, none, and some; in
   one item a padding token inside the text.  Scores climb along the keys, so the
-  running maximum is raised again and again."""
+  running maximum is raised again and again.  Many copies of the items are taken by
+  workgroups of 128 queries, few by workgroups of 64."""
   from t5x_amd import network
   H, lens = 2, np.array([E, 1, 32, 33, 64, 65, 96, 127], np.int32)
   B = len(lens)
@@ -289,11 +291,14 @@ def test_encoder_attention_at_the_edges_of_its_tiles(ops, E):
   v_t = torch.zeros((B, H, 64, (E + 31) // 32 * 32), dtype=torch.bfloat16,
                     device='cuda')
   v_t[..., :E] = dev(v, torch.bfloat16).permute(0, 2, 3, 1)
+  many = lambda x: x.repeat(copies, *[1] * (x.dim() - 1))
   out = ops.encoder_attention(
-      *(dev(x, torch.bfloat16).reshape(B * E, H * 64) for x in (q, k)),
-      ops.tile_cross_value(v_t), rel_bias, dev(lens),
-      valid_bits=ops.pack_valid_bits(dev(valid)))
-  np.testing.assert_allclose(host(out).reshape(B, E, H, 64), want, atol=2e-2,
+      *(many(dev(x, torch.bfloat16).reshape(B * E, H * 64)) for x in (q, k)),
+      many(ops.tile_cross_value(v_t)), rel_bias, many(dev(lens)),
+      valid_bits=many(ops.pack_valid_bits(dev(valid))))
+  out = out.reshape(copies, B, E, H, 64)
+  assert torch.equal(out, out[:1].expand_as(out))
+  np.testing.assert_allclose(host(out[0]), want, atol=2e-2,
                              rtol=2**-6)
 
 
@@ -320,20 +325,21 @@ def test_encoder_attention_repeated_launches(ops):
         assert torch.equal(first, again), (E, variant)
 
 
+@pytest.mark.parametrize('B', [2, 60])  # workgroups of 64 queries, of 128
 @pytest.mark.parametrize('E', [20, 100, 129, 135, 161, 1031, 1032, 1040])
-def test_encoder_attention_does_not_depend_on_what_lds_held(ops, E):
+def test_encoder_attention_does_not_depend_on_what_lds_held(ops, E, B):
   """Lengths whose last wavefront has queries past the end: the same bits whatever an
   earlier kernel (a dense layer whose operands are one value throughout) left in LDS.
   Scores of a standard deviation of 3 raise the running maxima again and again."""
   g = torch.Generator(device='cuda')
   g.manual_seed(E)
-  bf, B, H = torch.bfloat16, 2, 6
+  bf, H = torch.bfloat16, 6
   q, k = (torch.randn(B * E, H * 64, device='cuda', generator=g).to(bf)
           for _ in range(2))
   v_t = ops.tile_cross_value(
       torch.randn(B, H, 64, (E + 31) // 32 * 32, device='cuda', generator=g).to(bf))
   rel = (3 * torch.randn(H, 2 * E - 1, device='cuda', generator=g)).to(bf)
-  lens = torch.tensor([E, E - 1], dtype=torch.int32, device='cuda')
+  lens = torch.tensor([E, E - 1] * (B // 2), dtype=torch.int32, device='cuda')
   outs = []
   for left in (0.0, 1.0, -3e38, 3e38, float('nan')):
     a = torch.full((256 * 256, 96), left, dtype=bf, device='cuda')
