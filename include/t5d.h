@@ -312,9 +312,9 @@ int t5d_encoder_attention(void* stream, const void* q, const void* k,
                           void* out, int B, int H, int E, int Ep, int q_stride,
                           int k_stride);
 
-/* t5d_encoder_attention, with an argument that once chose between kernels: there is
- * one kernel per length (up to 128 positions, and beyond), so variant 0, 1 and, for
- * E <= 512, 2 give the same bits. */
+/* t5d_encoder_attention, with an argument that chooses nothing any more: the kernel
+ * follows from the sizes, so variant 0, 1 and, for E <= 512, 2 give the same bits.
+ * Kept for programs that pass it. */
 int t5d_encoder_attention_variant(void* stream, const void* q, const void* k,
                                   const void* v_t, const void* rel_bias,
                                   const int32_t* enc_len,

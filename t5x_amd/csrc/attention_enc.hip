@@ -3,10 +3,9 @@
 // (batch item, head), t5x/examples/t5/layers.py:52-129 with the encoder's
 // bidirectional bias (layers.py:560-677) and mask (network.py:325-328).
 //
-// Two kernels on the matrix cores, chosen by length: enc_attn_ring_kernel up to 128
-// positions (64 queries per workgroup, scores kept in registers between a pass over
-// the keys and one over the values), enc_attn_tile_kernel beyond (128 queries or 64,
-// one pass).  Both form S^T = K Q^T, keys as matrix rows, so that a lane ends up with 4
+// Two kernels on the matrix cores, chosen by length: enc_attn_short_kernel up to 64
+// positions (scores kept in registers between the keys and the values),
+// enc_attn_tile_kernel beyond (one pass over the keys, workgroups of 128 queries or 64).  Both form S^T = K Q^T, keys as matrix rows, so that a lane ends up with 4
 // consecutive keys of ONE query, which is the operand order of out^T = V^T P^T; V is
 // given transposed in 32-key blocks ([B, H, Ep / 32, 64, 32], what t5d_gemm_rows'
 // value layout writes).  Scores are rounded where the reference rounds them.
@@ -39,209 +38,163 @@ struct EncAttnArgs {
 
 constexpr int kMaxEncLen = 2048;
 
-// ---- up to 128 positions: scores kept in registers ------------------------------
-// The 16 x E scores of a wavefront fit its registers as bfloat16 pairs (they ARE
-// bfloat16 values at that point), so
-//   pass 1 forms the scores once, keeps them, and tracks max / sum;
-//   pass 2 turns the kept scores into P in registers, already in the layout
-//          of the matrix cores' B operand: a lane holds keys 4g .. 4g+3 of two
-//          neighbouring 16-key tiles, and the V^T operand is read from LDS in
-//          that same key order, so P never goes through LDS.
-// K (pass 1) and V^T (pass 2) are fetched once per workgroup, 64 keys = 8 KB
-// at a time, straight from memory into a ring of three LDS stages
-// (global_load_lds: lane l of an instruction lands at byte 16 l, so the
-// address each lane reads from picks the XOR swizzle that makes the operand
-// reads spread over the banks); the four wavefronts read their operand
-// fragments from there.  One barrier per 64 keys, placed by hand with the wait
-// for "all but my newest two loads"; the stages are separate arrays and the
-// loops are unrolled so that every stage is named at compile time.
+// ---- up to 64 positions: scores kept in registers -------------------------------
+// A wavefront's 16 queries against the one block of keys:
+//   the scores are formed once and kept as bfloat16 pairs (they ARE bfloat16 values
+//   at that point), their maximum and sum with them; then they are turned into P in
+//   registers, already in the layout of the matrix cores' B operand: a lane holds
+//   keys 4g .. 4g+3 of two neighbouring 16-key tiles, and the V^T operand is read
+//   from LDS in that same key order, so P never goes through LDS.
+// K and V^T are fetched once per workgroup, 8 KB each, straight from memory into LDS
+// (global_load_lds: lane l of an instruction lands at byte 16 l, so the address each
+// lane reads from picks the XOR swizzle that makes the operand reads spread over the
+// banks); the four wavefronts read their operand fragments from there.
 typedef __attribute__((address_space(3))) void* enc_lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* enc_glb_ptr_t;
 
-template <int MAXB>  // 64-key blocks: E <= 64 MAXB
+constexpr int kShortEnc = 64;  // its longest text
+
 __global__ void __launch_bounds__(256)
-enc_attn_ring_kernel(EncAttnArgs a) {
-  __shared__ uint4 s_r0[512];
-  __shared__ uint4 s_r1[512];
-  __shared__ uint4 s_r2[512];
-  __shared__ float s_bias[128 * MAXB + 16];
-  __shared__ uint32_t s_valid[2 * MAXB];
+enc_attn_short_kernel(EncAttnArgs a) {
+  __shared__ uint4 s_k[512], s_v[512];
+  __shared__ float s_bias[2 * kShortEnc + 16];
+  __shared__ uint32_t s_valid[2];
   // what a score is capped by, per key: [0] for a valid query (+inf for a
   // valid key, bf16(-1e10) for a masked one, -inf past E), [1] for a padded
   // query (bf16(-1e10) for every key that exists)
-  __shared__ __attribute__((aligned(16))) float s_lim[2][64 * MAXB + 16];
+  __shared__ __attribute__((aligned(16))) float s_lim[2][kShortEnc + 16];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, gq = lane >> 4;
   const int h = blockIdx.y, b = blockIdx.z;
   const int E = a.E;
+  const size_t row0 = (size_t)b * E;
+
+  // What this lane fetches of K: chunks (8 keys, 1 KB) wave and wave + 4; lane s
+  // lands at slot s & 7 of key s >> 3 and therefore reads piece (s & 7) ^ (s >> 3) of
+  // that key (past the end: the last key again).
+  const int k_r = lane >> 3, k_piece = (lane & 7) ^ k_r;
+  // ... and of V^T (two [64 d][32 keys] blocks, 4 KB each): chunks (16 rows d, 1 KB)
+  // wave and wave + 4; lane s lands at slot s & 3 of row s >> 2 and reads piece
+  // (s & 3) ^ ((row >> 1) & 1): one swizzle bit, so that the two pieces a lane needs
+  // (p and p + 2) stay 32 bytes apart and come with one two-address read, already in
+  // operand order.
+  const int v_r = lane >> 2, v_piece = (lane & 3) ^ ((v_r >> 1) & 1);
+  const char* kbase = reinterpret_cast<const char*>(a.k) + (size_t)h * 128 + k_piece * 16;
+  const char* vbase = reinterpret_cast<const char*>(a.vt) +
+                      ((size_t)b * a.H + h) * 128 * (size_t)a.Ep;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int c = wave + 4 * u;
+    const int key = min(8 * c + k_r, E - 1);
+    __builtin_amdgcn_global_load_lds(
+        (enc_glb_ptr_t)(kbase + (row0 + key) * (size_t)a.k_stride * 2),
+        (enc_lds_ptr_t)&s_k[64 * c], 16, 0, 0);
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int c = wave + 4 * u;
+    const int blk = min(c >> 2, (a.Ep >> 5) - 1);
+    __builtin_amdgcn_global_load_lds(
+        (enc_glb_ptr_t)(vbase + (size_t)blk * 4096 + (16 * (c & 3) + v_r) * 64 +
+                        v_piece * 16),
+        (enc_lds_ptr_t)&s_v[64 * c], 16, 0, 0);
+  }
+
   for (int i = threadIdx.x; i < 2 * E - 1; i += 256)
     s_bias[i] = bf16_to_f32(a.bias[(size_t)h * (2 * E - 1) + i]);
   int n = a.len[b];
   n = n < 0 ? 0 : (n > E ? E : n);
   const int words = (E + 31) >> 5;
-  for (int i = threadIdx.x; i < words; i += 256) {
-    const int left = n - 32 * i;
-    const uint32_t prefix =
-        left >= 32 ? 0xffffffffu : (left <= 0 ? 0u : ((1u << left) - 1u));
-    s_valid[i] = a.valid ? (a.valid[(size_t)b * words + i] & prefix) : prefix;
+  if (threadIdx.x < 2) {
+    const int left = n - 32 * threadIdx.x;
+    uint32_t prefix = left >= 32 ? 0xffffffffu : (left <= 0 ? 0u : ((1u << left) - 1u));
+    if (a.valid && (int)threadIdx.x < words)
+      prefix &= a.valid[(size_t)b * words + threadIdx.x];
+    s_valid[threadIdx.x] = prefix;
   }
-  __syncthreads();
-  const float kMasked = -9999220736.0f;  // bf16(-1e10) exactly, layers.py:309-311
-  for (int i = threadIdx.x; i < 64 * MAXB + 16; i += 256) {
-    const bool ok = i < E && ((s_valid[i >> 5] >> (i & 31)) & 1u) != 0;
-    s_lim[0][i] = ok ? INFINITY : (i < E ? kMasked : -INFINITY);
-    s_lim[1][i] = i < E ? kMasked : -INFINITY;
-  }
-  __syncthreads();
-  // Key tiles each wavefront walks (the valid prefix
-  // when all of its 16 queries are valid — the keys beyond add exact zeros —
-  // else every key; none when its queries lie beyond E) and what the
-  // workgroup as a whole must fetch, in 64-key blocks.
-  const int all_tiles = (E + 15) >> 4;
-  int my_tiles = 0, wg_tiles = 0;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const int qw = blockIdx.x * 64 + w * 16;
-    int t = 0;
-    if (qw < E) {
-      const bool all_valid =
-          qw + 15 < E &&
-          ((s_valid[qw >> 5] >> (qw & 31)) & 0xffffu) == 0xffffu;
-      t = all_valid ? (n + 15) >> 4 : all_tiles;
-    }
-    if (w == wave) my_tiles = t;
-    wg_tiles = max(wg_tiles, t);
-  }
-  my_tiles = __builtin_amdgcn_readfirstlane(my_tiles);
-  const int nb = __builtin_amdgcn_readfirstlane((wg_tiles + 3) >> 2);
-  const int q0 = blockIdx.x * 64 + wave * 16;
-  const size_t row0 = (size_t)b * E;
-
+  const int q0 = wave * 16;
   const int qi = min(q0 + l16, E - 1);
   FragE qb[2];
 #pragma unroll
   for (int c = 0; c < 2; ++c)
     qb[c].u = *reinterpret_cast<const uint4*>(
         a.q + (row0 + qi) * a.q_stride + h * 64 + 32 * c + 8 * gq);
+  __syncthreads();
+  const float kMasked = -9999220736.0f;  // bf16(-1e10) exactly, layers.py:309-311
+  if (threadIdx.x < kShortEnc + 16) {
+    const int i = threadIdx.x;
+    const bool ok = i < E && ((s_valid[i >> 5] >> (i & 31)) & 1u) != 0;
+    s_lim[0][i] = ok ? INFINITY : (i < E ? kMasked : -INFINITY);
+    s_lim[1][i] = i < E ? kMasked : -INFINITY;
+  }
+  // Key tiles this wavefront walks: the valid prefix when all of its 16 queries are
+  // valid (the keys beyond add exact zeros), else every key; none when its queries
+  // lie beyond E.
+  int my_tiles = 0;
+  if (q0 < E) {
+    const bool all_valid =
+        q0 + 15 < E && ((s_valid[q0 >> 5] >> (q0 & 31)) & 0xffffu) == 0xffffu;
+    my_tiles = ((all_valid ? n : E) + 15) >> 4;
+  }
+  my_tiles = __builtin_amdgcn_readfirstlane(my_tiles);
   const bool q_valid =
-      q0 + l16 < E &&
-      ((s_valid[(q0 + l16) >> 5] >> ((q0 + l16) & 31)) & 1u) != 0;
+      q0 + l16 < E && ((s_valid[(q0 + l16) >> 5] >> ((q0 + l16) & 31)) & 1u) != 0;
+  // All loads have landed; behind the barrier everyone's have.
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+
   // this lane's 4 keys of key tile kt: bias and cap at [16 kt .. 16 kt + 3].
   // Masking is a minimum with the cap: a score never lies below -1e10, so
   // min(x, bf16(-1e10)) is the reference's masked value, min(x, -inf) removes
   // a key that does not exist, min(x, +inf) keeps x.
   const float* bias_g = s_bias + (E - 1) - qi + 4 * gq;
   const float* lim_g = s_lim[q_valid ? 0 : 1] + 4 * gq;
-
-  // What this lane fetches of a 64-key block of K: chunks (8 keys, 1 KB)
-  // wave and wave + 4; lane s lands at slot s & 7 of key s >> 3 and therefore
-  // reads piece (s & 7) ^ (s >> 3) of that key.
-  const int k_r = lane >> 3, k_piece = (lane & 7) ^ k_r;
-  const char* kbase = reinterpret_cast<const char*>(a.k) +
-                      (size_t)h * 128 + k_piece * 16;
-  // ... and of a 64-key block of V^T (two [64 d][32 keys] blocks, 4 KB each):
-  // chunks (16 rows d, 1 KB) wave and wave + 4; lane s lands at slot s & 3 of
-  // row s >> 2 and reads piece (s & 3) ^ ((row >> 1) & 1): one swizzle bit, so
-  // that the two pieces a lane needs in pass 2 (p and p + 2) stay 32 bytes
-  // apart and come with one two-address read, already in operand order.
-  const int v_r = lane >> 2, v_piece = (lane & 3) ^ ((v_r >> 1) & 1);
-  const char* vbase = reinterpret_cast<const char*>(a.vt) +
-                      ((size_t)b * a.H + h) * 128 * (size_t)a.Ep;
-  const int v_blocks = a.Ep >> 5;
-#define T5D_ENC_ISSUE_K(i_, S_)                                                \
-  do {                                                                         \
-    _Pragma("unroll") for (int u = 0; u < 2; ++u) {                            \
-      const int c = wave + 4 * u;                                              \
-      const int key = min(64 * (i_) + 8 * c + k_r, E - 1);                     \
-      __builtin_amdgcn_global_load_lds(                                        \
-          (enc_glb_ptr_t)(kbase + (row0 + key) * (size_t)a.k_stride * 2),      \
-          (enc_lds_ptr_t)&S_[64 * c], 16, 0, 0);                               \
-    }                                                                          \
-  } while (0)
-#define T5D_ENC_ISSUE_V(i_, S_)                                                \
-  do {                                                                         \
-    _Pragma("unroll") for (int u = 0; u < 2; ++u) {                            \
-      const int c = wave + 4 * u;                                              \
-      const int blk = min(2 * (i_) + (c >> 2), v_blocks - 1);                  \
-      __builtin_amdgcn_global_load_lds(                                        \
-          (enc_glb_ptr_t)(vbase + (size_t)blk * 4096 +                         \
-                          (16 * (c & 3) + v_r) * 64 + v_piece * 16),           \
-          (enc_lds_ptr_t)&S_[64 * c], 16, 0, 0);                               \
-    }                                                                          \
-  } while (0)
-  // all but my newest two loads (the next block) have landed and my reads of
-  // LDS have returned (vmcnt(2) lgkmcnt(0): a barrier orders issued
-  // instructions, not completed LDS reads); after the barrier so have
-  // everyone's, and everyone is done with the stage that the loads issued
-  // next overwrite.  Nothing in a step is conditional — the loads past the
-  // last block fetch clamped addresses into a stage nobody reads, every
-  // wavefront forms all four key tiles of a block — and the only branch is
-  // the loop exit in front of a step: where two paths meet between a load
-  // into LDS and a read of LDS the compiler waits for every load in flight.
-#define T5D_ENC_STEP(i_, CUR_, NEXT2_, ISSUE_, BODY_)                          \
-  if ((i_) >= nb) break;                                                       \
-  __builtin_amdgcn_s_waitcnt(0x070 | 2);                                       \
-  __builtin_amdgcn_s_barrier();                                                \
-  ISSUE_((i_) + 2, NEXT2_);                                                    \
-  __builtin_amdgcn_sched_barrier(0);                                           \
-  BODY_(i_, CUR_);
-
   // scores of key tile kt for this lane: keys 16 kt + 4 g + i of query l16
-  constexpr int ROUNDS = (MAXB + 2) / 3;
-  uint32_t sc[12 * ROUNDS][2];
+  uint32_t sc[4][2];
 #pragma unroll
-  for (int t = 0; t < 12 * ROUNDS; ++t)
-    sc[t][0] = sc[t][1] = 0xFF80FF80u;  // -inf
+  for (int t = 0; t < 4; ++t) sc[t][0] = sc[t][1] = 0xFF80FF80u;  // -inf
   float m = -3.0e38f, l = 0.f;
   const int swz = l16 & 7;
-#define T5D_ENC_SCORES(i_, S_)                                                 \
-  _Pragma("unroll") for (int t = 0; t < 4; ++t) {                              \
-    const int kt = 4 * (i_) + t;                                               \
-    /* two key tiles per test: their chains of dependent instructions (LDS   \
-       read, matrix instruction, rounding, exp) interleave */                 \
-    if ((kt & ~1) < my_tiles) {                                                \
-      f32x4_e acc = (f32x4_e){0.f, 0.f, 0.f, 0.f};                             \
-      _Pragma("unroll") for (int c = 0; c < 2; ++c) {                          \
-        FragE kop;                                                             \
-        kop.u = S_[(16 * t + l16) * 8 + ((4 * c + gq) ^ swz)];                 \
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop.v, qb[c].v, acc, 0,  \
-                                                      0, 0);                   \
-      }                                                                        \
-      const float4 cap = *reinterpret_cast<const float4*>(lim_g + 16 * kt);    \
-      /* two values per rounding instruction; the cap as a median with -inf   \
-         (one instruction: fminf would first make both operands canonical) */ \
-      const uint32_t r01 = pack_bf16x2(acc[0], acc[1]);                        \
-      const uint32_t r23 = pack_bf16x2(acc[2], acc[3]);                        \
-      const uint32_t x01 =                                                     \
-          pack_bf16x2(bf16lo_to_f32(r01) + bias_g[16 * kt],                    \
-                      bf16hi_to_f32(r01) + bias_g[16 * kt + 1]);               \
-      const uint32_t x23 =                                                     \
-          pack_bf16x2(bf16lo_to_f32(r23) + bias_g[16 * kt + 2],                \
-                      bf16hi_to_f32(r23) + bias_g[16 * kt + 3]);               \
-      float s[4];                                                              \
-      s[0] = __builtin_amdgcn_fmed3f(bf16lo_to_f32(x01), cap.x, -INFINITY);    \
-      s[1] = __builtin_amdgcn_fmed3f(bf16hi_to_f32(x01), cap.y, -INFINITY);    \
-      s[2] = __builtin_amdgcn_fmed3f(bf16lo_to_f32(x23), cap.z, -INFINITY);    \
-      s[3] = __builtin_amdgcn_fmed3f(bf16hi_to_f32(x23), cap.w, -INFINITY);    \
-      const float tm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));            \
-      const float nm = fmaxf(m, tm);                                           \
-      float add = 0.f;                                                         \
-      _Pragma("unroll") for (int i = 0; i < 4; ++i) add += __expf(s[i] - nm);  \
-      l = l * __expf(m - nm) + add;                                            \
-      m = nm;                                                                  \
-      sc[kt][0] = pack_bf16x2(s[0], s[1]);                                     \
-      sc[kt][1] = pack_bf16x2(s[2], s[3]);                                     \
-    }                                                                          \
-  }
-
-  T5D_ENC_ISSUE_K(0, s_r0);
-  T5D_ENC_ISSUE_K(1, s_r1);
 #pragma unroll
-  for (int r = 0; r < ROUNDS; ++r) {
-    T5D_ENC_STEP(3 * r, s_r0, s_r2, T5D_ENC_ISSUE_K, T5D_ENC_SCORES)
-    T5D_ENC_STEP(3 * r + 1, s_r1, s_r0, T5D_ENC_ISSUE_K, T5D_ENC_SCORES)
-    T5D_ENC_STEP(3 * r + 2, s_r2, s_r1, T5D_ENC_ISSUE_K, T5D_ENC_SCORES)
+  for (int kt = 0; kt < 4; ++kt) {
+    // two key tiles per test: their chains of dependent instructions (LDS read,
+    // matrix instruction, rounding, exp) interleave
+    if ((kt & ~1) < my_tiles) {
+      f32x4_e acc = (f32x4_e){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        FragE kop;
+        kop.u = s_k[(16 * kt + l16) * 8 + ((4 * c + gq) ^ swz)];
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop.v, qb[c].v, acc, 0, 0, 0);
+      }
+      const float4 cap = *reinterpret_cast<const float4*>(lim_g + 16 * kt);
+      // two values per rounding instruction; the cap as a median with -inf (one
+      // instruction: fminf would first make both operands canonical)
+      const uint32_t r01 = pack_bf16x2(acc[0], acc[1]);
+      const uint32_t r23 = pack_bf16x2(acc[2], acc[3]);
+      const uint32_t x01 = pack_bf16x2(bf16lo_to_f32(r01) + bias_g[16 * kt],
+                                       bf16hi_to_f32(r01) + bias_g[16 * kt + 1]);
+      const uint32_t x23 = pack_bf16x2(bf16lo_to_f32(r23) + bias_g[16 * kt + 2],
+                                       bf16hi_to_f32(r23) + bias_g[16 * kt + 3]);
+      float s[4];
+      s[0] = __builtin_amdgcn_fmed3f(bf16lo_to_f32(x01), cap.x, -INFINITY);
+      s[1] = __builtin_amdgcn_fmed3f(bf16hi_to_f32(x01), cap.y, -INFINITY);
+      s[2] = __builtin_amdgcn_fmed3f(bf16lo_to_f32(x23), cap.z, -INFINITY);
+      s[3] = __builtin_amdgcn_fmed3f(bf16hi_to_f32(x23), cap.w, -INFINITY);
+      const float tm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+      const float nm = fmaxf(m, tm);
+      float add = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) add += __expf(s[i] - nm);
+      l = l * __expf(m - nm) + add;
+      m = nm;
+      sc[kt][0] = pack_bf16x2(s[0], s[1]);
+      sc[kt][1] = pack_bf16x2(s[2], s[3]);
+    }
   }
   // combine the 4 lanes (g) that share a query
 #pragma unroll
@@ -264,45 +217,23 @@ enc_attn_ring_kernel(EncAttnArgs a) {
     return pack_bf16x2(__expf(bf16lo_to_f32(packed) - m) * inv,
                        __expf(bf16hi_to_f32(packed) - m) * inv);
   };
-#define T5D_ENC_VALUES(i_, S_)                                                 \
-  _Pragma("unroll") for (int hb = 0; hb < 2; ++hb) {                           \
-    const int kt = 4 * (i_) + 2 * hb;                                          \
-    {                                                                          \
-      FragE pb;                                                                \
-      pb.u.x = prob2(sc[kt][0]);                                               \
-      pb.u.y = prob2(sc[kt][1]);                                               \
-      pb.u.z = prob2(sc[kt + 1][0]);                                           \
-      pb.u.w = prob2(sc[kt + 1][1]);                                           \
-      const char* blk = reinterpret_cast<const char*>(&S_[0]) + hb * 4096;     \
-      _Pragma("unroll") for (int dt = 0; dt < 4; ++dt) {                       \
-        const uint2* vp =                                                      \
-            reinterpret_cast<const uint2*>(blk + dt * 1024 + v_off0);          \
-        const uint2 lo = vp[0], hi = vp[4];                                    \
-        FragE va;                                                              \
-        va.u = make_uint4(lo.x, lo.y, hi.x, hi.y);                             \
-        oc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va.v, pb.v, oc[dt],   \
-                                                         0, 0, 0);             \
-      }                                                                        \
-    }                                                                          \
-  }
-  __builtin_amdgcn_s_waitcnt(0x070);
-  __builtin_amdgcn_s_barrier();  // every wavefront is done with the K stages
-  T5D_ENC_ISSUE_V(0, s_r0);
-  T5D_ENC_ISSUE_V(1, s_r1);
 #pragma unroll
-  for (int r = 0; r < ROUNDS; ++r) {
-    T5D_ENC_STEP(3 * r, s_r0, s_r2, T5D_ENC_ISSUE_V, T5D_ENC_VALUES)
-    T5D_ENC_STEP(3 * r + 1, s_r1, s_r0, T5D_ENC_ISSUE_V, T5D_ENC_VALUES)
-    T5D_ENC_STEP(3 * r + 2, s_r2, s_r1, T5D_ENC_ISSUE_V, T5D_ENC_VALUES)
+  for (int hb = 0; hb < 2; ++hb) {
+    FragE pb;
+    pb.u.x = prob2(sc[2 * hb][0]);
+    pb.u.y = prob2(sc[2 * hb][1]);
+    pb.u.z = prob2(sc[2 * hb + 1][0]);
+    pb.u.w = prob2(sc[2 * hb + 1][1]);
+    const char* blk = reinterpret_cast<const char*>(&s_v[0]) + hb * 4096;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      const uint2* vp = reinterpret_cast<const uint2*>(blk + dt * 1024 + v_off0);
+      const uint2 lo = vp[0], hi = vp[4];
+      FragE va;
+      va.u = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      oc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va.v, pb.v, oc[dt], 0, 0, 0);
+    }
   }
-  // the loads issued past the last block must land before this workgroup's
-  // LDS can go to another
-  __builtin_amdgcn_s_waitcnt(0x070);
-#undef T5D_ENC_ISSUE_K
-#undef T5D_ENC_ISSUE_V
-#undef T5D_ENC_STEP
-#undef T5D_ENC_SCORES
-#undef T5D_ENC_VALUES
   // oc[dt][i]: out[q = l16][d = 16 dt + 4 g + i]
   if (q0 + l16 < E) {
     bf16_t* o = a.out + (row0 + q0 + l16) * (size_t)(a.H * 64) + h * 64 + 4 * gq;
@@ -316,7 +247,7 @@ enc_attn_ring_kernel(EncAttnArgs a) {
   }
 }
 
-// ---- beyond 128 positions: one pass ----------------------------------------------
+// ---- beyond 64 positions: one pass -----------------------------------------------
 // A workgroup takes 64 MT queries of one (item, head), a wavefront 16 MT, and walks 64
 // keys at a time once: scores as above (rounded where the reference rounds them),
 // weights relative to a running maximum that is raised only when a score passes it
@@ -328,15 +259,20 @@ enc_attn_ring_kernel(EncAttnArgs a) {
 // exact zero) and a padded query scores 0 with every key that exists (it attends
 // uniformly), both in tiles that hold one of the two only; a wavefront of padded
 // queries alone forms no scores.
-// What bounds it: ~260 vector instructions per tile and wavefront (the two roundings
-// of a score, its exponential) against 32 matrix instructions; 49 KB of LDS and 164
-// registers let three workgroups share a CU.  Measured beside the kernels that were
-// here before (two passes over the keys; up to 512 positions the one above with 8
-// blocks of 64): 7 x 16 heads x 1032 (400 and more valid) 203 -> 82 us, 2 x 16 x 2048
-// 243 -> 82, 64 x 16 x 512 (all valid) 261 -> 159, 32 x 12 x 512 (128 and more) 98 ->
-// 66, 64 x 16 x 300 95 -> 73, 64 x 12 x 132 32 -> 31; at 64 positions the one above is
-// the better one (256 x 12: 24 against 28 us), at 16 by far (512 x 12: 26 / 40), as
-// half or more of a 128-query tile is then empty.
+// What bounds it: vector instructions (~260 per tile and wavefront of 32 queries: the
+// two roundings of a score, its exponential) against 32 matrix instructions; 49 KB of
+// LDS let three workgroups share a CU.  Measured, us, beside the kernels that were here
+// before (up to 512 positions all scores in registers as above, two passes beyond):
+//   7 x 16 heads x 1032 (400 and more valid)   180 -> 71.4
+//   1 x 12 x 2048                              158 -> 47.1
+//   64 x 16 x 512 (all valid)                  261 -> 159
+//   32 x 12 x 512 (200 and more)              84.6 -> 59.2
+//   256 x 12 x 66 / 96 / 128 (half and more)  48.1 / 48.7 / 55.3 -> 39.3 / 41.6 / 46.5
+//   1 x 12 x 128                               6.6 -> 4.9
+// The line to the kernel above lies where its one block of keys ends.  Below, the one
+// block needs no running maximum and half or more of a workgroup's queries are not
+// there: 512 x 12 x 16 18.2 us above / 30.9 here, 128 x 12 x 40 9.1 / 11.4, 256 x 12 x
+// 64 21.8 / 23.5 (with 64 queries per workgroup).
 constexpr float kMaxSlack = 8.0f;
 constexpr float kLog2eE = 1.4426950408889634f;
 
@@ -766,7 +702,7 @@ extern "C" int t5d_encoder_attention_variant(
   T5D_REQUIRE(E <= kMaxEncLen, T5D_ELIMIT,
               "t5d_encoder_attention: E=%d beyond %d", E, kMaxEncLen);
   T5D_REQUIRE(H <= 65535 && B <= 65535 &&
-                  (E <= 128 ||
+                  (E <= kShortEnc ||
                    ((int64_t)B * H + 7) * ((E + 127) / 128) < (1LL << 31)),
               T5D_ELIMIT, "t5d_encoder_attention: H=%d B=%d beyond the launch grid",
               H, B);
@@ -775,9 +711,9 @@ extern "C" int t5d_encoder_attention_variant(
   a.bias = (const bf16_t*)rel_bias; a.len = enc_len; a.out = (bf16_t*)out;
   a.valid = valid_bits;
   a.B = B; a.H = H; a.E = E; a.Ep = Ep; a.q_stride = q_stride; a.k_stride = k_stride;
-  if (E <= 128) {
-    hipLaunchKernelGGL(enc_attn_ring_kernel<2>, dim3((E + 63) / 64, H, B), dim3(256),
-                       0, as_stream(stream), a);
+  if (E <= kShortEnc) {
+    hipLaunchKernelGGL(enc_attn_short_kernel, dim3(1, H, B), dim3(256), 0,
+                       as_stream(stream), a);
   } else {
     const bool low = one_pass_64(B, H, E);
     const int tiles = low ? (E + 63) / 64 : (E + 127) / 128;

@@ -524,8 +524,8 @@ def encoder_attention(q, k, v_t, rel_bias, enc_len, out=None, valid_bits=None,
   """q, k: [B*E, >= H*64] row-major views (row stride = stride(0)); v_t
   [B, H, Ep/32, 64, 32] (tile_cross_value of [B, H, 64, Ep]); rel_bias
   [H, 2E-1]; enc_len [B]; valid_bits: None or pack_valid_bits of the
-  per-position mask -> out [B*E, H*64].  variant: 0, 1 or (E <= 512) 2, the
-  same kernel (t5d_encoder_attention_variant)."""
+  per-position mask -> out [B*E, H*64].  variant: 0, 1 or (E <= 512) 2,
+  which choose nothing: the kernel follows from the sizes."""
   _chk(v_t, 'v_t', torch.bfloat16, 5)
   _chk(rel_bias, 'rel_bias', torch.bfloat16, 2)
   _chk(enc_len, 'enc_len', torch.int32, 1)
