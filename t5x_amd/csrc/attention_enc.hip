@@ -544,6 +544,8 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
+  // (wg_keys >= 1, as a workgroup has a query, which is valid or walks all keys: every
+  // tile that is fetched is met before the end)
   for (int jt = 0; jt < wg_keys; jt += 2 * KB) {
     meet();
     if (jt + KB < wg_keys) fetch(jt + KB, s_k1, s_v1);
@@ -553,8 +555,6 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
     if (jt + 2 * KB < wg_keys) fetch(jt + 2 * KB, s_k0, s_v0);
     attend(jt + KB, s_k1, s_v1);
   }
-  // (a workgroup without keys has loads of the first tile under way)
-  __builtin_amdgcn_s_waitcnt(0x0070);
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const float inv = 1.0f / rows_sum(l[mt]);
