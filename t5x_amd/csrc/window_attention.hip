@@ -39,6 +39,7 @@ struct WinArgs {
   t5d_ragged b;
   int HP, gs, splits;
   int tiles;  // window_rows_kernel: tiles of rows of the longest portion
+  int flat;   // ... and whether its grid has one dimension, or (tiles, S, G)
   float* parts;  // [S, G, splits, gs, HP + 2]
   const int32_t* gate;
   // window_rows_kernel over a span instead of rings: position first[s] + i of
@@ -258,15 +259,20 @@ window_rows_kernel(WinArgs g) {
   // The tiles of one (portion, key/value head) read the same keys and values:
   // consecutive block ids go round-robin over the 8 XCDs, so theirs are 8 apart.
   const int gs = g.gs;
-  const int pair = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / g.tiles);
-  if (pair >= a.G * g.b.S) return;
-  const int seq = pair / a.G, kv = pair - seq * a.G;
+  int seq = blockIdx.y, kv = blockIdx.z, nth = blockIdx.x;
+  bool turn = false;
+  if (g.flat) {
+    const int pair = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / g.tiles);
+    if (pair >= a.G * g.b.S) return;
+    seq = pair / a.G;
+    kv = pair - seq * a.G;
+    nth = (int)(blockIdx.x >> 3) % g.tiles;
+    turn = (pair >> 3) * g.tiles / 32 % 2 != 0;
+  }
   const int off = g.b.seq_off[seq];
   const int rows = (g.b.seq_off[seq + 1] - off) * gs;
-  // Long tiles first, where the next 256 blocks begin the other way round: the two
-  // tiles of a CU are then a long one and a short one.
-  const int nth = (int)(blockIdx.x >> 3) % g.tiles;
-  const bool turn = (pair >> 3) * g.tiles / 32 % 2 != 0;
+  // Long tiles first, where the next 256 blocks begin the other way round (turn): the
+  // two tiles of a CU are then a long one and a short one.
   const int r0 = (turn ? nth : g.tiles - 1 - nth) * (64 * MT);
   if (r0 >= rows) return;
   const int start = g.b.seq_start[seq];
@@ -846,7 +852,12 @@ template <bool SPAN>
 static void launch_rows_tiles(hipStream_t s, WinArgs g) {
   g.tiles = ((int64_t)g.b.max_len * g.gs + 127) / 128;
   const int64_t pairs = (int64_t)g.b.S * g.a.G;
-  const dim3 grid((unsigned)((pairs + 7) / 8 * 8 * g.tiles)), block(256);
+  // A dimension of a grid holds fewer than 2^32 threads: many portions beside one of
+  // very many (token, head) pairs take three.
+  const int64_t blocks = (pairs + 7) / 8 * 8 * g.tiles;
+  g.flat = blocks < (1LL << 24);
+  const dim3 grid = g.flat ? dim3((unsigned)blocks) : dim3(g.tiles, g.b.S, g.a.G);
+  const dim3 block(256);
 #define T5D_ROWS(DT_)                                                              \
   do {                                                                             \
     if (g.a.slopes != nullptr || !(g.a.scale > 0.f))                               \

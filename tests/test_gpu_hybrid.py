@@ -338,6 +338,21 @@ def test_window_attention_rows_of_many_tiles():
     at += len(x)
 
 
+def test_window_attention_rows_beyond_one_dimension_of_a_grid():
+  """One long portion beside thousands of single tokens: 2^24 tiles, most of them empty,
+  whose threads no dimension of a launch grid holds; each portion as it is alone."""
+  n = 4096
+  a = Attention(torch.bfloat16, 128, 1, 16, 16, 64, n, n, n, norms=False)
+  g = torch.Generator(device='cuda')
+  g.manual_seed(3)
+  lens = [1] * 5 + [n] + [1] * (n - 6)
+  x = torch.randn((sum(lens), a.cols), device='cuda', generator=g).to(torch.bfloat16)
+  seqs = torch.split(x, lens)
+  got = np.split(a.run([(s, 0) for s in range(n)], seqs, 2), np.cumsum(lens)[:-1])
+  for s in (0, 4, 5, 6, n - 1):
+    assert np.array_equal(got[s], a.run([(s, 0)], [seqs[s]], 2)), s
+
+
 @pytest.mark.parametrize('bias,sink,norms', [(False, True, True),
                                              (True, False, True),
                                              (True, True, False)])
