@@ -979,7 +979,10 @@ extern "C" int t5d_window_attention_run(void* stream, const t5d_window_attention
   else
     hipLaunchKernelGGL(window_append_kernel<float>, agrid, ablock, 0, s, g);
   T5D_CHECK_LAUNCH("window attention (append)");
-  if (variant == 2 || (variant == 0 && can_rows)) {
+  // (the rows kernel's loads into LDS want whole 16-byte pieces: rings that start
+  // elsewhere go the general way)
+  const bool whole = (((uintptr_t)a->key_ring | (uintptr_t)a->value_ring) & 15) == 0;
+  if ((variant == 2 || (variant == 0 && can_rows)) && whole) {
     launch_rows_tiles<false>(s, g);
     T5D_CHECK_LAUNCH("window attention (rows)");
     return T5D_OK;

@@ -353,6 +353,20 @@ def test_window_attention_rows_beyond_one_dimension_of_a_grid():
     assert np.array_equal(got[s], a.run([(s, 0)], [seqs[s]], 2)), s
 
 
+@pytest.mark.parametrize('variant', [0, 2])
+def test_window_attention_rings_that_start_between_16_byte_pieces(variant):
+  from t5x_amd import _lib
+  a = Attention(torch.bfloat16, 6, 2, 48, 40, 30, 2, 70, 150)
+  flat = [torch.full((r.numel() + 4,), 7.0, dtype=r.dtype, device='cuda')
+          for r in a.rings]
+  a.rings = [f[4:].view_as(r) for f, r in zip(flat, a.rings)]
+  a.a.key_ring, a.a.value_ring = (_lib.ptr(r) for r in a.rings)
+  x = a.sequence(130)
+  got = np.concatenate([a.run([(1, at)], [x[at:at + 65]], variant) for at in (0, 65)])
+  assert rel(got, a.oracle(x)) < a.tol
+  assert all(bool((f[:4] == 7.0).all()) for f in flat)
+
+
 @pytest.mark.parametrize('bias,sink,norms', [(False, True, True),
                                              (True, False, True),
                                              (True, True, False)])
