@@ -24,6 +24,8 @@
 // the chunks with three matrix products each, in float32 on the matrix cores.
 // A step of one token per sequence is one kernel per (sequence, head) that reads
 // and writes the state once.
+#include <algorithm>
+
 #include "common.h"
 #include "gemm_tiles.h"
 
@@ -916,16 +918,27 @@ recurrence_finish_kernel(RecArgs g) {
 }
 
 // ---- one token per sequence ------------------------------------------------------------
-// One workgroup per (sequence, head), a wavefront per 32 columns: lane (quad, dg)
-// holds rows dg + 8 i of 4 neighbouring columns, so a load instruction reads 8
-// runs of 128 bytes.  The kernel is one chain of waits, so everything is requested
-// at its start, in the order in which it is needed (loads are waited for in order):
-// the projections, the taps and the ring of the convolution, the output's gate, then
-// the state; q, k, v and the decay are formed while the state is on its way.  With
-// loads in the convolution's own loop, behind the state, and the gate's at the end, one
-// token of 8 heads of 128 x 128 with convolutions lasted 10.8 us (now 8.2) and 64 of
-// them 21.2 us (now 17.6; their state alone takes 13.7 us at the rate of a large copy);
-// without convolutions 17.2 us (now 16.3).
+// One workgroup per (sequence, head), a wavefront per 32 columns and at least four, as
+// the first four form q, k, v and the decay, one each: lane (quad, dg) holds rows
+// dg + 8 i of 4 neighbouring columns, so a load instruction reads 8 runs of 128 bytes.
+// The kernel is one chain of waits, so everything is requested at its start, in the
+// order in which it is needed (loads are waited for in order): the projections, the
+// taps and the ring of the convolution, the output's gate, then the state; q, k, v and
+// the decay are formed while the state is on its way.  Without the delta rule, where
+// there is little to form, the state comes first: it then keeps the memory busy from
+// the start in launches of two workgroups per CU and more (8 heads of 128, 128 tokens:
+// 23.1 -> 21.0 us; 64 tokens: 10.4 -> 10.8).
+// us per launch, with loads in the convolution's own loop, behind the state, and the
+// gate's at the end / now (rows of the state past the last are not requested, by the
+// group of 8 x R; one token, then 64, 128, 256):
+//   delta rule, 8 heads of 128 x 128, 4 taps   7.2 14.4 29.1 51.7 /  5.9 11.7 23.9 43.8
+//   delta rule, 8 heads of 64 x 64, 4 taps     6.0  8.0  9.4 15.5 /  4.3  6.0  8.4 15.6
+//   delta rule, 4 heads of 200 x 200, 4 taps  11.8 22.3 43.5 81.2 / 11.1 21.8 41.9 79.4
+//   delta rule, 4 heads of 256 x 256, 4 taps  12.1 28.9 55.5  123 / 11.2 27.9 52.9  107
+//   delta rule, 4 heads of 32 x 32, 2 taps     6.3  6.6  6.7  7.3 /  3.9  4.2  4.6  6.0
+//   no delta rule, 8 heads of 128 x 128        5.8 11.4 21.7 42.6 /  5.0 10.8 21.0 40.6
+//   no delta rule, 4 heads of 48 x 64          4.3  4.8  5.6  6.7 /  3.7  4.2  4.9  6.7
+// (64 states of 8 x 128 x 128 take 13.7 us at the rate of a large copy from memory.)
 template <int DI, bool DELTA, typename T>
 __global__ void __launch_bounds__(512)
 recurrence_step_kernel(RecArgs g) {
@@ -940,17 +953,18 @@ recurrence_step_kernel(RecArgs g) {
   const int pos = g.b.seq_start[m], slot = g.b.seq_slot[m];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int waves = blockDim.x >> 6;
   const int quad = lane & 7, dg = lane >> 3;
   const int col = 4 * (8 * wave + quad);
   const bool col_ok = col < a.Dv;
   const T* p = reinterpret_cast<const T*>(a.proj) + (size_t)m * a.ld_proj;
-  // role 0, 1, 2: channels lane + 64 u of q, k, v; role 3: of the decay
+  // role 0, 1, 2: channels lane + 64 u of q, k, v; role 3: of the decay (the first four
+  // wavefronts, there whatever the columns, take one each)
+  constexpr int U = 4;  // groups of 64 channels
   constexpr int NT = DI <= 16 ? 4 : 2;  // taps requested ahead (registers)
   const int ring0 = a.taps > 0 ? pos % a.taps : 0;
   // (kept as loaded: a conversion here would wait for the load)
-  T now[4], past[4][NT - 1];
-  float tap[4][NT];
+  T now[U], past[U][NT - 1];
+  float tap[U][NT];
   const auto channels = [&](int role) { return role == 2 ? a.Dv : a.D; };
   const auto column = [&](int role) {
     return role == 0 ? a.off_q + hg * a.D
@@ -974,7 +988,7 @@ recurrence_step_kernel(RecArgs g) {
     }
     const int n = channels(role);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < U; ++u) {
       if (64 * u >= n) break;
       const int c = min(lane + 64 * u, n - 1), cc = channel(role) + c;
       now[u] = p[column(role) + c];
@@ -988,6 +1002,28 @@ recurrence_step_kernel(RecArgs g) {
       }
     }
   };
+  float* state = a.state + ((size_t)slot * a.H + h) * a.D * a.Dv + col;
+  float4 st[DI];
+  const auto request_state = [&] {
+    if (pos > 0 && col_ok) {
+      constexpr int R = DELTA && DI == 32 ? 1 : 4;  // rows of 8 per test of the size
+#pragma unroll
+      for (int i = 0; i < DI; i += R) {
+        const bool there = i == 0 || 8 * i < a.D;
+#pragma unroll
+        for (int e = i; e < i + R; ++e) {
+          st[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+          if (there)  // (past the last row the last one again)
+            st[e] = *reinterpret_cast<const float4*>(
+                state + (size_t)min(dg + 8 * e, a.D - 1) * a.Dv);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < DI; ++i) st[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  if (!DELTA) request_state();
   if (wave < 4) request(wave);
   const T beta_z = p[DELTA ? a.off_beta + h : 0];
   // the output channel of this lane
@@ -999,17 +1035,7 @@ recurrence_step_kernel(RecArgs g) {
   const float gate_low =
       a.low[(size_t)m * a.ld_low + (low_gate ? a.off_low_gate + h * a.Dv + cg : a.off_z)];
   const T gate_z = (low_gate ? p : p + a.off_gate + (size_t)h * a.Dv)[low_gate ? 0 : cg];
-  float* state = a.state + ((size_t)slot * a.H + h) * a.D * a.Dv + col;
-  float4 st[DI];
-  if (pos > 0 && col_ok) {
-#pragma unroll
-    for (int i = 0; i < DI; ++i)
-      st[i] = *reinterpret_cast<const float4*>(
-          state + (size_t)min(dg + 8 * i, a.D - 1) * a.Dv);
-  } else {
-#pragma unroll
-    for (int i = 0; i < DI; ++i) st[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
+  if (DELTA) request_state();
   const auto form = [&](int role) {
     if (role == 3) {
 #pragma unroll
@@ -1022,10 +1048,10 @@ recurrence_step_kernel(RecArgs g) {
       return;
     }
     const int n = channels(role), pad = role == 2 ? n : DP;
-    float x[4];
+    float x[U];
     float ss = 0.f;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int c = lane + 64 * u;
       x[u] = 0.f;
       if (c < n) {
@@ -1051,15 +1077,13 @@ recurrence_step_kernel(RecArgs g) {
     if (a.unit && role < 2) f /= sqrtf(wave_sum(ss) + a.unit_eps);
     float* dst = role == 0 ? s_q : role == 1 ? s_k : s_v;
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < U; ++u)
       if (lane + 64 * u < pad) dst[lane + 64 * u] = x[u] * f;
   };
   if (wave < 4) form(wave);
-  for (int role = wave + waves; role < 4; role += waves) {  // (under 128 columns)
-    request(role);
-    form(role);
-  }
   __syncthreads();
+  // (a wavefront that was there for its role; barriers wait for those that stay)
+  if (32 * wave >= a.Dv) return;
   if (a.D < DP) {  // rows past the last were read from it
 #pragma unroll
     for (int i = 0; i < DI; ++i)
@@ -1114,7 +1138,7 @@ recurrence_step_kernel(RecArgs g) {
 
 template <bool DELTA, typename T>
 static void launch_step(hipStream_t s, const RecArgs& g) {
-  const dim3 grid(g.b.S * g.a.H), block(64 * ((g.a.Dv + 31) / 32));
+  const dim3 grid(g.b.S * g.a.H), block(64 * std::max(4, (g.a.Dv + 31) / 32));
 #define T5D_RS(DI_) \
   hipLaunchKernelGGL((recurrence_step_kernel<DI_, DELTA, T>), grid, block, 0, s, g)
   if (g.a.D <= 32) T5D_RS(4);
