@@ -654,9 +654,18 @@ recurrence_chunk_kernel(RecArgs g) {
         if (DELTA) u[i] = down(s_t[4 * g4 + i], 4 * g4 + i, column, vs);
         y[i] = down(s_m[4 * g4 + i], 4 * g4 + i, column, vs);
       }
-    } else {
-      if (DELTA) u = times(tm, v, zero);
+    } else if (DELTA) {
+      u = times(tm, v, zero);
       y = times(mm, v, zero);
+    } else {
+      // tokens in their order: the last ones weigh most where decays are fast
+      float b[4], late[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        b[i] = s_b[x][4 * i + g4];
+        late[i] = s_v[(4 * i + g4) * vs + 16 * tile + x];
+      }
+      y = times(b, late, zero);
     }
     put(w + lay.us(), at, u);
     put(w + lay.os(), at, y);
