@@ -852,10 +852,17 @@ template <bool SPAN>
 static void launch_rows_tiles(hipStream_t s, WinArgs g) {
   g.tiles = ((int64_t)g.b.max_len * g.gs + 127) / 128;
   const int64_t pairs = (int64_t)g.b.S * g.a.G;
-  // A dimension of a grid holds fewer than 2^32 threads: many portions beside one of
-  // very many (token, head) pairs take three.
-  const int64_t blocks = (pairs + 7) / 8 * 8 * g.tiles;
-  g.flat = blocks < (1LL << 24);
+  // The one-dimensional grid keeps the tiles of a pair on one XCD, whose 32 CUs then
+  // share its keys and values: 3 to 20 % faster where every XCD gets about the same
+  // (heads of 128, 3000 tokens x 4 heads, us with it / without: 8 pairs 98 / 109, 16 172
+  // / 185, 32 309 / 333; heads of 200: 297 / 367, 545 / 711, 1116 / 1373).  Few pairs
+  // leave XCDs idle (1 pair 79 / 40, 2 85 / 47, 4 90 / 67, 6 93 / 94, 9 144 / 119, 12
+  // 150 / 150, 17 216 / 200; heads of 200, 1 pair 269 / 120), unless an XCD has a CU for
+  // each tile (heads of 64, 1500 tokens, 9 pairs: 31.8 / 33.7).  And a dimension of a
+  // grid holds fewer than 2^32 threads: many portions beside one of very many
+  // (token, head) pairs take three.
+  const int64_t turns = (pairs + 7) / 8, blocks = turns * 8 * g.tiles;
+  g.flat = blocks < (1LL << 24) && (turns * g.tiles <= 32 || turns * 24 <= pairs * 4);
   const dim3 grid = g.flat ? dim3((unsigned)blocks) : dim3(g.tiles, g.b.S, g.a.G);
   const dim3 block(256);
 #define T5D_ROWS(DT_)                                                              \

@@ -325,11 +325,13 @@ def test_window_attention_rows_with_scores_that_climb(H, G, D, scale, bias):
   assert rel(got, a.oracle(x)) < a.tol
 
 
-def test_window_attention_rows_of_many_tiles():
+@pytest.mark.parametrize('H,G', [(8, 2), (12, 6), (3, 1)])
+def test_window_attention_rows_of_many_tiles(H, G):
   """More tiles than one round of the compute units takes: the portions whose
-  tiles run in the other order, beside short ones."""
+  tiles run in the other order, beside short ones; both grids (30 pairs of a portion
+  and a key/value head are spread over the XCDs evenly, 10 and 5 are not)."""
   lens = [3, 64, 1, 70, 1100]
-  a = Attention(torch.bfloat16, 8, 2, 32, 32, 300, 5, 1100, 1100)
+  a = Attention(torch.bfloat16, H, G, 32, 32, 300, 5, 1100, 1100)
   seqs = [a.sequence(n) for n in lens]
   got = a.run([(s, 0) for s in range(5)], seqs, 2)
   at = 0
