@@ -702,8 +702,8 @@ extern "C" int t5d_encoder_attention_variant(
   T5D_REQUIRE(E <= kMaxEncLen, T5D_ELIMIT,
               "t5d_encoder_attention: E=%d beyond %d", E, kMaxEncLen);
   T5D_REQUIRE(H <= 65535 && B <= 65535 &&
-                  (E <= kShortEnc ||
-                   ((int64_t)B * H + 7) * ((E + 127) / 128) < (1LL << 31)),
+                  (E <= kShortEnc ||  // (one dimension: fewer than 2^32 threads)
+                   ((int64_t)B * H + 7) / 8 * 8 * ((E + 127) / 128) < (1LL << 24)),
               T5D_ELIMIT, "t5d_encoder_attention: H=%d B=%d beyond the launch grid",
               H, B);
   EncAttnArgs a;

@@ -81,6 +81,18 @@ def test_version_and_error_string_without_gpu():
   assert b'dtype' in lib.t5d_last_error()
 
 
+def test_encoder_attention_beyond_a_launch_grid_without_gpu():
+  """More tiles than one dimension of a grid holds are named, not left to the launch
+  (the buffers are not looked at before)."""
+  from t5x_amd import _lib
+  lib = _lib.load()
+  p, H = 4096, 300
+  rc = lib.t5d_encoder_attention_variant(None, p, p, p, p, p, None, p, 65535, H, 100,
+                                         128, H * 64, H * 64, 0)
+  assert rc == -3  # T5D_ELIMIT
+  assert b'launch grid' in lib.t5d_last_error()
+
+
 def test_many_row_tile_choice_without_gpu():
   """t5d_gemm_rows_tile: which workgroup tile the many-row dense kernel runs a
   shape on (1: 256 x 128, 2: 256 x 256, 3: 256 x 192), by the rounds of
