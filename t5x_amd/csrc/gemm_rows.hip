@@ -432,9 +432,10 @@ rows_gemm_kernel(RowsGemmArgs g) {
 // serves 16 lanes at a time: 0..3 and 12..15 of one quarter wavefront with 4..11
 // of its neighbour, which want the neighbouring piece.  With swap = 0, 0, 3, 3
 // their 16 slots differ mod 16.  (Slots that differ within a quarter, by a
-// rotation or an XOR by r / 4, made 40 % of the LDS cycles bank conflicts:
-// 8192 x 1024 x 5632 gated 97 us, 16384 x 768 x 4096 gated 123 us, now
-// 90 and 115 us.)
+// rotation or an XOR by r / 4, made 40 % of the cycles of LDS reads bank conflicts, now
+// 3 to 7 %, by the counters at 16384 x 4096 x 4096 (35.1 M -> 1.6 M cycles), 16384 x 2048
+// x 768 and 8192 x 1024 x 5632: the last, gated, 97 us, 16384 x 768 x 4096 gated 123 us,
+// now 90 and 115 us.)
 // bfloat16 weights (int8 tiles must be widened on the way).
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) const void* glb_ptr_t;
@@ -646,7 +647,7 @@ extern "C" int t5d_gemm_rows_tile(int w_dtype, int64_t M, int K, int N) {
 // long on an empty chip as on a full one (its k-steps follow one another), so while
 // there are fewer workgroups than CUs they are made lower: 128 rows, or 64.  Results
 // have the same bits.  Measured, us with 256 / 128 / 64 rows:
-//   600 x 2048 x 768 residual  34.6 / 20.8 / 16.7   (15 rows of workgroups of 64)
+//   600 x 2048 x 768 residual  34.6 / 20.8 / 16.7   (60 workgroups of 64 rows)
 //   2000 x 2048 x 768          35.3 / 22.5 / 17.6
 //   1000 x 5120 x 2048         70.9 / 45.5 / 39.6
 //   600 x 768 x 4096 gated     16.9 / 11.3 / 13.4

@@ -240,8 +240,8 @@ constexpr float kMaxSlack = 8.0f;
 // BIAS: with slopes, or a scale that is not positive.
 // Per tile and wavefront 96 matrix instructions (1536 cycles) stand against ~390
 // vector instructions (1950 cycles with the 32 exponentials): what bounds the kernel
-// is that the two hardly overlap at two wavefronts per SIMD (36 % and 40 % busy;
-// without any loads it would be 7 % faster).  Measured, heads of 128 over 1024
+// is that the two hardly overlap at two wavefronts per SIMD (38 % and 43 % busy by the
+// counters, no bank conflicts).  Measured, heads of 128 over 1024
 // positions, 4 x 4096 tokens: 8 heads over 2 key/value heads 206 -> 115 us, 8 heads
 // over expanded latents in pieces of 2048 118 -> 60 us each.  The kernel before
 // staged tiles through registers, with a second barrier and V transposed on the way
