@@ -121,6 +121,39 @@ def test_gemm_rows_repeated_launches_at_full_size(ops):
                          first_res)
 
 
+@pytest.mark.parametrize('M,rows', [(601, 64), (1985, 64), (4001, 128)])
+def test_gemm_rows_repeated_launches_of_low_tiles(ops, M, rows):
+  """The same for the tiles of 64 and 128 rows, which the 128-column tile gets while
+  its workgroups are fewer than the 256 compute units; lengths off the tile, the
+  residual overwritten by the result."""
+  groups = lambda n: -(-M // n) * (768 // 128)
+  assert (groups(64) <= 256) == (rows == 64) and groups(128) <= 256
+  g = torch.Generator(device='cuda')
+  g.manual_seed(M)
+  a = torch.randn(M, 768, device='cuda', generator=g).to(torch.bfloat16)
+  w0 = torch.randn(768, 768, device='cuda', generator=g) / 768**0.5
+  w1 = torch.randn(768, 384, device='cuda', generator=g) / 768**0.5
+  res = torch.randn(M, 768, device='cuda', generator=g).to(torch.bfloat16)
+  gated = ops.pack_weight(w0[:, :384].contiguous(), torch.bfloat16, gate_kernel=w1)
+  plain = ops.pack_weight(w0, torch.bfloat16)
+  want = (a.float() @ w0.to(torch.bfloat16).float()).to(torch.bfloat16).float()
+  want = (want + res.float()).to(torch.bfloat16).float()
+  first = ops.gemm_rows(a, gated, tile=1)
+  first_res = ops.gemm_rows(a, plain, residual=res, tile=1)
+  # (half a bfloat16 step of the product, one of the sum where a half lies between)
+  assert bool(((first_res.float() - want).abs() <= 2e-2 + 2.0**-7 * want.abs()).all())
+  h = (a.float() @ w0[:, :384].to(torch.bfloat16).float()).to(torch.bfloat16).float()
+  u = (a.float() @ w1.to(torch.bfloat16).float()).to(torch.bfloat16).float()
+  # (a step of the rounded gate moves the unit by up to two of its own)
+  unit = torch.nn.functional.gelu(h, approximate='tanh').to(torch.bfloat16).float() * u
+  assert bool(((first.float() - unit).abs() <= 2e-2 + 2.0**-6 * unit.abs()).all())
+  for _ in range(20):
+    assert torch.equal(ops.gemm_rows(a, gated, tile=1), first)
+    own = res.clone()
+    assert torch.equal(ops.gemm_rows(a, plain, out=own, residual=own, tile=1),
+                       first_res)
+
+
 def test_gemm_rows_plain_entry_point(ops):
   """t5d_gemm_rows itself (ops.gemm_rows goes through t5d_gemm_rows_tiled)."""
   from t5x_amd import _lib
