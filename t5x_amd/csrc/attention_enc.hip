@@ -5,10 +5,11 @@
 //
 // Two kernels on the matrix cores, chosen by length: enc_attn_short_kernel up to 64
 // positions (scores kept in registers between the keys and the values),
-// enc_attn_tile_kernel beyond (one pass over the keys, workgroups of 128 queries or 64).  Both form S^T = K Q^T, keys as matrix rows, so that a lane ends up with 4
-// consecutive keys of ONE query, which is the operand order of out^T = V^T P^T; V is
-// given transposed in 32-key blocks ([B, H, Ep / 32, 64, 32], what t5d_gemm_rows'
-// value layout writes).  Scores are rounded where the reference rounds them.
+// enc_attn_tile_kernel beyond (one pass over the keys, workgroups of 128 queries or 64).
+// Both form S^T = K Q^T, keys as matrix rows, so that a lane ends up with 4 consecutive
+// keys of ONE query, which is the operand order of out^T = V^T P^T; V is given transposed
+// in 32-key blocks ([B, H, Ep / 32, 64, 32], what t5d_gemm_rows' value layout writes).
+// Scores are rounded where the reference rounds them.
 // Masked keys weigh nothing beside a valid one, and a padded query attends uniformly
 // over all keys, as with the reference's -1e10; keys beyond E do not exist.
 #include <math.h>

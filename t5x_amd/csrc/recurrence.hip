@@ -408,8 +408,8 @@ constexpr int kChunkTaps = 8;  // longest convolution of the chunk kernel
 // whole columns on the matrix cores: Wk = T (k P), Us = T v, and with M = B T
 // Qs = q P - M (k P), Os = M v.
 // What bounds it: vector instructions (59 % of their slots by the counters; 1714 per
-// wavefront, half of them silu and decays) with four workgroups per CU, then 42 KB written per chunk and
-// head.  4 x 4096 tokens, 8 heads of 128: delta rule 160 us, gated linear attention
+// wavefront, half of them silu and decays) with four workgroups per CU, then 42 KB written
+// per chunk and head.  4 x 4096 tokens, 8 heads of 128: delta rule 160 us, gated linear attention
 // 103 us; 301 and 240 us with the triangular solve and the products with B down each
 // column on the vector ALUs, divisions instead of sigmoid_quick, the library's
 // logarithm, and loads that branches kept from being in flight together.
