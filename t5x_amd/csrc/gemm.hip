@@ -1028,13 +1028,16 @@ bool t5d::norm_gemm_is_wide(int w_dtype, int K, int N) {
          (K == 512 || K == 768 || K == 1024);
 }
 
-// One kernel shape for every M (rows in groups of 8 along grid.y), so the
-// summation order, and with it every bit of the result, does not depend on
-// how many rows a call carries.
+// The matrix cores where K comes in whole 32s (gemm_f32.hip), otherwise the kernel
+// above (rows in groups of 8 along grid.y).  Both add in the same order whatever M is,
+// so no bit of a result depends on how many rows a call carries.
 static void launch_gemm_f32(hipStream_t s, const float* A, const float* W,
                             const float* residual, float* C, int M, int K,
                             int N, int epilogue, const float* norm_scale,
                             float eps) {
+  if (launch_f32_mfma(s, {A, W, residual, C, M, K, N, K, epilogue, tls_gate, norm_scale,
+                          eps, 0.f, 0.f, 0.f}, false))
+    return;
   const int ncols = epilogue == T5D_EPI_GEGLU ? N / 2 : N;
   dim3 grid((ncols + kF32Cols - 1) / kF32Cols, (M + kF32Rows - 1) / kF32Rows);
 #define T5D_F32_LAUNCH(WV_, NORMED_)                                          \
@@ -1054,6 +1057,9 @@ static void launch_gemm_f32(hipStream_t s, const float* A, const float* W,
 static void launch_dense_f32(hipStream_t s, const float* A, int lda, const float* W,
                              float* C, int M, int K, int N, int epilogue,
                              float glu_limit, float glu_alpha, float glu_add) {
+  if (launch_f32_mfma(s, {A, W, nullptr, C, M, K, N, lda, epilogue, tls_gate, nullptr,
+                          0.f, glu_limit, glu_alpha, glu_add}, true))
+    return;
   const int ncols = epilogue == T5D_EPI_CLAMPED_GLU ? N / 2 : N;
   dim3 grid((ncols + kF32Cols - 1) / kF32Cols, (M + kF32Rows - 1) / kF32Rows);
 #define T5D_F32_LAUNCH(WV_)                                                     \

@@ -172,6 +172,21 @@ __device__ __forceinline__ void store_result(const DenseArgs& g, int m, int n,
 }
 
 
+// Float32 layers on the matrix cores (gemm_f32.hip).
+struct F32GemmArgs {
+  const float* A;         // [M, lda]
+  const float* W;         // [K, N]; gated: N / 2 values, then N / 2 gates
+  const float* residual;  // [M, N] or null
+  float* C;               // [M, columns of work]
+  int M, K, N, lda, epilogue;
+  const int32_t* gate;
+  const float* norm_scale;  // [K] or null
+  float eps, glu_limit, glu_alpha, glu_add;
+};
+// false: not a shape or alignment for it, nothing is launched.  dense: t5d_dense's
+// epilogues instead of t5d_gemm's.
+bool launch_f32_mfma(hipStream_t s, const F32GemmArgs& g, bool dense);
+
 struct GemmPlan {
   int mp, nt, m_parts, n_groups;
   int k_parts;  // > 1: K split over workgroups (large tiles only)

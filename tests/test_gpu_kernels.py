@@ -315,6 +315,58 @@ def test_norm_gemm_f32(ops, M, K, N, geglu):
   np.testing.assert_allclose(host(one), want, atol=1e-4, rtol=1e-4)
 
 
+def _f32_sums(a, w):
+  """a @ w as the float32 kernels add it: 16 parts of K, within a part chains of fused
+  multiply-adds over k % 32 / 8 = 0..3, one tree.  (A float64 sum rounded to float32 is
+  the fused multiply-add up to double rounding, one case in 2^29.)"""
+  M, K = a.shape
+  kq = ((K + 15) // 16 + 31) // 32 * 32
+  def chain(part, sub):
+    acc = np.zeros((M, w.shape[1]), np.float32)
+    for k in range(min(K, part * kq), min(K, part * kq + kq)):
+      if k % 32 // 8 == sub:
+        acc = (a[:, k:k + 1].astype(np.float64) * w[k] + acc).astype(np.float32)
+    return acc
+  part = lambda p: ((chain(p, 0) + chain(p, 1)) + (chain(p, 2) + chain(p, 3)))
+  r = [part(i) + part(i + 8) for i in range(8)]
+  return ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]))
+
+
+@pytest.mark.parametrize('M,K,N', [(1, 128, 16), (5, 512, 70), (17, 384, 48),
+                                   (16, 1024, 20), (700, 544, 200),
+                                   (600, 160, 331)])
+def test_gemm_f32_order_of_the_sums(ops, M, K, N):
+  """float32 dense layers, 16 and 4 wavefronts, 16 and 64 columns, empty parts of K and
+  edges of tiles: the bits of one order of additions, whatever the rows."""
+  rs = np.random.RandomState(M + K + N)
+  a = rs.randn(M, K).astype(np.float32)
+  w = (rs.randn(K, N) / np.sqrt(K)).astype(np.float32)
+  g = (1 + 0.1 * rs.randn(K)).astype(np.float32)
+  res = rs.randn(M, N).astype(np.float32)
+  want = _f32_sums(a, w)
+  pw = ops.pack_weight(dev(w), torch.float32)
+  np.testing.assert_array_equal(host(ops.gemm(dev(a), pw)), want)
+  np.testing.assert_array_equal(
+      host(ops.gemm(dev(a), pw, residual=dev(res))), want + res)
+  # normed: the scale multiplies the weights, 1 / rms the sum (the sum of squares, the
+  # quotient, the root and the product: within 4 half units)
+  one = ops.gemm(dev(a), pw, norm_scale=dev(g))
+  inv = 1 / np.sqrt(_f32_sums(a[:1], a[:1].T)[0, 0] / np.float32(K) + np.float32(1e-6))
+  np.testing.assert_allclose(host(one)[0], _f32_sums(a[:1], w * g[:, None])[0] * inv,
+                             rtol=4 * 2.0**-24, atol=0)
+  # a row alone has the bits that it has among others, gated layers too
+  assert torch.equal(ops.gemm(dev(a[-1:]), pw, norm_scale=dev(g)), one[-1:])
+  pair = ops.pack_weight(dev(w), torch.float32, gate_kernel=dev(w[:, ::-1].copy()))
+  for kw in ({}, {'norm_scale': dev(g)}):
+    both = ops.gemm(dev(a), pair, **kw)
+    assert torch.equal(ops.gemm(dev(a[-1:]), pair, **kw), both[-1:])
+    last = host(both)[-1]
+    v = host(ops.gemm(dev(a[-1:]), pw, **kw))[0]
+    # the tanh form: its exponential's error times the slope, below 2^-21
+    t = 0.5 * v * (1 + np.tanh(np.sqrt(2 / np.pi) * (v + 0.044715 * v**3)))
+    np.testing.assert_allclose(last, t * v[::-1], rtol=2.0**-20, atol=2.0**-22)
+
+
 @pytest.mark.parametrize('M,K,N', [(128, 768, 32128), (64, 1024, 32128),
                                    (20, 512, 8192), (100, 768, 8208),
                                    (1, 768, 32128), (65, 512, 16400)])
