@@ -87,6 +87,11 @@ int t5d_embed(void* stream, int dtype, const void* table, const int32_t* ids,
 int t5d_rmsnorm(void* stream, int dtype, const void* x, const void* scale,
                 void* out, int R, int d, float eps);
 
+/* t5d_rmsnorm in bfloat16 whose output row r is the norm of row row_of[r] of x; d a
+ * multiple of 8, 16-byte aligned operands. */
+int t5d_rmsnorm_rows(void* stream, const void* x, const void* scale,
+                     const int32_t* row_of, void* out, int R, int d, float eps);
+
 /* Bias-free dense layer for few rows (DenseGeneral,
  * t5x/examples/t5/layers.py:364-414; MlpBlock gate product :460-474; the
  * residual adds of t5x/examples/t5/network.py:146,163,177).
@@ -175,6 +180,13 @@ int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
                         const void* W, const float* scales,
                         const void* residual, void* C, int64_t M, int K, int N,
                         int epilogue, int out_layout, int E, int Ep, int tile);
+
+/* t5d_gemm_rows into the value layout (T5D_OUT_HEADS_VALUE) for rows that
+ * t5d_encoder_rows lists: rows 4 i .. 4 i + 3 are positions e .. e + 3 of text b,
+ * at[i] = b << 12 | e.  M a multiple of 4. */
+int t5d_gemm_rows_values(void* stream, int w_dtype, const void* A, const void* W,
+                         const float* scales, void* C, int64_t M, int K, int N,
+                         const int32_t* at, int E, int Ep);
 
 /* The workgroup tile (1, 2 or 3, as in t5d_gemm_rows_tiled) that t5d_gemm_rows
  * uses for a shape: the cheapest by the rounds of workgroups each tile needs
@@ -321,6 +333,27 @@ int t5d_encoder_attention_variant(void* stream, const void* q, const void* k,
                                   const uint32_t* valid_bits, void* out, int B,
                                   int H, int E, int Ep, int q_stride,
                                   int k_stride, int variant);
+
+/* The rows an encoder has to compute for texts of unequal length, each tokens > 0
+ * followed by zeros: a text of n < E tokens takes n + 1 rows, the last of which stands
+ * for all of its padding (whose results are the same at every position), one of n = E
+ * takes E; rounded up to multiples of 4 with more padding.
+ *   tokens [B, E]; len, odd [B]: length, and whether the text is anything else than
+ *   tokens and then zeros; first [B + 1]: first row of each text; ids (B * E rounded up
+ *   to 4): token of each row; row_of [B, E]: row of each position; at: see
+ *   t5d_gemm_rows_values; summary [3]: rows in all, rows of the longest text, whether
+ *   any text is odd (then nothing else is to be used).  E <= 2048. */
+int t5d_encoder_rows(void* stream, const int64_t* tokens, int B, int E, int32_t* len,
+                     int32_t* odd, int32_t* first, int32_t* ids, int32_t* row_of,
+                     int32_t* at, int32_t* summary);
+
+/* t5d_encoder_attention over the rows that t5d_encoder_rows lists: q, k and out hold
+ * first[B] rows; most: rows of the longest text (summary[1]). */
+int t5d_encoder_attention_rows(void* stream, const void* q, const void* k,
+                               const void* v_t, const void* rel_bias,
+                               const int32_t* enc_len, const int32_t* first, int most,
+                               void* out, int B, int H, int E, int Ep, int q_stride,
+                               int k_stride);
 
 /* The same attention in float32 (the dtype of the exactness tests), straight
  * from the fused projection: qkv [B*E, 3*H*64] holds q | k | v per row;

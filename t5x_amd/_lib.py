@@ -228,6 +228,7 @@ _SIGNATURES = {
     't5d_pack_weight': (c_int, [_P, c_int, _P, _P, _P, c_int, c_int, c_int]),
     't5d_embed': (c_int, [_P, c_int, _P, _P, _P, c_int, c_int, c_int]),
     't5d_rmsnorm': (c_int, [_P, c_int, _P, _P, _P, c_int, c_int, c_float]),
+    't5d_rmsnorm_rows': (c_int, [_P, _P, _P, _P, _P, c_int, c_int, c_float]),
     't5d_gemm_workspace_bytes': (c_int64, [c_int] * 5),
     't5d_gemm': (c_int, [_P, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_int,
                          c_int, c_int, c_int, _P, _P]),
@@ -236,6 +237,9 @@ _SIGNATURES = {
     't5d_encoder_attention_variant': (c_int, [_P, _P, _P, _P, _P, _P, _P, _P,
                                               c_int, c_int, c_int, c_int,
                                               c_int, c_int, c_int]),
+    't5d_encoder_rows': (c_int, [_P, _P, c_int, c_int] + [_P] * 7),
+    't5d_encoder_attention_rows': (c_int, [_P] * 7 + [c_int, _P] +
+                                   [c_int] * 6),
     't5d_encoder_attention_f32': (c_int, [_P, _P, _P, _P, _P, _P, c_int,
                                           c_int, c_int]),
     't5d_gemm_rows': (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int64, c_int,
@@ -243,6 +247,8 @@ _SIGNATURES = {
     't5d_gemm_rows_tiled': (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int64,
                                     c_int, c_int, c_int, c_int, c_int, c_int,
                                     c_int]),
+    't5d_gemm_rows_values': (c_int, [_P, c_int, _P, _P, _P, _P, c_int64, c_int,
+                                     c_int, _P, c_int, c_int]),
     't5d_gemm_rows_tile': (c_int, [c_int, c_int64, c_int, c_int]),
     't5d_gemm_tiled': (c_int, [_P, c_int, c_int, c_int, _P, _P, _P, _P, _P,
                                c_int, c_int, c_int, c_int, _P, c_int, c_int,

@@ -66,11 +66,12 @@ rmsnorm_kernel(const T* __restrict__ x, const T* __restrict__ scale,
 // threads per row (a wavefront per row when there are thousands of rows, the
 // whole workgroup on one row when rows are few and long).  Same roundings as
 // above; the row is read a second time for the output, from L1.
-template <int RPW>
+// SPREAD: output row r is the norm of row `row_of[r]`.
+template <int RPW, bool SPREAD = false>
 __global__ void __launch_bounds__(256)
 rmsnorm_vec_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ scale,
                    bf16_t* __restrict__ out, int R, int d, float eps,
-                   const int32_t* gate) {
+                   const int32_t* gate, const int32_t* row_of = nullptr) {
   constexpr int TPR = 256 / RPW;  // threads per row
   static_assert(TPR == 64 || TPR == 256, "a wavefront or the workgroup per row");
   T5D_GATE_READ(gate);
@@ -79,7 +80,9 @@ rmsnorm_vec_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ scal
   const int r = blockIdx.x * RPW + threadIdx.x / TPR;
   const bool row_ok = r < R;  // uniform per wavefront
   const int chunks = d >> 3;
-  const uint4* xr = reinterpret_cast<const uint4*>(x + (size_t)(row_ok ? r : 0) * d);
+  int from = row_ok ? r : 0;
+  if constexpr (SPREAD) from = row_of[from];
+  const uint4* xr = reinterpret_cast<const uint4*>(x + (size_t)from * d);
   float ss = 0.f;
   for (int c = t; c < chunks; c += TPR) {
     float f[8];
@@ -181,6 +184,21 @@ extern "C" int t5d_rmsnorm(void* stream, int dtype, const void* x,
                        as_stream(stream), (const bf16_t*)x,
                        (const bf16_t*)scale, (bf16_t*)out, d, eps, tls_gate);
   T5D_CHECK_LAUNCH("t5d_rmsnorm");
+  return T5D_OK;
+}
+
+extern "C" int t5d_rmsnorm_rows(void* stream, const void* x, const void* scale,
+                                const int32_t* row_of, void* out, int R, int d,
+                                float eps) {
+  T5D_REQUIRE(x && scale && row_of && out, T5D_EINVAL, "t5d_rmsnorm_rows: null pointer");
+  T5D_REQUIRE(R > 0 && d > 0 && d % 8 == 0, T5D_EINVAL, "t5d_rmsnorm_rows: R=%d d=%d", R,
+              d);
+  T5D_REQUIRE(((uintptr_t)x | (uintptr_t)scale | (uintptr_t)out) % 16 == 0, T5D_EINVAL,
+              "t5d_rmsnorm_rows: operand alignment");
+  hipLaunchKernelGGL((rmsnorm_vec_kernel<4, true>), dim3((R + 3) / 4), dim3(256), 0,
+                     as_stream(stream), (const bf16_t*)x, (const bf16_t*)scale,
+                     (bf16_t*)out, R, d, eps, tls_gate, row_of);
+  T5D_CHECK_LAUNCH("t5d_rmsnorm_rows");
   return T5D_OK;
 }
 

@@ -33,11 +33,21 @@ struct EncAttnArgs {
   const bf16_t* bias; // [H, 2E-1]: by (key - query + E - 1)
   const int32_t* len; // [B] valid prefix length (with `valid`: last valid + 1)
   const uint32_t* valid;  // optional [B, (E + 31) / 32]: bit e = position e valid
+  const int32_t* first;   // optional [B + 1]: rows first[b] .. first[b + 1] are text
+                          // b's instead of b * E .. (b + 1) * E (t5d_encoder_rows:
+                          // every position below len, then one or more of padding)
   bf16_t* out;        // [B*E, H*64]
   int B, H, E, Ep, q_stride, k_stride;
 };
 
-constexpr int kMaxEncLen = 2048;
+// Component 16 dt + 4 g + i of the value vector of position e, from V^T.
+__device__ __forceinline__ void value_at(const char* vt, int e, int dt, int gq,
+                                         float (&v)[4]) {
+  const bf16_t* p = reinterpret_cast<const bf16_t*>(vt) + (size_t)(e >> 5) * 2048 +
+                    (16 * dt + 4 * gq) * 32 + (e & 31);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = bf16_to_f32(p[32 * i]);
+}
 
 // ---- up to 64 positions: scores kept in registers -------------------------------
 // A wavefront's 16 queries against the one block of keys:
@@ -69,7 +79,8 @@ enc_attn_short_kernel(EncAttnArgs a) {
   const int l16 = lane & 15, gq = lane >> 4;
   const int h = blockIdx.y, b = blockIdx.z;
   const int E = a.E;
-  const size_t row0 = (size_t)b * E;
+  const size_t row0 = a.first ? a.first[b] : (size_t)b * E;
+  const int rows = a.first ? a.first[b + 1] - a.first[b] : E;  // that are there
 
   // What this lane fetches of K: chunks (8 keys, 1 KB) wave and wave + 4; lane s
   // lands at slot s & 7 of key s >> 3 and therefore reads piece (s & 7) ^ (s >> 3) of
@@ -87,7 +98,7 @@ enc_attn_short_kernel(EncAttnArgs a) {
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int c = wave + 4 * u;
-    const int key = min(8 * c + k_r, E - 1);
+    const int key = min(8 * c + k_r, rows - 1);
     __builtin_amdgcn_global_load_lds(
         (enc_glb_ptr_t)(kbase + (row0 + key) * (size_t)a.k_stride * 2),
         (enc_lds_ptr_t)&s_k[64 * c], 16, 0, 0);
@@ -115,7 +126,7 @@ enc_attn_short_kernel(EncAttnArgs a) {
     s_valid[threadIdx.x] = prefix;
   }
   const int q0 = wave * 16;
-  const int qi = min(q0 + l16, E - 1);
+  const int qi = min(q0 + l16, rows - 1);
   FragE qb[2];
 #pragma unroll
   for (int c = 0; c < 2; ++c)
@@ -133,7 +144,7 @@ enc_attn_short_kernel(EncAttnArgs a) {
   // valid (the keys beyond add exact zeros), else every key; none when its queries
   // lie beyond E.
   int my_tiles = 0;
-  if (q0 < E) {
+  if (q0 < rows) {
     const bool all_valid =
         q0 + 15 < E && ((s_valid[q0 >> 5] >> (q0 & 31)) & 0xffffu) == 0xffffu;
     my_tiles = ((all_valid ? n : E) + 15) >> 4;
@@ -152,7 +163,7 @@ enc_attn_short_kernel(EncAttnArgs a) {
   // Masking is a minimum with the cap: a score never lies below -1e10, so
   // min(x, bf16(-1e10)) is the reference's masked value, min(x, -inf) removes
   // a key that does not exist, min(x, +inf) keeps x.
-  const float* bias_g = s_bias + (E - 1) - qi + 4 * gq;
+  const float* bias_g = s_bias + (E - 1) - min(qi, E - 1) + 4 * gq;
   const float* lim_g = s_lim[q_valid ? 0 : 1] + 4 * gq;
   // scores of key tile kt for this lane: keys 16 kt + 4 g + i of query l16
   uint32_t sc[4][2];
@@ -235,8 +246,20 @@ enc_attn_short_kernel(EncAttnArgs a) {
       oc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va.v, pb.v, oc[dt], 0, 0, 0);
     }
   }
+  // A padded query weighs all E positions alike; padding beyond the rows that are there
+  // has the values of the padding that is.
+  if (rows < E && q0 + l16 < rows && !q_valid) {
+    const float w = (float)(E - rows) * bf16_to_f32(f32_to_bf16(inv));
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      float v[4];
+      value_at(vbase, rows - 1, dt, gq, v);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) oc[dt][i] = fmaf(w, v[i], oc[dt][i]);
+    }
+  }
   // oc[dt][i]: out[q = l16][d = 16 dt + 4 g + i]
-  if (q0 + l16 < E) {
+  if (q0 + l16 < rows) {
     bf16_t* o = a.out + (row0 + q0 + l16) * (size_t)(a.H * 64) + h * 64 + 4 * gq;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
@@ -297,7 +320,9 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, gq = lane >> 4;
   const int E = a.E;
-  const size_t row0 = (size_t)b * E;
+  const size_t row0 = a.first ? a.first[b] : (size_t)b * E;
+  const int rows = a.first ? a.first[b + 1] - a.first[b] : E;  // that are there
+  if (tile * 4 * QW >= rows) return;
 
   // the pieces this lane fetches: keys (rows of 128 bytes, clamped at the last),
   // V^T (blocks of 32 keys: rows of 64 bytes)
@@ -317,7 +342,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   const auto fetch = [&](int jt, uint4* sk, uint4* sv) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const size_t row = row0 + min(jt + k_row[i], E - 1);
+      const size_t row = row0 + min(jt + k_row[i], rows - 1);
       __builtin_amdgcn_global_load_lds(
           (enc_glb_ptr_t)(k_at + row * a.k_stride * 2 + k_piece[i]),
           (enc_lds_ptr_t)(sk + (wave * 2 + i) * 64), 16, 0, 0);
@@ -350,13 +375,16 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   int qi[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    qi[mt] = min(q0 + 16 * mt + l16, E - 1);  // past the end: not stored
+    qi[mt] = min(q0 + 16 * mt + l16, rows - 1);  // past the end: not stored
 #pragma unroll
     for (int c = 0; c < 2; ++c)
       qb[mt][c].u = *reinterpret_cast<const uint4*>(
           a.q + (row0 + qi[mt]) * a.q_stride + h * 64 + 32 * c + 8 * gq);
   }
   __syncthreads();
+  // The keys that a padded query weighs here.  Where rows are given, padding is left
+  // to the end: one of its rows stands for all of it.
+  const int E_here = a.first ? n : E;
   // Keys each wavefront of the workgroup walks: the valid prefix if all of its
   // queries are valid, else all there are (none past the end).
   int my_keys = 0, wg_keys = 0;
@@ -365,10 +393,11 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   for (int w = 0; w < 4; ++w) {
     const int qw = (tile * 4 + w) * QW;
     const uint32_t all = MT == 2 ? 0xffffffffu : 0xffffu;
-    const uint32_t want = qw + QW <= E ? all : qw < E ? (1u << (E - qw)) - 1 : 0;
-    const uint32_t there = qw < E ? (s_valid[qw >> 5] >> (qw & 31)) & want : 0;
-    const bool valid = qw < E && there == want;
-    const int keys = qw >= E ? 0 : valid ? n : E;
+    const uint32_t want =
+        qw + QW <= rows ? all : qw < rows ? (1u << (rows - qw)) - 1 : 0;
+    const uint32_t there = qw < rows ? (s_valid[qw >> 5] >> (qw & 31)) & want : 0;
+    const bool valid = qw < rows && there == want;
+    const int keys = qw >= rows ? 0 : valid ? n : E_here;
     if (w == wave) {
       my_keys = keys;
       my_valid = valid;
@@ -401,10 +430,10 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int key = jt + 32 * kb + 16 * (e >> 1) + 4 * gq + 2 * (e & 1);
-          w[e] = (key < E ? 0x3F80u : 0u) | (key + 1 < E ? 0x3F800000u : 0u);
+          w[e] = (key < E_here ? 0x3F80u : 0u) | (key + 1 < E_here ? 0x3F800000u : 0u);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
-            l[mt] += (float)((key < E) + (key + 1 < E));
+            l[mt] += (float)((key < E_here) + (key + 1 < E_here));
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
@@ -431,7 +460,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
           s[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][c].v, qb[mt][c].v,
                                                              s[t][mt], 0, 0, 0);
     // bias by key - query: 16 keys further on is 16 queries further back
-    const float* near = s_bias + 16 + (E - 1) - qi[0] + jt + 4 * gq;
+    const float* near = s_bias + 16 + (E - 1) - min(qi[0], E - 1) + jt + 4 * gq;
     float bias[5][4];
 #pragma unroll
     for (int t = 0; t < 5; ++t)
@@ -465,7 +494,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int key = 16 * t + 4 * gq + i;
-            const bool exists = jt + key < E;
+            const bool exists = jt + key < E_here;
             const bool ok = ((t < 2 ? v0 : v1) >> (key & 31)) & 1u;
             const float x = q_valid ? s[t][mt][i] : 0.f;
             s[t][mt][i] = (q_valid ? ok : exists) ? x : -INFINITY;
@@ -545,9 +574,9 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  // (wg_keys >= 1, as a workgroup has a query, which is valid or walks all keys: every
-  // tile that is fetched is met before the end)
-  for (int jt = 0; jt < wg_keys; jt += 2 * KB) {
+  // (the first tile has been fetched whatever there is to walk, and every tile that is
+  // fetched is met before the end)
+  for (int jt = 0; jt == 0 || jt < wg_keys; jt += 2 * KB) {
     meet();
     if (jt + KB < wg_keys) fetch(jt + KB, s_k1, s_v1);
     attend(jt, s_k0, s_v0);
@@ -558,9 +587,22 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    const float inv = 1.0f / rows_sum(l[mt]);
+    float sum = rows_sum(l[mt]);
     const int q = q0 + 16 * mt + l16;
-    if (q >= E) continue;
+    if (q >= rows) continue;
+    // (such a query's maximum is 0, or was never raised: its keys weigh 1)
+    if (a.first && n < E && q >= n) {
+      const float w = (float)(E - n);
+      sum += w;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        float v[4];
+        value_at(v_at, n, dt, gq, v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) oc[dt][mt][i] = fmaf(w, v[i], oc[dt][mt][i]);
+      }
+    }
+    const float inv = 1.0f / sum;
     bf16_t* o = a.out + (row0 + q) * (size_t)(a.H * 64) + h * 64 + 4 * gq;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
@@ -678,16 +720,11 @@ extern "C" int t5d_encoder_attention(void* stream, const void* q, const void* k,
                                        k_stride, 0);
 }
 
-extern "C" int t5d_encoder_attention_variant(
-    void* stream, const void* q, const void* k, const void* v_t,
-    const void* rel_bias, const int32_t* enc_len, const uint32_t* valid_bits,
-    void* out, int B, int H, int E, int Ep, int q_stride, int k_stride,
-    int variant) {
-  T5D_REQUIRE(variant >= 0 && variant <= 2 && (variant != 2 || E <= 512),
-              T5D_EINVAL,
-              "t5d_encoder_attention_variant: variant %d (0, 1, and 2 where "
-              "E <= 512)",
-              variant);
+static int encoder_attention(void* stream, const void* q, const void* k, const void* v_t,
+                             const void* rel_bias, const int32_t* enc_len,
+                             const uint32_t* valid_bits, const int32_t* first,
+                             int most, void* out, int B, int H, int E, int Ep,
+                             int q_stride, int k_stride) {
   T5D_REQUIRE(q && k && v_t && rel_bias && enc_len && out, T5D_EINVAL,
               "t5d_encoder_attention: null pointer");
   T5D_REQUIRE(B > 0 && H > 0 && E > 0 && Ep >= E && Ep % 32 == 0,
@@ -710,14 +747,14 @@ extern "C" int t5d_encoder_attention_variant(
   EncAttnArgs a;
   a.q = (const bf16_t*)q; a.k = (const bf16_t*)k; a.vt = (const bf16_t*)v_t;
   a.bias = (const bf16_t*)rel_bias; a.len = enc_len; a.out = (bf16_t*)out;
-  a.valid = valid_bits;
+  a.valid = valid_bits; a.first = first;
   a.B = B; a.H = H; a.E = E; a.Ep = Ep; a.q_stride = q_stride; a.k_stride = k_stride;
   if (E <= kShortEnc) {
     hipLaunchKernelGGL(enc_attn_short_kernel, dim3(1, H, B), dim3(256), 0,
                        as_stream(stream), a);
   } else {
-    const bool low = one_pass_64(B, H, E);
-    const int tiles = low ? (E + 63) / 64 : (E + 127) / 128;
+    const bool low = one_pass_64(B, H, most);
+    const int tiles = low ? (most + 63) / 64 : (most + 127) / 128;
     const dim3 groups(((unsigned)B * H + 7) / 8 * 8 * tiles);
     if (low)
       hipLaunchKernelGGL(enc_attn_tile_kernel<1>, groups, dim3(256), 0,
@@ -728,6 +765,31 @@ extern "C" int t5d_encoder_attention_variant(
   }
   T5D_CHECK_LAUNCH("t5d_encoder_attention");
   return T5D_OK;
+}
+
+extern "C" int t5d_encoder_attention_variant(
+    void* stream, const void* q, const void* k, const void* v_t,
+    const void* rel_bias, const int32_t* enc_len, const uint32_t* valid_bits,
+    void* out, int B, int H, int E, int Ep, int q_stride, int k_stride,
+    int variant) {
+  T5D_REQUIRE(variant >= 0 && variant <= 2 && (variant != 2 || E <= 512),
+              T5D_EINVAL,
+              "t5d_encoder_attention_variant: variant %d (0, 1, and 2 where "
+              "E <= 512)",
+              variant);
+  return encoder_attention(stream, q, k, v_t, rel_bias, enc_len, valid_bits, nullptr, E,
+                           out, B, H, E, Ep, q_stride, k_stride);
+}
+
+extern "C" int t5d_encoder_attention_rows(
+    void* stream, const void* q, const void* k, const void* v_t, const void* rel_bias,
+    const int32_t* enc_len, const int32_t* first, int most, void* out, int B, int H,
+    int E, int Ep, int q_stride, int k_stride) {
+  T5D_REQUIRE(first && most > 0 && most <= (E + 3) / 4 * 4, T5D_EINVAL,
+              "t5d_encoder_attention_rows: first %p, at most %d rows of a text of %d",
+              (const void*)first, most, E);
+  return encoder_attention(stream, q, k, v_t, rel_bias, enc_len, nullptr, first, most,
+                           out, B, H, E, Ep, q_stride, k_stride);
 }
 
 extern "C" int t5d_encoder_attention_f32(void* stream, const float* qkv,

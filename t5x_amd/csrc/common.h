@@ -9,6 +9,9 @@
 
 namespace t5d {
 
+constexpr int kMaxEncLen = 2048;  // positions of an encoder text
+
+
 // ---- error reporting --------------------------------------------------------
 void set_error(const char* fmt, ...);
 

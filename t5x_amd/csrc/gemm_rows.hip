@@ -71,6 +71,7 @@ struct RowsGemmArgs {
   int epilogue;            // T5D_EPI_*
   int layout;              // T5D_OUT_*
   int E, Ep, H;            // heads layouts: m = b * E + e, n = h * 64 + d
+  const int32_t* at;       // value layout: b << 12 | e of every 4 rows instead, or null
   int lda;                 // row stride of A
   float* C32;              // float32 output rows instead of C (rows layout, no
   int ldc, n_store;        // epilogue): row stride, columns stored of the N
@@ -103,7 +104,15 @@ __device__ __forceinline__ void rows_epilogue_values(
   for (int mt = 0; mt < MT; ++mt) {
     const int m = m0 + 16 * mt + 4 * gq;
     if (m >= g.M) continue;
-    const int b = m / g.E, e = m - b * g.E;
+    int b, e;
+    if (g.at) {
+      const int p = g.at[m >> 2];
+      b = p >> 12;
+      e = p & 4095;
+    } else {
+      b = m / g.E;
+      e = m - b * g.E;
+    }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       if (nt0 + nt >= n_tiles) continue;
@@ -753,11 +762,10 @@ extern "C" int t5d_gemm_rows(void* stream, int w_dtype, const void* A,
                              N, epilogue, out_layout, E, Ep, 0);
 }
 
-extern "C" int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
-                                   const void* W, const float* scales,
-                                   const void* residual, void* C, int64_t M,
-                                   int K, int N, int epilogue, int out_layout,
-                                   int E, int Ep, int tile) {
+static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
+                     const float* scales, const void* residual, void* C, int64_t M,
+                     int K, int N, int epilogue, int out_layout, int E, int Ep,
+                     const int32_t* at, int tile) {
   T5D_REQUIRE(A && W && C, T5D_EINVAL, "t5d_gemm_rows: null pointer");
   T5D_REQUIRE(tile >= 0 && tile <= 3, T5D_EINVAL,
               "t5d_gemm_rows_tiled: tile %d (0 chosen here, 1: 256 x 128, "
@@ -782,7 +790,7 @@ extern "C" int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
   int H = 0;
   if (out_layout != T5D_OUT_ROWS) {
     T5D_REQUIRE(epilogue == T5D_EPI_NONE && N % 64 == 0 && E > 0 && Ep >= E &&
-                    M % E == 0 && E % 4 == 0 && Ep % 32 == 0,
+                    (at ? M % 4 == 0 : M % E == 0 && E % 4 == 0) && Ep % 32 == 0,
                 T5D_EINVAL,
                 "t5d_gemm_rows: heads layout needs epilogue none, N %% 64 == 0,"
                 " M %% E == 0, E %% 4 == 0, Ep %% 32 == 0 (N=%d E=%d Ep=%d)", N,
@@ -795,11 +803,29 @@ extern "C" int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
   g.residual = (const bf16_t*)residual; g.C = (bf16_t*)C;
   g.M = (int)M; g.K = K; g.N = N;
   g.epilogue = epilogue; g.layout = out_layout;
-  g.E = E; g.Ep = Ep; g.H = H;
+  g.E = E; g.Ep = Ep; g.H = H; g.at = at;
   g.lda = K; g.C32 = nullptr; g.ldc = g.n_store = N;
   g.glu_limit = g.glu_alpha = g.glu_add = 0.f;
   g.gate = nullptr; g.grp = GroupTiles(); g.n_tiles = 0;
   return launch_rows(as_stream(stream), w_dtype, g, tile);
+}
+
+extern "C" int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
+                                   const void* W, const float* scales,
+                                   const void* residual, void* C, int64_t M,
+                                   int K, int N, int epilogue, int out_layout,
+                                   int E, int Ep, int tile) {
+  return gemm_rows(stream, w_dtype, A, W, scales, residual, C, M, K, N, epilogue,
+                   out_layout, E, Ep, nullptr, tile);
+}
+
+extern "C" int t5d_gemm_rows_values(void* stream, int w_dtype, const void* A,
+                                    const void* W, const float* scales, void* C,
+                                    int64_t M, int K, int N, const int32_t* at, int E,
+                                    int Ep) {
+  T5D_REQUIRE(at, T5D_EINVAL, "t5d_gemm_rows_values: null pointer");
+  return gemm_rows(stream, w_dtype, A, W, scales, nullptr, C, M, K, N, T5D_EPI_NONE,
+                   T5D_OUT_HEADS_VALUE, E, Ep, at, 0);
 }
 
 int t5d::launch_dense_rows(hipStream_t s, const void* A, int lda,
@@ -814,7 +840,7 @@ int t5d::launch_dense_rows(hipStream_t s, const void* A, int lda,
   g.C32 = out_f32 ? (float*)C : nullptr;
   g.M = M; g.K = K; g.N = N;
   g.epilogue = epilogue; g.layout = T5D_OUT_ROWS;
-  g.E = g.Ep = g.H = 0;
+  g.E = g.Ep = g.H = 0; g.at = nullptr;
   g.lda = lda; g.ldc = ldc; g.n_store = n_store;
   g.gate = nullptr; g.grp = GroupTiles(); g.n_tiles = 0;
   g.glu_limit = glu_limit; g.glu_alpha = glu_alpha; g.glu_add = glu_add;
@@ -828,7 +854,7 @@ int t5d::launch_grouped_rows(hipStream_t s, const GroupedArgs& a, int n_tiles) {
   g.C = (bf16_t*)a.C; g.C32 = nullptr;
   g.M = 0; g.K = a.K; g.N = a.N;
   g.epilogue = a.epilogue; g.layout = T5D_OUT_ROWS;
-  g.E = g.Ep = g.H = 0;
+  g.E = g.Ep = g.H = 0; g.at = nullptr;
   g.lda = a.lda; g.ldc = a.ldc; g.n_store = a.n_store;
   g.glu_limit = a.glu_limit; g.glu_alpha = a.glu_alpha; g.glu_add = a.glu_add;
   g.gate = a.gate; g.grp = a.grp; g.n_tiles = n_tiles;

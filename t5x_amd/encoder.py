@@ -56,14 +56,51 @@ class EncoderKernelWeights:
     return self._bias[E]
 
 
+def _encode_rows(cfg, w, rows, device):
+  """_encode_hip over the rows that there are (ops.EncoderRows)."""
+  from t5x_amd import ops
+  HD = cfg.num_heads * 64
+  bias = w.rel_bias(rows.E)
+  x = ops.embed(w.embedding, rows.ids)
+  v_t = torch.zeros((rows.B, cfg.num_heads, (rows.E + 31) // 32, 64, 32),
+                    dtype=x.dtype, device=device)
+  for l in w.layers:
+    xn = ops.rmsnorm(x, l['ln_attn'])
+    qk = ops.gemm_rows(xn, l['qk'])                       # [M, q | k]
+    ops.gemm_rows_values(xn, l['v'], rows, out=v_t)
+    attn = ops.encoder_attention_rows(qk[:, :HD], qk[:, HD:], v_t, bias, rows)
+    x = ops.gemm_rows(attn, l['o'], residual=x)
+    y = ops.rmsnorm(x, l['ln_mlp'])
+    h = ops.gemm_rows(y, l['wi'])
+    x = ops.gemm_rows(h, l['wo'], residual=x)
+  return ops.rmsnorm_rows(x, w.ln_final, rows.row_of).view(rows.B, rows.E,
+                                                          cfg.emb_dim)
+
+
 def _encode_hip(module, params, tokens):
   """bfloat16 encoder on the HIP kernels; tokens [B, E] int64 on the device."""
-  from t5x_amd import _lib, ops
+  from t5x_amd import ops
   cfg, dev = module.config, module._dev()
   key = ('hip', id(params))
   if key not in module._enc_weights:
     module._enc_weights[key] = (params, EncoderKernelWeights(cfg, params, dev))
   w = module._enc_weights[key][1]
+  B, E = tokens.shape
+  if E <= ops.MAX_ENCODER_LENGTH and cfg.emb_dim % 8 == 0:
+    rows = ops.EncoderRows(tokens)
+    if not rows.odd:
+      return _encode_rows(cfg, w, rows, dev)
+  if E % 4:
+    # The dense kernel's head-layout epilogue takes lengths in multiples of 4:
+    # pad with padding tokens (masked keys; their own rows are dropped again).
+    tokens = torch.nn.functional.pad(tokens, (0, -E % 4))
+    return _encode_positions(cfg, w, tokens, dev)[:, :E].contiguous()
+  return _encode_positions(cfg, w, tokens, dev)
+
+
+def _encode_positions(cfg, w, tokens, dev):
+  """_encode_hip over every position: padding inside a text is masked by bits."""
+  from t5x_amd import _lib, ops
   B, E = tokens.shape
   H = cfg.num_heads
   HD = H * 64
@@ -172,16 +209,8 @@ def encode(module, params, encoder_input_tokens):
   if not isinstance(tokens, torch.Tensor):
     tokens = torch.as_tensor(np.asarray(tokens), device=dev)
   tokens = tokens.to(dev).long()
-  B, E = tokens.shape
   if cfg.dtype == 'float32':
     return _encode_hip_f32(module, params, tokens)
   if cfg.dtype != 'bfloat16':
     raise ValueError(f'unsupported encoder dtype {cfg.dtype}')
-  if E % 4 == 0:
-    return _encode_hip(module, params, tokens)
-  # The dense kernel's head-layout epilogue takes lengths in multiples of 4:
-  # pad with padding tokens (masked keys; their own rows are dropped again).
-  E4 = (E + 3) // 4 * 4
-  padded = torch.zeros((B, E4), dtype=tokens.dtype, device=dev)
-  padded[:, :E] = tokens
-  return _encode_hip(module, params, padded)[:, :E].contiguous()
+  return _encode_hip(module, params, tokens.contiguous())

@@ -147,6 +147,20 @@ def rmsnorm(x, scale, out=None, eps=1e-6):
   return out
 
 
+def rmsnorm_rows(x, scale, row_of, eps=1e-6):
+  """[R, d] whose row r is the norm of x's row row_of[r] (bfloat16)."""
+  _chk(x, 'x', torch.bfloat16, 2)
+  _chk(scale, 'scale', x.dtype, 1)
+  _chk(row_of, 'row_of', torch.int32, 1)
+  R, d = row_of.shape[0], x.shape[1]
+  if scale.shape[0] != d:
+    raise ValueError('scale length mismatch')
+  out = torch.empty((R, d), dtype=x.dtype, device=x.device)
+  _lib.call('t5d_rmsnorm_rows', _s(), x.data_ptr(), scale.data_ptr(),
+            row_of.data_ptr(), out.data_ptr(), R, d, float(eps))
+  return out
+
+
 def gemm(a, w: PackedWeight, out=None, residual=None, out_dtype=None,
          norm_scale=None, eps=1e-6):
   """C = epilogue(a @ W).  a [M, K]; geglu weights give [M, F].  With
@@ -496,6 +510,47 @@ def gemm_rows(a, w: PackedWeight, out=None, residual=None,
   return out
 
 
+def gemm_rows_values(a, w: PackedWeight, rows, out):
+  """gemm_rows into `out` [B, H, Ep/32, 64, 32] for the rows of an EncoderRows."""
+  _chk(a, 'a', torch.bfloat16, 2)
+  _chk(out, 'out', a.dtype, 5)
+  M, K = a.shape
+  Ep = out.shape[2] * 32
+  if (M != rows.M or K != w.K or w.w_dtype == F32 or w.geglu or
+      tuple(out.shape) != (rows.B, w.N // 64, Ep // 32, 64, 32)):
+    raise ValueError(f'a is [{M}, {K}], out {tuple(out.shape)}: {rows.M} rows, '
+                     f'kernel K={w.K} N={w.N}')
+  _lib.call('t5d_gemm_rows_values', _s(), w.w_dtype, a.data_ptr(), w.data.data_ptr(),
+            _lib.ptr(w.scales), out.data_ptr(), M, K, w.N, rows.at.data_ptr(), rows.E,
+            Ep)
+  return out
+
+
+MAX_ENCODER_LENGTH = 2048  # positions of a text (kMaxEncLen)
+
+
+class EncoderRows:
+  """The rows an encoder computes for tokens [B, E] (t5d_encoder_rows): those of
+  every text and one that stands for its padding.  `odd`: a text is something else
+  than tokens > 0 followed by zeros, and only `len` (the number of tokens > 0) holds.
+  Waits for the device once, to learn how many rows there are."""
+
+  def __init__(self, tokens):
+    _chk(tokens, 'tokens', torch.int64, 2)
+    self.B, self.E = B, E = tokens.shape
+    E4 = (E + 3) // 4 * 4
+    sizes = [B, B, B + 1, B * E4, B * E, B * E4 // 4, 3]
+    (self.len, odd, self.first, self._ids, self.row_of, self._at,
+     summary) = torch.empty(sum(sizes), dtype=torch.int32,
+                            device=tokens.device).split(sizes)
+    _lib.call('t5d_encoder_rows', _s(), tokens.data_ptr(), B, E,
+              *(t.data_ptr() for t in (self.len, odd, self.first, self._ids,
+                                       self.row_of, self._at, summary)))
+    self.M, self.most, any_odd = summary.tolist()
+    self.odd = bool(any_odd)
+    self.ids, self.at = self._ids[:self.M], self._at[:self.M // 4]
+
+
 def _valid_bits(valid_bits, B, E):
   if valid_bits is None:
     return None
@@ -549,6 +604,28 @@ def encoder_attention(q, k, v_t, rel_bias, enc_len, out=None, valid_bits=None,
             v_t.data_ptr(), rel_bias.data_ptr(), enc_len.data_ptr(),
             _valid_bits(valid_bits, B, E), out.data_ptr(), B, H, E, Ep,
             q.stride(0), k.stride(0), int(variant))
+  return out
+
+
+def encoder_attention_rows(q, k, v_t, rel_bias, rows):
+  """encoder_attention over the rows of an EncoderRows: q, k [rows.M, H*64] views ->
+  [rows.M, H*64]."""
+  _chk(v_t, 'v_t', torch.bfloat16, 5)
+  _chk(rel_bias, 'rel_bias', torch.bfloat16, 2)
+  B, H, blocks, D, w = v_t.shape
+  if ((B, D, w) != (rows.B, 64, 32) or
+      tuple(rel_bias.shape) != (H, 2 * rows.E - 1)):
+    raise ValueError('v_t [B, H, Ep/32, 64, 32], rel_bias [H, 2E-1]')
+  for name, t in (('q', q), ('k', k)):
+    if (not t.is_cuda or t.dtype != torch.bfloat16 or t.dim() != 2 or
+        t.stride(1) != 1 or tuple(t.shape) != (rows.M, H * 64)):
+      raise ValueError(f'{name} must be a [{rows.M}, H*64] bfloat16 view with unit '
+                       f'column stride, got {tuple(t.shape)}')
+  out = torch.empty((rows.M, H * 64), dtype=torch.bfloat16, device=v_t.device)
+  _lib.call('t5d_encoder_attention_rows', _s(), q.data_ptr(), k.data_ptr(),
+            v_t.data_ptr(), rel_bias.data_ptr(), rows.len.data_ptr(),
+            rows.first.data_ptr(), rows.most, out.data_ptr(), B, H, rows.E, blocks * 32,
+            q.stride(0), k.stride(0))
   return out
 
 

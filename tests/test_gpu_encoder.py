@@ -787,3 +787,44 @@ def test_encoder_attention_random_shapes(ops):
     err = (got - want).abs()
     assert float(err.max()) <= 2e-2 + 2.0**-6 * float(want.abs().max()), (
         case, B, H, E, holes, float(err.max()))
+
+
+@pytest.mark.parametrize('E', [5, 20, 62, 64, 65, 130, 257])
+def test_encoder_over_the_rows_that_there_are(E):
+  """Texts that are empty, full and in between: the rows of the tokens have the bits
+  that the encoder over every position gives; padding, which is one row per text,
+  lies within the bfloat16 roundings of three layers (its uniform sum is added up in
+  another order: a result may round to its neighbour, 2^-8, in each of the 6
+  branches)."""
+  from t5x_amd import encoder, network, ops as o
+  ocfg, cfg = _tiny_cfgs()
+  params = ot5.init_params(ocfg, seed=3)
+  module = network.Transformer(cfg, torch.device('cuda'))
+  rs = np.random.RandomState(E)
+  lens = [0, E, 1, E - 1, E // 2, E, 0, max(1, E - 4)]
+  tokens = rs.randint(2, cfg.vocab_size, size=(len(lens), E))
+  tokens[np.arange(E)[None, :] >= np.array(lens)[:, None]] = 0
+  t = torch.as_tensor(tokens, device='cuda').long()
+  got = encoder.encode(module, params, t)
+  w = next(iter(module._enc_weights.values()))[1]
+  rows = o.EncoderRows(t)
+  assert rows.len.tolist() == lens and not rows.odd
+  per = [-(-(n + 1 if n < E else E) // 4) * 4 for n in lens]
+  assert rows.first.tolist() == list(np.concatenate([[0], np.cumsum(per)]))
+  assert (rows.M, rows.most) == (sum(per), max(per))
+  padded = torch.nn.functional.pad(t, (0, -E % 4))
+  want = encoder._encode_positions(cfg, w, padded, got.device)[:, :E]
+  valid = t > 0
+  assert torch.equal(got[valid], want[valid])
+  if E % 4 == 0:
+    a, b = got[~valid].double(), want[~valid].double()
+    assert ((a - b).norm() / b.norm()).item() < 6 * 2.0 ** -8
+  for text in (got[0], got[4, E // 2:]):  # one result for all padding of a text
+    assert torch.equal(text, text[:1].expand_as(text))
+  # tokens below zero or zeros inside a text: every position as before
+  t[3, 1] = -7 if E % 2 else 0
+  assert o.EncoderRows(t).odd
+  other = encoder.encode(module, params, t)
+  again = encoder._encode_positions(cfg, w, torch.nn.functional.pad(t, (0, -E % 4)),
+                                    got.device)[:, :E]
+  assert torch.equal(other, again)
