@@ -169,13 +169,11 @@ int t5d_gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
                   int64_t M, int K, int N, int epilogue, int out_layout, int E,
                   int Ep);
 
-/* t5d_gemm_rows with the workgroup tile of the caller's choice: tile 1 =
- * 256 rows x 128 columns (4 wavefronts, two workgroups per CU; 128 or 64 rows
- * where bfloat16 weights leave CUs without a workgroup otherwise), tile 2 =
- * 256 x 256 and tile 3 = 256 x 192 (8 wavefronts, one workgroup per CU;
- * bfloat16 weights and K >= 64, otherwise tile 1 is used), tile 0 = what
- * t5d_gemm_rows picks from the shape.  Results have the same bits for every
- * tile.  For tuning and for testing every kernel at any size. */
+/* t5d_gemm_rows with the workgroup tile of the caller's choice: tile 1 = 128 columns
+ * of 128 rows, or of 64 where those cost less, tile 2 = 256 and tile 3 = 192 columns
+ * of 128 rows (4 wavefronts each; bfloat16 weights and K >= 64, otherwise 256 rows x
+ * 128 columns), tile 0 = what t5d_gemm_rows picks from the shape.  Results have the
+ * same bits for every tile.  For tuning and for testing every kernel at any size. */
 int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
                         const void* W, const float* scales,
                         const void* residual, void* C, int64_t M, int K, int N,

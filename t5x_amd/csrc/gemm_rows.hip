@@ -142,12 +142,13 @@ __device__ __forceinline__ void rows_epilogue_values(
 // another lane's write (to it they are accesses of unrelated addresses).
 // DENSE: one of the epilogues of t5d_dense instead: 1 = T5D_EPI_CLAMPED_GLU (first
 // column of a pair: gate, second: up), 2 = float32 rows.
-constexpr int kRowsStageBytes = 16 * 144;
+template <int NT> constexpr int kRowsStageStride = NT == 2 ? 80 : 144;
+template <int NT> constexpr int kRowsStageBytes = 16 * kRowsStageStride<NT>;
 template <int DENSE, bool SCALED, int MT, int NT>
 __device__ __forceinline__ void rows_epilogue_staged(
     const RowsGemmArgs& g, const f32x4_r (&acc)[MT][NT], int m0, int nt0,
     int n_tiles, int lane, char* stage) {
-  static_assert(NT == 3 || NT == 4, "a wavefront's slice: 48 or 64 columns");
+  static_assert(NT >= 2 && NT <= 4, "a wavefront's slice: 32 to 64 columns");
   const int l16 = lane & 15, gq = lane >> 4;
   // int8 weights: the scale of each of this lane's 4 columns
   float4 sc[NT];
@@ -265,7 +266,7 @@ __device__ __forceinline__ void rows_epilogue_staged(
   for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-      *reinterpret_cast<uint2*>(stage + l16 * 144 + (16 * nt + 4 * gq) * 2) =
+      *reinterpret_cast<uint2*>(stage + l16 * kRowsStageStride<NT> + (16 * nt + 4 * gq) * 2) =
           pack4(value(mt, nt, 0), value(mt, nt, 1),
                 value(mt, nt, 2), value(mt, nt, 3));
     asm volatile("" ::: "memory");
@@ -273,7 +274,7 @@ __device__ __forceinline__ void rows_epilogue_staged(
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       back[j] = *reinterpret_cast<const uint4*>(
-          stage + min(RPI * j + prow, 15) * 144 + piece * 16);
+          stage + min(RPI * j + prow, 15) * kRowsStageStride<NT> + piece * 16);
     asm volatile("" ::: "memory");
     if (residual) {
 #pragma unroll
@@ -415,124 +416,139 @@ rows_gemm_kernel(RowsGemmArgs g) {
 
   if (SWAP) {
     // (the loop ends with a barrier: every wavefront is done with the tiles)
-    static_assert(sizeof(s_t[0]) >= 4 * kRowsStageBytes, "stage too small");
+    static_assert(sizeof(s_t[0]) >= 4 * kRowsStageBytes<NT>, "stage too small");
     rows_epilogue_staged<DENSE, sizeof(WT) == 1>(
         g, acc, m0, nt0, n_tiles, lane,
-        reinterpret_cast<char*>(&s_t[0][0][0]) + wave * kRowsStageBytes);
+        reinterpret_cast<char*>(&s_t[0][0][0]) + wave * kRowsStageBytes<NT>);
   } else {
     rows_epilogue_values(g, acc, m0, nt0, n_tiles, l16, gq);
   }
 }
 
-// ---- the same tile with operands loaded straight into LDS ---------------------
-// rows_gemm_kernel keeps one k-tile of loads in flight per workgroup (staging
-// registers), which covers a fifth of the memory latency; the matrix cores
-// wait for the rest.  Here the 24 operand tiles of a k-tile go from memory
-// into LDS without passing through registers (global_load_lds, 16 bytes per
-// lane, lane l of an instruction landing at byte 16 l of the destination), in
-// a ring of three stages, so two k-tiles are in flight while one is
-// multiplied.  One barrier per k-tile, placed by hand together with the wait
-// for "all but my newest six loads": the stages are three separate arrays and
-// the K loop handles three k-tiles per round, so that the compiler can tell a
-// read of one stage from a load into another and adds no wait of its own.
-// An activation tile is fetched with lane 4 q + j reading row q, piece
-// j ^ swap(q / 4) — four neighbouring lanes still read 64 contiguous bytes —
-// which puts piece p of row r at slot 4 r + (p ^ swap(r / 4)).  A 16-byte read
-// serves 16 lanes at a time: 0..3 and 12..15 of one quarter wavefront with 4..11
-// of its neighbour, which want the neighbouring piece.  With swap = 0, 0, 3, 3
-// their 16 slots differ mod 16.  (Slots that differ within a quarter, by a
-// rotation or an XOR by r / 4, made 40 % of the cycles of LDS reads bank conflicts, now
-// 3 to 7 %, by the counters at 16384 x 4096 x 4096 (35.1 M -> 1.6 M cycles), 16384 x 2048
-// x 768 and 8192 x 1024 x 5632: the last, gated, 97 us, 16384 x 768 x 4096 gated 123 us,
-// now 90 and 115 us.)
-// bfloat16 weights (int8 tiles must be widened on the way).
+// ---- bfloat16 weights, K >= 64: rows through LDS, weights into registers ---------
+// A workgroup of 4 wavefronts owns BM = 16 MT rows x BN = 64 NT columns, a wavefront all
+// rows of 16 NT columns.  So every weight is wanted by one wavefront only, and packed
+// weights come in operand order: they go straight from memory into registers, two
+// k-tiles of 32 ahead in three sets.  Rows are wanted by all four: they go straight into
+// LDS (buffer_load ... lds, 16 bytes per lane), 64 of K at a time in a ring of three
+// stages, whole 128-byte lines of 8 rows per instruction; one barrier per 64 of K.
+// Operand reads from LDS run 16 rows ahead of the products, behind scheduling fences.
+// Piece p of row r lies at slot p ^ (r / 2 % 8) of its 8: a 16-byte read serves lanes
+// 0..3 and 12..15 of one quarter wavefront with 4..11 of its neighbour, which want
+// the neighbouring piece, and these 16 then cover all banks.
+//
+// What bounds it, and why this split (measured, us; before: both operands through LDS,
+// 32 of K per barrier, 256 x 256 by 8 wavefronts or 256 x 192 or 256 x 128):
+//  - LDS: 128 x 64 per wavefront with both operands in LDS reads 24 KB and writes 8 KB
+//    per 64 of K and wavefront, 2048 clocks of LDS beside 2048 of the matrix cores.
+//    Weights in registers leave 1280.
+//  - the order loads return in: a wavefront's loads come back as they were issued, so a
+//    weight tile that is asked for behind rows that come from memory waits for them.
+//    Rows are therefore requested in the middle of a step, behind the weights of the
+//    next one (16384 x 768 x 768: 28.5 the other way round, 25.6 so).
+//  - prologue and epilogue, which one workgroup per CU cannot cover: two or more share
+//    one, each in its own phase.
+//  16384 x 768 x 4096 gated 113.8 -> 92, 10300 x 768 x 4096 gated 77 -> 61, 10300 x 2048
+//  x 768 46.7 -> 33, 5000 x 2816 x 1024 47 -> 34, 8192 x 1024 x 5632 gated 91 -> 81,
+//  14000 x 1024 x 5632 gated 161 -> 132, 16384 x 4096 x 4096 412 -> 385 (1428 TFLOP/s;
+//  matrix instructions alone, on random numbers, reach 2000 at the clock that is left
+//  then), 2000 x 2048 x 768 16.9 -> 13, 1000 x 1024 x 5632 20.8 -> 14.3.
+//
+// Every wait is counted: the loop is straight-line code (rounds of three steps, as the
+// ring and the register sets want; what is left over stands behind it), requests past
+// the end ask for the last step again.  (global_load ... lds would do for rows, but the
+// compiler takes it for a flat access, after which it waits for everything.)
+// GROUPED: see GroupTiles (gemm_tiles.h); a tile of 256 rows is two workgroups.
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef __attribute__((address_space(1))) const void* glb_ptr_t;
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_r;
 
-// WN: wavefront columns of the workgroup, 2 (256 x 128 tile, 4 wavefronts, two
-// workgroups per CU; 128 and 64 rows with MT 4 and 2) or 4 (256 x 256, 8 wavefronts, one per CU).
-// Measured on the gated MLP input projection of the T5.1.1-base encoder
-// (16384 x 768 x 4096): 182 -> 176 us per launch with the ring alone, 123 us
-// with the epilogue below (the library tanh and the 8-byte stores were a
-// third of the launch), 118 us with the 256 x 256 tile.  The same tile from 4
-// wavefronts of 128 x 128 (accumulators in the accumulation registers) lasts
-// 257 us: with one wavefront per SIMD nothing covers the operand reads from
-// LDS.
-// GROUPED: see GroupTiles (gemm_tiles.h).
-template <bool SWAP, int NT, int WN, int DENSE = 0, bool GROUPED = false,
-          int MT = kRowsMT>
-__global__ void __launch_bounds__(128 * WN, MT < 8 ? 3 : WN == 2 ? 2 : 1)
-rows_gemm_direct_kernel(RowsGemmArgs g) {
-  constexpr int BM = 32 * MT, ATILES = 2 * MT;
-  constexpr int WAVES = 2 * WN;         // 2 rows of WN wavefronts
-  constexpr int BN = WN * NT * 16;      // columns of the workgroup tile
-  constexpr int AL = ATILES / WAVES;    // activation tiles a wavefront loads per stage
-  constexpr int WTILES = WN * NT;       // weight tiles of a stage
-  // weight tiles a wavefront loads per stage; when they do not divide evenly
-  // some wavefronts load a tile a second time (same bytes to the same place)
-  constexpr int WL = (WTILES + WAVES - 1) / WAVES;
-  constexpr int TILES = ATILES + WN * NT;
-  // Before every barrier: all but my newest AL + WL loads have landed AND all
-  // my reads of LDS have returned, s_waitcnt vmcnt(AL + WL) lgkmcnt(0).  The
-  // second half matters: the barrier orders instructions that have been
-  // issued, not LDS reads that have completed, and the compiler is free to
-  // sink the last operand reads and matrix instructions of a k-tile below the
-  // next barrier.  Without the wait a workgroup's fastest wavefront could
-  // refill the stage while the slowest still had reads of it queued (seen as
-  // one wrong 16-row slice in about one launch in ten at 16384 x 768).
-  constexpr int kWaitStage = 0x070 | (AL + WL);
-  constexpr int kWaitAll = 0x070;
-  // [tile][lane]: activations (rows 16 t ..), then the weights
-  __shared__ uint4 s_t0[TILES][64];
-  __shared__ uint4 s_t1[TILES][64];
-  __shared__ uint4 s_t2[TILES][64];
-  int group_n_blk = 0;
-  if constexpr (GROUPED) {
-    T5D_GATED(g.gate);
-    // 4 consecutive tiles of rows, most of them of one group, on one XCD, all
-    // columns of a tile in a row: rows and kernels come from that XCD's L2.
-    const int n_blocks = ((g.N >> 4) + BN / 16 - 1) / (BN / 16);
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int t = slot / n_blocks;
-    const int tile = ((t >> 2) * 8 + xcd) * 4 + (t & 3);
-    if (tile >= g.n_tiles ||
-        !enter_group(g.grp, tile, g.A, g.lda, g.W, g.C, DENSE == 1 ? g.N >> 1 : g.N,
-                     g.M))
-      return;
-    group_n_blk = slot % n_blocks;
+union FragW {
+  u32x4_r r;
+  bf16x8_r v;
+};
+
+// What a 32-bit offset of a buffer access reaches.
+constexpr int64_t kRowsReach = 1LL << 31;
+
+// The same products with operands fetched where they are used: for grouped layers whose
+// rows or weights spread over more than a buffer access reaches.
+template <int MT, int NT>
+__device__ __forceinline__ void rows_multiply_far(const RowsGemmArgs& g,
+                                                  f32x4_r (&acc)[MT][NT], int m0,
+                                                  int nt0, int n_tiles, int lane) {
+  const int l16 = lane & 15, gq = lane >> 4;
+  const int KT = g.K >> 5;
+  for (int kt = 0; kt < KT; ++kt) {
+    FragR wb[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+      wb[nt].u = reinterpret_cast<const uint4*>(
+          g.W + ((size_t)min(nt0 + nt, n_tiles - 1) * KT + kt) * 1024)[lane];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int row = group_row(g.grp, min(m0 + 16 * mt + l16, g.M - 1));
+      FragR xa;
+      xa.u = *reinterpret_cast<const uint4*>(g.A + (size_t)row * g.lda + 32 * kt +
+                                             8 * gq);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[nt].v, xa.v,
+                                                              acc[mt][nt], 0, 0, 0);
+    }
   }
+}
+
+template <bool SWAP, int MT, int NT, int OCC, int DENSE = 0, bool GROUPED = false>
+__global__ void __launch_bounds__(256, OCC)
+rows_gemm_direct_kernel(RowsGemmArgs g) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (buffer descriptors are no host type)
+  constexpr int BM = 16 * MT, BN = 64 * NT;
+  constexpr int AL = BM / 32;  // 1 KB pieces (8 rows) a wavefront loads per stage
+  // Before every barrier: all but the newest rows and weights have landed (the stage
+  // and the weight tile about to be multiplied), and my reads of LDS have returned.  A
+  // barrier orders instructions that have been issued, not LDS reads that have
+  // completed.
+  constexpr int kWaitStage = 0x070 | (AL + NT);
+  static_assert(AL + NT < 16, "vmcnt");
+  constexpr int kWaitAll = 0x070;
+  __shared__ uint4 s_a0[BM * 8];
+  __shared__ uint4 s_a1[BM * 8];
+  __shared__ uint4 s_a2[BM * 8];
+  static_assert(sizeof(s_a0) >= 4 * kRowsStageBytes<NT>, "stage too small");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, gq = lane >> 4;
-  const int m_blocks = (g.M + BM - 1) / BM;
-  const int m_blk = GROUPED ? 0 : blockIdx.x % m_blocks;
-  const int n_blk = GROUPED ? group_n_blk : blockIdx.x / m_blocks;
-  const int wm = wave / WN, wn = wave % WN;
-  const int m0 = m_blk * BM + wm * (16 * MT);
-  const int nt0 = n_blk * (BN / 16) + wn * NT;
-  const int KT = g.K >> 5, n_tiles = g.N >> 4;
-
-  const auto swap = [](int q) { return q & 2 ? 3 : 0; };
-  const int ld_row = lane >> 2;
-  const int ld_piece = (lane & 3) ^ swap(ld_row >> 2);
-  const int read_slot = 4 * l16 + (gq ^ swap(l16 >> 2));
-  // this wavefront's tiles of every stage: activation tiles wave + WAVES i,
-  // weight tiles wave + WAVES i (rows / tiles past the edge clamped: their
-  // products are discarded in the epilogue)
-  const char* arow[AL];
-  const char* wtile[WL];
-#pragma unroll
-  for (int i = 0; i < AL; ++i) {
-    int row = min(m_blk * BM + 16 * (wave + WAVES * i) + ld_row, g.M - 1);
-    if constexpr (GROUPED) row = group_row(g.grp, row);
-    arow[i] = reinterpret_cast<const char*>(g.A + (size_t)row * g.lda +
-                                            8 * ld_piece);
+  const int KT = g.K >> 5, KS = (KT + 1) >> 1, n_tiles = g.N >> 4;
+  const int n_blocks = (n_tiles + BN / 16 - 1) / (BN / 16);
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  int m_blk, n_blk;
+  if constexpr (GROUPED) {
+    T5D_GATED(g.gate);
+    // 4 consecutive tiles of rows, most of them of one group, on one XCD, all
+    // columns of half a tile in a row: rows and kernels come from that XCD's L2.
+    const int t = slot / n_blocks;
+    const int tile = ((t >> 3) * 8 + xcd) * 4 + ((t & 7) >> 1);
+    m_blk = t & 1;
+    n_blk = slot % n_blocks;
+    if (tile >= g.n_tiles ||
+        !enter_group(g.grp, tile, g.A, g.lda, g.W, g.C, DENSE == 1 ? g.N >> 1 : g.N,
+                     g.M) ||
+        m_blk * BM >= g.M)
+      return;
+  } else {
+    // An XCD takes a run of consecutive tiles, column by column over 8 blocks of rows
+    // at a time: what its CUs hold at once is few rows and few weights.
+    const int m_blocks = (g.M + BM - 1) / BM;
+    const int total = m_blocks * n_blocks;
+    const int t = xcd * (total >> 3) + min(xcd, total & 7) + slot;
+    constexpr int GM = 8;
+    const int group = t / (GM * n_blocks), in = t - group * (GM * n_blocks);
+    const int rows = min(GM, m_blocks - group * GM);
+    m_blk = group * GM + in % rows;
+    n_blk = in / rows;
   }
-#pragma unroll
-  for (int i = 0; i < WL; ++i)
-    wtile[i] = g.W + (size_t)min(n_blk * (BN / 16) +
-                                     (wave + WAVES * i) % WTILES,
-                                 n_tiles - 1) * KT * 1024 + lane * 16;
+  const int m0 = m_blk * BM;
+  const int nt0 = n_blk * (BN / 16) + wave * NT;
 
   f32x4_r acc[MT][NT];
 #pragma unroll
@@ -540,203 +556,237 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = (f32x4_r){0.f, 0.f, 0.f, 0.f};
 
-#define T5D_ROWS_ISSUE(kt_, S_)                                                \
+  bool listed = false;
+  if constexpr (GROUPED) {
+    listed = g.grp.rows != nullptr;
+    bool far = 2LL * BN * g.K >= kRowsReach || 2LL * (BM + 1) * g.lda >= kRowsReach;
+    if (listed) {
+      const int reach = (int)((kRowsReach - 1) / (2LL * g.lda)) - 1;
+#pragma unroll
+      for (int r = 0; r < BM; r += 64)
+        far |= g.grp.rows[min(m0 + r + lane, g.M - 1)] > reach;
+    }
+    if (__builtin_amdgcn_ballot_w64(far) != 0) {
+      rows_multiply_far(g, acc, m0, nt0, n_tiles, lane);
+      rows_epilogue_staged<DENSE, false>(
+          g, acc, m0, nt0, n_tiles, lane,
+          reinterpret_cast<char*>(&s_a0[0]) + wave * kRowsStageBytes<NT>);
+      return;
+    }
+  }
+  // this wavefront's pieces of every stage: 8-row groups wave + 4 i (rows past the edge
+  // clamped: their products are discarded in the epilogue)
+  const __amdgpu_buffer_rsrc_t a_rows = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(listed ? g.A : g.A + (size_t)m0 * g.lda), 0, 0x7fffffff, 0x00020000);
+  const int ld_row = wave * 8 + (lane >> 3);
+  const int ld_piece = (lane & 7) ^ ((ld_row >> 1) & 7);  // (32 rows on: the same)
+  int a_off[AL];
+#pragma unroll
+  for (int i = 0; i < AL; ++i) {
+    const int row = min(m0 + ld_row + 32 * i, g.M - 1);
+    a_off[i] = (listed ? group_row(g.grp, row) : row - m0) * (g.lda * 2) + 16 * ld_piece;
+  }
+  // K of 32 modulo 64: the last step has no second half, whose pieces are the first's
+  const int a_back = (KT & 1) && ld_piece >= 4 ? 64 : 0;
+  const __amdgpu_buffer_rsrc_t w_rows = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(g.W + (size_t)n_blk * (BN / 16) * KT * 1024), 0, 0x7fffffff, 0x00020000);
+  int w_off[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+    w_off[nt] = min(wave * NT + nt, n_tiles - 1 - n_blk * (BN / 16)) * KT * 1024;
+  FragW w0[NT], w1[NT], w2[NT];
+
+#define T5D_ROWS_ISSUE_A(s_, S_)                                               \
   do {                                                                         \
+    const int step = min((s_), KS - 1);                                        \
+    const int back = step == KS - 1 ? a_back : 0;                              \
     _Pragma("unroll") for (int i = 0; i < AL; ++i)                             \
-      __builtin_amdgcn_global_load_lds((glb_ptr_t)(arow[i] + 64 * (kt_)),      \
-                                       (lds_ptr_t)&S_[wave + WAVES * i][0],    \
-                                       16, 0, 0);                              \
-    _Pragma("unroll") for (int i = 0; i < WL; ++i)                             \
-      __builtin_amdgcn_global_load_lds(                                        \
-          (glb_ptr_t)(wtile[i] + (size_t)(kt_) * 1024),                        \
-          (lds_ptr_t)&S_[ATILES + (wave + WAVES * i) % WTILES][0], 16, 0, 0);  \
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(                                \
+          a_rows, (lds_ptr_t)&S_[(wave + 4 * i) * 64], 16, a_off[i] - back,    \
+          128 * step, 0, 0);                                                   \
   } while (0)
-#define T5D_ROWS_MULTIPLY(S_)                                                  \
-  do {                                                                         \
-    FragR wb[NT];                                                              \
+#define T5D_ROWS_ISSUE_W(kt_, W_)                                              \
+  _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                            \
+    W_[nt].r = __builtin_amdgcn_raw_buffer_load_b128(                          \
+        w_rows, 16 * lane, w_off[nt] + min((kt_), KT - 1) * 1024, 0)
+#define T5D_ROWS_READ(S_, half_, p_, X_)                                       \
+  _Pragma("unroll") for (int j = 0; j < 2; ++j)                                \
+    X_[j].u = S_[(2 * (p_) + j) * 128 + l16 * 8 +                              \
+                 ((4 * (half_) + gq) ^ ((l16 >> 1) & 7))]
+#define T5D_ROWS_PRODUCTS(p_, X_, W_)                                          \
+  _Pragma("unroll") for (int j = 0; j < 2; ++j)                                \
     _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                          \
-      wb[nt].u = S_[ATILES + wn * NT + nt][lane];                              \
-    _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) {                        \
-      FragR xa;                                                                \
-      xa.u = S_[wm * MT + mt][read_slot];                                      \
-      _Pragma("unroll") for (int nt = 0; nt < NT; ++nt) {                      \
-        if (SWAP)                                                              \
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(               \
-              wb[nt].v, xa.v, acc[mt][nt], 0, 0, 0);                           \
-        else                                                                   \
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(               \
-              xa.v, wb[nt].v, acc[mt][nt], 0, 0, 0);                           \
-      }                                                                        \
-    }                                                                          \
-  } while (0)
-  // kWaitStage: all but this wavefront's newest loads have landed, i.e. its
-  // share of the stage about to be multiplied, and its reads of the previous
-  // stage have returned; after the barrier every wavefront's share has
-  // landed, and every wavefront is done with the stage that the next loads
-  // overwrite.
-#define T5D_ROWS_STEP(kt_, CUR_, NEXT2_)                                       \
+      acc[2 * (p_) + j][nt] =                                                  \
+          SWAP ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(                      \
+                     W_[nt].v, X_[j].v, acc[2 * (p_) + j][nt], 0, 0, 0)        \
+               : __builtin_amdgcn_mfma_f32_16x16x32_bf16(                      \
+                     X_[j].v, W_[nt].v, acc[2 * (p_) + j][nt], 0, 0, 0)
+#define T5D_FENCE __builtin_amdgcn_sched_barrier(0)
+  // Half a step: operands in x at its start, those of what follows in x at its end.
+#define T5D_ROWS_HALF(S_, half_, W_)                                           \
+  _Pragma("unroll") for (int p = 0; p < MT / 2; p += 2) {                      \
+    T5D_ROWS_READ(S_, half_, p + 1, y);                                        \
+    T5D_FENCE;                                                                 \
+    T5D_ROWS_PRODUCTS(p, x, W_);                                               \
+    T5D_FENCE;                                                                 \
+    if (p + 2 < MT / 2) T5D_ROWS_READ(S_, half_, p + 2, x);                    \
+    else if ((half_) == 0) T5D_ROWS_READ(S_, 1, 0, x);                         \
+    T5D_FENCE;                                                                 \
+    T5D_ROWS_PRODUCTS(p + 1, y, W_);                                           \
+    T5D_FENCE;                                                                 \
+  }
+  // Step s_ on stage CUR_ with weights WA_, WB_; WC_, then WA_ take the next step's.
+#define T5D_ROWS_STEP(s_, CUR_, NEXT2_, WA_, WB_, WC_, second_half_)           \
   do {                                                                         \
+    FragR x[2], y[2];                                                          \
     __builtin_amdgcn_s_waitcnt(kWaitStage);                                    \
     __builtin_amdgcn_s_barrier();                                              \
-    T5D_ROWS_ISSUE((kt_) + 2, NEXT2_);                                         \
-    __builtin_amdgcn_sched_barrier(0);                                         \
-    T5D_ROWS_MULTIPLY(CUR_);                                                   \
+    T5D_ROWS_READ(CUR_, 0, 0, x);                                              \
+    T5D_FENCE;                                                                 \
+    T5D_ROWS_ISSUE_W(2 * (s_) + 2, WC_);                                       \
+    T5D_FENCE;                                                                 \
+    T5D_ROWS_HALF(CUR_, 0, WA_)                                                \
+    T5D_ROWS_ISSUE_W(2 * (s_) + 3, WA_);                                       \
+    T5D_ROWS_ISSUE_A((s_) + 2, NEXT2_);                                        \
+    T5D_FENCE;                                                                 \
+    if (second_half_) {                                                        \
+      T5D_ROWS_HALF(CUR_, 1, WB_)                                              \
+    }                                                                          \
   } while (0)
-#define T5D_ROWS_LAST(kt_, CUR_, NEXT2_)                                       \
-  do {                                                                         \
-    if ((kt_) + 1 < KT) __builtin_amdgcn_s_waitcnt(kWaitStage);                \
-    else __builtin_amdgcn_s_waitcnt(kWaitAll);                                 \
-    __builtin_amdgcn_s_barrier();                                              \
-    if ((kt_) + 2 < KT) T5D_ROWS_ISSUE((kt_) + 2, NEXT2_);                     \
-    __builtin_amdgcn_sched_barrier(0);                                         \
-    T5D_ROWS_MULTIPLY(CUR_);                                                   \
-  } while (0)
-  T5D_ROWS_ISSUE(0, s_t0);
-  T5D_ROWS_ISSUE(1, s_t1);  // KT >= 2 (checked by the caller)
-  const int n_main = (KT - 2) / 3 * 3;
-  int kt = 0;
-  for (; kt < n_main; kt += 3) {
-    T5D_ROWS_STEP(kt, s_t0, s_t2);
-    T5D_ROWS_STEP(kt + 1, s_t1, s_t0);
-    T5D_ROWS_STEP(kt + 2, s_t2, s_t1);
+  T5D_ROWS_ISSUE_A(0, s_a0);
+  T5D_ROWS_ISSUE_W(0, w0);
+  T5D_ROWS_ISSUE_W(1, w1);
+  T5D_ROWS_ISSUE_A(1, s_a1);
+  T5D_FENCE;
+  int s = 0;
+  for (; s + 3 <= KT >> 1; s += 3) {
+    T5D_ROWS_STEP(s, s_a0, s_a2, w0, w1, w2, true);
+    T5D_ROWS_STEP(s + 1, s_a1, s_a0, w2, w0, w1, true);
+    T5D_ROWS_STEP(s + 2, s_a2, s_a1, w1, w2, w0, true);
   }
-  // the last 2 to 4 k-tiles
-  T5D_ROWS_LAST(kt, s_t0, s_t2);
-  T5D_ROWS_LAST(kt + 1, s_t1, s_t0);
-  if (kt + 2 < KT) T5D_ROWS_LAST(kt + 2, s_t2, s_t1);
-  if (kt + 3 < KT) T5D_ROWS_LAST(kt + 3, s_t0, s_t2);
-#undef T5D_ROWS_ISSUE
-#undef T5D_ROWS_MULTIPLY
+  // the last 0 to 3 steps
+  if (s < KS) {
+    T5D_ROWS_STEP(s, s_a0, s_a2, w0, w1, w2, 2 * s + 1 < KT);
+    if (s + 1 < KS) {
+      T5D_ROWS_STEP(s + 1, s_a1, s_a0, w2, w0, w1, 2 * s + 3 < KT);
+      if (s + 2 < KS) T5D_ROWS_STEP(s + 2, s_a2, s_a1, w1, w2, w0, 2 * s + 5 < KT);
+    }
+  }
+#undef T5D_ROWS_ISSUE_A
+#undef T5D_ROWS_ISSUE_W
+#undef T5D_ROWS_READ
+#undef T5D_ROWS_PRODUCTS
+#undef T5D_FENCE
+#undef T5D_ROWS_HALF
 #undef T5D_ROWS_STEP
-#undef T5D_ROWS_LAST
   if (SWAP) {
-    static_assert(sizeof(s_t0) >= WAVES * kRowsStageBytes, "stage too small");
-    __syncthreads();  // every wavefront is done with the ring
+    // the requests past the end have landed, every wavefront is done with the ring
+    __builtin_amdgcn_s_waitcnt(kWaitAll);
+    __syncthreads();
     rows_epilogue_staged<DENSE, false>(
         g, acc, m0, nt0, n_tiles, lane,
-        reinterpret_cast<char*>(&s_t0[0][0]) + wave * kRowsStageBytes);
+        reinterpret_cast<char*>(&s_a0[0]) + wave * kRowsStageBytes<NT>);
   } else {
+    __builtin_amdgcn_s_waitcnt(kWaitAll);
     rows_epilogue_values(g, acc, m0, nt0, n_tiles, l16, gq);
   }
+#endif
 }
 
 }  // namespace t5d
 
 using namespace t5d;
 
-// Three widths of workgroup tile.  256 x 256 (8 wavefronts, one workgroup per CU)
-// halves the operand bytes per flop of 256 x 128 (4 wavefronts, two per CU)
-// and measures 3-11 % faster whenever its workgroups fill the 256 CUs
-// evenly; 256 x 192 (8 wavefronts of 128 x 48) is for the shapes where
-// neither does: N = 768 over 16384 rows is 192 tiles of 256 x 256 (a quarter
-// of the chip idle) but exactly 256 of 256 x 192.  Picked by the cost of the
-// rounds each tile needs, a last round that fills at most half of the CUs'
-// two slots counting 0.6 for the 256 x 128 tile.
+// The workgroup tile of rows_gemm_direct_kernel: 128 rows x 256, 192 or 128 columns, or
+// 64 x 128; 2, 2, 3 and 4 of them share a CU.  What a step of 64 of K lasts (us) with
+// 1, 2, ... of a kind on each CU, fitted to M = 1000 .. 32768, K = 768 .. 4096, N = 768
+// .. 8192: a lone workgroup waits for its operands, several overlap, and beyond that
+// time goes by their area.  The tile whose rounds over the 256 CUs add up to least is
+// taken.  Measured, us, 256 / 192 / 128 columns / 64 rows (* taken):
+//   10300 x 768 x 768 residual  18.3 / 21.6 / 17.9* / 18.2
+//   5000 x 2816 x 1024          38.5 / 33.6* / 37.3 / 38.8
+//   2000 x 2048 x 768           28.4 / 24.1 / 18.0 / 12.9*
+//   4096 x 1024 x 1024          15.8 / 13.8 / 10.6* / 10.9
+//   14000 x 1024 x 1024         28.0* / 33.0 / 30.2 / 34.1
+//   16384 x 768 x 4096 gated    92* / 96 / 95 / 117
+//   16384 x 768 x 1536          34 / 37* / 36 / 45
+struct RowsTile {
+  int code, rows, cols, per_cu;
+  double step[4];
+};
+static const RowsTile kRowsTiles[] = {
+    {2, 128, 256, 2, {0.77, 1.30}},
+    {3, 128, 192, 2, {0.56, 1.03}},
+    {1, 128, 128, 3, {0.42, 0.755, 1.15}},
+    {1, 64, 128, 4, {0.28, 0.45, 0.80, 1.00}},
+};
+
+static double rows_tile_cost(const RowsTile& t, int64_t M, int N) {
+  const int64_t wgs = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
+  const int64_t slots = 256 * t.per_cu, left = wgs % slots;
+  return (double)(wgs / slots) * t.step[t.per_cu - 1] +
+         (left ? t.step[(left + 255) / 256 - 1] : 0.0);
+}
+
+// Whether the kernel takes the shape (offsets inside a workgroup's rows and weights are
+// 32 bits wide), else rows_gemm_kernel does.
+static bool rows_direct(int w_dtype, int K, int64_t lda) {
+  return w_dtype == T5D_BF16 && K >= 64 && 2LL * 256 * K < kRowsReach &&
+         2LL * 128 * lda + 2LL * K < kRowsReach;
+}
+
+// code 0: any.
+static const RowsTile& rows_tile(int64_t M, int N, int code) {
+  const RowsTile* best = nullptr;
+  double least = 0.0;
+  for (const RowsTile& t : kRowsTiles) {
+    if (code && t.code != code) continue;
+    const double c = rows_tile_cost(t, M, N);
+    if (best == nullptr || c < least) {
+      best = &t;
+      least = c;
+    }
+  }
+  return *best;
+}
+
 extern "C" int t5d_gemm_rows_tile(int w_dtype, int64_t M, int K, int N) {
-  if (w_dtype != T5D_BF16 || K < 64 || M <= 0 || N <= 0) return 1;
-  const auto rounds = [](int64_t wgs, int slots) {
-    return (double)((wgs + slots - 1) / slots);
-  };
-  const int64_t m_blocks = (M + kRowsBM - 1) / kRowsBM;
-  const int64_t wgs128 = m_blocks * ((N + 127) / 128),
-                wgs192 = m_blocks * ((N + 191) / 192),
-                wgs256 = m_blocks * ((N + 255) / 256);
-  double c128 = rounds(wgs128, 512) * 2.0 * 128;
-  if ((wgs128 - 1) % 512 < 256) c128 -= 0.4 * 2.0 * 128;
-  const double c192 = rounds(wgs192, 256) * 192.0,
-               c256 = rounds(wgs256, 256) * 256.0;
-  int pick = 2;
-  double best = c256;
-  if (c192 < best) { best = c192; pick = 3; }
-  if (c128 < 0.97 * best) pick = 1;
-  return pick;
+  if (M <= 0 || N <= 0 || K <= 0 || !rows_direct(w_dtype, K, K)) return 1;
+  return rows_tile(M, N, 0).code;
 }
 
-// Rows of the 128-column tile of bfloat16 weights.  A workgroup of 256 rows lasts as
-// long on an empty chip as on a full one (its k-steps follow one another), so while
-// there are fewer workgroups than CUs they are made lower: 128 rows, or 64.  Results
-// have the same bits.  Measured, us with 256 / 128 / 64 rows:
-//   600 x 2048 x 768 residual  34.6 / 20.8 / 16.7   (60 workgroups of 64 rows)
-//   2000 x 2048 x 768          35.3 / 22.5 / 17.6
-//   1000 x 5120 x 2048         70.9 / 45.5 / 39.6
-//   600 x 768 x 4096 gated     16.9 / 11.3 / 13.4
-//   4000 x 768 x 768           17.7 / 13.1 / 14.2
-// and no gain from where 128 rows give more than one workgroup per CU (8192 x 1024 x
-// 1024, 512 of them: 22.7 / 22.6 / 26.0; 1000 x 2048 x 5120, 320: 33.3 / 37.1 / 36.5).
-static int rows_of_tile(int M, int N) {
-  const int n_blocks = (N + kRowsBN - 1) / kRowsBN;
-  if ((int64_t)((M + 63) / 64) * n_blocks <= 256) return 64;
-  if ((int64_t)((M + 127) / 128) * n_blocks <= 256) return 128;
-  return 256;
-}
-
-// rows_gemm_direct_kernel with 128 columns and the rows that suit the shape.
 template <bool SWAP, int DENSE>
-static void launch_rows_128(hipStream_t s, const RowsGemmArgs& g) {
-  const int rows = rows_of_tile(g.M, g.N);
-  const dim3 grid((unsigned)((g.M + rows - 1) / rows) *
-                  ((g.N + kRowsBN - 1) / kRowsBN));
-  if (rows == 64)
-    hipLaunchKernelGGL((rows_gemm_direct_kernel<SWAP, kRowsNT, 2, DENSE, false, 2>),
-                       grid, dim3(256), 0, s, g);
-  else if (rows == 128)
-    hipLaunchKernelGGL((rows_gemm_direct_kernel<SWAP, kRowsNT, 2, DENSE, false, 4>),
-                       grid, dim3(256), 0, s, g);
-  else
-    hipLaunchKernelGGL((rows_gemm_direct_kernel<SWAP, kRowsNT, 2, DENSE>), grid,
-                       dim3(256), 0, s, g);
+static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int code) {
+  const RowsTile& t = rows_tile(g.M, g.N, code);
+  const dim3 grid((unsigned)((g.M + t.rows - 1) / t.rows) *
+                  ((g.N + t.cols - 1) / t.cols));
+#define T5D_ROWS_LAUNCH(MT_, NT_, OCC_)                                          \
+  hipLaunchKernelGGL((rows_gemm_direct_kernel<SWAP, MT_, NT_, OCC_, DENSE>), grid, \
+                     dim3(256), 0, s, g)
+  if (t.rows == 64) T5D_ROWS_LAUNCH(4, 2, 4);
+  else if (t.cols == 128) T5D_ROWS_LAUNCH(8, 2, 3);
+  else if (t.cols == 192) T5D_ROWS_LAUNCH(8, 3, 2);
+  else T5D_ROWS_LAUNCH(8, 4, 2);
+#undef T5D_ROWS_LAUNCH
 }
 
-// Picks the workgroup tile (tile 0) and launches checked arguments.
+// Picks the kernel and its workgroup tile (tile 0) and launches checked arguments.
 static int launch_rows(hipStream_t s, int w_dtype, const RowsGemmArgs& g,
                        int tile) {
   const int m_blocks = (g.M + kRowsBM - 1) / kRowsBM;
   const int n_blocks = (g.N + kRowsBN - 1) / kRowsBN;
-  dim3 grid((unsigned)m_blocks * n_blocks), block(256);
+  const dim3 grid((unsigned)m_blocks * n_blocks), block(256);
   const bool swap = g.layout != T5D_OUT_HEADS_VALUE;
-  const int pick = tile ? tile : t5d_gemm_rows_tile(w_dtype, g.M, g.K, g.N);
-  const int wgs192 = m_blocks * ((g.N + 191) / 192),
-            wgs256 = m_blocks * ((g.N + 255) / 256);
-  // bfloat16 weights, rows layout
-#define T5D_ROWS_DENSE(D_)                                                    \
-  do {                                                                        \
-    if (g.K >= 64 && pick == 3)                                               \
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 3, 4, D_>),           \
-                         dim3((unsigned)wgs192), dim3(512), 0, s, g);         \
-    else if (g.K >= 64 && pick == 2)                                          \
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 4, D_>),     \
-                         dim3((unsigned)wgs256), dim3(512), 0, s, g);         \
-    else if (g.K >= 64)                                                       \
-      launch_rows_128<true, D_>(s, g);                                        \
-    else                                                                      \
-      hipLaunchKernelGGL((rows_gemm_kernel<bf16_t, true, D_>), grid, block, 0, \
-                         s, g);                                               \
-  } while (0)
-  if (g.epilogue == T5D_EPI_CLAMPED_GLU) {
-    T5D_ROWS_DENSE(1);
-  } else if (g.C32 != nullptr) {
-    T5D_ROWS_DENSE(2);
-  } else if (w_dtype == T5D_BF16 && g.K >= 64 && pick == 3) {
-    dim3 wgrid((unsigned)wgs192), wblock(512);
-    if (swap)
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 3, 4>), wgrid, wblock,
-                         0, s, g);
-    else
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<false, 3, 4>), wgrid, wblock,
-                         0, s, g);
-  } else if (w_dtype == T5D_BF16 && g.K >= 64 && pick == 2) {
-    dim3 wgrid((unsigned)wgs256), wblock(512);
-    if (swap)
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 4>), wgrid,
-                         wblock, 0, s, g);
-    else
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<false, kRowsNT, 4>), wgrid,
-                         wblock, 0, s, g);
-  } else if (w_dtype == T5D_BF16 && g.K >= 64) {
-    if (swap)
-      launch_rows_128<true, 0>(s, g);
-    else
-      launch_rows_128<false, 0>(s, g);
+  const int dense = g.epilogue == T5D_EPI_CLAMPED_GLU ? 1 : g.C32 != nullptr ? 2 : 0;
+  if (rows_direct(w_dtype, g.K, g.lda)) {
+    if (dense == 1) launch_rows_direct<true, 1>(s, g, tile);
+    else if (dense == 2) launch_rows_direct<true, 2>(s, g, tile);
+    else if (swap) launch_rows_direct<true, 0>(s, g, tile);
+    else launch_rows_direct<false, 0>(s, g, tile);
+  } else if (dense == 1) {
+    hipLaunchKernelGGL((rows_gemm_kernel<bf16_t, true, 1>), grid, block, 0, s, g);
+  } else if (dense == 2) {
+    hipLaunchKernelGGL((rows_gemm_kernel<bf16_t, true, 2>), grid, block, 0, s, g);
   } else if (w_dtype == T5D_BF16) {
     if (swap)
       hipLaunchKernelGGL((rows_gemm_kernel<bf16_t, true>), grid, block, 0, s, g);
@@ -748,7 +798,6 @@ static int launch_rows(hipStream_t s, int w_dtype, const RowsGemmArgs& g,
     else
       hipLaunchKernelGGL((rows_gemm_kernel<int8_t, false>), grid, block, 0, s, g);
   }
-#undef T5D_ROWS_DENSE
   T5D_CHECK_LAUNCH("t5d_gemm_rows");
   return T5D_OK;
 }
@@ -768,8 +817,8 @@ static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
                      const int32_t* at, int tile) {
   T5D_REQUIRE(A && W && C, T5D_EINVAL, "t5d_gemm_rows: null pointer");
   T5D_REQUIRE(tile >= 0 && tile <= 3, T5D_EINVAL,
-              "t5d_gemm_rows_tiled: tile %d (0 chosen here, 1: 256 x 128, "
-              "2: 256 x 256, 3: 256 x 192)", tile);
+              "t5d_gemm_rows_tiled: tile %d (0 chosen here, columns: 1: 128, "
+              "2: 256, 3: 192)", tile);
   T5D_REQUIRE(w_dtype == T5D_BF16 || w_dtype == T5D_I8, T5D_EINVAL,
               "t5d_gemm_rows: w_dtype %d (packed bfloat16 or int8)", w_dtype);
   T5D_REQUIRE(w_dtype != T5D_I8 || scales, T5D_EINVAL,
@@ -858,27 +907,25 @@ int t5d::launch_grouped_rows(hipStream_t s, const GroupedArgs& a, int n_tiles) {
   g.lda = a.lda; g.ldc = a.ldc; g.n_store = a.n_store;
   g.glu_limit = a.glu_limit; g.glu_alpha = a.glu_alpha; g.glu_add = a.glu_add;
   g.gate = a.gate; g.grp = a.grp; g.n_tiles = n_tiles;
-  const unsigned t32 = (unsigned)(n_tiles + 31) / 32 * 32;
+  // (32 tiles, two workgroups of rows each, make a round over the XCDs)
+  const unsigned t64 = (unsigned)(n_tiles + 31) / 32 * 64;
   const unsigned n128 = (g.N + 127) / 128, n256 = (g.N + 255) / 256;
   const bool glu = g.epilogue == T5D_EPI_CLAMPED_GLU;
-  // the 256 x 256 tile unless much of its last column block would be empty
-  if (n256 * 256 <= n128 * 128 + 64) {
-    const dim3 grid(t32 * n256), block(512);
-    if (glu)
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 4, 1, true>), grid,
-                         block, 0, s, g);
-    else
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 4, 0, true>), grid,
-                         block, 0, s, g);
-  } else {
-    const dim3 grid(t32 * n128), block(256);
-    if (glu)
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 2, 1, true>), grid,
-                         block, 0, s, g);
-    else
-      hipLaunchKernelGGL((rows_gemm_direct_kernel<true, kRowsNT, 2, 0, true>), grid,
-                         block, 0, s, g);
-  }
+  // 256 columns unless much of the last column block would be empty
+  const bool wide = n256 * 256 <= n128 * 128 + 64;
+  const dim3 grid(t64 * (wide ? n256 : n128)), block(256);
+  if (wide && glu)
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 8, 4, 2, 1, true>), grid, block, 0,
+                       s, g);
+  else if (wide)
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 8, 4, 2, 0, true>), grid, block, 0,
+                       s, g);
+  else if (glu)
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 8, 2, 3, 1, true>), grid, block, 0,
+                       s, g);
+  else
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 8, 2, 3, 0, true>), grid, block, 0,
+                       s, g);
   T5D_CHECK_LAUNCH("t5d_grouped_dense_run(rows)");
   return T5D_OK;
 }

@@ -196,6 +196,22 @@ def test_gemm_rows_of_low_tiles(ops, M, K, N):
   assert bool(((unit.float() - parts).abs() <= 2.0**-7 * parts.abs() + 1e-5).all())
 
 
+@pytest.mark.parametrize('K', [64, 96, 128, 160, 192, 224, 256, 320, 384, 448])
+@pytest.mark.parametrize('tile', [1, 2, 3])
+def test_gemm_rows_of_every_tile_over_the_ends_of_k(ops, K, tile):
+  """1 to 7 steps of 64 of K, whole and half ones (the ring of three and what is left
+  behind its rounds), at edges of rows and columns: bfloat16 of the float32 product."""
+  rs = np.random.RandomState(K)
+  for M, N in ((130, 272), (255, 144), (4200, 400)):
+    a = dev(rs.randn(M, K).astype(np.float32), torch.bfloat16)
+    w = dev((rs.randn(K, N) / np.sqrt(K)).astype(np.float32), torch.bfloat16)
+    got = ops.gemm_rows(a, ops.pack_weight(w.float(), torch.bfloat16), tile=tile)
+    want = a.float() @ w.float()
+    # (half a step of bfloat16, and float32 sums in another order)
+    bound = want.abs() * (2.0**-8 + 1e-5) + 1e-5
+    assert bool(((got.float() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize('B,E,H', [(1, 132, 1), (5, 60, 4), (3, 344, 13)])
 def test_gemm_rows_head_layouts_of_low_tiles(ops, B, E, H):
   from t5x_amd import _lib

@@ -93,6 +93,30 @@ def test_groups_of_columns(dt, M):
     assert rel(got[:, h * keep:(h + 1) * keep], want) < tol(dt)
 
 
+def test_grouped_rows_beyond_a_32_bit_offset():
+  """Tiles of 256 rows whose rows of A lie more than 2^31 bytes apart: the bits of the
+  same rows side by side."""
+  from t5x_amd import ops
+  rs = np.random.RandomState(5)
+  K, N, lda, last = 96, 160, 8192, 150000
+  bf16 = torch.bfloat16
+  near = dev(rs.randn(300, K), bf16)
+  at = np.sort(rs.choice(np.r_[0:500, last - 500:last], 300, replace=False))
+  a = torch.empty((last, lda), dtype=bf16, device='cuda')
+  rows = torch.as_tensor(at.astype(np.int32), device='cuda')
+  a[rows.long(), :K] = near
+  kernels = [ops.pack_weight(dev(rs.randn(K, N) / 10), bf16) for _ in range(2)]
+  tiles = torch.tensor([[1, 0, 256, 0], [0, 256, 44, 0], [-1, 0, 0, 0]],
+                       dtype=torch.int32, device='cuda')
+  outs = []
+  for x, r in ((a[:, :K], rows), (near, None)):
+    out = torch.zeros((300, N), dtype=bf16, device='cuda')
+    ops.grouped_dense(x, kernels, out, tiles, r, 256)
+    outs.append(out)
+  assert torch.equal(outs[0], outs[1])
+
+
+
 @pytest.mark.parametrize('dt', DTYPES)
 def test_silu_unit(dt):
   from t5x_amd import ops
