@@ -1,24 +1,6 @@
-// Single-query ("decode step") attention over K/V stored [.., heads, 64, len]
-// with `len` contiguous — the reference's cache layout
-// (t5x/examples/t5/layers.py:226-241).
-//
-// The step is bound by streaming K and V once.  One workgroup handles one
-// (row-or-batch-item, head); wavefront w owns key positions
-// [w*BJ, (w+1)*BJ) (BJ = 128 bf16 / 64 f32 positions).  Inside a wavefront,
-// lane = (dg, jc): jc = lane % 16 selects a 16-byte chunk of consecutive key
-// positions, dg = lane / 16 selects head-dim rows d = dg + 4*i, i = 0..15.
-// Every load instruction therefore fetches 4 rows x 256 contiguous bytes and
-// only chunks that start inside the valid prefix are requested at all.
-//   scores : per-lane FMAs over its 16 rows, then 2 xor-shuffles across dg;
-//   softmax: 4 xor-shuffles across jc (+ an LDS exchange when several
-//            wavefronts share the key axis); probabilities are normalised and
-//            rounded to the activation dtype BEFORE the value product, as the
-//            reference does;
-//   P·V    : per-lane partial dot products, then a 15-step shuffle
-//            reduce-scatter across jc leaves lane (dg, jc) holding output
-//            element d = dg + 4*jc.
-// NQ queries share the K/V stream (the beams of one batch item in
-// cross-attention; 1 for self-attention, where each beam has its own cache).
+// Single-query ("decode step") attention in float32 — the dtype of exactness tests and
+// of users without bfloat16 checkpoints — and what the bfloat16 kernels
+// (attention_mfma.hip) share with it.
 #include <math.h>
 
 #include "common.h"
@@ -34,299 +16,220 @@ struct AttnArgs {
   void* out;            // [R, HD]
   int H, S, nq, q_stride;
   const int32_t* gate;  // optional device-side enable flag
+  // float32: the first wavefront asks for its keys and values before it knows how many
+  // positions are valid.  Set while workgroups are few (one per CU): the wait for the
+  // length then costs more than requests for positions that turn out to be masked.  With
+  // many the traffic does (64 items of 12 heads, 64 positions, 10 valid: 4.3 us, all
+  // asked for 6.6).
+  bool early;
 };
 
 constexpr int kD = 64;
 constexpr int kMaxWaves = 16;
 
+// ---- float32 self-attention ----------------------------------------------------
+// K and V [R, heads, 64, len] with `len` contiguous — the reference's cache layout
+// (t5x/examples/t5/layers.py:226-241).  A workgroup takes one (row, head), wavefront w
+// key positions 64 w .. 64 w + 63; inside a wavefront lane = (dg, jc): jc = lane % 16
+// selects 4 consecutive positions, dg = lane / 16 head-dim rows d = dg + 4 i, so every
+// load fetches 4 rows x 256 contiguous bytes.  Scores are sums over a lane's 16 rows,
+// then over dg; maximum and sum of the softmax go over jc (and over wavefronts through
+// LDS); weights are normalised before the value product, whose sums over jc end
+// scattered: lane (dg, jc) holds d = dg + 4 jc.
+//
+// What bounds it at the few rows it is used for is a chain of waits and the fetch of
+// its own code, whose every KB costs 0.2 us while it is cold.  So everything is asked
+// for at the start: new key and value and bias with the queries, the first
+// wavefront's keys and values before it knows how many positions are valid (see
+// AttnArgs::early); and the new column has a score and a weight of its own: merged into
+// the others by 32 branches of the lane that has it, with a comparison per element, the
+// kernel had 3456 instructions.  us, before / now: 8 rows of 6 heads over 32 positions
+// 8.4 / 3.5, 16 x 12 over 128 9.8 / 5.3, 16 x 6 over 256 10.4 / 5.8, 64 x 12 over 64
+// 11.3 / 6.3, 8 x 6 over 1000 20.3 / 12.4.  Error against float64 as before (1.8e-7 over
+// 32 positions, 3.4e-7 over 1000).
+//
 // WM = the most wavefronts a launch of this instance uses; it bounds the
 // workgroup size so short key axes get the full register file.
-template <typename T, int NQ, bool SELF, int WM>
-__global__ void __launch_bounds__(64 * WM)
-attn_step_kernel(AttnArgs a) {
-  constexpr int EL = Act<T>::kElemsPer16B;  // key positions per 16-byte chunk
-  constexpr int BJ = 16 * EL;               // key positions per wavefront
-  __shared__ float s_red[WM][NQ];
-  __shared__ float s_out[WM][NQ][kD];
-  T5D_GATED(a.gate);
+constexpr int kDppRotate8 = 0x128;  // lane i <-> (i + 8) % 16
+// One step of the scatter: ST of the 2 ST sums stay, the partner (CTRL: a lane that
+// differs in bit ST) adds its own.
+template <int ST, int CTRL>
+__device__ __forceinline__ void scatter_step(float (&o)[16], int jc) {
+  const bool up = (jc & ST) != 0;
+#pragma unroll
+  for (int k = 0; k < ST; ++k) {
+    const float mine = up ? o[k + ST] : o[k];
+    const float other = up ? o[k] : o[k + ST];
+    o[k] = mine + dpp_move<CTRL>(other);
+  }
+}
 
+template <int WM>
+__global__ void __launch_bounds__(64 * WM)
+self_attn_f32_kernel(AttnArgs a) {
+  __shared__ float s_red[2][WM];
+  __shared__ float s_out[WM][kD];
+  T5D_GATE_READ(a.gate);
   const int h = blockIdx.x, g = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nwaves = blockDim.x >> 6;
   const int jc = lane & 15, dg = lane >> 4;
   const int HD = a.H * kD;
+  const int j0 = wave * 64 + jc * 4;
+  // the cache of this row and head, and this lane's corner of it: row dg, position j0;
+  // its rows are 4 S floats apart
+  const size_t first = ((size_t)g * a.H + h) * kD * a.S;
+  const unsigned corner = dg * a.S + j0;
+  const int step = 4 * a.S;
+  float* kp = reinterpret_cast<float*>(a.k) + first;
+  float* vp = reinterpret_cast<float*>(a.v) + first;
+  const float* q = reinterpret_cast<const float*>(a.q) + (size_t)g * a.q_stride +
+                   h * kD + dg;
+  // (with 16 wavefronts there are no registers for values beside keys)
+  constexpr bool kAhead = WM < 16;
+  const bool early = kAhead && a.early && wave == 0;
 
-  int n, t = 0;
-  bool uniform = false;  // no valid key: the masked softmax is uniform
+  float qv[16], knew[16], vnew[16];
+  const auto request_new = [&](float (&to)[16], int at) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) to[i] = q[at + 4 * i];
+  };
+  request_new(qv, 0);
+  request_new(knew, HD);
+  if (kAhead) request_new(vnew, 2 * HD);
+  float4 kc[16], vc[16];
+  const auto request = [&](float4 (&to)[16], const float* from) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      to[i] = *reinterpret_cast<const float4*>(from + i * step + corner);
+  };
+  if (early && j0 < a.S) {
+    request(kc, kp);
+    request(vc, vp);
+  }
+
   // A cache index outside [0, S) (a decode loop longer than its cache) must
   // not become an address: nothing is inserted then and all S columns are
   // attended with the bias row of the last position, which is what the
   // reference's one-hot insert and clamped slices do (layers.py:258-303).
-  bool past_end = false;
-  if (SELF) {
-    t = *a.index;
-    past_end = t < 0 || t >= a.S;
-    if (past_end) t = a.S - 1;
-    n = t + 1;
-  } else {
-    n = a.index[g];
-    n = n < 0 ? 0 : (n > a.S ? a.S : n);
-    if (n == 0) { uniform = true; n = a.S; }
-  }
-
-  const int j0 = wave * BJ + jc * EL;
+  int t = *a.index;
+  T5D_GATE_TEST();
+  const bool past_end = t < 0 || t >= a.S;
+  if (past_end) t = a.S - 1;
+  const int n = t + 1;
   const bool live = j0 < n;
-  const T* kbase = reinterpret_cast<const T*>(a.k) +
-                   ((size_t)g * a.H + h) * kD * a.S;
-  const T* vbase = reinterpret_cast<const T*>(a.v) +
-                   ((size_t)g * a.H + h) * kD * a.S;
-  const T* qbase = reinterpret_cast<const T*>(a.q);
+  float bias[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    bias[e] = reinterpret_cast<const float*>(a.rel_bias)[(size_t)h * a.S +
+                                                         max(t - j0 - e, 0)];
+  if (!early && live) {
+    request(kc, kp);
+    if (kAhead) request(vc, vp);
+  }
+  // The lane whose positions contain column t takes the new key and value there, whose
+  // score is formed beside the others, and writes them to the cache.
+  const bool ins = !past_end && t >= j0 && t < j0 + 4;
+  float s_new = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) s_new = fmaf(qv[i], knew[i], s_new);
+  if (ins) {
+    const unsigned col = dg * a.S + t;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) *(kp + i * step + col) = knew[i];
+  }
+  if (!kAhead) __builtin_amdgcn_sched_barrier(0);  // (the new key's registers)
 
-  // Queries: lane needs q[d] for its 16 rows.
-  float qv[NQ][16];
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int qi = 0; qi < NQ; ++qi) {
-    const int row = SELF ? g : g * a.nq + qi;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      qv[qi][i] = (qi < a.nq)
-                      ? Act<T>::load(qbase + (size_t)row * a.q_stride + h * kD +
-                                     dg + 4 * i)
-                      : 0.f;
-    }
+  for (int i = 0; i < 16; ++i) {
+    s[0] = fmaf(qv[i], kc[i].x, s[0]);
+    s[1] = fmaf(qv[i], kc[i].y, s[1]);
+    s[2] = fmaf(qv[i], kc[i].z, s[2]);
+    s[3] = fmaf(qv[i], kc[i].w, s[3]);
+  }
+  if (!kAhead) {
+    __builtin_amdgcn_sched_barrier(0);  // (the keys' registers)
+    if (live) request(vc, vp);
+    request_new(vnew, 2 * HD);
   }
 
-  // The new key and value and the bias, with the queries: read by the one lane
-  // that inserts them, row by row, they were 32 waits in a row (8 rows of 6 heads
-  // in float32: 11.4 us, now 8.7 with the values requested with the keys).
-  // (With 16 wavefronts there are no registers for them.)
-  constexpr bool kAhead = SELF && WM < 16;
-  const T* fresh = qbase + (size_t)g * a.q_stride + HD + h * kD + dg;
-  T knew[kAhead ? 16 : 1], vnew[kAhead ? 16 : 1];
-  float bias[kAhead ? EL : 1];
-  if constexpr (kAhead) {
+  float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      knew[i] = fresh[4 * i];
-      vnew[i] = fresh[HD + 4 * i];
-    }
+  for (int e = 0; e < 4; ++e) {
+    if (ins && j0 + e == t) s[e] = s_new;
+    s[e] = j0 + e < n ? rows_sum(s[e]) + bias[e] : -INFINITY;
+    mx = fmaxf(mx, s[e]);
   }
-  const auto bias_of = [&](int e) {
-    return Act<T>::load(reinterpret_cast<const T*>(a.rel_bias) + (size_t)h * a.S +
-                        max(t - j0 - e, 0));
+  mx = lanes16_max(mx);
+  if (nwaves > 1) {
+    if (lane == 0) s_red[0][wave] = mx;
+    __syncthreads();
+    mx = s_red[0][0];
+    for (int w = 1; w < nwaves; ++w) mx = fmaxf(mx, s_red[0][w]);
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s[e] = s[e] == -INFINITY ? 0.f : expf(s[e] - mx);
+    sum += s[e];
+  }
+  sum = lanes16_sum(sum);
+  if (nwaves > 1) {
+    if (lane == 0) s_red[1][wave] = sum;
+    __syncthreads();
+    sum = s_red[1][0];
+    for (int w = 1; w < nwaves; ++w) sum += s_red[1][w];
+  }
+  // A zero weight must not pick up whatever lies past the prefix, nor the new column
+  // what its place held.
+  uint32_t there[4];
+  float p_new = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s[e] /= sum;
+    const bool fresh = ins && j0 + e == t;
+    if (fresh) p_new = s[e];
+    there[e] = s[e] != 0.f && !fresh ? 0xffffffffu : 0u;
+    s[e] = fresh ? 0.f : s[e];
+  }
+  const uint32_t there_new = p_new != 0.f ? 0xffffffffu : 0u;
+  const auto masked = [](uint32_t mask, float v) {
+    return __uint_as_float(mask & __float_as_uint(v));
   };
-  if constexpr (kAhead) {
-#pragma unroll
-    for (int e = 0; e < EL; ++e) bias[e] = bias_of(e);
-  }
 
-  // Self-attention: the lane whose chunk contains column t carries the new
-  // key/value, patches its registers and writes the column to the cache.
-  const bool ins = SELF && !past_end && live && (t >= j0) && (t < j0 + EL);
-  const int e_t = t - j0;
-
-  float s[NQ][EL];
-#pragma unroll
-  for (int qi = 0; qi < NQ; ++qi)
-#pragma unroll
-    for (int e = 0; e < EL; ++e) s[qi][e] = 0.f;
-
-  // the values do not depend on the softmax: requested with the keys
-  uint4 ahead[kAhead ? 16 : 1];
-  if constexpr (kAhead) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) ahead[i] = make_uint4(0, 0, 0, 0);
-  }
-  if (live) {
-    uint4 kc[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      kc[i] = *reinterpret_cast<const uint4*>(kbase + (size_t)(dg + 4 * i) * a.S + j0);
-    if constexpr (kAhead) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        ahead[i] =
-            *reinterpret_cast<const uint4*>(vbase + (size_t)(dg + 4 * i) * a.S + j0);
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float kf[EL];
-      unpack16(kc[i], kf);
-      if (SELF && ins) {
-        const int d = dg + 4 * i;
-        const T now = kAhead ? knew[kAhead ? i : 0] : fresh[4 * i];
-        const float kn = Act<T>::load(&now);
-#pragma unroll
-        for (int e = 0; e < EL; ++e) kf[e] = (e == e_t) ? kn : kf[e];
-        reinterpret_cast<T*>(a.k)[((size_t)g * a.H + h) * kD * a.S +
-                                  (size_t)d * a.S + t] = now;
-      }
-#pragma unroll
-      for (int qi = 0; qi < NQ; ++qi)
-#pragma unroll
-        for (int e = 0; e < EL; ++e) s[qi][e] = fmaf(qv[qi][i], kf[e], s[qi][e]);
-    }
-  }
-
-  // With 16 wavefronts they are requested here: into an array of their own and each
-  // under the condition, or its 128 registers do not suffice (14 spilled: 8 rows of 6
-  // heads over 1000 positions 23.4 us, 64 of 12 143.4; now 20.0 and 120.6).
-  uint4 vc[16];
+  float o[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    if constexpr (kAhead)
-      vc[i] = ahead[i];
-    else
-      vc[i] = live ? *reinterpret_cast<const uint4*>(vbase + (size_t)(dg + 4 * i) * a.S +
-                                                     j0)
-                   : make_uint4(0, 0, 0, 0);
+    o[i] = s[0] * masked(there[0], vc[i].x);
+    o[i] = fmaf(s[1], masked(there[1], vc[i].y), o[i]);
+    o[i] = fmaf(s[2], masked(there[2], vc[i].z), o[i]);
+    o[i] = fmaf(s[3], masked(there[3], vc[i].w), o[i]);
+    o[i] = fmaf(p_new, masked(there_new, vnew[i]), o[i]);
   }
-
-  // Sum the partial dot products of the 4 row groups.
+  if (ins) {
+    const unsigned col = dg * a.S + t;
 #pragma unroll
-  for (int qi = 0; qi < NQ; ++qi)
-#pragma unroll
-    for (int e = 0; e < EL; ++e) {
-      float x = s[qi][e];
-      x += __shfl_xor(x, 16, 64);
-      x += __shfl_xor(x, 32, 64);
-      s[qi][e] = x;
-    }
-
-  // Bias, mask, running max.
-  float mx[NQ];
-#pragma unroll
-  for (int qi = 0; qi < NQ; ++qi) {
-    float m = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < EL; ++e) {
-      const int j = j0 + e;
-      float x = Act<T>::round(s[qi][e]);
-      if (SELF) {
-        if (j < n) x = Act<T>::round(x + (kAhead ? bias[kAhead ? e : 0] : bias_of(e)));
-      }
-      if (uniform) x = 0.f;
-      x = (j < n) ? x : -INFINITY;
-      s[qi][e] = x;
-      m = fmaxf(m, x);
-    }
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    mx[qi] = m;
+    for (int i = 0; i < 16; ++i) *(vp + i * step + col) = vnew[i];
   }
-  if (nwaves > 1) {
-    if (lane == 0) {
-#pragma unroll
-      for (int qi = 0; qi < NQ; ++qi) s_red[wave][qi] = mx[qi];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int qi = 0; qi < NQ; ++qi) {
-      float m = s_red[0][qi];
-      for (int w = 1; w < nwaves; ++w) m = fmaxf(m, s_red[w][qi]);
-      mx[qi] = m;
-    }
-    __syncthreads();
-  }
-
-  // exp, sum, normalise, round to the activation dtype.
-  float p[NQ][EL];
-#pragma unroll
-  for (int qi = 0; qi < NQ; ++qi) {
-    float sum = 0.f;
-#pragma unroll
-    for (int e = 0; e < EL; ++e) {
-      const float x = s[qi][e];
-      const float ex = (x == -INFINITY) ? 0.f : expf(x - mx[qi]);
-      p[qi][e] = ex;
-      sum += ex;
-    }
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    if (nwaves > 1) {
-      if (lane == 0) s_red[wave][qi] = sum;
-    } else {
-#pragma unroll
-      for (int e = 0; e < EL; ++e) p[qi][e] = Act<T>::round(p[qi][e] / sum);
-    }
-  }
-  if (nwaves > 1) {
-    __syncthreads();
-#pragma unroll
-    for (int qi = 0; qi < NQ; ++qi) {
-      float sum = s_red[0][qi];
-      for (int w = 1; w < nwaves; ++w) sum += s_red[w][qi];
-#pragma unroll
-      for (int e = 0; e < EL; ++e) p[qi][e] = Act<T>::round(p[qi][e] / sum);
-    }
-  }
-
-  // P·V partial sums for this lane's 16 rows.
-  float o[NQ][16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    float vf[EL];
-    unpack16(vc[i], vf);
-    if (SELF && ins) {
-      const int d = dg + 4 * i;
-      const T now = kAhead ? vnew[kAhead ? i : 0] : fresh[HD + 4 * i];
-      const float vn = Act<T>::load(&now);
-#pragma unroll
-      for (int e = 0; e < EL; ++e) vf[e] = (e == e_t) ? vn : vf[e];
-      reinterpret_cast<T*>(a.v)[((size_t)g * a.H + h) * kD * a.S +
-                                (size_t)d * a.S + t] = now;
-    }
-#pragma unroll
-    for (int qi = 0; qi < NQ; ++qi) {
-      float acc = 0.f;
-#pragma unroll
-      for (int e = 0; e < EL; ++e) {
-        // A zero probability must not pick up whatever lies past the prefix.
-        const float pe = p[qi][e];
-        acc = fmaf(pe, pe != 0.f ? vf[e] : 0.f, acc);
-      }
-      o[qi][i] = acc;
-    }
-  }
-
-  // Reduce-scatter across the 16 chunk lanes: afterwards o[qi][0] in lane
-  // (dg, jc) is the sum over jc' of row index i = jc, i.e. d = dg + 4*jc.
-#pragma unroll
-  for (int qi = 0; qi < NQ; ++qi) {
-#pragma unroll
-    for (int st = 8; st >= 1; st >>= 1) {
-      const bool up = (jc & st) != 0;
-#pragma unroll
-      for (int k2 = 0; k2 < st; ++k2) {
-        const float mine = up ? o[qi][k2 + st] : o[qi][k2];
-        const float other = up ? o[qi][k2] : o[qi][k2 + st];
-        o[qi][k2] = mine + __shfl_xor(other, st, 64);
-      }
-    }
-  }
-  const int d_out = dg + 4 * jc;
-  T* outp = reinterpret_cast<T*>(a.out);
+  // Partners of the scatter: 8 lanes on, mirrored in 8, 2 on, 1 on (each differs in
+  // the step's bit; together they are all 16).
+  scatter_step<8, kDppRotate8>(o, jc);
+  scatter_step<4, kDppHalfMirror>(o, jc);
+  scatter_step<2, kDppXor2>(o, jc);
+  scatter_step<1, kDppXor1>(o, jc);
+  float* out = reinterpret_cast<float*>(a.out) + (size_t)g * HD + h * kD;
   if (nwaves == 1) {
-#pragma unroll
-    for (int qi = 0; qi < NQ; ++qi) {
-      if (qi < a.nq) {
-        const int row = SELF ? g : g * a.nq + qi;
-        Act<T>::store(outp + (size_t)row * HD + h * kD + d_out, o[qi][0]);
-      }
-    }
+    out[dg + 4 * jc] = o[0];
     return;
   }
-#pragma unroll
-  for (int qi = 0; qi < NQ; ++qi) s_out[wave][qi][d_out] = o[qi][0];
+  s_out[wave][dg + 4 * jc] = o[0];
   __syncthreads();
-  for (int e = threadIdx.x; e < NQ * kD; e += blockDim.x) {
-    const int qi = e / kD, d = e % kD;
-    if (qi >= a.nq) continue;
-    float acc = s_out[0][qi][d];
-    for (int w = 1; w < nwaves; ++w) acc += s_out[w][qi][d];
-    const int row = SELF ? g : g * a.nq + qi;
-    Act<T>::store(outp + (size_t)row * HD + h * kD + d, acc);
+  if (threadIdx.x < kD) {
+    float acc = s_out[0][threadIdx.x];
+    for (int w = 1; w < nwaves; ++w) acc += s_out[w][threadIdx.x];
+    out[threadIdx.x] = acc;
   }
 }
 
@@ -343,60 +246,69 @@ attn_step_kernel(AttnArgs a) {
 //   64 items, 12 heads, 256, 40 valid            7.7 / 20.2 / 6.2
 //   64 items, 12 heads, 512, 60 valid           11.1 / 35.2 / 7.6
 //   64 items, 12 heads, 64, 10 valid             4.4 / 6.6 / 4.3
+// and with probabilities read from LDS 16 positions at a time, the first wavefront's
+// requests in front of the length while workgroups are few, before / now: 8 items, 6
+// heads, 64 positions 5.7 / 3.85, 16 x 6 x 256 (100 valid) 7.0 / 5.2, 16 x 6 x 48 5.4 /
+// 3.8, 64 x 12 x 64 (10 valid) 4.8 / 4.5, 64 x 12 x 256 (40 valid) 9.0 / 7.6.
 template <int NQ, int WM>
 __global__ void __launch_bounds__(64 * WM)
 cross_attn_f32_kernel(AttnArgs a) {
-  __shared__ float s_q[NQ][kD];
+  __shared__ __attribute__((aligned(16))) float s_q[NQ][kD];
   __shared__ float s_red[WM][NQ];
-  __shared__ float s_p[NQ][WM * 64];
+  __shared__ __attribute__((aligned(16))) float s_p[NQ][WM * 64];
   __shared__ float s_out[WM][NQ][kD];
   T5D_GATE_READ(a.gate);
   const int h = blockIdx.x, b = blockIdx.y;
-  int n = a.index[b];  // (one wait for both)
-  T5D_GATE_TEST();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int HD = a.H * kD;
-  n = n < 0 ? 0 : (n > a.S ? a.S : n);
-  bool uniform = false;
-  if (n == 0) { uniform = true; n = a.S; }
-  // wavefronts without a position leave (barriers wait for those that are there)
-  if (wave * 64 >= n) return;
-  const int nwaves = (n + 63) >> 6, threads = 64 * nwaves;
   const float* kbase = reinterpret_cast<const float*>(a.k) +
                        ((size_t)b * a.H + h) * (size_t)a.S * kD;
   const float* vbase = reinterpret_cast<const float*>(a.v) +
                        ((size_t)b * a.H + h) * (size_t)kD * a.S;
   const float* qbase = reinterpret_cast<const float*>(a.q);
-  const int j = wave * 64 + lane;
-  const int jb = wave * 64, je = min(n, jb + 64);
-  // keys of this lane's position, values of this lane's row: nothing past the length
-  // but the last position's keys again and the rest of its four values
+  const int j = wave * 64 + lane, jb = wave * 64;
+  // keys of this lane's position, values of this lane's row
   float4 key[kD / 4], value[16];
-  const auto request_keys = [&] {
+  const auto request_keys = [&](int n) {
     const float4* row =
         reinterpret_cast<const float4*>(kbase + (size_t)min(j, n - 1) * kD);
 #pragma unroll
     for (int c = 0; c < kD / 4; ++c) key[c] = row[c];
   };
   // (rows of a multiple of 4 floats, aligned: checked by the caller)
-  const auto request_values = [&] {
+  const auto request_values = [&](int n) {
     const float* row = vbase + (size_t)lane * a.S + jb;
-    if (jb + 64 <= n) {
 #pragma unroll
-      for (int c = 0; c < 16; ++c) value[c] = *reinterpret_cast<const float4*>(row + 4 * c);
-    } else {
-#pragma unroll
-      for (int c = 0; c < 16; ++c) {  // (the others are not looked at)
-        if (jb + 4 * c >= n) break;
-        value[c] = *reinterpret_cast<const float4*>(row + 4 * c);
-      }
+    for (int c = 0; c < 16; ++c) {  // (what is left out is not looked at)
+      if (c % 4 == 0 && jb + 4 * c >= n) break;
+      value[c] = *reinterpret_cast<const float4*>(row + min(4 * c, a.S - 4 - jb));
     }
   };
   constexpr bool kAhead = WM <= 4;
+  const bool early = a.early && wave == 0;
+  int n = a.index[b];  // (one wait for both)
   if constexpr (kAhead) {
-    request_keys();
-    request_values();
+    if (early) {
+      request_keys(a.S);
+      request_values(a.S);
+    }
+  }
+  T5D_GATE_TEST();
+  n = n < 0 ? 0 : (n > a.S ? a.S : n);
+  bool uniform = false;
+  if (n == 0) { uniform = true; n = a.S; }
+  // wavefronts without a position leave (barriers wait for those that are there)
+  if (wave * 64 >= n) return;
+  const int nwaves = (n + 63) >> 6, threads = 64 * nwaves;
+  const int je = min(n, jb + 64);
+  // the others': nothing past the length but the last position's keys again and the
+  // rest of its sixteen values
+  if constexpr (kAhead) {
+    if (!early) {
+      request_keys(n);
+      request_values(n);
+    }
   }
   for (int e = threadIdx.x; e < NQ * kD; e += threads) {
     const int qi = e / kD, d = e % kD;
@@ -404,7 +316,7 @@ cross_attn_f32_kernel(AttnArgs a) {
                      ? qbase[(size_t)(b * a.nq + qi) * a.q_stride + h * kD + d]
                      : 0.f;
   }
-  if constexpr (!kAhead) request_keys();
+  if constexpr (!kAhead) request_keys(n);
   __syncthreads();
   float s[NQ];
 #pragma unroll
@@ -422,9 +334,7 @@ cross_attn_f32_kernel(AttnArgs a) {
       }
     }
   }
-  if constexpr (!kAhead) {
-    request_values();
-  }
+  if constexpr (!kAhead) request_values(n);
 #pragma unroll
   for (int qi = 0; qi < NQ; ++qi) {
     float x = uniform ? 0.f : s[qi];
@@ -459,18 +369,23 @@ cross_attn_f32_kernel(AttnArgs a) {
   float o[NQ];
 #pragma unroll
   for (int qi = 0; qi < NQ; ++qi) o[qi] = 0.f;
-  const auto add = [&](int jj, float v) {
-#pragma unroll
-    for (int qi = 0; qi < NQ; ++qi) o[qi] = fmaf(s_p[qi][jj], v, o[qi]);
-  };
+  // (a branch per 16 positions: with one per four every probability was a wait for LDS
+  // of its own; a masked position's is zero, and its value is not looked at)
 #pragma unroll
   for (int c = 0; c < 16; ++c) {
     const int jj = jb + 4 * c;
-    if (jj >= je) break;
-    add(jj, value[c].x);
-    if (jj + 1 < je) add(jj + 1, value[c].y);
-    if (jj + 2 < je) add(jj + 2, value[c].z);
-    if (jj + 3 < je) add(jj + 3, value[c].w);
+    if (c % 4 == 0 && jj >= je) break;
+    const float4 v = make_float4(jj < je ? value[c].x : 0.f, jj + 1 < je ? value[c].y : 0.f,
+                                 jj + 2 < je ? value[c].z : 0.f,
+                                 jj + 3 < je ? value[c].w : 0.f);
+#pragma unroll
+    for (int qi = 0; qi < NQ; ++qi) {
+      const float4 p = *reinterpret_cast<const float4*>(&s_p[qi][jj]);
+      o[qi] = fmaf(p.x, v.x, o[qi]);
+      o[qi] = fmaf(p.y, v.y, o[qi]);
+      o[qi] = fmaf(p.z, v.z, o[qi]);
+      o[qi] = fmaf(p.w, v.w, o[qi]);
+    }
   }
 #pragma unroll
   for (int qi = 0; qi < NQ; ++qi) s_out[wave][qi][lane] = o[qi];
@@ -485,21 +400,21 @@ cross_attn_f32_kernel(AttnArgs a) {
   }
 }
 
-template <typename T, int NQ, bool SELF>
-static void launch_attn_nq(const AttnArgs& a, int groups, hipStream_t s) {
-  constexpr int BJ = 16 * Act<T>::kElemsPer16B;
-  const int waves = (a.S + BJ - 1) / BJ;
-  dim3 grid(a.H, groups), block(64 * waves);
+static void launch_self_f32(AttnArgs a, int rows, hipStream_t s) {
+  const int waves = (a.S + 63) / 64;
+  dim3 grid(a.H, rows), block(64 * waves);
+  a.early = (int64_t)a.H * rows <= 256;
   if (waves <= 4)
-    hipLaunchKernelGGL((attn_step_kernel<T, NQ, SELF, 4>), grid, block, 0, s, a);
+    hipLaunchKernelGGL(self_attn_f32_kernel<4>, grid, block, 0, s, a);
   else if (waves <= 8)
-    hipLaunchKernelGGL((attn_step_kernel<T, NQ, SELF, 8>), grid, block, 0, s, a);
+    hipLaunchKernelGGL(self_attn_f32_kernel<8>, grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((attn_step_kernel<T, NQ, SELF, 16>), grid, block, 0, s, a);
+    hipLaunchKernelGGL(self_attn_f32_kernel<16>, grid, block, 0, s, a);
 }
 
-static void launch_cross_f32(const AttnArgs& a, int B, hipStream_t s) {
+static void launch_cross_f32(AttnArgs a, int B, hipStream_t s) {
   const int waves = (a.S + 63) / 64;
+  a.early = (int64_t)a.H * B <= 256;
   dim3 grid(a.H, B), block(64 * waves);
 #define T5D_CROSS_F32(NQ_)                                                        \
   do {                                                                            \
@@ -563,7 +478,7 @@ extern "C" int t5d_self_attention_step(void* stream, int dtype, const void* qkv,
   a.H = H; a.S = L; a.nq = 1; a.q_stride = 3 * H * kD;
   a.gate = tls_gate;
   if (dtype == T5D_F32)
-    launch_attn_nq<float, 1, true>(a, R, as_stream(stream));
+    launch_self_f32(a, R, as_stream(stream));
   else
     launch_self_attention_bf16(as_stream(stream), qkv, cached_key, cached_value,
                                rel_bias, cache_index, out, R, H, L, nullptr,

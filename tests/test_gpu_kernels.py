@@ -993,6 +993,30 @@ def test_float32_self_attention_step_of_one_to_sixteen_wavefronts(ops, L, t):
   np.testing.assert_allclose(out, want, atol=1e-5)  # as above
 
 
+@pytest.mark.parametrize('R', [2, 90])  # workgroups that ask early, that do not
+@pytest.mark.parametrize('L,t', [(4, 0), (32, 2), (68, 63), (128, 64), (600, 300)])
+def test_float32_self_attention_step_takes_nothing_from_beyond(ops, R, L, t):
+  """NaN in the cache at the new column and past it.  Bound as above."""
+  rs = np.random.RandomState(L + R)
+  H, D = 3, 64
+  qkv = rs.randn(R, 3, H, D)
+  qkv[:, 0] *= 0.125
+  ck, cv = rs.randn(R, H, D, L), rs.randn(R, H, D, L)
+  ck[..., t:], cv[..., t:] = np.nan, np.nan
+  bias = rs.randn(H, L)
+  dk, dv = dev(ck, torch.float32), dev(cv, torch.float32)
+  out = host(ops.self_attention_step(
+      dev(qkv.reshape(R, -1), torch.float32), dk, dv, dev(bias, torch.float32),
+      torch.tensor(t, dtype=torch.int32, device='cuda'))).reshape(R, H, D)
+  ck[..., t], cv[..., t] = qkv[:, 1], qkv[:, 2]
+  np.testing.assert_array_equal(host(dk), ck.astype(np.float32))
+  np.testing.assert_array_equal(host(dv), cv.astype(np.float32))
+  s = np.einsum('rhd,rhdj->rhj', qkv[:, 0], ck[..., :t + 1]) + bias[:, t::-1][:, :t + 1]
+  p = np.exp(s - s.max(-1, keepdims=True))
+  want = np.einsum('rhj,rhdj->rhd', p / p.sum(-1, keepdims=True), cv[..., :t + 1])
+  np.testing.assert_allclose(out, want, atol=1e-5)
+
+
 @pytest.mark.parametrize('B,beams,H,E', [(3, 4, 2, 512), (32, 4, 12, 512),
                                          (40, 1, 12, 256), (64, 1, 16, 512),
                                          (20, 2, 12, 96)])
