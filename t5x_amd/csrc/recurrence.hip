@@ -955,7 +955,11 @@ recurrence_finish_kernel(RecArgs g) {
 //   no delta rule, 8 heads of 128 x 128        5.8 11.4 21.7 42.6 /  5.0 10.8 21.0 40.6
 //   no delta rule, 4 heads of 48 x 64          4.3  4.8  5.6  6.7 /  3.7  4.2  4.9  6.7
 // (64 states of 8 x 128 x 128 take 13.7 us at the rate of a large copy from memory.)
-template <int DI, bool DELTA, typename T>
+// EXACT: heads of 128 x 128 (a workgroup's four wavefronts have 32 columns each) and
+// taps that are all requested ahead; nothing is tested then and 2100 instructions do
+// instead of 3480, which a lone launch has to fetch (8 heads, one token, in a model's
+// step: delta rule 8.0 -> 6.2 us, without 7.3 -> 5.6).
+template <int DI, bool DELTA, typename T, bool EXACT>
 __global__ void __launch_bounds__(512)
 recurrence_step_kernel(RecArgs g) {
   constexpr int DP = 8 * DI;
@@ -963,32 +967,33 @@ recurrence_step_kernel(RecArgs g) {
   __shared__ __align__(16) float s_v[256];
   __shared__ __align__(16) float s_o[256];
   __shared__ float s_b;
-  T5D_GATED(g.gate);
+  T5D_GATE_READ(g.gate);
   const t5d_recurrence& a = g.a;
   const int h = blockIdx.x % a.H, m = blockIdx.x / a.H, hg = h / (a.H / a.G);
   const int pos = g.b.seq_start[m], slot = g.b.seq_slot[m];
+  const int D = EXACT ? DP : a.D, Dv = EXACT ? DP : a.Dv;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int quad = lane & 7, dg = lane >> 3;
   const int col = 4 * (8 * wave + quad);
-  const bool col_ok = col < a.Dv;
+  const bool col_ok = EXACT || col < Dv;
   const T* p = reinterpret_cast<const T*>(a.proj) + (size_t)m * a.ld_proj;
   // role 0, 1, 2: channels lane + 64 u of q, k, v; role 3: of the decay (the first four
   // wavefronts, there whatever the columns, take one each)
-  constexpr int U = 4;  // groups of 64 channels
+  constexpr int U = EXACT ? (DP + 63) / 64 : 4;  // groups of 64 channels
   constexpr int NT = DI <= 16 ? 4 : 2;  // taps requested ahead (registers)
   const int ring0 = a.taps > 0 ? pos % a.taps : 0;
   // (kept as loaded: a conversion here would wait for the load)
   T now[U], past[U][NT - 1];
   float tap[U][NT];
-  const auto channels = [&](int role) { return role == 2 ? a.Dv : a.D; };
+  const auto channels = [&](int role) { return role == 2 ? Dv : D; };
   const auto column = [&](int role) {
-    return role == 0 ? a.off_q + hg * a.D
-           : role == 1 ? a.off_k + hg * a.D : a.off_v + h * a.Dv;
+    return role == 0 ? a.off_q + hg * D
+           : role == 1 ? a.off_k + hg * D : a.off_v + h * Dv;
   };
   const auto channel = [&](int role) {
-    return role == 0 ? hg * a.D
-           : role == 1 ? (a.G + hg) * a.D : 2 * a.G * a.D + h * a.Dv;
+    return role == 0 ? hg * D
+           : role == 1 ? (a.G + hg) * D : 2 * a.G * D + h * Dv;
   };
   const T* ring = reinterpret_cast<const T*>(a.conv_ring) +
                   (size_t)slot * a.taps * g.C;
@@ -996,16 +1001,16 @@ recurrence_step_kernel(RecArgs g) {
     if (role == 3) {
 #pragma unroll
       for (int u = 0; u < (DP + 63) / 64; ++u) {
-        const int c = min(lane + 64 * u, a.D - 1);
-        tap[u][0] = a.decay_bias[(size_t)h * a.D + c];
-        tap[u][1] = a.low[(size_t)m * a.ld_low + a.off_z + (size_t)h * a.D + c];
+        const int c = min(lane + 64 * u, D - 1);
+        tap[u][0] = a.decay_bias[(size_t)h * D + c];
+        tap[u][1] = a.low[(size_t)m * a.ld_low + a.off_z + (size_t)h * D + c];
       }
       return;
     }
     const int n = channels(role);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (64 * u >= n) break;
+      if (!EXACT && 64 * u >= n) break;
       const int c = min(lane + 64 * u, n - 1), cc = channel(role) + c;
       now[u] = p[column(role) + c];
       if (a.taps == 0) continue;
@@ -1018,20 +1023,24 @@ recurrence_step_kernel(RecArgs g) {
       }
     }
   };
-  float* state = a.state + ((size_t)slot * a.H + h) * a.D * a.Dv + col;
+  float* state = a.state + ((size_t)slot * a.H + h) * D * Dv + col;
   float4 st[DI];
   const auto request_state = [&] {
-    if (pos > 0 && col_ok) {
+    if constexpr (EXACT) {  // (a sequence's first token: not looked at)
+#pragma unroll
+      for (int i = 0; i < DI; ++i)
+        st[i] = *reinterpret_cast<const float4*>(state + (size_t)(dg + 8 * i) * Dv);
+    } else if (pos > 0 && col_ok) {
       constexpr int R = DELTA && DI == 32 ? 1 : 4;  // rows of 8 per test of the size
 #pragma unroll
       for (int i = 0; i < DI; i += R) {
-        const bool there = i == 0 || 8 * i < a.D;
+        const bool there = i == 0 || 8 * i < D;
 #pragma unroll
         for (int e = i; e < i + R; ++e) {
           st[e] = make_float4(0.f, 0.f, 0.f, 0.f);
           if (there)  // (past the last row the last one again)
             st[e] = *reinterpret_cast<const float4*>(
-                state + (size_t)min(dg + 8 * e, a.D - 1) * a.Dv);
+                state + (size_t)min(dg + 8 * e, D - 1) * Dv);
         }
       }
     } else {
@@ -1044,21 +1053,22 @@ recurrence_step_kernel(RecArgs g) {
   const T beta_z = p[DELTA ? a.off_beta + h : 0];
   // the output channel of this lane
   const int co = 64 * wave + lane;
-  const int cg = min(co, a.Dv - 1);
+  const int cg = EXACT ? co % Dv : min(co, Dv - 1);
   const float norm = a.norm[cg];
   // (each from a place that is there; one of them is used)
   const bool low_gate = a.gate == T5D_GATE_SIGMOID_LOW;
   const float gate_low =
-      a.low[(size_t)m * a.ld_low + (low_gate ? a.off_low_gate + h * a.Dv + cg : a.off_z)];
-  const T gate_z = (low_gate ? p : p + a.off_gate + (size_t)h * a.Dv)[low_gate ? 0 : cg];
+      a.low[(size_t)m * a.ld_low + (low_gate ? a.off_low_gate + h * Dv + cg : a.off_z)];
+  const T gate_z = (low_gate ? p : p + a.off_gate + (size_t)h * Dv)[low_gate ? 0 : cg];
   if (DELTA) request_state();
+  T5D_GATE_TEST();
   const auto form = [&](int role) {
     if (role == 3) {
 #pragma unroll
       for (int u = 0; u < (DP + 63) / 64; ++u) {
         const int c = lane + 64 * u;
         if (c < DP)
-          s_g[c] = c < a.D ? expf(log_decay_of(a, tap[u][1] + tap[u][0], h)) : 0.f;
+          s_g[c] = c < D ? expf(log_decay_of(a, tap[u][1] + tap[u][0], h)) : 0.f;
       }
       if (DELTA && lane == 0) s_b = sigmoid_f(to_f32<T>(beta_z));
       return;
@@ -1079,7 +1089,7 @@ recurrence_step_kernel(RecArgs g) {
           for (int j = 1; j < NT; ++j)
             if (j < a.taps && pos - j >= 0)
               v = fmaf(to_f32<T>(past[u][j - 1]), tap[u][j], v);
-          for (int j = NT; j < a.taps && pos - j >= 0; ++j)
+          for (int j = NT; !EXACT && j < a.taps && pos - j >= 0; ++j)
             v = fmaf(to_f32<T>(ring[(size_t)((pos - j) % a.taps) * g.C + cc]),
                      a.conv[(size_t)cc * a.taps + a.taps - 1 - j], v);
           x[u] = v * sigmoid_f(v);
@@ -1099,11 +1109,15 @@ recurrence_step_kernel(RecArgs g) {
   if (wave < 4) form(wave);
   __syncthreads();
   // (a wavefront that was there for its role; barriers wait for those that stay)
-  if (32 * wave >= a.Dv) return;
-  if (a.D < DP) {  // rows past the last were read from it
+  if (32 * wave >= Dv) return;
+  if (EXACT && pos <= 0) {
+#pragma unroll
+    for (int i = 0; i < DI; ++i) st[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if (D < DP) {  // rows past the last were read from it
 #pragma unroll
     for (int i = 0; i < DI; ++i)
-      if (dg + 8 * i >= a.D) st[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (dg + 8 * i >= D) st[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
   float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -1134,20 +1148,20 @@ recurrence_step_kernel(RecArgs g) {
     o.x = fmaf(st[i].x, q, o.x); o.y = fmaf(st[i].y, q, o.y);
     o.z = fmaf(st[i].z, q, o.z); o.w = fmaf(st[i].w, q, o.w);
     const int d = dg + 8 * i;
-    if (col_ok && d < a.D)
-      *reinterpret_cast<float4*>(state + (size_t)d * a.Dv) = st[i];
+    if (EXACT || (col_ok && d < D))
+      *reinterpret_cast<float4*>(state + (size_t)d * Dv) = st[i];
   }
   o.x = over_rows(o.x); o.y = over_rows(o.y);
   o.z = over_rows(o.z); o.w = over_rows(o.w);
   if (dg == 0 && col_ok) *reinterpret_cast<float4*>(s_o + col) = o;
   __syncthreads();
-  if (co - lane >= a.Dv) return;
+  if (co - lane >= Dv) return;
   float ss = 0.f;
-  for (int c = lane; c < a.Dv; c += 64) ss = fmaf(s_o[c], s_o[c], ss);
-  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)a.Dv + a.eps);
-  if (co < a.Dv)
+  for (int c = lane; c < Dv; c += 64) ss = fmaf(s_o[c], s_o[c], ss);
+  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)Dv + a.eps);
+  if (co < Dv)
     Act<T>::store(reinterpret_cast<T*>(a.out) + (size_t)m * a.ld_out +
-                      (size_t)h * a.Dv + co,
+                      (size_t)h * Dv + co,
                   s_o[co] * inv * norm *
                       out_gate_of(a, low_gate ? gate_low : to_f32<T>(gate_z)));
 }
@@ -1155,12 +1169,14 @@ recurrence_step_kernel(RecArgs g) {
 template <bool DELTA, typename T>
 static void launch_step(hipStream_t s, const RecArgs& g) {
   const dim3 grid(g.b.S * g.a.H), block(64 * std::max(4, (g.a.Dv + 31) / 32));
-#define T5D_RS(DI_) \
-  hipLaunchKernelGGL((recurrence_step_kernel<DI_, DELTA, T>), grid, block, 0, s, g)
-  if (g.a.D <= 32) T5D_RS(4);
-  else if (g.a.D <= 64) T5D_RS(8);
-  else if (g.a.D <= 128) T5D_RS(16);
-  else T5D_RS(32);
+#define T5D_RS(DI_, EXACT_)                                                       \
+  hipLaunchKernelGGL((recurrence_step_kernel<DI_, DELTA, T, EXACT_>), grid, block, 0, \
+                     s, g)
+  if (g.a.D <= 32) T5D_RS(4, false);
+  else if (g.a.D <= 64) T5D_RS(8, false);
+  else if (g.a.D == 128 && g.a.Dv == 128 && g.a.taps <= 4) T5D_RS(16, true);
+  else if (g.a.D <= 128) T5D_RS(16, false);
+  else T5D_RS(32, false);
 #undef T5D_RS
 }
 

@@ -545,21 +545,51 @@ window_step_kernel(WinArgs g) {
   constexpr int QS = HP + 8;
   constexpr int LPR = HP / 8;       // lanes on one value row
   constexpr int KPI = 64 / LPR;     // keys per value load
+  constexpr int VL = 64 / KPI;      // value loads of a tile
+  constexpr int VR = VL < 8 ? VL : 8;  // of them ahead (registers)
   __shared__ __align__(16) bf16_t s_q[16 * QS];
+  __shared__ __align__(16) bf16_t s_new[2][HP];  // the new key and value
   __shared__ __align__(16) float s_w[4][64 * GS];  // weights [key][head]
   __shared__ float s_alpha[4][16];
   __shared__ float s_m[4][16], s_l[4][16];
   __shared__ __align__(16) float s_o[4][GS * HP];
-  T5D_GATED(g.gate);
+  T5D_GATE_READ(g.gate);
   const t5d_window_attention& a = g.a;
   const int seq = blockIdx.x / a.G, kv = blockIdx.x % a.G, part = blockIdx.y;
   const int gs = g.gs;              // <= GS
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = lane & 15, gq = lane >> 4;
-  const int i = g.b.seq_start[seq];
   const int W = a.window > 0 ? a.window : (1 << 30);
+
+  // The group's queries (the last one again up to GS), the new key and value: vectors
+  // 0 .. GS - 1, GS, GS + 1.  They depend on nothing but the arguments and are requested
+  // first, the flag and the sequence's place with them.
+  constexpr int U = (HP + 63) / 64, NV = (GS + 5) / 4;  // vectors wave, wave + 4, ...
+  bf16_t raw[NV][U];
+  float scale[NV][U];
+  const auto width = [&](int vec) { return vec > GS ? a.Dv : a.D; };
+  const auto norm = [&](int vec) {
+    return vec < GS ? a.q_norm : vec == GS ? a.k_norm : nullptr;
+  };
+  const bf16_t* p = reinterpret_cast<const bf16_t*>(a.proj) + (size_t)seq * a.ld_proj;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int vec = min(wave + 4 * v, GS + 1);
+    const bf16_t* src = p + (vec < GS ? a.off_q + (kv * gs + min(vec, gs - 1)) * a.D
+                             : vec == GS ? a.off_k + kv * a.D
+                                         : a.off_v + kv * a.Dv);
+    const float* w = norm(vec);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int d = min(lane + 64 * u, width(vec) - 1);
+      raw[v][u] = src[d];
+      scale[v][u] = w != nullptr ? w[d] : 1.f;
+    }
+  }
+  const int i = g.b.seq_start[seq];
   const size_t base = ((size_t)g.b.seq_slot[seq] * a.G + kv) * a.ring;
+  T5D_GATE_TEST();
   bf16_t* K = reinterpret_cast<bf16_t*>(a.key_ring) + base * HP;
   bf16_t* V = reinterpret_cast<bf16_t*>(a.value_ring) + base * HP;
 
@@ -567,7 +597,7 @@ window_step_kernel(WinArgs g) {
   const int j_begin = max(0, i - W + 1) & ~63;
   const int vsub = lane / LPR, vpiece = lane % LPR;
   Frag kf[4][DT];
-  uint4 vr[8];
+  uint4 vr[VR];
   const auto request_tile = [&](int jt) {
     const size_t r = (size_t)(jt % a.ring);
     const bf16_t* kt = K + r * HP;
@@ -579,76 +609,53 @@ window_step_kernel(WinArgs g) {
         kf[t][kk].u = *reinterpret_cast<const uint4*>(
             kt + (size_t)(16 * t + n16) * HP + 32 * kk + 8 * gq);
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (u * KPI < 64)
-        vr[u] = *reinterpret_cast<const uint4*>(
-            vt + (size_t)(u * KPI + vsub) * HP + 8 * vpiece);
+    for (int u = 0; u < VR; ++u)
+      vr[u] = *reinterpret_cast<const uint4*>(
+          vt + (size_t)(u * KPI + vsub) * HP + 8 * vpiece);
   };
 
-  // The group's queries -> LDS, the new key and value -> ring (every part
-  // writes the same bytes there).  Vectors 0 .. gs-1: queries, gs: key, gs + 1:
-  // value; rows gs .. 15 of the query tile are zero.  All of a wavefront's vectors and
-  // its first tile (if the new row is not in it) are requested before the first is
-  // looked at: one after the other, and the tile behind the barrier, one row of 8 heads
-  // over 2 with a window of 1024 lasted 15.5 us, now 13.1 (64 rows: 14.2, now 11.5).
+  // The queries -> LDS, the new key and value -> ring (every part writes the same bytes
+  // there) and LDS.  (Rows GS .. 15 of the query tile are whatever is there: columns of
+  // the products that nothing looks at.)  All of a wavefront's
+  // vectors and its first tile are requested before the first is looked at; the tile that
+  // holds the new row's place does not wait for the ring: it gets the new key, and the
+  // new value is added at the end.
+  // One row of 8 heads over 2 with a window of 1024: 15.5 us one after the other and the
+  // tile behind the barrier, 13.1 with the tile of the new row only behind it, 11.0 so
+  // and with a third fewer instructions; with the kernel that merges the parts, for 1 x
+  // (16 over 4), 4 x (8 over 2) of 300 positions, 64 x (8 over 2), 256 x (8 over 2): 16.5
+  // -> 12.2, 13.4 -> 10.7, 23.6 -> 22.7, 54 -> 52.8.
   const int jt0 = j_begin + 64 * (part + g.splits * wave);
-  const bool ahead = jt0 + 63 < i;
   {
-    constexpr int U = (HP + 63) / 64, NV = 5;  // vectors wave, wave + 4, ...
-    const bf16_t* p = reinterpret_cast<const bf16_t*>(a.proj) + (size_t)seq * a.ld_proj;
-    bf16_t raw[NV][U];
-    float scale[NV][U];
-    const auto live = [&](int vec) { return vec < gs || vec == 16 || vec == 17; };
-    const auto width = [&](int vec) { return vec == 17 ? a.Dv : a.D; };
-    const auto norm = [&](int vec) {
-      return vec < 16 ? a.q_norm : vec == 16 ? a.k_norm : nullptr;
-    };
+    if (jt0 <= i) request_tile(jt0);
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const int vec = wave + 4 * v;
-      if (!live(vec)) continue;
-      const bf16_t* src = p + (vec < 16 ? a.off_q + (kv * gs + vec) * a.D
-                               : vec == 16 ? a.off_k + kv * a.D
-                                           : a.off_v + kv * a.Dv);
-      const float* w = norm(vec);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int d = min(lane + 64 * u, width(vec) - 1);
-        raw[v][u] = src[d];
-        if (w != nullptr) scale[v][u] = w[d];
-      }
-    }
-    if (ahead) request_tile(jt0);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int vec = wave + 4 * v;
-      if (vec >= 18) continue;
-      const bool query = vec < 16;
+      const int vec = min(wave + 4 * v, GS + 1);
       const int n = width(vec);
       const bool normed = norm(vec) != nullptr;
       float f[U];
       float ss = 0.f;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        f[u] = live(vec) && lane + 64 * u < n ? bf16_to_f32(raw[v][u]) : 0.f;
+        f[u] = lane + 64 * u < n ? bf16_to_f32(raw[v][u]) : 0.f;
         ss = fmaf(f[u], f[u], ss);
       }
-      const float inv = normed && live(vec)
-                            ? 1.0f / sqrtf(wave_sum(ss) / (float)n + a.eps) : 1.f;
-      bf16_t* dst = query ? s_q + vec * QS
-                          : (vec == 16 ? K : V) + (size_t)(i % a.ring) * HP;
+      const float inv = normed ? 1.0f / sqrtf(wave_sum(ss) / (float)n + a.eps) : 1.f;
+      bf16_t* dst = vec < GS ? s_q + vec * QS : s_new[vec - GS];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int d = lane + 64 * u;
-        if (d < HP)
-          dst[d] = f32_to_bf16(normed && live(vec) && d < n ? f[u] * inv * scale[v][u]
-                                                            : f[u]);
+        const bf16_t x = f32_to_bf16(f[u] * inv * scale[v][u]);
+        if (d < HP) dst[d] = x;
+        if (d < HP && vec >= GS)
+          ((vec == GS ? K : V) + (size_t)(i % a.ring) * HP)[d] = x;
       }
     }
-    // the key and value rows are in memory before any wavefront reads the ring
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  __syncthreads();
+  // (what goes to and comes from memory is not waited for)
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 
   Frag qf[DT];
 #pragma unroll
@@ -658,15 +665,27 @@ window_step_kernel(WinArgs g) {
   const float scale2 = a.scale * kLog2e;
   const float slope2 = a.slopes != nullptr ? a.slopes[head] * kLog2e : 0.f;
   float mx = kNoMax, l = 0.f;
-  float acc[GS][8];
+  float acc[GS][8], w_new[GS];
 #pragma unroll
-  for (int h = 0; h < GS; ++h)
+  for (int h = 0; h < GS; ++h) {
+    w_new[h] = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
+  }
 
   for (int jt = jt0; jt <= i; jt += 64 * 4 * g.splits) {
     const bf16_t* vt = V + (size_t)(jt % a.ring) * HP;
-    if (jt != jt0 || !ahead) request_tile(jt);
+    if (jt != jt0) request_tile(jt);
+    if (jt + 63 >= i) {  // the new row's place is in this tile
+      const int r = i - jt;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (16 * t + n16 == r) {
+#pragma unroll
+          for (int kk = 0; kk < DT; ++kk)
+            kf[t][kk].u = *reinterpret_cast<const uint4*>(s_new[0] + 32 * kk + 8 * gq);
+        }
+    }
     f32x4_v s[4];
     float top = mx;
 #pragma unroll
@@ -700,6 +719,14 @@ window_step_kernel(WinArgs g) {
     l = l * alpha + sum;
     if (gq == 0) s_alpha[wave][n16] = alpha;
     wave_lds_fence();
+    if (jt + 63 >= i) {  // the new value is added at the end (this is the last tile)
+      float* w = &s_w[wave][(i - jt) * GS];
+#pragma unroll
+      for (int h = 0; h < GS; ++h) w_new[h] = w[h];
+      wave_lds_fence();
+      if (lane < GS) w[lane] = 0.f;
+      wave_lds_fence();
+    }
 #pragma unroll
     for (int h = 0; h < GS; ++h) {
       const float al = s_alpha[wave][h];
@@ -707,17 +734,15 @@ window_step_kernel(WinArgs g) {
       for (int e = 0; e < 8; ++e) acc[h][e] *= al;
     }
 #pragma unroll
-    for (int u0 = 0; u0 * KPI < 64; u0 += 8) {
+    for (int u0 = 0; u0 < VL; u0 += VR) {
+      if (u0 > 0) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        if ((u0 + u) * KPI >= 64) continue;
-        if (u0 > 0)
+        for (int u = 0; u < VR; ++u)
           vr[u] = *reinterpret_cast<const uint4*>(
               vt + (size_t)((u0 + u) * KPI + vsub) * HP + 8 * vpiece);
       }
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        if ((u0 + u) * KPI >= 64) continue;
+      for (int u = 0; u < VR; ++u) {
         float f[8];
         unpack16(vr[u], f);
         const float* w = &s_w[wave][((u0 + u) * KPI + vsub) * GS];
@@ -730,6 +755,14 @@ window_step_kernel(WinArgs g) {
       }
     }
   }
+  if (vsub == 0) {
+    float f[8];
+    unpack16(*reinterpret_cast<const uint4*>(s_new[1] + 8 * vpiece), f);
+#pragma unroll
+    for (int h = 0; h < GS; ++h)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[h][e] = fmaf(w_new[h], f[e], acc[h][e]);
+  }
   // Sum over the lanes that took other keys of the same value piece, then the
   // wavefronts' results meet in LDS.
 #pragma unroll
@@ -737,8 +770,15 @@ window_step_kernel(WinArgs g) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       float v = acc[h][e];
-#pragma unroll
-      for (int step = LPR; step < 64; step *= 2) v += __shfl_xor(v, step, 64);
+      if (LPR <= 4) v += lane_xor4(v);
+      if (LPR <= 8) v += lane_xor8(v);
+      if (LPR <= 16) {
+        v = rows_sum(v);
+      } else {
+        const auto w = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+      }
       acc[h][e] = v;
     }
   if (vsub == 0) {
@@ -782,37 +822,63 @@ window_step_kernel(WinArgs g) {
   }
 }
 
-// The parts of window_step_kernel: one wavefront per (sequence, head).
+constexpr int kMaxSplits = 16;
+
+// The parts of window_step_kernel: one wavefront per (sequence, head).  Lane s looks at
+// the maximum and the sum of part s; the parts' rows are requested with them (a loop
+// over the parts, one wait each, three times over: 5.0 us for 64 rows of 8 heads and two
+// parts, now 4.6; 8 rows of 32 heads, 16 parts, with the kernel in front 26.0 -> 17.9).
 __global__ void __launch_bounds__(64)
 window_merge_kernel(WinArgs g) {
-  T5D_GATED(g.gate);
+  T5D_GATE_READ(g.gate);
   const t5d_window_attention& a = g.a;
   const int seq = blockIdx.x / a.H, h = blockIdx.x % a.H;
   const int kv = h / g.gs, hh = h % g.gs;
-  const size_t step = (size_t)g.gs * (g.HP + 2);
+  const int step = g.gs * (g.HP + 2);
   const float* p = g.parts + ((size_t)seq * a.G + kv) * g.splits * step +
                    (size_t)hh * (g.HP + 2);
+  const int lane = threadIdx.x, mine = min(lane & 15, g.splits - 1);
+  const float part_top = p[mine * step + g.HP];
+  const float part_den = p[mine * step + g.HP + 1];
   const float sink2 = a.sink != nullptr ? a.sink[h] * kLog2e : kNoMax;
-  float top = sink2;
-  for (int s = 0; s < g.splits; ++s) top = fmaxf(top, p[s * step + g.HP]);
+  float row[kMaxSplits];
+  const auto request = [&](int d) {
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s)
+      if (s < g.splits) row[s] = p[s * step + d];
+  };
+  request(min(lane, a.Dv - 1));
+  T5D_GATE_TEST();
+  const float top = fmaxf(lanes16_max(part_top), sink2);
+  const float weight = exp2f(part_top - top);
+  float c[kMaxSplits];
   float den = a.sink != nullptr ? exp2f(sink2 - top) : 0.f;
-  for (int s = 0; s < g.splits; ++s)
-    den = fmaf(exp2f(p[s * step + g.HP] - top), p[s * step + g.HP + 1], den);
-  for (int d = threadIdx.x; d < a.Dv; d += 64) {
+#pragma unroll
+  for (int s = 0; s < kMaxSplits; ++s) {
+    c[s] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), s));
+    if (s < g.splits)
+      den = fmaf(c[s],
+                 __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(part_den), s)),
+                 den);
+  }
+  for (int d = lane; d < a.Dv; d += 64) {
+    if (d >= 64) request(d);
     float num = 0.f;
-    for (int s = 0; s < g.splits; ++s)
-      num = fmaf(exp2f(p[s * step + g.HP] - top), p[s * step + d], num);
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s)
+      if (s < g.splits) num = fmaf(c[s], row[s], num);
     reinterpret_cast<bf16_t*>(a.out)[(size_t)seq * a.ld_out + (size_t)h * a.Dv + d] =
         f32_to_bf16(num / den);
   }
 }
 
-constexpr int kMaxSplits = 16;
-
 static int step_splits(const t5d_window_attention& a, int S) {
   const int span = a.window > 0 ? min(a.window, a.ring) : a.ring;
   int n = 1;
   while (n < kMaxSplits && S * a.G * n < 256 && span >= 512 * n) n *= 2;
+  // one tile of 64 positions per wavefront while CUs are left: a window of 1024 touches
+  // 17 tiles, the last of which made one of 16 wavefronts walk two
+  while (n < kMaxSplits && 4 * n < span / 64 + 1 && S * a.G * (n + 1) <= 256) ++n;
   return n;
 }
 

@@ -305,6 +305,29 @@ def test_window_attention_step_kernel(H, G, D, Dv, window):
       assert rel(row, wants[s][starts[s] + step]) < 1e-2, (step, s)
 
 
+@pytest.mark.parametrize('H,G,D,Dv', [(4, 1, 128, 128), (3, 1, 64, 40), (6, 1, 32, 32),
+                                      (2, 1, 200, 256), (5, 1, 100, 128)])
+@pytest.mark.parametrize('window', [0, 700, 1024])
+def test_window_attention_step_in_parts(H, G, D, Dv, window):
+  """One token per sequence over so many positions that several workgroups share them,
+  with the new one first, last and in between in its tile of 64."""
+  starts = [1085, 1150, 64, 0]
+  T = 1160
+  a = Attention(torch.bfloat16, H, G, D, Dv, window, len(starts), 290, T)
+  x = a.sequence(T)
+  want = a.oracle(x)
+  for slot, n in enumerate(starts):
+    for at in range(0, n, 290):
+      a.run([(slot, at)], [x[at:min(n, at + 290)]])
+  for step in range(5):
+    for order in ([0, 1, 2, 3], [0]) if step == 3 else ([1, 3, 0, 2],):
+      got = a.run([(s, starts[s] + step) for s in order],
+                  [x[starts[s] + step:starts[s] + step + 1] for s in order],
+                  variant=1)
+      for row, s in zip(got, order):
+        assert rel(row, want[starts[s] + step]) < 1e-2, (step, s)
+
+
 @pytest.mark.parametrize('H,G,D,scale,bias', [
     (4, 2, 128, 0.3, False), (4, 2, 64, 0.3, True), (2, 2, 32, -0.4, False),
     (2, 1, 200, 0.0, False)])
@@ -639,6 +662,24 @@ def test_recurrence_portions_and_steps(dt, strong, delta, H, G, D, Dv, taps):
   assert rel(np.concatenate(got), want) < r.tol
   got = [r.run([(0, t, t + 1)], [seq]) for t in range(20)]
   assert rel(np.concatenate(got), want[:20]) < r.tol
+
+
+@pytest.mark.parametrize('dt', DTYPES)
+@pytest.mark.parametrize('delta,H,G,taps', [
+    (True, 2, 2, 4), (True, 4, 2, 1), (True, 2, 2, 0), (True, 2, 1, 5), (False, 3, 3, 0)])
+def test_recurrence_steps_of_heads_of_128(dt, delta, H, G, taps):
+  """Token by token from the first one on (what its slot held is not looked at: NaN), and
+  behind a portion."""
+  T = 12
+  r = Recurrence(dt, delta, H, G, 128, 128, taps, 2, seed=taps)
+  seq = r.sequence(T)
+  want = r.oracle(seq)
+  r.state.fill_(float('nan'))
+  got = [r.run([(1, t, t + 1)], [seq]) for t in range(T)]
+  assert rel(np.concatenate(got), want) < r.tol
+  got = [r.run([(0, 0, 5)], [seq])] + [r.run([(0, t, t + 1)], [seq])
+                                       for t in range(5, T)]
+  assert rel(np.concatenate(got), want) < r.tol
 
 
 @pytest.mark.parametrize('dt', DTYPES)
