@@ -26,14 +26,33 @@ route_kernel(RouteArgs g) {
   const int t = threadIdx.x, E = r.experts, total = g.M * r.top;
   s_first[t] = 0;
   __syncthreads();
-  auto expert_of = [&](int i) {
-    const int m = i / r.top;
-    int id = g.tokens[m];
-    id = id < 0 ? 0 : (id >= g.V ? g.V - 1 : id);
-    const int e = r.table[(size_t)id * r.top + (i - m * r.top)];
-    return e < 0 ? 0 : (e >= E ? E - 1 : e);
+  // The experts of entries i, i + kRouteThreads, ...: two dependent loads an entry, so
+  // eight entries' are under way at a time (32768 entries: 64 us one after the other, 46
+  // so; the rest is the atomics).
+  constexpr int kAhead = 8;
+  auto experts_of = [&](int i, int (&e)[kAhead]) {
+    int m[kAhead], id[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      m[u] = min(i + u * kRouteThreads, total - 1) / r.top;
+      id[u] = g.tokens[m[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      id[u] = id[u] < 0 ? 0 : (id[u] >= g.V ? g.V - 1 : id[u]);
+      e[u] = r.table[(size_t)id[u] * r.top + min(i + u * kRouteThreads, total - 1) -
+                     m[u] * r.top];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) e[u] = e[u] < 0 ? 0 : (e[u] >= E ? E - 1 : e[u]);
   };
-  for (int i = t; i < total; i += kRouteThreads) atomicAdd(&s_first[expert_of(i)], 1);
+  for (int i = t; i < total; i += kAhead * kRouteThreads) {
+    int e[kAhead];
+    experts_of(i, e);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (i + u * kRouteThreads < total) atomicAdd(&s_first[e[u]], 1);
+  }
   __syncthreads();
   // Sums over the experts before this one: of entries, and of tiles.
   const int count = s_first[t];
@@ -67,10 +86,19 @@ route_kernel(RouteArgs g) {
                     min(r.tile_rows, count - i * r.tile_rows), 0);
   s_first[t] = before[0];
   __syncthreads();
-  for (int i = t; i < total; i += kRouteThreads) {
-    const int p = atomicAdd(&s_first[expert_of(i)], 1);
-    r.token_of[p] = i / r.top;
-    r.entry_of[i] = p;
+  for (int i = t; i < total; i += kAhead * kRouteThreads) {
+    int e[kAhead], p[kAhead];
+    experts_of(i, e);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (i + u * kRouteThreads < total) p[u] = atomicAdd(&s_first[e[u]], 1);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int at = i + u * kRouteThreads;
+      if (at >= total) break;
+      r.token_of[p[u]] = at / r.top;
+      r.entry_of[at] = p[u];
+    }
   }
 }
 

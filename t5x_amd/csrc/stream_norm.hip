@@ -241,26 +241,39 @@ struct HyperArgs {
 template <typename T, int S, int VPT>
 __global__ void __launch_bounds__(256)
 hyper_norm_kernel(HyperArgs h) {
-  T5D_GATED(h.gate);
+  T5D_GATE_READ(h.gate);
   const t5d_hyper_norm& g = h.a;
   __shared__ float s4[4];
-  __shared__ float s_mix[S * S], s_spread[S], s_collect[S];
   const int n = g.streams;
   const bool add = g.y != nullptr || g.parts != nullptr;
-  for (int i = threadIdx.x; i < S * S; i += 256) {
-    const int from = i / S, to = i % S;
-    float v = from == to ? 1.f : 0.f;
-    if (g.mix != nullptr && from < n && to < n) v = g.mix[from * n + to];
-    s_mix[i] = v;
+  // Of up to 4 streams the weights are in registers, requested with the row (through LDS,
+  // behind a barrier, and the experts' rows one after the other: 64 rows of 4 x 1024 5.8
+  // us, now 4.7; 8192 rows 55.6, now 53.2); of more they go through LDS.
+  constexpr bool kFew = S <= 4;
+  __shared__ float s_far[kFew ? 1 : S * S + 2 * S];
+  float s_near[kFew ? S * S + 2 * S : 1];
+  const auto weight = [&](int i) {
+    if (i < S * S) {
+      const int from = i / S, to = i % S;
+      return g.mix != nullptr && from < n && to < n ? g.mix[from * n + to]
+                                                    : from == to ? 1.f : 0.f;
+    }
+    const float* w = i < S * S + S ? g.spread : g.collect;
+    const int s = (i - S * S) % S;
+    return s >= n ? 0.f : w != nullptr ? w[s] : 1.f;
+  };
+  if constexpr (kFew) {
+#pragma unroll
+    for (int i = 0; i < S * S + 2 * S; ++i) s_near[i] = weight(i);
+  } else {
+    for (int i = threadIdx.x; i < S * S + 2 * S; i += 256) s_far[i] = weight(i);
+    __syncthreads();
   }
-  if (threadIdx.x < S) {
-    const int s = threadIdx.x;
-    s_spread[s] = s < n ? (g.spread != nullptr ? g.spread[s] : 1.f) : 0.f;
-    s_collect[s] = s < n ? (g.collect != nullptr ? g.collect[s] : 1.f) : 0.f;
-  }
-  __syncthreads();
+  const float* s_mix = kFew ? s_near : s_far;
+  const float *s_spread = s_mix + S * S, *s_collect = s_spread + S;
   const int m = blockIdx.x;
   const int src = g.rows != nullptr ? g.rows[m] : m;
+  T5D_GATE_TEST();
   float* xrow = g.x + (size_t)src * n * g.ld;
   const T* y = reinterpret_cast<const T*>(g.y);
   const T* parts = reinterpret_cast<const T*>(g.parts);
@@ -279,9 +292,17 @@ hyper_norm_kernel(HyperArgs h) {
     if (add) {
       float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
       if (parts != nullptr)
-        for (int t = 0; t < g.top; ++t) {
-          const int r = g.part_row[(size_t)src * g.top + t];
-          fma4(b, g.part_weight, load4<T>(parts + (size_t)r * g.ld + c));
+        for (int t = 0; t < g.top; t += 4) {  // (four rows under way at a time)
+          int r[4];
+          float4 part[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            r[k] = g.part_row[(size_t)src * g.top + min(t + k, g.top - 1)];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) part[k] = load4<T>(parts + (size_t)r[k] * g.ld + c);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (t + k < g.top) fma4(b, g.part_weight, part[k]);
         }
       if (y != nullptr) fma4(b, y_gate, load4<T>(y + (size_t)src * g.ld + c));
 #pragma unroll
