@@ -465,11 +465,11 @@ int t5d_beam_cond(void* stream, const t5d_beam_state* state, int B, int K,
  *   temperature [R] f32; tokens [R] i32, logprobs [R] f32 (out).
  *   workspace: NULL, or t5d_sample_tokens_workspace_bytes(R) bytes of device
  *   memory of the caller's (4-byte aligned, contents irrelevant): with it a
- *   top-k choice (topk <= 64, rescale, R <= 128 rows of >= 4096 logits) runs
- *   as two launches — every row cut into 4 parts that list their own k
- *   largest, then one workgroup per row on those lists alone, which reads
- *   Gumbel noise only for the kept candidates — instead of one workgroup per
- *   row over everything (46 -> 13 us at 64 rows of 32128, k = 40).  The chosen
+ *   top-k choice (topk <= 64) or a greedy one (gumbel NULL) of R <= 128 rows of
+ *   >= 4096 logits runs as two launches — every row cut into 4 parts that list
+ *   their own k largest, or the largest and a sum, then one workgroup per row on
+ *   those alone, which reads Gumbel noise only for the kept candidates — instead
+ *   of one workgroup per row over everything (46 -> 13 us at 64 rows of 32128, k = 40).  The chosen
  *   tokens are the same; log-probs are summed in another order (both exact to
  *   float32 rounding). */
 int64_t t5d_sample_tokens_workspace_bytes(int R);

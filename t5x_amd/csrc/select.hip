@@ -804,7 +804,7 @@ struct SampleArgs {
   const int32_t* noise_step; // null: slot 0
   int noise_ring, R;
   const int32_t* gate;
-  // optional: the rows' top-k candidates found by sample_topk_parts_kernel
+  // optional: the rows' top-k candidates found by sample_parts_kernel
   // (sample_parts_* below), or null
   int32_t* parts;
 };
@@ -1016,7 +1016,7 @@ __device__ __forceinline__ float kth_largest_by_radix(const float4 (&y)[8],
   return key_to_float(prefix);
 }
 
-// ---- top-k sampling in two launches ------------------------------------------------
+// ---- token choice in two launches --------------------------------------------------
 // A row per workgroup leaves three quarters of the device idle at 64 rows, and
 // the workgroup spends its time in a dozen block-wide exchanges.  With a
 // top-k mask only the k largest scaled logits (and their ties) can be chosen
@@ -1026,18 +1026,24 @@ __device__ __forceinline__ float kth_largest_by_radix(const float4 (&y)[8],
 // largest, ties at the k-th included; the row's k largest are among those
 // 4 k.  The row's workgroup then works on that list alone: the k-th largest
 // overall, Gumbel noise gathered for the kept candidates only (the noise
-// tensor is not read otherwise), argmax, log-softmax.  A part whose list
-// overflows (long runs of equal values), a greedy row, logits so low that
-// -1e7 is not far below them: the row is marked and its workgroup runs
-// the one-launch algorithm on the whole row.
-// Workspace (int32 words): counts [R][kSampleParts] (-1: marked), then values
+// tensor is not read otherwise), argmax, log-softmax.  Of a greedy row, and of one whose
+// log-probs are those of the raw logits, a part emits its maximum, the place of it and
+// the sum of exponentials relative to it, which the row's workgroup adds up (in double,
+// relative to the row's maximum).  A part whose list overflows (long runs of equal
+// values) or that holds nothing above -infinity, logits so low that -1e7 is not far below
+// them: the row is marked and its workgroup runs the one-launch algorithm on the whole
+// row.
+// In a model's step, us, one launch / two, rows of 32128: 64 rows, k = 40, log-probs of
+// the raw logits 53.2 / 13.7 + 11.3; 64 greedy rows 20.5 / 8.0 + 4.6; 8 greedy rows 16.2 /
+// 6.6 + 4.7.
+// Workspace (int32 words): counts [R][kSampleParts] (-1: marked, -2: greedy), then values
 // [R][kSampleParts][kSamplePartCap] (float bits), then indices of the same
-// shape.
+// shape, then the parts' sums [R][kSampleParts]: maximum, place, sum (two words).
 constexpr int kSampleParts = 4;
 constexpr int kSamplePartCap = 64;   // candidates a part may emit
 constexpr int kSamplePartList = 256; // elements at or above a part's bound
 __host__ __device__ inline size_t sample_parts_words(int R) {
-  return (size_t)R * kSampleParts * (1 + 2 * kSamplePartCap);
+  return (size_t)R * kSampleParts * (1 + 2 * kSamplePartCap + 4);
 }
 __device__ __forceinline__ int32_t* sample_parts_count(int32_t* ws, int r, int p) {
   return ws + (size_t)r * kSampleParts + p;
@@ -1051,8 +1057,40 @@ __device__ __forceinline__ int32_t* sample_parts_idx(int32_t* ws, int R, int r, 
          ((size_t)r * kSampleParts + p) * kSamplePartCap;
 }
 
+__device__ __forceinline__ int32_t* sample_parts_sums(int32_t* ws, int R, int r, int p) {
+  return ws + (size_t)R * kSampleParts * (1 + 2 * kSamplePartCap) +
+         ((size_t)r * kSampleParts + p) * 4;
+}
+// The row's maximum, the (first) place of it and the sum of exponentials relative to it.
+struct RowSum {
+  float top;
+  int place;
+  double sum;
+};
+__device__ __forceinline__ RowSum sample_row_sum(int32_t* ws, int R, int r) {
+  RowSum all = {-INFINITY, 0x7FFFFFFF, 0.0};
+  float top[kSampleParts];
+  double sum[kSampleParts];
+#pragma unroll
+  for (int p = 0; p < kSampleParts; ++p) {
+    const int32_t* w = sample_parts_sums(ws, R, r, p);
+    top[p] = __int_as_float(w[0]);
+    sum[p] = __hiloint2double(w[3], w[2]);
+    if (top[p] > all.top) {
+      all.top = top[p];
+      all.place = w[1];
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < kSampleParts; ++p)
+    all.sum += sum[p] * exp((double)top[p] - (double)all.top);
+  return all;
+}
+
 __global__ void __launch_bounds__(256)
-sample_topk_parts_kernel(SampleArgs a) {
+sample_parts_kernel(SampleArgs a) {
+  __shared__ Cand cscratch[4];
+  __shared__ double dscratch[4];
   __shared__ float s_wm[4];
   __shared__ float s_lv[kSamplePartList];
   __shared__ int s_li[kSamplePartList];
@@ -1076,9 +1114,41 @@ sample_topk_parts_kernel(SampleArgs a) {
   const float kMinT = 1e-4f;
   if (tid == 0) { s_count = 0; s_out = 0; }
   int32_t* count = sample_parts_count(a.parts, r, p);
-  if (!(T > kMinT)) {  // greedy rows take the one-launch path
-    if (tid == 0) *count = -1;
-    return;
+  const bool greedy = !(T > kMinT);
+  if (greedy || !a.rescale) {
+    Cand best = {-INFINITY, 0x7FFFFFFF};
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float e[4] = {y[u].x, y[u].y, y[u].z, y[u].w};
+#pragma unroll
+      for (int c = 0; c < 4; ++c)  // (ascending within the thread)
+        if (e[c] > best.v) {
+          best.v = e[c];
+          best.i = 4 * (v0 + u * 256 + tid) + c;
+        }
+    }
+    best = block_best(best, cscratch);
+    double sum = 0.0;
+    if (!a.rescale) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        sum += (double)expf(y[u].x - best.v);
+        sum += (double)expf(y[u].y - best.v);
+        sum += (double)expf(y[u].z - best.v);
+        sum += (double)expf(y[u].w - best.v);
+      }
+      sum = block_sum_f64(sum, dscratch);
+    }
+    const bool some = best.v > -INFINITY;
+    if (tid == 0) {
+      int32_t* w = sample_parts_sums(a.parts, a.R, r, p);
+      w[0] = __float_as_int(best.v);
+      w[1] = best.i;
+      w[2] = __double2loint(sum);
+      w[3] = __double2hiint(sum);
+      if (greedy || !some) *count = some ? -2 : -1;
+    }
+    if (greedy || !some) return;
   }
   const float Tm = fmaxf(T, kMinT);
 #pragma unroll
@@ -1160,15 +1230,24 @@ sample_tokens_fast_kernel(SampleArgs a) {
   const int lane = tid & 63, wave = tid >> 6;
   const int V = a.V, nvec = V >> 2;
   if (a.parts != nullptr) {
-    // The row's candidates from sample_topk_parts_kernel: at most
+    // The row's candidates from sample_parts_kernel: at most
     // kSampleParts * kSamplePartCap = 256 of them, one per thread.
     int n[kSampleParts], total = 0;
-    bool usable = true;
+    bool usable = true, greedy = true;
 #pragma unroll
     for (int p = 0; p < kSampleParts; ++p) {
       n[p] = *sample_parts_count(a.parts, r, p);
       usable = usable && n[p] >= 0;
+      greedy = greedy && n[p] == -2;
       total += n[p];
+    }
+    if (greedy) {
+      if (tid == 0) {
+        const RowSum row = sample_row_sum(a.parts, a.R, r);
+        a.tokens[r] = row.place;
+        a.logprobs[r] = a.rescale ? 0.f : 0.f - (float)log(row.sum);
+      }
+      return;
     }
     if (usable) {
       float v = -INFINITY;
@@ -1214,7 +1293,13 @@ sample_tokens_fast_kernel(SampleArgs a) {
         __syncthreads();
         if (tid == 0) {
           a.tokens[r] = best.i;
-          a.logprobs[r] = (fscratch[0] - mx) - (float)log(sum);
+          if (a.rescale) {
+            a.logprobs[r] = (fscratch[0] - mx) - (float)log(sum);
+          } else {
+            const RowSum row = sample_row_sum(a.parts, a.R, r);
+            a.logprobs[r] = (a.logits[(size_t)r * V + best.i] - row.top) -
+                            (float)log(row.sum);
+          }
         }
         return;
       }
@@ -1835,15 +1920,15 @@ static void launch_sample_tokens(hipStream_t s, SampleArgs a, int R) {
                        (a.gumbel == nullptr || ((uintptr_t)a.gumbel % 16) == 0);
   const bool fast = a.V % 4 == 0 && a.V <= 32768 && aligned;
   // Two launches when the rows' candidates can be found by parts: a top-k
-  // mask of at most kSamplePartCap, log-probs of the masked row, rows long
+  // mask of at most kSamplePartCap, or greedy rows alone (there is no noise), rows long
   // enough that every part holds k elements, few enough rows to leave CUs
   // idle otherwise.
-  const bool by_parts = fast && a.parts != nullptr && a.gumbel != nullptr &&
-                        a.topk > 0 && a.topk <= kSamplePartCap && a.rescale &&
-                        !(a.topp > 0.f) && a.V >= 4096 && R <= 128;
+  const bool by_parts = fast && a.parts != nullptr && a.V >= 4096 && R <= 128 &&
+                        (a.gumbel == nullptr ||
+                         (a.topk > 0 && a.topk <= kSamplePartCap && !(a.topp > 0.f)));
   if (!by_parts) a.parts = nullptr;
   if (by_parts)
-    hipLaunchKernelGGL(sample_topk_parts_kernel, dim3(kSampleParts, R),
+    hipLaunchKernelGGL(sample_parts_kernel, dim3(kSampleParts, R),
                        dim3(256), 0, s, a);
   if (fast)
     hipLaunchKernelGGL(sample_tokens_fast_kernel, dim3(R), dim3(1024), 0, s, a);

@@ -1338,6 +1338,41 @@ def test_sample_tokens_topk_in_two_launches(ops, R, V, k):
     assert (counts[3] < 0).all()
 
 
+@pytest.mark.parametrize('R,V', [(1, 4096), (6, 32128), (64, 32128), (128, 5000)])
+@pytest.mark.parametrize('rescale', [True, False])
+@pytest.mark.parametrize('k', [0, 40])
+def test_sample_tokens_by_parts_of_rows(ops, R, V, rescale, k):
+  """Greedy rows alone (k = 0, no noise), and top-k with some greedy rows, with the
+  log-probs of the raw logits and without: the tokens of the one-launch path and of the
+  oracle, log-probs to float32 rounding.  Ties across parts, a part of -infinity, NaN."""
+  rs = np.random.RandomState(R + V + k)
+  logits = (2 * rs.randn(R, V)).astype(np.float32)
+  logits[0, [V // 2 + 7, 5, V - 1]] = 50.0           # the first of equal maxima
+  if R > 3:
+    logits[1, V // 4 - 40:V // 2 + 60] = -np.inf     # a part without anything
+    logits[2, 17] = np.nan
+    logits[3] += np.float32(1e4)
+  temps = np.zeros((R,), np.float32)
+  g = None
+  if k:
+    temps[rs.rand(R) < 0.7] = 0.7
+    g = odec.GumbelNoise(seed=R).noise(0, (R, V))
+  args = (dev(logits), None if g is None else dev(g), dev(temps), k, 0.0, rescale)
+  tok, lp = ops.sample_tokens(*args, workspace=ops.sample_tokens_workspace(R, 'cuda'))
+  tok1, lp1 = ops.sample_tokens(*args)
+  np.testing.assert_array_equal(host(tok), host(tok1))
+  # (the part without anything: whole-row path; NaN: not a number on both)
+  np.testing.assert_allclose(host(lp), host(lp1), atol=2e-6, rtol=2e-6)
+  plain = [r for r in range(R) if temps[r] == 0 and r not in (1, 2)]
+  want = np.argmax(logits, axis=-1)
+  np.testing.assert_array_equal(host(tok)[plain], want[plain])
+  if not rescale:
+    x = logits[plain].astype(np.float64)
+    top = x.max(-1)
+    exact = -np.log(np.exp(x - top[:, None]).sum(-1))
+    np.testing.assert_allclose(host(lp)[plain], exact, rtol=2e-6)
+
+
 def test_sample_tokens_topp_table(ops):
   # t5x/binary_search_test.py:143-209 through the kernel: with a huge Gumbel
   # bonus on one index the sampled token reveals whether it survived the mask.
