@@ -1,6 +1,8 @@
 // Dense layers over many rows (the encoder side: M = batch x encoder length).
 //
-// Unlike the decode-step GEMMs these are compute-bound.  A workgroup (4
+// Unlike the decode-step GEMMs these are compute-bound.  Two kernels:
+// rows_gemm_direct_kernel, further down, and for K = 32 and operands beyond its reach
+// rows_gemm_kernel.  There a workgroup (4
 // wavefronts, 2 x 2) owns a 256 x 128 output tile, each wavefront a 128 x 64
 // sub-tile = 8 x 4 MFMA tiles (v_mfma_f32_16x16x32_bf16).  Per k-tile of 32 the
 // workgroup needs 16 activation fragments (16 rows x 64 bytes each) and 8
@@ -425,7 +427,7 @@ rows_gemm_kernel(RowsGemmArgs g) {
   }
 }
 
-// ---- bfloat16 weights, K >= 64: rows through LDS, weights into registers ---------
+// ---- K >= 64: rows through LDS, weights into registers --------------------------
 // A workgroup of 4 wavefronts owns BM = 16 MT rows x BN = 64 NT columns, a wavefront all
 // rows of 16 NT columns.  So every weight is wanted by one wavefront only, and packed
 // weights come in operand order: they go straight from memory into registers, two
@@ -452,7 +454,9 @@ rows_gemm_kernel(RowsGemmArgs g) {
 //  x 768 46.7 -> 33, 5000 x 2816 x 1024 47 -> 34, 8192 x 1024 x 5632 gated 91 -> 81,
 //  14000 x 1024 x 5632 gated 161 -> 132, 16384 x 4096 x 4096 412 -> 385 (1428 TFLOP/s;
 //  matrix instructions alone, on random numbers, reach 2000 at the clock that is left
-//  then), 2000 x 2048 x 768 16.9 -> 13, 1000 x 1024 x 5632 20.8 -> 14.3.
+//  then), 2000 x 2048 x 768 16.9 -> 13, 1000 x 1024 x 5632 20.8 -> 14.3.  int8 weights,
+//  widened in registers (before: 256 x 128 through staging registers): 8192 x 2048 x 2048
+//  80 -> 65, 8192 x 5120 x 2048 175 -> 147, 1000 x 2816 x 1024 63 -> 22.
 //
 // Every wait is counted: the loop is straight-line code (rounds of three steps, as the
 // ring and the register sets want; what is left over stands behind it), requests past
@@ -462,9 +466,34 @@ rows_gemm_kernel(RowsGemmArgs g) {
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_r;
 
-union FragW {
-  u32x4_r r;
-  bf16x8_r v;
+typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_r;
+
+// A weight tile's piece as a buffer load gives it, and as a matrix operand.
+template <typename WT> struct RowsWeight;
+template <> struct RowsWeight<bf16_t> {
+  static constexpr int kTileBytes = 1024;
+  u32x4_r raw;
+#if defined(__HIP_DEVICE_COMPILE__)
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t from, int lane, int at) {
+    raw = __builtin_amdgcn_raw_buffer_load_b128(from, 16 * lane, at, 0);
+  }
+#endif
+  __device__ __forceinline__ bf16x8_r frag() const {
+    return __builtin_bit_cast(bf16x8_r, raw);
+  }
+};
+template <> struct RowsWeight<int8_t> {
+  static constexpr int kTileBytes = 512;
+  u32x2_r raw;
+#if defined(__HIP_DEVICE_COMPILE__)
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t from, int lane, int at) {
+    raw = __builtin_amdgcn_raw_buffer_load_b64(from, 8 * lane, at, 0);
+  }
+#endif
+  __device__ __forceinline__ bf16x8_r frag() const {
+    return __builtin_bit_cast(
+        bf16x8_r, RowsWeightTile<int8_t>::frag(make_uint2(raw[0], raw[1])));
+  }
 };
 
 // What a 32-bit offset of a buffer access reaches.
@@ -498,11 +527,13 @@ __device__ __forceinline__ void rows_multiply_far(const RowsGemmArgs& g,
   }
 }
 
-template <bool SWAP, int MT, int NT, int OCC, int DENSE = 0, bool GROUPED = false>
+template <typename WT, bool SWAP, int MT, int NT, int OCC, int DENSE = 0,
+          bool GROUPED = false>
 __global__ void __launch_bounds__(256, OCC)
 rows_gemm_direct_kernel(RowsGemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (buffer descriptors are no host type)
   constexpr int BM = 16 * MT, BN = 64 * NT;
+  constexpr int TB = RowsWeight<WT>::kTileBytes;
   constexpr int AL = BM / 32;  // 1 KB pieces (8 rows) a wavefront loads per stage
   // Before every barrier: all but the newest rows and weights have landed (the stage
   // and the weight tile about to be multiplied), and my reads of LDS have returned.  A
@@ -589,12 +620,12 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   // K of 32 modulo 64: the last step has no second half, whose pieces are the first's
   const int a_back = (KT & 1) && ld_piece >= 4 ? 64 : 0;
   const __amdgpu_buffer_rsrc_t w_rows = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(g.W + (size_t)n_blk * (BN / 16) * KT * 1024), 0, 0x7fffffff, 0x00020000);
+      (void*)(g.W + (size_t)n_blk * (BN / 16) * KT * TB), 0, 0x7fffffff, 0x00020000);
   int w_off[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
-    w_off[nt] = min(wave * NT + nt, n_tiles - 1 - n_blk * (BN / 16)) * KT * 1024;
-  FragW w0[NT], w1[NT], w2[NT];
+    w_off[nt] = min(wave * NT + nt, n_tiles - 1 - n_blk * (BN / 16)) * KT * TB;
+  RowsWeight<WT> w0[NT], w1[NT], w2[NT];
 
 #define T5D_ROWS_ISSUE_A(s_, S_)                                               \
   do {                                                                         \
@@ -607,8 +638,7 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   } while (0)
 #define T5D_ROWS_ISSUE_W(kt_, W_)                                              \
   _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                            \
-    W_[nt].r = __builtin_amdgcn_raw_buffer_load_b128(                          \
-        w_rows, 16 * lane, w_off[nt] + min((kt_), KT - 1) * 1024, 0)
+    W_[nt].load(w_rows, lane, w_off[nt] + min((kt_), KT - 1) * TB)
 #define T5D_ROWS_READ(S_, half_, p_, X_)                                       \
   _Pragma("unroll") for (int j = 0; j < 2; ++j)                                \
     X_[j].u = S_[(2 * (p_) + j) * 128 + l16 * 8 +                              \
@@ -618,27 +648,29 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
     _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                          \
       acc[2 * (p_) + j][nt] =                                                  \
           SWAP ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(                      \
-                     W_[nt].v, X_[j].v, acc[2 * (p_) + j][nt], 0, 0, 0)        \
+                     W_[nt], X_[j].v, acc[2 * (p_) + j][nt], 0, 0, 0)          \
                : __builtin_amdgcn_mfma_f32_16x16x32_bf16(                      \
-                     X_[j].v, W_[nt].v, acc[2 * (p_) + j][nt], 0, 0, 0)
+                     X_[j].v, W_[nt], acc[2 * (p_) + j][nt], 0, 0, 0)
 #define T5D_FENCE __builtin_amdgcn_sched_barrier(0)
   // Half a step: operands in x at its start, those of what follows in x at its end.
 #define T5D_ROWS_HALF(S_, half_, W_)                                           \
+  _Pragma("unroll") for (int nt = 0; nt < NT; ++nt) wf[nt] = W_[nt].frag();    \
   _Pragma("unroll") for (int p = 0; p < MT / 2; p += 2) {                      \
     T5D_ROWS_READ(S_, half_, p + 1, y);                                        \
     T5D_FENCE;                                                                 \
-    T5D_ROWS_PRODUCTS(p, x, W_);                                               \
+    T5D_ROWS_PRODUCTS(p, x, wf);                                               \
     T5D_FENCE;                                                                 \
     if (p + 2 < MT / 2) T5D_ROWS_READ(S_, half_, p + 2, x);                    \
     else if ((half_) == 0) T5D_ROWS_READ(S_, 1, 0, x);                         \
     T5D_FENCE;                                                                 \
-    T5D_ROWS_PRODUCTS(p + 1, y, W_);                                           \
+    T5D_ROWS_PRODUCTS(p + 1, y, wf);                                           \
     T5D_FENCE;                                                                 \
   }
   // Step s_ on stage CUR_ with weights WA_, WB_; WC_, then WA_ take the next step's.
 #define T5D_ROWS_STEP(s_, CUR_, NEXT2_, WA_, WB_, WC_, second_half_)           \
   do {                                                                         \
     FragR x[2], y[2];                                                          \
+    bf16x8_r wf[NT];                                                           \
     __builtin_amdgcn_s_waitcnt(kWaitStage);                                    \
     __builtin_amdgcn_s_barrier();                                              \
     T5D_ROWS_READ(CUR_, 0, 0, x);                                              \
@@ -683,7 +715,7 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
     // the requests past the end have landed, every wavefront is done with the ring
     __builtin_amdgcn_s_waitcnt(kWaitAll);
     __syncthreads();
-    rows_epilogue_staged<DENSE, false>(
+    rows_epilogue_staged<DENSE, sizeof(WT) == 1>(
         g, acc, m0, nt0, n_tiles, lane,
         reinterpret_cast<char*>(&s_a0[0]) + wave * kRowsStageBytes<NT>);
   } else {
@@ -730,8 +762,8 @@ static double rows_tile_cost(const RowsTile& t, int64_t M, int N) {
 
 // Whether the kernel takes the shape (offsets inside a workgroup's rows and weights are
 // 32 bits wide), else rows_gemm_kernel does.
-static bool rows_direct(int w_dtype, int K, int64_t lda) {
-  return w_dtype == T5D_BF16 && K >= 64 && 2LL * 256 * K < kRowsReach &&
+static bool rows_direct(int K, int64_t lda) {
+  return K >= 64 && 2LL * 256 * K < kRowsReach &&
          2LL * 128 * lda + 2LL * K < kRowsReach;
 }
 
@@ -751,22 +783,32 @@ static const RowsTile& rows_tile(int64_t M, int N, int code) {
 }
 
 extern "C" int t5d_gemm_rows_tile(int w_dtype, int64_t M, int K, int N) {
-  if (M <= 0 || N <= 0 || K <= 0 || !rows_direct(w_dtype, K, K)) return 1;
+  if (w_dtype != T5D_BF16 || M <= 0 || N <= 0 || K <= 0 || !rows_direct(K, K)) return 1;
   return rows_tile(M, N, 0).code;
 }
 
 template <bool SWAP, int DENSE>
-static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int code) {
-  const RowsTile& t = rows_tile(g.M, g.N, code);
+static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int w_dtype,
+                               int code) {
+  // (int8 weights, which are widened in registers on their way to the matrix cores, have
+  // the tiles of 128 columns only)
+  const RowsTile& t = rows_tile(g.M, g.N, w_dtype == T5D_I8 ? 1 : code);
   const dim3 grid((unsigned)((g.M + t.rows - 1) / t.rows) *
                   ((g.N + t.cols - 1) / t.cols));
-#define T5D_ROWS_LAUNCH(MT_, NT_, OCC_)                                          \
-  hipLaunchKernelGGL((rows_gemm_direct_kernel<SWAP, MT_, NT_, OCC_, DENSE>), grid, \
-                     dim3(256), 0, s, g)
-  if (t.rows == 64) T5D_ROWS_LAUNCH(4, 2, 4);
-  else if (t.cols == 128) T5D_ROWS_LAUNCH(8, 2, 3);
-  else if (t.cols == 192) T5D_ROWS_LAUNCH(8, 3, 2);
-  else T5D_ROWS_LAUNCH(8, 4, 2);
+#define T5D_ROWS_LAUNCH(WT_, MT_, NT_, OCC_)                                     \
+  hipLaunchKernelGGL((rows_gemm_direct_kernel<WT_, SWAP, MT_, NT_, OCC_, DENSE>), \
+                     grid, dim3(256), 0, s, g)
+  if constexpr (DENSE == 0) {
+    if (w_dtype == T5D_I8) {
+      if (t.rows == 64) T5D_ROWS_LAUNCH(int8_t, 4, 2, 4);
+      else T5D_ROWS_LAUNCH(int8_t, 8, 2, 3);
+      return;
+    }
+  }
+  if (t.rows == 64) T5D_ROWS_LAUNCH(bf16_t, 4, 2, 4);
+  else if (t.cols == 128) T5D_ROWS_LAUNCH(bf16_t, 8, 2, 3);
+  else if (t.cols == 192) T5D_ROWS_LAUNCH(bf16_t, 8, 3, 2);
+  else T5D_ROWS_LAUNCH(bf16_t, 8, 4, 2);
 #undef T5D_ROWS_LAUNCH
 }
 
@@ -778,11 +820,11 @@ static int launch_rows(hipStream_t s, int w_dtype, const RowsGemmArgs& g,
   const dim3 grid((unsigned)m_blocks * n_blocks), block(256);
   const bool swap = g.layout != T5D_OUT_HEADS_VALUE;
   const int dense = g.epilogue == T5D_EPI_CLAMPED_GLU ? 1 : g.C32 != nullptr ? 2 : 0;
-  if (rows_direct(w_dtype, g.K, g.lda)) {
-    if (dense == 1) launch_rows_direct<true, 1>(s, g, tile);
-    else if (dense == 2) launch_rows_direct<true, 2>(s, g, tile);
-    else if (swap) launch_rows_direct<true, 0>(s, g, tile);
-    else launch_rows_direct<false, 0>(s, g, tile);
+  if (rows_direct(g.K, g.lda)) {
+    if (dense == 1) launch_rows_direct<true, 1>(s, g, w_dtype, tile);
+    else if (dense == 2) launch_rows_direct<true, 2>(s, g, w_dtype, tile);
+    else if (swap) launch_rows_direct<true, 0>(s, g, w_dtype, tile);
+    else launch_rows_direct<false, 0>(s, g, w_dtype, tile);
   } else if (dense == 1) {
     hipLaunchKernelGGL((rows_gemm_kernel<bf16_t, true, 1>), grid, block, 0, s, g);
   } else if (dense == 2) {
@@ -915,16 +957,16 @@ int t5d::launch_grouped_rows(hipStream_t s, const GroupedArgs& a, int n_tiles) {
   const bool wide = n256 * 256 <= n128 * 128 + 64;
   const dim3 grid(t64 * (wide ? n256 : n128)), block(256);
   if (wide && glu)
-    hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 8, 4, 2, 1, true>), grid, block, 0,
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<bf16_t, true, 8, 4, 2, 1, true>), grid, block, 0,
                        s, g);
   else if (wide)
-    hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 8, 4, 2, 0, true>), grid, block, 0,
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<bf16_t, true, 8, 4, 2, 0, true>), grid, block, 0,
                        s, g);
   else if (glu)
-    hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 8, 2, 3, 1, true>), grid, block, 0,
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<bf16_t, true, 8, 2, 3, 1, true>), grid, block, 0,
                        s, g);
   else
-    hipLaunchKernelGGL((rows_gemm_direct_kernel<true, 8, 2, 3, 0, true>), grid, block, 0,
+    hipLaunchKernelGGL((rows_gemm_direct_kernel<bf16_t, true, 8, 2, 3, 0, true>), grid, block, 0,
                        s, g);
   T5D_CHECK_LAUNCH("t5d_grouped_dense_run(rows)");
   return T5D_OK;

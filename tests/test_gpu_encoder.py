@@ -212,6 +212,24 @@ def test_gemm_rows_of_every_tile_over_the_ends_of_k(ops, K, tile):
     assert bool(((got.float() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize('K', [64, 96, 192, 224, 256, 320])
+@pytest.mark.parametrize('M', [130, 4200])  # tiles of 64 rows, of 128
+def test_gemm_rows_of_int8_weights_over_the_ends_of_k(ops, K, M):
+  """As above with int8 weights: a product with whole numbers, scaled per column."""
+  rs = np.random.RandomState(K + M)
+  N = 400
+  a = dev(rs.randn(M, K).astype(np.float32), torch.bfloat16)
+  w = ops.pack_weight(dev((rs.randn(K, N) / np.sqrt(K)).astype(np.float32)),
+                      torch.bfloat16, torch.int8)
+  q = torch.eye(K, dtype=torch.bfloat16, device='cuda')  # (what the weights stand for)
+  wide = torch.cat([ops.gemm(q[k:k + 64], w, out_dtype=torch.float32)
+                    for k in range(0, K, 64)])
+  want = a.float() @ wide
+  got = ops.gemm_rows(a, w)
+  assert bool(((got.float() - want).abs() <=
+               want.abs() * (2.0**-8 + 1e-5) + 1e-5).all())
+
+
 @pytest.mark.parametrize('B,E,H', [(1, 132, 1), (5, 60, 4), (3, 344, 13)])
 def test_gemm_rows_head_layouts_of_low_tiles(ops, B, E, H):
   from t5x_amd import _lib
