@@ -1184,6 +1184,23 @@ extern "C" int t5d_gemm(void* stream, int dtype, int w_dtype, int out_dtype,
   return T5D_OK;
 }
 
+// Whether up to kMaxRows rows with float32 results (the layer that gives logits) run on
+// the many-row kernel: where its tiles, 64 rows x 128 columns or beyond 64 rows 128 x 128,
+// give most CUs one.  It then streams the weights once and in step with the products,
+// where the kernels for few rows split K over wavefronts and fetch the rows per 64
+// columns.  us, few-row / many-row kernel, weights from memory, N = 32128 (251 tiles), 24,
+// 32, 64, 128 rows: K = 768 14.5 / 15.0, 15.5 / 15.1, 20.6 / 16.3, 29.8 / 19.0; K = 1024
+// 16.9 / 16.5, 17.9 / 16.9, 24.0 / 18.2, 34.1 / 21.5; K = 2048 30.3 / 28.9, 35.1 / 29.7,
+// 41.7 / 31.3, 57.6 / 35.3.  Beyond 64 rows K = 1024, N = 20000 (157 tiles): 96 rows
+// 20.0 / 18.4; N = 16384 (128): 96 rows 16.2 / 16.9.  With its sums not yet folded, so at
+// its fastest, it lost at 16 rows (K = 768, N = 32128: 12.2 / 13.4) and with few tiles
+// (K = 1024, N = 8000, 64 rows: 9.8 / 13.1).  K and lda: what the offsets of that kernel
+// reach.
+static bool many_columns(int M, int K, int N, int lda) {
+  return M > 24 && N >= 128 * (M > 64 ? 150 : 240) && K >= 64 &&
+         K < (1 << 22) && lda < (1 << 22);
+}
+
 extern "C" int t5d_dense(void* stream, int dtype, int out_dtype, const void* A,
                          int lda, const void* W, void* C, int ldc, int n_store,
                          int M, int K, int N, int epilogue, float glu_limit,
@@ -1220,7 +1237,7 @@ extern "C" int t5d_dense(void* stream, int dtype, int out_dtype, const void* A,
               "t5d_dense: K=%d N=%d must tile 32x16, lda=%d", K, N, lda);
   T5D_REQUIRE((((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16) == 0, T5D_EINVAL,
               "t5d_dense: operands must be 16-byte aligned");
-  if (M > kMaxRows)
+  if (M > kMaxRows || (out_dtype == T5D_F32 && many_columns(M, K, N, lda)))
     return launch_dense_rows(s, A, lda, W, C, out_dtype == T5D_F32, ldc, n_store,
                              M, K, N, epilogue, glu_limit, glu_alpha, glu_add);
   GemmPlan p;

@@ -78,8 +78,8 @@ struct RowsGemmArgs {
   float* C32;              // float32 output rows instead of C (rows layout, no
   int ldc, n_store;        // epilogue): row stride, columns stored of the N
   float glu_limit, glu_alpha, glu_add;  // T5D_EPI_CLAMPED_GLU
-  const int32_t* gate;     // GROUPED kernels only, with the next
-  GroupTiles grp;
+  const int32_t* gate;     // optional device-side enable flag (rows_gemm_direct_kernel)
+  GroupTiles grp;          // GROUPED kernels only, with the next
   int n_tiles;
 };
 
@@ -527,8 +527,13 @@ __device__ __forceinline__ void rows_multiply_far(const RowsGemmArgs& g,
   }
 }
 
+// FOLD: the sums of every step are added up apart from one another, as the kernels for
+// few rows, in whose place this one then stands, add up those of their wavefronts:
+// float32 results over K = 768, 1024, 2048 lie 8.3e-8, 9.4e-8, 1.31e-7 off the float64
+// ones there, 1.57e-7, 1.84e-7, 2.71e-7 with one sum over all of K, 8.0e-8, 8.8e-8,
+// 1.12e-7 so.
 template <typename WT, bool SWAP, int MT, int NT, int OCC, int DENSE = 0,
-          bool GROUPED = false>
+          bool GROUPED = false, bool FOLD = false>
 __global__ void __launch_bounds__(256, OCC)
 rows_gemm_direct_kernel(RowsGemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (buffer descriptors are no host type)
@@ -552,9 +557,9 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   const int KT = g.K >> 5, KS = (KT + 1) >> 1, n_tiles = g.N >> 4;
   const int n_blocks = (n_tiles + BN / 16 - 1) / (BN / 16);
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  T5D_GATED(g.gate);
   int m_blk, n_blk;
   if constexpr (GROUPED) {
-    T5D_GATED(g.gate);
     // 4 consecutive tiles of rows, most of them of one group, on one XCD, all
     // columns of half a tile in a row: rows and kernels come from that XCD's L2.
     const int t = slot / n_blocks;
@@ -690,11 +695,32 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   T5D_ROWS_ISSUE_W(1, w1);
   T5D_ROWS_ISSUE_A(1, s_a1);
   T5D_FENCE;
+  f32x4_r sums[FOLD ? MT : 1][FOLD ? NT : 1];
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) sums[mt][nt] = acc[mt][nt];
+  }
+  const auto fold = [&] {
+    if constexpr (FOLD) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          sums[mt][nt] += acc[mt][nt];
+          acc[mt][nt] = (f32x4_r){0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  };
   int s = 0;
   for (; s + 3 <= KT >> 1; s += 3) {
     T5D_ROWS_STEP(s, s_a0, s_a2, w0, w1, w2, true);
+    fold();
     T5D_ROWS_STEP(s + 1, s_a1, s_a0, w2, w0, w1, true);
+    fold();
     T5D_ROWS_STEP(s + 2, s_a2, s_a1, w1, w2, w0, true);
+    fold();
   }
   // the last 0 to 3 steps
   if (s < KS) {
@@ -711,6 +737,12 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
 #undef T5D_FENCE
 #undef T5D_ROWS_HALF
 #undef T5D_ROWS_STEP
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[mt][nt] += sums[mt][nt];
+  }
   if (SWAP) {
     // the requests past the end have landed, every wavefront is done with the ring
     __builtin_amdgcn_s_waitcnt(kWaitAll);
@@ -933,8 +965,19 @@ int t5d::launch_dense_rows(hipStream_t s, const void* A, int lda,
   g.epilogue = epilogue; g.layout = T5D_OUT_ROWS;
   g.E = g.Ep = g.H = 0; g.at = nullptr;
   g.lda = lda; g.ldc = ldc; g.n_store = n_store;
-  g.gate = nullptr; g.grp = GroupTiles(); g.n_tiles = 0;
+  g.gate = tls_gate; g.grp = GroupTiles(); g.n_tiles = 0;
   g.glu_limit = glu_limit; g.glu_alpha = glu_alpha; g.glu_add = glu_add;
+  if (g.M <= 128) {  // (float32 results of many columns: see t5d_dense)
+    const dim3 grid((g.N + 127) / 128), block(256);
+    if (g.M <= 64)
+      hipLaunchKernelGGL((rows_gemm_direct_kernel<bf16_t, true, 4, 2, 3, 2, false, true>),
+                         grid, block, 0, s, g);
+    else
+      hipLaunchKernelGGL((rows_gemm_direct_kernel<bf16_t, true, 8, 2, 2, 2, false, true>),
+                         grid, block, 0, s, g);
+    T5D_CHECK_LAUNCH("t5d_dense(columns)");
+    return T5D_OK;
+  }
   return launch_rows(s, T5D_BF16, g, 0);
 }
 

@@ -212,6 +212,25 @@ def test_gemm_rows_of_every_tile_over_the_ends_of_k(ops, K, tile):
     assert bool(((got.float() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize('M,N', [(24, 30720), (25, 30720), (64, 30736), (65, 19216),
+                                 (128, 19200), (128, 19184)])
+@pytest.mark.parametrize('K', [32, 64, 96, 320, 768])
+def test_dense_of_many_columns(ops, M, N, K):
+  """float32 results of few rows at both sides of the line to the many-row kernel: no
+  further off than sums of 64 products added up one after the other (2^-24 of the
+  largest partial sum a step), stored columns and strides of their own."""
+  rs = np.random.RandomState(M + K)
+  a = dev(rs.randn(M, K).astype(np.float32), torch.bfloat16)
+  w = dev((rs.randn(K, N) / np.sqrt(K)).astype(np.float32), torch.bfloat16)
+  pw = ops.pack_weight(w.float(), torch.bfloat16)
+  want = a.double() @ w.double()
+  bound = 2.0**-24 * (K / 64 + 8) * (a.double().abs() @ w.double().abs())
+  for n_store in (N, N - 5):
+    got = ops.dense(a, pw, out_dtype=torch.float32, n_store=n_store)
+    assert got.shape == (M, n_store)
+    assert bool(((got.double() - want[:, :n_store]).abs() <= bound[:, :n_store]).all())
+
+
 @pytest.mark.parametrize('K', [64, 96, 192, 224, 256, 320])
 @pytest.mark.parametrize('M', [130, 4200])  # tiles of 64 rows, of 128
 def test_gemm_rows_of_int8_weights_over_the_ends_of_k(ops, K, M):
