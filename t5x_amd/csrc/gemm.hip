@@ -79,6 +79,15 @@ gemm_mfma_kernel(Args g) {
   const char* wbase = reinterpret_cast<const char*>(g.W);
   constexpr int TB = WeightTile<WT>::kTileBytes;
 
+  // (NJ > 0: where this wavefront's first tiles lie; the others follow at constant
+  // distances, which the loads take as offsets)
+  const char* w_first = wbase + (size_t)wave * 2 * TB;
+  const bf16_t* a_first[MP];
+#pragma unroll
+  for (int mt = 0; mt < MP; ++mt)  // rows past the edge are never stored
+    a_first[mt] = g.A + (size_t)min(m0 + mt * 16 + arow, g.M - 1) * row_stride(g) +
+                  akoff + 64 * wave;
+
   typename WeightTile<WT>::Raw bq[PF][2][NT];
   auto load_b = [&](int slot_, int j) {
     const int kt = (wave + 4 * j) * 2;
@@ -89,7 +98,8 @@ gemm_mfma_kernel(Args g) {
         const int nt = nt0 + nn;
         if (NJ > 0)  // every k-tile exists; tiles past the edge are never stored
           bq[slot_][h][nn] = WeightTile<WT>::load(
-              wbase + ((size_t)min(nt, n_tiles_total - 1) * KT + kt + h) * TB,
+              w_first + (size_t)min(nt, n_tiles_total - 1) * KT * TB +
+                  (8 * j + h) * TB,
               lane);
         else if (nt < n_tiles_total && kt + h < KT)
           bq[slot_][h][nn] = WeightTile<WT>::load(
@@ -132,9 +142,9 @@ gemm_mfma_kernel(Args g) {
           continue;
         }
         const int row = m0 + mt * 16 + arow;
-        if (NJ > 0)  // rows past the edge are never stored
-          aq[slot_][h][mt] = *reinterpret_cast<const uint4*>(
-              g.A + (size_t)min(row, g.M - 1) * row_stride(g) + (kt + h) * 32 + akoff);
+        if (NJ > 0)
+          aq[slot_][h][mt] =
+              *reinterpret_cast<const uint4*>(a_first[mt] + 256 * j + 32 * h);
         else if (row < g.M && kt + h < KT)
           aq[slot_][h][mt] = *reinterpret_cast<const uint4*>(
               g.A + (size_t)row * row_stride(g) + (kt + h) * 32 + akoff);
@@ -294,7 +304,15 @@ gemm_mfma_kernel(Args g) {
 // the row statistics come from the fragments already loaded for the product:
 // one exchange through LDS, no second pass over x, and only 16 rows per
 // workgroup to normalise.
-template <int NT, int NJ, typename WT>
+// What bounds it is instructions, to fetch (each is new to a CU) and to issue: 16 rows of
+// 1024 are 600 vector instructions per wavefront.  EXACT (K = 256 NJ): every piece of a
+// wavefront exists, so there is no branch and one address serves all loads; rows past the
+// end repeat the last row and are never stored, and two values are rounded at a time.
+// 1268 -> 958 instructions at NT = 2, NJ = 4; us, weights from memory, before / so, same
+// tiles: 64 x 1024 x 1024 5.35 / 4.85, 64 x 1024 x 5632 gated 9.92 / 8.64, 64 x 768 x 2304
+// 5.75 / 5.17; of int8 32 x 2048 x 2048 8.94 / 7.93; 64 x 512 x 1536 4.39 / 3.66 (with
+// NJ = 2, before 3).
+template <int NT, int NJ, typename WT, bool EXACT>
 __global__ void __launch_bounds__(256)
 norm_gemm_kernel(GemmArgs g) {
   constexpr int TB = WeightTile<WT>::kTileBytes;
@@ -316,8 +334,7 @@ norm_gemm_kernel(GemmArgs g) {
   const OperandLanes ol(lane);
   const int n16 = ol.ld_row, gq = ol.ld_piece;
   const int KT = g.K >> 5, n_pairs = KT >> 1;
-  const int row = m0 + n16;
-  const bool row_ok = row < g.M;
+  const int row = min(m0 + n16, g.M - 1);  // past the end: not stored
 
   Frag xa[NJ][2];
   typename WeightTile<WT>::Raw wt[NJ][2][NT];
@@ -326,41 +343,39 @@ norm_gemm_kernel(GemmArgs g) {
     // Rows first, then the norm scale, then the weight tiles: loads return in
     // the order they were issued, and the row statistics need only the rows —
     // issued between the weight tiles they would wait for most of those too.
-    const bf16_t* xrow = g.A + (size_t)(row_ok ? row : g.M - 1) * g.K + 8 * gq;
-    const char* wbase = reinterpret_cast<const char*>(g.W);
+    const bf16_t* xrow = g.A + (size_t)row * g.K + 8 * gq + 64 * wave;
+    const bf16_t* scale = g.norm_scale + 64 * wave + 8 * gq;
+    const char* wbase = reinterpret_cast<const char*>(g.W) + (size_t)wave * 2 * TB;
+    // (k-tile of this wavefront's piece hh of step j, less that of its first)
+    auto tile = [&](int j, int hh) {
+      return EXACT ? 8 * j + hh : min(8 * j + hh, KT - 1 - 2 * wave);
+    };
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int kt = min((wave + 4 * j) * 2 + hh, KT - 1);
-        xa[j][hh].u = *reinterpret_cast<const uint4*>(xrow + 32 * kt);
-      }
+      for (int hh = 0; hh < 2; ++hh)
+        xa[j][hh].u = *reinterpret_cast<const uint4*>(xrow + 32 * tile(j, hh));
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int kt = min((wave + 4 * j) * 2 + hh, KT - 1);
-        lnv[j][hh] =
-            *reinterpret_cast<const uint4*>(g.norm_scale + 32 * kt + 8 * gq);
-      }
+      for (int hh = 0; hh < 2; ++hh)
+        lnv[j][hh] = *reinterpret_cast<const uint4*>(scale + 32 * tile(j, hh));
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int kt = min((wave + 4 * j) * 2 + hh, KT - 1);
+      for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
         for (int nn = 0; nn < NT; ++nn)
           wt[j][hh][nn] = WeightTile<WT>::load(
-              wbase + ((size_t)min(nt0 + nn, n_tiles_total - 1) * KT + kt) * TB,
+              wbase + ((ptrdiff_t)min(nt0 + nn, n_tiles_total - 1) * KT + tile(j, hh)) * TB,
               lane);
-      }
   }
   T5D_GATE_TEST();
 
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    if (wave + 4 * j < n_pairs) {
+    if (EXACT || wave + 4 * j < n_pairs) {
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         float f[8];
@@ -382,7 +397,7 @@ norm_gemm_kernel(GemmArgs g) {
   for (int nn = 0; nn < NT; ++nn) acc[nn] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    if (wave + 4 * j < n_pairs) {
+    if (EXACT || wave + 4 * j < n_pairs) {
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         float xf[8], sf[8];
@@ -391,13 +406,12 @@ norm_gemm_kernel(GemmArgs g) {
         uint32_t o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float y0 = round_bf16(xf[2 * e] * inv);
-          const float y1 = round_bf16(xf[2 * e + 1] * inv);
-          o[e] = pack_bf16x2(y0 * sf[2 * e], y1 * sf[2 * e + 1]);
+          const uint32_t y = pack_bf16x2(xf[2 * e] * inv, xf[2 * e + 1] * inv);
+          o[e] = pack_bf16x2(bf16lo_to_f32(y) * sf[2 * e],
+                             bf16hi_to_f32(y) * sf[2 * e + 1]);
         }
         Frag an;
-        an.u = ol.to_operand(row_ok ? make_uint4(o[0], o[1], o[2], o[3])
-                                    : make_uint4(0, 0, 0, 0));
+        an.u = ol.to_operand(make_uint4(o[0], o[1], o[2], o[3]));
 #pragma unroll
         for (int nn = 0; nn < NT; ++nn)
           acc[nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -1515,19 +1529,33 @@ extern "C" int t5d_norm_gemm(void* stream, int dtype, int w_dtype,
     return T5D_OK;
   }
   const int nj = (K / 64 + 3) / 4;  // k-tile pairs per wavefront
-  // 64-column tiles unless that leaves too few workgroups to fill the chip;
-  // beyond K = 1024 the fragments of fewer column tiles fit the registers
-  // (bfloat16 weights: one, int8: two).
-  int nt = (n_tiles / 4) * g.m_parts >= 256 ? 4 : (n_tiles >= 64 ? 2 : 1);
-  if (nj > 4) nt = min(nt, w_dtype == T5D_I8 ? 2 : 1);
+  // One column tile while every workgroup has a CU to itself, else two, or four where
+  // that still fills the chip (more tiles share a normalisation); us for 1 / 2 / 4
+  // tiles, weights from memory: 64 x 1024 x 1024 (256 workgroups of 1) 4.38 / 4.84 /
+  // 5.74, 16 x 768 x 2304 (144) 3.85 / 4.21 / 5.06, 32 x 768 x 2304 (288) 4.69 / 4.24 /
+  // 5.08, 128 x 768 x 768 (384) 4.66 / 4.25 / 5.01, 64 x 1024 x 3072 (768; 192 of 4)
+  // 6.81 / 6.43 / 6.47, 128 x 1024 x 3072 (384 of 4) 10.46 / 8.68 / 7.88.
+  // Beyond K = 1024 the fragments of fewer column tiles fit the registers (bfloat16
+  // weights: one; int8: two, which no second workgroup joins on a CU, so only while
+  // each has its own: K = 2048, int8, 32 x 2048 (256 of 1) 6.18 / 7.70, 64 x 2048 (256
+  // of 2) 8.08 / 7.73, 32 x 6144 (384 of 2) 11.9 / 14.8, 16 x 6144 (192) 8.89 / 8.80).
+  const int tiles = n_tiles * g.m_parts;
+  int nt = tiles <= 256 ? 1 : ((n_tiles / 4) * g.m_parts >= 256 ? 4 : 2);
+  if (nj > 4) nt = w_dtype == T5D_I8 && tiles > 256 && tiles <= 512 ? 2 : 1;
   const int n_groups = (n_tiles + nt - 1) / nt;
   dim3 grid((n_groups + 7) / 8 * 8 * g.m_parts), block(256);
-#define T5D_NG_LAUNCH(NT_, NJ_, WT_)                                          \
-  hipLaunchKernelGGL((norm_gemm_kernel<NT_, NJ_, WT_>), grid, block, 0, s, g)
+#define T5D_NG_LAUNCH(NT_, NJ_, WT_)                                            \
+  do {                                                                          \
+    if (K == 256 * NJ_)                                                         \
+      hipLaunchKernelGGL((norm_gemm_kernel<NT_, NJ_, WT_, true>), grid, block, 0, s, g); \
+    else                                                                        \
+      hipLaunchKernelGGL((norm_gemm_kernel<NT_, NJ_, WT_, false>), grid, block, 0, s, g); \
+  } while (0)
 #define T5D_NG_CASE(NT_, WT_)                                                 \
   if (nt == NT_) {                                                            \
-    if (nj <= 3) T5D_NG_LAUNCH(NT_, 3, WT_);                                  \
-    else if (nj <= 4) T5D_NG_LAUNCH(NT_, 4, WT_);                             \
+    if (nj <= 2) T5D_NG_LAUNCH(NT_, 2, WT_);                                    \
+    else if (nj <= 3) T5D_NG_LAUNCH(NT_, 3, WT_);                               \
+    else if (nj <= 4) T5D_NG_LAUNCH(NT_, 4, WT_);                               \
   }
   if (w_dtype == T5D_BF16) {
     if (nj > 4) T5D_NG_LAUNCH(1, 8, bf16_t);

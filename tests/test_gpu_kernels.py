@@ -1491,6 +1491,23 @@ def test_norm_gemm_random_shapes(ops):
     assert float((err > 0).float().mean()) < 0.2, (case, M, K, N)
 
 
+@pytest.mark.parametrize('K', [64, 192, 256, 448, 512, 768, 960, 1024, 2048])
+@pytest.mark.parametrize('N', [16, 528, 2064])
+@pytest.mark.parametrize('int8', [False, True])
+def test_norm_gemm_does_not_depend_on_its_tiles(ops, K, N, int8):
+  """Every row's result is the same whichever tile it falls into: 128 rows (four or
+  two column tiles per workgroup), 33 of them and single rows (one), bit for bit."""
+  rs = np.random.RandomState(K + N)
+  x = dev(rs.randn(128, K).astype(np.float32), torch.bfloat16)
+  scale = dev((1 + 0.1 * rs.randn(K)).astype(np.float32), torch.bfloat16)
+  pw = ops.pack_weight(dev((rs.randn(K, N) / np.sqrt(K)).astype(np.float32)),
+                       torch.bfloat16, torch.int8 if int8 else torch.bfloat16)
+  want = ops.gemm(x, pw, norm_scale=scale)
+  for a, b in ((0, 33), (40, 41), (111, 128)):
+    got = ops.gemm(x[a:b].contiguous(), pw, norm_scale=scale)
+    assert torch.equal(got, want[a:b]), (a, b)
+
+
 def test_cross_attention_random_shapes(ops):
   """t5d_cross_attention_step (bfloat16) over 40 random shapes — batch 1..48,
   1 / 2 / 4 / 8 beams, 1..16 heads, encoder length a multiple of 32 up to
