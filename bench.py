@@ -682,14 +682,16 @@ class EncoderStage:
       self.module._cross_kv(self.weights, encoded, self.tokens, self.K)
 
   def flops(self):
-    """Dense-equivalent multiply-adds x 2 of one pass (padding included)."""
+    """Multiply-adds x 2 of one pass, of what is computed: the encoder over every
+    text and one row for its padding, the projection over all positions."""
     c = self.cfg
     M, d, F = self.B * self.E, c.emb_dim, c.mlp_dim
     hd = c.num_heads * c.head_dim
-    enc = c.num_encoder_layers * (2 * M * d * (3 * hd) + 2 * M * hd * d +
-                                  2 * M * d * 2 * F + 2 * M * F * d +
-                                  4 * self.B * c.num_heads * self.E * self.E *
-                                  c.head_dim)
+    rows = [int(n) + (n < self.E) for n in self.lens]
+    R, pairs = sum(rows), sum(r * int(n) for r, n in zip(rows, self.lens))
+    enc = c.num_encoder_layers * (2 * R * d * (3 * hd) + 2 * R * hd * d +
+                                  2 * R * d * 2 * F + 2 * R * F * d +
+                                  4 * c.num_heads * pairs * c.head_dim)
     cross = c.num_decoder_layers * 2 * (2 * M * d * hd)
     return enc + cross
 
