@@ -346,7 +346,9 @@ int t5d_encoder_rows(void* stream, const int64_t* tokens, int B, int E, int32_t*
                      int32_t* at, int32_t* summary);
 
 /* t5d_encoder_attention over the rows that t5d_encoder_rows lists: q, k and out hold
- * first[B] rows; most: rows of the longest text (summary[1]). */
+ * first[B] rows; most: rows of the longest text (summary[1]); E: the positions that a
+ * text has and that a padded query weighs, at least the E of t5d_encoder_rows and at
+ * most that rounded up to a multiple of 4. */
 int t5d_encoder_attention_rows(void* stream, const void* q, const void* k,
                                const void* v_t, const void* rel_bias,
                                const int32_t* enc_len, const int32_t* first, int most,

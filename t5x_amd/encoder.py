@@ -60,9 +60,9 @@ def _encode_rows(cfg, w, rows, device):
   """_encode_hip over the rows that there are (ops.EncoderRows)."""
   from t5x_amd import ops
   HD = cfg.num_heads * 64
-  bias = w.rel_bias(rows.E)
+  bias = w.rel_bias(rows.positions)
   x = ops.embed(w.embedding, rows.ids)
-  v_t = torch.zeros((rows.B, cfg.num_heads, (rows.E + 31) // 32, 64, 32),
+  v_t = torch.zeros((rows.B, cfg.num_heads, (rows.positions + 31) // 32, 64, 32),
                     dtype=x.dtype, device=device)
   for l in w.layers:
     xn = ops.rmsnorm(x, l['ln_attn'])
@@ -204,6 +204,10 @@ def _encode_hip_f32(module, params, tokens):
 
 
 def encode(module, params, encoder_input_tokens):
+  """[B, E, emb_dim] of tokens [B, E].  In bfloat16 a text has E rounded up to a
+  multiple of 4 positions: tokens do not see the added ones, the padding behind them
+  does, whose queries weigh all positions alike (the reference's E, network.py:325-328;
+  nothing downstream looks at padding's rows)."""
   cfg, dev = module.config, module._dev()
   tokens = encoder_input_tokens
   if not isinstance(tokens, torch.Tensor):

@@ -521,8 +521,8 @@ def gemm_rows_values(a, w: PackedWeight, rows, out):
     raise ValueError(f'a is [{M}, {K}], out {tuple(out.shape)}: {rows.M} rows, '
                      f'kernel K={w.K} N={w.N}')
   _lib.call('t5d_gemm_rows_values', _s(), w.w_dtype, a.data_ptr(), w.data.data_ptr(),
-            _lib.ptr(w.scales), out.data_ptr(), M, K, w.N, rows.at.data_ptr(), rows.E,
-            Ep)
+            _lib.ptr(w.scales), out.data_ptr(), M, K, w.N, rows.at.data_ptr(),
+            rows.positions, Ep)
   return out
 
 
@@ -531,14 +531,16 @@ MAX_ENCODER_LENGTH = 2048  # positions of a text (kMaxEncLen)
 
 class EncoderRows:
   """The rows an encoder computes for tokens [B, E] (t5d_encoder_rows): those of
-  every text and one that stands for its padding.  `odd`: a text is something else
-  than tokens > 0 followed by zeros, and only `len` (the number of tokens > 0) holds.
-  Waits for the device once, to learn how many rows there are."""
+  every text and one that stands for its padding.  A text has `positions`: E rounded
+  up to a multiple of 4 with padding, which a padded query weighs as well (as it does
+  where every position is computed, see encoder.encode).  `odd`: a text is something
+  else than tokens > 0 followed by zeros, and only `len` (the number of tokens > 0)
+  holds.  Waits for the device once, to learn how many rows there are."""
 
   def __init__(self, tokens):
     _chk(tokens, 'tokens', torch.int64, 2)
     self.B, self.E = B, E = tokens.shape
-    E4 = (E + 3) // 4 * 4
+    self.positions = E4 = (E + 3) // 4 * 4
     sizes = [B, B, B + 1, B * E4, B * E, B * E4 // 4, 3]
     (self.len, odd, self.first, self._ids, self.row_of, self._at,
      summary) = torch.empty(sum(sizes), dtype=torch.int32,
@@ -614,8 +616,9 @@ def encoder_attention_rows(q, k, v_t, rel_bias, rows):
   _chk(rel_bias, 'rel_bias', torch.bfloat16, 2)
   B, H, blocks, D, w = v_t.shape
   if ((B, D, w) != (rows.B, 64, 32) or
-      tuple(rel_bias.shape) != (H, 2 * rows.E - 1)):
-    raise ValueError('v_t [B, H, Ep/32, 64, 32], rel_bias [H, 2E-1]')
+      tuple(rel_bias.shape) != (H, 2 * rows.positions - 1)):
+    raise ValueError('v_t [B, H, Ep/32, 64, 32], rel_bias [H, 2E-1], E the positions '
+                     'of a text')
   for name, t in (('q', q), ('k', k)):
     if (not t.is_cuda or t.dtype != torch.bfloat16 or t.dim() != 2 or
         t.stride(1) != 1 or tuple(t.shape) != (rows.M, H * 64)):
@@ -624,8 +627,8 @@ def encoder_attention_rows(q, k, v_t, rel_bias, rows):
   out = torch.empty((rows.M, H * 64), dtype=torch.bfloat16, device=v_t.device)
   _lib.call('t5d_encoder_attention_rows', _s(), q.data_ptr(), k.data_ptr(),
             v_t.data_ptr(), rel_bias.data_ptr(), rows.len.data_ptr(),
-            rows.first.data_ptr(), rows.most, out.data_ptr(), B, H, rows.E, blocks * 32,
-            q.stride(0), k.stride(0))
+            rows.first.data_ptr(), rows.most, out.data_ptr(), B, H, rows.positions,
+            blocks * 32, q.stride(0), k.stride(0))
   return out
 
 
