@@ -1282,26 +1282,30 @@ sample_tokens_fast_kernel(SampleArgs a) {
         const int slot = a.noise_step ? *a.noise_step % a.noise_ring : 0;
         Cand best = {-INFINITY, 0x7FFFFFFF};
         if (kept) {
-          best.v = v + a.gumbel[((size_t)slot * a.R + r) * V + j];
-          best.i = j;
+          const float noisy = v + a.gumbel[((size_t)slot * a.R + r) * V + j];
+          if (noisy > best.v) { best.v = noisy; best.i = j; }  // (no NaN)
         }
         best = block_best(best, cscratch);
-        double sum = kept ? (double)expf(v - mx) : 0.0;
-        sum = block_sum_f64(sum, dscratch);
-        __syncthreads();
-        if (kept && j == best.i) fscratch[0] = v;  // one thread holds the token
-        __syncthreads();
-        if (tid == 0) {
-          a.tokens[r] = best.i;
-          if (a.rescale) {
-            a.logprobs[r] = (fscratch[0] - mx) - (float)log(sum);
-          } else {
-            const RowSum row = sample_row_sum(a.parts, a.R, r);
-            a.logprobs[r] = (a.logits[(size_t)r * V + best.i] - row.top) -
-                            (float)log(row.sum);
+        // Noise that leaves no kept value above the masked ones (NaN, -infinity): the
+        // whole row is to be looked at, and best.i may be no place of it.
+        if (best.v > kNegInf + 1000.f) {
+          double sum = kept ? (double)expf(v - mx) : 0.0;
+          sum = block_sum_f64(sum, dscratch);
+          __syncthreads();
+          if (kept && j == best.i) fscratch[0] = v;  // one thread holds the token
+          __syncthreads();
+          if (tid == 0) {
+            a.tokens[r] = best.i;
+            if (a.rescale) {
+              a.logprobs[r] = (fscratch[0] - mx) - (float)log(sum);
+            } else {
+              const RowSum row = sample_row_sum(a.parts, a.R, r);
+              a.logprobs[r] = (a.logits[(size_t)r * V + best.i] - row.top) -
+                              (float)log(row.sum);
+            }
           }
+          return;
         }
-        return;
       }
       __syncthreads();  // (everyone has read what the path below reuses)
     }

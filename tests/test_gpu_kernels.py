@@ -1373,6 +1373,30 @@ def test_sample_tokens_by_parts_of_rows(ops, R, V, rescale, k):
     np.testing.assert_allclose(host(lp)[plain], exact, rtol=2e-6)
 
 
+@pytest.mark.parametrize('rescale', [True, False])
+@pytest.mark.parametrize('V,k', [(4096, 8), (32128, 64)])
+def test_sample_tokens_by_parts_with_noise_that_is_not_finite(ops, V, k, rescale):
+  """Noise of the kept values that is NaN or -infinity, for all of them and for all but
+  one, beside a value of +infinity too: what is chosen is a place of the row, the same
+  one as in one launch, with its log-prob."""
+  rs = np.random.RandomState(V)
+  R = 6
+  logits = (2 * rs.randn(R, V)).astype(np.float32)
+  g = odec.GumbelNoise(seed=k).noise(0, (R, V)).astype(np.float32).copy()
+  for r, value in enumerate([np.nan, -np.inf, np.nan, -np.inf, -np.inf]):
+    kept = np.argsort(-logits[r])[:k]
+    g[r, kept[1:] if r in (2, 3) else kept] = value
+  logits[4, np.argmax(logits[4])] = np.inf
+  args = (dev(logits), dev(g), dev(np.full((R,), 0.7, np.float32)), k, 0.0, rescale)
+  tok, lp = ops.sample_tokens(*args, workspace=ops.sample_tokens_workspace(R, 'cuda'))
+  tok1, lp1 = ops.sample_tokens(*args)
+  assert (host(tok) >= 0).all() and (host(tok) < V).all()
+  np.testing.assert_array_equal(host(tok), host(tok1))
+  np.testing.assert_allclose(host(lp), host(lp1), atol=2e-6, rtol=2e-6)
+  for r in (2, 3):
+    assert host(tok)[r] == np.argmax(logits[r])
+
+
 def test_sample_tokens_topp_table(ops):
   # t5x/binary_search_test.py:143-209 through the kernel: with a huge Gumbel
   # bonus on one index the sampled token reveals whether it survived the mask.
