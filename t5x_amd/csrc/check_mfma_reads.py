@@ -14,8 +14,8 @@ and fails when any path from a v_mfma / v_smfmac to a reader of its
 destination is shorter than NEED slots (9: what the compiler itself pads
 straight-line code to for the 16x16x32 instructions used here).
 
-A second check, for the kernels that fill LDS with global_load_lds behind
-hand-placed barriers: a barrier orders instructions that have been issued,
+A second check, for the kernels that fill LDS straight from memory (global_load_lds,
+buffer_load ... lds) behind hand-placed barriers: a barrier orders instructions that have been issued,
 not LDS reads that have completed, and the compiler may sink a k-tile's last
 operand reads below the next barrier; a faster wavefront could then refill
 the stage while those reads were still queued (seen as a wrong 16-row slice
@@ -117,13 +117,21 @@ def short_reads(text, need=NEED):
   return found, hist
 
 
+def kernels_that_load_into_lds(text):
+  """Kernels with loads from memory whose destination is LDS: global_load_lds_*, and
+  buffer loads with the modifier lds."""
+  return {k for k, t in parse(text)[0]
+          if t.startswith('global_load_lds') or
+          (t.startswith('buffer_load') and 'lds' in t.split())}
+
+
 def unguarded_barriers(text, depth=96):
   """-> [(kernel, index of the barrier among the kernel's barriers)] for
-  kernels that use global_load_lds: barriers that an LDS read can reach
+  kernels that load into LDS (kernels_that_load_into_lds): barriers that an LDS read can reach
   without a wait for lgkmcnt(0) in between, on any path (walking backwards
   from the barrier, over branches too, until such a wait ends the path)."""
   ins, labels = parse(text)
-  uses_dma = {k for k, t in ins if t.startswith('global_load_lds')}
+  uses_dma = kernels_that_load_into_lds(text)
   if not uses_dma:
     return []
   preds = collections.defaultdict(list)
@@ -160,12 +168,13 @@ def unguarded_barriers(text, depth=96):
 
 
 def main(paths):
-  bad = barriers = 0
+  bad = barriers = loading = 0
   total = collections.Counter()
   for path in paths:
     with open(path) as f:
       text = f.read()
     found, hist = short_reads(text)
+    loading += len(kernels_that_load_into_lds(text))
     for kernel, nth in unguarded_barriers(text):
       barriers += 1
       print(f'{path}: {kernel}: barrier {nth} of a kernel that loads into LDS '
@@ -178,7 +187,8 @@ def main(paths):
             f'(need {NEED})')
   print(f'check_mfma_reads: {sum(total.values())} reads of matrix results in '
         f'{len(paths)} files, shortest {min(total) if total else "-"} slots, '
-        f'{bad} too early; {barriers} unguarded barriers')
+        f'{bad} too early; {barriers} unguarded barriers in {loading} kernels that '
+        'load into LDS')
   return 1 if bad or barriers else 0
 
 

@@ -122,6 +122,10 @@ _Z6kernelv:
 	s_endpgm
 """
 
+# the same loads in the other form, and one that looks like it
+_BUFFER = 'buffer_load_dwordx4 v9, s[16:19], s5 offen lds'
+_BUFFER_NOT_INTO_LDS = 'buffer_load_dwordx4 v[4:7], v9, s[16:19], s5 offen'
+
 _NO_DMA = """
 _Z6kernelv:
 	ds_read_b128 v[0:3], v8
@@ -135,6 +139,12 @@ def test_barriers_of_kernels_that_load_into_lds_need_a_wait_for_lds_reads():
   assert mod.unguarded_barriers(_RING_GUARDED) == []
   assert mod.unguarded_barriers(_RING_SUNK_READ) == [('_Z6kernelv', 1)]
   assert mod.unguarded_barriers(_NO_DMA) == []   # other kernels: not checked
+  load = 'global_load_lds_dwordx4 v[4:5], off'
+  assert mod.unguarded_barriers(_RING_GUARDED.replace(load, _BUFFER)) == []
+  assert mod.unguarded_barriers(_RING_SUNK_READ.replace(load, _BUFFER)) == [
+      ('_Z6kernelv', 1)]
+  assert mod.unguarded_barriers(
+      _RING_SUNK_READ.replace(load, _BUFFER_NOT_INTO_LDS)) == []
 
 
 def test_built_kernels_have_no_early_read():
@@ -144,6 +154,13 @@ def test_built_kernels_have_no_early_read():
   mod = _checker()
   for path in files:
     with open(path) as f:
-      found, _ = mod.short_reads(f.read())
+      text = f.read()
+    found, _ = mod.short_reads(text)
     assert found == [], (path, found[:3])
-    assert mod.unguarded_barriers(open(path).read()) == [], path
+    assert mod.unguarded_barriers(text) == [], path
+    # every kernel that the sources give such loads is among those checked
+    name = os.path.basename(path)[:-2]
+    with open(os.path.join(CSRC, name + '.hip')) as f:
+      source = f.read()
+    if 'load_lds(' in source:
+      assert mod.kernels_that_load_into_lds(text), path
