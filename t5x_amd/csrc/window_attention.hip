@@ -614,12 +614,13 @@ window_step_kernel(WinArgs g) {
           vt + (size_t)(u * KPI + vsub) * HP + 8 * vpiece);
   };
 
-  // The queries -> LDS, the new key and value -> ring (every part writes the same bytes
-  // there) and LDS.  (Rows GS .. 15 of the query tile are whatever is there: columns of
-  // the products that nothing looks at.)  All of a wavefront's
-  // vectors and its first tile are requested before the first is looked at; the tile that
-  // holds the new row's place does not wait for the ring: it gets the new key, and the
-  // new value is added at the end.
+  // The queries, the new key and value -> LDS.  (Rows GS .. 15 of the query tile are
+  // whatever is there: columns of the products that nothing looks at.)  All of a
+  // wavefront's vectors and its first tile are requested before the first is looked at;
+  // the tile that holds the new row's place does not wait for the ring: it gets the new
+  // key, and the new value is added at the end.  The ring takes both from the one
+  // wavefront that has this tile, when it is done with it: what the tile read there,
+  // weighed by zero, is what the ring held before and nothing that is just being written.
   // One row of 8 heads over 2 with a window of 1024: 15.5 us one after the other and the
   // tile behind the barrier, 13.1 with the tile of the new row only behind it, 11.0 so
   // and with a third fewer instructions; with the kernel that merges the parts, for 1 x
@@ -645,10 +646,7 @@ window_step_kernel(WinArgs g) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int d = lane + 64 * u;
-        const bf16_t x = f32_to_bf16(f[u] * inv * scale[v][u]);
-        if (d < HP) dst[d] = x;
-        if (d < HP && vec >= GS)
-          ((vec == GS ? K : V) + (size_t)(i % a.ring) * HP)[d] = x;
+        if (d < HP) dst[d] = f32_to_bf16(f[u] * inv * scale[v][u]);
       }
     }
   }
@@ -666,6 +664,7 @@ window_step_kernel(WinArgs g) {
   const float slope2 = a.slopes != nullptr ? a.slopes[head] * kLog2e : 0.f;
   float mx = kNoMax, l = 0.f;
   float acc[GS][8], w_new[GS];
+  bool holds_new = false;  // this wavefront's last tile is the new row's
 #pragma unroll
   for (int h = 0; h < GS; ++h) {
     w_new[h] = 0.f;
@@ -720,6 +719,7 @@ window_step_kernel(WinArgs g) {
     if (gq == 0) s_alpha[wave][n16] = alpha;
     wave_lds_fence();
     if (jt + 63 >= i) {  // the new value is added at the end (this is the last tile)
+      holds_new = true;
       float* w = &s_w[wave][(i - jt) * GS];
 #pragma unroll
       for (int h = 0; h < GS; ++h) w_new[h] = w[h];
@@ -755,7 +755,13 @@ window_step_kernel(WinArgs g) {
       }
     }
   }
-  if (vsub == 0) {
+  if (holds_new && lane < 2 * LPR)
+    *reinterpret_cast<uint4*>((lane < LPR ? K : V) + (size_t)(i % a.ring) * HP +
+                              8 * vpiece) =
+        *reinterpret_cast<const uint4*>(s_new[lane < LPR ? 0 : 1] + 8 * vpiece);
+  // (the new value, by the wavefront that has its weight alone: it may be infinite, and
+  // nothing times that is not nothing)
+  if (holds_new && vsub == 0) {
     float f[8];
     unpack16(*reinterpret_cast<const uint4*>(s_new[1] + 8 * vpiece), f);
 #pragma unroll

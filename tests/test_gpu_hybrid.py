@@ -328,6 +328,24 @@ def test_window_attention_step_in_parts(H, G, D, Dv, window):
         assert rel(row, want[starts[s] + step]) < 1e-2, (step, s)
 
 
+@pytest.mark.parametrize('H,G,D,Dv', [(4, 1, 128, 128), (2, 2, 40, 64), (2, 1, 200, 256)])
+@pytest.mark.parametrize('pos', [3, 700])
+def test_window_attention_step_with_an_infinite_value(H, G, D, Dv, pos):
+  """A new value of +-infinity reaches its column of the output as that, the others not
+  at all, whichever wavefront and workgroup has the new row."""
+  a = Attention(torch.bfloat16, H, G, D, Dv, 0, 1, 8, 1024)
+  x = a.sequence(pos + 1)
+  want = a.oracle(x).reshape(pos + 1, H, Dv)[pos]
+  x[pos, a.off[2]], x[pos, a.off[2] + 5] = np.inf, -np.inf
+  for s in range(0, pos, 200):
+    a.run([(0, s)], [x[s:min(pos, s + 200)]])
+  got = a.run([(0, pos)], [x[pos:]], variant=1).reshape(H, Dv)
+  first = got[:H // G]  # the heads of the first key / value head
+  assert (first[:, 0] == np.inf).all() and (first[:, 5] == -np.inf).all()
+  first[:, [0, 5]] = want[:H // G, [0, 5]]
+  assert rel(got, want) < 1e-2
+
+
 @pytest.mark.parametrize('H,G,D,scale,bias', [
     (4, 2, 128, 0.3, False), (4, 2, 64, 0.3, True), (2, 2, 32, -0.4, False),
     (2, 1, 200, 0.0, False)])
