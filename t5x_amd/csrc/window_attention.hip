@@ -723,9 +723,9 @@ window_step_kernel(WinArgs g) {
       float* w = &s_w[wave][(i - jt) * GS];
 #pragma unroll
       for (int h = 0; h < GS; ++h) w_new[h] = w[h];
-      wave_lds_fence();
+      asm volatile("" ::: "memory");  // (an order for the compiler; no wait, see above)
       if (lane < GS) w[lane] = 0.f;
-      wave_lds_fence();
+      asm volatile("" ::: "memory");
     }
 #pragma unroll
     for (int h = 0; h < GS; ++h) {
@@ -882,9 +882,12 @@ static int step_splits(const t5d_window_attention& a, int S) {
   const int span = a.window > 0 ? min(a.window, a.ring) : a.ring;
   int n = 1;
   while (n < kMaxSplits && S * a.G * n < 256 && span >= 512 * n) n *= 2;
-  // one tile of 64 positions per wavefront while CUs are left: a window of 1024 touches
-  // 17 tiles, the last of which made one of 16 wavefronts walk two
-  while (n < kMaxSplits && 4 * n < span / 64 + 1 && S * a.G * (n + 1) <= 256) ++n;
+  // Where there are parts to be merged anyhow: one tile of 64 positions per wavefront
+  // while CUs are left.  A window of 1024 touches 17 tiles, the last of which made one of
+  // 16 wavefronts walk two.  (Two parts for the fifth tile of a window of 256, 1 row of 8
+  // heads over 2: 11.1 us as one part does, over 100 positions 10.3 against 8.1; 64 rows
+  // 13.5 against 12.7.)
+  while (n > 1 && n < kMaxSplits && 4 * n < span / 64 + 1 && S * a.G * (n + 1) <= 256) ++n;
   return n;
 }
 
