@@ -538,8 +538,11 @@ __device__ __forceinline__ void wave_lds_fence() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
+// (Heads of 129 to 256, a key head per query head: 268 registers as the compiler would
+// have it, 250 and a second workgroup per CU when asked to.  us, 268 / 250: 128 rows of 4
+// heads of 256, window 512 61.2 / 56.3; 64 of 8 heads of 200, window 1024 105 / 101.)
 template <int DT, int GS>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, DT == 8 && GS == 1 ? 2 : 1)
 window_step_kernel(WinArgs g) {
   constexpr int HP = DT * 32;
   constexpr int QS = HP + 8;
