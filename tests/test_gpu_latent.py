@@ -28,10 +28,13 @@ def tol(dt):
 
 @pytest.mark.parametrize('M,E,top,skew', [(1, 3, 1, False), (37, 5, 2, False),
                                           (300, 4, 3, False), (700, 40, 4, False),
-                                          (90, 7, 1, True), (2000, 3, 2, False)])
+                                          (90, 7, 1, True), (2000, 3, 2, False),
+                                          (4096, 5, 2, False), (2731, 3, 3, False),
+                                          (5000, 6, 5, False)])
 @pytest.mark.parametrize('dt', DTYPES)
 def test_experts_by_table(dt, M, E, top, skew):
-  """Every tile height; experts without tokens and one with all of them."""
+  """Every tile height; experts without tokens and one with all of them; entries that
+  fill whole rounds of 8192, one more, and several rounds and a rest."""
   from t5x_amd import ops
   rs = np.random.RandomState(M)
   V, K, F, N = 50, 96, 64, 128
