@@ -1208,11 +1208,14 @@ extern "C" int t5d_gemm(void* stream, int dtype, int w_dtype, int out_dtype,
 // 41.7 / 31.3, 57.6 / 35.3.  Beyond 64 rows K = 1024, N = 20000 (157 tiles): 96 rows
 // 20.0 / 18.4; N = 16384 (128): 96 rows 16.2 / 16.9.  With its sums not yet folded, so at
 // its fastest, it lost at 16 rows (K = 768, N = 32128: 12.2 / 13.4) and with few tiles
-// (K = 1024, N = 8000, 64 rows: 9.8 / 13.1).  K and lda: what the offsets of that kernel
-// reach.
+// (K = 1024, N = 8000, 64 rows: 9.8 / 13.1).  Beyond K = 2048 up to 32 rows take it only
+// where every CU has more than one tile: with one, its steps of K follow one another
+// alone, and the others win (N = 32128, 28 rows: K = 2560 35.5 / 37.2, 4096 52.4 / 58.4,
+// 8192 103 / 112; 32 rows, 8192: 107 / 114; N = 50000, 25 rows, 4096: 94 / 83; 33
+// rows, N = 32128, 4096: 68.9 / 58.1).  K and lda: what the offsets of that kernel reach.
 static bool many_columns(int M, int K, int N, int lda) {
-  return M > 24 && N >= 128 * (M > 64 ? 150 : 240) && K >= 64 &&
-         K < (1 << 22) && lda < (1 << 22);
+  const int least = M > 64 ? 150 : K > 2048 && M <= 32 ? 390 : 240;
+  return M > 24 && N >= 128 * least && K >= 64 && K < (1 << 22) && lda < (1 << 22);
 }
 
 extern "C" int t5d_dense(void* stream, int dtype, int out_dtype, const void* A,

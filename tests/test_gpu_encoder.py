@@ -231,6 +231,12 @@ def test_dense_of_many_columns(ops, M, N, K):
     assert bool(((got.double() - want[:, :n_store]).abs() <= bound[:, :n_store]).all())
 
 
+@pytest.mark.parametrize('M,N', [(25, 30720), (32, 49904), (32, 49920), (33, 30720)])
+def test_dense_of_many_columns_over_a_long_k(ops, M, N):
+  """The line lies elsewhere for up to 32 rows of more than 2048."""
+  test_dense_of_many_columns(ops, M, N, 2080)
+
+
 @pytest.mark.parametrize('K', [64, 96, 192, 224, 256, 320])
 @pytest.mark.parametrize('M', [130, 4200])  # tiles of 64 rows, of 128
 def test_gemm_rows_of_int8_weights_over_the_ends_of_k(ops, K, M):
