@@ -1212,10 +1212,12 @@ extern "C" int t5d_gemm(void* stream, int dtype, int w_dtype, int out_dtype,
 // where every CU has more than one tile: with one, its steps of K follow one another
 // alone, and the others win (N = 32128, 28 rows: K = 2560 35.5 / 37.2, 4096 52.4 / 58.4,
 // 8192 103 / 112; 32 rows, 8192: 107 / 114; N = 50000, 25 rows, 4096: 94 / 83; 33
-// rows, N = 32128, 4096: 68.9 / 58.1).  K and lda: what the offsets of that kernel reach.
+// rows, N = 32128, 4096: 68.9 / 58.1).  Below K = 512 the folds are so few that the sums
+// lie further off (from float64, K = 96: 4.67e-8 / 5.2e-8, 256: 5.7e-8 / 5.9e-8, 512:
+// 7.1e-8 / 6.9e-8).  K and lda: what the offsets of that kernel reach.
 static bool many_columns(int M, int K, int N, int lda) {
   const int least = M > 64 ? 150 : K > 2048 && M <= 32 ? 390 : 240;
-  return M > 24 && N >= 128 * least && K >= 64 && K < (1 << 22) && lda < (1 << 22);
+  return M > 24 && N >= 128 * least && K >= 512 && K < (1 << 22) && lda < (1 << 22);
 }
 
 extern "C" int t5d_dense(void* stream, int dtype, int out_dtype, const void* A,

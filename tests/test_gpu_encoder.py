@@ -214,7 +214,7 @@ def test_gemm_rows_of_every_tile_over_the_ends_of_k(ops, K, tile):
 
 @pytest.mark.parametrize('M,N', [(24, 30720), (25, 30720), (64, 30736), (65, 19216),
                                  (128, 19200), (128, 19184)])
-@pytest.mark.parametrize('K', [32, 64, 96, 320, 768])
+@pytest.mark.parametrize('K', [32, 64, 96, 320, 480, 512, 544, 576, 608, 640, 768])
 def test_dense_of_many_columns(ops, M, N, K):
   """float32 results of few rows at both sides of the line to the many-row kernel: no
   further off than sums of 64 products added up one after the other (2^-24 of the
@@ -229,6 +229,19 @@ def test_dense_of_many_columns(ops, M, N, K):
     got = ops.dense(a, pw, out_dtype=torch.float32, n_store=n_store)
     assert got.shape == (M, n_store)
     assert bool(((got.double() - want[:, :n_store]).abs() <= bound[:, :n_store]).all())
+
+
+@pytest.mark.parametrize('K', [96, 256, 480])
+def test_dense_of_many_columns_over_a_short_k(ops, K):
+  """No further off than products added up in the order of the kernels for few rows: K
+  over four wavefronts, one sum each (64 x 32128: the same bits as for 16 rows)."""
+  rs = np.random.RandomState(K)
+  a = dev(rs.randn(64, K).astype(np.float32), torch.bfloat16)
+  pw = ops.pack_weight(dev(rs.randn(K, 32128).astype(np.float32)), torch.bfloat16)
+  got = ops.dense(a, pw, out_dtype=torch.float32)
+  for at in range(0, 64, 16):
+    part = ops.dense(a[at:at + 16].contiguous(), pw, out_dtype=torch.float32)
+    assert torch.equal(got[at:at + 16], part)
 
 
 @pytest.mark.parametrize('M,N', [(25, 30720), (32, 49904), (32, 49920), (33, 30720)])
