@@ -79,8 +79,13 @@ gemm_mfma_kernel(Args g) {
   const char* wbase = reinterpret_cast<const char*>(g.W);
   constexpr int TB = WeightTile<WT>::kTileBytes;
 
-  // (NJ > 0: where this wavefront's first tiles lie; the others follow at constant
-  // distances, which the loads take as offsets)
+  // (NJ > 0 and NT = 4: where this wavefront's first tiles lie; the others follow at
+  // constant distances, which the loads take as offsets.  With fewer column tiles the
+  // addresses are formed where they are used, between the products: us, constant
+  // distances / so, residual layers: bfloat16 64 x 2048 x 2048 6.8 / 6.5, 128 x 2048 x
+  // 2048 9.9 / 9.4, 128 x 5120 x 2048 20.7 / 20.1; int8 64 x 2048 x 2048 5.6 / 5.4; but
+  // int8 128 x 2048 x 4208, of four tiles, 13.5 / 14.1.)
+  constexpr bool kConstant = NJ > 0 && NT == 4;
   const char* w_first = wbase + (size_t)wave * 2 * TB;
   const bf16_t* a_first[MP];
 #pragma unroll
@@ -96,11 +101,15 @@ gemm_mfma_kernel(Args g) {
 #pragma unroll
       for (int nn = 0; nn < NT; ++nn) {
         const int nt = nt0 + nn;
-        if (NJ > 0)  // every k-tile exists; tiles past the edge are never stored
+        // (NJ > 0: every k-tile exists; tiles past the edge are never stored)
+        if (kConstant)
           bq[slot_][h][nn] = WeightTile<WT>::load(
               w_first + (size_t)min(nt, n_tiles_total - 1) * KT * TB +
                   (8 * j + h) * TB,
               lane);
+        else if (NJ > 0)
+          bq[slot_][h][nn] = WeightTile<WT>::load(
+              wbase + ((size_t)min(nt, n_tiles_total - 1) * KT + kt + h) * TB, lane);
         else if (nt < n_tiles_total && kt + h < KT)
           bq[slot_][h][nn] = WeightTile<WT>::load(
               wbase + ((size_t)nt * KT + kt + h) * TB, lane);
@@ -142,9 +151,12 @@ gemm_mfma_kernel(Args g) {
           continue;
         }
         const int row = m0 + mt * 16 + arow;
-        if (NJ > 0)
+        if (kConstant)
           aq[slot_][h][mt] =
               *reinterpret_cast<const uint4*>(a_first[mt] + 256 * j + 32 * h);
+        else if (NJ > 0)
+          aq[slot_][h][mt] = *reinterpret_cast<const uint4*>(
+              g.A + (size_t)min(row, g.M - 1) * row_stride(g) + (kt + h) * 32 + akoff);
         else if (row < g.M && kt + h < KT)
           aq[slot_][h][mt] = *reinterpret_cast<const uint4*>(
               g.A + (size_t)row * row_stride(g) + (kt + h) * 32 + akoff);
