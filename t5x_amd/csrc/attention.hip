@@ -249,7 +249,8 @@ self_attn_f32_kernel(AttnArgs a) {
 // and with probabilities read from LDS 16 positions at a time, the first wavefront's
 // requests in front of the length while workgroups are few, before / now: 8 items, 6
 // heads, 64 positions 5.7 / 3.85, 16 x 6 x 256 (100 valid) 7.0 / 5.2, 16 x 6 x 48 5.4 /
-// 3.8, 64 x 12 x 64 (10 valid) 4.8 / 4.5, 64 x 12 x 256 (40 valid) 9.0 / 7.6.
+// 3.8, 64 x 12 x 64 (10 valid) 4.8 / 4.5, 64 x 12 x 256 (40 valid) 9.0 / 7.6.  What it
+// costs: 8 x 6 x 64 with 5 valid 3.7 / 4.2, 128 x 12 x 256, all valid, 36.1 / 37.7.
 template <int NQ, int WM>
 __global__ void __launch_bounds__(64 * WM)
 cross_attn_f32_kernel(AttnArgs a) {
@@ -276,16 +277,27 @@ cross_attn_f32_kernel(AttnArgs a) {
 #pragma unroll
     for (int c = 0; c < kD / 4; ++c) key[c] = row[c];
   };
+  constexpr bool kAhead = WM <= 4;
   // (rows of a multiple of 4 floats, aligned: checked by the caller)
   const auto request_values = [&](int n) {
     const float* row = vbase + (size_t)lane * a.S + jb;
+    // A whole wavefront's in one go: a lane's 16 loads lie in four lines of 64 bytes, and
+    // with addresses formed in between, the loads of 15 other wavefronts come in between
+    // and take the lines out of L1 (32 x 12 heads, 900 of 1000 valid, us: before the
+    // values were read 16 at a time 40.0, then 43.8, so 36.4).  Up to 4 wavefronts it costs
+    // 28 registers, and a third workgroup per CU.
+    if (!kAhead && jb + 64 <= n) {
+#pragma unroll
+      for (int c = 0; c < 16; ++c) value[c] = *reinterpret_cast<const float4*>(row + 4 * c);
+      asm volatile("");  // (or the first of them are made one with those below)
+      return;
+    }
 #pragma unroll
     for (int c = 0; c < 16; ++c) {  // (what is left out is not looked at)
       if (c % 4 == 0 && jb + 4 * c >= n) break;
       value[c] = *reinterpret_cast<const float4*>(row + min(4 * c, a.S - 4 - jb));
     }
   };
-  constexpr bool kAhead = WM <= 4;
   const bool early = a.early && wave == 0;
   int n = a.index[b];  // (one wait for both)
   if constexpr (kAhead) {
