@@ -246,11 +246,13 @@ hyper_norm_kernel(HyperArgs h) {
   __shared__ float s4[4];
   const int n = g.streams;
   const bool add = g.y != nullptr || g.parts != nullptr;
-  // Of up to 4 streams the weights are in registers, requested with the row (through LDS,
-  // behind a barrier, and the experts' rows one after the other: 64 rows of 4 x 1024 5.8
-  // us, now 4.7; 8192 rows 55.6, now 53.2); of more they go through LDS.
+  // The weights of 1 or 4 streams go into registers, a few wide loads requested with the
+  // row (through LDS, behind a barrier, and the experts' rows one after the other: 64 rows
+  // of 4 x 1024 5.8 us, now 4.7; 8192 rows 55.6, now 53.2).  Other numbers of streams take
+  // them through LDS: each by a load and a branch of its own, 2000 rows of 2 x 1024 with
+  // 3 parts lasted 10.4 us instead of 9.6.
   constexpr bool kFew = S <= 4;
-  __shared__ float s_far[kFew ? 1 : S * S + 2 * S];
+  __shared__ float s_far[S * S + 2 * S];
   float s_near[kFew ? S * S + 2 * S : 1];
   const auto weight = [&](int i) {
     if (i < S * S) {
@@ -262,12 +264,31 @@ hyper_norm_kernel(HyperArgs h) {
     const int s = (i - S * S) % S;
     return s >= n ? 0.f : w != nullptr ? w[s] : 1.f;
   };
-  if constexpr (kFew) {
+  if (kFew && n == S) {
+    const float *mix = g.mix, *spread = g.spread, *collect = g.collect;
 #pragma unroll
-    for (int i = 0; i < S * S + 2 * S; ++i) s_near[i] = weight(i);
+    for (int i = 0; i < S * S; ++i) s_near[i] = i / S == i % S ? 1.f : 0.f;
+#pragma unroll
+    for (int i = 0; i < 2 * S; ++i) s_near[S * S + i] = 1.f;
+    if (mix != nullptr) {
+#pragma unroll
+      for (int i = 0; i < S * S; ++i) s_near[i] = mix[i];
+    }
+    if (spread != nullptr) {
+#pragma unroll
+      for (int i = 0; i < S; ++i) s_near[S * S + i] = spread[i];
+    }
+    if (collect != nullptr) {
+#pragma unroll
+      for (int i = 0; i < S; ++i) s_near[S * S + S + i] = collect[i];
+    }
   } else {
     for (int i = threadIdx.x; i < S * S + 2 * S; i += 256) s_far[i] = weight(i);
     __syncthreads();
+    if constexpr (kFew) {
+#pragma unroll
+      for (int i = 0; i < S * S + 2 * S; ++i) s_near[i] = s_far[i];
+    }
   }
   const float* s_mix = kFew ? s_near : s_far;
   const float *s_spread = s_mix + S * S, *s_collect = s_spread + S;
