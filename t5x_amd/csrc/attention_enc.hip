@@ -33,8 +33,8 @@ struct EncAttnArgs {
   const bf16_t* bias; // [H, 2E-1]: by (key - query + E - 1)
   const int32_t* len; // [B] valid prefix length (with `valid`: last valid + 1)
   const uint32_t* valid;  // optional [B, (E + 31) / 32]: bit e = position e valid
-  const int32_t* first;   // optional [B + 1]: rows first[b] .. first[b + 1] are text
-                          // b's instead of b * E .. (b + 1) * E (t5d_encoder_rows:
+  const int32_t* first;   // ROWS kernels: [B + 1], rows first[b] .. first[b + 1] are
+                          // text b's instead of b * E .. (b + 1) * E (t5d_encoder_rows:
                           // every position below len, then one or more of padding)
   bf16_t* out;        // [B*E, H*64]
   int B, H, E, Ep, q_stride, k_stride;
@@ -65,6 +65,7 @@ typedef __attribute__((address_space(1))) const void* enc_glb_ptr_t;
 
 constexpr int kShortEnc = 64;  // its longest text
 
+template <bool ROWS>
 __global__ void __launch_bounds__(256)
 enc_attn_short_kernel(EncAttnArgs a) {
   __shared__ uint4 s_k[512], s_v[512];
@@ -79,8 +80,8 @@ enc_attn_short_kernel(EncAttnArgs a) {
   const int l16 = lane & 15, gq = lane >> 4;
   const int h = blockIdx.y, b = blockIdx.z;
   const int E = a.E;
-  const size_t row0 = a.first ? a.first[b] : (size_t)b * E;
-  const int rows = a.first ? a.first[b + 1] - a.first[b] : E;  // that are there
+  const size_t row0 = ROWS ? a.first[b] : (size_t)b * E;
+  const int rows = ROWS ? a.first[b + 1] - a.first[b] : E;  // that are there
 
   // What this lane fetches of K: chunks (8 keys, 1 KB) wave and wave + 4; lane s
   // lands at slot s & 7 of key s >> 3 and therefore reads piece (s & 7) ^ (s >> 3) of
@@ -248,7 +249,7 @@ enc_attn_short_kernel(EncAttnArgs a) {
   }
   // A padded query weighs all E positions alike; padding beyond the rows that are there
   // has the values of the padding that is.
-  if (rows < E && q0 + l16 < rows && !q_valid) {
+  if (ROWS && rows < E && q0 + l16 < rows && !q_valid) {
     const float w = (float)(E - rows) * bf16_to_f32(f32_to_bf16(inv));
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
@@ -300,7 +301,7 @@ enc_attn_short_kernel(EncAttnArgs a) {
 constexpr float kMaxSlack = 8.0f;
 constexpr float kLog2eE = 1.4426950408889634f;
 
-template <int MT>  // 16 queries each per wavefront: 2 or 1
+template <int MT, bool ROWS>  // 16 queries each per wavefront: 2 or 1
 __global__ void __launch_bounds__(256, 3)
 enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   constexpr int KB = 64, QW = 16 * MT;  // keys per tile, queries per wavefront
@@ -320,9 +321,9 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, gq = lane >> 4;
   const int E = a.E;
-  const size_t row0 = a.first ? a.first[b] : (size_t)b * E;
-  const int rows = a.first ? a.first[b + 1] - a.first[b] : E;  // that are there
-  if (tile * 4 * QW >= rows) return;
+  const size_t row0 = ROWS ? a.first[b] : (size_t)b * E;
+  const int rows = ROWS ? a.first[b + 1] - a.first[b] : E;  // that are there
+  if (ROWS && tile * 4 * QW >= rows) return;
 
   // the pieces this lane fetches: keys (rows of 128 bytes, clamped at the last),
   // V^T (blocks of 32 keys: rows of 64 bytes)
@@ -384,7 +385,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   __syncthreads();
   // The keys that a padded query weighs here.  Where rows are given, padding is left
   // to the end: one of its rows stands for all of it.
-  const int E_here = a.first ? n : E;
+  const int E_here = ROWS ? n : E;
   // Keys each wavefront of the workgroup walks: the valid prefix if all of its
   // queries are valid, else all there are (none past the end).
   int my_keys = 0, wg_keys = 0;
@@ -574,9 +575,10 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  // (the first tile has been fetched whatever there is to walk, and every tile that is
-  // fetched is met before the end)
-  for (int jt = 0; jt == 0 || jt < wg_keys; jt += 2 * KB) {
+  // (every tile that is fetched is met before the end.  wg_keys >= 1, as a workgroup has a
+  // query, which is valid or walks all keys; but not of given rows, where a text may have
+  // no token: the first tile has been fetched all the same)
+  for (int jt = 0; (ROWS && jt == 0) || jt < wg_keys; jt += 2 * KB) {
     meet();
     if (jt + KB < wg_keys) fetch(jt + KB, s_k1, s_v1);
     attend(jt, s_k0, s_v0);
@@ -591,7 +593,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
     const int q = q0 + 16 * mt + l16;
     if (q >= rows) continue;
     // (such a query's maximum is 0, or was never raised: its keys weigh 1)
-    if (a.first && n < E && q >= n) {
+    if (ROWS && n < E && q >= n) {
       const float w = (float)(E - n);
       sum += w;
 #pragma unroll
@@ -750,18 +752,24 @@ static int encoder_attention(void* stream, const void* q, const void* k, const v
   a.valid = valid_bits; a.first = first;
   a.B = B; a.H = H; a.E = E; a.Ep = Ep; a.q_stride = q_stride; a.k_stride = k_stride;
   if (E <= kShortEnc) {
-    hipLaunchKernelGGL(enc_attn_short_kernel, dim3(1, H, B), dim3(256), 0,
-                       as_stream(stream), a);
+    if (first)
+      hipLaunchKernelGGL(enc_attn_short_kernel<true>, dim3(1, H, B), dim3(256), 0,
+                         as_stream(stream), a);
+    else
+      hipLaunchKernelGGL(enc_attn_short_kernel<false>, dim3(1, H, B), dim3(256), 0,
+                         as_stream(stream), a);
   } else {
     const bool low = one_pass_64(B, H, most);
     const int tiles = low ? (most + 63) / 64 : (most + 127) / 128;
     const dim3 groups(((unsigned)B * H + 7) / 8 * 8 * tiles);
-    if (low)
-      hipLaunchKernelGGL(enc_attn_tile_kernel<1>, groups, dim3(256), 0,
-                         as_stream(stream), a, tiles);
-    else
-      hipLaunchKernelGGL(enc_attn_tile_kernel<2>, groups, dim3(256), 0,
-                         as_stream(stream), a, tiles);
+#define T5D_ENC(MT_, ROWS_)                                                       \
+  hipLaunchKernelGGL((enc_attn_tile_kernel<MT_, ROWS_>), groups, dim3(256), 0,    \
+                     as_stream(stream), a, tiles)
+    if (low && first) T5D_ENC(1, true);
+    else if (low) T5D_ENC(1, false);
+    else if (first) T5D_ENC(2, true);
+    else T5D_ENC(2, false);
+#undef T5D_ENC
   }
   T5D_CHECK_LAUNCH("t5d_encoder_attention");
   return T5D_OK;

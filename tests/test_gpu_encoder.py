@@ -899,3 +899,68 @@ def test_encoder_over_the_rows_that_there_are(E):
   again = encoder._encode_positions(cfg, w, torch.nn.functional.pad(t, (0, -E % 4)),
                                     got.device)[:, :E]
   assert torch.equal(other, again)
+
+
+@pytest.mark.parametrize('E', [62, 130, 257, 512, 1031, 2048])
+@pytest.mark.parametrize('wide', [False, True])
+def test_encoder_attention_over_rows_of_ragged_texts(ops, E, wide):
+  """Rows given one behind the other, with few workgroups and (wide) with so many that a
+  wavefront takes two tiles of queries, which padding may begin in: tokens have the bits
+  of the kernel over every position, padding is the mean of all values.  That is one
+  rounding to bfloat16 (2^-8) and float32 sums of at most E terms."""
+  lens = sorted({n for n in (0, 1, 31, 32, 33, 127, 128, E - 1, E) if n <= E})
+  B, E4 = len(lens), (E + 3) // 4 * 4
+  H = 1024 // (B * (-(-E4 // 64))) + 1 if wide else 2
+  gen = torch.Generator(device='cuda')
+  gen.manual_seed(E)
+  rnd = lambda *shape: torch.randn(shape, generator=gen, device='cuda').bfloat16()
+  tokens = torch.zeros((B, E), dtype=torch.int64, device='cuda')
+  for b, n in enumerate(lens):
+    tokens[b, :n] = 7
+  rows = ops.EncoderRows(tokens)
+  first = rows.first.tolist()
+  assert not rows.odd and rows.positions == E4 and rows.most == E4
+  Ep = (E4 + 31) // 32 * 32
+  q, k = rnd(B, E4, H * 64), rnd(B, E4, H * 64)
+  v = torch.zeros((B, H, 64, Ep), dtype=torch.bfloat16, device='cuda')
+  v[..., :E4] = rnd(B, H, 64, E4)
+  some = v.clone()
+  for b, n in enumerate(lens):
+    v[b, ..., n:E4] = v[b, ..., n:n + 1].clone() if n < E4 else 0
+    there = first[b + 1] - first[b]
+    some[b] = v[b]
+    some[b, ..., there:] = 0
+  rel = rnd(H, 2 * E4 - 1)
+  pick = lambda x: torch.cat([x[b, :first[b + 1] - first[b]] for b in range(B)])
+  got = ops.encoder_attention_rows(pick(q), pick(k), ops.tile_cross_value(some), rel, rows)
+  want = ops.encoder_attention(
+      q.view(B * E4, -1), k.view(B * E4, -1), ops.tile_cross_value(v), rel,
+      dev(np.array(lens, np.int32))).view(B, E4, -1)
+  mean = v[..., :E4].double().mean(-1).view(B, -1)
+  size = v[..., :E4].double().abs().mean(-1).view(B, -1)
+  for b, n in enumerate(lens):
+    mine = got[first[b]:first[b + 1]]
+    assert torch.equal(mine[:n], want[b, :n]), (b, n)
+    bound = 2.0**-8 * mean[b].abs() + E4 * 2.0**-24 * size[b]
+    assert bool(((mine[n:].double() - mean[b]).abs() <= bound).all()), (b, n)
+
+
+def test_encoder_of_many_ragged_texts():
+  """The whole encoder where its attention takes two tiles of queries per wavefront."""
+  from t5x_amd import encoder, network
+  ocfg, cfg = _tiny_cfgs()
+  module = network.Transformer(cfg, torch.device('cuda'))
+  params = ot5.init_params(ocfg, seed=3)
+  rs = np.random.RandomState(0)
+  B, E = 1024 // (3 * cfg.num_heads) + 1, 131
+  tokens = rs.randint(2, cfg.vocab_size, size=(B, E))
+  tokens[np.arange(E)[None, :] >= rs.randint(0, E + 1, (B, 1))] = 0
+  t = torch.as_tensor(tokens, device='cuda')
+  got = encoder.encode(module, params, t)
+  w = next(iter(module._enc_weights.values()))[1]
+  want = encoder._encode_positions(cfg, w, torch.nn.functional.pad(t, (0, 1)),
+                                   got.device)[:, :E]
+  valid = t > 0
+  assert torch.equal(got[valid], want[valid])
+  a, b = got[~valid].double(), want[~valid].double()
+  assert ((a - b).norm() / b.norm()).item() < 6 * 2.0 ** -8
