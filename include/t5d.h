@@ -345,6 +345,12 @@ int t5d_encoder_rows(void* stream, const int64_t* tokens, int B, int E, int32_t*
                      int32_t* odd, int32_t* first, int32_t* ids, int32_t* row_of,
                      int32_t* at, int32_t* summary);
 
+/* Which positions of tokens [B, E] hold a token > 0: bits [B, (E + 31) / 32], bit e % 32
+ * of word e / 32, and last [B], the last such position + 1 (0: none), as
+ * t5d_encoder_attention takes them. */
+int t5d_token_mask(void* stream, const int64_t* tokens, int B, int E, int32_t* last,
+                   uint32_t* bits);
+
 /* t5d_encoder_attention over the rows that t5d_encoder_rows lists: q, k and out hold
  * first[B] rows; most: rows of the longest text (summary[1]); E: the positions that a
  * text has and that a padded query weighs, at least the E of t5d_encoder_rows and at

@@ -85,9 +85,44 @@ encoder_rows_kernel(const int64_t* __restrict__ tokens, const int32_t* __restric
   for (int e = threadIdx.x; e < E; e += 256) row_of[(size_t)b * E + e] = r0 + min(e, n);
 }
 
+// One workgroup per text: a bit per position that holds a token, and the last such
+// position + 1.
+__global__ void __launch_bounds__(256)
+token_mask_kernel(const int64_t* __restrict__ tokens, int32_t* __restrict__ last,
+                  uint32_t* __restrict__ bits, int E) {
+  __shared__ int s_last;
+  if (threadIdx.x == 0) s_last = 0;
+  __syncthreads();
+  const int64_t* row = tokens + (size_t)blockIdx.x * E;
+  const int words = (E + 31) >> 5, lane = threadIdx.x & 63;
+  int end = 0;
+  for (int e0 = 0; e0 < E; e0 += 256) {  // (no lane leaves a wavefront early)
+    const int e = e0 + threadIdx.x;
+    const bool is = e < E && row[e] > 0;
+    const unsigned long long all = __builtin_amdgcn_ballot_w64(is);
+    if ((lane & 31) == 0 && (e >> 5) < words)
+      bits[(size_t)blockIdx.x * words + (e >> 5)] = (uint32_t)(all >> lane);
+    if (is) end = e + 1;
+  }
+  atomicMax(&s_last, end);
+  __syncthreads();
+  if (threadIdx.x == 0) last[blockIdx.x] = s_last;
+}
+
 }  // namespace t5d
 
 using namespace t5d;
+
+extern "C" int t5d_token_mask(void* stream, const int64_t* tokens, int B, int E,
+                              int32_t* last, uint32_t* bits) {
+  T5D_REQUIRE(tokens && last && bits, T5D_EINVAL, "t5d_token_mask: null pointer");
+  T5D_REQUIRE(B > 0 && E > 0 && E < (1 << 30), T5D_EINVAL, "t5d_token_mask: B=%d E=%d", B,
+              E);
+  hipLaunchKernelGGL(token_mask_kernel, dim3(B), dim3(256), 0, as_stream(stream), tokens,
+                     last, bits, E);
+  T5D_CHECK_LAUNCH("t5d_token_mask");
+  return T5D_OK;
+}
 
 extern "C" int t5d_encoder_rows(void* stream, const int64_t* tokens, int B, int E,
                                 int32_t* len, int32_t* odd, int32_t* first,

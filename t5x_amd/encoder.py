@@ -86,25 +86,28 @@ def _encode_hip(module, params, tokens):
     module._enc_weights[key] = (params, EncoderKernelWeights(cfg, params, dev))
   w = module._enc_weights[key][1]
   B, E = tokens.shape
+  odd = None
   if E <= ops.MAX_ENCODER_LENGTH and cfg.emb_dim % 8 == 0:
     rows = ops.EncoderRows(tokens)
     if not rows.odd:
       return _encode_rows(cfg, w, rows, dev)
+    odd = True
   if E % 4:
     # The dense kernel's head-layout epilogue takes lengths in multiples of 4:
     # pad with padding tokens (masked keys; their own rows are dropped again).
     tokens = torch.nn.functional.pad(tokens, (0, -E % 4))
-    return _encode_positions(cfg, w, tokens, dev)[:, :E].contiguous()
-  return _encode_positions(cfg, w, tokens, dev)
+    return _encode_positions(cfg, w, tokens, dev, odd)[:, :E].contiguous()
+  return _encode_positions(cfg, w, tokens, dev, odd)
 
 
-def _encode_positions(cfg, w, tokens, dev):
-  """_encode_hip over every position: padding inside a text is masked by bits."""
+def _encode_positions(cfg, w, tokens, dev, odd=None):
+  """_encode_hip over every position: padding inside a text is masked by bits.  odd:
+  that there is such padding is known (_key_mask)."""
   from t5x_amd import _lib, ops
   B, E = tokens.shape
   H = cfg.num_heads
   HD = H * 64
-  lens, bits = _key_mask(tokens, dev)
+  lens, bits = _key_mask(tokens, dev, odd)
   Ep = (E + 31) // 32 * 32  # values are stored in blocks of 32 positions
   bias = w.rel_bias(E)
   ids = tokens.reshape(-1).to(torch.int32).contiguous()
@@ -163,21 +166,22 @@ class EncoderKernelWeightsF32:
     return self._bias[E]
 
 
-def _key_mask(tokens, dev):
+def _key_mask(tokens, dev, odd=None):
   """The padding mask of t5x/examples/t5/network.py:325-328 (token > 0,
   element-wise) as the kernels take it: (lengths, bits).  Padding that is a
   suffix of zeros, the usual case, is a length per row and bits None; a
   padding token inside the text gives the last valid position + 1 and one bit
-  per position (ops.pack_valid_bits)."""
+  per position (ops.token_mask).  odd: take that form at once, instead of waiting
+  for the device to say which."""
   from t5x_amd import ops
   B, E = tokens.shape
-  valid = tokens > 0
-  lens = valid.sum(dim=1).to(torch.int32)
-  prefix = torch.arange(E, device=dev)[None, :] < lens[:, None]
-  if bool((prefix == valid).all()):
-    return lens.contiguous(), None
-  last = (valid * torch.arange(1, E + 1, device=dev)[None, :]).max(dim=1).values
-  return last.to(torch.int32).contiguous(), ops.pack_valid_bits(valid)
+  if not odd:
+    valid = tokens > 0
+    lens = valid.sum(dim=1).to(torch.int32)
+    prefix = torch.arange(E, device=dev)[None, :] < lens[:, None]
+    if bool((prefix == valid).all()):
+      return lens.contiguous(), None
+  return ops.token_mask(tokens.contiguous())
 
 
 def _encode_hip_f32(module, params, tokens):

@@ -576,6 +576,18 @@ def pack_valid_bits(valid):
   return packed.to(torch.int32).contiguous()
 
 
+def token_mask(tokens):
+  """(last, bits) of tokens [B, E] int64: the last position + 1 that holds a token > 0,
+  and pack_valid_bits(tokens > 0) (t5d_token_mask)."""
+  _chk(tokens, 'tokens', torch.int64, 2)
+  B, E = tokens.shape
+  last = torch.empty((B,), dtype=torch.int32, device=tokens.device)
+  bits = torch.empty((B, (E + 31) // 32), dtype=torch.int32, device=tokens.device)
+  _lib.call('t5d_token_mask', _s(), tokens.data_ptr(), B, E, last.data_ptr(),
+            bits.data_ptr())
+  return last, bits
+
+
 def encoder_attention(q, k, v_t, rel_bias, enc_len, out=None, valid_bits=None,
                       variant=0):
   """q, k: [B*E, >= H*64] row-major views (row stride = stride(0)); v_t

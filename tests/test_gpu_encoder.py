@@ -964,3 +964,18 @@ def test_encoder_of_many_ragged_texts():
   assert torch.equal(got[valid], want[valid])
   a, b = got[~valid].double(), want[~valid].double()
   assert ((a - b).norm() / b.norm()).item() < 6 * 2.0 ** -8
+
+
+@pytest.mark.parametrize('B,E', [(1, 1), (3, 31), (2, 32), (5, 33), (4, 255), (3, 256),
+                                 (2, 257), (7, 1031)])
+def test_token_mask(ops, B, E):
+  """Zeros and negative numbers are no tokens, nor are the low halves of large ones."""
+  rs = np.random.RandomState(E)
+  t = rs.choice([0, -1, -2**40, 1, 7, 2**33], size=(B, E))
+  t[-1] = 0
+  t[0, -1] = 5
+  last, bits = ops.token_mask(dev(t))
+  valid = t > 0
+  want = (valid * np.arange(1, E + 1)).max(1)
+  np.testing.assert_array_equal(host(last), want)
+  assert torch.equal(bits, ops.pack_valid_bits(dev(valid)))
