@@ -87,7 +87,7 @@ def _encode_hip(module, params, tokens):
   w = module._enc_weights[key][1]
   B, E = tokens.shape
   odd = None
-  if E <= ops.MAX_ENCODER_LENGTH and cfg.emb_dim % 8 == 0:
+  if ops.EncoderRows.covers(B, E) and cfg.emb_dim % 8 == 0:
     rows = ops.EncoderRows(tokens)
     if not rows.odd:
       return _encode_rows(cfg, w, rows, dev)

@@ -537,6 +537,12 @@ class EncoderRows:
   else than tokens > 0 followed by zeros, and only `len` (the number of tokens > 0)
   holds.  Waits for the device once, to learn how many rows there are."""
 
+  @staticmethod
+  def covers(B, E):
+    """What t5d_encoder_rows takes: 19 bits of text, 12 of position, 30 of rows."""
+    return (E <= MAX_ENCODER_LENGTH and B < 1 << 19 and
+            B * ((E + 3) // 4 * 4) < 1 << 30)
+
   def __init__(self, tokens):
     _chk(tokens, 'tokens', torch.int64, 2)
     self.B, self.E = B, E = tokens.shape

@@ -93,6 +93,17 @@ def test_encoder_attention_beyond_a_launch_grid_without_gpu():
   assert b'launch grid' in lib.t5d_last_error()
 
 
+@pytest.mark.parametrize('B,E', [(1, 2049), (1 << 19, 1), (1 << 20, 1023), (525000, 2046)])
+def test_encoder_rows_beyond_their_numbers_without_gpu(B, E):
+  """What t5d_encoder_rows names as too much, the encoder does not ask of it (it computes
+  every position then)."""
+  from t5x_amd import ops
+  assert _lib.load().t5d_encoder_rows(None, 16, B, E, *[16] * 7) == -3  # T5D_ELIMIT
+  assert not ops.EncoderRows.covers(B, E)
+  for there in ((1, 2048), ((1 << 19) - 1, 2044), (32, 512)):
+    assert ops.EncoderRows.covers(*there) == (there[0] * there[1] < 1 << 30)
+
+
 def test_many_row_tile_choice_without_gpu():
   """t5d_gemm_rows_tile: which workgroup tile the many-row dense kernel runs a
   shape on (1: 256 x 128, 2: 256 x 256, 3: 256 x 192), by the rounds of
