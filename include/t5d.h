@@ -181,7 +181,7 @@ int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
 
 /* t5d_gemm_rows into the value layout (T5D_OUT_HEADS_VALUE) for rows that
  * t5d_encoder_rows lists: rows 4 i .. 4 i + 3 are positions e .. e + 3 of text b,
- * at[i] = b << 12 | e.  M a multiple of 4. */
+ * at[i] = b << 12 | e.  M a multiple of 4.  Other positions of C are left as they are. */
 int t5d_gemm_rows_values(void* stream, int w_dtype, const void* A, const void* W,
                          const float* scales, void* C, int64_t M, int K, int N,
                          const int32_t* at, int E, int Ep);
@@ -354,7 +354,11 @@ int t5d_token_mask(void* stream, const int64_t* tokens, int B, int E, int32_t* l
 /* t5d_encoder_attention over the rows that t5d_encoder_rows lists: q, k and out hold
  * first[B] rows; most: rows of the longest text (summary[1]); E: the positions that a
  * text has and that a padded query weighs, at least the E of t5d_encoder_rows and at
- * most that rounded up to a multiple of 4. */
+ * most that rounded up to a multiple of 4.  v_t must hold zeros at all positions (up to
+ * Ep) that t5d_gemm_rows_values wrote nothing to: a padded query of a short text weighs
+ * those below E like the others, and all queries multiply those of their last keys' blocks
+ * by a weight of zero.  (Cleared once it can serve every layer: they write to the same
+ * positions.) */
 int t5d_encoder_attention_rows(void* stream, const void* q, const void* k,
                                const void* v_t, const void* rel_bias,
                                const int32_t* enc_len, const int32_t* first, int most,

@@ -511,7 +511,8 @@ def gemm_rows(a, w: PackedWeight, out=None, residual=None,
 
 
 def gemm_rows_values(a, w: PackedWeight, rows, out):
-  """gemm_rows into `out` [B, H, Ep/32, 64, 32] for the rows of an EncoderRows."""
+  """gemm_rows into `out` [B, H, Ep/32, 64, 32] for the rows of an EncoderRows; the
+  positions without a row are left as they are (encoder_attention_rows wants zeros)."""
   _chk(a, 'a', torch.bfloat16, 2)
   _chk(out, 'out', a.dtype, 5)
   M, K = a.shape
@@ -629,7 +630,8 @@ def encoder_attention(q, k, v_t, rel_bias, enc_len, out=None, valid_bits=None,
 
 def encoder_attention_rows(q, k, v_t, rel_bias, rows):
   """encoder_attention over the rows of an EncoderRows: q, k [rows.M, H*64] views ->
-  [rows.M, H*64]."""
+  [rows.M, H*64].  v_t as gemm_rows_values leaves it in what were zeros: it must be zero
+  at every position that has no row."""
   _chk(v_t, 'v_t', torch.bfloat16, 5)
   _chk(rel_bias, 'rel_bias', torch.bfloat16, 2)
   B, H, blocks, D, w = v_t.shape
