@@ -955,10 +955,12 @@ recurrence_finish_kernel(RecArgs g) {
 //   no delta rule, 8 heads of 128 x 128        5.8 11.4 21.7 42.6 /  5.0 10.8 21.0 40.6
 //   no delta rule, 4 heads of 48 x 64          4.3  4.8  5.6  6.7 /  3.7  4.2  4.9  6.7
 // (64 states of 8 x 128 x 128 take 13.7 us at the rate of a large copy from memory.)
-// EXACT: heads of 128 x 128 (a workgroup's four wavefronts have 32 columns each) and
-// taps that are all requested ahead; nothing is tested then and 2100 instructions do
-// instead of 3480, which a lone launch has to fetch (8 heads, one token, in a model's
-// step: delta rule 8.0 -> 6.2 us, without 7.3 -> 5.6).
+// EXACT: heads as wide as the template (32, 64 or 128 channels of keys and of values) and
+// taps that are all requested ahead; nothing is tested then: with 128, 2100 instructions
+// do instead of 3480, which a lone launch has to fetch (8 heads, one token, in a model's
+// step: delta rule 8.0 -> 6.2 us, without 7.3 -> 5.6; launches behind one another, 1 / 64
+// rows of 8 heads: 6.1 / 11.7 -> 5.0 / 10.3, of 64 x 64 4.6 / 6.2 -> 3.9 / 5.5, of 32 x 32
+// 4.1 / 4.8 -> 3.5 / 4.2).  Heads of 256 have two taps ahead and no registers to gain.
 template <int DI, bool DELTA, typename T, bool EXACT>
 __global__ void __launch_bounds__(512)
 recurrence_step_kernel(RecArgs g) {
@@ -1027,6 +1029,7 @@ recurrence_step_kernel(RecArgs g) {
   float4 st[DI];
   const auto request_state = [&] {
     if constexpr (EXACT) {  // (a sequence's first token: not looked at)
+      if (DP < 128 && 32 * wave >= DP) return;  // (there for its role alone)
 #pragma unroll
       for (int i = 0; i < DI; ++i)
         st[i] = *reinterpret_cast<const float4*>(state + (size_t)(dg + 8 * i) * Dv);
@@ -1172,9 +1175,12 @@ static void launch_step(hipStream_t s, const RecArgs& g) {
 #define T5D_RS(DI_, EXACT_)                                                       \
   hipLaunchKernelGGL((recurrence_step_kernel<DI_, DELTA, T, EXACT_>), grid, block, 0, \
                      s, g)
-  if (g.a.D <= 32) T5D_RS(4, false);
+  const bool exact = g.a.D == g.a.Dv && g.a.taps <= 4;
+  if (exact && g.a.D == 32) T5D_RS(4, true);
+  else if (g.a.D <= 32) T5D_RS(4, false);
+  else if (exact && g.a.D == 64) T5D_RS(8, true);
   else if (g.a.D <= 64) T5D_RS(8, false);
-  else if (g.a.D == 128 && g.a.Dv == 128 && g.a.taps <= 4) T5D_RS(16, true);
+  else if (exact && g.a.D == 128) T5D_RS(16, true);
   else if (g.a.D <= 128) T5D_RS(16, false);
   else T5D_RS(32, false);
 #undef T5D_RS

@@ -701,6 +701,25 @@ def test_recurrence_steps_of_heads_of_128(dt, delta, H, G, taps):
 
 
 @pytest.mark.parametrize('dt', DTYPES)
+@pytest.mark.parametrize('delta,H,G,taps', [
+    (True, 2, 2, 4), (True, 4, 2, 1), (True, 2, 2, 0), (True, 2, 1, 5), (False, 3, 3, 0)])
+@pytest.mark.parametrize('D', [32, 64])
+def test_recurrence_steps_of_heads_as_wide_as_a_template(dt, delta, H, G, taps, D):
+  """The same for the other sizes that have a kernel without tests; the states of the
+  last slot end with their buffer."""
+  T = 12
+  r = Recurrence(dt, delta, H, G, D, D, taps, 2, seed=taps)
+  seq = r.sequence(T)
+  want = r.oracle(seq)
+  r.state.fill_(float('nan'))
+  got = [r.run([(1, t, t + 1)], [seq]) for t in range(T)]
+  assert rel(np.concatenate(got), want) < r.tol
+  got = [r.run([(0, 0, 5)], [seq])] + [r.run([(0, t, t + 1)], [seq])
+                                       for t in range(5, T)]
+  assert rel(np.concatenate(got), want) < r.tol
+
+
+@pytest.mark.parametrize('dt', DTYPES)
 @pytest.mark.parametrize('delta', [True, False])
 def test_recurrence_batches_match_each_alone(dt, delta):
   r = Recurrence(dt, delta, 4, 2 if delta else 4, 48, 32, 3 if delta else 0, 6)
