@@ -169,11 +169,12 @@ int t5d_gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
                   int64_t M, int K, int N, int epilogue, int out_layout, int E,
                   int Ep);
 
-/* t5d_gemm_rows with the workgroup tile of the caller's choice: tile 1 = 128 columns
- * of 128 rows, or of 64 where those cost less, tile 2 = 256 and tile 3 = 192 columns
- * of 128 rows (4 wavefronts each; bfloat16 weights and K >= 64, otherwise 256 rows x
- * 128 columns), tile 0 = what t5d_gemm_rows picks from the shape.  Results have the
- * same bits for every tile.  For tuning and for testing every kernel at any size. */
+/* t5d_gemm_rows with the workgroup tile of the caller's choice (4 wavefronts each): tile
+ * 1 = 128 columns of 128 rows, or of 64 where those cost less, tile 2 = 256 and tile 3 =
+ * 192 columns of 128 rows, tile 0 = what t5d_gemm_rows picks from the shape.  int8 weights
+ * have tile 1 whatever is asked for; K < 64 and operands beyond 32-bit offsets run on 256
+ * rows x 128 columns.  Results have the same bits for every tile.  For tuning and for
+ * testing every kernel at any size. */
 int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
                         const void* W, const float* scales,
                         const void* residual, void* C, int64_t M, int K, int N,
@@ -188,7 +189,8 @@ int t5d_gemm_rows_values(void* stream, int w_dtype, const void* A, const void* W
 
 /* The workgroup tile (1, 2 or 3, as in t5d_gemm_rows_tiled) that t5d_gemm_rows
  * uses for a shape: the cheapest by the rounds of workgroups each tile needs
- * on 256 CUs.  No device work; for tests and for reading a profile. */
+ * on 256 CUs (1 where the tile is not chosen, see above).  No device work; for tests and
+ * for reading a profile. */
 int t5d_gemm_rows_tile(int w_dtype, int64_t M, int K, int N);
 
 /* One step of cached decoder self-attention

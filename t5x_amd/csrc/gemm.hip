@@ -1054,8 +1054,9 @@ bool t5d::norm_gemm_is_wide(int w_dtype, int K, int N) {
          (K == 512 || K == 768 || K == 1024);
 }
 
-// The matrix cores where K comes in whole 32s (gemm_f32.hip), otherwise the kernel
-// above (rows in groups of 8 along grid.y).  Both add in the same order whatever M is,
+// The matrix cores where K comes in whole 32s, 128 or more, and rows and norm scale lie on
+// 16 bytes (launch_f32_mfma), otherwise the kernel above (rows in groups of 8 along
+// grid.y).  Both add in the same order whatever M is,
 // so no bit of a result depends on how many rows a call carries.
 static void launch_gemm_f32(hipStream_t s, const float* A, const float* W,
                             const float* residual, float* C, int M, int K,

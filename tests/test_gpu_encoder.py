@@ -61,8 +61,8 @@ def test_gemm_rows(ops, M, K, N, mode):
     mid = ops.gemm_rows(a, pw, residual=res, tile=3)
   assert out.shape == want.shape
   np.testing.assert_allclose(host(out), want, atol=2e-2, rtol=2**-7)
-  # every workgroup tile (256 x 128, 256 x 256, 256 x 192) and the one picked
-  # from the shape give the same bits
+  # every workgroup tile (128, 256 and 192 columns) and the one picked from the
+  # shape give the same bits
   assert torch.equal(out, wide)
   assert torch.equal(out, mid)
   chosen = ops.gemm_rows(a, pw, residual=None if mode != 'residual' else res)
@@ -123,9 +123,9 @@ def test_gemm_rows_repeated_launches_at_full_size(ops):
 
 @pytest.mark.parametrize('M,rows', [(601, 64), (1985, 64), (4001, 128)])
 def test_gemm_rows_repeated_launches_of_low_tiles(ops, M, rows):
-  """The same for the tiles of 64 and 128 rows, which the 128-column tile gets while
-  its workgroups are fewer than the 256 compute units; lengths off the tile, the
-  residual overwritten by the result."""
+  """The same for the tiles of 64 and 128 rows, one of which the 128-column tile gets by
+  what its rounds of workgroups cost (`rows` at these lengths); lengths off the tile,
+  the residual overwritten by the result."""
   groups = lambda n: -(-M // n) * (768 // 128)
   assert (groups(64) <= 256) == (rows == 64) and groups(128) <= 256
   g = torch.Generator(device='cuda')
@@ -173,8 +173,9 @@ def test_gemm_rows_plain_entry_point(ops):
 @pytest.mark.parametrize('M', [129, 191, 192, 193, 640, 1000, 4104])
 @pytest.mark.parametrize('K,N', [(64, 16), (96, 208), (160, 832)])
 def test_gemm_rows_of_low_tiles(ops, M, K, N):
-  """Tiles of 64, 128 and 256 rows (by the number of workgroups) at their edges: the bits
-  of the 256 x 256 tile, which adds up K in the same order, and of the whole in parts."""
+  """Tiles of 64 and 128 rows x 128 columns (by what their rounds of workgroups cost) at
+  their edges: the bits of the tile of 256 columns, which adds up K in the same order, and
+  of the whole in parts."""
   rs = np.random.RandomState(M + N)
   a = dev(rs.randn(M, K).astype(np.float32), torch.bfloat16)
   w0, w1 = (dev((rs.randn(K, N) / np.sqrt(K)).astype(np.float32)) for _ in range(2))
