@@ -79,13 +79,16 @@ gemm_mfma_kernel(Args g) {
   const char* wbase = reinterpret_cast<const char*>(g.W);
   constexpr int TB = WeightTile<WT>::kTileBytes;
 
-  // (NJ > 0 and NT = 4: where this wavefront's first tiles lie; the others follow at
-  // constant distances, which the loads take as offsets.  With fewer column tiles the
-  // addresses are formed where they are used, between the products: us, constant
-  // distances / so, residual layers: bfloat16 64 x 2048 x 2048 6.8 / 6.5, 128 x 2048 x
-  // 2048 9.9 / 9.4, 128 x 5120 x 2048 20.7 / 20.1; int8 64 x 2048 x 2048 5.6 / 5.4; but
-  // int8 128 x 2048 x 4208, of four tiles, 13.5 / 14.1.)
-  constexpr bool kConstant = NJ > 0 && NT == 4;
+  // (kConstant: where this wavefront's first tiles lie; the others follow at constant
+  // distances, which the loads take as offsets: fewer instructions to fetch, which shows in
+  // a model's step, where each kernel's code is new to a CU (generation of 64 requests with
+  // layers of 1024 and 2816 inputs 36.1 -> 35.8 ms).  With 8 or 20 pairs and fewer than four
+  // column tiles the loads then bunch up, and addresses formed between the products are
+  // better, in a step too (beam search of the xl model in int8 159.9 -> 157.5 ms): us,
+  // constant / so, bfloat16 64 x 2048 x 2048 6.8 / 6.5, 128 x 2048 x 2048 9.9 / 9.4, 128 x
+  // 5120 x 2048 20.7 / 20.1; int8 64 x 2048 x 2048 5.6 / 5.4; four tiles, int8 128 x 2048 x
+  // 4208, 13.5 / 14.1.)
+  constexpr bool kConstant = NJ > 0 && (NT == 4 || (NJ != 8 && NJ != 20));
   const char* w_first = wbase + (size_t)wave * 2 * TB;
   const bf16_t* a_first[MP];
 #pragma unroll
