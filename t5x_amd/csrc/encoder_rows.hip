@@ -11,8 +11,8 @@
 // positions: 12 layers of width 768, 32 texts of 128 to 512 tokens 4.27 -> 3.41 ms; 24
 // of width 1024, 7 of 400 to 1031 8.56 -> 6.61 ms.
 // The two kernels last 16 us together at 32 x 512 (131 KB of tokens), 14 at 1 x 20 and 23 at
-// 1000 x 128: the first about 11 of them, bound by its threads' atomics on three words of
-// LDS, 256 on each, one after the other; the second by its launch.
+// 1000 x 128.  What bounds them: a launch each, and three atomics of 256 threads on one word
+// of LDS each (token_mask_kernel, which reads as much and has one, lasts 4.4 us).
 #include "common.h"
 
 namespace t5d {
