@@ -758,10 +758,17 @@ window_step_kernel(WinArgs g) {
       }
     }
   }
-  if (holds_new && lane < 2 * LPR)
-    *reinterpret_cast<uint4*>((lane < LPR ? K : V) + (size_t)(i % a.ring) * HP +
-                              8 * vpiece) =
-        *reinterpret_cast<const uint4*>(s_new[lane < LPR ? 0 : 1] + 8 * vpiece);
+  if (holds_new) {  // (element by element: a ring may start anywhere)
+    const size_t row = (size_t)(i % a.ring) * HP;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int d = lane + 64 * u;
+      if (d < HP) {
+        K[row + d] = s_new[0][d];
+        V[row + d] = s_new[1][d];
+      }
+    }
+  }
   // (the new value, by the wavefront that has its weight alone: it may be infinite, and
   // nothing times that is not nothing)
   if (holds_new && vsub == 0) {

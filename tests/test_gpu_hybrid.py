@@ -410,6 +410,20 @@ def test_window_attention_rings_that_start_between_16_byte_pieces(variant):
   assert all(bool((f[:4] == 7.0).all()) for f in flat)
 
 
+@pytest.mark.parametrize('H,G,D,Dv', [(6, 2, 48, 40), (3, 1, 20, 30), (2, 2, 200, 256)])
+def test_window_attention_steps_on_rings_that_start_between_16_byte_pieces(H, G, D, Dv):
+  from t5x_amd import _lib
+  a = Attention(torch.bfloat16, H, G, D, Dv, 30, 2, 35, 100)
+  flat = [torch.full((r.numel() + 8,), 7.0, dtype=r.dtype, device='cuda')
+          for r in a.rings]
+  a.rings = [f[4:-4].view_as(r) for f, r in zip(flat, a.rings)]
+  a.a.key_ring, a.a.value_ring = (_lib.ptr(r) for r in a.rings)
+  x = a.sequence(90)
+  got = np.concatenate([a.run([(1, at)], [x[at:at + 1]], 1) for at in range(90)])
+  assert rel(got, a.oracle(x)) < 1e-2
+  assert all(bool((f[:4] == 7.0).all() and (f[-4:] == 7.0).all()) for f in flat)
+
+
 @pytest.mark.parametrize('bias,sink,norms', [(False, True, True),
                                              (True, False, True),
                                              (True, True, False)])
