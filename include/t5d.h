@@ -347,6 +347,12 @@ int t5d_encoder_rows(void* stream, const int64_t* tokens, int B, int E, int32_t*
                      int32_t* odd, int32_t* first, int32_t* ids, int32_t* row_of,
                      int32_t* at, int32_t* summary);
 
+/* The same, and order [B]: the texts from the longest to the shortest. */
+int t5d_encoder_rows_ordered(void* stream, const int64_t* tokens, int B, int E,
+                             int32_t* len, int32_t* odd, int32_t* first, int32_t* ids,
+                             int32_t* row_of, int32_t* at, int32_t* summary,
+                             int32_t* order);
+
 /* Which positions of tokens [B, E] hold a token > 0: bits [B, (E + 31) / 32], bit e % 32
  * of word e / 32, and last [B], the last such position + 1 (0: none), as
  * t5d_encoder_attention takes them. */
@@ -366,6 +372,16 @@ int t5d_encoder_attention_rows(void* stream, const void* q, const void* k,
                                const int32_t* enc_len, const int32_t* first, int most,
                                void* out, int B, int H, int E, int Ep, int q_stride,
                                int k_stride);
+
+/* The same with what helps it spread over the chip and changes no result: the texts' order
+ * (t5d_encoder_rows_ordered; null: as they stand in the batch) and how many rows there are
+ * (first[B]; 0: not known). */
+int t5d_encoder_attention_ordered(void* stream, const void* q, const void* k,
+                                  const void* v_t, const void* rel_bias,
+                                  const int32_t* enc_len, const int32_t* first,
+                                  const int32_t* order, int rows, int most, void* out,
+                                  int B, int H, int E, int Ep, int q_stride,
+                                  int k_stride);
 
 /* The same attention in float32 (the dtype of the exactness tests), straight
  * from the fused projection: qkv [B*E, 3*H*64] holds q | k | v per row;

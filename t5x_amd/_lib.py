@@ -238,9 +238,12 @@ _SIGNATURES = {
                                               c_int, c_int, c_int, c_int,
                                               c_int, c_int, c_int]),
     't5d_encoder_rows': (c_int, [_P, _P, c_int, c_int] + [_P] * 7),
+    't5d_encoder_rows_ordered': (c_int, [_P, _P, c_int, c_int] + [_P] * 8),
     't5d_token_mask': (c_int, [_P, _P, c_int, c_int, _P, _P]),
     't5d_encoder_attention_rows': (c_int, [_P] * 7 + [c_int, _P] +
                                    [c_int] * 6),
+    't5d_encoder_attention_ordered': (c_int, [_P] * 8 + [c_int, c_int, _P] +
+                                      [c_int] * 6),
     't5d_encoder_attention_f32': (c_int, [_P, _P, _P, _P, _P, _P, c_int,
                                           c_int, c_int]),
     't5d_gemm_rows': (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int64, c_int,

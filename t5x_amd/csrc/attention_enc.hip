@@ -36,6 +36,7 @@ struct EncAttnArgs {
   const int32_t* first;   // ROWS kernels: [B + 1], rows first[b] .. first[b + 1] are
                           // text b's instead of b * E .. (b + 1) * E (t5d_encoder_rows:
                           // every position below len, then one or more of padding)
+  const int32_t* order;   // ROWS kernels, optional: [B] the texts, longest first
   bf16_t* out;        // [B*E, H*64]
   int B, H, E, Ep, q_stride, k_stride;
 };
@@ -284,14 +285,23 @@ enc_attn_short_kernel(EncAttnArgs a) {
 // exact zero) and a padded query scores 0 with every key that exists (it attends
 // uniformly), both in tiles that hold one of the two only; a wavefront of padded
 // queries alone forms no scores.
+// Which key a matrix row is follows from what the second product wants: rows 4 g + i of
+// tiles 2 kb and 2 kb + 1 are keys 8 g + i and 8 g + 4 + i of their 32, so a lane's
+// weights are those of 8 keys in a row and V^T comes in one 16-byte read, as it stands.
+// (With keys in their order it came in two reads of 8 bytes and 24 moves per tile.)  Of two
+// tiles of queries the second holds those 4 further on, so that both share bias entries.
 // What bounds it: vector instructions (~260 per tile and wavefront of 32 queries: the
 // two roundings of a score, its exponential) against 32 matrix instructions; 49 KB of
-// LDS let three workgroups share a CU.  Measured, us, beside the kernels that were here
-// before (up to 512 positions all scores in registers as above, two passes beyond):
+// LDS let three workgroups share a CU.  Then how evenly workgroups fall on the CUs: they
+// last as long as their text, so where the texts' order is given the longest start first.
+// Measured, us, beside the kernels that were here first (up to 512 positions all scores in
+// registers as above, two passes beyond) and keys in their order, texts in theirs:
 //   7 x 16 heads x 1032 (400 and more valid)   180 -> 71.4
+//     rows of 7 x 16 x 1031 (400 and more)            49.5 -> 41.6
 //   1 x 12 x 2048                              158 -> 47.1
-//   64 x 16 x 512 (all valid)                  261 -> 159
+//   64 x 16 x 512 (all valid)                  261 -> 140 -> 129
 //   32 x 12 x 512 (200 and more)              84.6 -> 59.2
+//     rows of 32 x 12 x 512 (128 and more)            51.2 -> 41.1 (45.4 without the order)
 //   256 x 12 x 66 / 96 / 128 (half and more)  48.1 / 48.7 / 55.3 -> 39.3 / 41.6 / 46.5
 //   1 x 12 x 128                               6.6 -> 4.9
 // The line to the kernel above lies where its one block of keys ends.  Below, the one
@@ -306,16 +316,17 @@ __global__ void __launch_bounds__(256, 3)
 enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   constexpr int KB = 64, QW = 16 * MT;  // keys per tile, queries per wavefront
   __shared__ uint4 s_k0[512], s_v0[512], s_k1[512], s_v1[512];
-  // 16 entries before the table (zeros: queries past the end, which are not stored but
-  // do decide with the others of their wavefront when maxima are raised) and 64 behind
-  // it (keys past the end, whose scores are replaced before they are looked at)
+  // 16 entries before the table (zeros, for queries past the end, which are not stored)
+  // and 64 behind it (keys past the end, whose scores are replaced before they are looked
+  // at)
   __shared__ float s_bias[16 + 2 * kMaxEncLen + 64];
   __shared__ uint32_t s_valid[kMaxEncLen / 32 + 2];
   // consecutive block ids go round-robin over the 8 XCDs: the tiles of one (item,
   // head) are 8 apart
   const int pair = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / tiles);
-  const int b = pair / a.H, h = pair - b * a.H;
-  if (b >= a.B) return;
+  const int at_b = pair / a.H, h = pair - at_b * a.H;
+  if (at_b >= a.B) return;
+  const int b = ROWS && a.order ? a.order[at_b] : at_b;
   const int tile = (blockIdx.x >> 3) % tiles;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -335,10 +346,10 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   for (int i = 0; i < 2; ++i) {
     const int f = (wave * 2 + i) * 64 + lane;
     k_row[i] = f >> 3;
-    k_piece[i] = 16 * ((f & 7) ^ ((k_row[i] >> 1) & 7));
+    k_piece[i] = 16 * ((f & 7) ^ (((k_row[i] >> 1) & 1) | ((k_row[i] >> 2) & 6)));
     v_blk[i] = f >> 8;
     const int d = (f >> 2) & 63;
-    v_off[i] = d * 64 + 16 * ((f & 3) ^ ((d >> 2) & 3));
+    v_off[i] = d * 64 + 16 * ((f & 3) ^ (3 * ((d >> 3) & 1)));
   }
   const auto fetch = [&](int jt, uint4* sk, uint4* sv) {
 #pragma unroll
@@ -358,11 +369,26 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   };
   fetch(0, s_k0, s_v0);
 
-  if (threadIdx.x < 16) s_bias[threadIdx.x] = 0.f;
-  for (int i = threadIdx.x; i < 2 * E - 1; i += 256)
-    s_bias[16 + i] = bf16_to_f32(a.bias[(size_t)h * (2 * E - 1) + i]);
   int n = a.len[b];
   n = n < 0 ? 0 : (n > E ? E : n);
+  // The part of the table that these queries and keys reach (a second tile's queries lie
+  // 4 further on), 4 entries per thread requested at a time.
+  if (threadIdx.x < 16) s_bias[threadIdx.x] = 0.f;
+  {
+    const int q_first = tile * 4 * QW;
+    const int q_last = min(q_first + 4 * QW, rows) - 1;
+    const int lo = max(E - 1 - q_last - 4, 0);
+    const int hi = min(E - 1 - q_first + ((ROWS ? n : E) + KB - 1) / KB * KB, 2 * E - 1);
+    const bf16_t* table = a.bias + (size_t)h * (2 * E - 1);
+    for (int i = lo + threadIdx.x; i < hi; i += 4 * 256) {
+      bf16_t v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = table[min(i + 256 * j, hi - 1)];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (i + 256 * j < hi) s_bias[16 + i + 256 * j] = bf16_to_f32(v[j]);
+    }
+  }
   const int words = (E + 31) >> 5;
   for (int i = threadIdx.x; i < kMaxEncLen / 32 + 2; i += 256) {
     const int left = n - 32 * i;
@@ -372,11 +398,13 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
     s_valid[i] = prefix;
   }
   const int q0 = (tile * 4 + wave) * QW;
+  // (of two tiles of queries the second holds those 4 further on)
+  const int q_at = MT == 2 ? q0 + 8 * (l16 >> 2) + (l16 & 3) : q0 + l16;
   FragE qb[MT][2];
   int qi[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    qi[mt] = min(q0 + 16 * mt + l16, rows - 1);  // past the end: not stored
+    qi[mt] = min(q_at + 4 * mt, rows - 1);  // past the end: not stored
 #pragma unroll
     for (int c = 0; c < 2; ++c)
       qb[mt][c].u = *reinterpret_cast<const uint4*>(
@@ -409,6 +437,10 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
   my_keys = __builtin_amdgcn_readfirstlane(my_keys);
   wg_keys = __builtin_amdgcn_readfirstlane(wg_keys);
 
+  bool q_valid[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+    q_valid[mt] = (s_valid[qi[mt] >> 5] >> (qi[mt] & 31)) & 1u;
   float mx[MT], l[MT];
   f32x4_e oc[4][MT];
 #pragma unroll
@@ -418,8 +450,8 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) oc[dt][mt] = (f32x4_e){0.f, 0.f, 0.f, 0.f};
   }
-  const int k_read = l16 * 8, k_x = (l16 >> 1) & 7;
-  const int v_read = l16 * 64 + 16 * ((gq >> 1) ^ ((l16 >> 2) & 3)) + 8 * (gq & 1);
+  const int k_read = (8 * (l16 >> 2) + (l16 & 3)) * 8, k_x = l16 >> 1;
+  const int v_read = l16 * 4 + (gq ^ (3 * (l16 >> 3)));
   const auto attend = [&](int jt, const uint4* sk, const uint4* sv) {
     if (jt >= my_keys) return;
     FragE pb[2][MT];
@@ -430,7 +462,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
         uint32_t w[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int key = jt + 32 * kb + 16 * (e >> 1) + 4 * gq + 2 * (e & 1);
+          const int key = jt + 32 * kb + 8 * gq + 2 * e;
           w[e] = (key < E_here ? 0x3F80u : 0u) | (key + 1 < E_here ? 0x3F800000u : 0u);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
@@ -447,7 +479,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        kf[t][c].u = sk[16 * t * 8 + k_read + ((4 * c + gq) ^ k_x)];
+        kf[t][c].u = sk[(32 * (t >> 1) + 4 * (t & 1)) * 8 + k_read + ((4 * c + gq) ^ k_x)];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -460,19 +492,21 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
         for (int mt = 0; mt < MT; ++mt)
           s[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][c].v, qb[mt][c].v,
                                                              s[t][mt], 0, 0, 0);
-    // bias by key - query: 16 keys further on is 16 queries further back
-    const float* near = s_bias + 16 + (E - 1) - min(qi[0], E - 1) + jt + 4 * gq;
-    float bias[5][4];
+    // bias by key - query: 4 keys further on is 4 queries further back
+    const float* near = s_bias + 16 + (E - 1) - min(qi[0], E - 1) + jt + 8 * gq;
+    float bias[2][MT + 1][4];
 #pragma unroll
-    for (int t = 0; t < 5; ++t)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        bias[t][i] = near[16 * (t - 1) + i];
+      for (int j = 0; j <= MT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          bias[kb][j][i] = near[32 * kb + 4 * (j - (MT - 1)) + i];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const float* add = bias[t - mt + 1];
+        const float* add = bias[t >> 1][(t & 1) - mt + MT - 1];
         const uint32_t r01 = pack_bf16x2(s[t][mt][0], s[t][mt][1]);
         const uint32_t r23 = pack_bf16x2(s[t][mt][2], s[t][mt][3]);
         const uint32_t x01 =
@@ -485,22 +519,29 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
         s[t][mt][3] = bf16hi_to_f32(x23);
       }
     const uint32_t v0 = s_valid[jt >> 5], v1 = s_valid[(jt >> 5) + 1];
-    if (!my_valid || (v0 & v1) != 0xffffffffu) {
+    if (!my_valid) {  // a padded query scores 0
       asm volatile("");  // (a branch: the compiler would select in every tile)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const bool q_valid = (s_valid[qi[mt] >> 5] >> (qi[mt] & 31)) & 1u;
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int key = 16 * t + 4 * gq + i;
-            const bool exists = jt + key < E_here;
-            const bool ok = ((t < 2 ? v0 : v1) >> (key & 31)) & 1u;
-            const float x = q_valid ? s[t][mt][i] : 0.f;
-            s[t][mt][i] = (q_valid ? ok : exists) ? x : -INFINITY;
-          }
-      }
+          for (int i = 0; i < 4; ++i) s[t][mt][i] = q_valid[mt] ? s[t][mt][i] : 0.f;
+    }
+    if ((v0 & v1) != 0xffffffffu) {  // with keys that it does weigh, if they exist
+      asm volatile("");
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = 32 * (t >> 1) + 8 * gq + 4 * (t & 1) + i;
+          const bool exists = jt + key < E_here;
+          // (of given rows the keys below E_here are the valid ones)
+          const bool ok = ROWS ? exists : ((t < 2 ? v0 : v1) >> (key & 31)) & 1u;
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+            s[t][mt][i] = (q_valid[mt] ? ok : exists) ? s[t][mt][i] : -INFINITY;
+        }
     }
     bool raise = false;
     float top[MT];
@@ -518,14 +559,18 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
       asm volatile("");
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const float to = fmaxf(mx[mt], top[mt]);
+        // (of those queries alone whose own score asks for it: what a query gets does
+        // not depend on the ones beside it)
+        const float to = top[mt] > mx[mt] + kMaxSlack ? top[mt] : mx[mt];
         const float alpha = __builtin_amdgcn_exp2f(mx[mt] - to);
         mx[mt] = to;
         l[mt] *= alpha;
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < 4; ++dt) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) oc[dt][mt][i] *= alpha;
+          asm volatile("" : "+v"(oc[dt][mt]));
+        }
       }
     }
 #pragma unroll
@@ -553,10 +598,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
       FragE va[4];
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) {
-        const char* v = reinterpret_cast<const char*>(sv) + kb * 4096 + dt * 1024;
-        const uint2 x = *reinterpret_cast<const uint2*>(v + v_read);
-        const uint2 y = *reinterpret_cast<const uint2*>(v + (v_read ^ 32));
-        va[dt].u = make_uint4(x.x, x.y, y.x, y.y);
+        va[dt].u = sv[kb * 256 + dt * 64 + v_read];
       }
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
@@ -590,7 +632,7 @@ enc_attn_tile_kernel(EncAttnArgs a, int tiles) {
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     float sum = rows_sum(l[mt]);
-    const int q = q0 + 16 * mt + l16;
+    const int q = q_at + 4 * mt;
     if (q >= rows) continue;
     // (such a query's maximum is 0, or was never raised: its keys weigh 1)
     if (ROWS && n < E && q >= n) {
@@ -703,7 +745,21 @@ enc_attn_f32_kernel(EncAttnF32Args a) {
 //   16 x 12 x 512, 200 and more (1536)            37.8 / 36.9
 //   32 x 12 x 200, 80 and more (1536)             20.0 / 22.6
 //   7 x 16 x 1032, 400 and more (1904)            71.5 / 73.8
-static bool one_pass_64(int B, int H, int E) {
+// Over given rows (there are `rows` of them) as many workgroups count as hold some, and
+// padding is one row of a text: 64 pay up to more of them, and longer where texts are long
+// (128 / 64, workgroups of 64):
+//   3 x 16 heads x 1031, 257 and more (480)       27.9 / 20.5
+//   17 x 12 x 512, 128 and more (1176)            28.4 / 26.3
+//   7 x 16 x 1031, 400 and more (1296)            45.5 / 41.6
+//   10 x 16 x 1500, 375 and more (2032)           72.9 / 69.5
+//   31 x 12 x 512, 128 and more (2064)            39.5 / 41.8
+//   15 x 16 x 1031, 257 and more (2560)           68.7 / 72.4
+//   70 x 12 x 128, 32 and more (1404)             16.7 / 18.1
+//   45 x 12 x 200, 50 and more (1152)             19.3 / 21.0
+//   45 x 16 x 200, 50 and more (1536)             22.5 / 26.9
+static bool one_pass_64(int B, int H, int E, int rows) {
+  if (rows > 0)
+    return (int64_t)H * (rows / 64 + B / 2) <= (rows >= (int64_t)B * 192 ? 1800 : 1000);
   return (int64_t)B * H * ((E + 63) / 64) <= 1024;
 }
 
@@ -725,8 +781,8 @@ extern "C" int t5d_encoder_attention(void* stream, const void* q, const void* k,
 static int encoder_attention(void* stream, const void* q, const void* k, const void* v_t,
                              const void* rel_bias, const int32_t* enc_len,
                              const uint32_t* valid_bits, const int32_t* first,
-                             int most, void* out, int B, int H, int E, int Ep,
-                             int q_stride, int k_stride) {
+                             const int32_t* order, int rows, int most, void* out,
+                             int B, int H, int E, int Ep, int q_stride, int k_stride) {
   T5D_REQUIRE(q && k && v_t && rel_bias && enc_len && out, T5D_EINVAL,
               "t5d_encoder_attention: null pointer");
   T5D_REQUIRE(B > 0 && H > 0 && E > 0 && Ep >= E && Ep % 32 == 0,
@@ -749,7 +805,7 @@ static int encoder_attention(void* stream, const void* q, const void* k, const v
   EncAttnArgs a;
   a.q = (const bf16_t*)q; a.k = (const bf16_t*)k; a.vt = (const bf16_t*)v_t;
   a.bias = (const bf16_t*)rel_bias; a.len = enc_len; a.out = (bf16_t*)out;
-  a.valid = valid_bits; a.first = first;
+  a.valid = valid_bits; a.first = first; a.order = order;
   a.B = B; a.H = H; a.E = E; a.Ep = Ep; a.q_stride = q_stride; a.k_stride = k_stride;
   if (E <= kShortEnc) {
     if (first)
@@ -759,7 +815,7 @@ static int encoder_attention(void* stream, const void* q, const void* k, const v
       hipLaunchKernelGGL(enc_attn_short_kernel<false>, dim3(1, H, B), dim3(256), 0,
                          as_stream(stream), a);
   } else {
-    const bool low = one_pass_64(B, H, most);
+    const bool low = one_pass_64(B, H, most, rows);
     const int tiles = low ? (most + 63) / 64 : (most + 127) / 128;
     const dim3 groups(((unsigned)B * H + 7) / 8 * 8 * tiles);
 #define T5D_ENC(MT_, ROWS_)                                                       \
@@ -785,19 +841,28 @@ extern "C" int t5d_encoder_attention_variant(
               "t5d_encoder_attention_variant: variant %d (0, 1, and 2 where "
               "E <= 512)",
               variant);
-  return encoder_attention(stream, q, k, v_t, rel_bias, enc_len, valid_bits, nullptr, E,
-                           out, B, H, E, Ep, q_stride, k_stride);
+  return encoder_attention(stream, q, k, v_t, rel_bias, enc_len, valid_bits, nullptr,
+                           nullptr, 0, E, out, B, H, E, Ep, q_stride, k_stride);
 }
 
 extern "C" int t5d_encoder_attention_rows(
     void* stream, const void* q, const void* k, const void* v_t, const void* rel_bias,
     const int32_t* enc_len, const int32_t* first, int most, void* out, int B, int H,
     int E, int Ep, int q_stride, int k_stride) {
-  T5D_REQUIRE(first && most > 0 && most <= (E + 3) / 4 * 4, T5D_EINVAL,
-              "t5d_encoder_attention_rows: first %p, at most %d rows of a text of %d",
-              (const void*)first, most, E);
-  return encoder_attention(stream, q, k, v_t, rel_bias, enc_len, nullptr, first, most,
-                           out, B, H, E, Ep, q_stride, k_stride);
+  return t5d_encoder_attention_ordered(stream, q, k, v_t, rel_bias, enc_len, first,
+                                       nullptr, 0, most, out, B, H, E, Ep, q_stride,
+                                       k_stride);
+}
+
+extern "C" int t5d_encoder_attention_ordered(
+    void* stream, const void* q, const void* k, const void* v_t, const void* rel_bias,
+    const int32_t* enc_len, const int32_t* first, const int32_t* order, int rows,
+    int most, void* out, int B, int H, int E, int Ep, int q_stride, int k_stride) {
+  T5D_REQUIRE(first && most > 0 && most <= (E + 3) / 4 * 4 && rows >= 0, T5D_EINVAL,
+              "t5d_encoder_attention_rows: first %p, %d rows, at most %d of a text of %d",
+              (const void*)first, rows, most, E);
+  return encoder_attention(stream, q, k, v_t, rel_bias, enc_len, nullptr, first, order,
+                           rows, most, out, B, H, E, Ep, q_stride, k_stride);
 }
 
 extern "C" int t5d_encoder_attention_f32(void* stream, const float* qkv,

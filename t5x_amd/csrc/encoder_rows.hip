@@ -46,20 +46,24 @@ encoder_lengths_kernel(const int64_t* __restrict__ tokens, int32_t* __restrict__
 }
 
 // One workgroup per text: its rows' ids, the row of every position, the position
-// (text << 12 | position) of every 4 rows; the last also sums up for the host.
+// (text << 12 | position) of every 4 rows, its place by length; the last also sums up for
+// the host.
 __global__ void __launch_bounds__(256)
 encoder_rows_kernel(const int64_t* __restrict__ tokens, const int32_t* __restrict__ len,
                     const int32_t* __restrict__ odd, int32_t* __restrict__ first,
                     int32_t* __restrict__ ids, int32_t* __restrict__ row_of,
-                    int32_t* __restrict__ at, int32_t* __restrict__ summary, int B,
-                    int E) {
-  __shared__ int s_first, s_most, s_odd;
-  if (threadIdx.x == 0) s_first = s_most = s_odd = 0;
+                    int32_t* __restrict__ at, int32_t* __restrict__ summary,
+                    int32_t* __restrict__ order, int B, int E) {
+  __shared__ int s_first, s_most, s_odd, s_longer;
+  if (threadIdx.x == 0) s_first = s_most = s_odd = s_longer = 0;
   __syncthreads();
-  const int b = blockIdx.x;
-  int before = 0, most = 0, any = 0;
-  for (int i = threadIdx.x; i <= b; i += 256) {
-    const int rows = rows_of_text(len[i], E);
+  const int b = blockIdx.x, n = len[b];
+  int before = 0, most = 0, any = 0, longer = 0;
+  for (int i = threadIdx.x; i < (order ? B : b + 1); i += 256) {
+    const int other = len[i];
+    longer += other > n || (other == n && i < b);
+    if (i > b) continue;
+    const int rows = rows_of_text(other, E);
     if (i < b) before += rows;
     most = max(most, rows);
     any |= odd[i];
@@ -67,10 +71,12 @@ encoder_rows_kernel(const int64_t* __restrict__ tokens, const int32_t* __restric
   atomicAdd(&s_first, before);
   atomicMax(&s_most, most);
   atomicOr(&s_odd, any);
+  atomicAdd(&s_longer, longer);
   __syncthreads();
-  const int r0 = s_first, n = len[b], rows = rows_of_text(n, E);
+  const int r0 = s_first, rows = rows_of_text(n, E);
   if (threadIdx.x == 0) {
     first[b] = r0;
+    if (order) order[s_longer] = b;
     if (b == B - 1) {
       first[B] = r0 + rows;
       summary[0] = r0 + rows;
@@ -129,6 +135,14 @@ extern "C" int t5d_encoder_rows(void* stream, const int64_t* tokens, int B, int 
                                 int32_t* len, int32_t* odd, int32_t* first,
                                 int32_t* ids, int32_t* row_of, int32_t* at,
                                 int32_t* summary) {
+  return t5d_encoder_rows_ordered(stream, tokens, B, E, len, odd, first, ids, row_of, at,
+                                  summary, nullptr);
+}
+
+extern "C" int t5d_encoder_rows_ordered(void* stream, const int64_t* tokens, int B, int E,
+                                        int32_t* len, int32_t* odd, int32_t* first,
+                                        int32_t* ids, int32_t* row_of, int32_t* at,
+                                        int32_t* summary, int32_t* order) {
   T5D_REQUIRE(tokens && len && odd && first && ids && row_of && at && summary,
               T5D_EINVAL, "t5d_encoder_rows: null pointer");
   T5D_REQUIRE(B > 0 && E > 0, T5D_EINVAL, "t5d_encoder_rows: B=%d E=%d", B, E);
@@ -137,7 +151,7 @@ extern "C" int t5d_encoder_rows(void* stream, const int64_t* tokens, int B, int 
   hipLaunchKernelGGL(encoder_lengths_kernel, dim3(B), dim3(256), 0, as_stream(stream),
                      tokens, len, odd, E);
   hipLaunchKernelGGL(encoder_rows_kernel, dim3(B), dim3(256), 0, as_stream(stream),
-                     tokens, len, odd, first, ids, row_of, at, summary, B, E);
+                     tokens, len, odd, first, ids, row_of, at, summary, order, B, E);
   T5D_CHECK_LAUNCH("t5d_encoder_rows");
   return T5D_OK;
 }

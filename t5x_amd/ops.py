@@ -548,13 +548,13 @@ class EncoderRows:
     _chk(tokens, 'tokens', torch.int64, 2)
     self.B, self.E = B, E = tokens.shape
     self.positions = E4 = (E + 3) // 4 * 4
-    sizes = [B, B, B + 1, B * E4, B * E, B * E4 // 4, 3]
-    (self.len, odd, self.first, self._ids, self.row_of, self._at,
-     summary) = torch.empty(sum(sizes), dtype=torch.int32,
-                            device=tokens.device).split(sizes)
-    _lib.call('t5d_encoder_rows', _s(), tokens.data_ptr(), B, E,
+    sizes = [B, B, B + 1, B * E4, B * E, B * E4 // 4, 3, B]
+    (self.len, odd, self.first, self._ids, self.row_of, self._at, summary,
+     self.order) = torch.empty(sum(sizes), dtype=torch.int32,
+                               device=tokens.device).split(sizes)
+    _lib.call('t5d_encoder_rows_ordered', _s(), tokens.data_ptr(), B, E,
               *(t.data_ptr() for t in (self.len, odd, self.first, self._ids,
-                                       self.row_of, self._at, summary)))
+                                       self.row_of, self._at, summary, self.order)))
     self.M, self.most, any_odd = summary.tolist()
     self.odd = bool(any_odd)
     self.ids, self.at = self._ids[:self.M], self._at[:self.M // 4]
@@ -645,10 +645,10 @@ def encoder_attention_rows(q, k, v_t, rel_bias, rows):
       raise ValueError(f'{name} must be a [{rows.M}, H*64] bfloat16 view with unit '
                        f'column stride, got {tuple(t.shape)}')
   out = torch.empty((rows.M, H * 64), dtype=torch.bfloat16, device=v_t.device)
-  _lib.call('t5d_encoder_attention_rows', _s(), q.data_ptr(), k.data_ptr(),
+  _lib.call('t5d_encoder_attention_ordered', _s(), q.data_ptr(), k.data_ptr(),
             v_t.data_ptr(), rel_bias.data_ptr(), rows.len.data_ptr(),
-            rows.first.data_ptr(), rows.most, out.data_ptr(), B, H, rows.positions,
-            blocks * 32, q.stride(0), k.stride(0))
+            rows.first.data_ptr(), rows.order.data_ptr(), rows.M, rows.most,
+            out.data_ptr(), B, H, rows.positions, blocks * 32, q.stride(0), k.stride(0))
   return out
 
 

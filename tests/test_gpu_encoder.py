@@ -946,6 +946,52 @@ def test_encoder_attention_over_rows_of_ragged_texts(ops, E, wide):
     assert bool(((mine[n:].double() - mean[b]).abs() <= bound).all()), (b, n)
 
 
+# (E, heads, shortest): workgroups of 128 queries and of 64, on both sides of the lines of
+# one_pass_64 for long texts and short ones
+@pytest.mark.parametrize('E,H,least,queries', [
+    (257, 32, 200, 64), (257, 40, 200, 128), (1031, 9, 900, 64), (1031, 12, 900, 128),
+    (130, 40, 1, 64), (130, 64, 1, 128), (66, 64, 0, 64), (66, 96, 0, 128)])
+def test_encoder_attention_in_the_order_of_the_texts(ops, E, H, least, queries):
+  """t5d_encoder_rows_ordered lists the texts from the longest on; attention with and
+  without the list has the same bits, and tokens those of the kernel over every position,
+  whichever number of queries a workgroup takes."""
+  from t5x_amd import _lib
+  rs = np.random.RandomState(E + H)
+  B, E4 = 12, (E + 3) // 4 * 4
+  lens = rs.randint(least, E + 1, size=B)
+  lens[3], lens[5], lens[7] = E, lens[4], E
+  tokens = torch.zeros((B, E), dtype=torch.int64, device='cuda')
+  for b, n in enumerate(lens):
+    tokens[b, :n] = 7
+  rows = ops.EncoderRows(tokens)
+  assert rows.order.tolist() == sorted(range(B), key=lambda b: (-lens[b], b))
+  limit = 1800 if rows.M >= B * 192 else 1000
+  assert (H * (rows.M // 64 + B // 2) <= limit) == (queries == 64)
+  first, Ep = rows.first.tolist(), (E4 + 31) // 32 * 32
+  gen = torch.Generator(device='cuda')
+  gen.manual_seed(E)
+  rnd = lambda *shape: torch.randn(shape, generator=gen, device='cuda').bfloat16()
+  q, k = 0.3 * rnd(B, E4, H * 64), rnd(B, E4, H * 64)
+  v = torch.zeros((B, H, 64, Ep), dtype=torch.bfloat16, device='cuda')
+  v[..., :E4] = rnd(B, H, 64, E4)
+  for b in range(B):
+    v[b, ..., first[b + 1] - first[b]:] = 0
+  v = ops.tile_cross_value(v)
+  rel = rnd(H, 2 * E4 - 1)
+  pick = lambda x: torch.cat([x[b, :first[b + 1] - first[b]] for b in range(B)])
+  qr, kr = pick(q), pick(k)
+  got = ops.encoder_attention_rows(qr, kr, v, rel, rows)
+  plain = torch.empty_like(got)
+  _lib.call('t5d_encoder_attention_ordered', ops._s(), qr.data_ptr(), kr.data_ptr(),
+            v.data_ptr(), rel.data_ptr(), rows.len.data_ptr(), rows.first.data_ptr(),
+            None, rows.M, rows.most, plain.data_ptr(), B, H, E4, Ep, H * 64, H * 64)
+  assert torch.equal(got, plain)
+  want = ops.encoder_attention(q.view(B * E4, -1), k.view(B * E4, -1), v, rel,
+                               dev(lens.astype(np.int32))).view(B, E4, -1)
+  for b, n in enumerate(lens):
+    assert torch.equal(got[first[b]:first[b] + n], want[b, :n]), b
+
+
 def test_encoder_of_many_ragged_texts():
   """The whole encoder where its attention takes two tiles of queries per wavefront."""
   from t5x_amd import encoder, network
