@@ -38,6 +38,7 @@ struct RecArgs {
   float *wq, *wk, *wv, *wbeta, *wo;
   float* wchunk;  // chunked portions: the chunks' operands (ChunkLayout)
   int chunks;     // of the longest portion: the chunk kernel's grid
+  int32_t* order;  // chunked portions, or null: [S] the sequences, longest first
   int C;  // channels of the convolution
   const int32_t* gate;
 };
@@ -428,11 +429,25 @@ recurrence_chunk_kernel(RecArgs g) {
   T5D_GATED(g.gate);
   const t5d_recurrence& a = g.a;
   const int chunk = blockIdx.x, h = blockIdx.y, seq = blockIdx.z;
-  const int off = g.b.seq_off[seq];
-  const int n = min(C, g.b.seq_off[seq + 1] - off - chunk * C);
+  const int off = g.b.seq_off[seq], len = g.b.seq_off[seq + 1] - off;
+  const int tid = threadIdx.x;
+  if (g.order && chunk == 0 && h == 0) {
+    // where the sequence stands by its length, for the chain kernel
+    __shared__ int s_longer;
+    if (tid == 0) s_longer = 0;
+    __syncthreads();
+    int longer = 0;
+    for (int i = tid; i < g.b.S; i += 256) {
+      const int other = g.b.seq_off[i + 1] - g.b.seq_off[i];
+      longer += other > len || (other == len && i < seq);
+    }
+    atomicAdd(&s_longer, longer);
+    __syncthreads();
+    if (tid == 0) g.order[s_longer] = seq;
+  }
+  const int n = min(C, len - chunk * C);
   if (n <= 0) return;
   const int m0 = off + chunk * C;
-  const int tid = threadIdx.x;
   const int vp = (a.Dv + 15) / 16 * 16, vs = vp + 4;
   if (a.taps == 0)
     chunk_columns<0, DP, T>(g, chunk, n, m0, h, seq, s_q, s_k, s_g, s_v, vp, vs);
@@ -679,69 +694,88 @@ recurrence_chunk_kernel(RecArgs g) {
   }
 }
 
-// Walks the chunks of one (sequence, head) for 16 value columns.  Each of 4
-// wavefronts holds NTW tiles of 16 channels x 16 columns of the state.
-// What bounds it: the chain of a step at one wavefront per SIMD where sequences are
-// few (24 dependent matrix products = 770 of its 1960 cycles, the exchange of partial
-// sums behind one barrier, the next step's first operands).  256 steps of 32
-// (sequence, head) pairs: 206 us with the delta rule, 153 without; 225 and 187 us
-// with the requests, their address arithmetic and the read-out in the chain's way and
-// a wait for every request each fourth step (at the head of the loop).
-template <int NTW, bool DELTA>
+// Walks the chunks of one (sequence, head) for 16 NC value columns.  Each of 4
+// wavefronts holds NTW tiles of 16 channels x 16 columns of the state per NC.
+// What bounds it where sequences are few: the chain of a step at one wavefront per SIMD (24
+// dependent matrix products = 770 of its 2000 cycles, the exchange of partial sums behind
+// one barrier, the requests).  Nothing that the state does not need stands in front of the
+// barrier; a read-out's parts wait for the next step's.  Where they are many: matrix
+// instructions and the operands' way into a CU, 24 KB per step that columns side by side
+// share, so two column tiles (NC = 2) go together once one alone has more than two
+// workgroups per CU (the line in launch_chunks); and how evenly the sequences fall on the
+// CUs, so the longest start first (RecArgs::order).  Chunk, chain and finish kernel together,
+// us, 8 heads of 128, delta rule / without, with the read-out in front of the barrier, one
+// column tile and sequences as they stand -> now:
+//   4 x 2048 tokens            213 -> 204    136 -> 132
+//   1 x 4096                   248 -> 244    163 -> 157
+//   40 of 3 to 611             281 -> 238    198 -> 162
+//   16 x 300                   120 -> 112     81 -> 76.5  (16 x 300 of 4 heads, one tile:
+//                               72 -> 72      50 -> 49.5)
+template <int NTW, bool DELTA, int NC>
 __global__ void __launch_bounds__(256, NTW <= 2 ? 2 : 1)
 recurrence_chain_kernel(RecArgs g) {
   constexpr int DP = 64 * NTW;
-  __shared__ float4 s_u[2][4][64];
-  __shared__ float4 s_o[2][4][64];
+  __shared__ float4 s_u[2][NC][4][64];
+  __shared__ float4 s_o[2][NC][4][64];
   T5D_GATED(g.gate);
   const t5d_recurrence& a = g.a;
   // The workgroups of one (sequence, head) read the same operands: consecutive
   // block ids go round-robin over the 8 XCDs, so theirs are 8 apart.
-  const int vp = (a.Dv + 15) / 16 * 16, vts = vp / 16;
+  const int vp = (a.Dv + 15) / 16 * 16, vts = (vp / 16 + NC - 1) / NC;
   const int pair = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / vts);
   if (pair >= a.H * g.b.S) return;
-  const int vt = (blockIdx.x >> 3) % vts, h = pair % a.H, seq = pair / a.H;
+  const int vt = NC * ((blockIdx.x >> 3) % vts), h = pair % a.H;
+  const int seq = g.order ? g.order[pair / a.H] : pair / a.H;
   const int off = g.b.seq_off[seq], len = g.b.seq_off[seq + 1] - off;
   if (len <= 0) return;
   const int start = g.b.seq_start[seq], slot = g.b.seq_slot[seq];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int x = lane & 15, g4 = lane >> 4;
-  const int col = 16 * vt + x;
-  const bool col_ok = col < a.Dv;
+  const int col = 16 * vt + x;  // and 16 further on
   const ChunkLayout lay(DP, vp);
   const int nc = (len + kChunk - 1) / kChunk;
 
   float* state = a.state + ((size_t)slot * a.H + h) * a.D * a.Dv + col;
-  f32x4_v st[NTW];
+  f32x4_v st[NC][NTW];
 #pragma unroll
-  for (int t = 0; t < NTW; ++t)
+  for (int n = 0; n < NC; ++n)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = 16 * (wave * NTW + t) + 4 * g4 + i;
-      st[t][i] = start > 0 && col_ok && d < a.D ? state[(size_t)d * a.Dv] : 0.f;
-    }
+    for (int t = 0; t < NTW; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * (wave * NTW + t) + 4 * g4 + i;
+        st[n][t][i] = start > 0 && col + 16 * n < a.Dv && d < a.D
+                          ? state[(size_t)d * a.Dv + 16 * n] : 0.f;
+      }
   const size_t row = (size_t)a.H * a.Dv;  // of the read-outs
   float* out = g.wo + (size_t)off * row + (size_t)h * a.Dv + col +
                (size_t)(4 * g4 + wave) * row;
 
   struct Operands {
-    float4 wk[NTW], qs[NTW], kh[NTW], pc[NTW], us;
-    float os;
+    float4 wk[NTW], qs[NTW], kh[NTW], pc[NTW], us[NC];
+    float os[NC];
   };
   // Operands: a uniform base per chunk, which stops at the last one, and offsets
-  // within a chunk that never change.
+  // within a chunk that never change.  (A column tile past the end has none: it takes the
+  // first one's, for columns that are not stored.)
   const size_t stride = (size_t)a.H * lay.size() * sizeof(float);
-  const char* next = reinterpret_cast<const char*>(
+  char* next = reinterpret_cast<char*>(
       g.wchunk + (chunk_base(off, seq) * a.H + h) * lay.size());
   int to_load = nc;  // chunks not yet requested
   const uint32_t at = (wave * NTW * 64 + lane) * 16;
   const uint32_t at_pc = (wave * NTW * 4 + g4) * 16;
   const uint32_t at_us = (vt * 64 + lane) * 16, at_os = at_us + 4 * wave;
-  const auto piece = [&](size_t of, uint32_t o) {
-    return *reinterpret_cast<const float4*>(next + 4 * of + o);
-  };
+  const uint32_t further = vt + 1 < vp / 16 ? 1024 : 0;
   auto load = [&](Operands& o) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (buffer descriptors are no host type)
+    // (the base moves with scalar additions)
+    const __amdgpu_buffer_rsrc_t chunk =
+        __builtin_amdgcn_make_buffer_rsrc(next, 0, 0x7fffffff, 0x00020000);
+    const auto piece = [&](size_t of, uint32_t o) {
+      return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                            chunk, (int)o, (int)(4 * of), 0));
+    };
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
       if (DELTA) o.wk[t] = piece(lay.wk(), at + 1024 * t);
@@ -749,76 +783,124 @@ recurrence_chain_kernel(RecArgs g) {
       o.kh[t] = piece(lay.kh(), at + 1024 * t);
       o.pc[t] = piece(lay.pc(), at_pc + 64 * t);
     }
-    o.us = piece(lay.us(), at_us);
-    // (only the row this wavefront stores is used)
-    o.os = *reinterpret_cast<const float*>(next + 4 * lay.os() + at_os);
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      o.us[n] = piece(lay.us(), at_us + n * further);
+      // (only the row this wavefront stores is used)
+      o.os[n] = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(
+                     chunk, (int)(at_os + n * further), (int)(4 * lay.os()), 0));
+    }
     next += --to_load > 0 ? stride : 0;
+#endif
   };
-  // A step: u (behind it the exchange of the wavefronts' parts), the read-out's
-  // product and the requests for a later chunk while the parts are on their way,
-  // the state's update, and the read-out behind its products.
+  // The read-out of a chunk, tokens 4 g + wave: its product's parts meet behind the barrier
+  // of the step after it.
+  float os[NC], y[NC][4];
+  const auto fetch_out = [&](int c) {
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        y[n][p] = reinterpret_cast<const float*>(&s_o[c & 1][n][p][lane])[wave];
+  };
+  const auto read_out = [&](int c) {
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      const float sum = (((os[n] + y[n][0]) + y[n][1]) + y[n][2]) + y[n][3];
+      if (kChunk * c + 4 * g4 + wave < len && col + 16 * n < a.Dv) out[16 * n] = sum;
+    }
+    out += kChunk * row;
+  };
+  // A step: u's product and the exchange of the wavefronts' parts; behind the barrier,
+  // while they are on their way, the requests for a later chunk and the read-out's
+  // product; then the state's update.
   auto step = [&](const Operands& o, Operands& later, int c) {
     const int buf = c & 1;
-    f32x4_v u = (f32x4_v){0.f, 0.f, 0.f, 0.f}, r = u;
     if (DELTA) {
+      f32x4_v u[NC];
+#pragma unroll
+      for (int n = 0; n < NC; ++n) u[n] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int t = 0; t < NTW; ++t) {
         const float wk[4] = {o.wk[t].x, o.wk[t].y, o.wk[t].z, o.wk[t].w};
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          u = __builtin_amdgcn_mfma_f32_16x16x4f32(wk[i], st[t][i], u, 0, 0, 0);
+#pragma unroll
+          for (int n = 0; n < NC; ++n)
+            u[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(wk[i], st[n][t][i], u[n], 0, 0, 0);
       }
-      s_u[buf][wave][lane] = make_float4(u[0], u[1], u[2], u[3]);
+#pragma unroll
+      for (int n = 0; n < NC; ++n)
+        s_u[buf][n][wave][lane] = make_float4(u[n][0], u[n][1], u[n][2], u[n][3]);
       __builtin_amdgcn_sched_barrier(0);
     }
+    f32x4_v old[NC][NTW];
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+#pragma unroll
+      for (int t = 0; t < NTW; ++t) {
+        old[n][t] = st[n][t];
+        st[n][t][0] *= o.pc[t].x; st[n][t][1] *= o.pc[t].y;
+        st[n][t][2] *= o.pc[t].z; st[n][t][3] *= o.pc[t].w;
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    float4 p[NC][4];
+    if (DELTA) {
+#pragma unroll
+      for (int n = 0; n < NC; ++n)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) p[n][w] = s_u[buf][n][w][lane];
+    }
+    fetch_out(c + 1);  // (the chunk before; of the first nothing is stored)
+    __builtin_amdgcn_sched_barrier(0);
     load(later);
+    f32x4_v r[NC];
+#pragma unroll
+    for (int n = 0; n < NC; ++n) r[n] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
       const float qs[4] = {o.qs[t].x, o.qs[t].y, o.qs[t].z, o.qs[t].w};
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        r = __builtin_amdgcn_mfma_f32_16x16x4f32(qs[i], st[t][i], r, 0, 0, 0);
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+          r[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(qs[i], old[n][t][i], r[n], 0, 0, 0);
     }
-    s_o[buf][wave][lane] = make_float4(r[0], r[1], r[2], r[3]);
+    float uu[NC][4];
 #pragma unroll
-    for (int t = 0; t < NTW; ++t) {
-      st[t][0] *= o.pc[t].x; st[t][1] *= o.pc[t].y;
-      st[t][2] *= o.pc[t].z; st[t][3] *= o.pc[t].w;
-    }
-    __syncthreads();
-    float uu[4] = {o.us.x, o.us.y, o.us.z, o.us.w};
-    float y[4];
-    if (DELTA) {
-      const float4 p0 = s_u[buf][0][lane], p1 = s_u[buf][1][lane];
-      const float4 p2 = s_u[buf][2][lane], p3 = s_u[buf][3][lane];
-#pragma unroll
-      for (int p = 0; p < 4; ++p)
-        y[p] = reinterpret_cast<const float*>(&s_o[buf][p][lane])[wave];
-      uu[0] -= (p0.x + p1.x) + (p2.x + p3.x);
-      uu[1] -= (p0.y + p1.y) + (p2.y + p3.y);
-      uu[2] -= (p0.z + p1.z) + (p2.z + p3.z);
-      uu[3] -= (p0.w + p1.w) + (p2.w + p3.w);
-    } else {
-#pragma unroll
-      for (int p = 0; p < 4; ++p)
-        y[p] = reinterpret_cast<const float*>(&s_o[buf][p][lane])[wave];
+    for (int n = 0; n < NC; ++n) {
+      uu[n][0] = o.us[n].x; uu[n][1] = o.us[n].y;
+      uu[n][2] = o.us[n].z; uu[n][3] = o.us[n].w;
+      if (DELTA) {
+        uu[n][0] -= (p[n][0].x + p[n][1].x) + (p[n][2].x + p[n][3].x);
+        uu[n][1] -= (p[n][0].y + p[n][1].y) + (p[n][2].y + p[n][3].y);
+        uu[n][2] -= (p[n][0].z + p[n][1].z) + (p[n][2].z + p[n][3].z);
+        uu[n][3] -= (p[n][0].w + p[n][1].w) + (p[n][2].w + p[n][3].w);
+      }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int t = 0; t < NTW; ++t) {
         const float kh[4] = {o.kh[t].x, o.kh[t].y, o.kh[t].z, o.kh[t].w};
-        st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[i], uu[i], st[t], 0, 0, 0);
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+          st[n][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kh[i], uu[n][i], st[n][t], 0, 0, 0);
       }
     __builtin_amdgcn_sched_barrier(0);
-    // the read-out of tokens 4 g + wave
-    const float sum = (((o.os + y[0]) + y[1]) + y[2]) + y[3];
-    if (kChunk * c + 4 * g4 + wave < len && col_ok) *out = sum;
-    out += kChunk * row;
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+      s_o[buf][n][wave][lane] = make_float4(r[n][0], r[n][1], r[n][2], r[n][3]);
+    if (c > 0) read_out(c - 1);
+#pragma unroll
+    for (int n = 0; n < NC; ++n) os[n] = o.os[n];
   };
   // The operands of the next chunks are on their way while one is multiplied.  The
   // compiler waits for all of them at the head of a loop, hence 16 steps per round.
-  constexpr int DEPTH = NTW <= 4 ? 4 : 2, ROUND = NTW <= 2 ? 4 * DEPTH : DEPTH;
+  constexpr int DEPTH = NTW > 4 ? 2 : NC > 1 ? 3 : 4;
+  constexpr int ROUND = NTW <= 2 ? NC > 1 ? 12 : 16 : DEPTH;
   Operands o[DEPTH];
 #pragma unroll
   for (int i = 0; i + 1 < DEPTH; ++i) load(o[i]);
@@ -829,13 +911,18 @@ recurrence_chain_kernel(RecArgs g) {
       step(o[i % DEPTH], o[(i + DEPTH - 1) % DEPTH], c0 + i);
     }
   }
+  __syncthreads();
+  fetch_out(nc - 1);
+  read_out(nc - 1);
 #pragma unroll
-  for (int t = 0; t < NTW; ++t)
+  for (int n = 0; n < NC; ++n)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = 16 * (wave * NTW + t) + 4 * g4 + i;
-      if (col_ok && d < a.D) state[(size_t)d * a.Dv] = st[t][i];
-    }
+    for (int t = 0; t < NTW; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = 16 * (wave * NTW + t) + 4 * g4 + i;
+        if (col + 16 * n < a.Dv && d < a.D) state[(size_t)d * a.Dv + 16 * n] = st[n][t][i];
+      }
 }
 
 // The convolution's last inputs of a portion, written once nothing of the portion
@@ -1206,12 +1293,17 @@ static void launch_chunks(hipStream_t s, const RecArgs& g) {
   const dim3 grid(g.chunks, g.a.H, g.b.S), block(256);
   const dim3 chain((pairs + 7) / 8 * 8 * vts);
   const size_t lds = (size_t)kChunk * (vts * 16 + 4) * sizeof(float);
+  const bool two = (int64_t)pairs * vts > 512;  // (see recurrence_chain_kernel)
 #define T5D_CH(E_)                                                               \
   do {                                                                           \
     hipLaunchKernelGGL((recurrence_chunk_kernel<64 * E_, DELTA, T>), grid, block, \
                        lds, s, g);                                               \
-    hipLaunchKernelGGL((recurrence_chain_kernel<E_, DELTA>), chain, block, 0, s, \
-                       g);                                                       \
+    if (E_ <= 2 && two)                                                          \
+      hipLaunchKernelGGL((recurrence_chain_kernel<E_, DELTA, E_ <= 2 ? 2 : 1>),  \
+                         dim3((pairs + 7) / 8 * 8 * ((vts + 1) / 2)), block, 0, s, g); \
+    else                                                                         \
+      hipLaunchKernelGGL((recurrence_chain_kernel<E_, DELTA, 1>), chain, block,  \
+                         0, s, g);                                               \
   } while (0)
   if (g.a.D <= 64) T5D_CH(1);
   else if (g.a.D <= 128) T5D_CH(2);
@@ -1331,6 +1423,7 @@ extern "C" int t5d_recurrence_run(void* stream, const t5d_recurrence* a,
   hipStream_t s = as_stream(stream);
   if (variant == 1 || (variant == 0 && can_step)) {
     g.wq = g.wk = g.wv = g.wbeta = g.wo = g.wchunk = nullptr;
+    g.order = nullptr;
     g.chunks = 0;
     const bool bf16 = a->dtype == T5D_BF16;
     if (a->delta) {
@@ -1350,6 +1443,8 @@ extern "C" int t5d_recurrence_run(void* stream, const t5d_recurrence* a,
                 hv = round4((int64_t)b->M * a->H * a->Dv);
   g.wq = w; g.wk = w + qk; g.wv = w + 2 * qk; g.wo = w + 2 * qk + hv;
   g.wbeta = w + 2 * qk + 2 * hv;
+  // (in chunks q has no scratch of its own)
+  g.order = b->S > 1 && b->S <= (int64_t)b->M * a->G * a->D ? (int32_t*)g.wq : nullptr;
   const int64_t plain = portion_floats(b->M, a->H, a->G, a->D, a->Dv);
   g.chunks = (b->max_len + kChunk - 1) / kChunk;
   const bool fits =

@@ -752,6 +752,36 @@ def test_recurrence_batches_match_each_alone(dt, delta):
       at[i] += n[i]
 
 
+# (D, Dv, sequences of 8 heads): one, three and eight tiles of 16 columns, on both sides of
+# the 512 workgroups of one tile from which two go together (launch_chunks); key sizes with
+# one, two and four tiles of channels per wavefront
+@pytest.mark.parametrize('dt', DTYPES)
+@pytest.mark.parametrize('delta,D,Dv,S', [
+    (True, 128, 128, 8), (True, 128, 128, 9), (False, 128, 100, 10), (True, 40, 40, 22),
+    (False, 64, 16, 65), (True, 100, 12, 65), (False, 160, 48, 22)])
+def test_recurrence_of_many_sequences(dt, delta, D, Dv, S):
+  """Chunks of many ragged sequences, one of them longer than a round of the chain and one of
+  a single token, have the bits of each sequence on its own, in outputs and states, first
+  portions and later ones; the first two lie at the oracle."""
+  r = Recurrence(dt, delta, 8, 4, D, Dv, 4 if delta else 0, S, seed=S + D)
+  lens = [1 + (37 * i) % 90 for i in range(S)]
+  lens[1] = 290
+  seqs = [r.sequence(n + 30) for n in lens]
+  for first, more in ((True, 0), (False, 30)):
+    portions = [(i, 0 if first else n, n + more) for i, n in enumerate(lens)]
+    before = r.state.clone(), r.ring.clone()
+    got, state = r.run(portions, seqs, 3), r.state.clone()
+    row = 0
+    for i, (slot, a, b) in enumerate(portions):
+      if i < 2:
+        assert rel(got[row:row + b - a], r.oracle(seqs[i])[a:b]) < 2 * r.tol
+      r.state[slot], r.ring[slot] = before[0][slot], before[1][slot]
+      alone = r.run([portions[i]], [seqs[i]], 3)
+      assert np.array_equal(got[row:row + b - a], alone), (i, first)
+      assert torch.equal(state[slot], r.state[slot]), (i, first)
+      row += b - a
+
+
 @pytest.mark.parametrize('dt', DTYPES)
 @pytest.mark.parametrize('delta', [True, False])
 def test_a_memory_from_far_back_survives(dt, delta):
