@@ -187,6 +187,25 @@ int t5d_gemm_rows_values(void* stream, int w_dtype, const void* A, const void* W
                          const float* scales, void* C, int64_t M, int K, int N,
                          const int32_t* at, int E, int Ep);
 
+/* The RMS norm between two layers of t5d_gemm_rows, without a pass over the rows.
+ * With scale [N] (bfloat16) and the residual epilogue: rows x = A W + residual go to C as
+ * they are and to scaled [M, N] as bfloat16(x * scale), the sums of their squares to
+ * squares [ceil(N / 64)][M], 64 columns each.  Without: A is such scaled rows (K their
+ * columns), squares those of the rows before, and results are divided by
+ * sqrt(sum / K + eps); at (NULL or) as in t5d_gemm_rows_values.  K as
+ * t5d_gemm_rows_takes_norm says (64 and more).  Other arguments as in t5d_gemm_rows_tiled. */
+typedef struct t5d_rows_norm {
+  const void* scale;
+  void* scaled;
+  float* squares;
+  float eps;
+} t5d_rows_norm;
+int t5d_gemm_rows_takes_norm(int K);
+int t5d_gemm_rows_normed(void* stream, int w_dtype, const void* A, const void* W,
+                         const float* scales, const void* residual, void* C, int64_t M,
+                         int K, int N, int epilogue, int out_layout, int E, int Ep,
+                         const int32_t* at, int tile, const t5d_rows_norm* norm);
+
 /* The workgroup tile (1, 2 or 3, as in t5d_gemm_rows_tiled) that t5d_gemm_rows
  * uses for a shape: the cheapest by the rounds of workgroups each tile needs
  * on 256 CUs (1 where the tile is not chosen, see above).  No device work; for tests and

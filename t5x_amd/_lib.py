@@ -99,6 +99,12 @@ class WindowAttention(Structure):
                      'out', i3='ld_out', p3='workspace')
 
 
+class RowsNorm(Structure):
+  """t5d_rows_norm."""
+  _fields_ = [('scale', c_void_p), ('scaled', c_void_p), ('squares', c_void_p),
+              ('eps', c_float)]
+
+
 class Span(Structure):
   """t5d_span."""
   _fields_ = _fields(i='window rows', p='off first')
@@ -246,6 +252,9 @@ _SIGNATURES = {
                                       [c_int] * 6),
     't5d_encoder_attention_f32': (c_int, [_P, _P, _P, _P, _P, _P, c_int,
                                           c_int, c_int]),
+    't5d_gemm_rows_takes_norm': (c_int, [c_int]),
+    't5d_gemm_rows_normed': (c_int, [_P, c_int] + [_P] * 5 + [c_int64] +
+                             [c_int] * 6 + [_P, c_int, POINTER(RowsNorm)]),
     't5d_gemm_rows': (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int64, c_int,
                               c_int, c_int, c_int, c_int, c_int]),
     't5d_gemm_rows_tiled': (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int64,

@@ -81,6 +81,13 @@ struct RowsGemmArgs {
   const int32_t* gate;     // optional device-side enable flag (rows_gemm_direct_kernel)
   GroupTiles grp;          // GROUPED kernels only, with the next
   int n_tiles;
+  // NORM kernels (see rows_gemm_direct_kernel)
+  const float* squares_in;   // [parts][M] of A's rows before they were scaled
+  int parts;                 // of 64 columns each
+  float norm_d, eps;         // columns of such a row
+  const bf16_t* next_scale;  // [N]
+  bf16_t* scaled;            // [M, N]
+  float* squares_out;        // [N / 64, rounded up][M]
 };
 
 __device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
@@ -99,7 +106,7 @@ constexpr int kRowsMT = 8, kRowsNT = 4;        // MFMA tiles per wavefront
 template <int MT, int NT>
 __device__ __forceinline__ void rows_epilogue_values(
     const RowsGemmArgs& g, const f32x4_r (&acc)[MT][NT], int m0,
-    int nt0, int n_tiles, int l16, int gq) {
+    int nt0, int n_tiles, int l16, int gq, const float* inv = nullptr) {
   // acc[mt][nt][i]: row m = m0 + 16 mt + 4 gq + i, column n = 16 (nt0 + nt) + l16
   // (values layout [B, H, Ep / 32, 64, 32]: 4 consecutive positions per store)
 #pragma unroll
@@ -120,13 +127,18 @@ __device__ __forceinline__ void rows_epilogue_values(
       if (nt0 + nt >= n_tiles) continue;
       const int n = 16 * (nt0 + nt) + l16;
       float s = g.scales ? g.scales[n] : 1.f;
+      float4 f = make_float4(s, s, s, s);
+      if (inv) {
+        f = *reinterpret_cast<const float4*>(inv + 16 * mt + 4 * gq);
+        f.x *= s; f.y *= s; f.z *= s; f.w *= s;
+      }
       const int hh = n >> 6, d = n & 63;
       const size_t o =
           ((((size_t)b * g.H + hh) * (g.Ep >> 5) + (e >> 5)) * 64 + d) * 32 +
           (e & 31);
       *reinterpret_cast<uint2*>(g.C + o) =
-          pack4(acc[mt][nt][0] * s, acc[mt][nt][1] * s, acc[mt][nt][2] * s,
-                acc[mt][nt][3] * s);
+          pack4(acc[mt][nt][0] * f.x, acc[mt][nt][1] * f.y, acc[mt][nt][2] * f.z,
+                acc[mt][nt][3] * f.w);
     }
   }
 }
@@ -144,12 +156,15 @@ __device__ __forceinline__ void rows_epilogue_values(
 // another lane's write (to it they are accesses of unrelated addresses).
 // DENSE: one of the epilogues of t5d_dense instead: 1 = T5D_EPI_CLAMPED_GLU (first
 // column of a pair: gate, second: up), 2 = float32 rows.
+// NORM: 1 = results are multiplied by shared[row]; 2 = with the residual added, a row's
+// squares go to shared[16-column tile of the workgroup][row], and scaled, it is stored a
+// second time.
 template <int NT> constexpr int kRowsStageStride = NT == 2 ? 80 : 144;
 template <int NT> constexpr int kRowsStageBytes = 16 * kRowsStageStride<NT>;
-template <int DENSE, bool SCALED, int MT, int NT>
+template <int DENSE, bool SCALED, int MT, int NT, int NORM = 0>
 __device__ __forceinline__ void rows_epilogue_staged(
     const RowsGemmArgs& g, const f32x4_r (&acc)[MT][NT], int m0, int nt0,
-    int n_tiles, int lane, char* stage) {
+    int n_tiles, int lane, char* stage, float* shared = nullptr, int wave = 0) {
   static_assert(NT >= 2 && NT <= 4, "a wavefront's slice: 32 to 64 columns");
   const int l16 = lane & 15, gq = lane >> 4;
   // int8 weights: the scale of each of this lane's 4 columns
@@ -162,11 +177,16 @@ __device__ __forceinline__ void rows_epilogue_staged(
                                                       16 * (nt0 + nt) + 4 * gq)
                    : make_float4(1.f, 1.f, 1.f, 1.f);
   }
+  float inv[MT];
+  if constexpr (NORM == 1) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) inv[mt] = shared[16 * mt + l16];
+  }
   const auto value = [&](int mt, int nt, int i) {
-    if constexpr (SCALED)
-      return acc[mt][nt][i] * reinterpret_cast<const float*>(&sc[nt])[i];
-    else
-      return acc[mt][nt][i];
+    float v = acc[mt][nt][i];
+    if constexpr (SCALED) v *= reinterpret_cast<const float*>(&sc[nt])[i];
+    if constexpr (NORM == 1) v *= inv[mt];
+    return v;
   };
   if constexpr (DENSE == 2) {
     // a lane holds 4 consecutive columns of one row: 64 bytes per row and store
@@ -248,7 +268,13 @@ __device__ __forceinline__ void rows_epilogue_staged(
   // The residual of AHEAD slices is under way while one is added (16384 x 768 x 768,
   // which waited for each slice: 31.9 -> 28.2 us with the bank conflicts gone too).
   constexpr int AHEAD = 4;
-  const bool residual = g.epilogue == T5D_EPI_RESIDUAL;
+  const bool residual = NORM == 2 || g.epilogue == T5D_EPI_RESIDUAL;
+  float next[8];
+  if constexpr (NORM == 2) {
+    const uint4 w = n_ok ? *reinterpret_cast<const uint4*>(g.next_scale + n)
+                         : make_uint4(0, 0, 0, 0);
+    unpack16(w, next);
+  }
   uint4 res[AHEAD][2];
   const auto fetch = [&](int mt) {
 #pragma unroll
@@ -300,6 +326,23 @@ __device__ __forceinline__ void rows_epilogue_staged(
       if (prow >= RPI || row >= 16) continue;
       const uint4 q = back[j];
       const int m = m0 + 16 * mt + row;
+      if constexpr (NORM == 2) {
+        float f[8];
+        unpack16(q, f);
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
+        ss = n_ok ? ss : 0.f;
+        ss += dpp_move<kDppXor1>(ss);  // the tile's other 8 columns
+        if ((piece & 1) == 0)
+          shared[(wave * NT + (piece >> 1)) * (16 * MT) + 16 * mt + row] = ss;
+        if (m < g.M && n_ok)
+          *reinterpret_cast<uint4*>(g.scaled + (size_t)m * g.N + n) = make_uint4(
+              pack_bf16x2(f[0] * next[0], f[1] * next[1]),
+              pack_bf16x2(f[2] * next[2], f[3] * next[3]),
+              pack_bf16x2(f[4] * next[4], f[5] * next[5]),
+              pack_bf16x2(f[6] * next[6], f[7] * next[7]));
+      }
       if (m >= g.M || !n_ok) continue;
       size_t o;
       if (g.layout == T5D_OUT_HEADS_KEY) {
@@ -532,8 +575,15 @@ __device__ __forceinline__ void rows_multiply_far(const RowsGemmArgs& g,
 // float32 results over K = 768, 1024, 2048 lie 8.3e-8, 9.4e-8, 1.31e-7 off the float64
 // ones there, 1.57e-7, 1.84e-7, 2.71e-7 with one sum over all of K, 8.0e-8, 8.8e-8,
 // 1.12e-7 so.
+// NORM: the RMS norm between layers without a pass of its own.  2: rows with the residual
+// added are stored as they are and times the norm's scale, with the sums of their squares,
+// 64 columns each (the same additions whatever the tile); 1: A is such scaled rows, and
+// results are divided by their root mean square, row by row.  The pass that this replaces
+// read and wrote every row at 2 to 3 TB/s, 11.0 us for 10312 rows of 768, 9.9 for 4976 of
+// 1024; the second store and the squares cost a layer 1 to 3 us.  Encoder of 12 layers of
+// 768, 10312 rows, 2796 -> 2680 us, of 24 of 1024, 4976 rows, 5218 -> 5000.
 template <typename WT, bool SWAP, int MT, int NT, int OCC, int DENSE = 0,
-          bool GROUPED = false, bool FOLD = false>
+          bool GROUPED = false, bool FOLD = false, int NORM = 0>
 __global__ void __launch_bounds__(256, OCC)
 rows_gemm_direct_kernel(RowsGemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (buffer descriptors are no host type)
@@ -585,6 +635,19 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   }
   const int m0 = m_blk * BM;
   const int nt0 = n_blk * (BN / 16) + wave * NT;
+  __shared__ __align__(16) float s_inv[NORM == 1 ? BM : 1];
+  constexpr int kSquares = NORM == 1 ? 16 : 1;
+  float squares[kSquares];
+  const float* row_squares = nullptr;
+  if constexpr (NORM == 1) {
+    // requested in front of the operands, looked at behind their first requests; the
+    // first barrier lies between here and the epilogue
+    row_squares = g.squares_in + min(m0 + (int)(threadIdx.x & (BM - 1)), g.M - 1);
+#pragma unroll
+    for (int p = 0; p < kSquares; ++p)
+      squares[p] = row_squares[(size_t)min(p, g.parts - 1) * g.M];
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   f32x4_r acc[MT][NT];
 #pragma unroll
@@ -695,6 +758,15 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   T5D_ROWS_ISSUE_W(1, w1);
   T5D_ROWS_ISSUE_A(1, s_a1);
   T5D_FENCE;
+  if constexpr (NORM == 1) {
+    float sum = squares[0];
+#pragma unroll
+    for (int p = 1; p < kSquares; ++p) sum += p < g.parts ? squares[p] : 0.f;
+    for (int p = kSquares; p < g.parts; ++p) sum += row_squares[(size_t)p * g.M];
+    if (threadIdx.x < BM)
+      s_inv[threadIdx.x] = 1.0f / sqrtf(sum / g.norm_d + g.eps);
+    T5D_FENCE;
+  }
   f32x4_r sums[FOLD ? MT : 1][FOLD ? NT : 1];
   if constexpr (FOLD) {
 #pragma unroll
@@ -747,12 +819,26 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
     // the requests past the end have landed, every wavefront is done with the ring
     __builtin_amdgcn_s_waitcnt(kWaitAll);
     __syncthreads();
-    rows_epilogue_staged<DENSE, sizeof(WT) == 1>(
+    float* shared = NORM == 1 ? s_inv : reinterpret_cast<float*>(&s_a1[0]);
+    static_assert(sizeof(s_a1) >= BN / 16 * BM * sizeof(float), "squares too many");
+    rows_epilogue_staged<DENSE, sizeof(WT) == 1, MT, NT, NORM>(
         g, acc, m0, nt0, n_tiles, lane,
-        reinterpret_cast<char*>(&s_a0[0]) + wave * kRowsStageBytes<NT>);
+        reinterpret_cast<char*>(&s_a0[0]) + wave * kRowsStageBytes<NT>, shared, wave);
+    if constexpr (NORM == 2) {
+      __syncthreads();
+      for (int i = threadIdx.x; i < NT * BM; i += 256) {
+        const int group = i / BM, row = i % BM;
+        const float* t = shared + 4 * group * BM + row;
+        const int m = m0 + row, at = n_blk * NT + group;
+        if (m < g.M && 64 * at < g.N)
+          g.squares_out[(size_t)at * g.M + m] =
+              (t[0] + t[BM]) + (t[2 * BM] + t[3 * BM]);
+      }
+    }
   } else {
     __builtin_amdgcn_s_waitcnt(kWaitAll);
-    rows_epilogue_values(g, acc, m0, nt0, n_tiles, l16, gq);
+    rows_epilogue_values(g, acc, m0, nt0, n_tiles, l16, gq,
+                         NORM == 1 ? s_inv : nullptr);
   }
 #endif
 }
@@ -819,7 +905,7 @@ extern "C" int t5d_gemm_rows_tile(int w_dtype, int64_t M, int K, int N) {
   return rows_tile(M, N, 0).code;
 }
 
-template <bool SWAP, int DENSE>
+template <bool SWAP, int DENSE, int NORM = 0>
 static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int w_dtype,
                                int code) {
   // (int8 weights, which are widened in registers on their way to the matrix cores, have
@@ -828,7 +914,8 @@ static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int w_dtype
   const dim3 grid((unsigned)((g.M + t.rows - 1) / t.rows) *
                   ((g.N + t.cols - 1) / t.cols));
 #define T5D_ROWS_LAUNCH(WT_, MT_, NT_, OCC_)                                     \
-  hipLaunchKernelGGL((rows_gemm_direct_kernel<WT_, SWAP, MT_, NT_, OCC_, DENSE>), \
+  hipLaunchKernelGGL((rows_gemm_direct_kernel<WT_, SWAP, MT_, NT_, OCC_, DENSE,  \
+                                              false, false, NORM>),              \
                      grid, dim3(256), 0, s, g)
   if constexpr (DENSE == 0) {
     if (w_dtype == T5D_I8) {
@@ -852,7 +939,12 @@ static int launch_rows(hipStream_t s, int w_dtype, const RowsGemmArgs& g,
   const dim3 grid((unsigned)m_blocks * n_blocks), block(256);
   const bool swap = g.layout != T5D_OUT_HEADS_VALUE;
   const int dense = g.epilogue == T5D_EPI_CLAMPED_GLU ? 1 : g.C32 != nullptr ? 2 : 0;
-  if (rows_direct(g.K, g.lda)) {
+  if (g.squares_in != nullptr) {  // (rows_direct is the caller's)
+    if (swap) launch_rows_direct<true, 0, 1>(s, g, w_dtype, tile);
+    else launch_rows_direct<false, 0, 1>(s, g, w_dtype, tile);
+  } else if (g.squares_out != nullptr) {
+    launch_rows_direct<true, 0, 2>(s, g, w_dtype, tile);
+  } else if (rows_direct(g.K, g.lda)) {
     if (dense == 1) launch_rows_direct<true, 1>(s, g, w_dtype, tile);
     else if (dense == 2) launch_rows_direct<true, 2>(s, g, w_dtype, tile);
     else if (swap) launch_rows_direct<true, 0>(s, g, w_dtype, tile);
@@ -888,7 +980,7 @@ extern "C" int t5d_gemm_rows(void* stream, int w_dtype, const void* A,
 static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
                      const float* scales, const void* residual, void* C, int64_t M,
                      int K, int N, int epilogue, int out_layout, int E, int Ep,
-                     const int32_t* at, int tile) {
+                     const int32_t* at, int tile, const t5d_rows_norm* norm = nullptr) {
   T5D_REQUIRE(A && W && C, T5D_EINVAL, "t5d_gemm_rows: null pointer");
   T5D_REQUIRE(tile >= 0 && tile <= 3, T5D_EINVAL,
               "t5d_gemm_rows_tiled: tile %d (0 chosen here, columns: 1: 128, "
@@ -920,7 +1012,7 @@ static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
                 E, Ep);
     H = N / 64;
   }
-  RowsGemmArgs g;
+  RowsGemmArgs g = {};
   g.A = (const bf16_t*)A; g.W = (const char*)W;
   g.scales = w_dtype == T5D_I8 ? scales : nullptr;
   g.residual = (const bf16_t*)residual; g.C = (bf16_t*)C;
@@ -930,7 +1022,42 @@ static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
   g.lda = K; g.C32 = nullptr; g.ldc = g.n_store = N;
   g.glu_limit = g.glu_alpha = g.glu_add = 0.f;
   g.gate = nullptr; g.grp = GroupTiles(); g.n_tiles = 0;
+  if (norm != nullptr) {
+    T5D_REQUIRE(rows_direct(K, K), T5D_ELIMIT, "t5d_gemm_rows_normed: K=%d", K);
+    T5D_REQUIRE(norm->squares && (norm->scale == nullptr) == (norm->scaled == nullptr) &&
+                    ((uintptr_t)norm->scale % 16) == 0 &&
+                    ((uintptr_t)norm->scaled % 16) == 0,
+                T5D_EINVAL, "t5d_gemm_rows_normed: norm buffers");
+    T5D_REQUIRE(norm->scale ? epilogue == T5D_EPI_RESIDUAL
+                            : epilogue != T5D_EPI_RESIDUAL && norm->eps > 0.f,
+                T5D_EINVAL, "t5d_gemm_rows_normed: epilogue %d, eps %f", epilogue,
+                (double)norm->eps);
+    if (norm->scale) {
+      T5D_REQUIRE(((uintptr_t)C % 16) == 0 && ((uintptr_t)residual % 16) == 0, T5D_EINVAL,
+                  "t5d_gemm_rows_normed: operand alignment");
+      g.next_scale = (const bf16_t*)norm->scale; g.scaled = (bf16_t*)norm->scaled;
+      g.squares_out = norm->squares;
+    } else {
+      g.squares_in = norm->squares; g.parts = (K + 63) / 64;
+      g.norm_d = (float)K; g.eps = norm->eps;
+    }
+  }
   return launch_rows(as_stream(stream), w_dtype, g, tile);
+}
+
+extern "C" int t5d_gemm_rows_takes_norm(int K) { return K > 0 && rows_direct(K, K); }
+
+extern "C" int t5d_gemm_rows_normed(void* stream, int w_dtype, const void* A,
+                                    const void* W, const float* scales,
+                                    const void* residual, void* C, int64_t M, int K,
+                                    int N, int epilogue, int out_layout, int E, int Ep,
+                                    const int32_t* at, int tile,
+                                    const t5d_rows_norm* norm) {
+  T5D_REQUIRE(norm, T5D_EINVAL, "t5d_gemm_rows_normed: null pointer");
+  T5D_REQUIRE(!at || out_layout == T5D_OUT_HEADS_VALUE, T5D_EINVAL,
+              "t5d_gemm_rows_normed: positions go with the value layout");
+  return gemm_rows(stream, w_dtype, A, W, scales, residual, C, M, K, N, epilogue,
+                   out_layout, E, Ep, at, tile, norm);
 }
 
 extern "C" int t5d_gemm_rows_tiled(void* stream, int w_dtype, const void* A,
@@ -956,7 +1083,7 @@ int t5d::launch_dense_rows(hipStream_t s, const void* A, int lda,
                            int n_store, int M, int K, int N, int epilogue,
                            float glu_limit, float glu_alpha,
                            float glu_add) {
-  RowsGemmArgs g;
+  RowsGemmArgs g = {};
   g.A = (const bf16_t*)A; g.W = (const char*)W;
   g.scales = nullptr; g.residual = nullptr;
   g.C = out_f32 ? nullptr : (bf16_t*)C;
@@ -982,7 +1109,7 @@ int t5d::launch_dense_rows(hipStream_t s, const void* A, int lda,
 }
 
 int t5d::launch_grouped_rows(hipStream_t s, const GroupedArgs& a, int n_tiles) {
-  RowsGemmArgs g;
+  RowsGemmArgs g = {};
   g.A = a.A; g.W = (const char*)a.W;
   g.scales = nullptr; g.residual = nullptr;
   g.C = (bf16_t*)a.C; g.C32 = nullptr;

@@ -56,6 +56,44 @@ class EncoderKernelWeights:
     return self._bias[E]
 
 
+def _layers(cfg, w, x, v_t, E, rows, attend):
+  """The encoder's layers over x, rows of texts of E positions each or those of an
+  EncoderRows; attend(q | k) with the values in v_t.  The norms between
+  layers ride in the dense layers on both sides of them (widths of 32 have their own
+  pass)."""
+  from t5x_amd import _lib, ops
+  Ep = v_t.shape[2] * 32
+  inside = ops.takes_norm(cfg.emb_dim, cfg.num_heads * 64, cfg.mlp_dim)
+
+  def residual_and_norm(a, kernel, x, scale):
+    if inside:
+      return ops.gemm_rows_residual_norm(a, kernel, x, scale)
+    x = ops.gemm_rows(a, kernel, residual=x)
+    return x, ops.rmsnorm(x, scale)
+
+  def dense(a, kernel):
+    return (ops.gemm_rows_of_scaled(a, kernel) if isinstance(a, ops.ScaledRows)
+            else ops.gemm_rows(a, kernel))
+
+  xn = ops.rmsnorm(x, w.layers[0]['ln_attn']) if w.layers else None
+  for i, l in enumerate(w.layers):
+    qk = dense(xn, l['qk'])                               # [M, q | k]
+    if isinstance(xn, ops.ScaledRows):
+      ops.gemm_rows_of_scaled(xn, l['v'], out=v_t, layout=_lib.OUT_HEADS_VALUE, E=E,
+                              Ep=Ep, at=None if rows is None else rows.at)
+    elif rows is not None:
+      ops.gemm_rows_values(xn, l['v'], rows, out=v_t)
+    else:
+      ops.gemm_rows(xn, l['v'], out=v_t, layout=_lib.OUT_HEADS_VALUE, E=E, Ep=Ep)
+    x, y = residual_and_norm(attend(qk), l['o'], x, l['ln_mlp'])
+    h = dense(y, l['wi'])
+    if i + 1 < len(w.layers):
+      x, xn = residual_and_norm(h, l['wo'], x, w.layers[i + 1]['ln_attn'])
+    else:
+      x = ops.gemm_rows(h, l['wo'], residual=x)
+  return x
+
+
 def _encode_rows(cfg, w, rows, device):
   """_encode_hip over the rows that there are (ops.EncoderRows)."""
   from t5x_amd import ops
@@ -64,15 +102,10 @@ def _encode_rows(cfg, w, rows, device):
   x = ops.embed(w.embedding, rows.ids)
   v_t = torch.zeros((rows.B, cfg.num_heads, (rows.positions + 31) // 32, 64, 32),
                     dtype=x.dtype, device=device)
-  for l in w.layers:
-    xn = ops.rmsnorm(x, l['ln_attn'])
-    qk = ops.gemm_rows(xn, l['qk'])                       # [M, q | k]
-    ops.gemm_rows_values(xn, l['v'], rows, out=v_t)
-    attn = ops.encoder_attention_rows(qk[:, :HD], qk[:, HD:], v_t, bias, rows)
-    x = ops.gemm_rows(attn, l['o'], residual=x)
-    y = ops.rmsnorm(x, l['ln_mlp'])
-    h = ops.gemm_rows(y, l['wi'])
-    x = ops.gemm_rows(h, l['wo'], residual=x)
+  def attend(qk):
+    return ops.encoder_attention_rows(qk[:, :HD], qk[:, HD:], v_t, bias, rows)
+
+  x = _layers(cfg, w, x, v_t, rows.positions, rows, attend)
   return ops.rmsnorm_rows(x, w.ln_final, rows.row_of).view(rows.B, rows.E,
                                                           cfg.emb_dim)
 
@@ -114,16 +147,11 @@ def _encode_positions(cfg, w, tokens, dev, odd=None):
   x = ops.embed(w.embedding, ids)
   M = B * E
   v_t = torch.zeros((B, H, Ep // 32, 64, 32), dtype=x.dtype, device=dev)
-  for l in w.layers:
-    xn = ops.rmsnorm(x, l['ln_attn'])
-    qk = ops.gemm_rows(xn, l['qk'])                       # [M, q | k]
-    ops.gemm_rows(xn, l['v'], out=v_t, layout=_lib.OUT_HEADS_VALUE, E=E, Ep=Ep)
-    attn = ops.encoder_attention(qk[:, :HD], qk[:, HD:], v_t, bias, lens,
+  def attend(qk):
+    return ops.encoder_attention(qk[:, :HD], qk[:, HD:], v_t, bias, lens,
                                  valid_bits=bits)
-    x = ops.gemm_rows(attn, l['o'], residual=x)
-    y = ops.rmsnorm(x, l['ln_mlp'])
-    h = ops.gemm_rows(y, l['wi'])
-    x = ops.gemm_rows(h, l['wo'], residual=x)
+
+  x = _layers(cfg, w, x, v_t, E, None, attend)
   return ops.rmsnorm(x, w.ln_final).view(B, E, cfg.emb_dim)
 
 

@@ -510,6 +510,67 @@ def gemm_rows(a, w: PackedWeight, out=None, residual=None,
   return out
 
 
+class ScaledRows:
+  """Rows times an RMS norm's scale, and the sums of squares they are still to be
+  divided by (gemm_rows_residual_norm)."""
+
+  def __init__(self, x, squares, eps):
+    self.x, self.squares, self.eps = x, squares, eps
+
+
+def takes_norm(*widths):
+  """Whether layers over rows of these widths have the norm between them inside."""
+  return all(_lib.load().t5d_gemm_rows_takes_norm(k) for k in widths)
+
+
+def _rows_normed(a, squares, w, residual, out, epi, layout, E, Ep, at, norm):
+  _chk(a, 'a', torch.bfloat16, 2)
+  M, K = a.shape
+  if K != w.K or w.w_dtype == F32:
+    raise ValueError(f'a is [{M}, {K}]; kernel K={w.K}, packed weights only')
+  _chk(squares, 'squares', torch.float32, 2)
+  width = w.N if norm.scale else K
+  if tuple(squares.shape) != ((width + 63) // 64, M):
+    raise ValueError(f'squares {tuple(squares.shape)} of {M} rows of {width}')
+  norm.squares = squares.data_ptr()
+  _lib.call('t5d_gemm_rows_normed', _s(), w.w_dtype, a.data_ptr(), w.data.data_ptr(),
+            _lib.ptr(w.scales), _lib.ptr(residual), out.data_ptr(), M, K, w.N, epi,
+            int(layout), int(E), int(Ep), _lib.ptr(at), 0, norm)
+
+
+def gemm_rows_residual_norm(a, w: PackedWeight, residual, scale, eps=1e-6):
+  """gemm_rows with a residual, and the RMS norm behind it as far as it goes without a
+  pass over the rows: (x [M, N], ScaledRows of bfloat16(x * scale))."""
+  M, N = a.shape[0], w.N
+  _chk(residual, 'residual', torch.bfloat16, 2)
+  _chk(scale, 'scale', torch.bfloat16, 1)
+  if tuple(residual.shape) != (M, N) or scale.shape[0] != N or w.geglu:
+    raise ValueError('residual [M, N], scale [N], no gated kernel')
+  make = lambda *s, dtype=a.dtype: torch.empty(s, dtype=dtype, device=a.device)
+  x, scaled = make(M, N), make(M, N)
+  squares = make((N + 63) // 64, M, dtype=torch.float32)
+  norm = _lib.RowsNorm(scale.data_ptr(), scaled.data_ptr(), None, 0.0)
+  _rows_normed(a, squares, w, residual, x, EPI_RESIDUAL, _lib.OUT_ROWS, 0, 0, None,
+               norm)
+  return x, ScaledRows(scaled, squares, eps)
+
+
+def gemm_rows_of_scaled(rows: ScaledRows, w: PackedWeight, out=None,
+                        layout=_lib.OUT_ROWS, E=0, Ep=0, at=None):
+  """gemm_rows of the rows that ScaledRows stands for; with layout OUT_HEADS_VALUE (and
+  at of an EncoderRows, as gemm_rows_values) into `out`."""
+  if layout == _lib.OUT_ROWS:
+    out = torch.empty((rows.x.shape[0], w.out_features), dtype=rows.x.dtype,
+                      device=rows.x.device)
+  elif out is None:
+    raise ValueError('the value layout needs out')
+  _chk(out, 'out', rows.x.dtype)
+  norm = _lib.RowsNorm(None, None, None, rows.eps)
+  _rows_normed(rows.x, rows.squares, w, None, out, EPI_GEGLU if w.geglu else EPI_NONE,
+               layout, E, Ep, at, norm)
+  return out
+
+
 def gemm_rows_values(a, w: PackedWeight, rows, out):
   """gemm_rows into `out` [B, H, Ep/32, 64, 32] for the rows of an EncoderRows; the
   positions without a row are left as they are (encoder_attention_rows wants zeros)."""

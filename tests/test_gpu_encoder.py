@@ -294,6 +294,69 @@ def _check_head_layouts(ops, rows, keys, vals, B, E, Ep, H):
   assert torch.equal(vals, ops.tile_cross_value(plain_v))
 
 
+# (rows, columns of the normed rows, columns behind): rows off every tile, columns off the
+# 64 whose squares go together, more than 16 such parts, tiles of 64 rows
+@pytest.mark.parametrize('M,D,N', [(1, 64, 64), (77, 96, 128), (300, 224, 192),
+                                   (1001, 768, 1536), (129, 1088, 320), (40, 2048, 64)])
+@pytest.mark.parametrize('wd', [torch.bfloat16, torch.int8])
+def test_gemm_rows_with_the_norm_between_them(ops, M, D, N, wd):
+  """x = a W + residual, then norm(x) W2, plain, gated and in the value layout, the norm
+  inside the two layers: x has the bits of the layer without it, squares are sums of 64
+  terms (64 x 2^-24 off float64's), scaled rows round x scale once, and a result lies as
+  near to float64 as one rounding of every row entry (2^-9 of the sum of |terms|, by its
+  2-norm) and one of its own (2^-9), and K float32 sums.  Every tile gives the same."""
+  from t5x_amd import _lib
+  bf = torch.bfloat16
+  gen = torch.Generator(device='cuda')
+  gen.manual_seed(M + D + N)
+  rnd = lambda *s: torch.randn(s, generator=gen, device='cuda')
+  K = 96
+  a, res = rnd(M, K).to(bf), (3 * rnd(M, D)).to(bf)
+  scale = (1 + 0.3 * rnd(D)).to(bf)
+  w1 = ops.pack_weight(rnd(K, D) * K ** -0.5, bf, wd)
+  k2, k3 = rnd(D, N) * D ** -0.5, rnd(D, N) * D ** -0.5
+  plain, gated = (ops.pack_weight(k2, bf, wd, **o) for o in ({}, {'gate_kernel': k3}))
+  x, y = ops.gemm_rows_residual_norm(a, w1, res, scale)
+  assert torch.equal(x, ops.gemm_rows(a, w1, residual=res))
+  assert torch.equal(y.x, (x.float() * scale.float()).to(bf))
+  x2 = torch.nn.functional.pad(x.double() ** 2, (0, -D % 64)).view(M, -1, 64).sum(2).t()
+  assert bool(((y.squares - x2).abs() <= 64 * 2.0**-24 * x2).all())
+  for tile in (1, 2, 3):
+    again = [torch.empty_like(t) for t in (x, y.x, y.squares)]
+    norm = _lib.RowsNorm(scale.data_ptr(), again[1].data_ptr(), again[2].data_ptr(), 0.0)
+    _lib.call('t5d_gemm_rows_normed', ops._s(), w1.w_dtype, a.data_ptr(),
+              w1.data.data_ptr(), _lib.ptr(w1.scales), res.data_ptr(),
+              again[0].data_ptr(), M, K, D, _lib.EPI_RESIDUAL, _lib.OUT_ROWS, 0, 0, None,
+              tile, norm)
+    assert all(torch.equal(p, q) for p, q in zip(again, (x, y.x, y.squares))), tile
+  xd = x.double()
+  normed = xd / torch.sqrt((xd ** 2).mean(1, keepdim=True) + 1e-6) * scale.double()
+  def kernel(k):
+    if wd == bf:
+      return k.to(bf).double()
+    s = k.abs().amax(0).clamp_min(1e-30) / 127
+    return (k / s).round().clamp(-127, 127).double() * s.double()
+  def near(got, want, spread):
+    bound = 2.0**-8 * want.abs() + (6 * 2.0**-9 + D * 2.0**-24) * spread
+    assert bool(((got.double() - want).abs() <= bound).all())
+  size = lambda k: torch.sqrt((normed ** 2) @ (k ** 2))
+  h, u = normed @ kernel(k2), normed @ kernel(k3)
+  got = ops.gemm_rows_of_scaled(y, plain)
+  near(got, h, size(kernel(k2)))
+  if N % 8 == 0:
+    act = torch.nn.functional.gelu(h, approximate='tanh')
+    # (the gate and the unit are rounded on the way: two more roundings of the product)
+    near(ops.gemm_rows_of_scaled(y, gated), act * u,
+         size(kernel(k2)) * u.abs() * 1.2 + size(kernel(k3)) * act.abs() + (act * u).abs())
+  if M % 4 == 0:
+    E, Ep, H = M // 4 if M % 16 == 0 else M, 0, N // 64
+    Ep = (E + 31) // 32 * 32
+    v = torch.zeros((M // E, H, Ep // 32, 64, 32), dtype=bf, device='cuda')
+    ops.gemm_rows_of_scaled(y, plain, out=v, layout=_lib.OUT_HEADS_VALUE, E=E, Ep=Ep)
+    rows = v.transpose(3, 4).reshape(M // E, H, Ep, 64)[:, :, :E]
+    assert torch.equal(rows.transpose(1, 2).reshape(M, N), got)
+
+
 def _against_float64(ops, out, q, k, v_t, rel_bias, lens, bits):
   """`out` is what every variant that is accepted gives, and the attention of the same
   operands in float64, its scores rounded to bfloat16 twice as in the reference.  With u
