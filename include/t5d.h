@@ -193,7 +193,8 @@ int t5d_gemm_rows_values(void* stream, int w_dtype, const void* A, const void* W
  * squares [ceil(N / 64)][M], 64 columns each.  Without: A is such scaled rows (K their
  * columns), squares those of the rows before, and results are divided by
  * sqrt(sum / K + eps); at (NULL or) as in t5d_gemm_rows_values.  K as
- * t5d_gemm_rows_takes_norm says (64 and more).  Other arguments as in t5d_gemm_rows_tiled. */
+ * t5d_gemm_rows_takes_norm says (64 and more), bfloat16 weights.  Other arguments as in
+ * t5d_gemm_rows_tiled. */
 typedef struct t5d_rows_norm {
   const void* scale;
   void* scaled;
@@ -205,6 +206,20 @@ int t5d_gemm_rows_normed(void* stream, int w_dtype, const void* A, const void* W
                          const float* scales, const void* residual, void* C, int64_t M,
                          int K, int N, int epilogue, int out_layout, int E, int Ep,
                          const int32_t* at, int tile, const t5d_rows_norm* norm);
+
+/* Two layers over the same rows in one launch: A W to C [M, N], row-major, and A second->W
+ * to second->C in the value layout (E, Ep, at as in t5d_gemm_rows_normed); norm (scale
+ * NULL) or NULL as there.  Results are those of two calls. */
+typedef struct t5d_rows_second {
+  const void* W;
+  const float* scales;
+  void* C;
+  int N;
+} t5d_rows_second;
+int t5d_gemm_rows_pair(void* stream, int w_dtype, const void* A, const void* W,
+                       const float* scales, void* C, int64_t M, int K, int N, int E,
+                       int Ep, const int32_t* at, int tile, const t5d_rows_second* second,
+                       const t5d_rows_norm* norm);
 
 /* The workgroup tile (1, 2 or 3, as in t5d_gemm_rows_tiled) that t5d_gemm_rows
  * uses for a shape: the cheapest by the rounds of workgroups each tile needs

@@ -105,6 +105,11 @@ class RowsNorm(Structure):
               ('eps', c_float)]
 
 
+class RowsSecond(Structure):
+  """t5d_rows_second."""
+  _fields_ = [('W', c_void_p), ('scales', c_void_p), ('C', c_void_p), ('N', c_int)]
+
+
 class Span(Structure):
   """t5d_span."""
   _fields_ = _fields(i='window rows', p='off first')
@@ -255,6 +260,8 @@ _SIGNATURES = {
     't5d_gemm_rows_takes_norm': (c_int, [c_int]),
     't5d_gemm_rows_normed': (c_int, [_P, c_int] + [_P] * 5 + [c_int64] +
                              [c_int] * 6 + [_P, c_int, POINTER(RowsNorm)]),
+    't5d_gemm_rows_pair': (c_int, [_P, c_int] + [_P] * 4 + [c_int64] + [c_int] * 4 +
+                           [_P, c_int, POINTER(RowsSecond), POINTER(RowsNorm)]),
     't5d_gemm_rows': (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int64, c_int,
                               c_int, c_int, c_int, c_int, c_int]),
     't5d_gemm_rows_tiled': (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int64,

@@ -88,6 +88,11 @@ struct RowsGemmArgs {
   const bf16_t* next_scale;  // [N]
   bf16_t* scaled;            // [M, N]
   float* squares_out;        // [N / 64, rounded up][M]
+  // rows_gemm_pair_kernel: the second layer
+  const char* W2;
+  const float* scales2;
+  bf16_t* C2;
+  int N2;
 };
 
 __device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
@@ -582,10 +587,11 @@ __device__ __forceinline__ void rows_multiply_far(const RowsGemmArgs& g,
 // read and wrote every row at 2 to 3 TB/s, 11.0 us for 10312 rows of 768, 9.9 for 4976 of
 // 1024; the second store and the squares cost a layer 1 to 3 us.  Encoder of 12 layers of
 // 768, 10312 rows, 2796 -> 2680 us, of 24 of 1024, 4976 rows, 5218 -> 5000.
-template <typename WT, bool SWAP, int MT, int NT, int OCC, int DENSE = 0,
-          bool GROUPED = false, bool FOLD = false, int NORM = 0>
-__global__ void __launch_bounds__(256, OCC)
-rows_gemm_direct_kernel(RowsGemmArgs g) {
+template <typename WT, bool SWAP, int MT, int NT, int DENSE, bool GROUPED, bool FOLD,
+          int NORM>
+__device__ __forceinline__ void rows_gemm_tile(
+    const RowsGemmArgs& g, int m_blk, int n_blk, uint4 (&s_a0)[128 * MT],
+    uint4 (&s_a1)[128 * MT], uint4 (&s_a2)[128 * MT], float* s_inv) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (buffer descriptors are no host type)
   constexpr int BM = 16 * MT, BN = 64 * NT;
   constexpr int TB = RowsWeight<WT>::kTileBytes;
@@ -597,47 +603,15 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
   constexpr int kWaitStage = 0x070 | (AL + NT);
   static_assert(AL + NT < 16, "vmcnt");
   constexpr int kWaitAll = 0x070;
-  __shared__ uint4 s_a0[BM * 8];
-  __shared__ uint4 s_a1[BM * 8];
-  __shared__ uint4 s_a2[BM * 8];
   static_assert(sizeof(s_a0) >= 4 * kRowsStageBytes<NT>, "stage too small");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, gq = lane >> 4;
   const int KT = g.K >> 5, KS = (KT + 1) >> 1, n_tiles = g.N >> 4;
-  const int n_blocks = (n_tiles + BN / 16 - 1) / (BN / 16);
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  T5D_GATED(g.gate);
-  int m_blk, n_blk;
-  if constexpr (GROUPED) {
-    // 4 consecutive tiles of rows, most of them of one group, on one XCD, all
-    // columns of half a tile in a row: rows and kernels come from that XCD's L2.
-    const int t = slot / n_blocks;
-    const int tile = ((t >> 3) * 8 + xcd) * 4 + ((t & 7) >> 1);
-    m_blk = t & 1;
-    n_blk = slot % n_blocks;
-    if (tile >= g.n_tiles ||
-        !enter_group(g.grp, tile, g.A, g.lda, g.W, g.C, DENSE == 1 ? g.N >> 1 : g.N,
-                     g.M) ||
-        m_blk * BM >= g.M)
-      return;
-  } else {
-    // An XCD takes a run of consecutive tiles, column by column over 8 blocks of rows
-    // at a time: what its CUs hold at once is few rows and few weights.
-    const int m_blocks = (g.M + BM - 1) / BM;
-    const int total = m_blocks * n_blocks;
-    const int t = xcd * (total >> 3) + min(xcd, total & 7) + slot;
-    constexpr int GM = 8;
-    const int group = t / (GM * n_blocks), in = t - group * (GM * n_blocks);
-    const int rows = min(GM, m_blocks - group * GM);
-    m_blk = group * GM + in % rows;
-    n_blk = in / rows;
-  }
   const int m0 = m_blk * BM;
   const int nt0 = n_blk * (BN / 16) + wave * NT;
-  __shared__ __align__(16) float s_inv[NORM == 1 ? BM : 1];
   constexpr int kSquares = NORM == 1 ? 16 : 1;
-  float squares[kSquares];
+  float squares[kSquares], more[kSquares];
   const float* row_squares = nullptr;
   if constexpr (NORM == 1) {
     // requested in front of the operands, looked at behind their first requests; the
@@ -646,6 +620,13 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
 #pragma unroll
     for (int p = 0; p < kSquares; ++p)
       squares[p] = row_squares[(size_t)min(p, g.parts - 1) * g.M];
+#pragma unroll
+    for (int p = 0; p < kSquares; ++p) more[p] = 0.f;
+    if (g.parts > kSquares) {
+#pragma unroll
+      for (int p = 0; p < kSquares; ++p)
+        more[p] = row_squares[(size_t)min(kSquares + p, g.parts - 1) * g.M];
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
 
@@ -762,7 +743,9 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
     float sum = squares[0];
 #pragma unroll
     for (int p = 1; p < kSquares; ++p) sum += p < g.parts ? squares[p] : 0.f;
-    for (int p = kSquares; p < g.parts; ++p) sum += row_squares[(size_t)p * g.M];
+#pragma unroll
+    for (int p = 0; p < kSquares; ++p) sum += kSquares + p < g.parts ? more[p] : 0.f;
+    for (int p = 2 * kSquares; p < g.parts; ++p) sum += row_squares[(size_t)p * g.M];
     if (threadIdx.x < BM)
       s_inv[threadIdx.x] = 1.0f / sqrtf(sum / g.norm_d + g.eps);
     T5D_FENCE;
@@ -843,6 +826,80 @@ rows_gemm_direct_kernel(RowsGemmArgs g) {
 #endif
 }
 
+// An XCD takes a run of consecutive tiles, column by column over 8 blocks of rows at a
+// time: what its CUs hold at once is few rows and few weights.
+__device__ __forceinline__ void rows_tile_of(int m_blocks, int n_blocks, int& m_blk,
+                                             int& n_blk) {
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int total = m_blocks * n_blocks;
+  const int t = xcd * (total >> 3) + min(xcd, total & 7) + slot;
+  constexpr int GM = 8;
+  const int group = t / (GM * n_blocks), in = t - group * (GM * n_blocks);
+  const int rows = min(GM, m_blocks - group * GM);
+  m_blk = group * GM + in % rows;
+  n_blk = in / rows;
+}
+
+template <typename WT, bool SWAP, int MT, int NT, int OCC, int DENSE = 0,
+          bool GROUPED = false, bool FOLD = false, int NORM = 0>
+__global__ void __launch_bounds__(256, OCC)
+rows_gemm_direct_kernel(RowsGemmArgs g) {
+  constexpr int BM = 16 * MT, BN = 64 * NT;
+  __shared__ uint4 s_a0[BM * 8];
+  __shared__ uint4 s_a1[BM * 8];
+  __shared__ uint4 s_a2[BM * 8];
+  __shared__ __align__(16) float s_inv[NORM == 1 ? BM : 4];
+  T5D_GATED(g.gate);
+  const int n_blocks = ((g.N >> 4) + BN / 16 - 1) / (BN / 16);
+  int m_blk, n_blk;
+  if constexpr (GROUPED) {
+    // 4 consecutive tiles of rows, most of them of one group, on one XCD, all
+    // columns of half a tile in a row: rows and kernels come from that XCD's L2.
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int t = slot / n_blocks;
+    const int tile = ((t >> 3) * 8 + xcd) * 4 + ((t & 7) >> 1);
+    m_blk = t & 1;
+    n_blk = slot % n_blocks;
+    if (tile >= g.n_tiles ||
+        !enter_group(g.grp, tile, g.A, g.lda, g.W, g.C, DENSE == 1 ? g.N >> 1 : g.N,
+                     g.M) ||
+        m_blk * BM >= g.M)
+      return;
+  } else {
+    rows_tile_of((g.M + BM - 1) / BM, n_blocks, m_blk, n_blk);
+  }
+  rows_gemm_tile<WT, SWAP, MT, NT, DENSE, GROUPED, FOLD, NORM>(g, m_blk, n_blk, s_a0,
+                                                               s_a1, s_a2, s_inv);
+}
+
+// Two layers over the same rows in one launch, the second into the value layout: an
+// encoder's q | k and v, which are too narrow to fill the rounds of workgroups each on its
+// own (see rows_pair).
+template <typename WT, int MT, int NT, int OCC, int NORM>
+__global__ void __launch_bounds__(256, OCC)
+rows_gemm_pair_kernel(RowsGemmArgs g) {
+  constexpr int BM = 16 * MT, BN = 64 * NT;
+  __shared__ uint4 s_a0[BM * 8];
+  __shared__ uint4 s_a1[BM * 8];
+  __shared__ uint4 s_a2[BM * 8];
+  __shared__ __align__(16) float s_inv[NORM == 1 ? BM : 4];
+  const int n1 = (g.N + BN - 1) / BN, n2 = (g.N2 + BN - 1) / BN;
+  int m_blk, n_blk;
+  rows_tile_of((g.M + BM - 1) / BM, n1 + n2, m_blk, n_blk);
+  if (n_blk < n1) {
+    g.layout = T5D_OUT_ROWS;
+    rows_gemm_tile<WT, true, MT, NT, 0, false, false, NORM>(g, m_blk, n_blk, s_a0, s_a1,
+                                                            s_a2, s_inv);
+  } else {
+    g.W = g.W2;
+    g.scales = g.scales2;
+    g.C = g.C2;
+    g.N = g.N2;
+    rows_gemm_tile<WT, false, MT, NT, 0, false, false, NORM>(g, m_blk, n_blk - n1, s_a0,
+                                                             s_a1, s_a2, s_inv);
+  }
+}
+
 }  // namespace t5d
 
 using namespace t5d;
@@ -871,8 +928,10 @@ static const RowsTile kRowsTiles[] = {
     {1, 64, 128, 4, {0.28, 0.45, 0.80, 1.00}},
 };
 
-static double rows_tile_cost(const RowsTile& t, int64_t M, int N) {
-  const int64_t wgs = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
+// N2: columns of a second layer in the same launch.
+static double rows_tile_cost(const RowsTile& t, int64_t M, int N, int N2 = 0) {
+  const int64_t wgs = ((M + t.rows - 1) / t.rows) *
+                      ((N + t.cols - 1) / t.cols + (N2 + t.cols - 1) / t.cols);
   const int64_t slots = 256 * t.per_cu, left = wgs % slots;
   return (double)(wgs / slots) * t.step[t.per_cu - 1] +
          (left ? t.step[(left + 255) / 256 - 1] : 0.0);
@@ -886,12 +945,12 @@ static bool rows_direct(int K, int64_t lda) {
 }
 
 // code 0: any.
-static const RowsTile& rows_tile(int64_t M, int N, int code) {
+static const RowsTile& rows_tile(int64_t M, int N, int code, int N2 = 0) {
   const RowsTile* best = nullptr;
   double least = 0.0;
   for (const RowsTile& t : kRowsTiles) {
     if (code && t.code != code) continue;
-    const double c = rows_tile_cost(t, M, N);
+    const double c = rows_tile_cost(t, M, N, N2);
     if (best == nullptr || c < least) {
       best = &t;
       least = c;
@@ -917,7 +976,68 @@ static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int w_dtype
   hipLaunchKernelGGL((rows_gemm_direct_kernel<WT_, SWAP, MT_, NT_, OCC_, DENSE,  \
                                               false, false, NORM>),              \
                      grid, dim3(256), 0, s, g)
-  if constexpr (DENSE == 0) {
+  if constexpr (DENSE == 0 && NORM == 0) {
+    if (w_dtype == T5D_I8) {
+      if (t.rows == 64) T5D_ROWS_LAUNCH(int8_t, 4, 2, 4);
+      else T5D_ROWS_LAUNCH(int8_t, 8, 2, 3);
+      return;
+    }
+  }
+  if (t.rows == 64) T5D_ROWS_LAUNCH(bf16_t, 4, 2, 4);
+  else if (t.cols == 128) T5D_ROWS_LAUNCH(bf16_t, 8, 2, 3);
+  else if (t.cols == 192) T5D_ROWS_LAUNCH(bf16_t, 8, 3, 2);
+  else T5D_ROWS_LAUNCH(bf16_t, 8, 4, 2);
+#undef T5D_ROWS_LAUNCH
+}
+
+// The workgroup tile of two layers in one launch; null: two launches.  Over up to 768
+// inputs that is 128 columns (10304 x 768 41.0 us, with 256 or 192 42.4).  One launch gains
+// where the two leave part of a round empty; beyond five rounds, and where the cost model
+// says that the two fit their rounds better, there are two.  us, two launches / one (rows x
+// inputs x columns + columns):
+//    1024 x  512 x  768 + 384   20.9 / 12.3      4096 x  768 x 1536 + 768   25.0 / 21.5
+//   10304 x  768 x 1536 + 768   42.3 / 41.0     12288 x  768 x 1536 + 768   50.7 / 46.2
+//   24576 x  768 x 1536 + 768   90.2 / 84.7     32768 x  768 x 1536 + 768    110 / 113*
+//    4992 x 1024 x 2048 + 1024  41.9 / 34.7     10304 x 1024 x 2048 + 1024  70.7 / 62.7
+//   12288 x 1024 x 2048 + 1024  70.7 / 73.6*    16384 x 1024 x 2048 + 1024  91.9 / 88.6
+//    6144 x 2048 x 4096 + 2048   128 / 131*     10304 x 2048 x 4096 + 2048   233 / 210
+// (* two are launched).
+static const RowsTile* rows_pair(const RowsGemmArgs& g, int w_dtype, int code) {
+  const bool narrow = g.K <= 768;
+  const RowsTile& t =
+      rows_tile(g.M, g.N, w_dtype == T5D_I8 || (code == 0 && narrow) ? 1 : code, g.N2);
+  if (code != 0) return &t;
+  const int64_t wgs = (int64_t)((g.M + t.rows - 1) / t.rows) *
+                      ((g.N + t.cols - 1) / t.cols + (g.N2 + t.cols - 1) / t.cols);
+  if (wgs > 5 * 256 * t.per_cu) return nullptr;
+  if (!narrow && wgs > 2 * 256 * t.per_cu) {
+    const int any = w_dtype == T5D_I8 ? 1 : 0;
+    const double apart = rows_tile_cost(rows_tile(g.M, g.N, any), g.M, g.N) +
+                         rows_tile_cost(rows_tile(g.M, g.N2, any), g.M, g.N2);
+    if (rows_tile_cost(t, g.M, g.N, g.N2) > 1.03 * apart) return nullptr;
+  }
+  return &t;
+}
+
+template <int NORM>
+static void launch_rows_pair(hipStream_t s, const RowsGemmArgs& g, int w_dtype, int code) {
+  const RowsTile* tile = rows_pair(g, w_dtype, code);
+  if (tile == nullptr) {
+    RowsGemmArgs one = g;
+    one.layout = T5D_OUT_ROWS;
+    launch_rows_direct<true, 0, NORM>(s, one, w_dtype, 0);
+    one.layout = T5D_OUT_HEADS_VALUE;
+    one.W = g.W2; one.scales = g.scales2; one.C = g.C2; one.N = g.N2;
+    launch_rows_direct<false, 0, NORM>(s, one, w_dtype, 0);
+    return;
+  }
+  const RowsTile& t = *tile;
+  const dim3 grid((unsigned)((g.M + t.rows - 1) / t.rows) *
+                  ((g.N + t.cols - 1) / t.cols + (g.N2 + t.cols - 1) / t.cols));
+#define T5D_ROWS_LAUNCH(WT_, MT_, NT_, OCC_)                                     \
+  hipLaunchKernelGGL((rows_gemm_pair_kernel<WT_, MT_, NT_, OCC_, NORM>), grid,   \
+                     dim3(256), 0, s, g)
+  if constexpr (NORM == 0) {
     if (w_dtype == T5D_I8) {
       if (t.rows == 64) T5D_ROWS_LAUNCH(int8_t, 4, 2, 4);
       else T5D_ROWS_LAUNCH(int8_t, 8, 2, 3);
@@ -939,7 +1059,10 @@ static int launch_rows(hipStream_t s, int w_dtype, const RowsGemmArgs& g,
   const dim3 grid((unsigned)m_blocks * n_blocks), block(256);
   const bool swap = g.layout != T5D_OUT_HEADS_VALUE;
   const int dense = g.epilogue == T5D_EPI_CLAMPED_GLU ? 1 : g.C32 != nullptr ? 2 : 0;
-  if (g.squares_in != nullptr) {  // (rows_direct is the caller's)
+  if (g.N2 > 0) {  // (rows_direct is the caller's)
+    if (g.squares_in != nullptr) launch_rows_pair<1>(s, g, w_dtype, tile);
+    else launch_rows_pair<0>(s, g, w_dtype, tile);
+  } else if (g.squares_in != nullptr) {
     if (swap) launch_rows_direct<true, 0, 1>(s, g, w_dtype, tile);
     else launch_rows_direct<false, 0, 1>(s, g, w_dtype, tile);
   } else if (g.squares_out != nullptr) {
@@ -980,7 +1103,8 @@ extern "C" int t5d_gemm_rows(void* stream, int w_dtype, const void* A,
 static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
                      const float* scales, const void* residual, void* C, int64_t M,
                      int K, int N, int epilogue, int out_layout, int E, int Ep,
-                     const int32_t* at, int tile, const t5d_rows_norm* norm = nullptr) {
+                     const int32_t* at, int tile, const t5d_rows_norm* norm = nullptr,
+                     const t5d_rows_second* second = nullptr) {
   T5D_REQUIRE(A && W && C, T5D_EINVAL, "t5d_gemm_rows: null pointer");
   T5D_REQUIRE(tile >= 0 && tile <= 3, T5D_EINVAL,
               "t5d_gemm_rows_tiled: tile %d (0 chosen here, columns: 1: 128, "
@@ -1004,13 +1128,14 @@ static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
               T5D_EINVAL, "t5d_gemm_rows: operand alignment");
   int H = 0;
   if (out_layout != T5D_OUT_ROWS) {
-    T5D_REQUIRE(epilogue == T5D_EPI_NONE && N % 64 == 0 && E > 0 && Ep >= E &&
+    T5D_REQUIRE(epilogue == T5D_EPI_NONE && (second ? second->N : N) % 64 == 0 &&
+                    E > 0 && Ep >= E &&
                     (at ? M % 4 == 0 : M % E == 0 && E % 4 == 0) && Ep % 32 == 0,
                 T5D_EINVAL,
                 "t5d_gemm_rows: heads layout needs epilogue none, N %% 64 == 0,"
                 " M %% E == 0, E %% 4 == 0, Ep %% 32 == 0 (N=%d E=%d Ep=%d)", N,
                 E, Ep);
-    H = N / 64;
+    H = (second ? second->N : N) / 64;
   }
   RowsGemmArgs g = {};
   g.A = (const bf16_t*)A; g.W = (const char*)W;
@@ -1024,6 +1149,8 @@ static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
   g.gate = nullptr; g.grp = GroupTiles(); g.n_tiles = 0;
   if (norm != nullptr) {
     T5D_REQUIRE(rows_direct(K, K), T5D_ELIMIT, "t5d_gemm_rows_normed: K=%d", K);
+    T5D_REQUIRE(w_dtype == T5D_BF16, T5D_EINVAL, "t5d_gemm_rows_normed: w_dtype %d",
+                w_dtype);
     T5D_REQUIRE(norm->squares && (norm->scale == nullptr) == (norm->scaled == nullptr) &&
                     ((uintptr_t)norm->scale % 16) == 0 &&
                     ((uintptr_t)norm->scaled % 16) == 0,
@@ -1042,7 +1169,27 @@ static int gemm_rows(void* stream, int w_dtype, const void* A, const void* W,
       g.norm_d = (float)K; g.eps = norm->eps;
     }
   }
+  if (second != nullptr) {
+    T5D_REQUIRE(rows_direct(K, K), T5D_ELIMIT, "t5d_gemm_rows_pair: K=%d", K);
+    T5D_REQUIRE(second->W && second->C && second->N > 0 &&
+                    (w_dtype != T5D_I8 || second->scales) &&
+                    ((uintptr_t)second->W % 16) == 0 && ((uintptr_t)second->C % 8) == 0 &&
+                    ((uintptr_t)C % 16) == 0 && (!norm || !norm->scale),
+                T5D_EINVAL, "t5d_gemm_rows_pair: second layer, N=%d", second->N);
+    g.W2 = (const char*)second->W; g.C2 = (bf16_t*)second->C; g.N2 = second->N;
+    g.scales2 = w_dtype == T5D_I8 ? second->scales : nullptr;
+  }
   return launch_rows(as_stream(stream), w_dtype, g, tile);
+}
+
+extern "C" int t5d_gemm_rows_pair(void* stream, int w_dtype, const void* A, const void* W,
+                                  const float* scales, void* C, int64_t M, int K, int N,
+                                  int E, int Ep, const int32_t* at, int tile,
+                                  const t5d_rows_second* second,
+                                  const t5d_rows_norm* norm) {
+  T5D_REQUIRE(second, T5D_EINVAL, "t5d_gemm_rows_pair: null pointer");
+  return gemm_rows(stream, w_dtype, A, W, scales, nullptr, C, M, K, N, T5D_EPI_NONE,
+                   T5D_OUT_HEADS_VALUE, E, Ep, at, tile, norm, second);
 }
 
 extern "C" int t5d_gemm_rows_takes_norm(int K) { return K > 0 && rows_direct(K, K); }

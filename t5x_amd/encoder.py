@@ -58,12 +58,14 @@ class EncoderKernelWeights:
 
 def _layers(cfg, w, x, v_t, E, rows, attend):
   """The encoder's layers over x, rows of texts of E positions each or those of an
-  EncoderRows; attend(q | k) with the values in v_t.  The norms between
-  layers ride in the dense layers on both sides of them (widths of 32 have their own
-  pass)."""
+  EncoderRows; attend(q | k) with the values in v_t.  The norms between layers ride in the
+  dense layers on both sides of them, but not with int8 weights, which keep the vector
+  units busy (8192 rows of 2048: v 75 us, with the norm inside 83, the gated layer 312 and
+  320; a pass of its own takes 15 for the two of them), nor over 32 inputs."""
   from t5x_amd import _lib, ops
-  Ep = v_t.shape[2] * 32
-  inside = ops.takes_norm(cfg.emb_dim, cfg.num_heads * 64, cfg.mlp_dim)
+  pair = ops.takes_norm(cfg.emb_dim)
+  inside = (pair and ops.takes_norm(cfg.num_heads * 64, cfg.mlp_dim) and
+            (cfg.weight_dtype or cfg.dtype) == 'bfloat16')
 
   def residual_and_norm(a, kernel, x, scale):
     if inside:
@@ -77,14 +79,16 @@ def _layers(cfg, w, x, v_t, E, rows, attend):
 
   xn = ops.rmsnorm(x, w.layers[0]['ln_attn']) if w.layers else None
   for i, l in enumerate(w.layers):
-    qk = dense(xn, l['qk'])                               # [M, q | k]
-    if isinstance(xn, ops.ScaledRows):
-      ops.gemm_rows_of_scaled(xn, l['v'], out=v_t, layout=_lib.OUT_HEADS_VALUE, E=E,
-                              Ep=Ep, at=None if rows is None else rows.at)
-    elif rows is not None:
-      ops.gemm_rows_values(xn, l['v'], rows, out=v_t)
+    if pair:
+      qk = ops.gemm_rows_pair(xn, l['qk'], l['v'], v_t, E,    # [M, q | k]
+                              at=None if rows is None else rows.at)
     else:
-      ops.gemm_rows(xn, l['v'], out=v_t, layout=_lib.OUT_HEADS_VALUE, E=E, Ep=Ep)
+      qk = ops.gemm_rows(xn, l['qk'])
+      if rows is not None:
+        ops.gemm_rows_values(xn, l['v'], rows, out=v_t)
+      else:
+        ops.gemm_rows(xn, l['v'], out=v_t, layout=_lib.OUT_HEADS_VALUE, E=E,
+                      Ep=v_t.shape[2] * 32)
     x, y = residual_and_norm(attend(qk), l['o'], x, l['ln_mlp'])
     h = dense(y, l['wi'])
     if i + 1 < len(w.layers):

@@ -555,19 +555,42 @@ def gemm_rows_residual_norm(a, w: PackedWeight, residual, scale, eps=1e-6):
   return x, ScaledRows(scaled, squares, eps)
 
 
-def gemm_rows_of_scaled(rows: ScaledRows, w: PackedWeight, out=None,
-                        layout=_lib.OUT_ROWS, E=0, Ep=0, at=None):
-  """gemm_rows of the rows that ScaledRows stands for; with layout OUT_HEADS_VALUE (and
-  at of an EncoderRows, as gemm_rows_values) into `out`."""
-  if layout == _lib.OUT_ROWS:
-    out = torch.empty((rows.x.shape[0], w.out_features), dtype=rows.x.dtype,
-                      device=rows.x.device)
-  elif out is None:
-    raise ValueError('the value layout needs out')
-  _chk(out, 'out', rows.x.dtype)
+def gemm_rows_of_scaled(rows: ScaledRows, w: PackedWeight):
+  """gemm_rows of the rows that ScaledRows stands for."""
+  out = torch.empty((rows.x.shape[0], w.out_features), dtype=rows.x.dtype,
+                    device=rows.x.device)
   norm = _lib.RowsNorm(None, None, None, rows.eps)
   _rows_normed(rows.x, rows.squares, w, None, out, EPI_GEGLU if w.geglu else EPI_NONE,
-               layout, E, Ep, at, norm)
+               _lib.OUT_ROWS, 0, 0, None, norm)
+  return out
+
+
+def gemm_rows_pair(a, w: PackedWeight, v: PackedWeight, v_out, E, at=None, tile=0):
+  """Two layers over a [M, K] or ScaledRows in one launch: gemm_rows of w -> [M, N], and
+  that of v in the value layout into v_out [B, H, Ep/32, 64, 32], texts of E positions
+  each or the rows that `at` of an EncoderRows places."""
+  rows = a if isinstance(a, ScaledRows) else None
+  a = rows.x if rows else a
+  _chk(a, 'a', torch.bfloat16, 2)
+  _chk(v_out, 'v_out', torch.bfloat16, 5)
+  M, K = a.shape
+  B, H, blocks, D, width = v_out.shape
+  if (K != w.K or K != v.K or w.w_dtype == F32 or w.w_dtype != v.w_dtype or w.geglu or
+      v.geglu or (H * 64, D, width) != (v.N, 64, 32) or
+      (at is None and M != B * E) or (at is not None and M != 4 * at.shape[0])):
+    raise ValueError(f'a [{M}, {K}], kernels K={w.K}, {v.K}, N={w.N}, {v.N}, v_out '
+                     f'{tuple(v_out.shape)} of {E} positions')
+  norm = None
+  if rows is not None:
+    _chk(rows.squares, 'squares', torch.float32, 2)
+    if tuple(rows.squares.shape) != ((K + 63) // 64, M):
+      raise ValueError(f'squares {tuple(rows.squares.shape)} of {M} rows of {K}')
+    norm = _lib.RowsNorm(None, None, rows.squares.data_ptr(), rows.eps)
+  out = torch.empty((M, w.N), dtype=a.dtype, device=a.device)
+  second = _lib.RowsSecond(v.data.data_ptr(), _lib.ptr(v.scales), v_out.data_ptr(), v.N)
+  _lib.call('t5d_gemm_rows_pair', _s(), w.w_dtype, a.data_ptr(), w.data.data_ptr(),
+            _lib.ptr(w.scales), out.data_ptr(), M, K, w.N, E, 32 * blocks, _lib.ptr(at),
+            int(tile), second, norm)
   return out
 
 

@@ -298,8 +298,7 @@ def _check_head_layouts(ops, rows, keys, vals, B, E, Ep, H):
 # 64 whose squares go together, more than 16 such parts, tiles of 64 rows
 @pytest.mark.parametrize('M,D,N', [(1, 64, 64), (77, 96, 128), (300, 224, 192),
                                    (1001, 768, 1536), (129, 1088, 320), (40, 2048, 64)])
-@pytest.mark.parametrize('wd', [torch.bfloat16, torch.int8])
-def test_gemm_rows_with_the_norm_between_them(ops, M, D, N, wd):
+def test_gemm_rows_with_the_norm_between_them(ops, M, D, N):
   """x = a W + residual, then norm(x) W2, plain, gated and in the value layout, the norm
   inside the two layers: x has the bits of the layer without it, squares are sums of 64
   terms (64 x 2^-24 off float64's), scaled rows round x scale once, and a result lies as
@@ -313,9 +312,9 @@ def test_gemm_rows_with_the_norm_between_them(ops, M, D, N, wd):
   K = 96
   a, res = rnd(M, K).to(bf), (3 * rnd(M, D)).to(bf)
   scale = (1 + 0.3 * rnd(D)).to(bf)
-  w1 = ops.pack_weight(rnd(K, D) * K ** -0.5, bf, wd)
+  w1 = ops.pack_weight(rnd(K, D) * K ** -0.5, bf)
   k2, k3 = rnd(D, N) * D ** -0.5, rnd(D, N) * D ** -0.5
-  plain, gated = (ops.pack_weight(k2, bf, wd, **o) for o in ({}, {'gate_kernel': k3}))
+  plain, gated = (ops.pack_weight(k2, bf, **o) for o in ({}, {'gate_kernel': k3}))
   x, y = ops.gemm_rows_residual_norm(a, w1, res, scale)
   assert torch.equal(x, ops.gemm_rows(a, w1, residual=res))
   assert torch.equal(y.x, (x.float() * scale.float()).to(bf))
@@ -331,11 +330,7 @@ def test_gemm_rows_with_the_norm_between_them(ops, M, D, N, wd):
     assert all(torch.equal(p, q) for p, q in zip(again, (x, y.x, y.squares))), tile
   xd = x.double()
   normed = xd / torch.sqrt((xd ** 2).mean(1, keepdim=True) + 1e-6) * scale.double()
-  def kernel(k):
-    if wd == bf:
-      return k.to(bf).double()
-    s = k.abs().amax(0).clamp_min(1e-30) / 127
-    return (k / s).round().clamp(-127, 127).double() * s.double()
+  kernel = lambda k: k.to(bf).double()
   def near(got, want, spread):
     bound = 2.0**-8 * want.abs() + (6 * 2.0**-9 + D * 2.0**-24) * spread
     assert bool(((got.double() - want).abs() <= bound).all())
@@ -349,12 +344,49 @@ def test_gemm_rows_with_the_norm_between_them(ops, M, D, N, wd):
     near(ops.gemm_rows_of_scaled(y, gated), act * u,
          size(kernel(k2)) * u.abs() * 1.2 + size(kernel(k3)) * act.abs() + (act * u).abs())
   if M % 4 == 0:
-    E, Ep, H = M // 4 if M % 16 == 0 else M, 0, N // 64
+    E, H = M // 4 if M % 16 == 0 else M, N // 64
     Ep = (E + 31) // 32 * 32
     v = torch.zeros((M // E, H, Ep // 32, 64, 32), dtype=bf, device='cuda')
-    ops.gemm_rows_of_scaled(y, plain, out=v, layout=_lib.OUT_HEADS_VALUE, E=E, Ep=Ep)
+    # two layers in one launch, whole blocks of columns and others
+    for other in (plain, ops.pack_weight(k3[:, :N - 16].contiguous(), bf)):
+      for tile in (0, 1, 2, 3):
+        v.zero_()
+        both = ops.gemm_rows_pair(y, other, plain, v, E, tile=tile)
+        rows = v.transpose(3, 4).reshape(M // E, H, Ep, 64)[:, :, :E]
+        assert torch.equal(rows.transpose(1, 2).reshape(M, N), got), tile
+        assert torch.equal(both, ops.gemm_rows_of_scaled(y, other)), tile
+    both = ops.gemm_rows_pair(y.x, other, plain, v, E)
+    assert torch.equal(both, ops.gemm_rows(y.x, other))
     rows = v.transpose(3, 4).reshape(M // E, H, Ep, 64)[:, :, :E]
-    assert torch.equal(rows.transpose(1, 2).reshape(M, N), got)
+    assert torch.equal(rows.transpose(1, 2).reshape(M, N), ops.gemm_rows(y.x, plain))
+
+
+@pytest.mark.parametrize('M,K,N', [(256, 512, 768), (1024, 512, 768),
+                                   (32768, 512, 1536), (12288, 1024, 2048)])
+@pytest.mark.parametrize('wd', [torch.bfloat16, torch.int8])
+def test_gemm_rows_pair_in_one_launch_and_in_two(ops, M, K, N, wd):
+  """Two layers over the same rows where one launch is chosen, where there are too many
+  rounds of workgroups for it, and where the two fit theirs better: the bits of the layers
+  on their own."""
+  from t5x_amd import _lib
+  gen = torch.Generator(device='cuda')
+  gen.manual_seed(M + K)
+  rnd = lambda *s: torch.randn(s, generator=gen, device='cuda')
+  a = rnd(M, K).bfloat16()
+  w, v = (ops.pack_weight(rnd(K, n) * K ** -0.5, torch.bfloat16, wd) for n in (N, N // 2))
+  y = ops.ScaledRows(a, 64 * torch.rand((K // 64, M), generator=gen, device='cuda'), 1e-6)
+  E, H = M // 8, N // 128
+  make = lambda: torch.zeros((8, H, E // 32, 64, 32), dtype=a.dtype, device='cuda')
+  for rows, one in ((a, lambda k: ops.gemm_rows(a, k)),
+                    (y, lambda k: ops.gemm_rows_of_scaled(y, k))):
+    if rows is y and wd == torch.int8:
+      with pytest.raises(ValueError):
+        ops.gemm_rows_pair(rows, w, v, make(), E)
+      continue
+    values = make()
+    assert torch.equal(ops.gemm_rows_pair(rows, w, v, values, E), one(w))
+    got = values.transpose(3, 4).reshape(8, H, E, 64).transpose(1, 2).reshape(M, N // 2)
+    assert torch.equal(got, one(v))
 
 
 def _against_float64(ops, out, q, k, v_t, rel_bias, lens, bits):
