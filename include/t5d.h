@@ -811,6 +811,16 @@ int t5d_embed_sinusoid(void* stream, int dtype, const void* table,
                        const int32_t* ids, const int32_t* positions, float* out,
                        float* out2, int M, int d, int ld, int V);
 
+/* t5d_stream_norm (y of bfloat16 or NULL, no add, x0 or rows) and t5d_dense behind it in one
+ * launch, with their bits: x_out [M, ld] = x + rms(y) * y_norm (another buffer than x; not
+ * written if y is NULL), C = the layer over rms(x_out) * norm.  bfloat16 only, up to
+ * t5d_stream_dense_rows rows (0: not for this dtype or ld). */
+int t5d_stream_dense_rows(int dtype, int ld);
+int t5d_stream_dense(void* stream, const void* y, const float* y_norm, const float* x,
+                     float* x_out, const float* norm, int d, float eps, const void* W,
+                     int out_dtype, void* C, int ldc, int n_store, int M, int ld, int N,
+                     int epilogue, float glu_limit, float glu_alpha, float glu_add);
+
 /* The row kernel between two dense layers of a float32 residual stream x [M, ld]:
  *   x += rms(y) * y_norm   (y [M, ld] of y_dtype; y_norm NULL: x += y; y NULL: no)
  *   x += add               (add [d] or NULL)
@@ -994,6 +1004,8 @@ typedef struct {
   int64_t workspace_bytes;
   float* trace;            /* NULL or [n_runs, M, ld]: x after every run */
   const int32_t* gate;     /* as t5d_model_step */
+  float* x2;               /* [M, ld] beside x (streams 0), or NULL: with it steps of a few
+                              rows take t5d_stream_dense */
 } t5d_hybrid_model;
 
 /* Runs the tokens of `batch` through the model.  Logits [n_want, V] of the tokens

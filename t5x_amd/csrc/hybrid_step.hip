@@ -2,7 +2,10 @@
 // attention, latent attention and recurrent layers, for portions of any lengths.
 // Between two dense layers there is one row kernel (t5d_stream_norm, or
 // t5d_hyper_norm for models with several streams) that adds the previous branch to
-// the float32 residual and norms it for the next one.
+// the float32 residual and norms it for the next one; for a few rows it and the dense layer
+// behind it are one launch (t5d_stream_dense).
+#include <utility>
+
 #include "common.h"
 
 using namespace t5d;
@@ -189,12 +192,32 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
     a.rows = c.rows; a.gate_w = c.gate_w; a.gate_out = c.gate;
     return t5d_hyper_norm_run(stream, &a, n);
   };
+  // The stream: in m->x, or with few rows in m->x and m->x2 in turn.
+  const bool few = m->x2 && !hyper && !looped && !m->trace &&
+                   M <= t5d_stream_dense_rows(dt, ld);
+  float *x = m->x, *other = m->x2;
   auto row = [&](const float* add, const float* norm, const float* x0, void* out) {
-    const int rc = t5d_stream_norm(stream, dt, dt, y, y_norm, add, m->x, norm, x0,
+    const int rc = t5d_stream_norm(stream, dt, dt, y, y_norm, add, x, norm, x0,
                                    nullptr, out, M, d, ld, m->eps);
     y = nullptr;
     y_norm = nullptr;
     return rc;
+  };
+  // The waiting branch added, the stream normed, and a layer over it.
+  auto row_dense = [&](const float* norm, const void* w, int out_dtype, void* out, int ldc,
+                       int n_store, int n, int epilogue, float limit, float alpha,
+                       float add) {
+    if (few) {
+      T5D_TRY(t5d_stream_dense(stream, y, y_norm, x, other, norm, d, m->eps, w, out_dtype,
+                               out, ldc, n_store, M, ld, n, epilogue, limit, alpha, add));
+      if (y) std::swap(x, other);
+      y = nullptr;
+      y_norm = nullptr;
+      return (int)T5D_OK;
+    }
+    T5D_TRY(row(nullptr, norm, nullptr, m->h));
+    return t5d_dense(stream, dt, out_dtype, m->h, ld, w, out, ldc, n_store, M, ld, n,
+                     epilogue, limit, alpha, add);
   };
   auto branch = [&](const void* in, int k, const void* w, const float* norm) {
     y = m->y;
@@ -210,12 +233,17 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
       T5D_TRY(t5d_dense(stream, dt, T5D_F32, m->cat, 2 * ld, m->loop_in, m->x, ld,
                         ld, M, 2 * ld, ld, T5D_EPI_NONE, 0.f, 0.f, 0.f));
     }
-    if (hyper)
-      T5D_TRY(collect({l.in1, l.norm1, m->h}, M));
-    else
-      T5D_TRY(row(run.enter ? run.enter_add : nullptr, l.norm1, nullptr, m->h));
-    T5D_TRY(t5d_dense(stream, dt, dt, m->h, ld, l.proj, m->proj, l.proj_n, l.proj_n,
-                      M, ld, l.proj_n, T5D_EPI_NONE, 0.f, 0.f, 0.f));
+    if (hyper || run.enter) {
+      if (hyper)
+        T5D_TRY(collect({l.in1, l.norm1, m->h}, M));
+      else
+        T5D_TRY(row(run.enter_add, l.norm1, nullptr, m->h));
+      T5D_TRY(t5d_dense(stream, dt, dt, m->h, ld, l.proj, m->proj, l.proj_n, l.proj_n,
+                        M, ld, l.proj_n, T5D_EPI_NONE, 0.f, 0.f, 0.f));
+    } else {
+      T5D_TRY(row_dense(l.norm1, l.proj, dt, m->proj, l.proj_n, l.proj_n, l.proj_n,
+                        T5D_EPI_NONE, 0.f, 0.f, 0.f));
+    }
     if (l.low) {
       const char* a = (const char*)m->proj + (size_t)l.off_low * (dt == T5D_F32 ? 4 : 2);
       T5D_TRY(t5d_dense(stream, dt, T5D_F32, a, l.proj_n, l.low, m->low, l.low_n,
@@ -240,12 +268,15 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
       wait.mix = l.mix2; wait.spread = l.out2;
     }
     if (l.glu) {
-      if (hyper)
+      if (hyper) {
         T5D_TRY(collect({l.in2, l.norm2, m->h}, M));
-      else
-        T5D_TRY(row(nullptr, l.norm2, nullptr, m->h));
-      T5D_TRY(t5d_dense(stream, dt, dt, m->h, ld, l.glu, l.ff_rows, l.F, 2 * l.F, M,
-                        ld, 2 * l.F, T5D_EPI_CLAMPED_GLU, l.glu_limit, l.glu_alpha, l.glu_add));
+        T5D_TRY(t5d_dense(stream, dt, dt, m->h, ld, l.glu, l.ff_rows, l.F, 2 * l.F, M, ld,
+                          2 * l.F, T5D_EPI_CLAMPED_GLU, l.glu_limit, l.glu_alpha,
+                          l.glu_add));
+      } else {
+        T5D_TRY(row_dense(l.norm2, l.glu, dt, l.ff_rows, l.F, 2 * l.F, 2 * l.F,
+                          T5D_EPI_CLAMPED_GLU, l.glu_limit, l.glu_alpha, l.glu_add));
+      }
       T5D_TRY(branch(l.ff_rows, l.F, l.down, l.norm2b));
       if (hyper) {
         wait.y = m->y; wait.mix = l.mix2; wait.spread = l.out2;
@@ -270,11 +301,12 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
     T5D_TRY(collect({nullptr, m->final_norm, m->h, nullptr, want_rows}, n_want));
   } else if (want_rows) {
     if (y) T5D_TRY(row(nullptr, nullptr, nullptr, nullptr));
-    T5D_TRY(t5d_stream_norm(stream, dt, dt, nullptr, nullptr, nullptr, m->x,
+    T5D_TRY(t5d_stream_norm(stream, dt, dt, nullptr, nullptr, nullptr, x,
                             m->final_norm, nullptr, want_rows, m->h, n_want, d, ld,
                             m->eps));
   } else {
-    T5D_TRY(row(nullptr, m->final_norm, nullptr, m->h));
+    return row_dense(m->final_norm, m->head, T5D_F32, logits, m->V, m->V, m->head_n,
+                     T5D_EPI_NONE, 0.f, 0.f, 0.f);
   }
   return t5d_dense(stream, dt, T5D_F32, m->h, ld, m->head, logits, m->V, m->V, n_want,
                    ld, m->head_n, T5D_EPI_NONE, 0.f, 0.f, 0.f);

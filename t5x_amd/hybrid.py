@@ -706,6 +706,9 @@ class _Buffers:
     lib = _lib.load()
     f32 = torch.float32
     self.x = rows(ld * max(1, cfg.streams), f32)
+    # (the stream of few rows goes back and forth between two buffers)
+    few = lib.t5d_stream_dense_rows(_lib.dtype_code(act), ld)
+    self.x2 = rows(ld, f32) if not cfg.streams and tokens <= few else None
     self.h, self.y = rows(ld), rows(ld)
     self.x0, self.cat = ((rows(ld, f32), rows(2 * ld)) if cfg.loop else
                          (None, None))
@@ -966,7 +969,7 @@ class HybridDecoder(network.DecodeContexts):
     mod.head, mod.final_norm = w.head, w.final_norm
     mod.layers, mod.runs = layers, cruns
     for name in ('x', 'x0', 'low', 'h', 'cat', 'proj', 'q_rows', 'y',
-                 'workspace'):
+                 'workspace', 'x2'):
       setattr(mod, name, P(getattr(bufs, name)))
     mod.workspace_bytes = bufs.workspace.numel()
     mod.gate = P(gate)

@@ -157,6 +157,60 @@ def test_stream_norm(dt, M, width, ld):
   np.testing.assert_allclose(host(x), before + host(y), rtol=2e-6, atol=1e-5)
 
 
+# (width, row, columns, kind): rows in one and two groups of 4 columns per thread, 1 to 8
+# pairs of k-tiles per wavefront and fewer pairs than wavefronts, one column tile per
+# workgroup and two, a last workgroup with one
+@pytest.mark.parametrize('width,ld,N,kind', [
+    (64, 64, 16, 'plain'), (500, 512, 96, 'glu'), (570, 576, 64, 'plain'),
+    (1000, 1024, 80, 'glu'), (1021, 1024, 8208, 'f32'), (1030, 1088, 48, 'f32'),
+    (2048, 2048, 160, 'glu')])
+@pytest.mark.parametrize('M', [1, 2, 3, 4])
+def test_stream_norm_and_the_layer_behind_it_in_one_launch(width, ld, N, kind, M):
+  """t5d_stream_dense has the bits of t5d_stream_norm and t5d_dense, with a branch and its
+  norm, without the norm, and without a branch."""
+  from t5x_amd import _lib, ops
+  rs = np.random.RandomState(ld + N + M)
+  pad = lambda x: np.pad(x, ((0, 0), (0, ld - width)))
+  x = dev(pad(3 * rs.randn(M, width)))
+  y = dev(pad(rs.randn(M, width)), torch.bfloat16)
+  wy, w = (dev(rs.randn(width)) for _ in range(2))
+  glu, f32 = kind == 'glu', kind == 'f32'
+  kernel = lambda n: dev(pad(rs.randn(n, width) * width ** -0.5).T.copy())
+  packed = (ops.pack_weight(kernel(N // 2), torch.bfloat16, gate_kernel=kernel(N // 2))
+            if glu else ops.pack_weight(kernel(N), torch.bfloat16))
+  n_store = N - 3 if f32 else N
+  ldc = N // 2 if glu else n_store
+  out_dt = torch.float32 if f32 else torch.bfloat16
+  tail = (_lib.EPI_CLAMPED_GLU if glu else _lib.EPI_NONE, 7.0, 1.702, 1.0)
+  code = _lib.dtype_code(out_dt)
+  for branch, normed in ((y, wy), (y, None), (None, None)):
+    old, h = x.clone(), torch.zeros((M, ld), dtype=torch.bfloat16, device='cuda')
+    want, got = (torch.full((M, ldc), 3.0, dtype=out_dt, device='cuda') for _ in range(2))
+    P = _lib.ptr
+    _lib.call('t5d_stream_norm', ops._s(), 1, 1, P(branch), P(normed), None,
+              old.data_ptr(), w.data_ptr(), None, None, h.data_ptr(), M, width, ld, 1e-5)
+    _lib.call('t5d_dense', ops._s(), 1, code, h.data_ptr(), ld, packed.data.data_ptr(),
+              want.data_ptr(), ldc, n_store, M, ld, N, *tail)
+    new = torch.full_like(x, 5.0)
+    _lib.call('t5d_stream_dense', ops._s(), P(branch), P(normed), x.data_ptr(),
+              new.data_ptr(), w.data_ptr(), width, 1e-5, packed.data.data_ptr(), code,
+              got.data_ptr(), ldc, n_store, M, ld, N, *tail)
+    assert torch.equal(got, want)
+    assert torch.equal(new, old if branch is not None else torch.full_like(x, 5.0))
+
+
+def test_stream_dense_refuses_what_it_does_not_take():
+  from t5x_amd import _lib
+  lib = _lib.load()
+  rows = lib.t5d_stream_dense_rows
+  assert rows(1, 64) == rows(1, 2048) == 4
+  assert rows(0, 64) == rows(1, 96) == rows(1, 2112) == rows(1, 0) == 0
+  call = lambda M, ld, x2=32, d=64: lib.t5d_stream_dense(
+      None, 16, 16, 16, x2, 16, d, 1e-6, 16, 1, 16, 64, 64, M, ld, 64, 0, 0.0, 0.0, 0.0)
+  assert call(5, 64) == call(1, 96) == call(0, 64) == call(1, 64, d=65) == -3
+  assert call(1, 64, x2=16) == call(1, 64, x2=36) == -1
+
+
 # ---- windowed attention ---------------------------------------------------------------
 
 
