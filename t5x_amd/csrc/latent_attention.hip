@@ -113,24 +113,40 @@ __device__ __forceinline__ f32x4_v mfma(const Frag& x, const Frag& y, f32x4_v c)
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, y.v, c, 0, 0, 0);
 }
 
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4_v;
+typedef __attribute__((address_space(3))) s16x4_v* lds_s16x4_t;
+// (a vector of the compiler's: an array of uint4 that is loaded and stored only is copied
+// piece by piece through scratch memory)
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_l;
+
 // A workgroup attends for 16 HG consecutive (token, head) rows of one portion over
-// every splits-th tile of 64 positions.  The tile's latents go to LDS twice: as
-// rows (scores S^T = C Q^T: wavefront w takes positions 16 w ..) and transposed
-// (O^T = C^T P^T: wavefront w takes a quarter of the latent's columns).  Between
-// the two the wavefronts exchange row maxima and weights through LDS; the weights
-// are kept to 16 bits of mantissa as value + remainder.  RP = 32 DT.
+// every splits-th tile of 64 positions.  The tile's latents go to LDS once, as rows: for
+// the scores (S^T = C Q^T: wavefront w takes positions 16 w ..) they are operands as they
+// stand, for the sums (O^T = C^T P^T: wavefront w takes a quarter of the latent's columns)
+// they are read with the transposing LDS read, 16 lanes of which give it 4 positions x 16
+// columns and get 4 positions of a column each.  Between the two the wavefronts exchange
+// row maxima and weights through LDS, the weights of 32 positions in the order of that
+// read: {4 g .. 4 g + 3, 16 + 4 g .. 16 + 4 g + 3} for g = 0 .. 3; they are kept to 16 bits
+// of mantissa as value + remainder.  RP = 32 DT.  Rows are 32 bytes longer than RP columns:
+// 8 rows of 32 bytes (transposing reads) and 16 of 16 bytes then lie in different banks.
+// What bounds it: a tile's way through four barriers with the next tile's loads in flight
+// behind them, four or five tiles per workgroup at a window of 1024.  With the tile in LDS
+// once (it was there transposed too, 32 writes of 8 bytes per thread and 144 KB) 64 rows of
+// one token, 16 heads, latents of 512, window 1024 take 19 us instead of 23 (the bytes alone
+// 13.7), a step of eight such layers 760 us instead of 791.  Two workgroups now fit a CU;
+// twice the parts to fill them were no faster there (764 us) and slower at 300 positions
+// (698 -> 714 us): each part is written and merged.
 template <int DT, int HG>
-__global__ void __launch_bounds__(256, DT >= 16 ? 1 : 2)
+__global__ void __launch_bounds__(256, DT >= 16 && HG > 1 ? 1 : 2)
 latent_tile_kernel(LatentArgs g) {
   constexpr int RP = DT * 32, KB = 64, R = 16 * HG;
-  constexpr int KS = RP + 8, VS = KB + 8, PS = KB + 8;  // LDS row strides
+  constexpr int KS = RP + 16, PS = KB + 8;              // LDS row strides
   constexpr int CT = RP / 16 / 4;                       // column tiles per wavefront
   constexpr int LPR = RP / 8;                           // lanes on one position
   constexpr int PPI = 64 / LPR;                         // positions per load
   constexpr int QUADS = 4 / PPI;                        // 4 positions, per thread
   static_assert(PPI >= 1 && PPI <= 4, "latents of 128, 256 or 512");
   __shared__ __align__(16) bf16_t s_k[KB * KS];         // [position][column]
-  __shared__ __align__(16) bf16_t s_v[RP * VS];         // [column][position]
   __shared__ __align__(16) bf16_t s_p[2][R * PS];       // weights, remainders
   __shared__ float s_max[4][R];
   T5D_GATED(g.gate);
@@ -178,9 +194,8 @@ latent_tile_kernel(LatentArgs g) {
   const int j_step = KB * g.splits;
 
   // A thread loads 8 columns of 4 consecutive positions (whole positions per
-  // wavefront and load: consecutive memory), so the transposed copy takes 8 bytes
-  // per column.  Its 16-byte pieces (8 positions) are XOR-swizzled by the column.
-  uint4 lat[QUADS][4];
+  // wavefront and load: consecutive memory).
+  u32x4_l lat[QUADS][4];
   const int piece = lane % LPR;
   const int quad0 = 4 * wave + lane / LPR;  // positions 4 quad ..
   auto fetch = [&](int jt) {
@@ -189,7 +204,7 @@ latent_tile_kernel(LatentArgs g) {
     for (int i = 0; i < QUADS; ++i)
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        lat[i][k] = *reinterpret_cast<const uint4*>(c + (4 * PPI * i + k) * RP);
+        lat[i][k] = *reinterpret_cast<const u32x4_l*>(c + (4 * PPI * i + k) * RP);
   };
   if (j_begin <= i_hi) fetch(j_begin);
   for (int jt = j_begin; jt <= i_hi; jt += j_step) {
@@ -199,19 +214,7 @@ latent_tile_kernel(LatentArgs g) {
       const int quad = quad0 + PPI * i;
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        *reinterpret_cast<uint4*>(s_k + (4 * quad + k) * KS + 8 * piece) = lat[i][k];
-      bf16_t* dst = s_v + (size_t)(8 * piece) * VS +
-                    8 * ((quad >> 1) ^ ((piece >> 1) & 7)) + 4 * (quad & 1);
-      auto put = [&](int e, uint32_t p, uint32_t q, uint32_t r, uint32_t s) {
-        *reinterpret_cast<uint2*>(dst + (2 * e) * VS) =
-            make_uint2((p & 0xFFFFu) | (q << 16), (r & 0xFFFFu) | (s << 16));
-        *reinterpret_cast<uint2*>(dst + (2 * e + 1) * VS) = make_uint2(
-            (p >> 16) | (q & 0xFFFF0000u), (r >> 16) | (s & 0xFFFF0000u));
-      };
-      put(0, lat[i][0].x, lat[i][1].x, lat[i][2].x, lat[i][3].x);
-      put(1, lat[i][0].y, lat[i][1].y, lat[i][2].y, lat[i][3].y);
-      put(2, lat[i][0].z, lat[i][1].z, lat[i][2].z, lat[i][3].z);
-      put(3, lat[i][0].w, lat[i][1].w, lat[i][2].w, lat[i][3].w);
+        *reinterpret_cast<u32x4_l*>(s_k + (4 * quad + k) * KS + 8 * piece) = lat[i][k];
     }
     __syncthreads();
     if (jt + j_step <= i_hi) fetch(jt + j_step);
@@ -256,7 +259,7 @@ latent_tile_kernel(LatentArgs g) {
       }
       l[hg] = l[hg] * alpha + sum;
       const uint32_t h0 = pack_bf16x2(p[0], p[1]), h1 = pack_bf16x2(p[2], p[3]);
-      const int at = r * PS + 16 * wave + 4 * gq;
+      const int at = r * PS + 32 * (wave >> 1) + 8 * gq + 4 * (wave & 1);
       *reinterpret_cast<uint2*>(s_p[0] + at) = make_uint2(h0, h1);
       *reinterpret_cast<uint2*>(s_p[1] + at) = make_uint2(
           pack_bf16x2(p[0] - bf16lo_to_f32(h0), p[1] - bf16hi_to_f32(h0)),
@@ -278,10 +281,12 @@ latent_tile_kernel(LatentArgs g) {
       }
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        const int tile = CT * wave + ct;  // (two pieces of 8 columns)
-        Frag vf;
-        vf.u = *reinterpret_cast<const uint4*>(
-            s_v + (16 * tile + n16) * VS + 8 * ((4 * kb + gq) ^ (tile & 7)));
+        const bf16_t* v = s_k + (32 * kb + 4 * gq + (n16 >> 2)) * KS +
+                          16 * (CT * wave + ct) + 4 * (n16 & 3);
+        union { s16x4_v h[2]; Frag f; } x;
+        x.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)v);
+        x.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(v + 16 * KS));
+        const Frag vf = x.f;
 #pragma unroll
         for (int hg = 0; hg < HG; ++hg) {
           o[ct][hg] = mfma(vf, hi[hg], o[ct][hg]);
