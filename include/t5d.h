@@ -784,7 +784,9 @@ int t5d_embed_streams(void* stream, int dtype, const void* table,
  *   x[t] = sum_s mix[s, t] x[s] + spread[t] b      (neither y nor parts: x stays)
  *   u = sum_s collect[s] x[s];  sum[m] = u;  out[m] = rms(u) * norm as dtype;
  *   gate_out[m] = sigmoid(gate_w . (rms(u) * norm))
- * mix NULL: the identity; spread, collect NULL: ones.  rows (no y, no parts): row m
+ * mix NULL: the identity; spread, collect NULL: ones.  With first, a branch that was not
+ * written before comes first: x[t] = sum_s mix_first[s, t] x[s] + spread_first[t] first[m].
+ * keep: the outputs are of the new x, x itself stays.  rows (no y, no parts): row m
  * of the outputs comes from x row rows[m].  At most 16 streams; ld a multiple of 8,
  * at most 16384. */
 typedef struct {
@@ -801,6 +803,9 @@ typedef struct {
   float* sum;                /* [M, ld] or NULL */
   const float* gate_w;       /* [d] or NULL */
   float* gate_out;           /* [M] */
+  const void* first;         /* [M, ld] of dtype or NULL; only with y or parts */
+  const float *mix_first, *spread_first;
+  int keep;
 } t5d_hyper_norm;
 int t5d_hyper_norm_run(void* stream, const t5d_hyper_norm* a, int M);
 
@@ -1006,6 +1011,8 @@ typedef struct {
   const int32_t* gate;     /* as t5d_model_step */
   float* x2;               /* [M, ld] beside x (streams 0), or NULL: with it steps of a few
                               rows take t5d_stream_dense */
+  void* y2;                /* [M, ld] beside y, or NULL: with it two to four streams of many
+                              rows are written once a layer */
 } t5d_hybrid_model;
 
 /* Runs the tokens of `batch` through the model.  Logits [n_want, V] of the tokens

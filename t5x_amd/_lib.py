@@ -133,7 +133,8 @@ class HyperNorm(Structure):
   """t5d_hyper_norm."""
   _fields_ = _fields(i='dtype d ld streams top', f='eps part_weight',
                      p='y parts y_gate part_row mix spread collect x norm out '
-                     'rows sum gate_w gate_out')
+                     'rows sum gate_w gate_out first mix_first spread_first',
+                     i2='keep')
 
 
 class LatentAttention(Structure):
@@ -187,7 +188,7 @@ class HybridModel(Structure):
                       p='embedding loop_in head final_norm') +
               [('layers', POINTER(HybridLayer)), ('runs', POINTER(HybridRun))] +
               _fields(p='x x0 low h cat proj q_rows y workspace',
-                      l='workspace_bytes', p2='trace gate x2'))
+                      l='workspace_bytes', p2='trace gate x2 y2'))
 
 
 _P = c_void_p

@@ -185,9 +185,14 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
     const float* gate_w;
     float* gate;
   };
-  auto collect = [&](const Collect& c, int n) {
+  // hold: the streams are not written; the branch waits on, behind the layer's next one.
+  auto collect = [&](const Collect& c, int n, bool hold = false) {
     t5d_hyper_norm a = wait;
     wait = none;
+    if (hold) {
+      a.keep = 1;
+      wait.first = a.y; wait.mix_first = a.mix; wait.spread_first = a.spread;
+    }
     a.collect = c.weights; a.norm = c.norm; a.out = c.out; a.sum = c.sum;
     a.rows = c.rows; a.gate_w = c.gate_w; a.gate_out = c.gate;
     return t5d_hyper_norm_run(stream, &a, n);
@@ -219,10 +224,10 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
     return t5d_dense(stream, dt, out_dtype, m->h, ld, w, out, ldc, n_store, M, ld, n,
                      epilogue, limit, alpha, add);
   };
-  auto branch = [&](const void* in, int k, const void* w, const float* norm) {
-    y = m->y;
+  auto branch = [&](const void* in, int k, const void* w, const float* norm, void* to) {
+    y = to;
     y_norm = norm;
-    return t5d_dense(stream, dt, dt, in, k, w, m->y, ld, ld, M, k, ld, T5D_EPI_NONE,
+    return t5d_dense(stream, dt, dt, in, k, w, to, ld, ld, M, k, ld, T5D_EPI_NONE,
                      0.f, 0.f, 0.f);
   };
   for (int r = 0; r < m->n_runs; ++r) {
@@ -250,14 +255,23 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
                         l.low_n, M, l.low_k, l.low_n, T5D_EPI_NONE, 0.f, 0.f, 0.f));
     }
     T5D_TRY(mixer(stream, m, l, run, b));
-    T5D_TRY(branch(l.mix_rows, l.out_k, l.out, l.norm1b));
+    // Two to four streams of some width, many rows: the row kernel behind the first branch
+    // only reads them, the one behind the second adds both.  us of both, written each time /
+    // once: 8192 rows of 4 x 1024 89.3 / 74.4, 1024 11.7 / 9.8, 512 8.5 / 7.6, 64 5.8 / 5.9;
+    // 2 x 1024 8192 rows 52.1 / 50.5, 512 7.1 / 7.0, 256 6.4 / 6.4, 64 5.8 / 6.0.  Narrower
+    // ones (4 x 256, 8192 rows 28.1 / 30.3), one stream (1024, 4096 rows 15.1 / 16.1) and
+    // more than four, whose weights come through LDS (8 x 1024, 8192 rows 174 / 178), lose.
+    const bool hold = hyper && m->y2 != nullptr && (l.experts.n > 0 || l.glu) &&
+                      m->streams >= 2 && m->streams <= 4 &&
+                      m->streams * ld >= 2048 && M >= 512;
+    T5D_TRY(branch(l.mix_rows, l.out_k, l.out, l.norm1b, hold ? m->y2 : m->y));
     if (hyper) {
-      wait.y = m->y; wait.mix = l.mix1; wait.spread = l.out1;
+      wait.y = hold ? m->y2 : m->y; wait.mix = l.mix1; wait.spread = l.out1;
     }
     if (l.experts.n > 0) {
       const t5d_experts& e = l.experts;
       T5D_TRY(collect({l.in2, l.norm2, m->h, nullptr, nullptr,
-                       e.shared_F ? e.shared_gate : nullptr, e.gate}, M));
+                       e.shared_F ? e.shared_gate : nullptr, e.gate}, M, hold));
       T5D_TRY(experts(stream, m, e, M));
       wait.parts = e.out; wait.part_row = e.entry_of; wait.top = e.top;
       wait.part_weight = 1.0f / (float)e.top;
@@ -269,7 +283,7 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
     }
     if (l.glu) {
       if (hyper) {
-        T5D_TRY(collect({l.in2, l.norm2, m->h}, M));
+        T5D_TRY(collect({l.in2, l.norm2, m->h}, M, hold && l.experts.n == 0));
         T5D_TRY(t5d_dense(stream, dt, dt, m->h, ld, l.glu, l.ff_rows, l.F, 2 * l.F, M, ld,
                           2 * l.F, T5D_EPI_CLAMPED_GLU, l.glu_limit, l.glu_alpha,
                           l.glu_add));
@@ -277,7 +291,7 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
         T5D_TRY(row_dense(l.norm2, l.glu, dt, l.ff_rows, l.F, 2 * l.F, 2 * l.F,
                           T5D_EPI_CLAMPED_GLU, l.glu_limit, l.glu_alpha, l.glu_add));
       }
-      T5D_TRY(branch(l.ff_rows, l.F, l.down, l.norm2b));
+      T5D_TRY(branch(l.ff_rows, l.F, l.down, l.norm2b, m->y));
       if (hyper) {
         wait.y = m->y; wait.mix = l.mix2; wait.spread = l.out2;
       }

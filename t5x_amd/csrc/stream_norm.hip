@@ -237,8 +237,12 @@ struct HyperArgs {
 // One workgroup per row; S streams (template: an upper bound, the real number is
 // a.streams) of VPT groups of 4 columns per thread.  A thread holds one group of
 // columns of every stream at a time and keeps only their weighted sum for the
-// norm.  Columns d .. ld - 1 are zero and stay zero.
-template <typename T, int S, int VPT>
+// norm.  Columns d .. ld - 1 are zero and stay zero.  FIRST: with a first branch.
+// Bound by the streams' bytes (4 x 1024: 32 KB in and out of a token's 38), so a layer of
+// two branches reads them twice and writes them once: the row kernel behind the first
+// branch keeps x, the one behind the second forms it again, from the same sums in the same
+// order.
+template <typename T, int S, int VPT, bool FIRST>
 __global__ void __launch_bounds__(256)
 hyper_norm_kernel(HyperArgs h) {
   T5D_GATE_READ(h.gate);
@@ -252,16 +256,19 @@ hyper_norm_kernel(HyperArgs h) {
   // them through LDS: each by a load and a branch of its own, 2000 rows of 2 x 1024 with
   // 3 parts lasted 10.4 us instead of 9.6.
   constexpr bool kFew = S <= 4;
-  __shared__ float s_far[S * S + 2 * S];
-  float s_near[kFew ? S * S + 2 * S : 1];
+  constexpr int W1 = S * S + 2 * S, W2 = FIRST ? S * S + S : 0;  // mix, spread, collect; the first's
+  __shared__ float s_far[W1 + W2];
+  float s_near[kFew ? W1 + W2 : 1];
+  const auto mixed = [&](const float* mix, int i) {
+    const int from = i / S, to = i % S;
+    return mix != nullptr && from < n && to < n ? mix[from * n + to]
+                                                : from == to ? 1.f : 0.f;
+  };
   const auto weight = [&](int i) {
-    if (i < S * S) {
-      const int from = i / S, to = i % S;
-      return g.mix != nullptr && from < n && to < n ? g.mix[from * n + to]
-                                                    : from == to ? 1.f : 0.f;
-    }
-    const float* w = i < S * S + S ? g.spread : g.collect;
-    const int s = (i - S * S) % S;
+    if (i < S * S) return mixed(g.mix, i);
+    if (i >= W1 && i < W1 + S * S) return mixed(g.mix_first, i - W1);
+    const float* w = i >= W1 ? g.spread_first : i < S * S + S ? g.spread : g.collect;
+    const int s = (i >= W1 ? i - W1 - S * S : i - S * S) % S;
     return s >= n ? 0.f : w != nullptr ? w[s] : 1.f;
   };
   if (kFew && n == S) {
@@ -270,6 +277,20 @@ hyper_norm_kernel(HyperArgs h) {
     for (int i = 0; i < S * S; ++i) s_near[i] = i / S == i % S ? 1.f : 0.f;
 #pragma unroll
     for (int i = 0; i < 2 * S; ++i) s_near[S * S + i] = 1.f;
+    if constexpr (FIRST) {
+      const float *mix1 = g.mix_first, *spread1 = g.spread_first;
+#pragma unroll
+      for (int i = 0; i < W2; ++i)
+        s_near[W1 + i] = i >= S * S || i / S == i % S ? 1.f : 0.f;
+      if (mix1 != nullptr) {
+#pragma unroll
+        for (int i = 0; i < S * S; ++i) s_near[W1 + i] = mix1[i];
+      }
+      if (spread1 != nullptr) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) s_near[W1 + S * S + i] = spread1[i];
+      }
+    }
     if (mix != nullptr) {
 #pragma unroll
       for (int i = 0; i < S * S; ++i) s_near[i] = mix[i];
@@ -283,11 +304,11 @@ hyper_norm_kernel(HyperArgs h) {
       for (int i = 0; i < S; ++i) s_near[S * S + S + i] = collect[i];
     }
   } else {
-    for (int i = threadIdx.x; i < S * S + 2 * S; i += 256) s_far[i] = weight(i);
+    for (int i = threadIdx.x; i < W1 + W2; i += 256) s_far[i] = weight(i);
     __syncthreads();
     if constexpr (kFew) {
 #pragma unroll
-      for (int i = 0; i < S * S + 2 * S; ++i) s_near[i] = s_far[i];
+      for (int i = 0; i < W1 + W2; ++i) s_near[i] = s_far[i];
     }
   }
   const float* s_mix = kFew ? s_near : s_far;
@@ -298,6 +319,7 @@ hyper_norm_kernel(HyperArgs h) {
   float* xrow = g.x + (size_t)src * n * g.ld;
   const T* y = reinterpret_cast<const T*>(g.y);
   const T* parts = reinterpret_cast<const T*>(g.parts);
+  const T* first = reinterpret_cast<const T*>(g.first);
   const float y_gate = add && g.y_gate != nullptr ? g.y_gate[src] : 1.f;
   float4 u[VPT];
 #pragma unroll
@@ -326,6 +348,20 @@ hyper_norm_kernel(HyperArgs h) {
             if (t + k < g.top) fma4(b, g.part_weight, part[k]);
         }
       if (y != nullptr) fma4(b, y_gate, load4<T>(y + (size_t)src * g.ld + c));
+      if constexpr (FIRST) {
+        const float *s_mix1 = s_mix + W1, *s_spread1 = s_mix1 + S * S;
+        const float4 b1 = load4<T>(first + (size_t)src * g.ld + c);
+        float4 x1[S];
+#pragma unroll
+        for (int t = 0; t < S; ++t) {
+          x1[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+          for (int s = 0; s < S; ++s) fma4(x1[t], s_mix1[s * S + t], x[s]);
+          fma4(x1[t], s_spread1[t], b1);
+        }
+#pragma unroll
+        for (int t = 0; t < S; ++t) x[t] = x1[t];
+      }
 #pragma unroll
       for (int t = 0; t < S; ++t) {
         if (t >= n) continue;
@@ -333,7 +369,7 @@ hyper_norm_kernel(HyperArgs h) {
 #pragma unroll
         for (int s = 0; s < S; ++s) fma4(z, s_mix[s * S + t], x[s]);
         fma4(z, s_spread[t], b);
-        *reinterpret_cast<float4*>(xrow + (size_t)t * g.ld + c) = z;
+        if (!g.keep) *reinterpret_cast<float4*>(xrow + (size_t)t * g.ld + c) = z;
         fma4(u[v], s_collect[t], z);
       }
     } else {
@@ -382,11 +418,16 @@ template <typename T, int S>
 static void launch_hyper(hipStream_t s, const HyperArgs& h, int M) {
   const int vpt = (h.a.ld + 1023) / 1024;
 #define T5D_HN(V_) \
-  hipLaunchKernelGGL((hyper_norm_kernel<T, S, V_>), dim3(M), dim3(256), 0, s, h)
-  if (vpt <= 1) T5D_HN(1);
-  else if (vpt <= 2) T5D_HN(2);
-  else if (vpt <= 4) T5D_HN(4);
-  else T5D_HN(16);
+  if (h.a.first)                                                                  \
+    hipLaunchKernelGGL((hyper_norm_kernel<T, S, V_, true>), dim3(M), dim3(256),   \
+                       0, s, h);                                                  \
+  else                                                                            \
+    hipLaunchKernelGGL((hyper_norm_kernel<T, S, V_, false>), dim3(M), dim3(256),  \
+                       0, s, h)
+  if (vpt <= 1) { T5D_HN(1); }
+  else if (vpt <= 2) { T5D_HN(2); }
+  else if (vpt <= 4) { T5D_HN(4); }
+  else { T5D_HN(16); }
 #undef T5D_HN
 }
 
@@ -493,9 +534,11 @@ extern "C" int t5d_hyper_norm_run(void* stream, const t5d_hyper_norm* a, int M) 
               T5D_EINVAL, "t5d_hyper_norm_run: missing operand");
   T5D_REQUIRE(!a->rows || (!a->y && !a->parts), T5D_EINVAL,
               "t5d_hyper_norm_run: picked rows are only read");
+  T5D_REQUIRE(!a->first || a->y || a->parts, T5D_EINVAL,
+              "t5d_hyper_norm_run: a first branch without a second");
   T5D_REQUIRE((((uintptr_t)a->x | (uintptr_t)a->y | (uintptr_t)a->parts |
                 (uintptr_t)a->norm | (uintptr_t)a->out | (uintptr_t)a->sum |
-                (uintptr_t)a->gate_w) % 16) == 0,
+                (uintptr_t)a->gate_w | (uintptr_t)a->first) % 16) == 0,
               T5D_EINVAL, "t5d_hyper_norm_run: operands must be 16-byte aligned");
   HyperArgs h;
   h.a = *a;

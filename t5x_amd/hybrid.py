@@ -710,6 +710,8 @@ class _Buffers:
     few = lib.t5d_stream_dense_rows(_lib.dtype_code(act), ld)
     self.x2 = rows(ld, f32) if not cfg.streams and tokens <= few else None
     self.h, self.y = rows(ld), rows(ld)
+    # (a layer's first branch waits for its second where the streams are many)
+    self.y2 = rows(ld) if cfg.streams > 1 else None
     self.x0, self.cat = ((rows(ld, f32), rows(2 * ld)) if cfg.loop else
                          (None, None))
     self.proj = rows(max(l.proj_n for l in w.layers))
@@ -969,7 +971,7 @@ class HybridDecoder(network.DecodeContexts):
     mod.head, mod.final_norm = w.head, w.final_norm
     mod.layers, mod.runs = layers, cruns
     for name in ('x', 'x0', 'low', 'h', 'cat', 'proj', 'q_rows', 'y',
-                 'workspace', 'x2'):
+                 'workspace', 'x2', 'y2'):
       setattr(mod, name, P(getattr(bufs, name)))
     mod.workspace_bytes = bufs.workspace.numel()
     mod.gate = P(gate)

@@ -1072,22 +1072,24 @@ def embed_streams(table, ids, scale, width, streams):
 
 def hyper_norm(x, width, dtype, y=None, y_gate=None, parts=None, part_row=None,
                part_weight=1.0, mix=None, spread=None, collect=None, norm=None,
-               rows=None, want_sum=False, gate_w=None, eps=1e-6):
+               rows=None, want_sum=False, gate_w=None, eps=1e-6, first=None,
+               mix_first=None, spread_first=None, keep=False):
   """The row kernel over several float32 streams x [M, streams, ld]
   (t5d_hyper_norm): adds the branch y + parts and mixes the streams in place, and
   returns (normed weighted sum as dtype, its float32 sum, sigmoid gate), None where
-  not asked for."""
+  not asked for.  first: a branch that comes before this one; keep: x is not written."""
   _chk(x, 'x', torch.float32, 3)
   M, n, ld = x.shape
   for t, name, shape in (
       (y_gate, 'y_gate', (M,)), (mix, 'mix', (n, n)), (spread, 'spread', (n,)),
       (collect, 'collect', (n,)), (norm, 'norm', (width,)),
+      (mix_first, 'mix_first', (n, n)), (spread_first, 'spread_first', (n,)),
       (gate_w, 'gate_w', (width,))):
     if t is not None:
       _chk(t, name, torch.float32, len(shape))
       if tuple(t.shape) != shape:
         raise ValueError(f'{name} must be {shape}')
-  for t, name, rows_ in ((y, 'y', M), (parts, 'parts', None)):
+  for t, name, rows_ in ((y, 'y', M), (parts, 'parts', None), (first, 'first', M)):
     if t is not None:
       _chk(t, name, dtype, 2)
       if t.shape[1] != ld or (rows_ is not None and t.shape[0] != rows_):
@@ -1113,8 +1115,10 @@ def hyper_norm(x, width, dtype, y=None, y_gate=None, parts=None, part_row=None,
                   ('part_row', part_row), ('mix', mix), ('spread', spread),
                   ('collect', collect), ('x', x), ('norm', norm), ('out', out),
                   ('rows', rows), ('sum', total), ('gate_w', gate_w),
-                  ('gate_out', gate)):
+                  ('gate_out', gate), ('first', first), ('mix_first', mix_first),
+                  ('spread_first', spread_first)):
     setattr(a, name, _lib.ptr(t))
+  a.keep = int(keep)
   _lib.call('t5d_hyper_norm_run', _s(), a, count)
   return out, total, gate
 

@@ -928,6 +928,41 @@ def test_logits_whole_in_portions_and_token_by_token(name, dtype):
 
 
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('streams,width,rows', [(2, 1000, 512), (4, 500, 513),
+                                                (4, 500, 511), (3, 640, 700)])
+def test_streams_written_once_a_layer(monkeypatch, dtype, streams, width, rows):
+  """From 512 rows on a layer's first branch waits for its second: the same bits as
+  without the buffer it waits in.  The second layer has no second branch."""
+  from t5x_amd import hybrid, sequences
+  mixer = lambda i, **kw: cases.latent(2 + i, 16, 16, 24, 72, 33, **kw)
+  cfg = cases.latent_config(width, 101, [
+      cases.moe(mixer(0), 6, 2, 40, 0.8, (72, 1.1)), cases.layer(mixer(1, kv_from=0)),
+      cases.dense(mixer(2), 104), cases.moe(mixer(0, kv_from=2), 5, 3, 24, 2.0)], streams)
+  monkeypatch.setitem(cases.CONFIGS, 'here', cfg)
+  tokens = np.random.RandomState(7).randint(0, 101, rows).tolist()
+  made = hybrid._Buffers.__init__
+
+  def without(self, *args):
+    made(self, *args)
+    assert self.y2 is not None
+    self.y2 = None
+
+  got = []
+  for init in (made, without):
+    monkeypatch.setattr(hybrid._Buffers, '__init__', init)
+    _, params, module = build('here', dtype, max_portion=1024)
+    live = sequences.Sequences(module, params, 1, 1024)
+    trace = []
+    out = live.step([('a', tokens, list(range(rows)))], trace=trace)
+    got.append((host(out), host(trace[0])))
+    again = sequences.Sequences(module, params, 1, 1024)
+    got[-1] += (host(again.step([('b', tokens, [3, rows - 1])])),)
+  for a, b in zip(*got):
+    assert np.array_equal(a, b)
+  assert np.isfinite(got[0][0]).all()
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
 @pytest.mark.parametrize('name', ['all', 'latent', 'latent_plain'])
 def test_residual_stream_after_every_layer_run(name, dtype):
   from t5x_amd import sequences

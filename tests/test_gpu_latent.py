@@ -199,6 +199,40 @@ def test_hyper_norm(dt, M, n, width, ld):
                              atol=1e-5)
 
 
+@pytest.mark.parametrize('M,n,width,ld', [(1, 1, 40, 64), (5, 3, 90, 128),
+                                          (3, 4, 1100, 1152), (7, 4, 1024, 1024),
+                                          (2, 16, 64, 64), (2, 2, 5000, 5056)])
+@pytest.mark.parametrize('dt', DTYPES)
+@pytest.mark.parametrize('plain', [False, True])
+def test_hyper_norm_of_two_branches(dt, M, n, width, ld, plain):
+  """The first branch only looked at, then written with the second: the same sums in the
+  same order, so the same bits as one after the other."""
+  from t5x_amd import ops
+  rs = np.random.RandomState(M + n)
+  x = dev(2 * rs.randn(M, n, ld))
+  one, two, parts = (dev(rs.randn(r, ld), dt) for r in (M, M, 2 * M))
+  part_row = dev(rs.randint(0, 2 * M, (M, 3)), torch.int32)
+  mixes = [None if plain else dev(rs.randn(n, n)) for _ in range(2)]
+  spreads = [None if plain else dev(rs.randn(n)) for _ in range(2)]
+  reads = [dict(collect=dev(rs.randn(n)), norm=dev(rs.randn(width)), want_sum=True)
+           for _ in range(2)]
+  for last in (dict(y=two), dict(parts=parts, part_row=part_row, part_weight=1 / 3),
+               dict(y=two, y_gate=dev(rs.rand(M)), parts=parts, part_row=part_row)):
+    apart, held = x.clone(), x.clone()
+    a = ops.hyper_norm(apart, width, dt, y=one, mix=mixes[0], spread=spreads[0],
+                       **reads[0])
+    b = ops.hyper_norm(held, width, dt, y=one, mix=mixes[0], spread=spreads[0], keep=True,
+                       **reads[0])
+    assert torch.equal(held, x)
+    a += ops.hyper_norm(apart, width, dt, mix=mixes[1], spread=spreads[1], **last,
+                        **reads[1])
+    b += ops.hyper_norm(held, width, dt, mix=mixes[1], spread=spreads[1], first=one,
+                        mix_first=mixes[0], spread_first=spreads[0], **last, **reads[1])
+    assert torch.equal(apart, held)
+    for i in (0, 1, 3, 4):
+      assert torch.equal(a[i], b[i])
+
+
 # ---- latent attention ------------------------------------------------------------------
 
 
