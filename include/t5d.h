@@ -1009,8 +1009,8 @@ typedef struct {
   int64_t workspace_bytes;
   float* trace;            /* NULL or [n_runs, M, ld]: x after every run */
   const int32_t* gate;     /* as t5d_model_step */
-  float* x2;               /* [M, ld] beside x (streams 0), or NULL: with it steps of a few
-                              rows take t5d_stream_dense */
+  float* x2;               /* [t5d_stream_dense_rows, ld] beside x (streams 0), or NULL: with it
+                              steps of so few rows take t5d_stream_dense */
   void* y2;                /* [M, ld] beside y, or NULL: with it two to four streams of many
                               rows are written once a layer */
 } t5d_hybrid_model;

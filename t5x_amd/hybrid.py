@@ -706,9 +706,13 @@ class _Buffers:
     lib = _lib.load()
     f32 = torch.float32
     self.x = rows(ld * max(1, cfg.streams), f32)
-    # (the stream of few rows goes back and forth between two buffers)
+    # (the stream of few rows goes back and forth between two buffers; calls of few rows
+    # may come with buffers that longer ones have left)
     few = lib.t5d_stream_dense_rows(_lib.dtype_code(act), ld)
-    self.x2 = rows(ld, f32) if not cfg.streams and tokens <= few else None
+    self.x2 = None
+    if few and not cfg.streams:
+      self.x2 = torch.empty((few, ld), dtype=f32, device=device)
+      kept.append(self.x2)
     self.h, self.y = rows(ld), rows(ld)
     # (a layer's first branch waits for its second where the streams are many)
     self.y2 = rows(ld) if cfg.streams > 1 else None

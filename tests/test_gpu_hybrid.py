@@ -927,6 +927,30 @@ def test_logits_whole_in_portions_and_token_by_token(name, dtype):
     assert close(got, whole, dtype), cuts
 
 
+@pytest.mark.parametrize('name', ['no_loop', 'odd_values'])
+def test_few_rows_behind_a_long_prompt(monkeypatch, name):
+  """Steps of a few rows take the kernel of norm and layer whatever buffers longer calls
+  have left, with the bits of the two kernels apart."""
+  from t5x_amd import hybrid, sequences
+  monkeypatch.setitem(cases.CONFIGS, name, dict(cases.CONFIGS[name]))
+  cases.CONFIGS[name].pop('loop', None)
+  made = hybrid._Buffers.__init__
+
+  def without(self, *args):
+    made(self, *args)
+    assert self.x2 is not None
+    self.x2 = None
+
+  got = []
+  for init in (made, without):
+    monkeypatch.setattr(hybrid._Buffers, '__init__', init)
+    cfg, params, module = build(name, 'bfloat16')
+    tokens = np.random.RandomState(8).randint(0, cfg['vocab'], 120).tolist()
+    live = sequences.Sequences(module, params, 2, 200)
+    got.append(feed(live, 'a', tokens, [100, 104, 107, 109, 110, 111]))
+  assert np.array_equal(*got)
+
+
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
 @pytest.mark.parametrize('streams,width,rows', [(2, 1000, 512), (4, 500, 513),
                                                 (4, 500, 511), (3, 640, 700)])
