@@ -132,6 +132,7 @@ constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141; // lane i <-> 7 - i within 8
 constexpr int kDppMirror = 0x140;     // lane i <-> 15 - i within 16
+constexpr int kDppRor8 = 0x128;       // lane i <-> i + 8 within 16
 
 constexpr int kDppReverse4 = 0x1B;    // quad_perm [3,2,1,0]
 template <int CTRL>

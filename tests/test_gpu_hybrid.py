@@ -56,6 +56,24 @@ def test_dense_row_strides_and_partial_stores(dt, M):
     assert rel(host(ops.dense(a, packed)), want) < 4e-3
 
 
+@pytest.mark.parametrize('M', [70, 129, 300, 1031])
+@pytest.mark.parametrize('K,N,keep', [(64, 16, 16), (64, 48, 48), (128, 208, 204),
+                                      (96, 208, 201), (64, 2048, 2048), (128, 592, 576),
+                                      (64, 784, 769), (128, 1536, 1535)])
+def test_dense_float32_rows_in_whole_lines(M, K, N, keep):
+  """Odd numbers of column tiles, columns that are not kept, rows that are not there: sums
+  of K products of two bfloat16 numbers, each within K units of 2^-24 of the magnitudes."""
+  from t5x_amd import ops
+  rs = np.random.RandomState(M + N)
+  a = dev(rs.randn(M, K), torch.bfloat16)
+  w = dev(rs.randn(K, N), torch.bfloat16)
+  packed = ops.pack_weight(w.float(), torch.bfloat16)
+  got = host(ops.dense(a, packed, out_dtype=torch.float32, n_store=keep))
+  want = (host(a) @ host(w))[:, :keep]
+  assert (np.abs(got - want) <= K * 2.0**-24 * (np.abs(host(a)) @ np.abs(host(w)))[:, :keep]
+          ).all()
+
+
 @pytest.mark.parametrize('dt', DTYPES)
 @pytest.mark.parametrize('M,K,F', [(3, 64, 40), (128, 96, 72), (200, 64, 136),
                                    (400, 32, 200), (520, 128, 512)])
