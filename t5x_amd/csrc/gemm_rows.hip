@@ -955,10 +955,20 @@ static const RowsTile kRowsTiles[] = {
     {1, 64, 128, 4, {0.28, 0.45, 0.80, 1.00}},
 };
 
-// N2: columns of a second layer in the same launch.
-static double rows_tile_cost(const RowsTile& t, int64_t M, int N, int N2 = 0) {
+// N2: columns of a second layer in the same launch.  Where all of the layer is one round of
+// lone workgroups of 256 columns, they read the rows half as often as the two of 128 columns
+// per CU, which counts for more than their overlap once the rows are more than the L2s keep.
+// us, 128 / 256 columns, rows x K x N (plain; with residual and norm):
+//   6360 x 1536 x 1024 (20 MB)  24.2 / 24.6; 28.5 / 29.0    7256 (22 MB)  26.8 / 24.9; 32.2 / 30.1
+//   9688 x 1024 x 768  (20 MB)  20.1 / 19.7; 25.0 / 24.2   10840 (22 MB)  21.3 / 20.0; 27.6 / 25.0
+//   3160 x 2816 x 2048 (18 MB)  38.3 / 37.9; 42.5 / 42.4    4056 (23 MB)  44.0 / 41.6; 49.6 / 47.2
+//   8152 x 2816 x 1024 (46 MB)  48.3 / 42.8; 52.5 / 48.0
+//   10840 x 2048 x 768 (44 MB)  40.7 / 33.5; 46.8 / 39.8
+//   3160 x 1024 x 2048 (6 MB)   17.5 / 18.4; 20.6 / 23.1
+static double rows_tile_cost(const RowsTile& t, int64_t M, int K, int N, int N2 = 0) {
   const int64_t wgs = ((M + t.rows - 1) / t.rows) *
                       ((N + t.cols - 1) / t.cols + (N2 + t.cols - 1) / t.cols);
+  if (t.cols == 256 && wgs <= 256 && 2 * M * K >= 22000000) return 0.70;
   const int64_t slots = 256 * t.per_cu, left = wgs % slots;
   return (double)(wgs / slots) * t.step[t.per_cu - 1] +
          (left ? t.step[(left + 255) / 256 - 1] : 0.0);
@@ -972,12 +982,12 @@ static bool rows_direct(int K, int64_t lda) {
 }
 
 // code 0: any.
-static const RowsTile& rows_tile(int64_t M, int N, int code, int N2 = 0) {
+static const RowsTile& rows_tile(int64_t M, int K, int N, int code, int N2 = 0) {
   const RowsTile* best = nullptr;
   double least = 0.0;
   for (const RowsTile& t : kRowsTiles) {
     if (code && t.code != code) continue;
-    const double c = rows_tile_cost(t, M, N, N2);
+    const double c = rows_tile_cost(t, M, K, N, N2);
     if (best == nullptr || c < least) {
       best = &t;
       least = c;
@@ -988,7 +998,7 @@ static const RowsTile& rows_tile(int64_t M, int N, int code, int N2 = 0) {
 
 extern "C" int t5d_gemm_rows_tile(int w_dtype, int64_t M, int K, int N) {
   if (w_dtype != T5D_BF16 || M <= 0 || N <= 0 || K <= 0 || !rows_direct(K, K)) return 1;
-  return rows_tile(M, N, 0).code;
+  return rows_tile(M, K, N, 0).code;
 }
 
 template <bool SWAP, int DENSE, int NORM = 0>
@@ -996,7 +1006,7 @@ static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int w_dtype
                                int code) {
   // (int8 weights, which are widened in registers on their way to the matrix cores, have
   // the tiles of 128 columns only)
-  const RowsTile& t = rows_tile(g.M, g.N, w_dtype == T5D_I8 ? 1 : code);
+  const RowsTile& t = rows_tile(g.M, g.K, g.N, w_dtype == T5D_I8 ? 1 : code);
   const dim3 grid((unsigned)((g.M + t.rows - 1) / t.rows) *
                   ((g.N + t.cols - 1) / t.cols));
 #define T5D_ROWS_LAUNCH(WT_, MT_, NT_, OCC_)                                     \
@@ -1032,16 +1042,17 @@ static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int w_dtype
 static const RowsTile* rows_pair(const RowsGemmArgs& g, int w_dtype, int code) {
   const bool narrow = g.K <= 768;
   const RowsTile& t =
-      rows_tile(g.M, g.N, w_dtype == T5D_I8 || (code == 0 && narrow) ? 1 : code, g.N2);
+      rows_tile(g.M, g.K, g.N, w_dtype == T5D_I8 || (code == 0 && narrow) ? 1 : code,
+                g.N2);
   if (code != 0) return &t;
   const int64_t wgs = (int64_t)((g.M + t.rows - 1) / t.rows) *
                       ((g.N + t.cols - 1) / t.cols + (g.N2 + t.cols - 1) / t.cols);
   if (wgs > 5 * 256 * t.per_cu) return nullptr;
   if (!narrow && wgs > 2 * 256 * t.per_cu) {
     const int any = w_dtype == T5D_I8 ? 1 : 0;
-    const double apart = rows_tile_cost(rows_tile(g.M, g.N, any), g.M, g.N) +
-                         rows_tile_cost(rows_tile(g.M, g.N2, any), g.M, g.N2);
-    if (rows_tile_cost(t, g.M, g.N, g.N2) > 1.03 * apart) return nullptr;
+    const double apart = rows_tile_cost(rows_tile(g.M, g.K, g.N, any), g.M, g.K, g.N) +
+                         rows_tile_cost(rows_tile(g.M, g.K, g.N2, any), g.M, g.K, g.N2);
+    if (rows_tile_cost(t, g.M, g.K, g.N, g.N2) > 1.03 * apart) return nullptr;
   }
   return &t;
 }

@@ -213,6 +213,24 @@ def test_gemm_rows_of_every_tile_over_the_ends_of_k(ops, K, tile):
     assert bool(((got.float() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize('M,K,N,tile', [(7160, 1536, 1024, 1), (7162, 1536, 1024, 2),
+                                        (8192, 2816, 1024, 2), (8193, 2816, 1024, 3),
+                                        (10751, 1024, 752, 2), (4000, 2752, 2048, 2)])
+def test_gemm_rows_of_wide_tiles_where_rows_are_many(ops, M, K, N, tile):
+  """Both sides of the line to one workgroup of 256 columns per CU: the tile as the rule
+  has it, and the bits of the other tiles."""
+  from t5x_amd import _lib
+  assert _lib.load().t5d_gemm_rows_tile(_lib.BF16, M, K, N) == tile
+  rs = np.random.RandomState(M)
+  a = dev(rs.randn(M, K).astype(np.float32), torch.bfloat16)
+  w = ops.pack_weight(dev((rs.randn(K, N) / np.sqrt(K)).astype(np.float32)), torch.bfloat16)
+  res = dev(rs.randn(M, N).astype(np.float32), torch.bfloat16)
+  for residual in (None, res):
+    got = ops.gemm_rows(a, w, residual=residual)
+    for other in (1, 2, 3):
+      assert torch.equal(got, ops.gemm_rows(a, w, residual=residual, tile=other))
+
+
 @pytest.mark.parametrize('M,N', [(24, 30720), (25, 30720), (64, 30736), (65, 19216),
                                  (128, 19200), (128, 19184)])
 @pytest.mark.parametrize('K', [32, 64, 96, 320, 480, 512, 544, 576, 608, 640, 768])
