@@ -11,7 +11,7 @@
 // positions: 12 layers of width 768, 32 texts of 128 to 512 tokens 4.27 -> 3.41 ms; 24
 // of width 1024, 7 of 400 to 1031 8.56 -> 6.61 ms.
 // The two kernels last 16 us together at 32 x 512 (131 KB of tokens), 14 at 1 x 20 and 23 at
-// 1000 x 128.  What bounds them: a launch each, and three atomics of 256 threads on one word
+// 1000 x 128, and 3 more where the texts are listed by length.  What bounds them: a launch each, and three atomics of 256 threads on one word
 // of LDS each (token_mask_kernel, which reads as much and has one, lasts 4.4 us).
 #include "common.h"
 
@@ -46,8 +46,9 @@ encoder_lengths_kernel(const int64_t* __restrict__ tokens, int32_t* __restrict__
 }
 
 // One workgroup per text: its rows' ids, the row of every position, the position
-// (text << 12 | position) of every 4 rows, its place by length; the last also sums up for
-// the host.
+// (text << 12 | position) of every 4 rows, and (ORDERED) its place by length, for which it
+// looks at every text and not only at those before it; the last also sums up for the host.
+template <bool ORDERED>
 __global__ void __launch_bounds__(256)
 encoder_rows_kernel(const int64_t* __restrict__ tokens, const int32_t* __restrict__ len,
                     const int32_t* __restrict__ odd, int32_t* __restrict__ first,
@@ -57,12 +58,16 @@ encoder_rows_kernel(const int64_t* __restrict__ tokens, const int32_t* __restric
   __shared__ int s_first, s_most, s_odd, s_longer;
   if (threadIdx.x == 0) s_first = s_most = s_odd = s_longer = 0;
   __syncthreads();
-  const int b = blockIdx.x, n = len[b];
+  const int b = blockIdx.x;
+  int n = 0;
+  if constexpr (ORDERED) n = len[b];
   int before = 0, most = 0, any = 0, longer = 0;
-  for (int i = threadIdx.x; i < (order ? B : b + 1); i += 256) {
+  for (int i = threadIdx.x; i < (ORDERED ? B : b + 1); i += 256) {
     const int other = len[i];
-    longer += other > n || (other == n && i < b);
-    if (i > b) continue;
+    if constexpr (ORDERED) {
+      longer += other > n || (other == n && i < b);
+      if (i > b) continue;
+    }
     const int rows = rows_of_text(other, E);
     if (i < b) before += rows;
     most = max(most, rows);
@@ -71,12 +76,13 @@ encoder_rows_kernel(const int64_t* __restrict__ tokens, const int32_t* __restric
   atomicAdd(&s_first, before);
   atomicMax(&s_most, most);
   atomicOr(&s_odd, any);
-  atomicAdd(&s_longer, longer);
+  if constexpr (ORDERED) atomicAdd(&s_longer, longer);
   __syncthreads();
+  if constexpr (!ORDERED) n = len[b];
   const int r0 = s_first, rows = rows_of_text(n, E);
   if (threadIdx.x == 0) {
     first[b] = r0;
-    if (order) order[s_longer] = b;
+    if constexpr (ORDERED) order[s_longer] = b;
     if (b == B - 1) {
       first[B] = r0 + rows;
       summary[0] = r0 + rows;
@@ -150,8 +156,14 @@ extern "C" int t5d_encoder_rows_ordered(void* stream, const int64_t* tokens, int
               T5D_ELIMIT, "t5d_encoder_rows: B=%d E=%d", B, E);
   hipLaunchKernelGGL(encoder_lengths_kernel, dim3(B), dim3(256), 0, as_stream(stream),
                      tokens, len, odd, E);
-  hipLaunchKernelGGL(encoder_rows_kernel, dim3(B), dim3(256), 0, as_stream(stream),
-                     tokens, len, odd, first, ids, row_of, at, summary, order, B, E);
+  if (order)
+    hipLaunchKernelGGL(encoder_rows_kernel<true>, dim3(B), dim3(256), 0,
+                       as_stream(stream), tokens, len, odd, first, ids, row_of, at,
+                       summary, order, B, E);
+  else
+    hipLaunchKernelGGL(encoder_rows_kernel<false>, dim3(B), dim3(256), 0,
+                       as_stream(stream), tokens, len, odd, first, ids, row_of, at,
+                       summary, order, B, E);
   T5D_CHECK_LAUNCH("t5d_encoder_rows");
   return T5D_OK;
 }

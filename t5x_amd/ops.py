@@ -632,13 +632,22 @@ class EncoderRows:
     _chk(tokens, 'tokens', torch.int64, 2)
     self.B, self.E = B, E = tokens.shape
     self.positions = E4 = (E + 3) // 4 * 4
-    sizes = [B, B, B + 1, B * E4, B * E, B * E4 // 4, 3, B]
+    # The order of the texts (None: as they stand) spreads attention over the chip where
+    # texts are long and few.  Each text is compared with every other for it, which many
+    # short ones notice: 65536 of 8 positions were listed in 2343 us, 1436 without; and
+    # attention is no faster in it (12 heads, up to 128 positions, us, ordered / not:
+    # 256 texts 36.7 / 38.2, 1024 158.3 / 155.8; 512 of 512 574.9 / 579.3).  Up to 64
+    # positions attention does not read it.
+    ordered = 64 < E4 and B <= 512
+    sizes = [B, B, B + 1, B * E4, B * E, B * E4 // 4, 3] + [B] * ordered
     (self.len, odd, self.first, self._ids, self.row_of, self._at, summary,
-     self.order) = torch.empty(sum(sizes), dtype=torch.int32,
-                               device=tokens.device).split(sizes)
-    _lib.call('t5d_encoder_rows_ordered', _s(), tokens.data_ptr(), B, E,
+     *order) = torch.empty(sum(sizes), dtype=torch.int32,
+                           device=tokens.device).split(sizes)
+    self.order = order[0] if ordered else None
+    _lib.call('t5d_encoder_rows_ordered' if ordered else 't5d_encoder_rows', _s(),
+              tokens.data_ptr(), B, E,
               *(t.data_ptr() for t in (self.len, odd, self.first, self._ids,
-                                       self.row_of, self._at, summary, self.order)))
+                                       self.row_of, self._at, summary, *order)))
     self.M, self.most, any_odd = summary.tolist()
     self.odd = bool(any_odd)
     self.ids, self.at = self._ids[:self.M], self._at[:self.M // 4]
@@ -731,7 +740,7 @@ def encoder_attention_rows(q, k, v_t, rel_bias, rows):
   out = torch.empty((rows.M, H * 64), dtype=torch.bfloat16, device=v_t.device)
   _lib.call('t5d_encoder_attention_ordered', _s(), q.data_ptr(), k.data_ptr(),
             v_t.data_ptr(), rel_bias.data_ptr(), rows.len.data_ptr(),
-            rows.first.data_ptr(), rows.order.data_ptr(), rows.M, rows.most,
+            rows.first.data_ptr(), _lib.ptr(rows.order), rows.M, rows.most,
             out.data_ptr(), B, H, rows.positions, blocks * 32, q.stride(0), k.stride(0))
   return out
 

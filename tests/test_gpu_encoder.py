@@ -1105,6 +1105,32 @@ def test_encoder_attention_in_the_order_of_the_texts(ops, E, H, least, queries):
     assert torch.equal(got[first[b]:first[b] + n], want[b, :n]), b
 
 
+@pytest.mark.parametrize('B,E,ordered', [(3, 61, False), (3, 64, False), (3, 65, True),
+                                         (512, 66, True), (513, 66, False)])
+def test_texts_are_listed_by_length_where_that_pays(ops, B, E, ordered):
+  """Short texts and very many are not compared with each other: attention does not read
+  their order, or is no faster in it.  Everything else is listed the same."""
+  from t5x_amd import _lib
+  rs = np.random.RandomState(B + E)
+  lens = rs.randint(0, E + 1, size=B)
+  tokens = torch.as_tensor((np.arange(E)[None] < lens[:, None]) * 5, device='cuda')
+  rows = ops.EncoderRows(tokens)
+  assert (rows.order is not None) == ordered
+  E4 = (E + 3) // 4 * 4
+  outs = [torch.zeros(n, dtype=torch.int32, device='cuda')
+          for n in (B, B, B + 1, B * E4, B * E, B * E4 // 4, 3, B)]
+  _lib.call('t5d_encoder_rows_ordered', ops._s(), tokens.data_ptr(), B, E,
+            *(t.data_ptr() for t in outs))
+  order = sorted(range(B), key=lambda b: (-lens[b], b))
+  assert outs[7].tolist() == order
+  if ordered:
+    assert rows.order.tolist() == order
+  for got, want in ((rows.len, outs[0]), (rows.first, outs[2]), (rows.ids, outs[3]),
+                    (rows.row_of, outs[4]), (rows.at, outs[5])):
+    assert torch.equal(got, want[:got.numel()].view(got.shape))
+  assert [rows.M, rows.most, int(rows.odd)] == outs[6].tolist()
+
+
 def test_encoder_of_many_ragged_texts():
   """The whole encoder where its attention takes two tiles of queries per wavefront."""
   from t5x_amd import encoder, network
