@@ -819,8 +819,10 @@ int t5d_embed_sinusoid(void* stream, int dtype, const void* table,
 /* t5d_stream_norm (y of bfloat16 or NULL, no add, x0 or rows) and t5d_dense behind it in one
  * launch, with their bits: x_out [M, ld] = x + rms(y) * y_norm (another buffer than x; not
  * written if y is NULL), C = the layer over rms(x_out) * norm.  bfloat16 only, up to
- * t5d_stream_dense_rows rows (0: not for this dtype or ld). */
+ * t5d_stream_dense_rows rows (0: not for this dtype or ld).  t5d_stream_dense_pays: whether
+ * that is faster than the two of them for M such rows; t5d_hybrid_step goes by it. */
 int t5d_stream_dense_rows(int dtype, int ld);
+int t5d_stream_dense_pays(int M, int ld, int N);
 int t5d_stream_dense(void* stream, const void* y, const float* y_norm, const float* x,
                      float* x_out, const float* norm, int d, float eps, const void* W,
                      int out_dtype, void* C, int ldc, int n_store, int M, int ld, int N,

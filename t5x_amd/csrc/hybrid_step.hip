@@ -212,7 +212,7 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
   auto row_dense = [&](const float* norm, const void* w, int out_dtype, void* out, int ldc,
                        int n_store, int n, int epilogue, float limit, float alpha,
                        float add) {
-    if (few) {
+    if (few && t5d_stream_dense_pays(M, ld, n)) {
       T5D_TRY(t5d_stream_dense(stream, y, y_norm, x, other, norm, d, m->eps, w, out_dtype,
                                out, ldc, n_store, M, ld, n, epilogue, limit, alpha, add));
       if (y) std::swap(x, other);

@@ -204,6 +204,28 @@ extern "C" int t5d_stream_dense_rows(int dtype, int ld) {
   return dtype == T5D_BF16 && ld > 0 && ld % 64 == 0 && ld <= 2048 ? 4 : 0;
 }
 
+// Where the many workgroups of a wide layer cost more than the launch they save: each forms
+// the rows anew, for few weights where ld is small, and where ld is just above 1024 with
+// requests for the pairs of 2048.  us, the two kernels / this one, float32 results (rows x ld
+// x columns):
+//   4 x   64 x  4096   4.67 /  4.54    4 x   64 x 32128   5.79 /  6.99
+//   4 x  128 x  8192   5.44 /  5.36    4 x  128 x 32128   6.41 /  6.97
+//   4 x  256 x 32128   8.24 /  7.61    4 x  256 x 50304  10.6 /  11.0
+//   4 x  384 x 24576   8.66 /  8.28    4 x  384 x 32128   9.59 / 10.01
+//   4 x 1152 x 16384   13.4 /  11.9    4 x 1152 x 32128   19.2 /  20.0
+//   4 x 1408 x 16384   14.9 /  13.5    4 x 1408 x 24576   18.2 /  18.7
+//   2 x 1088 x 32128   18.8 /  18.3    2 x 1088 x 50304   27.3 /  28.2
+//   1 x 1088 x 50304   27.6 /  26.6    1 x 1088 x 131072  54.5 /  57.3
+//   2 x  128 x 50304   8.89 /  7.72    2 x  128 x 131072  13.2 /  14.0
+//   4 x  512 x 131072  29.7 /  26.9    4 x 1536 x 131072  75.1 /  73.2
+//   4 x 1024 x 131072  51.1 /  45.9    4 x 2048 x 131072  95.6 /  86.1
+extern "C" int t5d_stream_dense_pays(int M, int ld, int N) {
+  const bool between = ld > 1024 && ld < (M >= 3 ? 1536 : 1280);
+  if (M >= 3 && ld < 512) return N <= (ld % 256 == 0 ? 128 : 64) * ld;
+  if (between) return N <= (M == 1 ? 98304 : M == 2 ? 40960 : 20480);
+  return M == 1 || ld >= 256 || N <= 98304;
+}
+
 extern "C" int t5d_stream_dense(void* stream, const void* y, const float* y_norm,
                                 const float* x, float* x_out, const float* norm, int d,
                                 float eps, const void* W, int out_dtype, void* C, int ldc,

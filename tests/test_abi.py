@@ -104,6 +104,22 @@ def test_encoder_rows_beyond_their_numbers_without_gpu(B, E):
     assert ops.EncoderRows.covers(*there) == (there[0] * there[1] < 1 << 30)
 
 
+@pytest.mark.parametrize('M,ld,N,one', [
+    # widths that fill the kernel's variants, whatever the columns
+    (4, 512, 131072, 1), (4, 1024, 131072, 1), (4, 1536, 131072, 1), (4, 2048, 131072, 1),
+    (1, 64, 131072, 1), (2, 128, 50304, 1), (2, 64, 131072, 0),
+    # few weights per workgroup
+    (3, 64, 4096, 1), (3, 64, 32128, 0), (4, 256, 32128, 1), (4, 256, 50304, 0),
+    (4, 384, 24576, 1), (4, 384, 32128, 0), (2, 384, 131072, 1),
+    # the variant of 2048 inputs at a little over 1024
+    (4, 1088, 16384, 1), (3, 1152, 32128, 0), (4, 1408, 24576, 0), (2, 1088, 32128, 1),
+    (2, 1088, 50304, 0), (2, 1280, 131072, 1), (1, 1088, 50304, 1), (1, 1088, 131072, 0)])
+def test_where_the_row_kernel_and_the_layer_behind_it_go_in_one_launch(M, ld, N, one):
+  """t5d_stream_dense_pays: not where the two launches were measured to be faster."""
+  from t5x_amd import _lib
+  assert _lib.load().t5d_stream_dense_pays(M, ld, N) == one
+
+
 def test_many_row_tile_choice_without_gpu():
   """t5d_gemm_rows_tile: which workgroup tile the many-row dense kernel runs a
   shape on (1: 128 columns, 2: 256, 3: 192, each of 128 rows, or 1 of 64), by what
