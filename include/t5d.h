@@ -223,7 +223,8 @@ int t5d_gemm_rows_pair(void* stream, int w_dtype, const void* A, const void* W,
 
 /* The workgroup tile (1, 2 or 3, as in t5d_gemm_rows_tiled) that t5d_gemm_rows
  * uses for a shape: the cheapest by the rounds of workgroups each tile needs
- * on 256 CUs (1 where the tile is not chosen, see above).  No device work; for tests and
+ * on 256 CUs, but 2 where that is one round at most and the rows are 22 MB and more, so
+ * that reading them counts for more (1 where the tile is not chosen, see above).  No device work; for tests and
  * for reading a profile. */
 int t5d_gemm_rows_tile(int w_dtype, int64_t M, int K, int N);
 

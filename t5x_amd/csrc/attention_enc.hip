@@ -859,7 +859,7 @@ extern "C" int t5d_encoder_attention_ordered(
     const int32_t* enc_len, const int32_t* first, const int32_t* order, int rows,
     int most, void* out, int B, int H, int E, int Ep, int q_stride, int k_stride) {
   T5D_REQUIRE(first && most > 0 && most <= (E + 3) / 4 * 4 && rows >= 0, T5D_EINVAL,
-              "t5d_encoder_attention_rows: first %p, %d rows, at most %d of a text of %d",
+              "t5d_encoder_attention_ordered: first %p, %d rows, at most %d of a text of %d",
               (const void*)first, rows, most, E);
   return encoder_attention(stream, q, k, v_t, rel_bias, enc_len, nullptr, first, order,
                            rows, most, out, B, H, E, Ep, q_stride, k_stride);

@@ -613,7 +613,8 @@ __device__ __forceinline__ void rows_multiply_far(const RowsGemmArgs& g,
 // results are divided by their root mean square, row by row.  The pass that this replaces
 // read and wrote every row at 2 to 3 TB/s, 11.0 us for 10312 rows of 768, 9.9 for 4976 of
 // 1024; the second store and the squares cost a layer 1 to 3 us.  Encoder of 12 layers of
-// 768, 10312 rows, 2796 -> 2680 us, of 24 of 1024, 4976 rows, 5218 -> 5000.
+// 768, 9380 rows, in passes of its own / inside 2541 / 2490 us, of 24 of 1024, 4900 rows,
+// 4975 / 4890, both with everything else as it is here.
 template <typename WT, bool SWAP, int MT, int NT, int DENSE, bool GROUPED, bool FOLD,
           int NORM>
 __device__ __forceinline__ void rows_gemm_tile(
@@ -1028,7 +1029,14 @@ static void launch_rows_direct(hipStream_t s, const RowsGemmArgs& g, int w_dtype
 }
 
 // The workgroup tile of two layers in one launch; null: two launches.  Over up to 768
-// inputs that is 128 columns (10304 x 768 41.0 us, with 256 or 192 42.4).  One launch gains
+// inputs that is 128 columns: with 64 to 768 inputs and 128 to 32768 rows it is within 4 %
+// of the fastest, but that 256 lead by 5 % over 16384 rows of 512 + 512 columns and more.
+// us, 128 / 192 / 256 columns; two launches (rows x inputs, thrice as many columns):
+//    2048 x 384   8.8 / 11.0 / 13.2; 10.1     10304 x 640  33.8 / 36.1 / 34.5; 37.6
+//   10304 x 384  16.8 / 17.5 / 19.7; 20.3     10304 x 768  41.2 / 43.1 / 43.0; 44.0
+//    4096 x 512  13.2 / 16.4 / 15.8; 14.1     16384 x 768  61.1 / 59.9 / 59.9; 64.1
+//   16384 x 512  33.3 / 37.1 / 31.6; 35.9     24576 x 768  88.0 / 89.3 / 89.0; 92.4
+// One launch gains
 // where the two leave part of a round empty; beyond five rounds, and where the cost model
 // says that the two fit their rounds better, there are two.  us, two launches / one (rows x
 // inputs x columns + columns):

@@ -898,9 +898,11 @@ recurrence_chain_kernel(RecArgs g) {
     for (int n = 0; n < NC; ++n) os[n] = o.os[n];
   };
   // The operands of the next chunks are on their way while one is multiplied.  The
-  // compiler waits for all of them at the head of a loop, hence 16 steps per round.
+  // compiler waits for all of them at the head of a loop, hence 16 steps per round, 12 with
+  // two column tiles (three sets of operands: a round ends on the set it began with).
   constexpr int DEPTH = NTW > 4 ? 2 : NC > 1 ? 3 : 4;
   constexpr int ROUND = NTW <= 2 ? NC > 1 ? 12 : 16 : DEPTH;
+  static_assert(ROUND % DEPTH == 0, "operands of one chunk, steps of another");
   Operands o[DEPTH];
 #pragma unroll
   for (int i = 0; i + 1 < DEPTH; ++i) load(o[i]);

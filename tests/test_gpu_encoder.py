@@ -1131,6 +1131,35 @@ def test_texts_are_listed_by_length_where_that_pays(ops, B, E, ordered):
   assert [rows.M, rows.most, int(rows.odd)] == outs[6].tolist()
 
 
+@pytest.mark.parametrize('E,B,H', [(20, 5, 3), (65, 2, 6), (130, 12, 40), (1031, 12, 12)])
+def test_encoder_attention_over_rows_of_an_unknown_number(ops, E, B, H):
+  """t5d_encoder_attention_rows, which is told neither the rows nor the order of the texts,
+  has the bits of the call that is, on both sides of its own line between workgroups."""
+  from t5x_amd import _lib
+  rs = np.random.RandomState(E)
+  lens = rs.randint(1, E + 1, size=B)
+  tokens = torch.as_tensor((np.arange(E)[None] < lens[:, None]) * 5, device='cuda')
+  rows = ops.EncoderRows(tokens)
+  gen = torch.Generator(device='cuda')
+  gen.manual_seed(E)
+  rnd = lambda *shape: torch.randn(shape, generator=gen, device='cuda').bfloat16()
+  q, k = 0.3 * rnd(rows.M, H * 64), rnd(rows.M, H * 64)
+  blocks = (rows.positions + 31) // 32
+  v, rel = rnd(B, H, blocks, 64, 32), rnd(H, 2 * rows.positions - 1)
+  got = torch.empty_like(q)
+  _lib.call('t5d_encoder_attention_rows', ops._s(), q.data_ptr(), k.data_ptr(),
+            v.data_ptr(), rel.data_ptr(), rows.len.data_ptr(), rows.first.data_ptr(),
+            rows.most, got.data_ptr(), B, H, rows.positions, 32 * blocks, H * 64, H * 64)
+  assert torch.equal(got, ops.encoder_attention_rows(q, k, v, rel, rows))
+
+
+# more than 32 parts of 64 columns, the last of them partial, and between 16 and 32 an odd
+# number of them
+@pytest.mark.parametrize('M,D,N', [(68, 2144, 128), (44, 2080, 64), (40, 1312, 64)])
+def test_gemm_rows_with_the_norm_of_wide_rows_between_them(ops, M, D, N):
+  test_gemm_rows_with_the_norm_between_them(ops, M, D, N)
+
+
 def test_encoder_of_many_ragged_texts():
   """The whole encoder where its attention takes two tiles of queries per wavefront."""
   from t5x_amd import encoder, network

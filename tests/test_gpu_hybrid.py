@@ -217,6 +217,45 @@ def test_stream_norm_and_the_layer_behind_it_in_one_launch(width, ld, N, kind, M
     assert torch.equal(new, old if branch is not None else torch.full_like(x, 5.0))
 
 
+# an odd number of column tiles beyond 512, gated and not, for every number of pairs of
+# k-tiles per wavefront
+@pytest.mark.parametrize('width,ld,N,kind', [
+    (500, 512, 8208, 'glu'), (768, 768, 8208, 'f32'), (1024, 1024, 8240, 'glu'),
+    (1150, 1152, 8208, 'plain'), (2048, 2048, 10256, 'glu'), (2040, 2048, 8208, 'f32')])
+@pytest.mark.parametrize('M', [1, 2, 4])
+def test_two_column_tiles_per_workgroup_behind_the_norm(width, ld, N, kind, M):
+  test_stream_norm_and_the_layer_behind_it_in_one_launch(width, ld, N, kind, M)
+
+
+@pytest.mark.parametrize('rows', [1, 2, 3, 4])
+def test_steps_where_only_some_layers_go_with_the_row_kernel(monkeypatch, rows):
+  """A model whose layers go in one launch and whose wide head does not: the bits of one
+  launch each."""
+  from t5x_amd import _lib, hybrid, sequences
+  V = 131072 if rows < 3 else 16400
+  cfg = dict(cases.CONFIGS['no_loop'], vocab=V)
+  cfg.pop('loop', None)
+  monkeypatch.setitem(cases.CONFIGS, 'here', cfg)
+  made = hybrid._Buffers.__init__
+
+  def without(self, *args):
+    made(self, *args)
+    self.x2 = None
+
+  pays = _lib.load().t5d_stream_dense_pays
+  ld = (cfg['width'] + 63) // 64 * 64
+  assert pays(rows, ld, 64) == 1
+  assert pays(rows, ld, V) == (1 if rows == 1 or (rows == 2 and ld >= 256) else 0)
+  got = []
+  for init in (made, without):
+    monkeypatch.setattr(hybrid._Buffers, '__init__', init)
+    _, params, module = build('here', 'bfloat16')
+    tokens = np.random.RandomState(rows).randint(0, V, 20).tolist()
+    live = sequences.Sequences(module, params, 2, 64)
+    got.append(feed(live, 'a', tokens, [12, 12 + rows]))
+  assert np.array_equal(*got)
+
+
 def test_stream_dense_refuses_what_it_does_not_take():
   from t5x_amd import _lib
   lib = _lib.load()
