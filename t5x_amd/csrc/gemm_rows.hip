@@ -613,7 +613,7 @@ __device__ __forceinline__ void rows_multiply_far(const RowsGemmArgs& g,
 // results are divided by their root mean square, row by row.  The pass that this replaces
 // read and wrote every row at 2 to 3 TB/s, 11.0 us for 10312 rows of 768, 9.9 for 4976 of
 // 1024; the second store and the squares cost a layer 1 to 3 us.  Encoder of 12 layers of
-// 768, 9380 rows, in passes of its own / inside 2541 / 2490 us, of 24 of 1024, 4900 rows,
+// 768, 9372 rows, in passes of its own / inside 2541 / 2490 us, of 24 of 1024, 4896 rows,
 // 4975 / 4890, both with everything else as it is here.
 template <typename WT, bool SWAP, int MT, int NT, int DENSE, bool GROUPED, bool FOLD,
           int NORM>
