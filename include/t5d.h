@@ -829,6 +829,15 @@ int t5d_stream_dense(void* stream, const void* y, const float* y_norm, const flo
                      int out_dtype, void* C, int ldc, int n_store, int M, int ld, int N,
                      int epilogue, float glu_limit, float glu_alpha, float glu_add);
 
+/* t5d_stream_dense for up to t5d_stream_rows_dense_rows rows, on a kernel that norms 16 rows
+ * for many columns. */
+int t5d_stream_rows_dense_rows(int dtype, int ld);
+int t5d_stream_rows_dense_pays(int M, int ld, int N);
+int t5d_stream_rows_dense(void* stream, const void* y, const float* y_norm, const float* x,
+                          float* x_out, const float* norm, int d, float eps, const void* W,
+                          int out_dtype, void* C, int ldc, int n_store, int M, int ld, int N,
+                          int epilogue, float glu_limit, float glu_alpha, float glu_add);
+
 /* The row kernel between two dense layers of a float32 residual stream x [M, ld]:
  *   x += rms(y) * y_norm   (y [M, ld] of y_dtype; y_norm NULL: x += y; y NULL: no)
  *   x += add               (add [d] or NULL)
@@ -1012,10 +1021,12 @@ typedef struct {
   int64_t workspace_bytes;
   float* trace;            /* NULL or [n_runs, M, ld]: x after every run */
   const int32_t* gate;     /* as t5d_model_step */
-  float* x2;               /* [t5d_stream_dense_rows, ld] beside x (streams 0), or NULL: with it
-                              steps of so few rows take t5d_stream_dense */
+  float* x2;               /* [max(t5d_stream_dense_rows, x2_rows), ld] beside x (streams 0), or
+                              NULL: with it steps of so few rows take t5d_stream_dense or, up
+                              to x2_rows, t5d_stream_rows_dense */
   void* y2;                /* [M, ld] beside y, or NULL: with it two to four streams of many
                               rows are written once a layer */
+  int x2_rows;
 } t5d_hybrid_model;
 
 /* Runs the tokens of `batch` through the model.  Logits [n_want, V] of the tokens

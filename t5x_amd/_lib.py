@@ -188,7 +188,7 @@ class HybridModel(Structure):
                       p='embedding loop_in head final_norm') +
               [('layers', POINTER(HybridLayer)), ('runs', POINTER(HybridRun))] +
               _fields(p='x x0 low h cat proj q_rows y workspace',
-                      l='workspace_bytes', p2='trace gate x2 y2'))
+                      l='workspace_bytes', p2='trace gate x2 y2', i2='x2_rows'))
 
 
 _P = c_void_p
@@ -204,6 +204,12 @@ _SIGNATURES = {
     't5d_stream_dense_rows': (c_int, [c_int] * 2),
     't5d_stream_dense_pays': (c_int, [c_int] * 3),
     't5d_stream_dense': (c_int, [_P] * 6 + [c_int, c_float, _P, c_int, _P] +
+                         [c_int] * 6 + [c_float] * 3),
+    't5d_grouped_tile_rows': (c_int, [c_int] * 3),
+    't5d_grouped_dense_run': (c_int, [_P, POINTER(GroupedDense)]),
+    't5d_stream_rows_dense_rows': (c_int, [c_int] * 2),
+    't5d_stream_rows_dense_pays': (c_int, [c_int] * 3),
+    't5d_stream_rows_dense': (c_int, [_P] * 6 + [c_int, c_float, _P, c_int, _P] +
                          [c_int] * 6 + [c_float] * 3),
     't5d_grouped_tile_rows': (c_int, [c_int] * 3),
     't5d_grouped_dense_run': (c_int, [_P, POINTER(GroupedDense)]),

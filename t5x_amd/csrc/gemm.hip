@@ -22,6 +22,7 @@
 
 #include "common.h"
 #include "gemm_tiles.h"
+#include "norm_dense.h"
 
 namespace t5d {
 
@@ -387,7 +388,9 @@ norm_gemm_kernel(GemmArgs g) {
   }
   T5D_GATE_TEST();
 
-  float ss = 0.f;
+  // (in the order of norm_dense_kernel, whose lanes hold 4 columns in a row, and of a sum over
+  // its wavefront)
+  float part[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     if (EXACT || wave + 4 * j < n_pairs) {
@@ -396,15 +399,20 @@ norm_gemm_kernel(GemmArgs g) {
         float f[8];
         unpack16(xa[j][hh].u, f);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
+        for (int e = 0; e < 8; ++e) part[hh][e >> 2] = fmaf(f[e], f[e], part[hh][e >> 2]);
       }
     }
   }
-  ss += dpp_move<kDppXor1>(ss);  // over the 4 pieces of the row
-  ss += dpp_move<kDppXor2>(ss);
-  if (gq == 0) s_ss[wave][n16] = ss;
+  float ss[2];
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh) {
+    ss[hh] = part[hh][0] + part[hh][1];
+    ss[hh] += dpp_move<kDppXor1>(ss[hh]);  // over the 4 pieces of the row
+    ss[hh] += dpp_move<kDppXor2>(ss[hh]);
+  }
+  if (gq == 0) s_ss[wave][n16] = ss[0] + ss[1];
   __syncthreads();
-  const float tot = (s_ss[0][n16] + s_ss[2][n16]) + (s_ss[1][n16] + s_ss[3][n16]);
+  const float tot = (s_ss[0][n16] + s_ss[1][n16]) + (s_ss[2][n16] + s_ss[3][n16]);
   const float inv = 1.0f / sqrtf(tot / (float)g.K + g.eps);
 
   f32x4_v acc[NT];
@@ -1547,6 +1555,10 @@ extern "C" int t5d_norm_gemm(void* stream, int dtype, int w_dtype,
     else
       hipLaunchKernelGGL(norm_gemm_wide_kernel<32>, grid, block, 0, s, g, G, halves);
     T5D_CHECK_LAUNCH("t5d_norm_gemm(wide)");
+    return T5D_OK;
+  }
+  if (launch_norm_dense(w_dtype, g, s)) {
+    T5D_CHECK_LAUNCH("t5d_norm_gemm(norm_dense)");
     return T5D_OK;
   }
   const int nj = (K / 64 + 3) / 4;  // k-tile pairs per wavefront

@@ -2,15 +2,9 @@
 // launch, for a few rows: every workgroup forms the rows it multiplies by itself.
 #include "common.h"
 #include "gemm_tiles.h"
+#include "norm_dense.h"
 
 namespace t5d {
-
-struct StreamDenseArgs : DenseArgs {
-  const bf16_t* y;                  // [M, lda] branch output, or null
-  const float *y_norm, *x, *norm;   // [d] or null; [M, lda]; [d]
-  float* x_out;                     // [M, lda], not x: the stream with the branch added
-  int d;
-};
 
 // Rows x + norm(y) and their norm as t5d_stream_norm forms them, then 16 NT columns of the
 // layer as gemm_mfma_kernel does: the same bits as the two of them.  256 threads hold RM
@@ -59,20 +53,12 @@ stream_dense_kernel(StreamDenseArgs g) {
                                         : make_uint2(0, 0);
     }
   }
-  auto column = [&](const float* p, int c) {  // 4 entries of a [d] vector
-    float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (c + 4 <= g.d) return *reinterpret_cast<const float4*>(p + c);
-    if (c < g.d) w.x = p[c];
-    if (c + 1 < g.d) w.y = p[c + 1];
-    if (c + 2 < g.d) w.z = p[c + 2];
-    return w;
-  };
   float4 wy[VPT], wx[VPT];
 #pragma unroll
   for (int v = 0; v < VPT; ++v) {
     const int c = 4 * (threadIdx.x + 256 * v);
-    wy[v] = g.y_norm != nullptr ? column(g.y_norm, c) : make_float4(1.f, 1.f, 1.f, 1.f);
-    wx[v] = column(g.norm, c);
+    wy[v] = g.y_norm != nullptr ? norm_column(g.y_norm, c, g.d) : make_float4(1.f, 1.f, 1.f, 1.f);
+    wx[v] = norm_column(g.norm, c, g.d);
   }
   uint4 w[NJ][2][NT];
 #pragma unroll
@@ -226,15 +212,15 @@ extern "C" int t5d_stream_dense_pays(int M, int ld, int N) {
   return M == 1 || ld >= 256 || N <= 98304;
 }
 
-extern "C" int t5d_stream_dense(void* stream, const void* y, const float* y_norm,
-                                const float* x, float* x_out, const float* norm, int d,
-                                float eps, const void* W, int out_dtype, void* C, int ldc,
-                                int n_store, int M, int ld, int N, int epilogue,
-                                float glu_limit, float glu_alpha, float glu_add) {
+int t5d::stream_dense_args(const char* name, StreamDenseArgs* g, int most_rows, const void* y,
+                           const float* y_norm, const float* x, float* x_out,
+                           const float* norm, int d, float eps, const void* W, int out_dtype,
+                           void* C, int ldc, int n_store, int M, int ld, int N, int epilogue,
+                           float glu_limit, float glu_alpha, float glu_add) {
   T5D_REQUIRE(x && norm && W && C && (!y || (x_out && x_out != x)), T5D_EINVAL,
-              "t5d_stream_dense: null pointer, or the stream in place");
-  T5D_REQUIRE(M > 0 && M <= t5d_stream_dense_rows(T5D_BF16, ld) && d > 0 && d <= ld,
-              T5D_ELIMIT, "t5d_stream_dense: M=%d d=%d ld=%d", M, d, ld);
+              "%s: null pointer, or the stream in place", name);
+  T5D_REQUIRE(M > 0 && M <= most_rows && d > 0 && d <= ld, T5D_ELIMIT,
+              "%s: M=%d d=%d ld=%d", name, M, d, ld);
   const bool glu = epilogue == T5D_EPI_CLAMPED_GLU;
   T5D_REQUIRE((epilogue == T5D_EPI_NONE || glu) && N > 0 && N % 16 == 0 &&
                   (out_dtype == T5D_F32
@@ -242,21 +228,33 @@ extern "C" int t5d_stream_dense(void* stream, const void* y, const float* y_norm
                        : out_dtype == T5D_BF16 &&
                              (glu ? ldc == N / 2 && n_store == N
                                   : ldc == N && n_store == N)),
-              T5D_EINVAL,
-              "t5d_stream_dense: out_dtype %d with epilogue %d, N=%d ldc=%d n_store=%d",
+              T5D_EINVAL, "%s: out_dtype %d with epilogue %d, N=%d ldc=%d n_store=%d", name,
               out_dtype, epilogue, N, ldc, n_store);
   T5D_REQUIRE((((uintptr_t)y | (uintptr_t)x | (uintptr_t)x_out | (uintptr_t)W |
                 (uintptr_t)C | (uintptr_t)norm | (uintptr_t)y_norm) % 16) == 0,
-              T5D_EINVAL, "t5d_stream_dense: operands must be 16-byte aligned");
+              T5D_EINVAL, "%s: operands must be 16-byte aligned", name);
+  g->A = nullptr; g->W = W; g->scales = nullptr; g->residual = nullptr;
+  g->C = C; g->M = M; g->K = ld; g->N = N; g->m_parts = 1;
+  g->gate = tls_gate; g->epilogue = epilogue; g->out_f32 = out_dtype == T5D_F32;
+  g->norm_scale = nullptr; g->eps = eps;
+  g->lda = ld; g->ldc = ldc; g->n_store = n_store;
+  g->glu_limit = glu_limit; g->glu_alpha = glu_alpha; g->glu_add = glu_add;
+  g->y = (const bf16_t*)y; g->y_norm = y_norm; g->x = x; g->norm = norm;
+  g->x_out = x_out; g->d = d;
+  return T5D_OK;
+}
+
+extern "C" int t5d_stream_dense(void* stream, const void* y, const float* y_norm,
+                                const float* x, float* x_out, const float* norm, int d,
+                                float eps, const void* W, int out_dtype, void* C, int ldc,
+                                int n_store, int M, int ld, int N, int epilogue,
+                                float glu_limit, float glu_alpha, float glu_add) {
   StreamDenseArgs g;
-  g.A = nullptr; g.W = W; g.scales = nullptr; g.residual = nullptr;
-  g.C = C; g.M = M; g.K = ld; g.N = N; g.m_parts = 1;
-  g.gate = tls_gate; g.epilogue = epilogue; g.out_f32 = out_dtype == T5D_F32;
-  g.norm_scale = nullptr; g.eps = eps;
-  g.lda = ld; g.ldc = ldc; g.n_store = n_store;
-  g.glu_limit = glu_limit; g.glu_alpha = glu_alpha; g.glu_add = glu_add;
-  g.y = (const bf16_t*)y; g.y_norm = y_norm; g.x = x; g.norm = norm;
-  g.x_out = x_out; g.d = d;
+  const int rc = stream_dense_args("t5d_stream_dense", &g,
+                                   t5d_stream_dense_rows(T5D_BF16, ld), y, y_norm, x, x_out,
+                                   norm, d, eps, W, out_dtype, C, ldc, n_store, M, ld, N,
+                                   epilogue, glu_limit, glu_alpha, glu_add);
+  if (rc != T5D_OK) return rc;
   const int tiles = N / 16;
   const int nt = tiles > 512 ? 2 : 1;
   const dim3 grid((tiles + nt - 1) / nt), block(256);

@@ -708,7 +708,8 @@ class _Buffers:
     self.x = rows(ld * max(1, cfg.streams), f32)
     # (the stream of few rows goes back and forth between two buffers; calls of few rows
     # may come with buffers that longer ones have left)
-    few = lib.t5d_stream_dense_rows(_lib.dtype_code(act), ld)
+    self.x2_rows = lib.t5d_stream_rows_dense_rows(_lib.dtype_code(act), ld)
+    few = max(self.x2_rows, lib.t5d_stream_dense_rows(_lib.dtype_code(act), ld))
     self.x2 = None
     if few and not cfg.streams:
       self.x2 = torch.empty((few, ld), dtype=f32, device=device)
@@ -977,6 +978,7 @@ class HybridDecoder(network.DecodeContexts):
     for name in ('x', 'x0', 'low', 'h', 'cat', 'proj', 'q_rows', 'y',
                  'workspace', 'x2', 'y2'):
       setattr(mod, name, P(getattr(bufs, name)))
+    mod.x2_rows = bufs.x2_rows
     mod.workspace_bytes = bufs.workspace.numel()
     mod.gate = P(gate)
     mod._keepalive = (layers, cruns, kept, w, bufs, gate)

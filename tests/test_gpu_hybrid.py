@@ -268,6 +268,59 @@ def test_stream_dense_refuses_what_it_does_not_take():
   assert call(1, 64, x2=16) == call(1, 64, x2=36) == -1
 
 
+# 16 rows per workgroup: a last row tile of one row and of all; widths that fill the three
+# variants and that do not; one to four column tiles per half of a workgroup, a last
+# workgroup with one
+@pytest.mark.parametrize('M,width,ld,N,kind', [
+    (5, 64, 64, 16, 'plain'), (16, 500, 512, 96, 'glu'), (17, 570, 576, 8208, 'glu'),
+    (33, 1000, 1024, 4112, 'plain'), (48, 768, 768, 5648, 'glu'), (64, 1021, 1024, 5632, 'f32'),
+    (64, 1024, 1024, 8192, 'glu'), (97, 512, 512, 4112, 'f32'), (128, 1024, 1024, 4096, 'glu'),
+    (128, 320, 320, 8208, 'plain')])
+def test_stream_norm_and_the_layer_behind_it_for_more_rows(monkeypatch, M, width, ld, N, kind):
+  """t5d_stream_rows_dense has the bits of t5d_stream_norm and t5d_dense."""
+  from t5x_amd import _lib
+  call = _lib.call
+  monkeypatch.setattr(_lib, 'call', lambda name, *a: call(
+      't5d_stream_rows_dense' if name == 't5d_stream_dense' else name, *a))
+  test_stream_norm_and_the_layer_behind_it_in_one_launch(width, ld, N, kind, M)
+
+
+@pytest.mark.parametrize('rows', [5, 16, 17, 64])
+def test_steps_whose_layers_go_with_the_row_kernel(monkeypatch, rows):
+  """Steps of some rows have the bits of one launch each."""
+  from t5x_amd import hybrid, sequences
+  cfg = dict(cases.CONFIGS['no_loop'])
+  cfg.pop('loop', None)
+  monkeypatch.setitem(cases.CONFIGS, 'here', cfg)
+  made = hybrid._Buffers.__init__
+
+  def without(self, *args):
+    made(self, *args)
+    self.x2 = None
+
+  got = []
+  for init in (made, without):
+    monkeypatch.setattr(hybrid._Buffers, '__init__', init)
+    _, params, module = build('here', 'bfloat16')
+    tokens = np.random.RandomState(rows).randint(0, module.config.vocab_size,
+                                                 12 + rows).tolist()
+    live = sequences.Sequences(module, params, 2, 128)
+    got.append(feed(live, 'a', tokens, [12, 12 + rows]))
+  assert np.array_equal(*got)
+
+
+def test_stream_rows_dense_refuses_what_it_does_not_take():
+  from t5x_amd import _lib
+  lib = _lib.load()
+  rows = lib.t5d_stream_rows_dense_rows
+  assert rows(1, 64) == rows(1, 1024) == 128
+  assert rows(0, 64) == rows(1, 96) == rows(1, 1088) == rows(1, 0) == 0
+  call = lambda M, ld, x2=32, d=64: lib.t5d_stream_rows_dense(
+      None, 16, 16, 16, x2, 16, d, 1e-6, 16, 1, 16, 64, 64, M, ld, 64, 0, 0.0, 0.0, 0.0)
+  assert call(129, 64) == call(1, 96) == call(0, 64) == call(1, 64, d=65) == -3
+  assert call(1, 64, x2=16) == call(1, 64, x2=36) == -1
+
+
 # ---- windowed attention ---------------------------------------------------------------
 
 

@@ -1532,6 +1532,36 @@ def test_norm_gemm_does_not_depend_on_its_tiles(ops, K, N, int8):
     assert torch.equal(got, want[a:b]), (a, b)
 
 
+# one to four column tiles per half of a workgroup, a last workgroup with one, a last row
+# tile of one row; for 512 inputs and fewer, 768 and fewer, 1024 and fewer
+@pytest.mark.parametrize('M,K,N,kind', [
+    (33, 192, 3088, 'plain'), (48, 512, 4096, 'geglu'), (65, 448, 5648, 'f32'),
+    (128, 512, 4096, 'geglu'), (17, 768, 2320, 'plain'), (49, 704, 3088, 'geglu'),
+    (128, 768, 2304, 'f32'), (16, 1024, 5632, 'geglu'), (33, 960, 4112, 'f32'),
+    (64, 1024, 5632, 'geglu'), (81, 832, 3072, 'plain')])
+@pytest.mark.parametrize('int8', [False, True])
+def test_norm_in_front_of_many_columns(ops, M, K, N, kind, int8):
+  """Rows normed once for many columns have the bits of 16 rows at a time, whose columns
+  are few enough for the other kernel, and they are the layer's over normed rows."""
+  rs = np.random.RandomState(M + K + N)
+  x = dev(rs.randn(M, K).astype(np.float32), torch.bfloat16)
+  scale = dev((1 + 0.1 * rs.randn(K)).astype(np.float32), torch.bfloat16)
+  kernel = lambda n: dev((rs.randn(K, n) / np.sqrt(K)).astype(np.float32))
+  wdt = torch.int8 if int8 else torch.bfloat16
+  if kind == 'geglu':
+    pw = ops.pack_weight(kernel(N // 2), torch.bfloat16, wdt, gate_kernel=kernel(N // 2))
+  else:
+    pw = ops.pack_weight(kernel(N), torch.bfloat16, wdt)
+  od = torch.float32 if kind == 'f32' else torch.bfloat16
+  got = ops.gemm(x, pw, norm_scale=scale, out_dtype=od)
+  want = torch.cat([ops.gemm(x[a:a + 4].contiguous(), pw, norm_scale=scale, out_dtype=od)
+                    for a in range(0, M, 4)])
+  two = ops.gemm(ops.rmsnorm(x, scale), pw, out_dtype=od).float()
+  assert torch.equal(got, want)
+  err = (got.float() - two).abs()  # (a normed value may round the other way)
+  assert bool((err <= 2e-2 + 2.0**-6 * two.abs()).all())
+
+
 def test_cross_attention_random_shapes(ops):
   """t5d_cross_attention_step (bfloat16) over 40 random shapes — batch 1..48,
   1 / 2 / 4 / 8 beams, 1..16 heads, encoder length a multiple of 32 up to
