@@ -652,6 +652,16 @@ typedef struct {
    * cache_src[b, e], and from the next iteration's self-attention on in row
    * cache_dst[b, e] = cache_slot[b, e]. */
   int32_t *cache_slot, *cache_src, *cache_dst;
+  /* n_lanes > 1: this is slice `lane` of a batch whose slices are stepped on separate streams
+   * without waiting for each other; the condition is that of the whole batch all the same,
+   * and every slice makes exactly the loop's iterations.  Its keep_going (its model's gate) is
+   * its own.  lane_alive [n_lanes]: 1 until the slice has come to the loop's end;
+   * lane_records [n_lanes, S + 1], zeros before the first iteration.  An enqueued iteration
+   * leaves everything as it is where the slice is done or must know first what another one,
+   * not as far yet, says of this iteration (keep_going 0, lane_alive 1): enqueue further
+   * ones until lane_alive is 0.  skip_cond is not looked at. */
+  int n_lanes, lane;
+  int32_t *lane_alive, *lane_records;
 } t5d_beam_step;
 
 /* One iteration of the beam_search loop body plus the loop condition

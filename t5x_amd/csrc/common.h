@@ -325,6 +325,10 @@ int launch_beam_tail(hipStream_t s, const t5d_beam_state* state, int B, int K,
                      int32_t* keep_going, int do_cond, int32_t* counters,
                      int n_counters);
 
+// The same for one lane of a batch whose lanes do not wait for each other (n_lanes > 1).
+int launch_beam_lane_tail(hipStream_t s, const t5d_beam_step* b, int B, int K,
+                          int32_t* counters, int n_counters);
+
 // The two kernels of a temperature_sample iteration after the decoder step:
 // token choice, then the bookkeeping, which also advances `counters` (the
 // layers' cache indices) and the step count and sets the loop flag.

@@ -739,6 +739,28 @@ __global__ void gather_ids_kernel(const int32_t* __restrict__ live_seqs,
   if (r < R) ids[r] = live_seqs[(size_t)r * S + *cur_index];
 }
 
+// Of this thread's items (b, b + 256, ...): how many the search has not terminated, and how
+// many may still pass the least log-probability.
+__device__ __forceinline__ void count_open(const t5d_beam_state& st, int B, int K,
+                                           float min_brevity, float min_log_prob,
+                                           int* not_terminated, int* passes_min) {
+  const float raw_min = min_log_prob / min_brevity;
+  *not_terminated = *passes_min = 0;
+  for (int b = threadIdx.x; b < B; b += 256) {
+    const float best_live = st.live_logprobs[(size_t)b * K + K - 1] / min_brevity;
+    float worst = INFINITY;
+    for (int e = 0; e < K; ++e)
+      worst = fminf(worst, st.finished_scores[(size_t)b * K + e]);
+    bool term = true;
+    for (int e = 0; e < K; ++e) {
+      const float w = st.finished_flags[(size_t)b * K + e] ? worst : kNegInf;
+      term = term && (w > best_live);
+    }
+    if (!term) ++*not_terminated;
+    if (!(best_live < raw_min)) ++*passes_min;
+  }
+}
+
 __global__ void __launch_bounds__(256)
 beam_cond_kernel(t5d_beam_state st, int B, int K, int S, float min_brevity,
                  float min_log_prob, int max_decode_step, int min_initial_index,
@@ -755,21 +777,8 @@ beam_cond_kernel(t5d_beam_state st, int B, int K, int S, float min_brevity,
     if ((int)threadIdx.x < n_counters) counters[threadIdx.x] += 1;
   }
   if (!do_cond) return;
-  const float raw_min = min_log_prob / min_brevity;
-  int not_terminated = 0, passes_min = 0;
-  for (int b = threadIdx.x; b < B; b += 256) {
-    const float best_live = st.live_logprobs[(size_t)b * K + K - 1] / min_brevity;
-    float worst = INFINITY;
-    for (int e = 0; e < K; ++e)
-      worst = fminf(worst, st.finished_scores[(size_t)b * K + e]);
-    bool term = true;
-    for (int e = 0; e < K; ++e) {
-      const float w = st.finished_flags[(size_t)b * K + e] ? worst : kNegInf;
-      term = term && (w > best_live);
-    }
-    if (!term) ++not_terminated;
-    if (!(best_live < raw_min)) ++passes_min;
-  }
+  int not_terminated, passes_min;
+  count_open(st, B, K, min_brevity, min_log_prob, &not_terminated, &passes_min);
   not_terminated = block_sum_i32(not_terminated, iscratch);
   passes_min = block_sum_i32(passes_min, iscratch);
   if (threadIdx.x == 0) {
@@ -779,6 +788,57 @@ beam_cond_kernel(t5d_beam_state st, int B, int K, int S, float min_brevity,
     const bool none_pass = (passes_min == 0) && (cur > 0);
     *keep_going = (not_at_end && !search_terminated && !none_pass && !exceed) ? 1 : 0;
   }
+}
+
+// The end of an iteration of one slice (lane) of a batch whose lanes run on streams of their
+// own.  The loop goes on while any item of the whole batch may still change, but a lane need
+// not wait for the others to know: what each one's items say after every iteration is
+// recorded, and as long as this lane's own say yes it goes on.  Only where they do not, the
+// others are asked for the same iteration; one that has not come that far is waited for by
+// leaving iterations out (the lane's gate is closed, its state untouched) until its record is
+// there.  So every lane makes exactly the iterations of the loop, whatever the streams do.
+// A record: 4, 1 if all of the lane's items are terminated, 2 if none passes the least
+// log-probability; 0: not there yet.  It and its readers go past the L2s, which do not see
+// each other's writes (agent scope).
+__global__ void __launch_bounds__(256)
+beam_lane_tail_kernel(t5d_beam_state st, int B, int K, int S, float min_brevity,
+                      float min_log_prob, int max_decode_step, int min_initial_index,
+                      int32_t* gate, int n_lanes, int lane, int32_t* alive, int32_t* records,
+                      int32_t* counters, int n_counters) {
+  __shared__ int iscratch[4];
+  if (alive[lane] == 0) return;
+  const bool ran = *gate != 0;
+  const int cur = *st.cur_index + (ran ? 1 : 0);
+  __syncthreads();  // every thread has read the old values
+  int32_t* own = records + (size_t)lane * (S + 1) + cur;
+  int bits = 0;
+  if (ran) {
+    if (threadIdx.x == 0) *st.cur_index = cur;
+    if ((int)threadIdx.x < n_counters) counters[threadIdx.x] += 1;
+    int not_terminated, passes_min;
+    count_open(st, B, K, min_brevity, min_log_prob, &not_terminated, &passes_min);
+    not_terminated = block_sum_i32(not_terminated, iscratch);
+    passes_min = block_sum_i32(passes_min, iscratch);
+    bits = 4 | (not_terminated == 0 ? 1 : 0) | (passes_min == 0 && cur > 0 ? 2 : 0);
+  }
+  if (threadIdx.x != 0) return;
+  if (ran)
+    __hip_atomic_store(own, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    bits = *own;
+  int all = bits & 3;
+  bool unknown = false;
+  for (int l = 0; l < n_lanes && all != 0; ++l) {
+    if (l == lane) continue;
+    const int other = __hip_atomic_load(records + (size_t)l * (S + 1) + cur,
+                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (other == 0) unknown = true;
+    else all &= other;
+  }
+  const bool last = !(cur + min_initial_index < S - 1) ||
+                    (max_decode_step > 0 && cur >= max_decode_step);
+  *gate = !last && all == 0 ? 1 : 0;
+  if (last || (all != 0 && !unknown)) alive[lane] = 0;
 }
 
 // ---- sampling -----------------------------------------------------------------
@@ -1916,6 +1976,23 @@ int t5d::launch_beam_tail(hipStream_t s, const t5d_beam_state* state, int B,
                      min_initial_index, keep_going, tls_gate, 1, do_cond,
                      counters, n_counters);
   T5D_CHECK_LAUNCH("beam tail");
+  return T5D_OK;
+}
+
+int t5d::launch_beam_lane_tail(hipStream_t s, const t5d_beam_step* b, int B, int K,
+                               int32_t* counters, int n_counters) {
+  int rc = check_state("beam lane tail", &b->state);
+  if (rc) return rc;
+  T5D_REQUIRE(b->keep_going && b->lane_alive && b->lane_records && b->lane >= 0 &&
+                  b->lane < b->n_lanes && B > 0 && K > 0 && b->S > 1 && n_counters >= 0 &&
+                  n_counters <= 256 && (counters || n_counters == 0),
+              T5D_EINVAL, "beam lane tail: lane %d of %d, B=%d K=%d S=%d counters=%d",
+              b->lane, b->n_lanes, B, K, b->S, n_counters);
+  hipLaunchKernelGGL(beam_lane_tail_kernel, dim3(1), dim3(256), 0, s, b->state, B, K, b->S,
+                     b->min_brevity, b->min_log_prob, b->max_decode_step,
+                     b->min_initial_index, b->keep_going, b->n_lanes, b->lane, b->lane_alive,
+                     b->lane_records, counters, n_counters);
+  T5D_CHECK_LAUNCH("beam lane tail");
   return T5D_OK;
 }
 

@@ -233,6 +233,8 @@ extern "C" int t5d_beam_search_step(void* stream, const t5d_model_step* m,
         b->state.cur_index, 1));
   // The tail advances cur_index and the cache indices and evaluates the loop
   // condition.
+  if (b->n_lanes > 1)
+    return launch_beam_lane_tail(hs, b, B, K, m->cache_index, m->NL);
   T5D_TRY(launch_beam_tail(hs, &b->state, B, K, b->S, b->min_brevity,
                            b->min_log_prob, b->max_decode_step,
                            b->min_initial_index, b->keep_going, !b->skip_cond,

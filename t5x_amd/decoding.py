@@ -857,7 +857,7 @@ class BeamLoop(_InFlight):
                   self.max_decode_step, self.min_initial, self.keep_going)
     return bool(self.keep_going.item())
 
-  def run(self, check_every: int = 8):
+  def run(self, check_every: int = 4):
     """Runs the loop to termination.  With a fused step the condition is read
     back only every `check_every` iterations: iterations enqueued after it
     turned false are no-ops on the device, so the final state is the same."""
@@ -865,9 +865,10 @@ class BeamLoop(_InFlight):
       while self.cond():
         self.body()
       return
-    while self.fused.keep_going():
-      self.fused.launch(check_every)
-      self.step += check_every
+    # Two chunks are ahead of the host, so that the device never waits for it.
+    self.start(check_every)
+    while not self.poll(block=True):
+      pass
 
   def advance(self, n: int):
     """n loop iterations without looking at the condition in between (with the

@@ -750,8 +750,13 @@ class Transformer(DecodeContexts):
     if loop.beam_size > 8:
       return None
     w = self.decoder_weights(params)
+    # Two lanes where their kernels are long enough for the overlap to make up
+    # for twice as many of them: ms with one / two, 64 tokens, 32 x 4 rows of
+    # small 22.0 / 22.5, 16 x 4 of base 35.7 / 37.0 and of large 80.4 / 85.5,
+    # 22 x 4 of base 40.2 / 38.4, 8 x 4 of xl (int8) 105 / 117, 16 x 4 136.6 / 136.7.
+    wide = loop.batch_size * loop.beam_size * self.config.emb_dim > 65536
     lanes = self.decode_lanes or (
-        1 if in_flight or self.streams_side_by_side() < 2 else 2)
+        2 if wide and not in_flight and self.streams_side_by_side() >= 2 else 1)
     lanes = max(1, min(int(lanes), loop.batch_size))
     key = (id(w), tuple(encoded.x.shape), encoded.x.dtype, encoded.beams,
            loop.batch_size, loop.beam_size, loop.max_decode_len,
@@ -820,6 +825,7 @@ class _OwnedContext:
   their loop alive."""
 
   CHUNK_SLOTS = 4  # chunks a caller may have outstanding per context
+  n_lanes = 1
   _owner = None
   _flag_host = None
   _n_chunks = 0
@@ -838,11 +844,11 @@ class _OwnedContext:
     device flag to pinned host memory and records an event behind it.
     Returns the ticket for _chunk_flag()."""
     if self._flag_host is None:
-      self._flag_host = torch.zeros((self.CHUNK_SLOTS,), dtype=torch.int32,
+      slots = self.CHUNK_SLOTS * self.n_lanes
+      self._flag_host = torch.zeros((slots,), dtype=torch.int32,
                                     pin_memory=True)
-      self._chunk_events = [torch.cuda.Event()
-                            for _ in range(self.CHUNK_SLOTS)]
-    slot = self._n_chunks % self.CHUNK_SLOTS
+      self._chunk_events = [torch.cuda.Event() for _ in range(slots)]
+    slot = self._n_chunks % len(self._chunk_events)
     self._n_chunks += 1
     with torch.cuda.stream(stream):
       self._flag_host[slot:slot + 1].copy_(flag.reshape(1), non_blocking=True)
@@ -1136,7 +1142,10 @@ class _BeamLane:
                           dtype=act, device=dev)
     self.cache_index = torch.zeros((nl,), dtype=torch.int32, device=dev)
     self.bufs = _StepBuffers(cfg, R, dev, act)
-    self.keep_going = loop.keep_going      # one flag for the whole batch
+    # one flag for the whole batch, or the lane's own (the loop's end is the
+    # whole batch's all the same)
+    self.keep_going = (loop.keep_going if owner.n_lanes == 1 else
+                       owner.lane_words[0, index])
     self.cur_index = owner.lane_cur_index[index]
     k2 = 2 * K
     f32, i32 = torch.float32, torch.int32
@@ -1188,13 +1197,15 @@ class _BeamLane:
     bs.kv_base = P(self.kv)
     bs.kv_tensor_stride_bytes = self.kv[0, 0].numel() * self.kv.element_size()
     bs.n_kv_tensors = 2 * nl
-    bs.skip_cond = 1 if owner.n_lanes > 1 else 0
+    if owner.n_lanes > 1:
+      bs.n_lanes, bs.lane = owner.n_lanes, index
+      bs.lane_alive = P(owner.lane_words[1])
+      bs.lane_records = P(owner.lane_records)
     if owner.deferred_gather:
       bs.cache_slot, bs.cache_src, bs.cache_dst = (
           P(self.cache_slot), P(self.cache_src), P(self.cache_dst))
     self.beam = bs
     self.stream = module.decode_stream(owner.slot * owner.n_lanes + index)
-    self.event = torch.cuda.Event()
     self.graph = None
     self.graph_long = None
 
@@ -1208,11 +1219,13 @@ class FusedBeamStep(_OwnedContext):
   replays its own graph on its own stream, so the lanes' kernels overlap on
   the device: while one lane sits in a latency-bound phase another one
   streams.  The loop condition stays the reference's single whole-batch
-  condition: after every iteration the lanes' streams join, one kernel
-  evaluates it over the whole (contiguous) beam state into the one device
-  flag that gates every kernel of every lane, and the lanes fork again, all
-  without the host.  Iterations enqueued after the flag turned 0 change
-  nothing, so the host may look at it only every few iterations."""
+  condition, but no lane waits for another after an iteration: each records
+  what its items say and goes on as long as they say yes, and only then looks
+  at the others' records (t5d_beam_step.lane_records).  Iterations enqueued
+  after the end, or while a lane has to know first what one behind it says,
+  change nothing, so the host may look only every few iterations.  (Streams
+  that joined after every iteration for one kernel that evaluated the
+  condition, base beam 4, 32 texts, 128 iterations: 89.4 ms; so: 83.2.)"""
 
   def __init__(self, module, loop, params, encoded, enc_tokens, lanes=None,
                slot=0):
@@ -1262,7 +1275,10 @@ class FusedBeamStep(_OwnedContext):
     self.slot = slot
     bounds = [B * i // n for i in range(n + 1)]
     self.lane_cur_index = loop.cur.cur_index.to(torch.int32).reshape(1).repeat(n)
-    self.cond_event = torch.cuda.Event()
+    # [0]: the lanes' gates, [1]: whether they have yet to reach the loop's end
+    self.lane_words = torch.zeros((2, n), dtype=torch.int32, device=dev)
+    self.lane_records = torch.zeros((n, S + 1), dtype=torch.int32, device=dev)
+    self._enqueued = 0  # iterations since the loop was bound
     # What the captured graphs hold addresses of, beyond the lanes' own
     # buffers: the loop's state.  A later loop is re-bound onto these.
     self.w, self.cross = w, cross
@@ -1323,8 +1339,18 @@ class FusedBeamStep(_OwnedContext):
     self.loop = loop
     for lane in self.lanes:
       lane.stream.wait_stream(cur)
-    self._cond(self.lanes[0].stream)
-    self.lanes[0].stream.synchronize()
+    self._open()
+
+  def _open(self):
+    """The loop condition of a freshly bound loop -> the gates."""
+    first = self.lanes[0].stream
+    self._cond(first)
+    if self.n_lanes > 1:
+      with torch.cuda.stream(first):
+        self.lane_words.copy_(self.flag.expand_as(self.lane_words))
+        self.lane_records.zero_()
+    self._enqueued = 0
+    first.synchronize()
 
   def _enqueue(self, lane):
     self._lib.call('t5d_beam_search_step', lane.stream.cuda_stream,
@@ -1347,9 +1373,9 @@ class FusedBeamStep(_OwnedContext):
                    int(loop.max_decode_step), int(loop.min_initial),
                    loop.keep_going.data_ptr())
 
-  # Iterations recorded in the long graph of a single-lane loop: one launch
-  # (and one gap between launches) per that many iterations.
-  GRAPH_STEPS = 8
+  # Iterations recorded in the long graph: one launch (and one gap between
+  # launches) per that many.
+  GRAPH_STEPS = 4
 
   def _record(self, lane, steps):
     lib = self._lib
@@ -1399,53 +1425,67 @@ class FusedBeamStep(_OwnedContext):
         self._enqueue(lane)
         lane.stream.synchronize()
         lane.graph = self._record(lane, 1)
-        if self.n_lanes == 1:
-          lane.graph_long = self._record(lane, self.GRAPH_STEPS)
+        lane.graph_long = self._record(lane, self.GRAPH_STEPS)
       lane.stream.synchronize()
-    self._cond(self.lanes[0].stream)
-    self.lanes[0].stream.synchronize()
+    self._open()
+
+  def _launch_lane(self, lane, n):
+    lib, stream = self._lib, lane.stream.cuda_stream
+    while n >= self.GRAPH_STEPS:
+      lib.call('t5d_graph_launch', lane.graph_long, stream)
+      n -= self.GRAPH_STEPS
+    for _ in range(n):
+      lib.call('t5d_graph_launch', lane.graph, stream)
 
   def launch(self, n=1):
-    lanes, lib = self.lanes, self._lib
-    first = lanes[0].stream
-    if len(lanes) == 1:
-      lane = lanes[0]
-      while n >= self.GRAPH_STEPS:
-        lib.call('t5d_graph_launch', lane.graph_long, first.cuda_stream)
-        n -= self.GRAPH_STEPS
-      for _ in range(n):
-        lib.call('t5d_graph_launch', lane.graph, first.cuda_stream)
-      return
-    for _ in range(n):
-      for lane in lanes:
-        lib.call('t5d_graph_launch', lane.graph, lane.stream.cuda_stream)
-      # join -> one condition for the whole batch -> fork
-      for lane in lanes[1:]:
-        lane.event.record(lane.stream)
-        first.wait_event(lane.event)
-      self._cond(first)
-      self.cond_event.record(first)
-      for lane in lanes[1:]:
-        lane.stream.wait_event(self.cond_event)
+    self._enqueued += n
+    while n > 0:  # (the lanes in turn, so that none starts late)
+      k = min(n, self.GRAPH_STEPS)
+      for lane in self.lanes:
+        self._launch_lane(lane, k)
+      n -= k
 
   def launch_chunk(self, n):
-    """launch(n), and a ticket for chunk_running().  (The loop condition
-    bounds the loop: there is always a next iteration to enqueue.)"""
+    """launch(n), and a ticket for chunk_running(); None once as many
+    iterations are enqueued as the loop can have."""
+    if self._enqueued >= self.loop.max_decode_len - 1:
+      return None
     self.launch(n)
-    # the last condition of a chunk is evaluated on the first lane's stream
-    # after all lanes joined; a single lane's kernels are on that stream too
-    return self._end_chunk(self.flag, self.lanes[0].stream)
+    if self.n_lanes == 1:
+      return [self._end_chunk(self.flag, self.lanes[0].stream)]
+    return [self._end_chunk(self.lane_words[1, i], lane.stream)
+            for i, lane in enumerate(self.lanes)]
 
   def chunk_running(self, ticket, block=False):
     """Whether the loop condition still held after that chunk; None while the
     chunk is running (block: wait for it)."""
-    flag = self._chunk_flag(ticket, block)
-    return None if flag is None else flag != 0
+    flags = [self._chunk_flag(t, block) for t in ticket]
+    return None if None in flags else any(flags)
 
-  def synchronize(self):
+  def _drain(self):
     for lane in self.lanes:
       lane.stream.synchronize()
-    # the lanes advance in lock step
+
+  def synchronize(self):
+    """Waits for what is enqueued; every lane has then made all of the loop's
+    iterations up to there."""
+    self._drain()
+    n = self.n_lanes
+    while n > 1:
+      # A lane that had to know first what another one says has left
+      # iterations out; the one furthest behind can always go on.
+      state = torch.cat([self.lane_words.reshape(-1),
+                         self.lane_cur_index]).tolist()
+      gates, alive, at = state[:n], state[n:2 * n], state[2 * n:]
+      behind = [i for i in range(n)
+                if alive[i] and (not gates[i] or at[i] < self._enqueued)]
+      if not behind:
+        self.flag.fill_(int(any(alive)))
+        break
+      for i in behind:
+        self._launch_lane(self.lanes[i],
+                          self._enqueued - at[i] if gates[i] else 1)
+      self._drain()
     self.loop.cur.cur_index.copy_(self.lane_cur_index[0])
 
   def keep_going(self) -> bool:

@@ -461,6 +461,40 @@ def test_fused_loop_early_stop_is_independent_of_check_interval(check_every,
   assert torch.equal(torch.as_tensor(gs), torch.as_tensor(ws))
 
 
+@pytest.mark.parametrize('lanes,order', [(2, [0, 1]), (2, [1, 0]), (3, [2, 0, 1]),
+                                         (4, [3, 1, 0, 2])])
+@pytest.mark.parametrize('seed,eos_bias', [(11, 6.0), (12, 3.0), (13, 0.0)])
+def test_lanes_that_run_far_apart_make_the_loops_iterations(lanes, order, seed,
+                                                            eos_bias):
+  """Lanes whose iterations are all enqueued one lane after the other: those whose items
+  have ended wait for what the others say, and every lane stops where the loop does."""
+  from t5x_amd import decoding
+  B, K, L = 4, 4, 40
+  module, fn = _decode_setup('bfloat16', B, K, 16, L, seed=seed, eos_bias=eos_bias)
+  module.decode_lanes = lanes
+  inputs = np.zeros((B, L), np.int32)
+  plain = decoding.BeamLoop(inputs, dict(module.init_cache(B, L)), fn,
+                            eos_id=1, num_decodes=K)
+  plain.run()
+  want, ws = plain.finish()
+  steps = int(plain.cur.cur_index.item())
+  fused = decoding.BeamLoop(inputs, module.init_cache(B, L), fn, eos_id=1,
+                            num_decodes=K)
+  step = fused.fused
+  assert step.keep_going()
+  step._enqueued = L
+  for i in order:
+    step._launch_lane(step.lanes[i], L)
+    step.lanes[i].stream.synchronize()
+  assert step.lane_cur_index.max().item() <= steps
+  assert not step.keep_going()
+  assert step.lane_cur_index.tolist() == [steps] * lanes
+  got, gs = fused.finish()
+  assert int(fused.cur.cur_index.item()) == steps
+  assert torch.equal(torch.as_tensor(got), torch.as_tensor(want))
+  assert torch.equal(torch.as_tensor(gs), torch.as_tensor(ws))
+
+
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
 def test_fused_loop_context_is_reused_across_batches(dtype):
   """A second (and third) batch of the same shape on the same module re-binds
