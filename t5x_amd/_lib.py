@@ -163,7 +163,8 @@ class Recurrence(Structure):
                      i2='ld_proj off_q off_k off_v off_beta off_gate', p2='low',
                      i3='ld_low off_z off_low_gate',
                      p3='decay_bias A_log conv norm conv_ring state out',
-                     i4='ld_out', p4='workspace', l='workspace_bytes')
+                     i4='ld_out', p4='workspace', l='workspace_bytes', p5='low_w',
+                     i5='off_low low_k low_n')
 
 
 class HybridLayer(Structure):

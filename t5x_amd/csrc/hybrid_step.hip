@@ -88,6 +88,7 @@ int mixer(void* stream, const t5d_hybrid_model* m, const t5d_hybrid_layer& l,
   t5d_recurrence a = l.recurrence;
   a.dtype = m->dtype; a.proj = m->proj; a.ld_proj = l.proj_n;
   a.low = m->low; a.ld_low = l.low_n;
+  a.low_w = l.low; a.off_low = l.off_low; a.low_k = l.low_k; a.low_n = l.low_n;
   a.state = (float*)run.cache0; a.conv_ring = run.cache1;
   a.out = l.mix_rows; a.ld_out = l.out_k;
   a.workspace = m->workspace;
@@ -254,11 +255,6 @@ extern "C" int t5d_hybrid_step(void* stream, const t5d_hybrid_model* m,
     } else {
       T5D_TRY(row_dense(l.norm1, l.proj, dt, m->proj, l.proj_n, l.proj_n, l.proj_n,
                         T5D_EPI_NONE, 0.f, 0.f, 0.f));
-    }
-    if (l.low) {
-      const char* a = (const char*)m->proj + (size_t)l.off_low * (dt == T5D_F32 ? 4 : 2);
-      T5D_TRY(t5d_dense(stream, dt, T5D_F32, a, l.proj_n, l.low, m->low, l.low_n,
-                        l.low_n, M, l.low_k, l.low_n, T5D_EPI_NONE, 0.f, 0.f, 0.f));
     }
     T5D_TRY(mixer(stream, m, l, run, b));
     // Two to four streams of some width, many rows: the row kernel behind the first branch

@@ -1050,10 +1050,17 @@ recurrence_finish_kernel(RecArgs g) {
 // step: delta rule 8.0 -> 6.2 us, without 7.3 -> 5.6; launches behind one another, 1 / 64
 // rows of 8 heads: 6.1 / 11.7 -> 5.0 / 10.3, of 64 x 64 4.6 / 6.2 -> 3.9 / 5.5, of 32 x 32
 // 4.1 / 4.8 -> 3.5 / 4.2).  Heads of 256 have two taps ahead and no registers to gain.
-template <int DI, bool DELTA, typename T, bool EXACT>
+// LOWP > 0: the low-rank stage too, of LOWP pairs of k-tiles.  Every wavefront multiplies the
+// token's inputs by its part of the head's columns (one row, in all 16 of the matrix cores;
+// summed as t5d_dense does, so with its bits), and the decays are formed where their z lies.
+template <int DI, bool DELTA, typename T, bool EXACT, int LOWP>
 __global__ void __launch_bounds__(512)
 recurrence_step_kernel(RecArgs g) {
   constexpr int DP = 8 * DI;
+  constexpr bool LOW = LOWP > 0;
+  constexpr int TPW = DP >= 64 ? DP / 64 : 1;  // LOW: column tiles of 16 per wavefront
+  static_assert(!LOW || (EXACT && sizeof(T) == 2), "which heads have the low-rank stage");
+  __shared__ float s_lg[LOW ? DP : 1];
   __shared__ float s_q[DP], s_k[DP], s_g[DP];
   __shared__ __align__(16) float s_v[256];
   __shared__ __align__(16) float s_o[256];
@@ -1088,7 +1095,65 @@ recurrence_step_kernel(RecArgs g) {
   };
   const T* ring = reinterpret_cast<const T*>(a.conv_ring) +
                   (size_t)slot * a.taps * g.C;
+  // (tiles of z, then of the gate; a wavefront past the head's columns has none)
+  const bool low_gate = a.gate == T5D_GATE_SIGMOID_LOW;
+  const bool has_low = LOW && 16 * TPW * wave < DP;
+  uint4 low_in[LOW ? 2 * LOWP : 1], low_w[LOW ? 2 : 1][TPW][LOW ? 2 * LOWP : 1];
+  float low_bias = 0.f;
+  const int low_c = min(16 * TPW * wave + (lane & (16 * TPW - 1)), DP - 1);
+  const auto request_low = [&] {
+    if constexpr (LOW) {
+      const uint4* in = reinterpret_cast<const uint4*>(p + a.off_low) + (lane >> 4);
+#pragma unroll
+      for (int k = 0; k < 2 * LOWP; ++k) low_in[k] = in[4 * k];
+      low_bias = a.decay_bias[(size_t)h * DP + low_c];
+#pragma unroll
+      for (int which = 0; which < 2; ++which) {
+        if (which == 1 && !low_gate) break;
+        const int tile = ((which ? a.off_low_gate : a.off_z) + h * DP) / 16 + TPW * wave;
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+          for (int k = 0; k < 2 * LOWP; ++k)
+            low_w[which][t][k] = reinterpret_cast<const uint4*>(
+                a.low_w)[((size_t)(tile + t) * 2 * LOWP + k) * 64 + lane];
+      }
+    }
+  };
+  const auto form_low = [&] {
+    if constexpr (LOW) {
+#pragma unroll
+      for (int which = 0; which < 2; ++which) {
+        if (which == 1 && !low_gate) break;
+        float z[TPW];
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+          f32x4_v acc[LOWP];
+#pragma unroll
+          for (int q = 0; q < LOWP; ++q) {
+            acc[q] = (f32x4_v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 2 * q; k < 2 * q + 2; ++k) {
+              Frag x, w;
+              x.u = low_in[k];
+              w.u = low_w[which][t][k];
+              acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, w.v, acc[q], 0, 0, 0);
+            }
+          }
+          z[t] = LOWP > 1 ? acc[0][0] + acc[LOWP - 1][0] : acc[0][0];
+        }
+        // (every group of 16 lanes holds all tiles: lane l takes its l / 16th)
+        float v = z[0];
+        if constexpr (TPW > 1) v = (lane & 16) ? z[1] : z[0];
+        if (lane < 16 * TPW) {
+          if (which == 0) s_g[low_c] = expf(log_decay_of(a, v + low_bias, h));
+          else s_lg[low_c] = v;
+        }
+      }
+    }
+  };
   const auto request = [&](int role) {
+    if (LOW && role == 3) return;
     if (role == 3) {
 #pragma unroll
       for (int u = 0; u < (DP + 63) / 64; ++u) {
@@ -1142,22 +1207,23 @@ recurrence_step_kernel(RecArgs g) {
   };
   if (!DELTA) request_state();
   if (wave < 4) request(wave);
+  if (has_low) request_low();
   const T beta_z = p[DELTA ? a.off_beta + h : 0];
   // the output channel of this lane
   const int co = 64 * wave + lane;
   const int cg = EXACT ? co % Dv : min(co, Dv - 1);
   const float norm = a.norm[cg];
   // (each from a place that is there; one of them is used)
-  const bool low_gate = a.gate == T5D_GATE_SIGMOID_LOW;
   const float gate_low =
-      a.low[(size_t)m * a.ld_low + (low_gate ? a.off_low_gate + h * Dv + cg : a.off_z)];
+      LOW ? 0.f
+          : a.low[(size_t)m * a.ld_low + (low_gate ? a.off_low_gate + h * Dv + cg : a.off_z)];
   const T gate_z = (low_gate ? p : p + a.off_gate + (size_t)h * Dv)[low_gate ? 0 : cg];
   if (DELTA) request_state();
   T5D_GATE_TEST();
   const auto form = [&](int role) {
     if (role == 3) {
 #pragma unroll
-      for (int u = 0; u < (DP + 63) / 64; ++u) {
+      for (int u = 0; !LOW && u < (DP + 63) / 64; ++u) {
         const int c = lane + 64 * u;
         if (c < DP)
           s_g[c] = c < D ? expf(log_decay_of(a, tap[u][1] + tap[u][0], h)) : 0.f;
@@ -1199,6 +1265,7 @@ recurrence_step_kernel(RecArgs g) {
       if (lane + 64 * u < pad) dst[lane + 64 * u] = x[u] * f;
   };
   if (wave < 4) form(wave);
+  if (has_low) form_low();
   __syncthreads();
   // (a wavefront that was there for its role; barriers wait for those that stay)
   if (32 * wave >= Dv) return;
@@ -1255,16 +1322,46 @@ recurrence_step_kernel(RecArgs g) {
     Act<T>::store(reinterpret_cast<T*>(a.out) + (size_t)m * a.ld_out +
                       (size_t)h * Dv + co,
                   s_o[co] * inv * norm *
-                      out_gate_of(a, low_gate ? gate_low : to_f32<T>(gate_z)));
+                      out_gate_of(a, !low_gate ? to_f32<T>(gate_z)
+                                     : LOW     ? s_lg[cg]
+                                               : gate_low));
+}
+
+// Whether a step forms its low-rank columns itself: where heads are as wide as the kernel's
+// variant, up to the rows measured.  Steps of 8 layers (6 of them recurrences, heads of 128,
+// 64 to 128 inputs), us with a dense layer in front / so, rows 1, 8, 64, 256: 8 heads (width
+// 1024) 224.7 / 216.2, 302 / 287, 438 / 424, 1114 / 1090; 16 heads 357 / 341, 468 / 451,
+// 785 / 773, 2013 / 1971.
+static bool low_rides(const t5d_recurrence& a, int64_t rows) {
+  return a.dtype == T5D_BF16 && a.D == a.Dv && (a.D == 32 || a.D == 64 || a.D == 128) &&
+         a.taps <= 4 && (a.low_k == 64 || a.low_k == 128) && a.off_z % 16 == 0 &&
+         (a.gate != T5D_GATE_SIGMOID_LOW || a.off_low_gate % 16 == 0) &&
+         a.off_low % 8 == 0 && a.ld_proj % 8 == 0 &&
+         ((uintptr_t)a.proj | (uintptr_t)a.low_w) % 16 == 0 && rows * a.H <= 4096;
 }
 
 template <bool DELTA, typename T>
 static void launch_step(hipStream_t s, const RecArgs& g) {
   const dim3 grid(g.b.S * g.a.H), block(64 * std::max(4, (g.a.Dv + 31) / 32));
-#define T5D_RS(DI_, EXACT_)                                                       \
-  hipLaunchKernelGGL((recurrence_step_kernel<DI_, DELTA, T, EXACT_>), grid, block, 0, \
-                     s, g)
+#define T5D_RSL(DI_, EXACT_, LOWP_)                                                     \
+  hipLaunchKernelGGL((recurrence_step_kernel<DI_, DELTA, T, EXACT_, LOWP_>), grid, block, \
+                     0, s, g)
+#define T5D_RS(DI_, EXACT_) T5D_RSL(DI_, EXACT_, 0)
   const bool exact = g.a.D == g.a.Dv && g.a.taps <= 4;
+  if constexpr (sizeof(T) == 2) {
+    if (g.a.low_w != nullptr) {  // (low_rides)
+#define T5D_RSW(DI_)                             \
+  do {                                           \
+    if (g.a.low_k == 64) T5D_RSL(DI_, true, 1);  \
+    else T5D_RSL(DI_, true, 2);                  \
+  } while (0)
+      if (g.a.D == 32) T5D_RSW(4);
+      else if (g.a.D == 64) T5D_RSW(8);
+      else T5D_RSW(16);
+#undef T5D_RSW
+      return;
+    }
+  }
   if (exact && g.a.D == 32) T5D_RS(4, true);
   else if (g.a.D <= 32) T5D_RS(4, false);
   else if (exact && g.a.D == 64) T5D_RS(8, true);
@@ -1273,6 +1370,7 @@ static void launch_step(hipStream_t s, const RecArgs& g) {
   else if (g.a.D <= 128) T5D_RS(16, false);
   else T5D_RS(32, false);
 #undef T5D_RS
+#undef T5D_RSL
 }
 
 template <bool DELTA, typename TQ>
@@ -1423,7 +1521,17 @@ extern "C" int t5d_recurrence_run(void* stream, const t5d_recurrence* a,
   T5D_REQUIRE(variant != 1 || can_step, T5D_EINVAL,
               "t5d_recurrence_run: variant 1 does not cover this call");
   hipStream_t s = as_stream(stream);
-  if (variant == 1 || (variant == 0 && can_step)) {
+  const bool step = variant == 1 || (variant == 0 && can_step);
+  if (a->low_w != nullptr && !(step && low_rides(*a, b->S))) {
+    const char* in =
+        (const char*)a->proj + (size_t)a->off_low * (a->dtype == T5D_F32 ? 4 : 2);
+    const int rc = t5d_dense(stream, a->dtype, T5D_F32, in, a->ld_proj, a->low_w, a->low,
+                             a->ld_low, a->low_n, b->M, a->low_k, a->low_n, T5D_EPI_NONE,
+                             0.f, 0.f, 0.f);
+    if (rc != T5D_OK) return rc;
+    g.a.low_w = nullptr;
+  }
+  if (step) {
     g.wq = g.wk = g.wv = g.wbeta = g.wo = g.wchunk = nullptr;
     g.order = nullptr;
     g.chunks = 0;

@@ -768,6 +768,63 @@ class Recurrence:
     return 1e-5 if self.dt == torch.float32 else 4e-3
 
 
+# every head size that has it, one and two pairs of k-tiles, fewer keys than heads, taps of
+# which the last are not there
+@pytest.mark.parametrize('delta,D,taps,rank', [
+    (True, 128, 4, 128), (True, 64, 3, 128), (True, 32, 4, 64), (False, 128, 0, 64),
+    (False, 64, 0, 128), (False, 32, 0, 64), (True, 48, 2, 64), (True, 128, 4, 192)])
+@pytest.mark.parametrize('dt,S', [(torch.bfloat16, 1), (torch.bfloat16, 7),
+                                  (torch.float32, 2)])
+def test_steps_that_form_their_low_rank_columns(dt, S, delta, D, taps, rank):
+  """With low_w a call has the bits, outputs, states and rings, of t5d_dense in front of it,
+  in steps, whose kernel forms the columns itself (not of 48 channels, of 192 inputs or in
+  float32), and in a portion."""
+  from t5x_amd import _lib, ops
+  H, G = 4, 2 if delta else 4
+  r = Recurrence(dt, delta, H, G, D, D, taps, S, seed=D + rank)
+  rs, d = np.random.RandomState(S + D), r.r
+  d.off_low = (r.cols + 7) // 8 * 8
+  d.ld_proj = d.off_low + rank
+  d.off_z, d.off_low_gate = 16, 32 + H * D
+  d.low_k, d.low_n = rank, 48 + 2 * H * D
+  d.ld_low = d.low_n + (4 if dt == torch.bfloat16 else 0)
+  w = ops.pack_weight(dev(2 * rs.randn(rank, d.low_n) * rank ** -0.5), dt)
+  P, el = _lib.ptr, torch.empty((), dtype=dt).element_size()
+
+  def run(portions, proj, given):
+    M = len(proj)
+    x = Ragged(portions)
+    low = torch.full((M, d.ld_low), float('nan'), device='cuda')
+    out = torch.full((M, H * D), 3.0, dtype=dt, device='cuda')
+    ws = torch.empty((_lib.load().t5d_recurrence_workspace_bytes(
+        M, len(portions), H, G, D, D),), dtype=torch.uint8, device='cuda')
+    d.proj, d.low, d.out, d.ld_out = P(proj), P(low), P(out), H * D
+    d.workspace, d.workspace_bytes = P(ws), ws.numel()
+    d.low_w = None if given else w.data.data_ptr()
+    if given:
+      _lib.call('t5d_dense', ops._s(), d.dtype, _lib.F32, P(proj) + d.off_low * el,
+                d.ld_proj, w.data.data_ptr(), P(low), d.ld_low, d.low_n, M, rank, d.low_n,
+                _lib.EPI_NONE, 0.0, 0.0, 0.0)
+    ops.recurrence(d, x.ragged, 0)
+    return out
+
+  seen = []
+  for given in (True, False):
+    r.state.fill_(float('nan'))
+    r.ring.fill_(float('nan'))
+    rs = np.random.RandomState(5)
+    outs = []
+    for n in (1, 1, 1, 40):
+      at = sum(len(o) for o in outs) // S
+      proj = dev(rs.randn(S * n, d.ld_proj), dt)
+      outs.append(run([(i, at, n) for i in range(S)], proj, given))
+    assert all(bool(torch.isfinite(t.float()).all()) for t in outs + [r.state])
+    # (a place of the ring that no later token looks at may be as it was)
+    seen.append(outs + [r.state.clone(), r.ring.nan_to_num()])
+  for a, b in zip(*seen):
+    assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize('dt', DTYPES)
 @pytest.mark.parametrize('delta,D,Dv,taps', [(True, 128, 40, 4), (True, 40, 128, 6),
                                              (False, 128, 48, 0), (True, 200, 20, 0)])
