@@ -14,6 +14,7 @@
 //     short portions.
 #include "common.h"
 #include "gemm_tiles.h"
+#include "norm_dense.h"
 
 namespace t5d {
 
@@ -31,6 +32,7 @@ struct LatentArgs {
 };
 
 // ---- norms of the new latents, ring update --------------------------------------
+// (Of up to 128 rows in one launch with the queries' layer: norm_dense_kernel.)
 // One wavefront per (token, query latent or cached latent).  The projection's
 // columns and the norm's weights are zero from the latent's size to the next
 // multiple of 16 and RP / QP, so the padding of what is written is zero.
@@ -386,6 +388,28 @@ static int tile_splits(const t5d_latent_attention& a, const t5d_ragged& b) {
   return n;
 }
 
+// latent_append_kernel and the queries' dense layer in one launch, with their bits, for up to
+// 128 rows.
+static bool new_latents_and_queries(hipStream_t s, const LatentArgs& g, int QN) {
+  const t5d_latent_attention& a = g.a;
+  if (((uintptr_t)a.uq | (uintptr_t)a.q_norm | (uintptr_t)a.kv_norm) % 16 != 0 ||
+      QN % 16 != 0)
+    return false;
+  LatentDenseArgs d = {};
+  d.A = reinterpret_cast<const bf16_t*>(a.proj) + a.off_q; d.lda = a.ld_proj;
+  d.W = a.uq; d.C = a.q; d.M = g.b.M; d.K = g.QP; d.N = QN;
+  d.ldc = d.n_store = QN;
+  d.gate = g.gate; d.epilogue = T5D_EPI_NONE; d.eps = a.eps;
+  d.norm = a.q_norm; d.d = a.q_rank;
+  if (a.off_kv >= 0) {
+    d.kv = reinterpret_cast<const bf16_t*>(a.proj) + a.off_kv;
+    d.kv_norm = a.kv_norm; d.kv_d = a.rank; d.kv_pad = g.RP;
+    d.ring = reinterpret_cast<bf16_t*>(a.latent_ring); d.ring_len = a.ring;
+    d.seq_slot = g.b.seq_slot; d.tok_seq = g.b.tok_seq; d.tok_pos = g.b.tok_pos;
+  }
+  return launch_latent_dense(d, s);
+}
+
 }  // namespace t5d
 
 using namespace t5d;
@@ -462,16 +486,21 @@ extern "C" int t5d_latent_attention_run(void* stream, const t5d_latent_attention
               "t5d_latent_attention_run: variant %d does not cover this call",
               variant);
 
-  const int64_t units = (int64_t)b->M * (a->off_kv >= 0 ? 2 : 1);
-  const dim3 agrid((unsigned)((units + 3) / 4)), block(256);
-  if (bf16)
-    hipLaunchKernelGGL(latent_append_kernel<bf16_t>, agrid, block, 0, s, g);
-  else
-    hipLaunchKernelGGL(latent_append_kernel<float>, agrid, block, 0, s, g);
-  T5D_CHECK_LAUNCH("latent attention (append)");
   const int QN = a->H * g.HP;
-  T5D_TRY(t5d_dense(stream, a->dtype, a->dtype, a->cq, g.QP, a->uq, a->q, QN, QN, b->M,
-                    g.QP, QN, T5D_EPI_NONE, 0.f, 0.f, 0.f));
+  const dim3 block(256);
+  // (cq is not written then; nothing else reads it)
+  if (!(bf16 && new_latents_and_queries(s, g, QN))) {
+    const int64_t units = (int64_t)b->M * (a->off_kv >= 0 ? 2 : 1);
+    const dim3 agrid((unsigned)((units + 3) / 4));
+    if (bf16)
+      hipLaunchKernelGGL(latent_append_kernel<bf16_t>, agrid, block, 0, s, g);
+    else
+      hipLaunchKernelGGL(latent_append_kernel<float>, agrid, block, 0, s, g);
+    T5D_CHECK_LAUNCH("latent attention (append)");
+    T5D_TRY(t5d_dense(stream, a->dtype, a->dtype, a->cq, g.QP, a->uq, a->q, QN, QN, b->M,
+                      g.QP, QN, T5D_EPI_NONE, 0.f, 0.f, 0.f));
+  }
+  T5D_CHECK_LAUNCH("latent attention (queries)");
 
   if (variant == 2 || (variant == 0 && can_span)) {
     const int64_t n = (int64_t)span->rows * (g.RP / 8);

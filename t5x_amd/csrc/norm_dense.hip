@@ -33,13 +33,36 @@ namespace t5d {
 template <typename Args, int NT, int KQ, typename WT>
 __global__ void __launch_bounds__(512)
 norm_dense_kernel(Args g) {
-  constexpr bool kStream = IsStream<Args>::value;
+  constexpr bool kStream = IsStream<Args>::value, kLatent = IsLatent<Args>::value;
   constexpr int LD = 256 * KQ, HS = LD + 8;  // row stride of the normed rows
   constexpr int TB = WeightTile<WT>::kTileBytes, TN = 32 * NT;
   __shared__ __align__(16) bf16_t s_h[16 * HS];
   __shared__ float red[8][NT * 4][64];
   __shared__ __align__(16) float s_norm[kStream ? 2 : 1][LD];
   T5D_GATE_READ(g.gate);
+  if constexpr (kLatent) {
+    if ((int)blockIdx.x >= g.dense_blocks) {  // a cached latent per wavefront
+      const int m = 8 * (blockIdx.x - g.dense_blocks) + (threadIdx.x >> 6);
+      T5D_GATE_TEST();
+      if (m >= g.M) return;
+      const int at = 8 * (threadIdx.x & 63), have = (g.kv_d + 15) & ~15;
+      const bf16_t* row = g.kv + (size_t)m * g.lda;
+      bf16_t* dst = g.ring + ((size_t)g.seq_slot[g.tok_seq[m]] * g.ring_len +
+                              g.tok_pos[m] % g.ring_len) * g.kv_pad;
+      float ss = 0.f;
+      for (int c = at; c < have; c += 512) {
+        float f[8];
+        unpack16(latent_piece(row, c, have), f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
+      }
+      const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)g.kv_d + g.eps);
+      for (int c = at; c < g.kv_pad; c += 512)
+        *reinterpret_cast<uint4*>(dst + c) =
+            latent_normed(latent_piece(row, c, have), inv, g.kv_norm + c);
+      return;
+    }
+  }
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int n_group = (slot / g.m_parts) * 8 + xcd;
   const int m_part = slot % g.m_parts;
@@ -63,6 +86,8 @@ norm_dense_kernel(Args g) {
       vec_y[v] = g.y_norm != nullptr ? norm_column(g.y_norm, c, d)
                                      : make_float4(1.f, 1.f, 1.f, 1.f);
       vec[v] = norm_column(g.norm, c, d);
+    } else if constexpr (kLatent) {
+      vec[v] = norm_column(g.norm, c, d);
     } else {
       uint2 q = make_uint2(0, 0);
       if (c < d) q = *reinterpret_cast<const uint2*>(g.norm_scale + c);
@@ -70,15 +95,23 @@ norm_dense_kernel(Args g) {
                            bf16hi_to_f32(q.y));
     }
   }
+  constexpr int KP8 = (KQ + 1) / 2;  // groups of 8 columns per lane
+  uint4 x8[kLatent ? 2 : 1][KP8];
+  const int have = kLatent ? (d_of_norm(g) + 15) & ~15 : 0;
   float4 x[kStream ? 2 : 1][KQ];
   uint2 y[2][KQ];  // (not a stream: the rows themselves)
   const bool add = has_branch(g);
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     // (past the end: the last row, not stored)
-    const size_t row = (size_t)min(m0 + 2 * wave + r, g.M - 1) * K;
+    const size_t row = (size_t)min(m0 + 2 * wave + r, g.M - 1) * row_stride(g);
+    if constexpr (kLatent) {
 #pragma unroll
-    for (int q = 0; q < KQ; ++q) {
+      for (int q = 0; q < KP8; ++q)
+        x8[r][q] = latent_piece(g.A + row, 8 * lane + 512 * q, have);
+    }
+#pragma unroll
+    for (int q = 0; !kLatent && q < KQ; ++q) {
       const int c = 4 * lane + 256 * q;
       const bool on = c < K;
       y[r][q] = make_uint2(0, 0);
@@ -180,6 +213,29 @@ norm_dense_kernel(Args g) {
         *reinterpret_cast<uint2*>(s_h + (2 * wave + r) * HS + c) = make_uint2(
             pack_bf16x2(x[r][q].x * inv[r] * wx.x, x[r][q].y * inv[r] * wx.y),
             pack_bf16x2(x[r][q].z * inv[r] * wx.z, x[r][q].w * inv[r] * wx.w));
+    }
+  } else if constexpr (kLatent) {  // (summed as latent_append_kernel does)
+    float inv[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      float ss = 0.f;
+#pragma unroll
+      for (int q = 0; q < KP8; ++q) {
+        float f[8];
+        unpack16(x8[r][q], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
+      }
+      inv[r] = 1.0f / sqrtf(wave_sum(ss) / (float)d_of_norm(g) + g.eps);
+    }
+#pragma unroll
+    for (int q = 0; q < KP8; ++q) {
+      const int c = 8 * lane + 512 * q;
+      if (KQ % 2 != 0 && c >= LD) break;
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+        *reinterpret_cast<uint4*>(s_h + (2 * wave + r) * HS + c) =
+            latent_normed(x8[r][q], inv[r], &s_norm[0][c]);
     }
   } else {
     // (summed as norm_gemm_kernel does, so that a row has the same bits in both)
@@ -300,6 +356,35 @@ bool launch_norm_dense(int w_dtype, const GemmArgs& g, hipStream_t s) {
   if (nt == 0 || g.N / 16 * ((g.M + 15) / 16) <= (g.K <= 512 ? 512 : 256)) return false;
   if (w_dtype == T5D_I8) launch<GemmArgs, int8_t>(nt, g, s);
   else launch<GemmArgs, bf16_t>(nt, g, s);
+  return true;
+}
+
+// Up to 128 rows whose columns fit 256 workgroups of four column tiles (two halves of two).
+// Steps of 8 layers, 4 of them with a cache of their own, us with two launches / so, rows 1,
+// 8, 64, 128: 6 heads of 128 (width 768) 405 / 387, 497 / 480, 646 / 624, 821 / 799; 8 heads
+// 458 / 435, 562 / 539, 756 / 732, 963 / 936; 16 heads 649 / 627, 863 / 837, 1414 / 1382,
+// 1722 / 1687.
+bool launch_latent_dense(LatentDenseArgs g, hipStream_t s) {
+  if (g.M > 128 || g.K > 1024 || g.K % 64 != 0) return false;
+  const int nt = tiles_per_half(g.M, g.N, 2);
+  if (nt == 0) return false;
+  const int groups = (g.N / 16 + 2 * nt - 1) / (2 * nt);
+  g.m_parts = (g.M + 15) / 16;
+  g.dense_blocks = (groups + 7) / 8 * 8 * g.m_parts;
+  const dim3 grid(g.dense_blocks + (g.kv != nullptr ? (g.M + 7) / 8 : 0)), block(512);
+#define T5D_LD_K(NT_, KQ_)                                                               \
+  hipLaunchKernelGGL((norm_dense_kernel<LatentDenseArgs, NT_, KQ_, bf16_t>), grid, block, \
+                     0, s, g)
+#define T5D_LD(NT_)                        \
+  do {                                     \
+    if (g.K <= 512) T5D_LD_K(NT_, 2);      \
+    else if (g.K <= 768) T5D_LD_K(NT_, 3); \
+    else T5D_LD_K(NT_, 4);                 \
+  } while (0)
+  if (nt == 1) T5D_LD(1);
+  else T5D_LD(2);
+#undef T5D_LD
+#undef T5D_LD_K
   return true;
 }
 

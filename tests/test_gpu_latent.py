@@ -514,3 +514,27 @@ def test_token_ids_choose_the_experts(dtype):
   got = host(live.step([(t, [3, t], [1]) for t in (4, 5, 6)]))
   np.testing.assert_array_equal(got[0], got[2])
   assert abs(got[0] - got[1]).max() > 0.1
+
+
+# queries of 64 to 1000 columns (the kernel's three widths), one and two column tiles per half
+# of a workgroup, a last row tile of one row; layers with a cache of their own and without
+@pytest.mark.parametrize('S,H,D,q_rank,rank,own', [
+    (1, 3, 20, 40, 24, True), (7, 8, 128, 512, 512, True), (16, 4, 64, 700, 300, False),
+    (17, 8, 128, 512, 100, True), (64, 16, 128, 256, 512, True), (128, 2, 32, 1000, 40, True),
+    (128, 16, 128, 512, 512, False)])
+def test_new_latents_and_queries_in_one_launch(S, H, D, q_rank, rank, own):
+  """The norms of the new latents and the queries' layer in one launch have the bits, outputs
+  and rings, of two; norm weights that lie between 16 bytes keep these."""
+  got = []
+  for shift in (0, 1):
+    lat = Latent(torch.bfloat16, H, D, D, q_rank, rank, 64, S, 4, 64, own=own, seed=S + H)
+    lat.ring.normal_(generator=torch.Generator('cuda').manual_seed(S))
+    w = torch.zeros((lat.qp + 4,), device='cuda')
+    w[shift:shift + q_rank] = dev(lat.w['dq.norm'])
+    lat.a.q_norm = w.data_ptr() + 4 * shift
+    lat.rs.seed(S)
+    outs = [lat.run([(i, at) for i in range(S)], [lat.sequence(1) for _ in range(S)])
+            for at in (0, 1)]
+    got.append(outs + [host(lat.ring)])
+  for a, b in zip(*got):
+    assert np.array_equal(a, b) and np.isfinite(a).all()
