@@ -423,11 +423,11 @@ class Transformer(DecodeContexts):
   # Batch slices ("lanes") that a fused beam search steps on separate streams.
   # A decode step is a chain of dependent kernels that leaves most of the
   # device waiting, so two half-batches side by side finish an iteration
-  # sooner than the whole batch in one chain (measured: base beam 4
-  # 0.789 -> 0.738 ms, XL int8 2.61 -> 2.46 ms; three lanes are slower
-  # again, and a fourth stream shares a hardware queue).  None: 2 lanes for a
-  # decode on its own, 1 when several batches are in flight (those fill the
-  # device better than lanes do, and streams that run side by side are few).
+  # sooner than the whole batch in one chain where the batch is large (see
+  # make_fused_beam_step); three lanes are slower again, and a fourth stream
+  # shares a hardware queue.  None: 2 lanes for a large decode on its own, 1
+  # when several batches are in flight (those fill the device better than
+  # lanes do, and streams that run side by side are few).
   decode_lanes = None
 
   def __init__(self, config: T5Config, device=None, scan_layers: bool = False):
