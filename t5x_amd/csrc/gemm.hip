@@ -1562,12 +1562,10 @@ extern "C" int t5d_norm_gemm(void* stream, int dtype, int w_dtype,
     return T5D_OK;
   }
   const int nj = (K / 64 + 3) / 4;  // k-tile pairs per wavefront
-  // One column tile while every workgroup has a CU to itself, else two, or four where
-  // that still fills the chip (more tiles share a normalisation); us for 1 / 2 / 4
-  // tiles, weights from memory: 64 x 1024 x 1024 (256 workgroups of 1) 4.38 / 4.84 /
-  // 5.74, 16 x 768 x 2304 (144) 3.85 / 4.21 / 5.06, 32 x 768 x 2304 (288) 4.69 / 4.24 /
-  // 5.08, 128 x 768 x 768 (384) 4.66 / 4.25 / 5.01, 64 x 1024 x 3072 (768; 192 of 4)
-  // 6.81 / 6.43 / 6.47, 128 x 1024 x 3072 (384 of 4) 10.46 / 8.68 / 7.88.
+  // One column tile while every workgroup has a CU to itself; what norm_dense_kernel leaves of
+  // the rest takes two (up to 512 inputs and twice as many workgroups as CUs) or four (columns
+  // beyond its 256 workgroups).  us for 1 / 2 / 4 tiles, weights from memory: 64 x 1024 x 1024
+  // (256 workgroups of 1) 4.38 / 4.84 / 5.74, 16 x 768 x 2304 (144) 3.85 / 4.21 / 5.06.
   // Beyond K = 1024 the fragments of fewer column tiles fit the registers (bfloat16
   // weights: one; int8: two, which no second workgroup joins on a CU, so only while
   // each has its own: K = 2048, int8, 32 x 2048 (256 of 1) 6.18 / 7.70, 64 x 2048 (256
@@ -1587,8 +1585,8 @@ extern "C" int t5d_norm_gemm(void* stream, int dtype, int w_dtype,
 #define T5D_NG_CASE(NT_, WT_)                                                 \
   if (nt == NT_) {                                                            \
     if (nj <= 2) T5D_NG_LAUNCH(NT_, 2, WT_);                                    \
-    else if (nj <= 3) T5D_NG_LAUNCH(NT_, 3, WT_);                               \
-    else if (nj <= 4) T5D_NG_LAUNCH(NT_, 4, WT_);                               \
+    else if (NT_ != 2 && nj <= 3) T5D_NG_LAUNCH(NT_ != 2 ? NT_ : 1, 3, WT_);    \
+    else if (NT_ != 2 && nj <= 4) T5D_NG_LAUNCH(NT_ != 2 ? NT_ : 1, 4, WT_);    \
   }
   if (w_dtype == T5D_BF16) {
     if (nj > 4) T5D_NG_LAUNCH(1, 8, bf16_t);
