@@ -388,9 +388,8 @@ norm_gemm_kernel(GemmArgs g) {
   }
   T5D_GATE_TEST();
 
-  // (in the order of norm_dense_kernel, whose lanes hold 4 columns in a row, and of a sum over
-  // its wavefront)
-  float part[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+  // (norm_dense_kernel adds in the same order)
+  float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     if (EXACT || wave + 4 * j < n_pairs) {
@@ -399,20 +398,15 @@ norm_gemm_kernel(GemmArgs g) {
         float f[8];
         unpack16(xa[j][hh].u, f);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) part[hh][e >> 2] = fmaf(f[e], f[e], part[hh][e >> 2]);
+        for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
       }
     }
   }
-  float ss[2];
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
-    ss[hh] = part[hh][0] + part[hh][1];
-    ss[hh] += dpp_move<kDppXor1>(ss[hh]);  // over the 4 pieces of the row
-    ss[hh] += dpp_move<kDppXor2>(ss[hh]);
-  }
-  if (gq == 0) s_ss[wave][n16] = ss[0] + ss[1];
+  ss += dpp_move<kDppXor1>(ss);  // over the 4 pieces of the row
+  ss += dpp_move<kDppXor2>(ss);
+  if (gq == 0) s_ss[wave][n16] = ss;
   __syncthreads();
-  const float tot = (s_ss[0][n16] + s_ss[1][n16]) + (s_ss[2][n16] + s_ss[3][n16]);
+  const float tot = (s_ss[0][n16] + s_ss[2][n16]) + (s_ss[1][n16] + s_ss[3][n16]);
   const float inv = 1.0f / sqrtf(tot / (float)g.K + g.eps);
 
   f32x4_v acc[NT];

@@ -17,28 +17,32 @@ namespace t5d {
 // to 0.9 us).  So columns are spread over as many CUs as there are, and no further: each
 // workgroup norms its rows anew.  us, weights from memory:
 //   norm in norm_gemm_kernel / here       rows 16       32            64            128
-//     768 x 2304                     3.89 / 4.07   4.30 / 4.12   5.21 / 4.65   6.50 / 5.60
-//     768 x 4096 gated               4.31 / 4.32   4.81 / 4.55   5.82 / 5.21   7.10 / 8.32
-//     1024 x 3072                    4.59 / 4.73   5.19 / 4.85   6.27 / 5.78   7.66 / 7.17
-//     1024 x 5632 gated              5.75 / 5.61   7.10 / 6.64   8.71 / 8.16  11.59 / 13.5
-//     512 x 5632 gated               4.04 / 4.19   4.80 / 4.30   5.80 / 5.36   6.77 / 6.90
-//     1024 x 5632 gated, int8        5.52 / 5.10   6.78 / 5.92   8.67 / 7.42  11.89 / 10.8
+//     768 x 2304                     3.90          4.34 / 4.04   5.31 / 4.55   6.61 / 5.41
+//     768 x 4096 gated               4.38          4.91 / 4.47   5.84 / 4.90   7.28
+//     1024 x 3072                    4.69          5.19 / 4.70   6.46 / 5.13   7.97 / 7.06
+//     1024 x 5632 gated              5.89 / 5.63   7.30 / 6.45   9.02 / 7.96  12.08
+//     512 x 5632 gated               4.09          4.88 / 4.27   5.92 / 5.25   7.21
+//     1024 x 5632 gated, int8        5.58 / 5.11   6.94 / 6.11   8.98 / 7.80  12.50
 //   float32 stream, two kernels / here
 //     512 x 3328                     6.04 / 5.01   6.44 / 5.10   6.98 / 5.62   7.90 / 6.70
 //     768 x 4096 gated               6.60 / 6.15   7.06 / 6.34   8.23 / 7.23   9.95 / 9.12
 //     1024 x 3328                    6.77 / 6.96   7.49 / 7.10   8.76 / 8.17  10.77 / 10.37
 //     1024 x 5632 gated              8.58 / 7.89   9.43 / 8.81  11.09 / 10.41  13.6 / 17.8
+// A row in the lanes' own groups of 4 columns, its norm through LDS and another barrier, was
+// slower than these pieces, each half a wavefront reading what the other does too (64 x 1024 x
+// 5632 8.46 / 7.96, 64 x 768 x 2304 4.65 / 4.55), and gave sums another order.
 // Tried and slower: 16 wavefronts (64 x 1024 x 5632 8.85), 4 (8.94), 32 rows per workgroup
 // with K over 8 wavefronts (8.67, 64 x 768 x 4096 6.70 instead of 5.36).
 template <typename Args, int NT, int KQ, typename WT>
 __global__ void __launch_bounds__(512)
 norm_dense_kernel(Args g) {
   constexpr bool kStream = IsStream<Args>::value, kLatent = IsLatent<Args>::value;
+  constexpr bool kPlain = !kStream && !kLatent;
   constexpr int LD = 256 * KQ, HS = LD + 8;  // row stride of the normed rows
   constexpr int TB = WeightTile<WT>::kTileBytes, TN = 32 * NT;
   __shared__ __align__(16) bf16_t s_h[16 * HS];
   __shared__ float red[8][NT * 4][64];
-  __shared__ __align__(16) float s_norm[kStream ? 2 : 1][LD];
+  __shared__ __align__(16) float s_norm[kStream ? 2 : 1][kPlain ? 4 : LD];
   T5D_GATE_READ(g.gate);
   if constexpr (kLatent) {
     if ((int)blockIdx.x >= g.dense_blocks) {  // a cached latent per wavefront
@@ -75,12 +79,14 @@ norm_dense_kernel(Args g) {
   const int K = g.K, KT = K >> 5, n_pairs = KT >> 1;
 
   // The norms' vectors (4 columns of one or of both per thread), two rows per wavefront in
-  // groups of 4 columns, the weights: in the order in which they are used.
+  // groups of 4 columns, the weights: in the order in which they are used.  (Plain rows: in
+  // the pieces that norm_gemm_kernel adds up, a row in lanes % 32 / 16, twice; lane l norms
+  // half l / 32 of each.)
   constexpr int PV = (LD / 4 + 511) / 512;
   float4 vec[PV], vec_y[kStream ? PV : 1];
   const int d = columns_of_norm(g);
 #pragma unroll
-  for (int v = 0; v < PV; ++v) {
+  for (int v = 0; !kPlain && v < PV; ++v) {
     const int c = 4 * (threadIdx.x + 512 * v);
     if constexpr (kStream) {
       vec_y[v] = g.y_norm != nullptr ? norm_column(g.y_norm, c, d)
@@ -88,21 +94,34 @@ norm_dense_kernel(Args g) {
       vec[v] = norm_column(g.norm, c, d);
     } else if constexpr (kLatent) {
       vec[v] = norm_column(g.norm, c, d);
-    } else {
-      uint2 q = make_uint2(0, 0);
-      if (c < d) q = *reinterpret_cast<const uint2*>(g.norm_scale + c);
-      vec[v] = make_float4(bf16lo_to_f32(q.x), bf16hi_to_f32(q.x), bf16lo_to_f32(q.y),
-                           bf16hi_to_f32(q.y));
     }
   }
   constexpr int KP8 = (KQ + 1) / 2;  // groups of 8 columns per lane
   uint4 x8[kLatent ? 2 : 1][KP8];
   const int have = kLatent ? (d_of_norm(g) + 15) & ~15 : 0;
   float4 x[kStream ? 2 : 1][KQ];
-  uint2 y[2][KQ];  // (not a stream: the rows themselves)
+  uint2 y[2][KQ];
   const bool add = has_branch(g);
+  const int p_row = 2 * wave + (lane >> 4 & 1), p_half = lane >> 5;
+  const int p_at = 64 * (lane >> 2 & 3) + 8 * (lane & 3);
+  uint4 xp[kPlain ? KQ : 1][2], sp[kPlain ? KQ : 1];
+  if constexpr (kPlain) {
+    const bf16_t* from = g.A + (size_t)min(m0 + p_row, g.M - 1) * K + p_at;
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
+    for (int j = 0; j < KQ; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        xp[j][h] = p_at + 256 * j < K
+                       ? *reinterpret_cast<const uint4*>(from + 256 * j + 32 * h)
+                       : make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < KQ; ++j)
+      sp[j] = p_at + 256 * j < K ? *reinterpret_cast<const uint4*>(g.norm_scale + p_at +
+                                                                   256 * j + 32 * p_half)
+                                 : make_uint4(0, 0, 0, 0);
+  }
+#pragma unroll
+  for (int r = 0; !kPlain && r < 2; ++r) {
     // (past the end: the last row, not stored)
     const size_t row = (size_t)min(m0 + 2 * wave + r, g.M - 1) * row_stride(g);
     if constexpr (kLatent) {
@@ -119,8 +138,6 @@ norm_dense_kernel(Args g) {
         x[r][q] = on ? *reinterpret_cast<const float4*>(g.x + row + c)
                      : make_float4(0.f, 0.f, 0.f, 0.f);
         if (on && add) y[r][q] = *reinterpret_cast<const uint2*>(g.y + row + c);
-      } else {
-        if (on) y[r][q] = *reinterpret_cast<const uint2*>(g.A + row + c);
       }
     }
   }
@@ -137,18 +154,20 @@ norm_dense_kernel(Args g) {
                  2 * min(part + 4 * j, n_pairs - 1) + h) * TB,
             lane);
   T5D_GATE_TEST();
+  if constexpr (!kPlain) {
 #pragma unroll
-  for (int v = 0; v < PV; ++v) {
-    const int c = 4 * (threadIdx.x + 512 * v);
-    if (c < LD) {
-      *reinterpret_cast<float4*>(&s_norm[0][c]) = vec[v];
-      if constexpr (kStream) *reinterpret_cast<float4*>(&s_norm[1][c]) = vec_y[v];
+    for (int v = 0; v < PV; ++v) {
+      const int c = 4 * (threadIdx.x + 512 * v);
+      if (c < LD) {
+        *reinterpret_cast<float4*>(&s_norm[0][c]) = vec[v];
+        if constexpr (kStream) *reinterpret_cast<float4*>(&s_norm[1][c]) = vec_y[v];
+      }
     }
+    // (what is requested may come later: no wait for it at the barriers)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   }
-  // (what is requested may come later: no wait for it at the barriers)
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 
   if constexpr (kStream) {
     // as stream_norm_kernel, whose 4 wavefronts hold columns 256 w + 1024 v of a row: one
@@ -238,34 +257,36 @@ norm_dense_kernel(Args g) {
             latent_normed(x8[r][q], inv[r], &s_norm[0][c]);
     }
   } else {
-    // (summed as norm_gemm_kernel does, so that a row has the same bits in both)
-    float inv[2];
+    // (summed as norm_gemm_kernel does, so that a row has the same bits in both: its wavefronts
+    // w are lanes % 16 / 4 here)
+    float ss = 0.f;
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      float ss = 0.f;
+    for (int j = 0; j < KQ; ++j)
 #pragma unroll
-      for (int q = 0; q < KQ; ++q) {
-        const float y0 = bf16lo_to_f32(y[r][q].x), y1 = bf16hi_to_f32(y[r][q].x);
-        const float y2 = bf16lo_to_f32(y[r][q].y), y3 = bf16hi_to_f32(y[r][q].y);
-        ss = fmaf(y0, y0, ss); ss = fmaf(y1, y1, ss);
-        ss = fmaf(y2, y2, ss); ss = fmaf(y3, y3, ss);
+      for (int h = 0; h < 2; ++h) {
+        float f[8];
+        unpack16(xp[j][h], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
       }
-      inv[r] = 1.0f / sqrtf(wave_sum(ss) / (float)K + g.eps);
-    }
+    ss += dpp_move<kDppXor1>(ss);
+    ss += dpp_move<kDppXor2>(ss);
+    ss += lane_xor8(ss);
+    ss += lane_xor4(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)K + g.eps);
 #pragma unroll
-    for (int q = 0; q < KQ; ++q) {
-      const int c = 4 * lane + 256 * q;
-      const float4 sf = *reinterpret_cast<const float4*>(&s_norm[0][c]);
+    for (int j = 0; j < KQ; ++j) {
+      float xf[8], sf[8];
+      unpack16(p_half ? xp[j][1] : xp[j][0], xf);
+      unpack16(sp[j], sf);
+      uint32_t o[4];
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const uint32_t a = pack_bf16x2(bf16lo_to_f32(y[r][q].x) * inv[r],
-                                       bf16hi_to_f32(y[r][q].x) * inv[r]);
-        const uint32_t b = pack_bf16x2(bf16lo_to_f32(y[r][q].y) * inv[r],
-                                       bf16hi_to_f32(y[r][q].y) * inv[r]);
-        *reinterpret_cast<uint2*>(s_h + (2 * wave + r) * HS + c) =
-            make_uint2(pack_bf16x2(bf16lo_to_f32(a) * sf.x, bf16hi_to_f32(a) * sf.y),
-                       pack_bf16x2(bf16lo_to_f32(b) * sf.z, bf16hi_to_f32(b) * sf.w));
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t n = pack_bf16x2(xf[2 * e] * inv, xf[2 * e + 1] * inv);
+        o[e] = pack_bf16x2(bf16lo_to_f32(n) * sf[2 * e], bf16hi_to_f32(n) * sf[2 * e + 1]);
       }
+      *reinterpret_cast<uint4*>(s_h + p_row * HS + p_at + 256 * j + 32 * p_half) =
+          make_uint4(o[0], o[1], o[2], o[3]);
     }
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

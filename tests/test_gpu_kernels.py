@@ -1562,6 +1562,49 @@ def test_norm_in_front_of_many_columns(ops, M, K, N, kind, int8):
   assert bool((err <= 2e-2 + 2.0**-6 * two.abs()).all())
 
 
+# norm_gemm_kernel: one, two and four column tiles, 64 to 2048 inputs; norm_dense_kernel: one to
+# four of each half, its three widths full and not
+@pytest.mark.parametrize('M,K,N', [
+    (16, 64, 64), (16, 768, 2304), (33, 448, 4112), (128, 1024, 5632), (64, 2048, 2048),
+    (33, 192, 5648), (128, 512, 4096), (64, 512, 5632), (48, 704, 3088), (64, 768, 2304),
+    (128, 768, 2304), (17, 832, 4112), (64, 1024, 5632)])
+def test_norm_in_front_of_a_layer_adds_squares_in_its_order(ops, M, K, N):
+  """The normed rows, through a layer that hands them on as they are, have the bits of the
+  order of sums that the kernels promise: 16 sums of pieces of 8 columns (k-tile pairs w, w +
+  4, .., piece g of each k-tile), over g in pairs, over w as (0 + 2) + (1 + 3).  Rows in which
+  one large value swallows what its own sum adds behind it, and of these such as the exact
+  sum rounds elsewhere, so that another order shows."""
+  rs = np.random.RandomState(M + K + N)
+  bf16 = lambda a: torch.as_tensor(a).to(torch.bfloat16)
+  n = 2**22 // K
+  rows = rs.uniform(0.6, 0.98, (n, K)).astype(np.float32)
+  rows[np.arange(n), rs.randint(0, K, n)] = 4096.0
+  rows[:, rs.randint(0, K, 5)] = rs.uniform(200, 2000, (n, 5))
+  x, scale = bf16(rows), bf16((1 + 0.1 * rs.randn(K)).astype(np.float32))
+  f = x.float().numpy()
+  part = np.zeros((n, 4, 4), np.float32)
+  for pair in range(K // 64):
+    piece = f[:, 64 * pair:64 * pair + 64].reshape(n, 2, 4, 8)
+    for half in range(2):
+      for e in range(8):  # (a square of a bfloat16 value is exact in float32)
+        part[:, pair % 4] += piece[:, half, :, e] * piece[:, half, :, e]
+  w = (part[..., 0] + part[..., 1]) + (part[..., 2] + part[..., 3])
+
+  def norms(total):
+    inv = np.float32(1) / np.sqrt(total / np.float32(K) + np.float32(1e-6))
+    return bf16(bf16(f * inv[:, None]).float() * scale.float()).float().numpy()
+
+  normed = norms((w[:, 0] + w[:, 2]) + (w[:, 1] + w[:, 3]))
+  telling = (normed != norms(np.square(f, dtype=np.float64).sum(1).astype(np.float32))).any(1)
+  pick = np.resize(np.flatnonzero(telling), M)
+  x, normed = x[pick], normed[pick]
+  kernel = np.zeros((K, N), np.float32)
+  kernel[np.arange(N) % K, np.arange(N)] = 1.0
+  pw = ops.pack_weight(dev(kernel), torch.bfloat16, torch.bfloat16)
+  got = ops.gemm(x.cuda(), pw, norm_scale=scale.cuda(), out_dtype=torch.float32)
+  assert np.array_equal(host(got), normed[:, np.arange(N) % K])
+
+
 def test_cross_attention_random_shapes(ops):
   """t5d_cross_attention_step (bfloat16) over 40 random shapes — batch 1..48,
   1 / 2 / 4 / 8 beams, 1..16 heads, encoder length a multiple of 32 up to
