@@ -869,6 +869,7 @@ class BeamLoop(_InFlight):
     self.start(check_every)
     while not self.poll(block=True):
       pass
+    self.fused.synchronize()  # (lanes level, cur_index and keep_going written)
 
   def advance(self, n: int):
     """n loop iterations without looking at the condition in between (with the

@@ -1279,6 +1279,7 @@ class FusedBeamStep(_OwnedContext):
     self.lane_words = torch.zeros((2, n), dtype=torch.int32, device=dev)
     self.lane_records = torch.zeros((n, S + 1), dtype=torch.int32, device=dev)
     self._enqueued = 0  # iterations since the loop was bound
+    self._last_chunk = None  # the last launch_chunk's ticket
     # What the captured graphs hold addresses of, beyond the lanes' own
     # buffers: the loop's state.  A later loop is re-bound onto these.
     self.w, self.cross = w, cross
@@ -1349,7 +1350,7 @@ class FusedBeamStep(_OwnedContext):
       with torch.cuda.stream(first):
         self.lane_words.copy_(self.flag.expand_as(self.lane_words))
         self.lane_records.zero_()
-    self._enqueued = 0
+    self._enqueued, self._last_chunk = 0, None
     first.synchronize()
 
   def _enqueue(self, lane):
@@ -1447,14 +1448,19 @@ class FusedBeamStep(_OwnedContext):
 
   def launch_chunk(self, n):
     """launch(n), and a ticket for chunk_running(); None once as many
-    iterations are enqueued as the loop can have."""
-    if self._enqueued >= self.loop.max_decode_len - 1:
+    iterations are enqueued as the loop can have and no lane is known to have
+    left some of them out."""
+    if self._enqueued >= self.loop.max_decode_len - 1 and not (
+        self._last_chunk and self.chunk_running(self._last_chunk)):
       return None
     self.launch(n)
     if self.n_lanes == 1:
-      return [self._end_chunk(self.flag, self.lanes[0].stream)]
-    return [self._end_chunk(self.lane_words[1, i], lane.stream)
-            for i, lane in enumerate(self.lanes)]
+      ticket = [self._end_chunk(self.flag, self.lanes[0].stream)]
+    else:
+      ticket = [self._end_chunk(self.lane_words[1, i], lane.stream)
+                for i, lane in enumerate(self.lanes)]
+    self._last_chunk = ticket
+    return ticket
 
   def chunk_running(self, ticket, block=False):
     """Whether the loop condition still held after that chunk; None while the

@@ -495,6 +495,49 @@ def test_lanes_that_run_far_apart_make_the_loops_iterations(lanes, order, seed,
   assert torch.equal(torch.as_tensor(gs), torch.as_tensor(ws))
 
 
+@pytest.mark.parametrize('lanes', [1, 2, 3])
+@pytest.mark.parametrize('seed,eos_bias', [(11, 6.0), (12, 3.0), (13, 2.0), (14, 0.0)])
+@pytest.mark.parametrize('polled', [False, True])
+def test_run_ends_at_the_loops_end(monkeypatch, lanes, seed, eos_bias, polled):
+  """After run(), and after start() and poll(), every lane has made all of the loop's
+  iterations, also where a lane ran ahead of the others in every chunk and left some out; after
+  run() the loop's state is the whole of it, counter and flag too."""
+  from t5x_amd import decoding
+  B, K, L = 4, 4, 40
+  module, fn = _decode_setup('bfloat16', B, K, 16, L, seed=seed, eos_bias=eos_bias)
+  module.decode_lanes = lanes
+  inputs = np.zeros((B, L), np.int32)
+  plain = decoding.BeamLoop(inputs, dict(module.init_cache(B, L)), fn, eos_id=1,
+                            num_decodes=K)
+  plain.run()
+  for order in (list(range(lanes)), list(range(lanes))[::-1]):
+    loop = decoding.BeamLoop(inputs, module.init_cache(B, L), fn, eos_id=1,
+                             num_decodes=K)
+    step = loop.fused
+
+    def launch(n):
+      step._enqueued += n
+      for i in order:
+        step._launch_lane(step.lanes[i], n)
+        step.lanes[i].stream.synchronize()
+
+    monkeypatch.setattr(step, 'launch', launch)
+    if polled:
+      loop.start(check_every=4)
+      while not loop.poll(block=True):
+        pass
+    else:
+      loop.run()
+      assert int(loop.keep_going.item()) == 0
+    torch.cuda.synchronize()
+    steps = int(plain.cur.cur_index.item())
+    assert step.lane_cur_index.tolist() == [steps] * lanes
+    for name in ('live_logprobs', 'finished_scores', 'live_seqs', 'finished_seqs',
+                 'finished_flags') + (() if polled else ('cur_index',)):
+      assert torch.equal(getattr(loop.cur, name), getattr(plain.cur, name)), name
+    loop.finish()
+
+
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
 def test_fused_loop_context_is_reused_across_batches(dtype):
   """A second (and third) batch of the same shape on the same module re-binds
