@@ -952,8 +952,9 @@ typedef struct {
   void* workspace;         /* t5d_recurrence_workspace_bytes(...), 16-aligned */
   int64_t workspace_bytes;
   /* NULL: low is given.  Otherwise the call forms it: low [M, low_n] = columns off_low ..
-   * off_low + low_k of proj times low_w [low_k, low_n] (packed as t5d_dense takes it); where
-   * a step's kernel does that itself, low is not written. */
+   * off_low + low_k of proj times low_w [low_k, low_n] (packed as t5d_dense takes it, and
+   * with its limits; off_z + H D and, of a low-rank gate, off_low_gate + H Dv are at most
+   * low_n); where a step's kernel does that itself, low is not written. */
   const void* low_w;
   int off_low, low_k, low_n;
 } t5d_recurrence;

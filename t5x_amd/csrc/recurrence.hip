@@ -1337,7 +1337,10 @@ static bool low_rides(const t5d_recurrence& a, int64_t rows) {
          a.taps <= 4 && (a.low_k == 64 || a.low_k == 128) && a.off_z % 16 == 0 &&
          (a.gate != T5D_GATE_SIGMOID_LOW || a.off_low_gate % 16 == 0) &&
          a.off_low % 8 == 0 && a.ld_proj % 8 == 0 &&
-         ((uintptr_t)a.proj | (uintptr_t)a.low_w) % 16 == 0 && rows * a.H <= 4096;
+         // (what t5d_dense refuses is left for it to refuse)
+         a.low_n % 16 == 0 && a.ld_low >= a.low_n &&
+         ((uintptr_t)a.proj | (uintptr_t)a.low_w | (uintptr_t)a.low) % 16 == 0 &&
+         rows * a.H <= 4096;
 }
 
 template <bool DELTA, typename T>
@@ -1512,6 +1515,18 @@ extern "C" int t5d_recurrence_run(void* stream, const t5d_recurrence* a,
               b->max_len);
   T5D_REQUIRE(variant >= 0 && variant <= 3, T5D_EINVAL,
               "t5d_recurrence_run: variant %d", variant);
+  if (a->low_w != nullptr) {  // the columns that are read, of those that it has
+    const int64_t z = a->off_z + (int64_t)a->H * a->D,
+                  gate = a->off_low_gate + (int64_t)a->H * a->Dv;
+    T5D_REQUIRE(a->off_low >= 0 && a->low_k > 0 &&
+                    (int64_t)a->off_low + a->low_k <= a->ld_proj && a->off_z >= 0 &&
+                    z <= a->low_n && (a->gate != T5D_GATE_SIGMOID_LOW ||
+                                      (a->off_low_gate >= 0 && gate <= a->low_n)),
+                T5D_EINVAL,
+                "t5d_recurrence_run: low-rank inputs %d + %d of %d, columns from %d and %d "
+                "of %d", a->off_low, a->low_k, a->ld_proj, a->off_z, a->off_low_gate,
+                a->low_n);
+  }
   RecArgs g;
   g.a = *a; g.b = *b; g.gate = tls_gate;
   g.C = 2 * a->G * a->D + a->H * a->Dv;

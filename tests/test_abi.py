@@ -120,6 +120,41 @@ def test_where_the_row_kernel_and_the_layer_behind_it_go_in_one_launch(M, ld, N,
   assert _lib.load().t5d_stream_dense_pays(M, ld, N) == one
 
 
+# (float32 rows may lie anywhere, with any number of columns)
+_BOTH = [dict(low_n=528), dict(off_z=320), dict(off_z=-16), dict(off_low_gate=320),
+         dict(off_low_gate=-16), dict(off_low=1736), dict(off_low=-8), dict(low_k=0),
+         dict(ld_low=304)]
+_BF16 = [dict(low=8), dict(low_w=8), dict(low_n=558, ld_low=560)]
+
+
+@pytest.mark.parametrize('dtype,wrong', [(_lib.F32, w) for w in _BOTH] +
+                         [(_lib.BF16, w) for w in _BOTH + _BF16])
+@pytest.mark.parametrize('rows', [1, 40])
+def test_low_rank_columns_that_are_not_there_without_gpu(rows, dtype, wrong):
+  """t5d_recurrence_run with low_w refuses sizes beyond its columns and what t5d_dense
+  refuses, whichever of them would form the columns."""
+  r = _lib.Recurrence()
+  r.dtype, r.H, r.G, r.D, r.Dv = dtype, 4, 4, 64, 64
+  r.delta = r.decay = r.unit = r.gate = 1
+  for name in ('proj', 'low', 'decay_bias', 'A_log', 'norm', 'state', 'out', 'workspace',
+               'low_w'):
+    setattr(r, name, 4096)
+  r.ld_proj, r.ld_out, r.workspace_bytes = 1664, 256, 1 << 40
+  r.off_q, r.off_k, r.off_v, r.off_beta, r.off_gate = 0, 256, 512, 768, 1024
+  r.off_low, r.low_k, r.low_n, r.ld_low = 1536, 128, 560, 560
+  r.off_z, r.off_low_gate = 16, 288
+  for name, value in wrong.items():
+    setattr(r, name, value)
+  b = _lib.Ragged()
+  b.M = b.max_len = rows
+  b.S = 1
+  for name in ('tokens', 'tok_pos', 'tok_seq', 'seq_off', 'seq_start', 'seq_slot'):
+    setattr(b, name, 4096)
+  lib = _lib.load()
+  assert lib.t5d_recurrence_run(None, ctypes.byref(r), ctypes.byref(b), 0) == -1
+  assert b'low-rank' in lib.t5d_last_error() or b't5d_dense' in lib.t5d_last_error()
+
+
 def test_many_row_tile_choice_without_gpu():
   """t5d_gemm_rows_tile: which workgroup tile the many-row dense kernel runs a
   shape on (1: 128 columns, 2: 256, 3: 192, each of 128 rows, or 1 of 64), by what
