@@ -392,9 +392,7 @@ static int tile_splits(const t5d_latent_attention& a, const t5d_ragged& b) {
 // 128 rows.
 static bool new_latents_and_queries(hipStream_t s, const LatentArgs& g, int QN) {
   const t5d_latent_attention& a = g.a;
-  if (((uintptr_t)a.uq | (uintptr_t)a.q_norm | (uintptr_t)a.kv_norm) % 16 != 0 ||
-      QN % 16 != 0)
-    return false;
+  if (((uintptr_t)a.q_norm | (uintptr_t)a.kv_norm) % 16 != 0 || QN % 16 != 0) return false;
   LatentDenseArgs d = {};
   d.A = reinterpret_cast<const bf16_t*>(a.proj) + a.off_q; d.lda = a.ld_proj;
   d.W = a.uq; d.C = a.q; d.M = g.b.M; d.K = g.QP; d.N = QN;
@@ -469,7 +467,8 @@ extern "C" int t5d_latent_attention_run(void* stream, const t5d_latent_attention
   const bool bf16 = a->dtype == T5D_BF16;
   T5D_REQUIRE((((uintptr_t)a->proj | (uintptr_t)a->cq | (uintptr_t)a->latent_ring |
                 (uintptr_t)a->lat | (uintptr_t)a->kv | (uintptr_t)a->ql |
-                (uintptr_t)a->ol) % 16) == 0 &&
+                (uintptr_t)a->ol |
+                (bf16 ? (uintptr_t)a->uq | (uintptr_t)a->q : 0)) % 16) == 0 &&
                   ((a->ld_proj | a->off_q | (a->off_kv < 0 ? 0 : a->off_kv)) & 7) == 0,
               T5D_EINVAL, "t5d_latent_attention_run: operand alignment");
   g.splits = 1; g.parts = (float*)a->workspace;

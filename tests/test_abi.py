@@ -155,6 +155,27 @@ def test_low_rank_columns_that_are_not_there_without_gpu(rows, dtype, wrong):
   assert b'low-rank' in lib.t5d_last_error() or b't5d_dense' in lib.t5d_last_error()
 
 
+@pytest.mark.parametrize('name', ['proj', 'cq', 'q', 'uq', 'ql', 'ol', 'latent_ring'])
+@pytest.mark.parametrize('rows', [1, 200])
+def test_latent_operands_off_16_bytes_without_gpu(rows, name):
+  """t5d_latent_attention_run refuses them before it launches anything, whether the queries'
+  layer goes alone or with the latents' norms."""
+  a = _lib.LatentAttention()
+  a.dtype, a.H, a.D, a.Dv, a.rank, a.q_rank = _lib.BF16, 4, 64, 64, 128, 256
+  a.ring, a.ld_proj, a.off_q, a.off_kv, a.ld_out = 256, 512, 0, 256, 256
+  for p in ('proj', 'q_norm', 'kv_norm', 'uq', 'absorb', 'expand', 'latent_ring', 'cq', 'q',
+            'ql', 'ol', 'out'):
+    setattr(a, p, 4096 + 8 * (p == name))
+  b = _lib.Ragged()
+  b.M = b.max_len = rows
+  b.S = 1
+  for p in ('tokens', 'tok_pos', 'tok_seq', 'seq_off', 'seq_start', 'seq_slot'):
+    setattr(b, p, 4096)
+  lib = _lib.load()
+  assert lib.t5d_latent_attention_run(None, ctypes.byref(a), ctypes.byref(b), 0) == -1
+  assert b'operand alignment' in lib.t5d_last_error()
+
+
 def test_many_row_tile_choice_without_gpu():
   """t5d_gemm_rows_tile: which workgroup tile the many-row dense kernel runs a
   shape on (1: 128 columns, 2: 256, 3: 192, each of 128 rows, or 1 of 64), by what
