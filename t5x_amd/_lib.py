@@ -207,8 +207,6 @@ _SIGNATURES = {
     't5d_stream_dense_pays': (c_int, [c_int] * 3),
     't5d_stream_dense': (c_int, [_P] * 6 + [c_int, c_float, _P, c_int, _P] +
                          [c_int] * 6 + [c_float] * 3),
-    't5d_grouped_tile_rows': (c_int, [c_int] * 3),
-    't5d_grouped_dense_run': (c_int, [_P, POINTER(GroupedDense)]),
     't5d_stream_rows_dense_rows': (c_int, [c_int] * 2),
     't5d_stream_rows_dense_pays': (c_int, [c_int] * 3),
     't5d_stream_rows_dense': (c_int, [_P] * 6 + [c_int, c_float, _P, c_int, _P] +

@@ -38,6 +38,12 @@ def test_binding_covers_every_declared_symbol():
   assert set(declared_names()) == set(_lib.exported_names())
 
 
+def test_binding_names_each_symbol_once():
+  text = open(os.path.join(ROOT, 't5x_amd', '_lib.py')).read()
+  names = re.findall(r"^    '(t5d_[a-z0-9_]+)': \(", text, flags=re.M)
+  assert set(names) == set(_lib._SIGNATURES) and len(names) == len(set(names))
+
+
 def test_measurement_aids_stay_out_of_the_boundary():
   """The work-skipping switch bench.py uses lives in its own header and entry
   point; the boundary's structs and declarations carry none."""
