@@ -1565,7 +1565,7 @@ extern "C" int t5d_norm_gemm(void* stream, int dtype, int w_dtype,
   // each has its own: K = 2048, int8, 32 x 2048 (256 of 1) 6.18 / 7.70, 64 x 2048 (256
   // of 2) 8.08 / 7.73, 32 x 6144 (384 of 2) 11.9 / 14.8, 16 x 6144 (192) 8.89 / 8.80).
   const int tiles = n_tiles * g.m_parts;
-  int nt = tiles <= 256 ? 1 : ((n_tiles / 4) * g.m_parts >= 256 ? 4 : 2);
+  int nt = tiles <= 256 ? 1 : nj <= 2 && (n_tiles / 4) * g.m_parts < 256 ? 2 : 4;
   if (nj > 4) nt = w_dtype == T5D_I8 && tiles > 256 && tiles <= 512 ? 2 : 1;
   const int n_groups = (n_tiles + nt - 1) / nt;
   dim3 grid((n_groups + 7) / 8 * 8 * g.m_parts), block(256);

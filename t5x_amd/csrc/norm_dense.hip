@@ -362,7 +362,8 @@ static void launch(int nt, Args g, hipStream_t s) {
   if (nt == 1) T5D_ND(1);
   else if (nt == 2) T5D_ND(2);
   else if (nt == 3) T5D_ND(3);
-  else T5D_ND(4);
+  else if constexpr (IsStream<Args>::value) T5D_ND(4);
+  else T5D_ND_K(4, 2);  // (launch_norm_dense: 4 tiles up to 512 inputs)
 #undef T5D_ND
 #undef T5D_ND_K
 }
