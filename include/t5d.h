@@ -636,10 +636,6 @@ typedef struct {
   void* kv_base;               /* first cache tensor [B, K, H, 64, L] */
   int64_t kv_tensor_stride_bytes;
   int n_kv_tensors;            /* 2 * NL when all layers share one block */
-  /* non-zero: *keep_going is only read (as the gate); the caller runs
-   * t5d_beam_cond itself, e.g. once over all slices of a batch that it steps
-   * on separate streams */
-  int skip_cond;
   /* optional, all three or none, [B, K] each: where the beams' cache rows
    * live.  cache_slot[b, e] = slot of beam e (identity before the first
    * iteration; updated in place).  Every iteration writes, for the next reader
@@ -659,7 +655,7 @@ typedef struct {
    * lane_records [n_lanes, S + 1], zeros before the first iteration.  An enqueued iteration
    * leaves everything as it is where the slice is done or must know first what another one,
    * not as far yet, says of this iteration (keep_going 0, lane_alive 1): enqueue further
-   * ones until lane_alive is 0.  skip_cond is not looked at. */
+   * ones until lane_alive is 0. */
   int n_lanes, lane;
   int32_t *lane_alive, *lane_records;
 } t5d_beam_step;

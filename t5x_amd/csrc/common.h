@@ -318,12 +318,11 @@ int launch_beam_select(hipStream_t s, const float* logits,
                        int32_t* cache_dst);
 // End of a beam-search iteration in one single-workgroup kernel: advance
 // *state.cur_index, add 1 to `counters[0..n_counters)` (the layers' cache
-// indices), and, if do_cond, evaluate the loop condition into *keep_going.
+// indices), and evaluate the loop condition into *keep_going.
 int launch_beam_tail(hipStream_t s, const t5d_beam_state* state, int B, int K,
                      int S, float min_brevity, float min_log_prob,
                      int max_decode_step, int min_initial_index,
-                     int32_t* keep_going, int do_cond, int32_t* counters,
-                     int n_counters);
+                     int32_t* keep_going, int32_t* counters, int n_counters);
 
 // The same for one lane of a batch whose lanes do not wait for each other (n_lanes > 1).
 int launch_beam_lane_tail(hipStream_t s, const t5d_beam_step* b, int B, int K,

@@ -765,7 +765,7 @@ __global__ void __launch_bounds__(256)
 beam_cond_kernel(t5d_beam_state st, int B, int K, int S, float min_brevity,
                  float min_log_prob, int max_decode_step, int min_initial_index,
                  int32_t* keep_going, const int32_t* gate, int advance,
-                 int do_cond, int32_t* counters, int n_counters) {
+                 int32_t* counters, int n_counters) {
   __shared__ int iscratch[4];
   T5D_GATED(gate);
   // advance: this launch also ends the iteration (cur_index and the layers'
@@ -776,7 +776,6 @@ beam_cond_kernel(t5d_beam_state st, int B, int K, int S, float min_brevity,
     if (threadIdx.x == 0) *st.cur_index = cur;
     if ((int)threadIdx.x < n_counters) counters[threadIdx.x] += 1;
   }
-  if (!do_cond) return;
   int not_terminated, passes_min;
   count_open(st, B, K, min_brevity, min_log_prob, &not_terminated, &passes_min);
   not_terminated = block_sum_i32(not_terminated, iscratch);
@@ -1921,7 +1920,7 @@ extern "C" int t5d_beam_cond(void* stream, const t5d_beam_state* state, int B,
   hipLaunchKernelGGL(beam_cond_kernel, dim3(1), dim3(256), 0,
                      as_stream(stream), *state, B, K, S, min_brevity,
                      min_log_prob, max_decode_step, min_initial_index,
-                     keep_going, tls_gate, 0, 1, nullptr, 0);
+                     keep_going, tls_gate, 0, nullptr, 0);
   T5D_CHECK_LAUNCH("t5d_beam_cond");
   return T5D_OK;
 }
@@ -1962,19 +1961,19 @@ int t5d::launch_beam_select(hipStream_t s, const float* logits,
 int t5d::launch_beam_tail(hipStream_t s, const t5d_beam_state* state, int B,
                           int K, int S, float min_brevity, float min_log_prob,
                           int max_decode_step, int min_initial_index,
-                          int32_t* keep_going, int do_cond, int32_t* counters,
+                          int32_t* keep_going, int32_t* counters,
                           int n_counters) {
   int rc = check_state("beam tail", state);
   if (rc) return rc;
-  T5D_REQUIRE((keep_going || !do_cond) && B > 0 && K > 0 && S > 1 &&
+  T5D_REQUIRE(keep_going && B > 0 && K > 0 && S > 1 &&
                   n_counters >= 0 && n_counters <= 256 &&
                   (counters || n_counters == 0),
               T5D_EINVAL, "beam tail: B=%d K=%d S=%d counters=%d", B, K, S,
               n_counters);
   hipLaunchKernelGGL(beam_cond_kernel, dim3(1), dim3(256), 0, s, *state, B, K,
                      S, min_brevity, min_log_prob, max_decode_step,
-                     min_initial_index, keep_going, tls_gate, 1, do_cond,
-                     counters, n_counters);
+                     min_initial_index, keep_going, tls_gate, 1, counters,
+                     n_counters);
   T5D_CHECK_LAUNCH("beam tail");
   return T5D_OK;
 }

@@ -237,8 +237,8 @@ extern "C" int t5d_beam_search_step(void* stream, const t5d_model_step* m,
     return launch_beam_lane_tail(hs, b, B, K, m->cache_index, m->NL);
   T5D_TRY(launch_beam_tail(hs, &b->state, B, K, b->S, b->min_brevity,
                            b->min_log_prob, b->max_decode_step,
-                           b->min_initial_index, b->keep_going, !b->skip_cond,
-                           m->cache_index, m->NL));
+                           b->min_initial_index, b->keep_going, m->cache_index,
+                           m->NL));
   return T5D_OK;
 }
 
