@@ -751,9 +751,13 @@ class Transformer(DecodeContexts):
       return None
     w = self.decoder_weights(params)
     # Two lanes where their kernels are long enough for the overlap to make up
-    # for twice as many of them: ms with one / two, 64 tokens, 32 x 4 rows of
-    # small 22.0 / 22.5, 16 x 4 of base 35.7 / 37.0 and of large 80.4 / 85.5,
-    # 22 x 4 of base 40.2 / 38.4, 8 x 4 of xl (int8) 105 / 117, 16 x 4 136.6 / 136.7.
+    # for twice as many of them.  ms with one / two, 64 iterations, bfloat16
+    # (xl: int8), on either side of the line: small 128 rows 22.1 / 23.2, 132
+    # 30.6 / 23.4; base 80 37.5 / 38.1, 84 39.2 / 39.1, 88 40.4 / 38.8; large 64
+    # 80.4 / 80.8, 68 86.6 / 83.3; xl 32 104.8 / 110.9, 36 120.6 / 116.0.  Beyond
+    # it up to 128 rows: base 43.9 / 40.4, large 102.3 / 94.2, xl 215.2 / 185.9;
+    # in float32 less (base 84 rows 121.0 / 118.8, 128 160.9 / 154.4, large 84
+    # 341 / 316, xl 48 640 / 649, 64 777 / 762).
     wide = loop.batch_size * loop.beam_size * self.config.emb_dim > 65536
     lanes = self.decode_lanes or (
         2 if wide and not in_flight and self.streams_side_by_side() >= 2 else 1)
@@ -1206,6 +1210,7 @@ class _BeamLane:
           P(self.cache_slot), P(self.cache_src), P(self.cache_dst))
     self.beam = bs
     self.stream = module.decode_stream(owner.slot * owner.n_lanes + index)
+    self.event = torch.cuda.Event()
     self.graph = None
     self.graph_long = None
 
@@ -1225,7 +1230,8 @@ class FusedBeamStep(_OwnedContext):
   after the end, or while a lane has to know first what one behind it says,
   change nothing, so the host may look only every few iterations.  (Streams
   that joined after every iteration for one kernel that evaluated the
-  condition, base beam 4, 32 texts, 128 iterations: 89.4 ms; so: 83.2.)"""
+  condition, base beam 4, 32 texts, 128 iterations: 90.6 ms; so: 83.2.)  Every
+  GRAPH_STEPS iterations the lanes meet (_meet)."""
 
   def __init__(self, module, loop, params, encoded, enc_tokens, lanes=None,
                slot=0):
@@ -1444,7 +1450,23 @@ class FusedBeamStep(_OwnedContext):
       k = min(n, self.GRAPH_STEPS)
       for lane in self.lanes:
         self._launch_lane(lane, k)
+      self._meet()
       n -= k
+
+  def _meet(self):
+    """What is enqueued from here on waits for all lanes.  Lanes that keep
+    drifting apart no longer read the same weights at about the same time, and
+    memory has to give them twice.  ms of 128 iterations, two lanes that meet
+    never / after every 8 / 4 / 1: xl 32 x 4 rows 401.9 / 370.6 / 369.6 / 370.2,
+    in int8 16 x 4 268.7 / 252.9 / 253.2 / 253.7, large 32 x 4 194.4 / 186.6 /
+    187.6 / 189.8, base 32 x 4 84.1 / 83.1 / 83.2 / 84.9."""
+    for lane in self.lanes:
+      if self.n_lanes > 1:
+        lane.event.record(lane.stream)
+    for lane in self.lanes:
+      for other in self.lanes:
+        if other is not lane:
+          lane.stream.wait_event(other.event)
 
   def launch_chunk(self, n):
     """launch(n), and a ticket for chunk_running(); None once as many

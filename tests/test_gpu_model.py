@@ -538,6 +538,31 @@ def test_run_ends_at_the_loops_end(monkeypatch, lanes, seed, eos_bias, polled):
     loop.finish()
 
 
+@pytest.mark.parametrize('slow', [0, 1])
+def test_lanes_meet_every_few_iterations(slow):
+  """A lane whose stream is held up is not left behind by more iterations than a graph has
+  (lanes that are further apart read their weights twice)."""
+  from t5x_amd import decoding
+  B, K, L = 4, 4, 40
+  module, fn = _decode_setup('bfloat16', B, K, 16, L, seed=14)
+  module.decode_lanes = 2
+  loop = decoding.BeamLoop(np.zeros((B, L), np.int32), module.init_cache(B, L), fn,
+                           eos_id=1, num_decodes=K)
+  step = loop.fused
+  seen = torch.zeros((5,), dtype=torch.int32, device='cuda')
+  torch.cuda.synchronize()
+  with torch.cuda.stream(step.lanes[slow].stream):
+    torch.cuda._sleep(20000000)
+  for i in range(5):
+    loop.advance(step.GRAPH_STEPS)
+    with torch.cuda.stream(step.lanes[1 - slow].stream):
+      seen[i:i + 1].copy_(step.lane_cur_index[slow:slow + 1])
+  step.synchronize()
+  assert (seen.cpu().numpy() >= step.GRAPH_STEPS * np.arange(1, 6)).all()
+  assert step.lane_cur_index.tolist() == [5 * step.GRAPH_STEPS] * 2
+  loop.finish()
+
+
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
 def test_fused_loop_context_is_reused_across_batches(dtype):
   """A second (and third) batch of the same shape on the same module re-binds
