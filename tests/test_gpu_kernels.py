@@ -1519,8 +1519,9 @@ def test_norm_gemm_random_shapes(ops):
 @pytest.mark.parametrize('N', [16, 528, 2064])
 @pytest.mark.parametrize('int8', [False, True])
 def test_norm_gemm_does_not_depend_on_its_tiles(ops, K, N, int8):
-  """Every row's result is the same whichever tile it falls into: 128 rows (four or
-  two column tiles per workgroup), 33 of them and single rows (one), bit for bit."""
+  """Every row's result is the same whichever tile it falls into: 128 rows (norm_dense_kernel
+  where there are columns enough, else two column tiles per workgroup), 33 of them and single
+  rows (one), bit for bit."""
   rs = np.random.RandomState(K + N)
   x = dev(rs.randn(128, K).astype(np.float32), torch.bfloat16)
   scale = dev((1 + 0.1 * rs.randn(K)).astype(np.float32), torch.bfloat16)
@@ -1541,21 +1542,26 @@ def test_norm_gemm_does_not_depend_on_its_tiles(ops, K, N, int8):
     (64, 1024, 5632, 'geglu'), (81, 832, 3072, 'plain')])
 @pytest.mark.parametrize('int8', [False, True])
 def test_norm_in_front_of_many_columns(ops, M, K, N, kind, int8):
-  """Rows normed once for many columns have the bits of 16 rows at a time, whose columns
-  are few enough for the other kernel, and they are the layer's over normed rows."""
+  """Rows normed once for many columns have the bits of the other kernel, which 4 rows at a
+  time by at most 4096 columns go to (its rule leaves it 256 column tiles, 512 up to 512
+  inputs), and they are the layer's over normed rows."""
   rs = np.random.RandomState(M + K + N)
   x = dev(rs.randn(M, K).astype(np.float32), torch.bfloat16)
   scale = dev((1 + 0.1 * rs.randn(K)).astype(np.float32), torch.bfloat16)
   kernel = lambda n: dev((rs.randn(K, n) / np.sqrt(K)).astype(np.float32))
   wdt = torch.int8 if int8 else torch.bfloat16
-  if kind == 'geglu':
-    pw = ops.pack_weight(kernel(N // 2), torch.bfloat16, wdt, gate_kernel=kernel(N // 2))
-  else:
-    pw = ops.pack_weight(kernel(N), torch.bfloat16, wdt)
+  w, gate = ((kernel(N // 2), kernel(N // 2)) if kind == 'geglu' else (kernel(N), None))
+  pack = lambda part: ops.pack_weight(
+      w[:, part].contiguous(), torch.bfloat16, wdt,
+      gate_kernel=None if gate is None else gate[:, part].contiguous())
+  pw = pack(slice(None))
   od = torch.float32 if kind == 'f32' else torch.bfloat16
   got = ops.gemm(x, pw, norm_scale=scale, out_dtype=od)
-  want = torch.cat([ops.gemm(x[a:a + 4].contiguous(), pw, norm_scale=scale, out_dtype=od)
-                    for a in range(0, M, 4)])
+  step = 4096 // (1 if gate is None else 2)
+  want = torch.cat([
+      torch.cat([ops.gemm(x[a:a + 4].contiguous(), some, norm_scale=scale, out_dtype=od)
+                 for a in range(0, M, 4)])
+      for some in (pack(slice(n, n + step)) for n in range(0, w.shape[1], step))], 1)
   two = ops.gemm(ops.rmsnorm(x, scale), pw, out_dtype=od).float()
   assert torch.equal(got, want)
   err = (got.float() - two).abs()  # (a normed value may round the other way)

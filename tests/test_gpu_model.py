@@ -463,23 +463,38 @@ def test_fused_loop_early_stop_is_independent_of_check_interval(check_every,
 
 @pytest.mark.parametrize('lanes,order', [(2, [0, 1]), (2, [1, 0]), (3, [2, 0, 1]),
                                          (4, [3, 1, 0, 2])])
-@pytest.mark.parametrize('seed,eos_bias', [(11, 6.0), (12, 3.0), (13, 0.0)])
-def test_lanes_that_run_far_apart_make_the_loops_iterations(lanes, order, seed,
-                                                            eos_bias):
+@pytest.mark.parametrize('seed,eos_bias,kw,ended', [
+    (11, 6.0, {}, None), (12, 3.0, {}, None), (13, 0.0, {}, None),
+    (14, 0.0, dict(max_decode_step=17), None), (15, 0.0, dict(max_decode_step=1), 1),
+    (16, 0.0, dict(min_log_prob=-60.0), None), (16, 0.0, dict(min_log_prob=-60.0), 0),
+    (16, 0.0, dict(min_log_prob=-60.0), 1), (17, 0.0, dict(min_log_prob=-60.0), 0),
+    (17, 0.0, dict(min_log_prob=-60.0), 1), (18, 0.0, dict(min_log_prob=0.0), 0)])
+def test_lanes_that_run_far_apart_make_the_loops_iterations(lanes, order, seed, eos_bias,
+                                                            kw, ended):
   """Lanes whose iterations are all enqueued one lane after the other: those whose items
-  have ended wait for what the others say, and every lane stops where the loop does."""
+  have ended wait for what the others say, and every lane stops where the loop does, at its
+  end, at a step, or where no item passes the least log-probability.  ended: a half of the
+  items, terminated from the start (by a finished sequence that nothing passes), so that
+  lanes may say yes for different reasons, which is no reason to stop."""
   from t5x_amd import decoding
   B, K, L = 4, 4, 40
   module, fn = _decode_setup('bfloat16', B, K, 16, L, seed=seed, eos_bias=eos_bias)
   module.decode_lanes = lanes
   inputs = np.zeros((B, L), np.int32)
-  plain = decoding.BeamLoop(inputs, dict(module.init_cache(B, L)), fn,
-                            eos_id=1, num_decodes=K)
+  def new_loop(cache):
+    loop = decoding.BeamLoop(inputs, cache, fn, eos_id=1, num_decodes=K, **kw)
+    if ended is not None:
+      half = slice(ended * B // 2, (ended + 1) * B // 2)
+      loop.cur.finished_scores[half] = 1.0
+      loop.cur.finished_flags[half] = 1
+    torch.cuda.synchronize()
+    return loop
+
+  plain = new_loop(dict(module.init_cache(B, L)))
   plain.run()
   want, ws = plain.finish()
   steps = int(plain.cur.cur_index.item())
-  fused = decoding.BeamLoop(inputs, module.init_cache(B, L), fn, eos_id=1,
-                            num_decodes=K)
+  fused = new_loop(module.init_cache(B, L))
   step = fused.fused
   assert step.keep_going()
   step._enqueued = L
@@ -493,6 +508,9 @@ def test_lanes_that_run_far_apart_make_the_loops_iterations(lanes, order, seed,
   assert int(fused.cur.cur_index.item()) == steps
   assert torch.equal(torch.as_tensor(got), torch.as_tensor(want))
   assert torch.equal(torch.as_tensor(gs), torch.as_tensor(ws))
+  if (seed, ended) == (16, 0):  # an iteration after which each lane said yes, to no one end
+    said = host(step.lane_records[:, 1:steps + 1]) & 3
+    assert (said.all(0) & (np.bitwise_and.reduce(said) == 0)).any()
 
 
 @pytest.mark.parametrize('lanes', [1, 2, 3])
@@ -563,13 +581,14 @@ def test_lanes_meet_every_few_iterations(slow):
   loop.finish()
 
 
+@pytest.mark.parametrize('lanes', [1, 2, 3])
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
-def test_fused_loop_context_is_reused_across_batches(dtype):
-  """A second (and third) batch of the same shape on the same module re-binds
+def test_fused_loop_context_is_reused_across_batches(dtype, lanes):
+  """Further batches of the same shape on the same module re-bind
   the first one's decode context — caches, cross K/V buffers, state, captured
-  graphs — instead of building a new one; every batch must still equal the
-  kernel-per-call loop, also after a batch that stopped early and with a
-  decode length that is not a multiple of the long graph's 8 iterations."""
+  graphs, what its lanes have recorded — instead of building a new one; every batch must still
+  equal the kernel-per-call loop, also a long one after one that stopped early and the
+  reverse, and with a decode length that is not a multiple of the long graph's 4 iterations."""
   from t5x_amd import decoding, models, network
   B, K, E, L = 3, 4, 16, 21
   _, gcfg = tiny(dtype)
@@ -577,10 +596,11 @@ def test_fused_loop_context_is_reused_across_batches(dtype):
   params = network.init_params(gcfg, 3, dev, with_encoder=False)
   params['decoder']['logits_dense']['kernel'][:, 1] *= 3.0  # some early EOS
   module = network.Transformer(gcfg, dev)
+  module.decode_lanes = lanes
   model = models.EncoderDecoderModel(module, decode_fn=decoding.beam_search)
   inputs = np.zeros((B, L), np.int32)
-  first = None
-  for batch in range(3):
+  first, lengths = None, []
+  for batch in range(8):
     rs = np.random.RandomState(100 + batch)
     tok = torch.as_tensor(ragged_tokens(rs, B, E, gcfg.vocab_size, 3),
                           device=dev)
@@ -602,9 +622,12 @@ def test_fused_loop_context_is_reused_across_batches(dtype):
     assert fused.fused is first and len(module._beam_ctx) == 1
     fused.run()
     got, gs = fused.finish()
-    assert int(fused.cur.cur_index.item()) == int(plain.cur.cur_index.item())
+    lengths.append(int(plain.cur.cur_index.item()))
+    assert int(fused.cur.cur_index.item()) == lengths[-1]
     assert torch.equal(torch.as_tensor(got), torch.as_tensor(want)), batch
     assert torch.equal(torch.as_tensor(gs), torch.as_tensor(ws)), batch
+  turns = np.sign(np.diff(lengths))
+  assert turns.min() < 0 < turns.max(), lengths  # shorter and longer than the one before
 
 
 @pytest.mark.parametrize('dtype,decode_fn_name,kw,lanes', [
@@ -664,7 +687,8 @@ def test_batches_in_flight_equal_batches_one_by_one(dtype, decode_fn_name, kw,
   assert len(pools[0]) == n_contexts
 
 
-def test_loops_in_flight_with_poll_equal_run():
+@pytest.mark.parametrize('lanes', [1, 2, 3])
+def test_loops_in_flight_with_poll_equal_run(lanes):
   """BeamLoop.start / poll (chunks enqueued ahead, the flag read without
   waiting) against BeamLoop.run, two loops interleaved by hand, and
   decoding.run_in_flight over three."""
@@ -675,6 +699,7 @@ def test_loops_in_flight_with_poll_equal_run():
   params = network.init_params(gcfg, 3, dev, with_encoder=False)
   params['decoder']['logits_dense']['kernel'][:, 1] *= 3.0
   module = network.Transformer(gcfg, dev)
+  module.decode_lanes = lanes
   model = models.EncoderDecoderModel(module, decode_fn=decoding.beam_search)
   inputs = np.zeros((B, L), np.int32)
 
