@@ -1330,8 +1330,15 @@ recurrence_step_kernel(RecArgs g) {
 // Whether a step forms its low-rank columns itself: where heads are as wide as the kernel's
 // variant, up to the rows measured.  Steps of 8 layers (6 of them recurrences, heads of 128,
 // 64 to 128 inputs), us with a dense layer in front / so, rows 1, 8, 64, 256: 8 heads (width
-// 1024) 224.7 / 216.2, 302 / 287, 438 / 424, 1114 / 1090; 16 heads 357 / 341, 468 / 451,
-// 785 / 773, 2013 / 1971.
+// 1024) 224.7 / 216.2, 302 / 287, 438 / 424, 1114 / 1090, rows 512 1589 / 1551; 16 heads
+// 357 / 341, 468 / 451, 785 / 773, 2013 / 1971.  Launches behind one another, us, dense layer
+// and step / so, 64 inputs, rows 1, 64, 128, 256, delta rule: 32 heads of 32 6.0 / 4.5, 10.6 /
+// 9.0, 15.7 / 14.2; 16 of 64 6.4 / 4.6, 10.4 / 8.7, 16.1 / 15.1, 28.5 / 24.8; 8 of 128 7.5 /
+// 5.9, 13.8 / 11.4, 25.8 / 24.1, 47.6 / 43.9; without it 5.4 / 3.7, 8.9 / 6.8, 13.0 / 10.5; 5.7
+// / 3.6, 9.1 / 7.5, 13.5 / 12.0, 26.5 / 22.7; 6.8 / 4.6, 12.8 / 10.1, 25.1 / 22.4, 45.9 / 41.7.
+// With 128 inputs up to 1 us of it goes: 32 heads of 32 with 128 rows 15.8 / 15.5, 16 of 64 16.3 /
+// 16.8, 256 rows 28.7 / 27.2, 8 of 128 48.1 / 44.9.  (Of 512 rows alone 91.4 / 98.3, in the
+// steps above it is the faster one.)
 static bool low_rides(const t5d_recurrence& a, int64_t rows) {
   return a.dtype == T5D_BF16 && a.D == a.Dv && (a.D == 32 || a.D == 64 || a.D == 128) &&
          a.taps <= 4 && (a.low_k == 64 || a.low_k == 128) && a.off_z % 16 == 0 &&
