@@ -6,6 +6,22 @@
 
 namespace t5d {
 
+// The workgroups of a launch, and which row tile of which columns each takes.  All row tiles of
+// the same columns go to one XCD, whose L2 has the weights then, and columns to the XCDs in turn
+// where that gives none more workgroups than its 32 CUs.  For 3, 5, 6 and 7 row tiles it may
+// give some 33 to 36 of up to 256, and these a second round (steps of 112 rows, width 1024, 599
+// us, two kernels 582; of 80 rows 508 and 516): then each takes an eighth of all in a row
+// (567 and 496).
+struct Work {
+  int blocks, per_xcd, part;  // part: 65536 / row tiles, rounded up (exact for 8 and 2^12)
+  Work(int N, int nt, int m_parts) {
+    const int groups = (N / 16 + 2 * nt - 1) / (2 * nt), columns = (groups + 7) / 8;
+    per_xcd = columns * m_parts > 32 ? (groups * m_parts + 7) / 8 : 0;
+    blocks = 8 * (per_xcd ? per_xcd : columns * m_parts);
+    part = (65536 + m_parts - 1) / m_parts;
+  }
+};
+
 // 512 threads own 16 rows and 2 NT column tiles.  Each of the 8 wavefronts norms two whole
 // rows, without a barrier; they meet the matrix cores through LDS.  For the products wavefront
 // (half, part) = (w / 4, w % 4) takes NT of the column tiles and every fourth pair of k-tiles
@@ -35,7 +51,7 @@ namespace t5d {
 // with K over 8 wavefronts (8.67, 64 x 768 x 4096 6.70 instead of 5.36).
 template <typename Args, int NT, int KQ, typename WT>
 __global__ void __launch_bounds__(512)
-norm_dense_kernel(Args g) {
+norm_dense_kernel(Args g, Work work) {
   constexpr bool kStream = IsStream<Args>::value, kLatent = IsLatent<Args>::value;
   constexpr bool kPlain = !kStream && !kLatent;
   constexpr int LD = 256 * KQ, HS = LD + 8;  // row stride of the normed rows
@@ -67,9 +83,9 @@ norm_dense_kernel(Args g) {
       return;
     }
   }
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int n_group = (slot / g.m_parts) * 8 + xcd;
-  const int m_part = slot % g.m_parts;
+  const int xcd = blockIdx.x & 7, slot = (blockIdx.x >> 3) + xcd * work.per_xcd;
+  const int q = slot * work.part >> 16, m_part = slot - q * g.m_parts;
+  const int n_group = work.per_xcd ? q : q * 8 + xcd;
   const int n_tiles_total = g.N >> 4, nt0 = n_group * 2 * NT;
   if (nt0 >= n_tiles_total) return;
   const int m0 = m_part * 16;
@@ -349,10 +365,10 @@ static int tiles_per_half(int M, int N, int most) {
 template <typename Args, typename WT>
 static void launch(int nt, Args g, hipStream_t s) {
   g.m_parts = (g.M + 15) / 16;
-  const int groups = (g.N / 16 + 2 * nt - 1) / (2 * nt);
-  const dim3 grid((groups + 7) / 8 * 8 * g.m_parts), block(512);
-#define T5D_ND_K(NT_, KQ_) \
-  hipLaunchKernelGGL((norm_dense_kernel<Args, NT_, KQ_, WT>), grid, block, 0, s, g)
+  const Work work(g.N, nt, g.m_parts);
+  const dim3 grid(work.blocks), block(512);
+#define T5D_ND_K(NT_, KQ_)                                                             \
+  hipLaunchKernelGGL((norm_dense_kernel<Args, NT_, KQ_, WT>), grid, block, 0, s, g, work)
 #define T5D_ND(NT_)                          \
   do {                                       \
     if (g.K <= 512) T5D_ND_K(NT_, 2);        \
@@ -390,13 +406,13 @@ bool launch_latent_dense(LatentDenseArgs g, hipStream_t s) {
   if (g.M > 128 || g.K > 1024 || g.K % 64 != 0) return false;
   const int nt = tiles_per_half(g.M, g.N, 2);
   if (nt == 0) return false;
-  const int groups = (g.N / 16 + 2 * nt - 1) / (2 * nt);
   g.m_parts = (g.M + 15) / 16;
-  g.dense_blocks = (groups + 7) / 8 * 8 * g.m_parts;
+  const Work work(g.N, nt, g.m_parts);
+  g.dense_blocks = work.blocks;
   const dim3 grid(g.dense_blocks + (g.kv != nullptr ? (g.M + 7) / 8 : 0)), block(512);
 #define T5D_LD_K(NT_, KQ_)                                                               \
   hipLaunchKernelGGL((norm_dense_kernel<LatentDenseArgs, NT_, KQ_, bf16_t>), grid, block, \
-                     0, s, g)
+                     0, s, g, work)
 #define T5D_LD(NT_)                        \
   do {                                     \
     if (g.K <= 512) T5D_LD_K(NT_, 2);      \
@@ -421,9 +437,16 @@ extern "C" int t5d_stream_rows_dense_rows(int dtype, int ld) {
 // Where the columns fit 256 workgroups of at most 8 column tiles (80 x 1024 x 8192 13.8 us as
 // two kernels, 18 here) and, beyond 768 inputs, take more than one tile of each: fewer are
 // not worth 96 KB of rows per workgroup (16 x 1024 x 3328 6.77 / 6.96, 64 x 1024 x 1024
-// 6.51 / 6.43, 24 x 1024 x 2304 6.80 / 6.48, 16 x 1024 x 5632 8.58 / 7.89).
+// 6.51 / 6.43, 24 x 1024 x 2304 6.80 / 6.48, 16 x 1024 x 5632 8.58 / 7.89).  There four
+// tiles of each half also want more than 192 workgroups (33 x 896 x 8192, 192, 10.25 / 10.94;
+// 64 x 896 x 8192, 256, 11.4 / 11.2; three tiles pay with 177: steps with a gated layer of 33 x
+// 1024 x 5632 378 / 372), and for 64 and 128 inputs three and four tiles do not pay (33 x 64 x
+// 8192 5.53 / 5.80, 80 x 128 x 4608 5.78 / 5.97).
 extern "C" int t5d_stream_rows_dense_pays(int M, int ld, int N) {
-  return tiles_per_half(M, N, 4) > 0 && (ld <= 768 || N / 16 * ((M + 15) / 16) > 256);
+  const int nt = tiles_per_half(M, N, 4), m_parts = (M + 15) / 16, tiles = N / 16;
+  if (nt == 0 || ld <= 128) return nt > 0 && nt < 3;
+  return ld <= 768 || (tiles * m_parts > 256 &&
+                       (nt < 4 || (tiles + 2 * nt - 1) / (2 * nt) * m_parts > 192));
 }
 
 extern "C" int t5d_stream_rows_dense(void* stream, const void* y, const float* y_norm,

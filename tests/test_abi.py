@@ -161,6 +161,21 @@ def test_low_rank_columns_that_are_not_there_without_gpu(rows, dtype, wrong):
   assert b'low-rank' in lib.t5d_last_error() or b't5d_dense' in lib.t5d_last_error()
 
 
+@pytest.mark.parametrize('M,ld,N,one', [
+    # columns that fit 256 workgroups, and not
+    (16, 512, 32768, 1), (16, 512, 32784, 0), (128, 768, 4096, 1), (128, 768, 4112, 0),
+    # beyond 768 inputs more than one column tile per CU, and of four tiles more than 192
+    # workgroups
+    (16, 1024, 4096, 0), (16, 1024, 4112, 1), (33, 1024, 5632, 1), (64, 1024, 5632, 1),
+    (33, 896, 8192, 0), (64, 896, 8192, 1), (96, 1024, 4096, 0), (112, 1024, 3328, 1),
+    (112, 1024, 4096, 1),
+    # few inputs, three and four tiles
+    (33, 64, 8192, 0), (33, 192, 8192, 1), (80, 128, 4608, 0), (80, 128, 3072, 1)])
+def test_where_the_row_kernel_and_a_layer_of_more_rows_go_in_one_launch(M, ld, N, one):
+  """t5d_stream_rows_dense_pays: not where the two launches were measured to be faster."""
+  assert _lib.load().t5d_stream_rows_dense_pays(M, ld, N) == one
+
+
 @pytest.mark.parametrize('name', ['proj', 'cq', 'q', 'uq', 'ql', 'ol', 'latent_ring'])
 @pytest.mark.parametrize('rows', [1, 200])
 def test_latent_operands_off_16_bytes_without_gpu(rows, name):

@@ -1539,7 +1539,9 @@ def test_norm_gemm_does_not_depend_on_its_tiles(ops, K, N, int8):
     (33, 192, 3088, 'plain'), (48, 512, 4096, 'geglu'), (65, 448, 5648, 'f32'),
     (128, 512, 4096, 'geglu'), (17, 768, 2320, 'plain'), (49, 704, 3088, 'geglu'),
     (128, 768, 2304, 'f32'), (16, 1024, 5632, 'geglu'), (33, 960, 4112, 'f32'),
-    (64, 1024, 5632, 'geglu'), (81, 832, 3072, 'plain')])
+    (64, 1024, 5632, 'geglu'), (81, 832, 3072, 'plain'),
+    # 5 and 7 row tiles of 50 and 36 columns of workgroups, an eighth of them to an XCD
+    (80, 512, 3200, 'plain'), (112, 768, 2304, 'geglu')])
 @pytest.mark.parametrize('int8', [False, True])
 def test_norm_in_front_of_many_columns(ops, M, K, N, kind, int8):
   """Rows normed once for many columns have the bits of the other kernel, which 4 rows at a

@@ -517,11 +517,13 @@ def test_token_ids_choose_the_experts(dtype):
 
 
 # queries of 64 to 1000 columns (the kernel's three widths), one and two column tiles per half
-# of a workgroup, a last row tile of one row; layers with a cache of their own and without
+# of a workgroup, a last row tile of one row; layers with a cache of their own and without;
+# 5 and 7 row tiles whose workgroups go to the XCDs an eighth each
 @pytest.mark.parametrize('S,H,D,q_rank,rank,own', [
     (1, 3, 20, 40, 24, True), (7, 8, 128, 512, 512, True), (16, 4, 64, 700, 300, False),
     (17, 8, 128, 512, 100, True), (64, 16, 128, 256, 512, True), (128, 2, 32, 1000, 40, True),
-    (128, 16, 128, 512, 512, False)])
+    (128, 16, 128, 512, 512, False), (80, 25, 64, 512, 512, True),
+    (112, 18, 128, 256, 512, True)])
 def test_new_latents_and_queries_in_one_launch(S, H, D, q_rank, rank, own):
   """The norms of the new latents and the queries' layer in one launch have the bits, outputs
   and rings, of two; norm weights that lie between 16 bytes keep these."""
