@@ -1384,7 +1384,9 @@ class FusedBeamStep(_OwnedContext):
                    loop.keep_going.data_ptr())
 
   # Iterations recorded in the long graph: one launch (and one gap between
-  # launches) per that many.
+  # launches) per that many.  (With 8, and chunks of 8 or 16: 36.7 / 36.8 ms for
+  # small 8 x 4 rows, one lane, 128 iterations, 66.2 / 66.6 base 8 x 4, 83.4 / 83.6
+  # base 32 x 4 with two; a loop that ends early runs up to two chunks on.)
   GRAPH_STEPS = 4
 
   def _record(self, lane, steps):
