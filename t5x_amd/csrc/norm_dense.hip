@@ -33,20 +33,21 @@ struct Work {
 // to 0.9 us).  So columns are spread over as many CUs as there are, and no further: each
 // workgroup norms its rows anew.  us, weights from memory:
 //   norm in norm_gemm_kernel / here       rows 16       32            64            128
-//     768 x 2304                     3.90          4.34 / 4.04   5.31 / 4.55   6.61 / 5.41
-//     768 x 4096 gated               4.38          4.91 / 4.47   5.84 / 4.90   7.28
-//     1024 x 3072                    4.69          5.19 / 4.70   6.46 / 5.13   7.97 / 7.06
-//     1024 x 5632 gated              5.89 / 5.63   7.30 / 6.45   9.02 / 7.96  12.08
-//     512 x 5632 gated               4.09          4.88 / 4.27   5.92 / 5.25   7.21
-//     1024 x 5632 gated, int8        5.58 / 5.11   6.94 / 6.11   8.98 / 7.80  12.50
+//     768 x 2304                     3.90          4.34 / 3.95   5.31 / 4.45   6.61 / 5.30
+//     768 x 4096 gated               4.38          4.91 / 4.35   5.84 / 4.80   7.28
+//     1024 x 3072                    4.69          5.19 / 4.57   6.46 / 5.30   7.97 / 6.92
+//     1024 x 5632 gated              5.89 / 5.52   7.30 / 6.40   9.02 / 7.80  12.08
+//     512 x 5632 gated               4.09          4.88 / 4.10   5.92 / 5.10   7.21
+//     1024 x 5632 gated, int8        5.58 / 5.10   6.94 / 6.18   8.98 / 7.73  12.50
 //   float32 stream, two kernels / here
-//     512 x 3328                     6.04 / 5.01   6.44 / 5.10   6.98 / 5.62   7.90 / 6.70
-//     768 x 4096 gated               6.60 / 6.15   7.06 / 6.34   8.23 / 7.23   9.95 / 9.12
-//     1024 x 3328                    6.77 / 6.96   7.49 / 7.10   8.76 / 8.17  10.77 / 10.37
-//     1024 x 5632 gated              8.58 / 7.89   9.43 / 8.81  11.09 / 10.41  13.6 / 17.8
+//     512 x 3328                     6.20 / 5.04   6.50 / 5.12   7.04 / 5.51   7.98 / 6.70
+//     768 x 4096 gated               6.55 / 6.00   6.87 / 6.16   7.79 / 6.76   9.52 / 8.18
+//     1024 x 3328                    6.63 / 6.45   7.07 / 6.72   8.35 / 7.58  10.12 / 9.70
+//     1024 x 5632 gated              8.06 / 7.31   8.69 / 8.28  10.37 / 9.82  12.91 / 18.6
 // A row in the lanes' own groups of 4 columns, its norm through LDS and another barrier, was
 // slower than these pieces, each half a wavefront reading what the other does too (64 x 1024 x
-// 5632 8.46 / 7.96, 64 x 768 x 2304 4.65 / 4.55), and gave sums another order.
+// 5632 8.46 / 7.96, 64 x 768 x 2304 4.65 / 4.55), and gave sums another order.  What stands in
+// front of the first load counts: a second division there, or gridDim, 0.3 to 0.5 us.
 // Tried and slower: 16 wavefronts (64 x 1024 x 5632 8.85), 4 (8.94), 32 rows per workgroup
 // with K over 8 wavefronts (8.67, 64 x 768 x 4096 6.70 instead of 5.36).
 template <typename Args, int NT, int KQ, typename WT>
@@ -435,9 +436,9 @@ extern "C" int t5d_stream_rows_dense_rows(int dtype, int ld) {
 }
 
 // Where the columns fit 256 workgroups of at most 8 column tiles (80 x 1024 x 8192 13.8 us as
-// two kernels, 18 here) and, beyond 768 inputs, take more than one tile of each: fewer are
-// not worth 96 KB of rows per workgroup (16 x 1024 x 3328 6.77 / 6.96, 64 x 1024 x 1024
-// 6.51 / 6.43, 24 x 1024 x 2304 6.80 / 6.48, 16 x 1024 x 5632 8.58 / 7.89).  There four
+// two kernels, 18 here) and, beyond 768 inputs, take more than one tile of each: for fewer both
+// are the same within a few percent (16 x 1024 x 2304 6.37 / 6.43, 33 x 1024 x 1024 6.39 / 6.43,
+// 16 x 1024 x 3328 6.63 / 6.45; 24 x 1024 x 2304 6.87 / 6.55, 16 x 1024 x 5632 8.06 / 7.31).  There four
 // tiles of each half also want more than 192 workgroups (33 x 896 x 8192, 192, 10.25 / 10.94;
 // 64 x 896 x 8192, 256, 11.4 / 11.2; three tiles pay with 177: steps with a gated layer of 33 x
 // 1024 x 5632 378 / 372), and for 64 and 128 inputs three and four tiles do not pay (33 x 64 x
