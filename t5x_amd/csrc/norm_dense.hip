@@ -438,11 +438,11 @@ extern "C" int t5d_stream_rows_dense_rows(int dtype, int ld) {
 // Where the columns fit 256 workgroups of at most 8 column tiles (80 x 1024 x 8192 13.8 us as
 // two kernels, 18 here) and, beyond 768 inputs, take more than one tile of each: for fewer both
 // are the same within a few percent (16 x 1024 x 2304 6.37 / 6.43, 33 x 1024 x 1024 6.39 / 6.43,
-// 16 x 1024 x 3328 6.63 / 6.45; 24 x 1024 x 2304 6.87 / 6.55, 16 x 1024 x 5632 8.06 / 7.31).  There four
-// tiles of each half also want more than 192 workgroups (33 x 896 x 8192, 192, 10.25 / 10.94;
-// 64 x 896 x 8192, 256, 11.4 / 11.2; three tiles pay with 177: steps with a gated layer of 33 x
-// 1024 x 5632 378 / 372), and for 64 and 128 inputs three and four tiles do not pay (33 x 64 x
-// 8192 5.53 / 5.80, 80 x 128 x 4608 5.78 / 5.97).
+// 16 x 1024 x 3328 6.63 / 6.45; 24 x 1024 x 2304 6.87 / 6.55, 16 x 1024 x 5632 8.06 / 7.31).
+// There four tiles of each half also want more than 192 workgroups (33 x 896 x 8192, 192, 10.25 /
+// 10.94; 64 x 896 x 8192, 256, 11.4 / 11.2; three tiles pay with 177: steps with a gated layer of
+// 33 x 1024 x 5632 378 / 372), and for 64 and 128 inputs three and four tiles do not pay (33 x
+// 64 x 8192 5.53 / 5.80, 80 x 128 x 4608 5.78 / 5.97).
 extern "C" int t5d_stream_rows_dense_pays(int M, int ld, int N) {
   const int nt = tiles_per_half(M, N, 4), m_parts = (M + 15) / 16, tiles = N / 16;
   if (nt == 0 || ld <= 128) return nt > 0 && nt < 3;
